@@ -74,26 +74,26 @@ def _case(model, dtype, layers, decoding=0, context=(0, 0), prompts=0, prompt=(0
 def listed():
     return [
         # somebody types to a small model and waits for the next word: latency and launches
-        _case("llama-3b", "bf16", 28, 1, (150, 150), name="3b, one reply"),
+        _case("llama-3b", "bf16", 28, 1, (150, 150), name="3b one reply"),
         # the decode step that bench.py quotes: eight requests of about 2,048 tokens
-        _case("llama-8b", "bf16", 32, 8, (1900, 2200), name="8b, decode 8"),
+        _case("llama-8b", "bf16", 32, 8, (1900, 2200), name="8b decode 8"),
         # a busy server: many requests of all lengths
-        _case("llama-8b", "bf16", 16, 64, (100, 2400), name="8b, decode 64"),
+        _case("llama-8b", "bf16", 16, 64, (100, 2400), name="8b decode 64"),
         # two people in long documents: the cache is most of what a step reads
-        _case("llama-8b", "bf16", 8, 2, (12000, 20000), name="8b, long documents"),
+        _case("llama-8b", "bf16", 8, 2, (12000, 20000), name="8b long documents"),
         # the prompt that bench.py quotes
-        _case("llama-8b", "bf16", 32, prompts=1, prompt=(2048, 2048), name="8b, prompt 2048"),
+        _case("llama-8b", "bf16", 32, prompts=1, prompt=(2048, 2048), name="8b prompt 2048"),
         # continuous batching: new prompts beside the requests that decode
-        _case("llama-3b", "bf16", 28, 24, (100, 1500), 2, (300, 1100), name="3b, prompts beside decode"),
+        _case("llama-3b", "bf16", 28, 24, (100, 1500), 2, (300, 1100), name="3b prompts beside decode"),
         # the 32-bit path: a prompt, and the next token of a few requests
-        _case("llama-3b", "fp32", 7, prompts=1, prompt=(400, 400), name="3b fp32, prompt 400"),
-        _case("llama-3b", "fp32", 7, 4, (200, 500), name="3b fp32, decode 4"),
+        _case("llama-3b", "fp32", 7, prompts=1, prompt=(400, 400), name="3b fp32 prompt 400"),
+        _case("llama-3b", "fp32", 7, 4, (200, 500), name="3b fp32 decode 4"),
         # routed experts: two prompts of odd lengths, and a batch that decodes
-        _case("buderax", "bf16", 8, prompts=2, prompt=(611, 1437), name="buderax, two prompts"),
-        _case("buderax", "bf16", 8, 12, (300, 1400), name="buderax, decode 12"),
+        _case("buderax", "bf16", 8, prompts=2, prompt=(611, 1437), name="buderax two prompts"),
+        _case("buderax", "bf16", 8, 12, (300, 1400), name="buderax decode 12"),
         # recurrent, windowed and latent layers: one prompt, and a batch that decodes
-        _case("gisodra", "bf16", 8, prompts=1, prompt=(2000, 2000), name="gisodra, prompt 2000"),
-        _case("gisodra", "bf16", 8, 8, (900, 1200), name="gisodra, decode 8"),
+        _case("gisodra", "bf16", 8, prompts=1, prompt=(2000, 2000), name="gisodra prompt 2000"),
+        _case("gisodra", "bf16", 8, 8, (900, 1200), name="gisodra decode 8"),
     ]
 
 
