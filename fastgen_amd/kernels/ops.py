@@ -802,10 +802,38 @@ def paged_attention(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v
 
 
 # ----------------------------------------------------------------------- gemm
+# k of a group: the 32-bit product's order of summation (and what its split over workgroups follows)
+GEMM_F32_GROUP = 1024
+
+
+def gemm_f32_plan(M: int, N: int, K: int, cus: int) -> Tuple[int, int, bool]:
+    """How the 32-bit product is cut: (tile rows / 32, tile columns / 32, whether every group of k has a workgroup
+    of its own); (0, 0, False): the kernel of up to 16 rows.  Every cut gives the same bits.
+
+    Measured on 256 compute units (us; N x K 3072 x 3072, 16384 x 3072, 3072 x 8192).  Tiles of 64 x 64 while they
+    give 600 workgroups (2048 rows: 374, 1883, 975 against 401, 2098, 1051 with 64 x 32), smaller ones below (64 rows,
+    64 x 64 / 64 x 32 / 32 x 32: 40 / 36 / 33, 77 / 81 / 90, 60 / 51 / 54); 32 rows where the last tile of 64 would be
+    at least half empty (200 rows: 59, 247, 140 against 75, 252, 143).  A workgroup a group of k while whole ranges
+    would be fewer than 1536 workgroups (400 rows: 103 against 112, 239 against 289; 16384 x 3072, 3328
+    workgroups: 447 against 440), if the groups' sums stay under 256 MB."""
+    if M <= 16:
+        return 0, 0, False
+    groups = -(-K // GEMM_F32_GROUP)
+    tiles = lambda mb, nb: -(-M // (32 * mb)) * -(-N // (32 * nb))
+    splits = lambda mb, nb: groups > 1 and tiles(mb, nb) < 6 * cus and M <= 4096 and groups * M * N * 4 <= 256 << 20
+    units = lambda mb, nb: tiles(mb, nb) * (groups if splits(mb, nb) else 1)
+    mb, nb = (1 if 0 < M % 64 <= 32 else 2), 2
+    if units(mb, nb) < 600 * cus // 256:
+        nb = 1
+    if units(mb, nb) < 600 * cus // 256:
+        mb = 1
+    return mb, nb, splits(mb, nb)
+
+
 def gemm_nt(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None,
             out_dtype: Optional[torch.dtype] = None) -> torch.Tensor:
-    """``x @ w.T`` with ``w [N, K]``, by the engine's own fp32-FMA kernel (sum
-    over k in ascending order; a row's result does not depend on the others)."""
+    """``x @ w.T`` with ``w [N, K]``, by the engine's own kernels: float32 on the fp32 matrix cores, bfloat16 by
+    fp32 FMA (sums over k in an order fixed by K; a row's result does not depend on the others)."""
     _gpu(x, w, out)
     _need(x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[1], "x [M,K] and w [N,K] must share K")
     _need(x.stride(1) == 1 and w.stride(1) == 1, "x and w need unit column stride")
@@ -815,6 +843,13 @@ def gemm_nt(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None
     if out is None:
         out = torch.empty((M, N), dtype=out_dtype or x.dtype, device=x.device)
     _need(out.shape == (M, N) and out.stride(1) == 1, "out must be [M, N]")
+    if x.dtype == torch.float32 and out.dtype == torch.float32:
+        mb, nb, split = gemm_f32_plan(M, N, K, compute_units())
+        part = torch.empty((-(-K // GEMM_F32_GROUP), M, N), dtype=torch.float32, device=x.device) if split else None
+        st = _lib.load("gemm").fg_gemm_f32(
+            _ptr(x), _ptr(w), _ptr(out), _ptr(part), M, N, K, x.stride(0), w.stride(0), out.stride(0), mb, nb, _stream(out))
+        _check(st, "gemm_nt")
+        return out
     for m0 in range(0, M, 65535 * 64):  # grid.y limit
         m1 = min(M, m0 + 65535 * 64)
         st = _lib.load("gemm").fg_gemm_nt(

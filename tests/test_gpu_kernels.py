@@ -332,6 +332,35 @@ def test_gemm_rows_do_not_depend_on_the_batch(ops):
         assert torch.equal(part, full[rows])  # bit for bit
 
 
+@pytest.mark.parametrize("N,K", [(1, 8), (33, 17), (130, 128), (68, 132), (515, 1028), (3072, 3072), (96, 8200)])
+def test_gemm_f32_every_cut_gives_the_same_bits(ops, N, K):
+    """The 32-bit product at the edges of its tiles, segments of 128 k and groups of 1024: the rows of a call, alone or
+    beside others, in rows of another stride (unaligned: the scalar loads), within the bound of the longest chain of
+    additions (32 in a chain of instructions, 4 chains, 8 segments, K / 1024 groups) of the double product."""
+    torch.manual_seed(N + K)
+    x, w = torch.randn(203, K).to(DEV), torch.randn(N, K).to(DEV)
+    x[7, K // 2] = float("nan")  # its row and no other
+    wide = torch.zeros(203, K + 5, device=DEV)
+    wide[:, 1:K + 1] = x
+    full = ops.gemm_nt(x, w)
+    assert torch.isnan(full[7]).all()
+    ok = [i for i in range(203) if i != 7]
+    bound = (32 + 4 + 8 + K / 1024 + 1) * 2.0 ** -24 * (x[ok].double().abs() @ w.double().abs().T)
+    assert ((full[ok].double() - x[ok].double() @ w.double().T).abs() <= bound).all()
+    assert torch.equal(ops.gemm_nt(wide[:, 1:K + 1], w)[ok], full[ok])
+    for first, last in ((0, 1), (10, 26), (10, 27), (8, 40), (8, 41), (8, 72), (8, 73), (11, 203)):
+        assert torch.equal(ops.gemm_nt(x[first:last], w), full[first:last]), (first, last)
+
+
+def test_gemm_f32_plan_is_bounded(ops):
+    for M in (1, 16, 17, 64, 65, 400, 4096, 4097, 200000):
+        for N in (1, 64, 3072, 128256):
+            for K in (8, 1024, 1025, 3072, 28672):
+                mb, nb, split = ops.gemm_f32_plan(M, N, K, 256)
+                assert (mb, nb) in ((0, 0), (1, 1), (1, 2), (2, 1), (2, 2)) and (mb > 0 or M <= 16)
+                assert not split or (M <= 65535 and -(-K // 1024) * M * N * 4 <= 256 << 20)
+
+
 @pytest.mark.parametrize("M", [1, 2, 8, 16, 17, 33, 64])
 @pytest.mark.parametrize("N,K", [(515, 240), (4096, 4096), (6144, 64), (48, 8), (1000, 14336), (16, 328)])
 @pytest.mark.parametrize("odtype", [torch.bfloat16, torch.float32])
