@@ -5,8 +5,9 @@
 // token's own position, in tiles of 64 keys that start at multiples of 64.
 // The arithmetic for a (token, head) therefore depends on nothing but that
 // token's keys: not on the batch, on how the prompt was cut, or on which
-// pages hold the keys.  This is the kernel of the 32-bit path and the
-// fallback of the bf16 path for shapes the MFMA kernel refuses.
+// pages hold the keys.  This is the fallback for shapes the matrix-core
+// kernels refuse; the 32-bit path runs `attention_f32_kernel` (below) for up
+// to 16 query heads a kv head, with the same guarantee.
 //
 // Semantics (fastgen/forward.py:176-258): query at position p of sequence b
 // sees keys 0..p of b through block_table[b]; scores (q.k)*scale, softmax in
@@ -145,6 +146,213 @@ __global__ __launch_bounds__(ATT_WAVES* FG_WAVE) void paged_attention_general_ke
   }
 }
 
+// ------------------------------------------------------------------ float32
+// The 32-bit path's attention on v_mfma_f32_16x16x4_f32 (fp32 products and sums).  A workgroup owns up to 16 rows:
+// the query heads of one kv head for a few consecutive tokens of one sequence (blocks of 16 / group tokens, cut where
+// the sequence changes; a workgroup a token is launched and all but a run's first leave, so that a prompt fills the
+// rows and the decoded tokens of many sequences do not wait for one another).  Tiles of 64 keys start at multiples of
+// 64; tile i belongs to wave i % 8 whatever the workgroup holds, a wave's tiles follow one another with a running
+// maximum, the eight waves' results are merged in order: a (token, head)'s arithmetic depends on its own keys alone,
+// so the bits are the same for a prompt, a decoded token and any cut.  S^T = K Q^T leaves a lane 4 keys of one row,
+// which is how O^T += V^T P^T takes them: nothing moves between lanes but a row's maximum and sum.  Keys and values
+// come straight from the pages, 1 KB (keys) and two halves of 2 KB (values) a load.
+//
+// Before: a wave a (token, head), a lane a key.  24 heads on 8 kv heads of 128, us before and now: a prompt of 400 /
+// 2048 tokens 174 / 3628 -> 59 / 592 (a third of the fp32 matrix cores' rate), one token of 4 sequences of 500 keys
+// 117 -> 30, of one of 4000 1243 -> 133 (the chain of a wave's 8 tiles), of 64 of 1000 455 -> 122, of 200 of 300 184 ->
+// 188 (both bound by the pages' reads, 2.6 TB/s).
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+#define AF_WAVES 8
+
+// DB: head dims in blocks of 16, at least hd / 16 (hd is a multiple of 8).
+template <int DB>
+__global__ __launch_bounds__(AF_WAVES* FG_WAVE) void attention_f32_kernel(
+    const float* __restrict__ q, int q_stride, float* __restrict__ out, int out_stride,
+    const float* __restrict__ k_pages, const float* __restrict__ v_pages, const int* __restrict__ block_table,
+    int bt_stride, const int* __restrict__ seq_of_token, const int* __restrict__ positions, int n_tokens, int n_heads,
+    int n_kv, int hd, int page_size, float scale, int window, const float* __restrict__ sinks,
+    const float* __restrict__ dist) {
+  constexpr int MB = DB < 8 ? DB : 8;             // dim blocks merged at a time
+  __shared__ f32x4 q_s[DB * 4][16];               // [4 dims][row]
+  __shared__ f32x4 o_s[AF_WAVES][MB][FG_WAVE];
+  __shared__ float m_s[AF_WAVES][16], l_s[AF_WAVES][16];
+  const int tid = threadIdx.x, lane = tid % FG_WAVE, wave = tid / FG_WAVE;
+  const int r = lane % 16, g = lane / 16;
+  const int kvh = blockIdx.x % n_kv, group = n_heads / n_kv;
+  // (the blocks' first tokens come first, a token's kv heads side by side: every die gets as many of them)
+  const int full = 16 / group, blocks = (n_tokens + full - 1) / full, place = blockIdx.x / n_kv;
+  const int t0 = place % blocks * full + place / blocks;
+  if (t0 >= n_tokens) return;
+  const int seq = seq_of_token[t0];
+  if (t0 % full && seq_of_token[t0 - 1] == seq) return;  // an earlier workgroup's run holds this token
+  int n_here = 1, p_lo = positions[t0], p_hi = p_lo;
+  for (; t0 + n_here < n_tokens && (t0 + n_here) % full && seq_of_token[t0 + n_here] == seq; ++n_here) {
+    const int p = positions[t0 + n_here];
+    p_lo = min(p_lo, p);
+    p_hi = max(p_hi, p);
+  }
+  const KvLayout lay(page_size, hd);
+  const size_t head_elems = (size_t)page_size * hd;
+
+  // this lane's row: a token of the block and one of its heads (rows behind the last repeat the last token)
+  const int mine = min(r / group, n_here - 1);
+  const bool live = r < n_here * group;
+  const int head = kvh * group + r % group, pos = positions[t0 + mine], first = first_key(pos, window);
+  const float d1 = dist ? dist[2 * head] : 0.f, d2 = dist ? dist[2 * head + 1] : 0.f;
+  for (int i = tid; i < DB * 4 * 16 * 4; i += AF_WAVES * FG_WAVE) {  // element by element: q may lie anywhere
+    const int d = i % (DB * 16), row = i / (DB * 16);
+    const int t = t0 + min(row / group, n_here - 1), h = kvh * group + row % group;
+    ((float*)&q_s[d / 4][row])[d % 4] = d < hd ? q[(size_t)t * q_stride + (size_t)h * hd + d] : 0.f;
+  }
+  __syncthreads();
+
+  const int* table = block_table + (size_t)seq * bt_stride;
+  const int lo = first_key(p_lo, window), hi = p_hi;  // the keys that some row of the run sees: their pages are held
+
+  f32x4 acc[DB];
+#pragma unroll
+  for (int i = 0; i < DB; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, l = 0.f;
+  for (int tile = lo / ATT_TILE + ((wave - lo / ATT_TILE) & (AF_WAVES - 1)); tile * ATT_TILE <= hi; tile += AF_WAVES) {
+    const int kb = tile * ATT_TILE;
+    const float* kp[4];
+    const float* vp[4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {  // (keys that no row sees are read as the nearest one that some row does)
+      const int key = min(max(kb + 16 * b + r, lo), hi);
+      kp[b] = k_pages + ((size_t)table[key / page_size] * n_kv + kvh) * head_elems + lay.k_off(key % page_size, 0);
+      const int four = min(max(kb + 16 * b + 4 * g, lo & ~3), hi & ~3), slot = lay.v_slot(four % page_size);
+      vp[b] = v_pages + ((size_t)table[four / page_size] * n_kv + kvh) * head_elems + slot % 8 +
+              lay.v_chunk_off(slot / 8, 0);
+    }
+    const size_t chunk = (size_t)8 << lay.kb_shift;  // from 8 head dims of a key to the next 8
+    f32x4 s[4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b) s[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < DB; ++i) {
+      const f32x4 qv = q_s[4 * i + g][r];
+      f32x4 kv[4];
+      const bool in = 16 * i + 4 * g < hd;
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+        kv[b] = in ? *(const f32x4*)(kp[b] + chunk * (2 * i + g / 2) + g % 2 * 4) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int b = 0; b < 4; ++b) s[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[b][e], qv[e], s[b], 0, 0, 0);
+    }
+    float top = -INFINITY;
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int key = kb + 16 * b + 4 * g + e;
+        float v = s[b][e] * scale;
+        if (dist) v -= d1 * log1pf(d2 * (float)(pos - key));
+        s[b][e] = live && key >= first && key <= pos ? v : -INFINITY;
+        top = fmaxf(top, s[b][e]);
+      }
+    top = fmaxf(top, __shfl_xor(top, 16, FG_WAVE));
+    top = fmaxf(top, __shfl_xor(top, 32, FG_WAVE));
+    const float m_new = fmaxf(m, top);
+    // a row that has seen no key yet, or sees none in this tile, stays as it is
+    const float alpha = m == m_new ? 1.f : expf(m - m_new);
+    float sum = 0.f;
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int key = kb + 16 * b + 4 * g + e;
+        s[b][e] = live && key >= first && key <= pos ? expf(s[b][e] - m_new) : 0.f;
+        sum += s[b][e];
+      }
+    sum += __shfl_xor(sum, 16, FG_WAVE);
+    sum += __shfl_xor(sum, 32, FG_WAVE);
+    l = l * alpha + sum;
+    m = m_new;
+    // whether some key of the tile is seen by one row of the run and not by another
+    const bool mixed = kb + ATT_TILE - 1 > p_lo || kb < first_key(p_hi, window);
+#pragma unroll
+    for (int i = 0; i < DB; ++i) {
+      acc[i] *= alpha;
+      const int d = 16 * i + r;
+      f32x4 vv[4];
+      const size_t at = lay.v_chunk_off(0, d);
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        vv[b] = d < hd ? *(const f32x4*)(vp[b] + at) : f32x4{0.f, 0.f, 0.f, 0.f};
+        // what lies behind the keys was never written and may be anything
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int key = kb + 16 * b + 4 * g + e;
+          if (key < lo || key > hi) vv[b][e] = 0.f;
+        }
+      }
+      bool bad = false;
+      if (mixed && p_lo != p_hi) {
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) bad |= !(fabsf(vv[b][e]) <= 3.402823466e38f);
+      }
+      if (!__any(bad)) {
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[b][e], s[b][e], acc[i], 0, 0, 0);
+      } else {  // an infinity or NaN among the values: a weight of zero would not keep it from the rows before it
+        for (int row = 0; row < 16; ++row) {
+          const int p = __shfl(pos, row, FG_WAVE), f = __shfl(first, row, FG_WAVE);
+          f32x4 one = acc[i];
+#pragma unroll
+          for (int b = 0; b < 4; ++b)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const int key = kb + 16 * b + 4 * g + e;
+              one = __builtin_amdgcn_mfma_f32_16x16x4f32(key >= f && key <= p ? vv[b][e] : 0.f, s[b][e], one, 0, 0, 0);
+            }
+          if (r == row) acc[i] = one;
+        }
+      }
+    }
+  }
+
+  // ---- the waves' results, in order
+  if (lane < 16) m_s[wave][r] = m, l_s[wave][r] = l;
+  __syncthreads();
+  float top = m_s[0][r];
+#pragma unroll
+  for (int w = 1; w < AF_WAVES; ++w) top = fmaxf(top, m_s[w][r]);
+  const float factor = m == top ? 1.f : expf(m - top);
+  float total = 0.f;
+#pragma unroll
+  for (int w = 0; w < AF_WAVES; ++w) total += l_s[w][r] * (m_s[w][r] == top ? 1.f : expf(m_s[w][r] - top));
+  // a sink: one more term exp(sinks[h]) in the softmax's denominator, which brings no value
+  if (sinks) total += expf(sinks[head] - top);
+  const float inv = 1.f / total;
+#pragma unroll
+  for (int i0 = 0; i0 < DB; i0 += MB) {
+#pragma unroll
+    for (int i = 0; i < MB; ++i) o_s[wave][i][lane] = acc[i0 + i] * factor;
+    __syncthreads();
+    if (wave < MB) {  // (a thread's lane stands for the same row and dims as above, its wave for the dim block)
+      f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int w = 0; w < AF_WAVES; ++w) o += o_s[w][wave][lane];
+      const int d = 16 * (i0 + wave) + 4 * g;
+      if (live) {
+        float* at = out + (size_t)(t0 + mine) * out_stride + (size_t)head * hd + d;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (d + e < hd) at[e] = o[e] * inv;
+      }
+    }
+    __syncthreads();
+  }
+}
+
 extern "C" int fg_paged_attention_general_sink(
     const void* q, int q_stride, void* out, int out_stride, const void* k_pages,
     const void* v_pages, const int* block_table, int bt_stride, const int* seq_of_token,
@@ -154,6 +362,22 @@ extern "C" int fg_paged_attention_general_sink(
   if (hd <= 0 || hd % 8 || hd > ATT_MAX_HD || page_size <= 0 || page_size % 8 || n_kv <= 0 ||
       n_heads <= 0 || n_heads % n_kv)
     return FG_ERR_ARG;
+  const int group = n_heads / n_kv;
+  if (dtype == FG_F32 && group <= 16) {
+    const int full = 16 / group;
+    const long long grid = (long long)((n_tokens + full - 1) / full * full) * n_kv;
+    if (grid > 2147483647LL) return FG_ERR_ARG;
+#define ATTENTION_F32(DB)                                                                                           \
+  attention_f32_kernel<DB><<<(unsigned)grid, AF_WAVES * FG_WAVE, 0, stream>>>(                                                \
+      (const float*)q, q_stride, (float*)out, out_stride, (const float*)k_pages, (const float*)v_pages, block_table, \
+      bt_stride, seq_of_token, positions, n_tokens, n_heads, n_kv, hd, page_size, scale, window, sinks, dist)
+    if (hd <= 64) ATTENTION_F32(4);
+    else if (hd <= 128) ATTENTION_F32(8);
+    else if (hd <= 256) ATTENTION_F32(16);
+    else ATTENTION_F32(32);
+#undef ATTENTION_F32
+    return fg_launch_status();
+  }
   const long long items = (long long)n_tokens * n_heads;
   const long long blocks = (items + ATT_WAVES - 1) / ATT_WAVES;
   if (blocks > 2147483647LL) return FG_ERR_ARG;

@@ -15,7 +15,7 @@ from plain_llama import (
     plain_top_p_keep,
 )
 
-from fastgen_amd.cache.layout import pack_k, pack_v, unpack_k, unpack_v
+from fastgen_amd.cache.layout import pack_k, pack_v, store_v, unpack_k, unpack_v
 
 pytestmark = pytest.mark.gpu
 
@@ -273,6 +273,37 @@ def test_paged_attention_general(ops, dtype, H, KV, hd, P, window):
     assert torch.isfinite(out).all()  # poison in unwritten slots never reaches the output
     assert torch.allclose(out.cpu().float(), want, **(dict(atol=2e-5, rtol=1e-5) if dtype == torch.float32
                                                        else dict(atol=1.5e-2, rtol=2e-2)))
+
+
+@pytest.mark.parametrize("H,KV,hd,P", [(24, 8, 128, 64), (16, 1, 24, 8), (5, 5, 136, 16), (34, 2, 64, 32), (3, 1, 512, 64),
+                                       (32, 2, 256, 32)])
+@pytest.mark.parametrize("window", [0, 100, -96])
+def test_paged_attention_f32_every_cut_gives_the_same_bits(ops, H, KV, hd, P, window):
+    """The 32-bit attention over the edges of its tiles of 64 keys and its blocks of 16 rows: a token alone (a workgroup
+    a token) gives the bits it gives beside the others (blocks of tokens, sequences meeting inside a block), within the
+    tolerance of `test_paged_attention_general`; a value that is not a number reaches the tokens that see it only."""
+    seqs = [(0, 330), (700, 1), (3, 2), (211, 130), (64, 1), (63, 1)]
+    case = _paged_case(torch.float32, seqs, H, KV, hd, P, seed=8)
+
+    def run(rows=slice(None)):
+        out = torch.empty_like(case["q"][rows])
+        return ops.paged_attention_general(case["q"][rows], out, case["kp"], case["vp"], case["table"],
+                                           case["seq_of"][rows], case["pos"][rows], H, hd**-0.5, window)
+
+    out = run()
+    if window >= 0:
+        assert torch.allclose(out.cpu(), _plain_rows(case, seqs, window or None), atol=2e-5, rtol=1e-5)
+    for t in (0, 1, 63, 64, 329, 330, 331, 332, 333, 380, 462, 463, 464):
+        assert torch.equal(run(slice(t, t + 1))[0], out[t]), t
+    assert torch.equal(run(slice(100, 170)), out[100:170])
+    # token 70 of the first sequence has a value of infinities in the first kv head
+    store_v(case["vp"], int(case["table"][0, 70 // P]), 0, 70 % P, torch.full((hd,), float("inf"), device=DEV))
+    got = run()
+    pos = case["pos"]
+    sees = (case["seq_of"] == 0) & (pos >= 70) & ((pos < 70 + window) if window > 0 else
+                                                  (pos < 96) if window < 0 else (pos >= 0))
+    assert torch.equal(got[~sees], out[~sees])
+    assert not torch.isfinite(got[sees][:, 0]).any()
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
