@@ -16,6 +16,11 @@
 // matrix as the A operand: 16 of its rows x 32 k, a tile's rows of x as B), one wave per 16 output
 // channels of a tile, its matrices streamed once for up to 16 * MB rows; the generic kernels (fp32 FMA,
 // any dtype and size) are the true 32-bit path.
+//
+// The matrix-core kernels take the experts' matrices row by row or packed (ldw = 0): per expert blocks of 16 rows x
+// 32 k in operand order, [expert][ceil(rows / 16)][ceil(k / 32)][64 lanes][8], zeros behind the last row and k.  A
+// wave's load is then 1 KB of whole lines; from rows it is 16 halves of a line, and the other halves are asked for
+// again a step later.
 #include "common.h"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -363,13 +368,80 @@ __device__ __forceinline__ bf16x8 moe_zero8() {
   for (int i = 0; i < 8; ++i) z[i] = (__bf16)0.f;
   return z;
 }
-// 16 bytes at row + k if k < K, else zeros; the load is always issued (from the row's start if not)
-__device__ __forceinline__ bf16x8 load_k(const bf16_t* row, int k, int K) {
-  const bf16x8 v = *(const bf16x8*)(row + (k < K ? k : 0));
-  return k < K ? v : moe_zero8();
+// What lies 32 s elements behind a lane's first chunk (k 8 g) of a row, or, if that is beyond k, a chunk that is there.
+__device__ __forceinline__ int moe_k_at(int s, int K, int g) {
+  return 32 * s + 8 * g < K ? 32 * s : (8 * g < K ? 0 : -8 * g);
 }
 
-template <int MB>
+// Where a lane finds its part of 16 matrix rows from `row` on at step s of 32 k: at base + s * stride elements.
+template <bool PACKED>
+struct MoeOperand {
+  const bf16_t* base;
+  __device__ __forceinline__ MoeOperand() {}
+  __device__ __forceinline__ MoeOperand(const bf16_t* w, int ldw, int expert, int rows, int row, int K, int lane) {
+    if constexpr (PACKED) {
+      const int blocks = (rows + 15) / 16, steps = (K + 31) / 32;
+      base = w + ((size_t)expert * blocks + min(row / 16, blocks - 1)) * steps * 512 + lane * 8;
+    } else {
+      base = w + ((size_t)expert * rows + min(row + lane % 16, rows - 1)) * ldw + 8 * (lane / 16);
+    }
+  }
+  // (behind k: any readable place; what stands there meets zeros of x)
+  __device__ __forceinline__ bf16x8 load(int s, int K, int g) const {
+    if constexpr (PACKED) return *(const bf16x8*)(base + (size_t)(32 * s < K ? s : 0) * 512);
+    else return *(const bf16x8*)(base + moe_k_at(s, K, g));
+  }
+};
+
+// The products of up to 16 MB rows of x (B operands at px) with NM blocks of 16 matrix rows: a wave alone streams the
+// matrices, U steps of 32 k a round, the next round's loads in flight while a round is multiplied.
+template <int NM, int MB, bool PACKED>
+__device__ __forceinline__ void moe_stream(const MoeOperand<PACKED> (&w)[NM], const bf16_t* const (&px)[MB], int K, int g,
+                                           f32x4 (&acc)[NM][MB]) {
+  constexpr int U = MB == 1 ? 4 : 2;
+  bf16x8 a[2][U][NM], b[2][U][MB];
+  auto load = [&](int s0, int set) {
+#pragma unroll
+    for (int i = 0; i < U; ++i)
+#pragma unroll
+      for (int m = 0; m < NM; ++m) a[set][i][m] = w[m].load(s0 + i, K, g);
+#pragma unroll
+    for (int i = 0; i < U; ++i)
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) b[set][i][mb] = *(const bf16x8*)(px[mb] + moe_k_at(s0 + i, K, g));
+  };
+  auto multiply = [&](int s0, int set) {
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+      const bool in = 32 * (s0 + i) + 8 * g < K;
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) {
+        const bf16x8 bv = in ? b[set][i][mb] : moe_zero8();
+#pragma unroll
+        for (int m = 0; m < NM; ++m) acc[m][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[set][i][m], bv, acc[m][mb], 0, 0, 0);
+      }
+    }
+  };
+#pragma unroll
+  for (int m = 0; m < NM; ++m)
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) acc[m][mb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int steps = (K + 31) / 32;
+  load(0, 0);
+  for (int s = 0; s < steps; s += 2 * U) {
+    load(s + U, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(s, 0);
+    load(s + 2 * U, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(s + U, 1);
+  }
+}
+
+// Bound by the experts' matrices (12 tokens of 32 experts of 768 x 2048, top 4: 161 and 80 MB): 39 / 21 us from packed
+// matrices, 54 / 24 from rows (and 50 / 23 with rounds of 8 steps whose loads all returned before the next were asked for);
+// one token 16.5 / 8.2 us (23.7 / 9.3 from rows).
+template <int MB, bool PACKED>
 __global__ __launch_bounds__(256) void moe_gate_up_mfma_kernel(
     const bf16_t* __restrict__ x, int ldx, const bf16_t* __restrict__ wg, const bf16_t* __restrict__ wu, int ldw,
     const int* __restrict__ sorted, const int* __restrict__ tiles, int max_tiles, int top, int dim, int hidden,
@@ -382,40 +454,16 @@ __global__ __launch_bounds__(256) void moe_gate_up_mfma_kernel(
   const int4 tile = *(const int4*)(tiles + 4 * (size_t)ti);
   if (tile.z <= 0) return;
   const int r16 = lane & 15, g = lane >> 4;
-  const size_t wrow = ((size_t)tile.x * hidden + min(c0 + r16, hidden - 1)) * ldw;  // rows beyond the matrix: clamped, not stored
-  const bf16_t* pg = wg + wrow;
-  const bf16_t* pu = wu + wrow;
+  // (rows beyond the matrix: clamped, not stored)
+  const MoeOperand<PACKED> w[2] = {{wg, ldw, tile.x, hidden, c0, dim, lane}, {wu, ldw, tile.x, hidden, c0, dim, lane}};
   const bf16_t* px[MB];
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb) {
     const int r = min(mb * 16 + r16, tile.z - 1);
-    px[mb] = x + (size_t)(sorted[tile.y + r] / top) * ldx;
+    px[mb] = x + (size_t)(sorted[tile.y + r] / top) * ldx + 8 * g;
   }
-  f32x4 ag[MB], au[MB];
-#pragma unroll
-  for (int mb = 0; mb < MB; ++mb) ag[mb] = au[mb] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // U steps of 32 k a round, all their loads issued before the first MFMA: with few rows a wave is a chain of
-  // memory round trips, and the fewer of them the better (8 steps for one block of rows: 24 loads in flight)
-  constexpr int U = MB == 1 ? 8 : (MB == 2 ? 4 : 2);
-  for (int k0 = 8 * g; k0 < dim + 8 * g; k0 += 32 * U) {  // this lane's k: 8 g, 8 g + 32, ...
-    bf16x8 a[U], u[U], b[U][MB];
-#pragma unroll
-    for (int i = 0; i < U; ++i) {
-      a[i] = load_k(pg, k0 + 32 * i, dim);
-      u[i] = load_k(pu, k0 + 32 * i, dim);
-    }
-#pragma unroll
-    for (int i = 0; i < U; ++i)
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb) b[i][mb] = load_k(px[mb], k0 + 32 * i, dim);
-#pragma unroll
-    for (int i = 0; i < U; ++i)
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb) {
-        ag[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[i][mb], ag[mb], 0, 0, 0);
-        au[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(u[i], b[i][mb], au[mb], 0, 0, 0);
-      }
-  }
+  f32x4 acc[2][MB];
+  moe_stream<2, MB, PACKED>(w, px, dim, g, acc);
   // the lane holds, for the tile's row mb * 16 + r16, channels c0 + 4 g .. + 3
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb) {
@@ -424,7 +472,7 @@ __global__ __launch_bounds__(256) void moe_gate_up_mfma_kernel(
     bf16x4 o;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      o[i] = (__bf16)gated_act<true>(ag[mb][i], au[mb][i], fn);
+      o[i] = (__bf16)gated_act<true>(acc[0][mb][i], acc[1][mb][i], fn);
     }
     bf16_t* dst = act + (size_t)(tile.y + r) * lda + c;
     if (c + 3 < hidden) {
@@ -435,7 +483,7 @@ __global__ __launch_bounds__(256) void moe_gate_up_mfma_kernel(
   }
 }
 
-template <int MB>
+template <int MB, bool PACKED>
 __global__ __launch_bounds__(256) void moe_down_mfma_kernel(
     const bf16_t* __restrict__ act, int lda, const bf16_t* __restrict__ wd, int ldw, const int* __restrict__ sorted,
     const int* __restrict__ tiles, int max_tiles, int dim, int hidden, float* __restrict__ y) {
@@ -447,180 +495,189 @@ __global__ __launch_bounds__(256) void moe_down_mfma_kernel(
   const int4 tile = *(const int4*)(tiles + 4 * (size_t)ti);
   if (tile.z <= 0) return;
   const int r16 = lane & 15, g = lane >> 4;
-  const bf16_t* pw = wd + ((size_t)tile.x * dim + min(c0 + r16, dim - 1)) * ldw;
+  const MoeOperand<PACKED> w[1] = {{wd, ldw, tile.x, dim, c0, hidden, lane}};
   const bf16_t* pa[MB];
 #pragma unroll
-  for (int mb = 0; mb < MB; ++mb) pa[mb] = act + (size_t)(tile.y + min(mb * 16 + r16, tile.z - 1)) * lda;
-  f32x4 acc[MB];
-#pragma unroll
-  for (int mb = 0; mb < MB; ++mb) acc[mb] = f32x4{0.f, 0.f, 0.f, 0.f};
-  constexpr int U = MB == 1 ? 8 : (MB == 2 ? 4 : 2);  // as in gate_up
-  for (int k0 = 8 * g; k0 < hidden + 8 * g; k0 += 32 * U) {
-    bf16x8 a[U], b[U][MB];
-#pragma unroll
-    for (int i = 0; i < U; ++i) a[i] = load_k(pw, k0 + 32 * i, hidden);
-#pragma unroll
-    for (int i = 0; i < U; ++i)
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb) b[i][mb] = load_k(pa[mb], k0 + 32 * i, hidden);
-#pragma unroll
-    for (int i = 0; i < U; ++i)
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb) acc[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[i][mb], acc[mb], 0, 0, 0);
-  }
+  for (int mb = 0; mb < MB; ++mb) pa[mb] = act + (size_t)(tile.y + min(mb * 16 + r16, tile.z - 1)) * lda + 8 * g;
+  f32x4 acc[1][MB];
+  moe_stream<1, MB, PACKED>(w, pa, hidden, g, acc);
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb) {
     const int r = mb * 16 + r16, c = c0 + 4 * g;
     if (r >= tile.z || c >= dim) continue;
     float* dst = y + (size_t)sorted[tile.y + r] * dim + c;
     if (c + 3 < dim && dim % 4 == 0) {
-      *(f32x4*)dst = acc[mb];
+      *(f32x4*)dst = acc[0][mb];
     } else {
-      for (int i = 0; c + i < dim; ++i) dst[i] = acc[mb][i];
+      for (int i = 0; c + i < dim; ++i) dst[i] = acc[0][mb][i];
     }
   }
 }
 
-// ------------------------------------------------------- large tiles through LDS
-// Many rows an expert (prompt steps): a workgroup owns a tile of up to 64 WM rows of one expert and 128
-// output columns, its WM x 2 waves 64 x 64 each; both operands go from memory straight into LDS
-// (global_load_lds) through a ring of NST stages of 32 k, as in gemm_tiled.hip, whose loop this is.  What
-// differs is where the rows come from and go to: the tile's rows of x are gathered by token (gate_up) or
-// are its sorted places (down), the matrix is the tile's expert's, and for gate_up its 16-row blocks are
-// made of 8 gate rows and the 8 up rows of the same channels as they are loaded (nothing is stored
-// interleaved), so that silu(gate) * up is applied to the accumulators.
+// ------------------------------------------------------- large tiles
+// Many rows an expert (prompt steps): a workgroup owns a tile of up to 128 WM rows of one expert and 256 rows of its
+// matrix, a wave 128 x 64.  A compute unit takes in 64 bytes a clock from the vector memory path and reads 128 from LDS,
+// and a wave's tile of 64 x 64 with both operands through LDS (the loop of gemm_tiled.hip) needs all of the one and one
+// and a half times the other at the matrix cores' full rate.  So the rows of x, which the waves share, go through LDS
+// and the rows of the matrix, which are a wave's own, from memory into its registers in operand order: 48 bytes a clock
+// and 0.6 of LDS.  Rows of x are asked for two steps of 32 k ahead (registers, then one of two LDS buffers), rows of the
+// matrix three; one barrier a step.  1897 tokens, 32 experts of 768 x 2048, top 4 (237 rows an expert, 48 + 24 GFLOP): 86 /
+// 67 us, 116 / 83 with the matrices in rows, 150 / 87 with tiles of 64 x 64 a wave; 6000 tokens 182 / 142 us against 344 /
+// 210, 0.83 / 0.53 PFLOP/s.  The tile's rows are gathered by token (gate_up) or are its sorted places (down);
+// for gate_up a block of 16 matrix rows is 8 gate rows and the 8 up rows of the same channels, so that silu(gate) * up is
+// applied to the accumulators.
 #define MT_GATE_UP 0
 #define MT_DOWN 1
+#define MT_RUN 4
 
-template <int N>
-__device__ __forceinline__ void moe_wait_vmcnt() {
-  static_assert(N >= 0 && N < 64, "vmcnt has six bits");
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
-}
-
-template <int WM, int NST, int EPI>
-__global__ __launch_bounds__(128 * WM) void moe_tiled_kernel(
+template <int WM, int NB, bool PACKED, int EPI>
+__global__ __launch_bounds__(256 * WM, 2) void moe_tiled_kernel(
     const bf16_t* __restrict__ x, int ldx, const bf16_t* __restrict__ w0, const bf16_t* __restrict__ w1, int ldw,
-    void* __restrict__ y, int ldy, const int* __restrict__ sorted, const int* __restrict__ tiles, int top,
-    int N /* rows of the matrix as the tile sees it: 2 * hidden (gate_up), dim (down) */, int K, const GatedAct fn) {
-  constexpr int WN = 2, NW = WM * WN, WB = 4 * WN, XB = 4 * WM, NB = WB + XB, LPW = NB / NW, BLOCK = 16 * 32;
-  static_assert(NB % NW == 0 && NST >= 3 && LPW * (NST - 2) < 64, "blocks divide over the waves; loads fit the counter");
-  extern __shared__ __attribute__((aligned(16))) bf16_t ring[];  // [NST][NB][BLOCK]
-  const int4 tile = *(const int4*)(tiles + 4 * (size_t)blockIdx.y);
+    void* __restrict__ y, int ldy, const int* __restrict__ sorted, const int* __restrict__ tiles, int max_tiles, int top,
+    int N /* columns of the result: hidden (gate_up), dim (down) */, int K, const GatedAct fn) {
+  constexpr int XB = 8 * WM, BLOCK = 16 * 32;  // blocks of 16 rows of x; each lies in LDS as its lanes' operands
+  constexpr int WAVE_N = EPI == MT_GATE_UP ? 8 * NB : 16 * NB, COLS = 4 * WAVE_N;  // columns of a wave, of the workgroup
+  __shared__ __attribute__((aligned(16))) bf16_t xs[2][XB][BLOCK];
+  // a run of MT_RUN tiles (an expert's mostly) and one block of columns stays on one die, whose L2 the matrix is read
+  // into once
+  const int cols = (N + COLS - 1) / COLS, place = blockIdx.x / 8, run = place / MT_RUN * 8 + blockIdx.x % 8;
+  const int ti = run / cols * MT_RUN + place % MT_RUN;
+  if (ti >= max_tiles) return;
+  const int4 tile = *(const int4*)(tiles + 4 * (size_t)ti);
   if (tile.z <= 0) return;  // (the whole workgroup)
   const int lane = threadIdx.x % FG_WAVE, wave = threadIdx.x / FG_WAVE;
   const int r16 = lane & 15, g = lane >> 4;
-  const int wm = wave / WN, wn = wave % WN;
-  const int n_base = blockIdx.x * (64 * WN);
-  const int n_stages = (K + 31) / 32;
+  const int wm = wave / 4, wn = wave % 4;
+  const int n_base = run % cols * COLS + wn * WAVE_N;
+  const int n_steps = (K + 31) / 32;
 
-  const bf16_t* src[LPW];
+  const bf16_t* xsrc[2];  // a wave brings two blocks of x a step
 #pragma unroll
-  for (int j = 0; j < LPW; ++j) {
-    const int b = wave + NW * j;
-    if (b >= WB) {
-      const int pos = tile.y + min(16 * (b - WB) + r16, tile.z - 1);  // rows beyond the tile: its last row, not stored
-      src[j] = x + (size_t)(EPI == MT_GATE_UP ? sorted[pos] / top : pos) * ldx + 8 * g;
-    } else {
-      const int vr = min(n_base + 16 * b + r16, N - 1);
-      if (EPI == MT_GATE_UP)
-        src[j] = ((vr & 8) ? w1 : w0) + ((size_t)tile.x * (N >> 1) + ((vr >> 4) << 3) + (vr & 7)) * ldw + 8 * g;
-      else
-        src[j] = w0 + ((size_t)tile.x * N + vr) * ldw + 8 * g;
-    }
+  for (int j = 0; j < 2; ++j) {
+    const int pos = tile.y + min(16 * (wave + 4 * WM * j) + r16, tile.z - 1);  // rows beyond the tile: its last row, not stored
+    xsrc[j] = x + (size_t)(EPI == MT_GATE_UP ? sorted[pos] / top : pos) * ldx + 8 * g;
   }
-  auto issue = [&](int s) {
-    const int k = 32 * min(s, n_stages - 1);
-    const int koff = k + 8 * g < K ? k : 0;  // a chunk beyond k: any readable one, zeroed at use
-    bf16_t* slot = ring + (size_t)(s % NST) * NB * BLOCK;
+  MoeOperand<PACKED> w[NB];  // gate_up: the first half gate rows, the second the up rows of the same channels
 #pragma unroll
-    for (int j = 0; j < LPW; ++j)
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src[j] + koff),
-                                       (__attribute__((address_space(3))) void*)(slot + (wave + NW * j) * BLOCK), 16, 0, 0);
+  for (int nb = 0; nb < NB; ++nb)
+    w[nb] = EPI == MT_DOWN ? MoeOperand<PACKED>(w0, ldw, tile.x, N, n_base + 16 * nb, K, lane)
+                           : MoeOperand<PACKED>(nb < NB / 2 ? w0 : w1, ldw, tile.x, N, n_base + 16 * (nb % (NB / 2)), K, lane);
+  bf16x8 xr[2][2], wr[4][NB];
+  f32x4 acc[8][NB];  // [row block mb][matrix block nb]
+#pragma unroll
+  for (int mb = 0; mb < 8; ++mb)
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) acc[mb][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  // what step s needs: a chunk beyond k is any readable one and multiplied by a row of x of zeros
+  auto load_x = [&](int s, bf16x8(&to)[2]) {
+    const int at = moe_k_at(s, K, g);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) to[j] = *(const bf16x8*)(xsrc[j] + at);
   };
-
-  f32x4 acc[4][4];  // [row block mb][column block nb]
+  auto load_w = [&](int s, bf16x8(&to)[NB]) {
 #pragma unroll
-  for (int mb = 0; mb < 4; ++mb)
+    for (int nb = 0; nb < NB; ++nb) to[nb] = w[nb].load(s, K, g);
+  };
+  auto store_x = [&](int s, int buf, const bf16x8(&from)[2]) {
+    const bool in = 32 * s + 8 * g < K;  // (asked here: behind the load it would wait for the load)
 #pragma unroll
-    for (int nb = 0; nb < 4; ++nb) acc[mb][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < 2; ++j) *(bf16x8*)(&xs[buf][wave + 4 * WM * j][lane * 8]) = in ? from[j] : moe_zero8();
+  };
+  load_x(0, xr[0]);
+  load_w(0, wr[0]);
+  load_x(1, xr[1]);
+  load_w(1, wr[1]);
+  load_w(2, wr[2]);
+  store_x(0, 0, xr[0]);
+  __syncthreads();
+  // Four steps a round, so that the register sets have fixed names, in one block of code: with an exit between them
+  // the compiler moves the loads behind it, to where their results are used.  (The last round's steps beyond k
+  // multiply by zeros.)
+  for (int i0 = 0; i0 < n_steps; i0 += 4) {
 #pragma unroll
-  for (int s = 0; s < NST - 1; ++s) issue(s);
-  for (int i = 0; i < n_stages; ++i) {
-    moe_wait_vmcnt<LPW*(NST - 2)>();  // this wave's loads of stage i have landed
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();  // everybody's have, and nobody reads stage i - 1 any more
-    asm volatile("" ::: "memory");
-    issue(i + NST - 1);
-    const bf16_t* st = ring + (size_t)(i % NST) * NB * BLOCK;
-    const bool in = 32 * i + 8 * g < K;
-    bf16x8 a[4], b[4];
+    for (int u = 0; u < 4; ++u) {
+      const int i = i0 + u;
+      load_x(i + 2, xr[u % 2]);
+      load_w(i + 3, wr[(u + 3) % 4]);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int nb = 0; nb < 4; ++nb) {
-      a[nb] = *(const bf16x8*)(st + (wn * 4 + nb) * BLOCK + lane * 8);
-      a[nb] = in ? a[nb] : moe_zero8();
+      for (int half = 0; half < 2; ++half) {
+        bf16x8 b[4];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) b[m] = *(const bf16x8*)(&xs[u % 2][8 * wm + 4 * half + m][lane * 8]);
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+          for (int m = 0; m < 4; ++m)
+            acc[4 * half + m][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wr[u % 4][nb], b[m], acc[4 * half + m][nb], 0, 0, 0);
+      }
+      store_x(i + 1, (u + 1) % 2, xr[(u + 1) % 2]);
+      __syncthreads();
     }
-#pragma unroll
-    for (int mb = 0; mb < 4; ++mb) b[mb] = *(const bf16x8*)(st + (WB + wm * 4 + mb) * BLOCK + lane * 8);
-#pragma unroll
-    for (int nb = 0; nb < 4; ++nb)
-#pragma unroll
-      for (int mb = 0; mb < 4; ++mb) acc[mb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[nb], b[mb], acc[mb][nb], 0, 0, 0);
   }
-  moe_wait_vmcnt<0>();  // the loads issued past the end land before the workgroup's LDS is given up
 
-  // acc[mb][nb][i]: the tile's row 64 wm + 16 mb + r16, matrix row n_base + 64 wn + 16 nb + 4 g + i
+  // acc[mb][nb][i]: the tile's row 128 wm + 16 mb + r16, row 4 g + i of the matrix block nb
 #pragma unroll
-  for (int mb = 0; mb < 4; ++mb) {
-    const int ml = 64 * wm + 16 * mb + r16;
-    const bool valid = ml < tile.z;
-    const int pos = tile.y + min(ml, tile.z - 1);
+  for (int mb = 0; mb < 8; ++mb) {
+    const int ml = 128 * wm + 16 * mb + r16;
+    if (ml >= tile.z) continue;
+    const int pos = tile.y + ml;
+    if constexpr (EPI == MT_DOWN) {
+      float* row = (float*)y + (size_t)sorted[pos] * ldy;
 #pragma unroll
-    for (int nb = 0; nb < 4; ++nb) {
-      const int n0 = n_base + 64 * wn + 16 * nb;
-      if (EPI == MT_DOWN) {
-        const int n = n0 + 4 * g;
-        if (!valid) continue;
-        float* dst = (float*)y + (size_t)sorted[pos] * ldy + n;
+      for (int nb = 0; nb < NB; ++nb) {
+        const int n = n_base + 16 * nb + 4 * g;
         if (n + 3 < N && (ldy & 3) == 0) {
-          *(f32x4*)dst = acc[mb][nb];
+          *(f32x4*)(row + n) = acc[mb][nb];
         } else {
 #pragma unroll
           for (int i = 0; i < 4; ++i)
-            if (n + i < N) dst[i] = acc[mb][nb][i];
+            if (n + i < N) row[n + i] = acc[mb][nb][i];
         }
-      } else {
-        // lane groups 0, 1 hold the gate rows 4 g + i of 8 channels, groups 2, 3 the up rows of the same channels
+      }
+    } else {
+#pragma unroll
+      for (int nb = 0; nb < NB / 2; ++nb) {
+        const int n = n_base + 16 * nb + 4 * g;
         bf16x4 v;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float up = __shfl_xor(acc[mb][nb][i], 32, FG_WAVE);
-          const float gate = acc[mb][nb][i];
-          v[i] = (__bf16)gated_act<true>(gate, up, fn);
-        }
-        if (g < 2 && valid && n0 + 15 < N) *(bf16x4*)((bf16_t*)y + (size_t)pos * ldy + n0 / 2 + 4 * g) = v;
+        for (int i = 0; i < 4; ++i) v[i] = (__bf16)gated_act<true>(acc[mb][nb][i], acc[mb][nb + NB / 2][i], fn);
+        if (n < N) *(bf16x4*)((bf16_t*)y + (size_t)pos * ldy + n) = v;  // (N is a multiple of 8)
       }
     }
   }
+}
+
+template <int WM, int NB, int EPI>
+static int launch_moe_tiled_as(const void* x, int ldx, const void* w0, const void* w1, int ldw, void* y, int ldy,
+                               const int* sorted, const int* tiles, int max_tiles, int top, int N, int K, const GatedAct fn,
+                               hipStream_t stream) {
+  constexpr int COLS = (EPI == MT_GATE_UP ? 32 : 64) * NB;
+  const long long runs = (long long)((max_tiles + MT_RUN - 1) / MT_RUN) * ((N + COLS - 1) / COLS);
+  const long long grid = (runs + 7) / 8 * 8 * MT_RUN;
+  if (grid > 2147483647LL) return FG_ERR_ARG;
+  if (ldw == 0)
+    moe_tiled_kernel<WM, NB, true, EPI><<<(unsigned)grid, 256 * WM, 0, stream>>>(
+        (const bf16_t*)x, ldx, (const bf16_t*)w0, (const bf16_t*)w1, ldw, y, ldy, sorted, tiles, max_tiles, top, N, K, fn);
+  else
+    moe_tiled_kernel<WM, NB, false, EPI><<<(unsigned)grid, 256 * WM, 0, stream>>>(
+        (const bf16_t*)x, ldx, (const bf16_t*)w0, (const bf16_t*)w1, ldw, y, ldy, sorted, tiles, max_tiles, top, N, K, fn);
+  return fg_launch_status();
 }
 
 template <int WM, int EPI>
 static int launch_moe_tiled(const void* x, int ldx, const void* w0, const void* w1, int ldw, void* y, int ldy,
                             const int* sorted, const int* tiles, int max_tiles, int top, int N, int K, const GatedAct fn,
                             hipStream_t stream) {
-  constexpr int NST = 4, lds = NST * 4 * (WM + 2) * 1024;
-  static bool raised = false;  // more than 64 KB of dynamic LDS has to be asked for once
-  auto kernel = moe_tiled_kernel<WM, NST, EPI>;
-  if (lds > 65536 && !raised) {
-    if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
-      return FG_ERR_LAUNCH;
-    raised = true;
-  }
-  if (max_tiles > 65535) return FG_ERR_ARG;
-  const dim3 grid((N + 127) / 128, max_tiles);
-  kernel<<<grid, 128 * WM, lds, stream>>>((const bf16_t*)x, ldx, (const bf16_t*)w0, (const bf16_t*)w1, ldw, y, ldy, sorted,
-                                          tiles, top, N, K, fn);
-  return fg_launch_status();
+  // Narrow matrix tiles (a wave 128 x 32) while wide ones would leave a third of the compute units without a workgroup.
+  // Measured (us, gate_up / down, packed, narrow against wide): 16 experts of 704 x 1024, top 2, 700 tokens (at most 26
+  // tiles, 156 / 104 wide workgroups) 24 / 20 against 29 / 24, 1897 tokens (270 / 180) 35 / 31 against 31 / 27; 32 of 768 x
+  // 2048, top 4, 700 tokens (318 / 424) 59 / 34 against 51 / 33.
+  const long long wide = (long long)max_tiles * ((N + (EPI == MT_GATE_UP ? 127 : 255)) / (EPI == MT_GATE_UP ? 128 : 256));
+  if (wide < 170)
+    return launch_moe_tiled_as<WM, 2, EPI>(x, ldx, w0, w1, ldw, y, ldy, sorted, tiles, max_tiles, top, N, K, fn, stream);
+  return launch_moe_tiled_as<WM, 4, EPI>(x, ldx, w0, w1, ldw, y, ldy, sorted, tiles, max_tiles, top, N, K, fn, stream);
 }
 
 // x [T, dim] rows gathered by token; wg, wu [E, hidden, ldw], act [n_pairs, lda] in the sorted order.
@@ -634,25 +691,31 @@ extern "C" int fg_moe_gate_up_act(const void* x, int ldx, const void* wg, const 
   if (max_tiles <= 0) return FG_OK;
   if (act_kind != FG_ACT_SILU && !(act_kind == FG_ACT_LIMITED && limit > 0.f)) return FG_ERR_ARG;
   const GatedAct fn = {act_kind, limit, alpha};
-  if (dim <= 0 || hidden <= 0 || top <= 0 || ldx < dim || ldw < dim || lda < hidden) return FG_ERR_ARG;
+  if (dim <= 0 || hidden <= 0 || top <= 0 || ldx < dim || (ldw < dim && !(mfma && ldw == 0)) || lda < hidden) return FG_ERR_ARG;
   if (mfma) {
     if (dtype != FG_BF16 || dim % 8 || ldx % 8 || ldw % 8 || lda % 4) return FG_ERR_ARG;
     if (tile_rows == 128 || tile_rows == 256) {
       if (hidden % 8 || dim < 32) return FG_ERR_ARG;  // (a lane's stand-in load reads the row's first 32 k)
       return tile_rows == 128
-                 ? launch_moe_tiled<2, MT_GATE_UP>(x, ldx, wg, wu, ldw, act, lda, sorted, tiles, max_tiles, top, 2 * hidden, dim, fn, stream)
-                 : launch_moe_tiled<4, MT_GATE_UP>(x, ldx, wg, wu, ldw, act, lda, sorted, tiles, max_tiles, top, 2 * hidden, dim, fn, stream);
+                 ? launch_moe_tiled<1, MT_GATE_UP>(x, ldx, wg, wu, ldw, act, lda, sorted, tiles, max_tiles, top, hidden, dim, fn, stream)
+                 : launch_moe_tiled<2, MT_GATE_UP>(x, ldx, wg, wu, ldw, act, lda, sorted, tiles, max_tiles, top, hidden, dim, fn, stream);
     }
     const long long items = (long long)max_tiles * ((hidden + 15) / 16);
     const unsigned blocks = (unsigned)((items + 3) / 4);
-#define GO(MB)                                                                                                   \
-  moe_gate_up_mfma_kernel<MB><<<blocks, 256, 0, stream>>>((const bf16_t*)x, ldx, (const bf16_t*)wg, (const bf16_t*)wu, \
-                                                          ldw, sorted, tiles, max_tiles, top, dim, hidden, (bf16_t*)act, lda, fn)
+#define GO_AS(MB, PACKED)                                                                                         \
+  moe_gate_up_mfma_kernel<MB, PACKED><<<blocks, 256, 0, stream>>>((const bf16_t*)x, ldx, (const bf16_t*)wg, (const bf16_t*)wu, \
+                                                                  ldw, sorted, tiles, max_tiles, top, dim, hidden, (bf16_t*)act, lda, fn)
+#define GO(MB)                    \
+  do {                            \
+    if (ldw == 0) GO_AS(MB, true); \
+    else GO_AS(MB, false);        \
+  } while (0)
     if (tile_rows == 16) GO(1);
     else if (tile_rows == 32) GO(2);
     else if (tile_rows == 64) GO(4);
     else return FG_ERR_ARG;
 #undef GO
+#undef GO_AS
     return fg_launch_status();
   }
   if (tile_rows != 16 || max_tiles > 2147483647 / 4) return FG_ERR_ARG;
@@ -682,24 +745,30 @@ extern "C" int fg_moe_down(const void* act, int lda, const void* wd, int ldw, co
                            int max_tiles, int tile_rows, int dim, int hidden, float* y, int dtype, int mfma,
                            hipStream_t stream) {
   if (max_tiles <= 0) return FG_OK;
-  if (dim <= 0 || hidden <= 0 || lda < hidden || ldw < hidden) return FG_ERR_ARG;
+  if (dim <= 0 || hidden <= 0 || lda < hidden || (ldw < hidden && !(mfma && ldw == 0))) return FG_ERR_ARG;
   if (mfma) {
     if (dtype != FG_BF16 || hidden % 8 || lda % 8 || ldw % 8) return FG_ERR_ARG;
     if ((tile_rows == 128 || tile_rows == 256) && hidden < 32) return FG_ERR_ARG;
     if (tile_rows == 128 || tile_rows == 256)
       return tile_rows == 128
-                 ? launch_moe_tiled<2, MT_DOWN>(act, lda, wd, nullptr, ldw, y, dim, sorted, tiles, max_tiles, 1, dim, hidden, GatedAct{0, 0.f, 1.f}, stream)
-                 : launch_moe_tiled<4, MT_DOWN>(act, lda, wd, nullptr, ldw, y, dim, sorted, tiles, max_tiles, 1, dim, hidden, GatedAct{0, 0.f, 1.f}, stream);
+                 ? launch_moe_tiled<1, MT_DOWN>(act, lda, wd, nullptr, ldw, y, dim, sorted, tiles, max_tiles, 1, dim, hidden, GatedAct{0, 0.f, 1.f}, stream)
+                 : launch_moe_tiled<2, MT_DOWN>(act, lda, wd, nullptr, ldw, y, dim, sorted, tiles, max_tiles, 1, dim, hidden, GatedAct{0, 0.f, 1.f}, stream);
     const long long items = (long long)max_tiles * ((dim + 15) / 16);
     const unsigned blocks = (unsigned)((items + 3) / 4);
-#define GO(MB)                                                                                                      \
-  moe_down_mfma_kernel<MB><<<blocks, 256, 0, stream>>>((const bf16_t*)act, lda, (const bf16_t*)wd, ldw, sorted, tiles, \
-                                                       max_tiles, dim, hidden, y)
+#define GO_AS(MB, PACKED)                                                                                            \
+  moe_down_mfma_kernel<MB, PACKED><<<blocks, 256, 0, stream>>>((const bf16_t*)act, lda, (const bf16_t*)wd, ldw, sorted, \
+                                                               tiles, max_tiles, dim, hidden, y)
+#define GO(MB)                    \
+  do {                            \
+    if (ldw == 0) GO_AS(MB, true); \
+    else GO_AS(MB, false);        \
+  } while (0)
     if (tile_rows == 16) GO(1);
     else if (tile_rows == 32) GO(2);
     else if (tile_rows == 64) GO(4);
     else return FG_ERR_ARG;
 #undef GO
+#undef GO_AS
     return fg_launch_status();
   }
   if (tile_rows != 16) return FG_ERR_ARG;

@@ -18,7 +18,7 @@ import torch
 
 from ..config import ModelLayout, PartSpec, get_architecture, read_config_json
 from ..kernels.linear import StreamedMatrix, packing, packing_fits
-from ..kernels.ops import (PostNormed, ScaledDelta, ScaledRows, StreamTerms, post_add_rmsnorm, stream_add, stream_terms,
+from ..kernels.ops import (PackedExperts, PostNormed, ScaledDelta, ScaledRows, StreamTerms, post_add_rmsnorm, stream_add, stream_terms,
                            streams_spread)
 from ..parts import LayerStore, PagedNeed, StateNeed, TensorSpec, build_part
 from ..parts.base import MATRIX
@@ -164,7 +164,8 @@ class Model:
         seen, total = set(), 0
         for p in self.parts.all_parts:
             for v in vars(p).values():
-                held = [v.rows, v.packed.data if v.packed is not None else None] if isinstance(v, StreamedMatrix) else [v]
+                held = [v.rows, v.packed.data if v.packed is not None else None] if isinstance(v, StreamedMatrix) else (
+                    [v.data] if isinstance(v, PackedExperts) else [v])
                 for t in held:
                     if isinstance(t, torch.Tensor) and t.data_ptr() not in seen:
                         seen.add(t.data_ptr())

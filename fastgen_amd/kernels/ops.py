@@ -1256,9 +1256,54 @@ def moe_sort(choice: torch.Tensor, n_experts: int, tile_rows: int, n_identity: i
     return sorted_, tiles
 
 
-def _moe_mfma_ok(x: torch.Tensor, *weights: torch.Tensor) -> bool:
+@dataclass
+class PackedExperts:
+    """The experts' bfloat16 matrices ``[E, n, k]``, each in the order of :class:`PackedWeight`: ``data [E,
+    ceil(n / 16), ceil(k / 32), 64, 8]``.  Every kernel that takes a bfloat16 expert reads this order, so it is
+    the only copy that a model keeps."""
+
+    data: torch.Tensor
+    n: int
+    k: int
+
+    @property
+    def shape(self):
+        return torch.Size((self.data.shape[0], self.n, self.k))
+
+    @property
+    def dtype(self) -> torch.dtype:
+        return self.data.dtype
+
+
+def pack_experts(w: torch.Tensor) -> PackedExperts:
+    """``w [E, n, k]`` (bfloat16) as :class:`PackedExperts`: a copy, on the device of ``w``."""
+    _need(w.dim() == 3 and w.dtype == torch.bfloat16, "pack_experts takes bfloat16 matrices [E, n, k]")
+    E, n, k = w.shape
+    nb, ks = -(-n // 16), -(-k // 32)
+    if (nb * 16, ks * 32) != (n, k):
+        padded = w.new_zeros((E, nb * 16, ks * 32))
+        padded[:, :n, :k] = w
+        w = padded
+    # [E, nb, r, ks, g, 8] -> [E, nb, ks, g, r, 8]
+    data = w.reshape(E, nb, 16, ks, 4, 8).permute(0, 1, 3, 4, 2, 5).contiguous().view(E, nb, ks, 64, 8)
+    return PackedExperts(data, n, k)
+
+
+def _moe_mfma_ok(x: torch.Tensor, *weights) -> bool:
     return (x.dtype == torch.bfloat16 and x.shape[1] % 8 == 0 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
-            and all(w.shape[2] % 8 == 0 and w.data_ptr() % 16 == 0 for w in weights))
+            and all(isinstance(w, PackedExperts) or (w.shape[2] % 8 == 0 and w.data_ptr() % 16 == 0) for w in weights))
+
+
+def _experts_args(w, what: str):
+    """C arguments (pointer, ldw) for the experts' matrices, contiguous ``[E, n, k]`` or :class:`PackedExperts` (ldw = 0)."""
+    if isinstance(w, PackedExperts):
+        _gpu(w.data)
+        _need(w.data.is_contiguous() and w.data.data_ptr() % 16 == 0
+              and w.data.shape[1:] == (-(-w.n // 16), -(-w.k // 32), 64, 8), f"{what}: the packed experts do not fit their sizes")
+        return _ptr(w.data), 0
+    _gpu(w)
+    _need(w.dim() == 3 and w.is_contiguous(), f"{what}: the experts' matrices must be contiguous [E, n, k]")
+    return _ptr(w), w.shape[2]
 
 
 def moe_gate_up(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, sorted_: torch.Tensor, tiles: torch.Tensor,
@@ -1266,20 +1311,22 @@ def moe_gate_up(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, sorte
     """``silu(x_t W_gate[e]^T) * (x_t W_up[e]^T)`` for every pair, in the sorted order: ``[T * top, hidden]``.
     With ``limit`` > 0 the activation is the limited one: ``g = min(gate, limit)``, ``u = clamp(up, -limit, limit)``,
     ``g * sigmoid(alpha * g) * (u + 1)``.
-    ``w_gate``, ``w_up``: ``[E, hidden, dim]`` of ``x``'s dtype.  bfloat16 with sizes in multiples of 8
-    runs on the matrix cores; everything else the fp32-FMA kernel (tiles of 16 rows only)."""
-    _gpu(x, w_gate, w_up, sorted_, tiles)
-    _need(x.dim() == 2 and x.stride(1) == 1 and w_gate.dim() == 3 and w_gate.shape == w_up.shape
-          and w_gate.shape[2] == x.shape[1] and w_gate.is_contiguous() and w_up.is_contiguous()
-          and w_gate.dtype == x.dtype == w_up.dtype, "x [T, dim], w_gate and w_up contiguous [E, hidden, dim] of x's dtype")
+    ``w_gate``, ``w_up``: ``[E, hidden, dim]`` of ``x``'s dtype, or both :class:`PackedExperts`.  bfloat16 with sizes in
+    multiples of 8 runs on the matrix cores; everything else the fp32-FMA kernel (tiles of 16 rows only)."""
+    _gpu(x, sorted_, tiles)
+    (gate, ldw), (up, ldu) = _experts_args(w_gate, "moe_gate_up"), _experts_args(w_up, "moe_gate_up")
+    _need(x.dim() == 2 and x.stride(1) == 1 and w_gate.shape == w_up.shape and w_gate.shape[2] == x.shape[1]
+          and w_gate.dtype == x.dtype == w_up.dtype and ldw == ldu,
+          "x [T, dim], w_gate and w_up [E, hidden, dim] of x's dtype, stored alike")
     _i32(sorted_, "sorted", x.shape[0] * top)
     _i32(tiles, "tiles")
     _need(tiles.dim() == 2 and tiles.shape[1] == 4 and tiles.data_ptr() % 16 == 0, "tiles must be [n, 4], 16-byte aligned")
     hidden, dim = w_gate.shape[1], w_gate.shape[2]
     mfma = _moe_mfma_ok(x, w_gate) and hidden % 8 == 0
     _need(tile_rows in MOE_TILE_ROWS and (mfma or tile_rows == 16), "tile_rows does not fit the kernel")
+    _need(mfma or ldw, "moe_gate_up: packed experts need x and sizes in multiples of 8, 16-byte aligned")
     act = torch.empty((sorted_.numel(), hidden), dtype=x.dtype, device=x.device)
-    st = _lib.load("moe").fg_moe_gate_up_act(_ptr(x), x.stride(0), _ptr(w_gate), _ptr(w_up), dim, _ptr(sorted_), _ptr(tiles),
+    st = _lib.load("moe").fg_moe_gate_up_act(_ptr(x), x.stride(0), gate, up, ldw, _ptr(sorted_), _ptr(tiles),
                                              tiles.shape[0], tile_rows, top, dim, hidden, _ptr(act), hidden, _code(x),
                                              int(mfma), ACT_LIMITED if limit > 0 else 0, ctypes.c_float(limit),
                                              ctypes.c_float(alpha), _stream(x))
@@ -1290,19 +1337,20 @@ def moe_gate_up(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, sorte
 def moe_down(act: torch.Tensor, w_down: torch.Tensor, sorted_: torch.Tensor, tiles: torch.Tensor,
              tile_rows: int) -> torch.Tensor:
     """``act_p W_down[e]^T`` for every pair as fp32 ``[T * top, dim]``, row = pair (not the sorted order).
-    ``w_down``: ``[E, dim, hidden]`` of ``act``'s dtype."""
-    _gpu(act, w_down, sorted_, tiles)
-    _need(act.dim() == 2 and act.is_contiguous() and w_down.dim() == 3 and w_down.is_contiguous()
-          and w_down.shape[2] == act.shape[1] and w_down.dtype == act.dtype,
-          "act contiguous [pairs, hidden], w_down contiguous [E, dim, hidden] of act's dtype")
+    ``w_down``: ``[E, dim, hidden]`` of ``act``'s dtype, or :class:`PackedExperts`."""
+    _gpu(act, sorted_, tiles)
+    down, ldw = _experts_args(w_down, "moe_down")
+    _need(act.dim() == 2 and act.is_contiguous() and w_down.shape[2] == act.shape[1] and w_down.dtype == act.dtype,
+          "act contiguous [pairs, hidden], w_down [E, dim, hidden] of act's dtype")
     _i32(sorted_, "sorted", act.shape[0])
     _i32(tiles, "tiles")
     _need(tiles.dim() == 2 and tiles.shape[1] == 4 and tiles.data_ptr() % 16 == 0, "tiles must be [n, 4], 16-byte aligned")
     dim, hidden = w_down.shape[1], w_down.shape[2]
     mfma = _moe_mfma_ok(act, w_down)
     _need(tile_rows in MOE_TILE_ROWS and (mfma or tile_rows == 16), "tile_rows does not fit the kernel")
+    _need(mfma or ldw, "moe_down: packed experts need act in multiples of 8, 16-byte aligned")
     y = torch.empty((act.shape[0], dim), dtype=torch.float32, device=act.device)
-    st = _lib.load("moe").fg_moe_down(_ptr(act), hidden, _ptr(w_down), hidden, _ptr(sorted_), _ptr(tiles), tiles.shape[0],
+    st = _lib.load("moe").fg_moe_down(_ptr(act), hidden, down, ldw, _ptr(sorted_), _ptr(tiles), tiles.shape[0],
                                       tile_rows, dim, hidden, _ptr(y), _code(act), int(mfma), _stream(act))
     _check(st, "moe_down")
     return y

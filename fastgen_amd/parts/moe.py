@@ -86,9 +86,10 @@ class MoE(FeedForward):
             raise ValueError(f"{self.prefix}: a gate of the shared expert needs a shared expert")
         self.router: Optional[torch.Tensor] = None
         self.bias: Optional[torch.Tensor] = None
-        self.w_gate: Optional[torch.Tensor] = None  # [E, hidden (padded to 8), dim]
-        self.w_up: Optional[torch.Tensor] = None
-        self.w_down: Optional[torch.Tensor] = None  # [E, dim, hidden (padded to 8)]
+        # [E, hidden (padded to 8), dim], a tensor or ops.PackedExperts
+        self.w_gate: Any = None
+        self.w_up: Any = None
+        self.w_down: Any = None  # [E, dim, hidden (padded to 8)]
 
     def _expert(self, e: int, which: str) -> str:
         names = self.spec.options.get("names", {})
@@ -132,25 +133,25 @@ class MoE(FeedForward):
             gate = torch.cat([gate, gate.new_zeros(self.n_experts, pad, self.dim)], dim=1)
             up = torch.cat([up, up.new_zeros(self.n_experts, pad, self.dim)], dim=1)
             down = torch.cat([down, down.new_zeros(self.n_experts, self.dim, pad)], dim=2)
-        self.w_gate = place(gate, MATRIX, dtype, device)
-        self.w_up = place(up, MATRIX, dtype, device)
-        self.w_down = place(down, MATRIX, dtype, device)
+        # the matrix-core kernels' order, where they take the sizes: then nothing reads the rows
+        packs = dtype == torch.bfloat16 and self.dim % 8 == 0
+        stored = lambda w: ops.pack_experts(place(w, MATRIX, dtype, device)) if packs else place(w, MATRIX, dtype, device)
+        self.w_gate, self.w_up, self.w_down = stored(gate), stored(up), stored(down)
 
     def tile_rows(self, n_rows: int) -> int:
-        """Rows of one expert a tile holds: 16 for few rows (decode: an expert's matrices are read once for
-        its rows), more where the experts get so many rows each that their matrices would otherwise be
-        read many times over; from about a hundred rows an expert the tiles that go through LDS (the
-        matrix-core kernels only)."""
+        """Rows of one expert a tile holds: 16 for few rows (decode: an expert's matrices are read once for its
+        rows), 32 and 128 where the experts get so many rows each that their matrices would otherwise be read many
+        times over; from 128 on the rows of x go through LDS (the matrix-core kernels only).  Measured (us, gate_up
+        + down, 32 experts of 768 x 2048, top 4; tiles of 16 / 32 / 64 / 128 rows): 12 rows an expert 72 / 74 / 84 / -,
+        19: 95 / 81 / 91 / -, 25: 112 / 88 / 94 / 68, 50: 150 / 128 / 130 / 73, 237 (tiles of 256 rows 165): - / - /
+        434 / 153; 16 experts of 704 x 1024, top 2: 19: 37 / 28 / 31 / -, 25: 40 / 34 / 34 / 36, 50: 54 / 47 / 44 / 39."""
         if self.w_gate.dtype != torch.bfloat16 or self.dim % 8:
             return 16
         per_expert = n_rows * self.top / self.n_scored
         lds_ok = min(self.dim, self.w_down.shape[2]) >= 32  # the tiles through LDS load k in steps of 32
-        # a tile is computed whole whatever it holds, and every expert's last tile is half empty on average:
-        # the largest tiles only where an expert has several of them
-        for rows, least in ((256, 768), (128, 96), (64, 48), (32, 24)):
-            if per_expert >= least and (rows < 128 or lds_ok):
-                return rows
-        return 16
+        if per_expert >= 24 and lds_ok:
+            return 128
+        return 32 if per_expert >= 14 else 16
 
     def forward(self, x: torch.Tensor, plus: Optional[torch.Tensor] = None) -> torch.Tensor:
         """fp32 ``[1, T, dim]``: the experts' weighted sum (plus ``plus``, rows that go to the

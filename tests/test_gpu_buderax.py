@@ -297,3 +297,40 @@ def test_command_lines(cases, tmp_path):
     chat = subprocess.run([sys.executable, str(root / "bin" / "fgchat"), str(folder), "--prompt-ids", "1,2,3", "--max-tokens",
                            "5", "--temperature", "0"], capture_output=True, text=True, timeout=600)
     assert chat.returncode == 0, chat.stderr[-2000:]
+
+
+@pytest.mark.parametrize("E,top,T,D,F", [(3, 2, 40, 40, 24), (5, 1, 700, 2048, 136), (4, 3, 300, 104, 520), (32, 4, 257, 64, 32)])
+@pytest.mark.parametrize("tile_rows", [16, 32, 64, 128, 256])
+def test_packed_experts_give_the_rows_bits(E, top, T, D, F, tile_rows):
+    """The routed products from packed experts and from matrices stored row by row, for every tile: the same bits whatever
+    the storage and the tile (k in steps of 32, ascending), at sizes that end inside a block of 16 rows, a step of 32 k
+    and a wave's columns; and the products themselves, against fp32 with one rounding of the activation to bfloat16."""
+    from fastgen_amd.kernels import ops
+
+    torch.manual_seed(T)
+    x = torch.randn(T, D, device="cuda").bfloat16()
+    wg, wu = ((torch.randn(E, F, D, device="cuda") / D ** 0.5).bfloat16() for _ in range(2))
+    wd = (torch.randn(E, D, F, device="cuda") / F ** 0.5).bfloat16()
+    choice = torch.stack([torch.randperm(E, device="cuda")[:top] for _ in range(T)]).int()
+    if F < 32 and tile_rows >= 128:
+        pytest.skip("tiles through LDS take sizes from 32 on")
+    sorted_, tiles = ops.moe_sort(choice, E, tile_rows)
+    act = ops.moe_gate_up(x, wg, wu, sorted_, tiles, top, tile_rows)
+    y = ops.moe_down(act, wd, sorted_, tiles, tile_rows)
+    packed_act = ops.moe_gate_up(x, ops.pack_experts(wg), ops.pack_experts(wu), sorted_, tiles, top, tile_rows)
+    assert torch.equal(packed_act, act)
+    assert torch.equal(ops.moe_down(act, ops.pack_experts(wd), sorted_, tiles, tile_rows), y)
+    small, small_tiles = ops.moe_sort(choice, E, 16)
+    small_act = ops.moe_gate_up(x, wg, wu, small, small_tiles, top, 16)
+    assert torch.equal(ops.moe_down(small_act, wd, small, small_tiles, 16), y)
+    pair = sorted_.long()
+    expert, rows = choice.reshape(-1)[pair].long(), x[pair // top].float()
+    # a value at a time: the matrices of all pairs would not be small
+    gate, up = torch.empty(2, T * top, F, device="cuda").unbind(0)
+    want = torch.empty(T * top, D, device="cuda")
+    for e in range(E):
+        at = expert == e
+        gate[at], up[at] = rows[at] @ wg[e].float().T, rows[at] @ wu[e].float().T
+        want[pair[at]] = act[at].float() @ wd[e].float().T
+    torch.testing.assert_close(act.float(), torch.nn.functional.silu(gate) * up, rtol=2 ** -7, atol=1e-4)
+    torch.testing.assert_close(y, want, rtol=1e-4, atol=1e-4)
