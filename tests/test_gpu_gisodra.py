@@ -61,6 +61,31 @@ def test_post_add_rmsnorm_gelu_and_softcap_kernels(dtype, T, D, S):
     torch.testing.assert_close(ops.softcap(x.clone().to(DEV), 9.0).cpu(), twins.softcap(x.clone(), 9.0), rtol=1e-5, atol=1e-5)
 
 
+@pytest.mark.parametrize("D", [8, 2040, 2048, 2056, 4096, 4104, 8192, 8200])
+@pytest.mark.parametrize("how", ["delta", "sums", "nothing"])
+def test_post_add_rmsnorm_at_the_edges_of_its_rows(D, how):
+    """Rows around the sizes that a thread's shares of 8 elements end at, once from memory that is 16-byte aligned and
+    once from memory that is not (the kernel that goes element by element): both give the twin's result."""
+    from fastgen_amd.kernels import ops, twins
+
+    torch.manual_seed(D)
+    dtype = torch.bfloat16
+    odd = lambda t: torch.cat([t.new_zeros(1), t.reshape(-1)])[1:].view(t.shape)
+    h, wp, w = torch.randn(3, D), torch.randn(D).to(dtype), torch.randn(D).to(dtype)
+    delta = {"delta": torch.randn(3, D).to(dtype), "sums": torch.randn(5, 3, D), "nothing": None}[how]
+    rows = torch.tensor([2, 0], dtype=torch.int32)
+    for gathered in (None, rows):
+        n = 3 if gathered is None else 2
+        hc, oc = h.clone(), torch.empty(n, D, dtype=dtype)
+        twins.post_add_rmsnorm(hc, delta, wp, 1e-5, w, 1e-6, oc, gathered)
+        for place in (lambda t: t, odd):
+            hg, og = h.clone().to(DEV), torch.empty(n, D, dtype=dtype, device=DEV)
+            ops.post_add_rmsnorm(hg, None if delta is None else delta.to(DEV), place(wp.to(DEV)), 1e-5, w.to(DEV), 1e-6, og,
+                                 None if gathered is None else gathered.to(DEV))
+            _close(hg, hc, torch.float32, "post_add_rmsnorm h")
+            _close(og, oc, dtype, "post_add_rmsnorm")
+
+
 @pytest.mark.parametrize("M,N,K", [(3, 64, 64), (16, 96, 128), (40, 176, 72), (100, 128, 256), (300, 256, 128)])
 def test_products_with_the_gelu_epilogue(M, N, K):
     """Every kernel that can take a gate/up product applies the tanh form of GELU where it stores."""
