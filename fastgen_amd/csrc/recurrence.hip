@@ -178,6 +178,9 @@ __global__ __launch_bounds__(FG_WAVE) void decay_scan_kernel(const ScanArgs a) {
 
 // out[t, c] = sigmoid(z[t, c] + bias[c])^(1/tau) for c < width, as exp(log sigmoid(.) / tau) with
 // log sigmoid(x) = min(x, 0) - log1p(exp(-|x|)); fp32.
+// LOG: its logarithm to the base 2, at least DC_LEAST.
+#define DC_LEAST (-60.f)
+template <bool LOG>
 __global__ __launch_bounds__(256) void decay_from_logits_kernel(const float* __restrict__ z, int z_stride,
                                                                 const float* __restrict__ bias, float inv_tau,
                                                                 float* __restrict__ out, int width) {
@@ -185,17 +188,26 @@ __global__ __launch_bounds__(256) void decay_from_logits_kernel(const float* __r
   const int c = blockIdx.x * 256 + threadIdx.x;
   if (c >= width) return;
   const float x = z[t * z_stride + c] + (bias ? bias[c] : 0.f);
-  out[t * width + c] = expf((fminf(x, 0.f) - log1pf(expf(-fabsf(x)))) * inv_tau);
+  const float l = (fminf(x, 0.f) - log1pf(expf(-fabsf(x)))) * inv_tau;
+  if constexpr (LOG) {
+    const float l2 = l * 1.44269504088896340736f;
+    out[t * width + c] = l2 < DC_LEAST ? DC_LEAST : l2;  // (not fmaxf: a NaN stays one)
+  } else {
+    out[t * width + c] = expf(l);
+  }
 }
 
 extern "C" int fg_decay_from_logits(const float* z, int z_stride, const float* bias, float inv_tau, float* out,
-                                    int n_rows, int width, hipStream_t stream) {
+                                    int n_rows, int width, int log2_of_it, hipStream_t stream) {
   if (n_rows <= 0) return FG_OK;
   if (width <= 0 || z_stride < width || !(inv_tau > 0.f) || !z || !out) return FG_ERR_ARG;
   for (int r0 = 0; r0 < n_rows; r0 += 65535) {
     const int nr = n_rows - r0 < 65535 ? n_rows - r0 : 65535;
-    decay_from_logits_kernel<<<dim3((width + 255) / 256, nr), 256, 0, stream>>>(
-        z + (size_t)r0 * z_stride, z_stride, bias, inv_tau, out + (size_t)r0 * width, width);
+    const dim3 grid((width + 255) / 256, nr);
+    const float* from = z + (size_t)r0 * z_stride;
+    float* to = out + (size_t)r0 * width;
+    if (log2_of_it) decay_from_logits_kernel<true><<<grid, 256, 0, stream>>>(from, z_stride, bias, inv_tau, to, width);
+    else decay_from_logits_kernel<false><<<grid, 256, 0, stream>>>(from, z_stride, bias, inv_tau, to, width);
   }
   return fg_launch_status();
 }
@@ -230,11 +242,23 @@ __global__ __launch_bounds__(256) void decay_chunk_states_kernel(float* __restri
   const size_t row = i / e;  // (head, key channel)
   float* S_mem = state + (size_t)slot_ids[b] * per + i;
   float S = *S_mem;
-  for (int c = seq_chunk[b]; c < seq_chunk[b + 1]; ++c) {
-    float* at = chunks + (size_t)c * per + i;
-    const float add = *at;
-    *at = S;
-    S = prod[(size_t)c * H * d + row] * S + add;
+  constexpr int AHEAD = 8;  // chunks whose loads are in flight together
+  const int c_end = seq_chunk[b + 1];
+  for (int c = seq_chunk[b]; c < c_end; c += AHEAD) {
+    float add[AHEAD], keep[AHEAD];
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j) {
+      const size_t cc = min(c + j, c_end - 1);
+      add[j] = chunks[cc * per + i];
+      keep[j] = prod[cc * H * d + row];
+    }
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j) {
+      if (c + j < c_end) {  // uniform
+        chunks[(size_t)(c + j) * per + i] = S;
+        S = keep[j] * S + add[j];
+      }
+    }
   }
   *S_mem = S;
 }
@@ -257,6 +281,347 @@ extern "C" int fg_decay_chunk_states(float* chunks, const float* prod, float* st
     return FG_ERR_ARG;
   decay_chunk_states_kernel<<<dim3((unsigned)((per + 255) / 256), n_seqs), 256, 0, stream>>>(chunks, prod, state, slot_ids,
                                                                                              seq_chunk, H, d, e);
+  return fg_launch_status();
+}
+
+// ------------------------------------------- long prompts, 64 tokens at a time as matrix products
+// The same in matrix products, for head sizes in multiples of 16 up to 128.  Chunks of 64 tokens, in blocks of 16; l the
+// decays' logarithms to the base 2, L_t their sum over a block's tokens up to t (its own included), E_b over block b's:
+//   states   C = sum_s (k_s 2^(what follows s in the chunk)) v_s^T, prod = 2^(E_0 + .. + E_3)    (a chunk's own part)
+//   fg_decay_chunk_states
+//   outputs  o_t = (q_t 2^(E of the blocks before + L_t))^T S0 + sum_s M[t, s] v_s;  for s in an earlier block
+//            M = (q_t 2^(L_t)) . (k_s 2^(E_b - L_s + E of the blocks between)), in t's own block
+//            M = sum_r q_tr k_sr 2^(L_tr - L_sr), element by element.
+// No exponent is positive, so nothing overflows whatever the decays are, and sums over 16 tokens alone are
+// subtracted, so a difference keeps its digits (a decay under 2^-60 counts as that).  Products on
+// v_mfma_f32_16x16x4_f32; an operand's k index runs as 16 j + 4 (lane / 16) + i over the four products i of a block j.
+// All of it in fp32.  2000 tokens, 16 heads of 128 x 128: 24 + 14 + 56 us behind 17 us for the decays, against
+// 137 + 137 (the scans of chunks of 128 token by token, twice) + 32 (the products of the decays) + 9 + 16 us.  A call of its
+// own, in and out: 142 against 383 us; 8000 tokens 427 against 1329, 256 tokens 101 against 186, 4 times 300 tokens 130
+// against 346.  Error against 64 bits 2.5e-7 of the values, before 2.9e-7.  The outputs' kernel is bound by what a
+// workgroup does alone: M's own blocks element by element (a 2^x for each element of 16 x 16 x d), two workgroups a CU.
+#define DC 64
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+struct ChunkArgs {
+  const void* qkv; int row_stride, q_col, k_col, v_col;
+  const float* logs;       // [T, H * d]
+  float q_scale;
+  const int* chunk_start;  // [n_chunks + 1]
+  float* states;           // [n_chunks, H, d, e]: C, then S0
+  float* prod;             // [n_chunks, H * d]
+  float* out;              // [T, H * e]
+  int H, d, e;
+};
+
+__device__ __forceinline__ f32x4 dc_mfma4(const f32x4 x, const f32x4 y, f32x4 acc) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[i], y[i], acc, 0, 0, 0);
+  return acc;
+}
+template <class T> __device__ __forceinline__ f32x4 dc_load4(const T* p);
+template <> __device__ __forceinline__ f32x4 dc_load4<float>(const float* p) { return *(const f32x4*)p; }
+template <> __device__ __forceinline__ f32x4 dc_load4<bf16_t>(const bf16_t* p) {
+  const uint2 w = *(const uint2*)p;
+  return f32x4{__uint_as_float(w.x << 16), __uint_as_float(w.x & 0xffff0000u), __uint_as_float(w.y << 16),
+               __uint_as_float(w.y & 0xffff0000u)};
+}
+__device__ __forceinline__ f32x4 dc_exp2(const f32x4 x) {
+  return f32x4{__builtin_amdgcn_exp2f(x[0]), __builtin_amdgcn_exp2f(x[1]), __builtin_amdgcn_exp2f(x[2]),
+               __builtin_amdgcn_exp2f(x[3])};
+}
+
+// L of the chunk's blocks into LDS, tokens behind the chunk's last with a decay of one.  256 threads; ends in a barrier.
+template <int NDM>
+__device__ __forceinline__ void dc_sums(const ChunkArgs& a, int t0, int n, int h, float (*L_s)[16 * NDM + 4]) {
+  for (int i = threadIdx.x; i < 4 * a.d; i += 256) {
+    const int b = i / a.d, r = i % a.d;
+    float l[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) l[u] = a.logs[(size_t)(t0 + min(16 * b + u, n - 1)) * a.H * a.d + h * a.d + r];
+    float sum = 0.f;
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+      sum += 16 * b + u < n ? l[u] : 0.f;
+      L_s[16 * b + u][r] = sum;
+    }
+  }
+  __syncthreads();
+}
+
+// grid (n_chunks, H, ceil(e / 128)), 4 waves; wave w the state's rows of the blocks w, w + 4 of 16 key channels.
+template <class TA, int NDM>
+__global__ __launch_bounds__(256) void decay_chunk_sums_kernel(const ChunkArgs a) {
+  constexpr int NT = (NDM + 3) / 4;
+  __shared__ float L_s[DC][16 * NDM + 4];
+  __shared__ float V_s[DC][128 + 4];
+  const int lane = threadIdx.x % FG_WAVE, g = lane >> 4, r16 = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / FG_WAVE);  // (so that what depends on it is a scalar branch)
+  const int c = blockIdx.x, h = blockIdx.y, c0 = blockIdx.z * 128, nd = a.d / 16, cols = min(128, a.e - c0);
+  const int t0 = a.chunk_start[c], n = a.chunk_start[c + 1] - t0;
+  const TA* rows = (const TA*)a.qkv;
+  float kt[NT][4][4];
+#pragma unroll
+  for (int m = 0; m < NT; ++m)
+    if (wave + 4 * m < nd) {  // uniform in the wave
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          kt[m][j][i] = to_f<TA>(rows[(size_t)(t0 + min(16 * j + 4 * g + i, n - 1)) * a.row_stride + a.k_col + h * a.d + 16 * (wave + 4 * m) + r16]);
+    }
+  {
+    const int col = threadIdx.x % 128, t_own = threadIdx.x / 128;  // two tokens at a time
+    const TA* vp = rows + a.v_col + h * a.e + c0 + min(col, cols - 1);
+#pragma unroll
+    for (int u0 = 0; u0 < DC / 2; u0 += 16) {
+      float v[16];
+#pragma unroll
+      for (int u = 0; u < 16; ++u) v[u] = to_f<TA>(vp[(size_t)(t0 + min(2 * (u0 + u) + t_own, n - 1)) * a.row_stride]);
+#pragma unroll
+      for (int u = 0; u < 16; ++u) V_s[2 * (u0 + u) + t_own][col] = v[u];
+    }
+  }
+  dc_sums<NDM>(a, t0, n, h, L_s);
+  if (blockIdx.z == 0)
+    for (int r = threadIdx.x; r < a.d; r += 256)
+      a.prod[((size_t)c * a.H + h) * a.d + r] = __builtin_amdgcn_exp2f((L_s[15][r] + L_s[31][r]) + (L_s[47][r] + L_s[63][r]));
+#pragma unroll
+  for (int m = 0; m < NT; ++m)
+    if (wave + 4 * m < nd) {
+      const int r = 16 * (wave + 4 * m) + r16;
+      const float after[4] = {(L_s[31][r] + L_s[47][r]) + L_s[63][r], L_s[47][r] + L_s[63][r], L_s[63][r], 0.f};
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int s = 16 * j + 4 * g + i;
+          kt[m][j][i] = s < n ? kt[m][j][i] * __builtin_amdgcn_exp2f((L_s[16 * j + 15][r] - L_s[s][r]) + after[j]) : 0.f;
+        }
+    }
+  float* out = a.states + ((size_t)c * a.H + h) * a.d * a.e + c0;
+  for (int cb = 0; 16 * cb < cols; ++cb) {
+    f32x4 v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[j][i] = V_s[16 * j + 4 * g + i][16 * cb + r16];
+#pragma unroll
+    for (int m = 0; m < NT; ++m) {
+      const int ti = wave + 4 * m;
+      if (ti < nd) {
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc = dc_mfma4(f32x4{kt[m][j][0], kt[m][j][1], kt[m][j][2], kt[m][j][3]}, v[j], acc);
+        if (16 * cb + r16 < cols) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) out[(size_t)(16 * ti + 4 * g + i) * a.e + 16 * cb + r16] = acc[i];
+        }
+      }
+    }
+  }
+}
+
+// grid (n_chunks, H, ceil(e / 128)), 4 waves: M by rows (wave w the tokens of block w), then each wave blocks of 16 value
+// channels for all 64 tokens.  M takes the keys' place in LDS and the queries with their decays that of the sums.
+template <class TA, int NDM>
+__global__ __launch_bounds__(256) void decay_chunk_outputs_kernel(const ChunkArgs a) {
+  constexpr int D = 16 * NDM, LD = D + 4, LQ = D + 16 / (int)sizeof(TA);
+  constexpr int KEYS = DC * LQ * (int)sizeof(TA), MS = DC * (DC + 4) * 4;
+  __shared__ __attribute__((aligned(16))) float L_s[DC][LD];
+  __shared__ __attribute__((aligned(16))) TA Q_s[DC][LQ];
+  __shared__ __attribute__((aligned(16))) char km[KEYS > MS ? KEYS : MS];
+  TA(*K_s)[LQ] = (TA(*)[LQ])km;
+  float(*M_s)[DC + 4] = (float(*)[DC + 4])km;
+  const int lane = threadIdx.x % FG_WAVE, g = lane >> 4, r16 = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / FG_WAVE);  // (so that what depends on it is a scalar branch)
+  const int c = blockIdx.x, h = blockIdx.y, c0 = blockIdx.z * 128, d = a.d, nd = d / 16, cols = min(128, a.e - c0);
+  const int t0 = a.chunk_start[c], n = a.chunk_start[c + 1] - t0;
+  const TA* rows = (const TA*)a.qkv;
+  struct __attribute__((aligned(4 * sizeof(TA)))) Four { TA v[4]; };
+  const bool vec = a.row_stride % 4 == 0 && a.q_col % 4 == 0 && a.k_col % 4 == 0 && (uintptr_t)rows % sizeof(Four) == 0;
+  for (int i = threadIdx.x; i < DC * (d / 4); i += 256) {  // four elements at a time; tokens behind the last: zeros
+    const int t = i / (d / 4), r = i % (d / 4) * 4;
+    const TA* row = rows + (size_t)(t0 + min(t, n - 1)) * a.row_stride + h * d + r;
+    Four q4, k4;
+    if (vec) {  // uniform
+      q4 = *(const Four*)(row + a.q_col);
+      k4 = *(const Four*)(row + a.k_col);
+    } else {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) q4.v[u] = row[a.q_col + u], k4.v[u] = row[a.k_col + u];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      q4.v[u] = t < n ? q4.v[u] : from_f<TA>(0.f);
+      k4.v[u] = t < n ? k4.v[u] : from_f<TA>(0.f);
+    }
+    *(Four*)&Q_s[t][r] = q4;
+    *(Four*)&K_s[t][r] = k4;
+  }
+  dc_sums<NDM>(a, t0, n, h, L_s);
+
+  f32x4 m[4];  // M of this wave's 16 tokens (4 g + i) with the keys 16 b + r16 of block b
+#pragma unroll
+  for (int b = 0; b < 4; ++b) m[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int j = 0; j < NDM; ++j) {
+    if (j < nd) {  // uniform
+      const int r = 16 * j + 4 * g, t = 16 * wave + r16;
+      const f32x4 qv = dc_load4<TA>(&Q_s[t][r]) * dc_exp2(*(const f32x4*)&L_s[t][r]);
+      f32x4 between = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int b = 2; b >= 0; --b) {
+        if (b < wave) {  // uniform in the wave
+          const f32x4 end = *(const f32x4*)&L_s[16 * b + 15][r];
+          const int s = 16 * b + r16;
+          const f32x4 kv = dc_load4<TA>(&K_s[s][r]) * dc_exp2((end - *(const f32x4*)&L_s[s][r]) + between);
+          m[b] = dc_mfma4(qv, kv, m[b]);
+          between += end;
+        }
+      }
+    }
+  }
+  {  // its own block
+    const int s = 16 * wave + r16;
+    f32x4 own = {0.f, 0.f, 0.f, 0.f};
+    for (int r = 0; r < d; r += 4) {
+      const f32x4 kv = dc_load4<TA>(&K_s[s][r]), ls = *(const f32x4*)&L_s[s][r];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int t = 16 * wave + 4 * g + i;
+        // (a key behind the token: its exponent would be positive, its weight is struck below)
+        const f32x4 x = dc_load4<TA>(&Q_s[t][r]) * kv * dc_exp2(s <= t ? *(const f32x4*)&L_s[t][r] - ls : f32x4{0.f, 0.f, 0.f, 0.f});
+        own[i] += (x[0] + x[1]) + (x[2] + x[3]);
+      }
+    }
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+      if (b == wave) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) m[b][i] = r16 <= 4 * g + i ? own[i] : 0.f;
+      }
+  }
+  constexpr int PER = DC * D / 4 / 256;  // fours of the decayed queries a thread makes
+  f32x4 qt[PER];
+#pragma unroll
+  for (int u = 0; u < PER; ++u) {
+    const int i = threadIdx.x + 256 * u, t = i / (D / 4), r = i % (D / 4) * 4;
+    if (r < d) {
+      f32x4 l = *(const f32x4*)&L_s[t][r];
+      for (int b = t / 16 - 1; b >= 0; --b) l += *(const f32x4*)&L_s[16 * b + 15][r];
+      qt[u] = dc_load4<TA>(&Q_s[t][r]) * dc_exp2(l);
+    }
+  }
+  __syncthreads();  // keys and sums have been read
+#pragma unroll
+  for (int b = 0; b < 4; ++b)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      // in a vector register by decree: where some of these sums lay in accumulator registers the compiler (of ROCm 7.2)
+      // began to pair two stores, gave up over the two kinds of register, and left an offset divided by four behind
+      float x = m[b][i];
+      asm volatile("" : "+v"(x));
+      M_s[16 * wave + 4 * g + i][16 * b + r16] = x;
+    }
+#pragma unroll
+  for (int u = 0; u < PER; ++u) {
+    const int i = threadIdx.x + 256 * u, t = i / (D / 4), r = i % (D / 4) * 4;
+    if (r < d) *(f32x4*)&L_s[t][r] = qt[u];
+  }
+  __syncthreads();
+  const float* S0 = a.states + ((size_t)c * a.H + h) * d * a.e + c0;
+  for (int cb = wave; 16 * cb < cols; cb += 4) {
+    const int col = min(16 * cb + r16, cols - 1);
+    f32x4 acc[4], v[4];
+#pragma unroll
+    for (int tb = 0; tb < 4; ++tb) acc[tb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const TA* vp = rows + a.v_col + h * a.e + c0 + col;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[j][i] = to_f<TA>(vp[(size_t)(t0 + min(16 * j + 4 * g + i, n - 1)) * a.row_stride]);
+    f32x4 s4[NDM];
+#pragma unroll
+    for (int j = 0; j < NDM; ++j)
+      if (j < nd) {
+        const float* sp = S0 + (size_t)(16 * j + 4 * g) * a.e + col;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s4[j][i] = sp[(size_t)i * a.e];
+      }
+#pragma unroll
+    for (int j = 0; j < NDM; ++j)
+      if (j < nd) {
+#pragma unroll
+        for (int tb = 0; tb < 4; ++tb) acc[tb] = dc_mfma4(*(const f32x4*)&L_s[16 * tb + r16][16 * j + 4 * g], s4[j], acc[tb]);
+      }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      // an infinity or NaN among the values is added by hand: a weight of zero would not keep it from earlier tokens
+      f32x4 whole;
+      bool odd = false;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const bool fine = fabsf(v[j][i]) <= 3.402823466e38f;
+        whole[i] = fine ? v[j][i] : 0.f;
+        odd |= !fine;
+      }
+#pragma unroll
+      for (int tb = j; tb < 4; ++tb) acc[tb] = dc_mfma4(*(const f32x4*)&M_s[16 * tb + r16][16 * j + 4 * g], whole, acc[tb]);
+      if (__any(odd)) {
+        for (int u = 0; u < 16; ++u) {
+          const int s = 16 * j + u;
+          const float mine = u % 4 == 0 ? v[j][0] : u % 4 == 1 ? v[j][1] : u % 4 == 2 ? v[j][2] : v[j][3];
+          const float x = __shfl(mine, 16 * (u / 4) + r16, FG_WAVE);  // token s's value in this lane's column
+          if (fabsf(x) <= 3.402823466e38f) continue;
+#pragma unroll
+          for (int tb = 0; tb < 4; ++tb)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              if (16 * tb + 4 * g + i >= s) acc[tb][i] += M_s[16 * tb + 4 * g + i][s] * x;
+        }
+      }
+    }
+    if (16 * cb + r16 < cols) {
+#pragma unroll
+      for (int tb = 0; tb < 4; ++tb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int t = 16 * tb + 4 * g + i;
+          if (t < n) a.out[(size_t)(t0 + t) * ((size_t)a.H * a.e) + h * a.e + c0 + col] = acc[tb][i] * a.q_scale;
+        }
+    }
+  }
+}
+
+extern "C" int fg_decay_chunk_tokens() { return DC; }
+
+// Chunk by chunk as above: d a multiple of 16 up to 128.  `state` [n_slots, H, d, e] is read and left at slot_ids.
+extern "C" int fg_decay_chunk_scan(const ChunkArgs* args, const int* slot_ids, const int* seq_chunk, float* state,
+                                   int n_chunks, int n_seqs, int act_dtype, hipStream_t stream) {
+  if (n_seqs <= 0 || n_chunks <= 0) return FG_OK;
+  const ChunkArgs& a = *args;
+  if (a.H <= 0 || a.H > 65535 || a.d <= 0 || a.d % 16 || a.d > 128 || a.e <= 0 || (a.e + 127) / 128 > 65535 || !a.qkv ||
+      !a.logs || !a.chunk_start || !a.states || !a.prod || !a.out)
+    return FG_ERR_ARG;
+  const dim3 grid(n_chunks, a.H, (a.e + 127) / 128);
+#define GO(TA, NDM)                                                                                                     \
+  do {                                                                                                                  \
+    decay_chunk_sums_kernel<TA, NDM><<<grid, 256, 0, stream>>>(a);                                                      \
+    const int st = fg_decay_chunk_states(a.states, a.prod, state, slot_ids, seq_chunk, n_seqs, a.H, a.d, a.e, stream);  \
+    if (st != FG_OK) return st;                                                                                         \
+    decay_chunk_outputs_kernel<TA, NDM><<<grid, 256, 0, stream>>>(a);                                                   \
+  } while (0)
+  if (act_dtype == FG_F32) {
+    if (a.d <= 64) GO(float, 4);
+    else GO(float, 8);
+  } else if (act_dtype == FG_BF16) {
+    if (a.d <= 64) GO(bf16_t, 4);
+    else GO(bf16_t, 8);
+  } else {
+    return FG_ERR_ARG;
+  }
+#undef GO
   return fg_launch_status();
 }
 

@@ -1787,6 +1787,13 @@ class _ScanArgs(ctypes.Structure):
                 ("write_state", ctypes.c_int)]
 
 
+class _DecayChunkArgs(ctypes.Structure):
+    _fields_ = [("qkv", ctypes.c_void_p), ("row_stride", ctypes.c_int), ("q_col", ctypes.c_int), ("k_col", ctypes.c_int),
+                ("v_col", ctypes.c_int), ("logs", ctypes.c_void_p), ("q_scale", ctypes.c_float), ("chunk_start", ctypes.c_void_p),
+                ("states", ctypes.c_void_p), ("prod", ctypes.c_void_p), ("out", ctypes.c_void_p),
+                ("H", ctypes.c_int), ("d", ctypes.c_int), ("e", ctypes.c_int)]
+
+
 SCAN_CHUNK = 128  # tokens of a chunk where long runs of tokens are scanned chunk by chunk, side by side
 SCAN_CHUNKED_FROM = 256  # the shortest run of tokens of one sequence for which a step is scanned so
 
@@ -1803,9 +1810,10 @@ def decay_scan(qkv: torch.Tensor, q_col: int, k_col: int, v_col: int, z: torch.T
     ``q_start[b] .. q_start[b+1]-1``; ``out`` is fp32 ``[T, H*e]``.
 
     ``q_start_host``: ``q_start`` on the host.  With it, a step in which a sequence brings ``SCAN_CHUNKED_FROM``
-    tokens or more is scanned in chunks of ``SCAN_CHUNK`` tokens side by side (every chunk from a zero state,
-    then the states that the chunks start from, then every chunk from its start); the result differs from
-    the token-by-token scan's by rounding (a chunk's start state is summed in another order)."""
+    tokens or more is scanned in chunks side by side (every chunk from a zero state, then the states that the
+    chunks start from, then every chunk from its start): 64 tokens at a time as fp32 matrix products where ``d``
+    is a multiple of 16 up to 128, else ``SCAN_CHUNK`` tokens one by one.  The result differs from the
+    token-by-token scan's by rounding (sums are taken in another order)."""
     _gpu(qkv, z, z_bias, state, slot_ids, q_start, out)
     _need(state.dtype == torch.float32 and state.dim() == 4 and state.is_contiguous(), "state must be contiguous float32 [n_slots, H, d, e]")
     _, H, d, e = state.shape
@@ -1819,34 +1827,44 @@ def decay_scan(qkv: torch.Tensor, q_col: int, k_col: int, v_col: int, z: torch.T
     _i32(slot_ids, "slot_ids", n_seqs)
     _i32(q_start, "q_start", n_seqs + 1)
     _need(d <= 512 and tau > 0, "at most 512 key channels a head; tau positive")
-    a = _ScanArgs()
-    a.qkv, a.row_stride, a.q_col, a.k_col, a.v_col = qkv.data_ptr(), qkv.stride(0), q_col, k_col, v_col
-    # the decays of every token at once (exponentials and logarithms stay out of the chain of tokens)
     lib = _lib.load("recurrence")
+    lens = np.diff(np.asarray(q_start_host[: n_seqs + 1])) if q_start_host is not None else None
+    chunked = lens is not None and len(lens) and int(lens.max()) >= SCAN_CHUNKED_FROM and not torch.cuda.is_current_stream_capturing()
+    products = chunked and d % 16 == 0 and d <= 128
+    # the decays of every token at once (exponentials and logarithms stay out of the chain of tokens), or their logarithms
     decay = torch.empty((T, H * d), dtype=torch.float32, device=z.device)
     st = lib.fg_decay_from_logits(_ptr(z), z.stride(0), _ptr(z_bias), ctypes.c_float(1.0 / tau), _ptr(decay), T, H * d,
-                                  _stream(z))
+                                  int(products), _stream(z))
     _check(st, "decay_from_logits")
+    a = _ScanArgs()
+    a.qkv, a.row_stride, a.q_col, a.k_col, a.v_col = qkv.data_ptr(), qkv.stride(0), q_col, k_col, v_col
     a.decay, a.decay_stride, a.q_scale, a.state = decay.data_ptr(), decay.stride(0), q_scale, state.data_ptr()
     a.slot_ids, a.q_start, a.out, a.H, a.d, a.e = slot_ids.data_ptr(), q_start.data_ptr(), out.data_ptr(), H, d, e
     a.write_out = a.write_state = 1
-    lens = np.diff(np.asarray(q_start_host[: n_seqs + 1])) if q_start_host is not None else None
-    if lens is None or not len(lens) or int(lens.max()) < SCAN_CHUNKED_FROM or torch.cuda.is_current_stream_capturing():
+    if not chunked:
         st = lib.fg_decay_scan(ctypes.byref(a), int(n_seqs), _code(qkv), _stream(qkv))
         _check(st, "decay_scan")
         return out
     # chunk by chunk: the chunks' first tokens, and which chunks each sequence has
+    size = lib.fg_decay_chunk_tokens() if products else SCAN_CHUNK
     starts, seq_chunk = [], [0]
     for b in range(n_seqs):
-        starts.extend(range(int(q_start_host[b]), int(q_start_host[b + 1]), SCAN_CHUNK))
+        starts.extend(range(int(q_start_host[b]), int(q_start_host[b + 1]), size))
         seq_chunk.append(len(starts))
     n_chunks = len(starts)
-    _need(n_chunks <= 65535 and n_seqs <= 65535, "too many chunks or sequences in one step")
+    _need((products or n_chunks <= 65535) and n_seqs <= 65535, "too many chunks or sequences in one step")
     plan = upload(np.asarray(starts + [int(q_start_host[n_seqs])] + seq_chunk + list(range(n_chunks)), dtype=np.int32),
                   torch.int32, qkv.device)
     chunk_start, seq_chunk_d, chunk_ids = plan[: n_chunks + 1], plan[n_chunks + 1 : n_chunks + n_seqs + 2], plan[n_chunks + n_seqs + 2 :]
-    chunks = torch.zeros((n_chunks, H, d, e), dtype=torch.float32, device=qkv.device)
     prod = torch.empty((n_chunks, H * d), dtype=torch.float32, device=qkv.device)
+    if products:
+        chunks = torch.empty((n_chunks, H, d, e), dtype=torch.float32, device=qkv.device)
+        c = _DecayChunkArgs(qkv.data_ptr(), qkv.stride(0), q_col, k_col, v_col, decay.data_ptr(), q_scale, chunk_start.data_ptr(),
+                            chunks.data_ptr(), prod.data_ptr(), out.data_ptr(), H, d, e)
+        _check(lib.fg_decay_chunk_scan(ctypes.byref(c), _ptr(slot_ids), _ptr(seq_chunk_d), _ptr(state), n_chunks, int(n_seqs),
+                                       _code(qkv), _stream(qkv)), "decay_scan (chunks as products)")
+        return out
+    chunks = torch.zeros((n_chunks, H, d, e), dtype=torch.float32, device=qkv.device)
     _check(lib.fg_decay_chunk_product(_ptr(decay), decay.stride(0), _ptr(chunk_start), _ptr(prod), n_chunks, H * d,
                                       _stream(qkv)), "decay_chunk_product")
     a.state, a.slot_ids, a.q_start = chunks.data_ptr(), chunk_ids.data_ptr(), chunk_start.data_ptr()
@@ -2025,7 +2043,7 @@ def selective_scan(u: torch.Tensor, dt: torch.Tensor, dt_bias: Optional[torch.Te
         starts.extend(range(int(q_start_host[b]), int(q_start_host[b + 1]), SELECTIVE_CHUNK))
         seq_chunk.append(len(starts))
     n_chunks = len(starts)
-    _need(n_chunks <= 65535 and n_seqs <= 65535, "too many chunks or sequences in one step")
+    _need((products or n_chunks <= 65535) and n_seqs <= 65535, "too many chunks or sequences in one step")
     plan = upload(np.asarray(starts + [int(q_start_host[n_seqs])] + seq_chunk + list(range(n_chunks)), dtype=np.int32),
                   torch.int32, u.device)
     chunk_start, seq_chunk_d, chunk_ids = plan[: n_chunks + 1], plan[n_chunks + 1 : n_chunks + n_seqs + 2], plan[n_chunks + n_seqs + 2 :]

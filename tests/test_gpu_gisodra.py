@@ -211,6 +211,47 @@ def test_decay_scan_and_head_norm_gate_kernels(dtype, H, d, e, lens):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,d,e,lens", [(2, 16, 8, [256, 1, 300]), (1, 128, 130, [65, 700]), (3, 48, 40, [257, 64, 15, 65]),
+                                        (2, 112, 256, [319])])
+@pytest.mark.parametrize("least", [-3.0, -400.0])
+def test_decay_scan_as_products_of_chunks(dtype, H, d, e, lens, least):
+    """Long runs as matrix products of 64 tokens: chunks and blocks of 16 that a run ends inside, columns beyond the
+    queries' alignment, decays from near one down to 2^-60 and below (which the products count as 2^-60), within the
+    tolerance of the scan token by token; and a value that is no number reaches no earlier token and no other sequence."""
+    from fastgen_amd.kernels import ops, twins
+
+    g = torch.Generator().manual_seed(d + e)
+    T, B, q_col = sum(lens), len(lens), 3 if d == 48 else 0
+    k_col, v_col = q_col + H * d, q_col + 2 * H * d
+    rows = torch.randn(T, v_col + H * e + 5, generator=g).to(dtype)
+    z = torch.randn(T, H * d, generator=g) + 4
+    z[torch.rand(T, H * d, generator=g) < 0.02] = least
+    state = torch.randn(B + 1, H, d, e, generator=g)
+    slots = torch.randperm(B + 1, generator=g)[:B].to(torch.int32)
+    q_start = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32)
+    oc, sc = torch.empty(T, H * e), state.clone()
+    twins.decay_scan(rows, q_col, k_col, v_col, z, None, 4.0, d ** -0.5, sc, slots, q_start, B, oc)
+
+    def run(rows):
+        og, sg = torch.empty(T, H * e, device=DEV), state.to(DEV)
+        ops.decay_scan(rows.to(DEV), q_col, k_col, v_col, z.to(DEV), None, 4.0, d ** -0.5, sg, slots.to(DEV),
+                       q_start.to(DEV), B, og, q_start_host=q_start.numpy())
+        return og.cpu(), sg.cpu()
+
+    og, sg = run(rows)
+    torch.testing.assert_close(og, oc, rtol=1e-4, atol=1e-4)
+    torch.testing.assert_close(sg, sc, rtol=1e-4, atol=1e-4)
+    at = int(q_start[1]) - 9  # near the end of the first sequence, inside a block
+    bad = rows.clone()
+    bad[at, v_col] = float("nan")
+    ob, sb = run(bad)
+    first = torch.arange(T) < at
+    later = torch.arange(T) >= int(q_start[1])
+    assert torch.equal(ob[first | later], og[first | later]) and torch.isnan(ob[at, 0])
+    assert torch.equal(sb[slots[1:].long()], sg[slots[1:].long()]) and torch.isnan(sb[slots[0], 0, 0, 0])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("H,G,hd,P,window,n", [(4, 2, 16, 16, 9, 70), (5, 1, 80, 64, 110, 300), (2, 2, 48, 32, 33, 150),
                                                (12, 1, 176, 64, 56, 200), (3, 3, 24, 8, 0, 50)])
 def test_attention_kernels_with_a_sink_and_a_window_edge_that_decides(dtype, H, G, hd, P, window, n):
