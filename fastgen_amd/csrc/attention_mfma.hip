@@ -168,6 +168,10 @@ __device__ __forceinline__ void attend_tile(int k0, const ItemRows (&me)[RB], co
       for (int rb = 0; rb < RB; ++rb)
         s[rb][kb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k, qop[rb][ks], s[rb][kb], 0, 0, 0);
     }
+    // At the largest head sizes the operands of all four blocks, read ahead, cost the tile kernel its last registers, and
+    // what it then keeps in memory is read back behind the next tile's loads: 151 us against 104 without, for 2000
+    // tokens of 16 heads on one kv head of 256 (2048 tokens on 8 kv heads: 147 / 98).  Up to 192 there is room (73 / 73).
+    if (!PREFETCH && HD > 192) __builtin_amdgcn_sched_barrier(0);
   }
   if (PREFETCH) {
 #pragma unroll
@@ -846,13 +850,21 @@ constexpr bool TILE_PAIR_OK = HD <= 128;
 constexpr int TILE_ROWS = TILE_PAIR_OK ? 128 : 64;   // query rows of an item of the first form that this head size has
 constexpr int TILE_ROWS_SMALL = 64;                // of the second form
 
-template <bool PERM, bool TILE_PAIR>
+// PAGES: what the page size is a multiple of, as far as the copies into LDS care.  PAGES_TILE (64, the engine's own): a
+// tile is part of one page, in the order LDS wants it, whatever of it the item's rows see: one lookup, and at the ends
+// of the key range a mask on the values.  The others look up the page of every 8 keys (PAGES_CHUNK) or 4 keys
+// (PAGES_ANY) at the ends of the range, one after the other.  That chain cost 1 to 3 us an item, of which most have
+// such an end: 64 / 300 / 2000 tokens at head size 128 with it 7.2 / 12.0 / 49.2 us, without 6.1 / 10.8 / 48.3.
+enum { PAGES_ANY = 0, PAGES_CHUNK = 1, PAGES_TILE = 2 };  // multiples of 8, 32, 64
+
+template <int PAGES, bool TILE_PAIR>
 __global__ __launch_bounds__(TILE_PAIR ? 512 : 256, TILE_PAIR ? 1 : 2) void attn_tile_kernel(
     const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, int out_stride,
     const bf16_t* __restrict__ k_pages, const bf16_t* __restrict__ v_pages,
     const int* __restrict__ block_table, int bt_stride, const int* __restrict__ items, int n_heads, int n_kv,
     int page_size, int page_shift, float scale, int window, const float* __restrict__ sinks,
     const float* __restrict__ dist) {
+  constexpr bool PERM = PAGES >= PAGES_CHUNK, WHOLE = PAGES == PAGES_TILE;
   constexpr int TILE_RB = TILE_PAIR ? 2 : 1;  // row blocks a wave holds
   constexpr int TILE_THREADS = TILE_PAIR ? 512 : 256;
   constexpr int NT = TILE_THREADS;
@@ -925,14 +937,13 @@ __global__ __launch_bounds__(TILE_PAIR ? 512 : 256, TILE_PAIR ? 1 : 2) void attn
   // A tile's chunks on their way through registers.  Loads are never conditional within a tile:
   // addresses are clamped into the item's key range, value slots outside it are masked, keys
   // outside it give scores that the select discards.
-  auto fetch = [&](int k0, bf16x8(&kr)[KN], bf16x8(&vr)[VN]) {
-    if (PERM && (page_size & 63) == 0 && k0 >= first_min && k0 + TILE - 1 <= pos_last) {
-      // The whole tile lies in one page and inside the key range: K's four 16-key blocks are 64*HD
-      // contiguous elements in the order LDS wants them, V's eight key chunks are a contiguous run
-      // per block of 16 head dims.  No masks, one page lookup.
+  auto fetch = [&](int k0, int page, bf16x8(&kr)[KN], bf16x8(&vr)[VN]) {
+    if (WHOLE) {
+      // The whole tile lies in one page: K's four 16-key blocks are 64*HD contiguous elements in the
+      // order LDS wants them, V's eight key chunks are a contiguous run per block of 16 head dims.
       const int kin = pager.in_page(k0);
-      const bf16_t* base_k = k_pages + ((size_t)pager.page_of(k0) * n_kv + kvh) * head_elems + (size_t)kin * HD;
-      const bf16_t* base_v = v_pages + ((size_t)pager.page_of(k0) * n_kv + kvh) * head_elems + (size_t)(kin >> 3) * 128;
+      const bf16_t* base_k = k_pages + ((size_t)page * n_kv + kvh) * head_elems + (size_t)kin * HD;
+      const bf16_t* base_v = v_pages + ((size_t)page * n_kv + kvh) * head_elems + (size_t)(kin >> 3) * 128;
       const size_t v_block = (size_t)(page_size >> 3) * 128;  // elements of one block of 16 head dims
 #pragma unroll
       for (int j = 0; j < KN; ++j) {
@@ -943,6 +954,13 @@ __global__ __launch_bounds__(TILE_PAIR ? 512 : 256, TILE_PAIR ? 1 : 2) void attn
       for (int j = 0; j < VN; ++j) {
         const int w = min((int)threadIdx.x + NT * j, VTOT - 1);
         vr[j] = *(const bf16x8*)(base_v + (size_t)(w >> 7) * v_block + (size_t)(w & 127) * 8);
+      }
+      if (k0 < first_min || k0 + TILE - 1 > pos_last) {  // uniform
+#pragma unroll
+        for (int j = 0; j < VN; ++j) {
+          const int kc = (min((int)threadIdx.x + NT * j, VTOT - 1) >> 4) & 7;
+          vr[j] = and_mask(vr[j], slot_mask(k0 + 32 * (kc >> 2) + 4 * (kc & 3), first_min, pos_last));
+        }
       }
       return;
     }
@@ -1022,7 +1040,7 @@ __global__ __launch_bounds__(TILE_PAIR ? 512 : 256, TILE_PAIR ? 1 : 2) void attn
     auto page_ahead = [&](int k0) { return pager.page_of(min(k0, pos_last)); };
     auto bring = [&](int k0, int slot, int page) {
       if (k0 > pos_last) return;  // uniform
-      if (PERM && (page_size & 63) == 0 && k0 >= first_min && k0 + TILE - 1 <= pos_last) {
+      if (WHOLE && k0 >= first_min && k0 + TILE - 1 <= pos_last) {
         const int kin = pager.in_page(k0);
         const bf16_t* base_k = k_pages + ((size_t)page * n_kv + kvh) * head_elems + (size_t)kin * HD;
         const bf16_t* base_v = v_pages + ((size_t)page * n_kv + kvh) * head_elems + (size_t)(kin >> 3) * 128;
@@ -1044,7 +1062,7 @@ __global__ __launch_bounds__(TILE_PAIR ? 512 : 256, TILE_PAIR ? 1 : 2) void attn
                 (__attribute__((address_space(3))) void*)(v_lds[slot] + (size_t)(w - lane) * 8), 16, 0, 0);
         }
       } else {
-        fetch(k0, kreg, vreg);
+        fetch(k0, page, kreg, vreg);
         stash(slot, kreg, vreg);
       }
     };
@@ -1064,12 +1082,16 @@ __global__ __launch_bounds__(TILE_PAIR ? 512 : 256, TILE_PAIR ? 1 : 2) void attn
     }
   } else {
     // one tile at a time: the next tile's chunks fly into registers during this tile's MFMAs
-    fetch(k_first, kreg, vreg);
+    // (the page of a tile is looked up a tile earlier)
+    auto page_ahead = [&](int k0) { return WHOLE ? pager.page_of(min(k0, pos_last)) : 0; };
+    int page = page_ahead(k_first + STEP);
+    fetch(k_first, page_ahead(k_first), kreg, vreg);
     for (int k0 = k_first; k0 <= pos_last; k0 += STEP) {
       __syncthreads();  // the previous tile is no longer read
       stash(0, kreg, vreg);
       __syncthreads();
-      if (k0 + STEP <= pos_last) fetch(k0 + STEP, kreg, vreg);
+      if (k0 + STEP <= pos_last) fetch(k0 + STEP, page, kreg, vreg);
+      page = page_ahead(k0 + 2 * STEP);
       compute(k0, 0);
     }
   }
@@ -1130,17 +1152,21 @@ struct TileArgs {
   const int* block_table; int bt_stride; const int* items; int n_items, n_heads, n_kv, page_size; float scale;
   int window; const float* sinks; const float* dist; hipStream_t stream;
 };
-template <bool PERM, bool PAIR>
-static void launch_tile(const TileArgs& a) {
-  attn_tile_kernel<PERM, PAIR><<<a.n_items * a.n_kv, PAIR ? 512 : 256, 0, a.stream>>>(
+template <int PAGES, bool PAIR>
+static void launch_pages(const TileArgs& a) {
+  attn_tile_kernel<PAGES, PAIR><<<a.n_items * a.n_kv, PAIR ? 512 : 256, 0, a.stream>>>(
       a.q, a.q_stride, a.out, a.out_stride, a.k_pages, a.v_pages, a.block_table, a.bt_stride, a.items, a.n_heads,
       a.n_kv, a.page_size, page_shift_of(a.page_size), a.scale, a.window, a.sinks, a.dist);
 }
+template <bool PAIR>
+static void launch_tile(const TileArgs& a) {
+  if (a.page_size % 64 == 0) launch_pages<PAGES_TILE, PAIR>(a);
+  else if (a.page_size % 32 == 0) launch_pages<PAGES_CHUNK, PAIR>(a);
+  else launch_pages<PAGES_ANY, PAIR>(a);
+}
 // the form with two tiles at a time exists up to head size 128 only (its LDS)
 template <bool EXISTS> struct PairForm {
-  static void go(const TileArgs& a) {
-    if (a.page_size % 32 == 0) launch_tile<true, true>(a); else launch_tile<false, true>(a);
-  }
+  static void go(const TileArgs& a) { launch_tile<true>(a); }
 };
 template <> struct PairForm<false> { static void go(const TileArgs&) {} };
 
@@ -1159,8 +1185,7 @@ extern "C" int fg_attn_tile_sink(const void* q, int q_stride, void* out, int out
   const TileArgs a{(const bf16_t*)q, q_stride, (bf16_t*)out, out_stride, (const bf16_t*)k_pages, (const bf16_t*)v_pages,
                    block_table, bt_stride, items, n_items, n_heads, n_kv, page_size, scale, window, sinks, dist, stream};
   if (TILE_PAIR_OK && item_rows == TILE_ROWS) PairForm<TILE_PAIR_OK>::go(a);
-  else if (page_size % 32 == 0) launch_tile<true, false>(a);
-  else launch_tile<false, false>(a);
+  else launch_tile<false>(a);
   return fg_launch_status();
 }
 

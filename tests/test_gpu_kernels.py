@@ -859,6 +859,22 @@ def test_paged_attention_mfma(ops, H, KV, hd, P, window, cut):
     assert torch.allclose(out.cpu().float(), want, atol=1.5e-2, rtol=2e-2)
 
 
+@pytest.mark.parametrize("P", [64, 96, 128, 192])
+@pytest.mark.parametrize("H,KV,hd", [(4, 1, 256), (3, 3, 208), (2, 1, 192), (8, 2, 128), (5, 5, 16)])
+@pytest.mark.parametrize("window", [0, 37, 64])
+@pytest.mark.parametrize("small_tiles", [False, True])
+def test_paged_attention_mfma_pages_of_whole_tiles(ops, H, KV, hd, P, window, small_tiles):
+    """Pages of which a tile of 64 keys is a part (all but 96 tokens): portions that begin and end inside a tile, at its
+    last key and at its first, with and without earlier keys; what the pages hold beyond the last key is no number.
+    Tolerance: that of the other shapes above (outputs rounded to bfloat16)."""
+    seqs = [(0, 70), (0, 64), (1, 63), (63, 66), (64, 64), (130, 61), (0, 129), (200, 121)]
+    case = _paged_case(torch.bfloat16, seqs, H, KV, hd, P, seed=31)
+    out, _, n_big = _run_mfma(ops, case, seqs, H, KV, window, "coarse", small_tiles=small_tiles)
+    assert n_big
+    assert torch.isfinite(out).all()
+    assert torch.allclose(out.cpu().float(), _plain_rows(case, seqs, window or None), atol=1.5e-2, rtol=2e-2)
+
+
 def test_paged_attention_mfma_two_streams(ops, monkeypatch):
     """Prompt portions beside decoded tokens: the tile kernel runs on a second stream beside the
     split kernel.  The result is there when the caller's stream goes on (work queued behind the
