@@ -2043,7 +2043,7 @@ def selective_scan(u: torch.Tensor, dt: torch.Tensor, dt_bias: Optional[torch.Te
         starts.extend(range(int(q_start_host[b]), int(q_start_host[b + 1]), SELECTIVE_CHUNK))
         seq_chunk.append(len(starts))
     n_chunks = len(starts)
-    _need((products or n_chunks <= 65535) and n_seqs <= 65535, "too many chunks or sequences in one step")
+    _need(n_chunks <= 65535 and n_seqs <= 65535, "too many chunks or sequences in one step")
     plan = upload(np.asarray(starts + [int(q_start_host[n_seqs])] + seq_chunk + list(range(n_chunks)), dtype=np.int32),
                   torch.int32, u.device)
     chunk_start, seq_chunk_d, chunk_ids = plan[: n_chunks + 1], plan[n_chunks + 1 : n_chunks + n_seqs + 2], plan[n_chunks + n_seqs + 2 :]
