@@ -178,8 +178,7 @@ __global__ __launch_bounds__(FG_WAVE) void decay_scan_kernel(const ScanArgs a) {
 
 // out[t, c] = sigmoid(z[t, c] + bias[c])^(1/tau) for c < width, as exp(log sigmoid(.) / tau) with
 // log sigmoid(x) = min(x, 0) - log1p(exp(-|x|)); fp32.
-// LOG: its logarithm to the base 2, at least DC_LEAST.
-#define DC_LEAST (-60.f)
+// LOG: its logarithm to the base 2.
 template <bool LOG>
 __global__ __launch_bounds__(256) void decay_from_logits_kernel(const float* __restrict__ z, int z_stride,
                                                                 const float* __restrict__ bias, float inv_tau,
@@ -189,12 +188,7 @@ __global__ __launch_bounds__(256) void decay_from_logits_kernel(const float* __r
   if (c >= width) return;
   const float x = z[t * z_stride + c] + (bias ? bias[c] : 0.f);
   const float l = (fminf(x, 0.f) - log1pf(expf(-fabsf(x)))) * inv_tau;
-  if constexpr (LOG) {
-    const float l2 = l * 1.44269504088896340736f;
-    out[t * width + c] = l2 < DC_LEAST ? DC_LEAST : l2;  // (not fmaxf: a NaN stays one)
-  } else {
-    out[t * width + c] = expf(l);
-  }
+  out[t * width + c] = LOG ? l * 1.44269504088896340736f : expf(l);
 }
 
 extern "C" int fg_decay_from_logits(const float* z, int z_stride, const float* bias, float inv_tau, float* out,
@@ -285,21 +279,27 @@ extern "C" int fg_decay_chunk_states(float* chunks, const float* prod, float* st
 }
 
 // ------------------------------------------- long prompts, 64 tokens at a time as matrix products
-// The same in matrix products, for head sizes in multiples of 16 up to 128.  Chunks of 64 tokens, in blocks of 16; l the
-// decays' logarithms to the base 2, L_t their sum over a block's tokens up to t (its own included), E_b over block b's:
-//   states   C = sum_s (k_s 2^(what follows s in the chunk)) v_s^T, prod = 2^(E_0 + .. + E_3)    (a chunk's own part)
+// The same in matrix products, for head sizes in multiples of 16 up to 128.  Chunks of 64 tokens, in blocks of 16.  With l
+// the decays' logarithms to the base 2, P_t = 2^(the sum of l over t's block up to t, its own included), R_s = 2^(the sum
+// over s's block behind s) and E_b = 2^(the sum over block b):
+//   states   C = sum_s (k_s R_s E of the blocks behind) v_s^T, prod = 2^(the sum over the chunk)    (a chunk's own part)
 //   fg_decay_chunk_states
-//   outputs  o_t = (q_t 2^(E of the blocks before + L_t))^T S0 + sum_s M[t, s] v_s;  for s in an earlier block
-//            M = (q_t 2^(L_t)) . (k_s 2^(E_b - L_s + E of the blocks between)), in t's own block
-//            M = sum_r q_tr k_sr 2^(L_tr - L_sr), element by element.
-// No exponent is positive, so nothing overflows whatever the decays are, and sums over 16 tokens alone are
-// subtracted, so a difference keeps its digits (a decay under 2^-60 counts as that).  Products on
-// v_mfma_f32_16x16x4_f32; an operand's k index runs as 16 j + 4 (lane / 16) + i over the four products i of a block j.
-// All of it in fp32.  2000 tokens, 16 heads of 128 x 128: 24 + 14 + 56 us behind 17 us for the decays, against
-// 137 + 137 (the scans of chunks of 128 token by token, twice) + 32 (the products of the decays) + 9 + 16 us.  A call of its
-// own, in and out: 142 against 383 us; 8000 tokens 427 against 1329, 256 tokens 101 against 186, 4 times 300 tokens 130
-// against 346.  Error against 64 bits 2.5e-7 of the values, before 2.9e-7.  The outputs' kernel is bound by what a
-// workgroup does alone: M's own blocks element by element (a 2^x for each element of 16 x 16 x d), two workgroups a CU.
+//   outputs  o_t = (q_t P_t E of the blocks before)^T S0 + sum_s M[t, s] v_s;  for s in an earlier block
+//            M = (q_t P_t) . (k_s R_s E of the blocks between), in t's own block
+//            M = sum_r q_tr (k_sr a_(s+1)r .. a_tr), the key taken along from token to token.
+// Sums of logarithms are added up only, never subtracted from one another (the difference of two long ones would keep
+// few of its digits), so a weight is as exact as the decays that make it up, however strong other decays beside it are;
+// no exponent is positive, and no decay needs a bound (2^x under 2^-126 is zero).  Products on v_mfma_f32_16x16x4_f32; an
+// operand's k index runs as 16 j + 4 (lane / 16) + i over the four products i of a block j.  All of it in fp32, with at
+// most 32 products in a chain (chains of 128: 1.3 to 1.45 times the error).  Error of the outputs against 64 bits (500
+// tokens of 128 channels), products / token by token: decays near one 1.4 / 1.5e-7, lasting ones 1.8e-7 / 1.5e-6, 5 %
+// of them strong 1.3 / 1.5e-7, half of them 1.1 / 1.05e-7, of every strength 1.04e-7 / 8.9e-8.  (With differences of
+// sums in the place of R and of the own block's products: 1.9e-7, 2.9e-7, 1.1e-6, 2.3 to 8.9e-6, 3.5e-7.)
+// 2000 tokens, 16 heads of 128 x 128: 23 + 14 + 47 us behind 16 us for the decays, against 137 + 137 (the scans of
+// chunks of 128 token by token, twice) + 32 (the products of the decays) + 9 + 16 us.  A call of its own, in and out:
+// 127 against 365 us; 8000 tokens 377 against 1210, 256 tokens 90 against 179, 4 times 300 tokens 118 against 338; float32
+// operands 148 against 359, 483 against 1242, 90 against 177, 139 against 330.  The outputs' kernel is bound by what a
+// workgroup does alone (its stages with a barrier between each), two workgroups a CU.
 #define DC 64
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -326,34 +326,23 @@ template <> __device__ __forceinline__ f32x4 dc_load4<bf16_t>(const bf16_t* p) {
   return f32x4{__uint_as_float(w.x << 16), __uint_as_float(w.x & 0xffff0000u), __uint_as_float(w.y << 16),
                __uint_as_float(w.y & 0xffff0000u)};
 }
-__device__ __forceinline__ f32x4 dc_exp2(const f32x4 x) {
-  return f32x4{__builtin_amdgcn_exp2f(x[0]), __builtin_amdgcn_exp2f(x[1]), __builtin_amdgcn_exp2f(x[2]),
-               __builtin_amdgcn_exp2f(x[3])};
-}
+__device__ __forceinline__ float dc_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
-// L of the chunk's blocks into LDS, tokens behind the chunk's last with a decay of one.  256 threads; ends in a barrier.
-template <int NDM>
-__device__ __forceinline__ void dc_sums(const ChunkArgs& a, int t0, int n, int h, float (*L_s)[16 * NDM + 4]) {
-  for (int i = threadIdx.x; i < 4 * a.d; i += 256) {
-    const int b = i / a.d, r = i % a.d;
-    float l[16];
+// The logarithms of token u of block i / d, channel i % d, for the item i < 4 d; tokens behind the chunk's last: 0.
+__device__ __forceinline__ void dc_logs(const ChunkArgs& a, int t0, int n, int h, int i, float (&l)[16]) {
+  const int b = i / a.d, r = i % a.d;
 #pragma unroll
-    for (int u = 0; u < 16; ++u) l[u] = a.logs[(size_t)(t0 + min(16 * b + u, n - 1)) * a.H * a.d + h * a.d + r];
-    float sum = 0.f;
+  for (int u = 0; u < 16; ++u) l[u] = a.logs[(size_t)(t0 + min(16 * b + u, n - 1)) * a.H * a.d + h * a.d + r];
 #pragma unroll
-    for (int u = 0; u < 16; ++u) {
-      sum += 16 * b + u < n ? l[u] : 0.f;
-      L_s[16 * b + u][r] = sum;
-    }
-  }
-  __syncthreads();
+  for (int u = 0; u < 16; ++u) l[u] = 16 * b + u < n ? l[u] : 0.f;
 }
 
 // grid (n_chunks, H, ceil(e / 128)), 4 waves; wave w the state's rows of the blocks w, w + 4 of 16 key channels.
 template <class TA, int NDM>
 __global__ __launch_bounds__(256) void decay_chunk_sums_kernel(const ChunkArgs a) {
   constexpr int NT = (NDM + 3) / 4;
-  __shared__ float L_s[DC][16 * NDM + 4];
+  __shared__ float R_s[DC][16 * NDM + 4];
+  __shared__ float sum_s[4][16 * NDM];  // of each block's logarithms
   __shared__ float V_s[DC][128 + 4];
   const int lane = threadIdx.x % FG_WAVE, g = lane >> 4, r16 = lane & 15;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / FG_WAVE);  // (so that what depends on it is a scalar branch)
@@ -382,21 +371,33 @@ __global__ __launch_bounds__(256) void decay_chunk_sums_kernel(const ChunkArgs a
       for (int u = 0; u < 16; ++u) V_s[2 * (u0 + u) + t_own][col] = v[u];
     }
   }
-  dc_sums<NDM>(a, t0, n, h, L_s);
+  for (int i = threadIdx.x; i < 4 * a.d; i += 256) {
+    const int b = i / a.d, r = i % a.d;
+    float l[16], behind = 0.f;
+    dc_logs(a, t0, n, h, i, l);
+#pragma unroll
+    for (int u = 15; u >= 0; --u) {
+      R_s[16 * b + u][r] = dc_exp2(behind);
+      behind += l[u];
+    }
+    sum_s[b][r] = behind;
+  }
+  __syncthreads();
   if (blockIdx.z == 0)
     for (int r = threadIdx.x; r < a.d; r += 256)
-      a.prod[((size_t)c * a.H + h) * a.d + r] = __builtin_amdgcn_exp2f((L_s[15][r] + L_s[31][r]) + (L_s[47][r] + L_s[63][r]));
+      a.prod[((size_t)c * a.H + h) * a.d + r] = dc_exp2((sum_s[0][r] + sum_s[1][r]) + (sum_s[2][r] + sum_s[3][r]));
 #pragma unroll
   for (int m = 0; m < NT; ++m)
     if (wave + 4 * m < nd) {
       const int r = 16 * (wave + 4 * m) + r16;
-      const float after[4] = {(L_s[31][r] + L_s[47][r]) + L_s[63][r], L_s[47][r] + L_s[63][r], L_s[63][r], 0.f};
+      const float after[4] = {dc_exp2((sum_s[1][r] + sum_s[2][r]) + sum_s[3][r]), dc_exp2(sum_s[2][r] + sum_s[3][r]),
+                              dc_exp2(sum_s[3][r]), 1.f};
 #pragma unroll
       for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int s = 16 * j + 4 * g + i;
-          kt[m][j][i] = s < n ? kt[m][j][i] * __builtin_amdgcn_exp2f((L_s[16 * j + 15][r] - L_s[s][r]) + after[j]) : 0.f;
+          kt[m][j][i] = s < n ? kt[m][j][i] * (R_s[s][r] * after[j]) : 0.f;
         }
     }
   float* out = a.states + ((size_t)c * a.H + h) * a.d * a.e + c0;
@@ -410,12 +411,14 @@ __global__ __launch_bounds__(256) void decay_chunk_sums_kernel(const ChunkArgs a
     for (int m = 0; m < NT; ++m) {
       const int ti = wave + 4 * m;
       if (ti < nd) {
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        f32x4 acc[2];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc = dc_mfma4(f32x4{kt[m][j][0], kt[m][j][1], kt[m][j][2], kt[m][j][3]}, v[j], acc);
+        for (int j = 0; j < 4; ++j)
+          acc[j / 2] = dc_mfma4(f32x4{kt[m][j][0], kt[m][j][1], kt[m][j][2], kt[m][j][3]}, v[j],
+                                j % 2 ? acc[j / 2] : f32x4{0.f, 0.f, 0.f, 0.f});
         if (16 * cb + r16 < cols) {
 #pragma unroll
-          for (int i = 0; i < 4; ++i) out[(size_t)(16 * ti + 4 * g + i) * a.e + 16 * cb + r16] = acc[i];
+          for (int i = 0; i < 4; ++i) out[(size_t)(16 * ti + 4 * g + i) * a.e + 16 * cb + r16] = acc[0][i] + acc[1][i];
         }
       }
     }
@@ -423,16 +426,20 @@ __global__ __launch_bounds__(256) void decay_chunk_sums_kernel(const ChunkArgs a
 }
 
 // grid (n_chunks, H, ceil(e / 128)), 4 waves: M by rows (wave w the tokens of block w), then each wave blocks of 16 value
-// channels for all 64 tokens.  M takes the keys' place in LDS and the queries with their decays that of the sums.
+// channels for all 64 tokens.  The decays' place in LDS is taken by q P, that by the queries against the state; that of
+// the keys and queries by k R, and that by M.
 template <class TA, int NDM>
-__global__ __launch_bounds__(256) void decay_chunk_outputs_kernel(const ChunkArgs a) {
-  constexpr int D = 16 * NDM, LD = D + 4, LQ = D + 16 / (int)sizeof(TA);
-  constexpr int KEYS = DC * LQ * (int)sizeof(TA), MS = DC * (DC + 4) * 4;
-  __shared__ __attribute__((aligned(16))) float L_s[DC][LD];
-  __shared__ __attribute__((aligned(16))) TA Q_s[DC][LQ];
-  __shared__ __attribute__((aligned(16))) char km[KEYS > MS ? KEYS : MS];
-  TA(*K_s)[LQ] = (TA(*)[LQ])km;
-  float(*M_s)[DC + 4] = (float(*)[DC + 4])km;
+__global__ __launch_bounds__(256, sizeof(TA) == 2 ? 2 : 1) void decay_chunk_outputs_kernel(const ChunkArgs a) {
+  constexpr int D = 16 * NDM, LD = D + 4, LQ = D + 16 / (int)sizeof(TA), NI = (4 * D + 255) / 256;
+  constexpr int ROWS = DC * LQ * (int)sizeof(TA), KR = DC * LD * 4, MS = DC * (DC + 4) * 4;
+  static_assert(2 * ROWS >= KR && 2 * ROWS >= MS, "k R and M fit where the queries and keys were");
+  __shared__ __attribute__((aligned(16))) float A_s[DC][LD];
+  __shared__ __attribute__((aligned(16))) char qk[2 * ROWS];
+  __shared__ __attribute__((aligned(16))) float E_s[4][D];
+  TA(*Q_s)[LQ] = (TA(*)[LQ])qk;
+  TA(*K_s)[LQ] = (TA(*)[LQ])(qk + ROWS);
+  float(*R_s)[LD] = (float(*)[LD])qk;
+  float(*M_s)[DC + 4] = (float(*)[DC + 4])qk;
   const int lane = threadIdx.x % FG_WAVE, g = lane >> 4, r16 = lane & 15;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / FG_WAVE);  // (so that what depends on it is a scalar branch)
   const int c = blockIdx.x, h = blockIdx.y, c0 = blockIdx.z * 128, d = a.d, nd = d / 16, cols = min(128, a.e - c0);
@@ -459,61 +466,109 @@ __global__ __launch_bounds__(256) void decay_chunk_outputs_kernel(const ChunkArg
     *(Four*)&Q_s[t][r] = q4;
     *(Four*)&K_s[t][r] = k4;
   }
-  dc_sums<NDM>(a, t0, n, h, L_s);
+  float l[NI][16];
+#pragma unroll
+  for (int m = 0; m < NI; ++m) {
+    const int i = threadIdx.x + 256 * m, b = i / d, r = i % d;
+    if (i < 4 * d) {
+      dc_logs(a, t0, n, h, i, l[m]);
+      float sum = 0.f;
+#pragma unroll
+      for (int u = 0; u < 16; ++u) {
+        A_s[16 * b + u][r] = dc_exp2(l[m][u]);
+        sum += l[m][u];
+      }
+      E_s[b][r] = dc_exp2(sum);
+    }
+  }
+  __syncthreads();
 
-  f32x4 m[4];  // M of this wave's 16 tokens (4 g + i) with the keys 16 b + r16 of block b
+  // M of the wave's own block: a lane takes key r16 along the tokens, for a quarter of the channels
+  f32x4 own;
+  {
+    float sum[16];
 #pragma unroll
-  for (int b = 0; b < 4; ++b) m[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < 16; ++t) sum[t] = 0.f;
+    for (int j = 0; j < nd; ++j) {
+      const int r = 16 * j + 4 * g;
+      const f32x4 kv = dc_load4<TA>(&K_s[16 * wave + r16][r]);
+      f32x4 w = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int j = 0; j < NDM; ++j) {
-    if (j < nd) {  // uniform
-      const int r = 16 * j + 4 * g, t = 16 * wave + r16;
-      const f32x4 qv = dc_load4<TA>(&Q_s[t][r]) * dc_exp2(*(const f32x4*)&L_s[t][r]);
-      f32x4 between = {0.f, 0.f, 0.f, 0.f};
+      for (int t = 0; t < 16; ++t) {
+        const f32x4 at = *(const f32x4*)&A_s[16 * wave + t][r], qv = dc_load4<TA>(&Q_s[16 * wave + t][r]);
 #pragma unroll
-      for (int b = 2; b >= 0; --b) {
-        if (b < wave) {  // uniform in the wave
-          const f32x4 end = *(const f32x4*)&L_s[16 * b + 15][r];
-          const int s = 16 * b + r16;
-          const f32x4 kv = dc_load4<TA>(&K_s[s][r]) * dc_exp2((end - *(const f32x4*)&L_s[s][r]) + between);
-          m[b] = dc_mfma4(qv, kv, m[b]);
-          between += end;
+        for (int i = 0; i < 4; ++i) w[i] = t == r16 ? kv[i] : w[i] * at[i];
+        sum[t] += (qv[0] * w[0] + qv[1] * w[1]) + (qv[2] * w[2] + qv[3] * w[3]);
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < 16; ++t) {
+      sum[t] += __shfl_xor(sum[t], 16, FG_WAVE);
+      sum[t] += __shfl_xor(sum[t], 32, FG_WAVE);
+    }
+    // this lane's four tokens 4 g + i (a token before the key sees nothing of it, whatever its decays are)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float x = g == 0 ? sum[i] : g == 1 ? sum[4 + i] : g == 2 ? sum[8 + i] : sum[12 + i];
+      own[i] = r16 <= 4 * g + i ? x : 0.f;
+    }
+  }
+  float qp[NI][16], kr[NI][16];
+#pragma unroll
+  for (int m = 0; m < NI; ++m) {
+    const int i = threadIdx.x + 256 * m, b = i / d, r = i % d;
+    if (i < 4 * d) {
+      float sum = 0.f;
+#pragma unroll
+      for (int u = 0; u < 16; ++u) {
+        sum += l[m][u];
+        qp[m][u] = to_f<TA>(Q_s[16 * b + u][r]) * dc_exp2(sum);
+      }
+      sum = 0.f;
+#pragma unroll
+      for (int u = 15; u >= 0; --u) {
+        kr[m][u] = to_f<TA>(K_s[16 * b + u][r]) * dc_exp2(sum);
+        sum += l[m][u];
+      }
+    }
+  }
+  __syncthreads();  // decays, queries and keys have been read
+#pragma unroll
+  for (int m = 0; m < NI; ++m) {
+    const int i = threadIdx.x + 256 * m, b = i / d, r = i % d;
+    if (i < 4 * d) {
+#pragma unroll
+      for (int u = 0; u < 16; ++u) {
+        A_s[16 * b + u][r] = qp[m][u];
+        R_s[16 * b + u][r] = kr[m][u];
+      }
+    }
+  }
+  __syncthreads();
+  f32x4 m[4], part[4];  // M of this wave's 16 tokens (4 g + i) with the keys 16 b + r16 of block b; 32 channels of it
+#pragma unroll
+  for (int b = 0; b < 4; ++b) m[b] = part[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 2
+  for (int j = 0; j < nd; ++j) {
+    const int r = 16 * j + 4 * g;
+    const f32x4 qv = *(const f32x4*)&A_s[16 * wave + r16][r];
+    f32x4 between = {1.f, 1.f, 1.f, 1.f};
+#pragma unroll
+    for (int b = 2; b >= 0; --b) {
+      if (b < wave) {  // uniform in the wave
+        part[b] = dc_mfma4(qv, *(const f32x4*)&R_s[16 * b + r16][r] * between, part[b]);
+        between *= *(const f32x4*)&E_s[b][r];
+        if (j % 2 || j == nd - 1) {
+          m[b] += part[b];
+          part[b] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
       }
     }
   }
-  {  // its own block
-    const int s = 16 * wave + r16;
-    f32x4 own = {0.f, 0.f, 0.f, 0.f};
-    for (int r = 0; r < d; r += 4) {
-      const f32x4 kv = dc_load4<TA>(&K_s[s][r]), ls = *(const f32x4*)&L_s[s][r];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int t = 16 * wave + 4 * g + i;
-        // (a key behind the token: its exponent would be positive, its weight is struck below)
-        const f32x4 x = dc_load4<TA>(&Q_s[t][r]) * kv * dc_exp2(s <= t ? *(const f32x4*)&L_s[t][r] - ls : f32x4{0.f, 0.f, 0.f, 0.f});
-        own[i] += (x[0] + x[1]) + (x[2] + x[3]);
-      }
-    }
-#pragma unroll
-    for (int b = 0; b < 4; ++b)
-      if (b == wave) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) m[b][i] = r16 <= 4 * g + i ? own[i] : 0.f;
-      }
-  }
-  constexpr int PER = DC * D / 4 / 256;  // fours of the decayed queries a thread makes
-  f32x4 qt[PER];
-#pragma unroll
-  for (int u = 0; u < PER; ++u) {
-    const int i = threadIdx.x + 256 * u, t = i / (D / 4), r = i % (D / 4) * 4;
-    if (r < d) {
-      f32x4 l = *(const f32x4*)&L_s[t][r];
-      for (int b = t / 16 - 1; b >= 0; --b) l += *(const f32x4*)&L_s[16 * b + 15][r];
-      qt[u] = dc_load4<TA>(&Q_s[t][r]) * dc_exp2(l);
-    }
-  }
-  __syncthreads();  // keys and sums have been read
+  for (int b = 0; b < 4; ++b)
+    if (b == wave) m[b] = own;
+  __syncthreads();  // q P and k R have been read
 #pragma unroll
   for (int b = 0; b < 4; ++b)
 #pragma unroll
@@ -525,17 +580,22 @@ __global__ __launch_bounds__(256) void decay_chunk_outputs_kernel(const ChunkArg
       M_s[16 * wave + 4 * g + i][16 * b + r16] = x;
     }
 #pragma unroll
-  for (int u = 0; u < PER; ++u) {
-    const int i = threadIdx.x + 256 * u, t = i / (D / 4), r = i % (D / 4) * 4;
-    if (r < d) *(f32x4*)&L_s[t][r] = qt[u];
+  for (int m = 0; m < NI; ++m) {
+    const int i = threadIdx.x + 256 * m, b = i / d, r = i % d;
+    if (i < 4 * d && b > 0) {
+      float before = 1.f;
+      for (int b2 = 0; b2 < b; ++b2) before *= E_s[b2][r];
+#pragma unroll
+      for (int u = 0; u < 16; ++u) A_s[16 * b + u][r] *= before;
+    }
   }
   __syncthreads();
   const float* S0 = a.states + ((size_t)c * a.H + h) * d * a.e + c0;
   for (int cb = wave; 16 * cb < cols; cb += 4) {
     const int col = min(16 * cb + r16, cols - 1);
-    f32x4 acc[4], v[4];
+    f32x4 acc[4], part[4], v[4];
 #pragma unroll
-    for (int tb = 0; tb < 4; ++tb) acc[tb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int tb = 0; tb < 4; ++tb) acc[tb] = part[tb] = f32x4{0.f, 0.f, 0.f, 0.f};
     const TA* vp = rows + a.v_col + h * a.e + c0 + col;
 #pragma unroll
     for (int j = 0; j < 4; ++j)
@@ -553,7 +613,13 @@ __global__ __launch_bounds__(256) void decay_chunk_outputs_kernel(const ChunkArg
     for (int j = 0; j < NDM; ++j)
       if (j < nd) {
 #pragma unroll
-        for (int tb = 0; tb < 4; ++tb) acc[tb] = dc_mfma4(*(const f32x4*)&L_s[16 * tb + r16][16 * j + 4 * g], s4[j], acc[tb]);
+        for (int tb = 0; tb < 4; ++tb) {
+          part[tb] = dc_mfma4(*(const f32x4*)&A_s[16 * tb + r16][16 * j + 4 * g], s4[j], part[tb]);
+          if (j % 2 || j == nd - 1) {
+            acc[tb] += part[tb];
+            part[tb] = f32x4{0.f, 0.f, 0.f, 0.f};
+          }
+        }
       }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -567,7 +633,13 @@ __global__ __launch_bounds__(256) void decay_chunk_outputs_kernel(const ChunkArg
         odd |= !fine;
       }
 #pragma unroll
-      for (int tb = j; tb < 4; ++tb) acc[tb] = dc_mfma4(*(const f32x4*)&M_s[16 * tb + r16][16 * j + 4 * g], whole, acc[tb]);
+      for (int tb = j; tb < 4; ++tb) {
+        part[tb] = dc_mfma4(*(const f32x4*)&M_s[16 * tb + r16][16 * j + 4 * g], whole, part[tb]);
+        if (j % 2 || j == tb) {
+          acc[tb] += part[tb];
+          part[tb] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+      }
       if (__any(odd)) {
         for (int u = 0; u < 16; ++u) {
           const int s = 16 * j + u;

@@ -216,7 +216,7 @@ def test_decay_scan_and_head_norm_gate_kernels(dtype, H, d, e, lens):
 @pytest.mark.parametrize("least", [-3.0, -400.0])
 def test_decay_scan_as_products_of_chunks(dtype, H, d, e, lens, least):
     """Long runs as matrix products of 64 tokens: chunks and blocks of 16 that a run ends inside, columns beyond the
-    queries' alignment, decays from near one down to 2^-60 and below (which the products count as 2^-60), within the
+    queries' alignment, decays from near one down to nothing (2^-144 at tau 4), within the
     tolerance of the scan token by token; and a value that is no number reaches no earlier token and no other sequence."""
     from fastgen_amd.kernels import ops, twins
 
@@ -249,6 +249,51 @@ def test_decay_scan_as_products_of_chunks(dtype, H, d, e, lens, least):
     later = torch.arange(T) >= int(q_start[1])
     assert torch.equal(ob[first | later], og[first | later]) and torch.isnan(ob[at, 0])
     assert torch.equal(sb[slots[1:].long()], sg[slots[1:].long()]) and torch.isnan(sb[slots[0], 0, 0, 0])
+
+
+# how the gates stand: tau, and the logits that z takes
+GATES = {
+    "near one": (16.0, lambda g, s: torch.randn(s, generator=g)),
+    "lasting": (16.0, lambda g, s: torch.randn(s, generator=g) + 8),
+    "wide": (1.0, lambda g, s: 4 * torch.randn(s, generator=g)),
+    "some close": (1.0, lambda g, s: torch.randn(s, generator=g) + 4 - 34 * (torch.rand(s, generator=g) < 0.05)),
+    "some shut": (4.0, lambda g, s: torch.randn(s, generator=g) + 4 - 400 * (torch.rand(s, generator=g) < 0.02)),
+    "half close": (1.0, lambda g, s: torch.randn(s, generator=g) + 6 - 13.0 * (torch.arange(s[0]) % 16 < 8)[:, None]),
+    "half shut": (1.0, lambda g, s: torch.randn(s, generator=g) + 6 - 56.0 * (torch.arange(s[0]) % 16 < 8)[:, None]),
+}
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("d", [48, 128])
+@pytest.mark.parametrize("gates", sorted(GATES))
+def test_decay_scan_as_products_is_as_exact_as_the_scan(dtype, d, gates):
+    """The error of the outputs and of the state against 64 bits (2-norms), as products of chunks and token by token: no
+    step on a value's way is less exact than the scan's and about as many roundings come together on it, so the two
+    errors may differ by a fifth and one rounding of the result, whatever the gates are (a weight taken from the
+    difference of two long sums of logarithms is off by 4 to 90 times as much)."""
+    from fastgen_amd.kernels import ops
+
+    g = torch.Generator().manual_seed(d)
+    T, e, (tau, draw) = 500, 32, GATES[gates]
+    rows, z = torch.randn(T, 2 * d + e, generator=g).to(dtype), draw(g, (T, d))
+    state = torch.randn(1, 1, d, e, generator=g)
+    a = torch.exp(torch.nn.functional.logsigmoid(z.double()) / tau)
+    q, k, v = (t.double() for t in rows.split([d, d, e], dim=1))
+    S, want = state[0, 0].double(), torch.empty(T, e, dtype=torch.float64)
+    for t in range(T):
+        S = a[t][:, None] * S + k[t][:, None] * v[t]
+        want[t] = (q[t] * d ** -0.5) @ S
+    q_start = torch.tensor([0, T], dtype=torch.int32)
+
+    def errors(host):
+        o, s = torch.empty(T, e, device=DEV), state.to(DEV)
+        ops.decay_scan(rows.to(DEV), 0, d, 2 * d, z.to(DEV), None, tau, d ** -0.5, s, torch.zeros(1, dtype=torch.int32, device=DEV),
+                       q_start.to(DEV), 1, o, q_start_host=host)
+        return [float((x.cpu().double() - y).norm() / y.norm()) for x, y in ((o, want), (s[0, 0], S))]
+
+    scan, products = errors(None), errors(q_start.numpy())
+    print(f"{gates} d {d}: token by token {scan[0]:.2e} {scan[1]:.2e}, products {products[0]:.2e} {products[1]:.2e}")
+    assert all(p <= 1.2 * s + 2.0 ** -24 for p, s in zip(products, scan)), (products, scan)
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
