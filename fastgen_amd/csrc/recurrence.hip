@@ -368,7 +368,7 @@ __global__ __launch_bounds__(256) void decay_chunk_sums_kernel(const ChunkArgs a
 #pragma unroll
       for (int u = 0; u < 16; ++u) v[u] = to_f<TA>(vp[(size_t)(t0 + min(2 * (u0 + u) + t_own, n - 1)) * a.row_stride]);
 #pragma unroll
-      for (int u = 0; u < 16; ++u) V_s[2 * (u0 + u) + t_own][col] = v[u];
+      for (int u = 0; u < 16; ++u) V_s[2 * (u0 + u) + t_own][col] = 2 * (u0 + u) + t_own < n ? v[u] : 0.f;
     }
   }
   for (int i = threadIdx.x; i < 4 * a.d; i += 256) {

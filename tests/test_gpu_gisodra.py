@@ -296,6 +296,33 @@ def test_decay_scan_as_products_is_as_exact_as_the_scan(dtype, d, gates):
     assert all(p <= 1.2 * s + 2.0 ** -24 for p, s in zip(products, scan)), (products, scan)
 
 
+@pytest.mark.parametrize("T", [300, 320, 321])
+def test_decay_scan_as_products_leaves_an_infinite_value_infinite(T):
+    """An infinity among the last token's values, in a chunk that its sequence ends inside or fills: the state's column is
+    infinite with the keys' signs, as token by token, and the others are what they are without it."""
+    from fastgen_amd.kernels import ops
+
+    torch.manual_seed(T)
+    d, e = 32, 24
+    rows, z = torch.randn(T, 2 * d + e), torch.randn(T, d)
+    q_start = torch.tensor([0, T], dtype=torch.int32)
+
+    def states(rows):
+        for host in (None, q_start.numpy()):
+            s = torch.zeros(1, 1, d, e, device=DEV)
+            ops.decay_scan(rows.to(DEV), 0, d, 2 * d, z.to(DEV), None, 16.0, 1.0, s, torch.zeros(1, dtype=torch.int32, device=DEV),
+                           q_start.to(DEV), 1, torch.empty(T, e, device=DEV), q_start_host=host)
+            yield s[0, 0].cpu()
+
+    _, plain = states(rows)
+    rows[T - 1, 2 * d + 5] = float("inf")
+    scan, products = states(rows)
+    assert torch.isinf(scan[:, 5]).all()
+    assert torch.equal(products[:, 5], scan[:, 5])
+    other = torch.arange(e) != 5
+    assert torch.equal(products[:, other], plain[:, other])
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("H,G,hd,P,window,n", [(4, 2, 16, 16, 9, 70), (5, 1, 80, 64, 110, 300), (2, 2, 48, 32, 33, 150),
                                                (12, 1, 176, 64, 56, 200), (3, 3, 24, 8, 0, 50)])
