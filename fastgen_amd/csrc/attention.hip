@@ -147,215 +147,421 @@ __global__ __launch_bounds__(ATT_WAVES* FG_WAVE) void paged_attention_general_ke
 }
 
 // ------------------------------------------------------------------ float32
-// The 32-bit path's attention on v_mfma_f32_16x16x4_f32 (fp32 products and sums).  A workgroup owns up to 16 rows:
-// the query heads of one kv head for a few consecutive tokens of one sequence (blocks of 16 / group tokens, cut where
-// the sequence changes; a workgroup a token is launched and all but a run's first leave, so that a prompt fills the
-// rows and the decoded tokens of many sequences do not wait for one another).  Tiles of 64 keys start at multiples of
-// 64; tile i belongs to wave i % 8 whatever the workgroup holds, a wave's tiles follow one another with a running
-// maximum, the eight waves' results are merged in order: a (token, head)'s arithmetic depends on its own keys alone,
-// so the bits are the same for a prompt, a decoded token and any cut.  S^T = K Q^T leaves a lane 4 keys of one row,
-// which is how O^T += V^T P^T takes them: nothing moves between lanes but a row's maximum and sum.  Keys and values
-// come straight from the pages, 1 KB (keys) and two halves of 2 KB (values) a load.
+// The 32-bit path's attention on v_mfma_f32_16x16x4_f32 (fp32 products and sums).  A run is up to 16 rows: the query
+// heads of one kv head for a few consecutive tokens of one sequence (blocks of 16 / group tokens, cut where the sequence
+// changes; a workgroup a token is launched and all but a run's first leave, so that a prompt fills the rows and the
+// decoded tokens of many sequences do not wait for one another).  Tiles of 64 keys start at multiples of 64; tile i
+// belongs to part i % 8 whatever the run holds, a part's tiles follow one another with a running maximum, the eight
+// parts' results are merged in order: a (token, head)'s arithmetic depends on its own keys alone, so the bits are the
+// same for a prompt, a decoded token and any cut.  S^T = K Q^T leaves a lane 4 keys of one row, which is how
+// O^T += V^T P^T takes them: nothing moves between lanes but a row's maximum and sum.  Keys and values come straight
+// from the pages, 1 KB (keys) and two halves of 2 KB (values) a load.
 //
-// Before: a wave a (token, head), a lane a key.  24 heads on 8 kv heads of 128, us before and now: a prompt of 400 /
-// 2048 tokens 174 / 3628 -> 59 / 592 (a third of the fp32 matrix cores' rate), one token of 4 sequences of 500 keys
-// 117 -> 30, of one of 4000 1243 -> 133 (the chain of a wave's 8 tiles), of 64 of 1000 455 -> 122, of 200 of 300 184 ->
-// 188 (both bound by the pages' reads, 2.6 TB/s).
+// A workgroup's eight waves take the parts of its run.  Where many sequences have few keys each, most waves would have no
+// tile and the others one, and a compute unit holds one such workgroup at a time (its registers).  So a run of at most 4
+// rows and 8 tiles (a part has one tile at most) is, if there are many (`af_alone_from`), a single wave's: a workgroup
+// takes eight runs, one a wave, which keeps the scores of its tiles in LDS until it knows the rows' maxima and then does
+// what the eight waves' merge does, operation for operation: the same bits, so the choice is free to follow the load.
+//
+// Bound by the latency of a tile's loads in each wave (the next block of 16 dims in flight while one is multiplied; more
+// of them in flight cost the registers) and, for long sequences, by the pages' reads.  Before: a wave a (token, head), a
+// lane a key (`paged_attention_general_kernel`).  us, before and now (heads / kv heads x head size):
+//                                   24/8x128    32/32x128    16/16x64     16/4x256    16/16x256      8/8x512
+//   a prompt of 400 tokens         181 /  58   230 /  94    94 /  38    251 /  64    267 /  68    415 /  79
+//   a prompt of 2048 tokens       3682 / 516  4627 / 781  1295 / 267   4009 / 535   4394 / 608   5180 / 626
+//   4 sequences of 500 keys        116 /  24   175 /  23    74 /  18    194 /  33    297 /  34    552 /  71
+//   32 of 4000                    1589 / 296  1773 / 700  1024 / 201   2803 / 229   3050 / 688   5708 / 800
+//   64 of 60, a wave a run          32 /  27    35 /  40    17 /  18     42 /  25*    45 /  38     75 /  83
+//   64 of 60, a workgroup a run     32 /  30    35 / 108    17 /  41     42 /  25     45 /  86     75 / 102
+//   200 of 100, a wave a run        61 /  45   177 / 168    41 /  52     84 /  62    155 / 150    206 / 217
+//   200 of 300, a wave a run       180 / 101   430 / 409   123 / 116    274 / 141*   386 / 372    541 / 524
+//   200 of 300, a workgroup a run  180 / 147   430 / 497   123 / 180    274 / 141    386 / 431    541 / 566
+// (* too few runs: a workgroup each.)
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 #define AF_WAVES 8
+#define AF_ALONE_ROWS 4
 
-// DB: head dims in blocks of 16, at least hd / 16 (hd is a multiple of 8).
-template <int DB>
-__global__ __launch_bounds__(AF_WAVES* FG_WAVE) void attention_f32_kernel(
-    const float* __restrict__ q, int q_stride, float* __restrict__ out, int out_stride,
-    const float* __restrict__ k_pages, const float* __restrict__ v_pages, const int* __restrict__ block_table,
-    int bt_stride, const int* __restrict__ seq_of_token, const int* __restrict__ positions, int n_tokens, int n_heads,
-    int n_kv, int hd, int page_size, float scale, int window, const float* __restrict__ sinks,
-    const float* __restrict__ dist) {
-  constexpr int MB = DB < 8 ? DB : 8;             // dim blocks merged at a time
-  __shared__ f32x4 q_s[DB * 4][16];               // [4 dims][row]
-  __shared__ f32x4 o_s[AF_WAVES][MB][FG_WAVE];
-  __shared__ float m_s[AF_WAVES][16], l_s[AF_WAVES][16];
-  const int tid = threadIdx.x, lane = tid % FG_WAVE, wave = tid / FG_WAVE;
-  const int r = lane % 16, g = lane / 16;
-  const int kvh = blockIdx.x % n_kv, group = n_heads / n_kv;
-  // (the blocks' first tokens come first, a token's kv heads side by side: every die gets as many of them)
-  const int full = 16 / group, blocks = (n_tokens + full - 1) / full, place = blockIdx.x / n_kv;
+// From how many runs on a wave alone takes a run of `tiles` tiles.  As measured, a wave a run / a workgroup a run: with 256
+// runs of one tile 36 / 26 us (head size 256), with 512 25 / 30 (128); 512 runs of 4 tiles 66 / 36, 1024 of 4 125 / 120
+// (256), 2048 of 4 107 / 139 (128); 800 of 5 145 / 144 (256), 1600 of 5 100 / 151 (128); 1600 of 8 152 / 179, 3200 of 8
+// 581 / 571 (256).  Head sizes up to 64, where a workgroup's chain is shorter: 1024 of 4 45 / 45, 3200 of 5 116 / 180, 1600
+// of 5 beside a prompt of 400 tokens 143 / 133.
+__host__ __device__ constexpr int af_alone_from(int db, int tiles) { return db <= 4 ? 350 * tiles : 160 * (tiles + 1); }
+
+struct AfArgs {
+  const float* q; int q_stride;
+  float* out; int out_stride;
+  const float *k_pages, *v_pages;
+  const int* block_table; int bt_stride;
+  const int *seq_of_token, *positions;
+  int n_tokens, n_heads, n_kv, hd, page_size;
+  float scale; int window;
+  const float *sinks, *dist;
+  int few_runs;  // how many runs of few rows there may be: one a sequence and kv head
+};
+
+struct AfRun {
+  int t0, n_here, seq, kvh, p_lo, p_hi;  // its tokens, and their lowest and highest position
+  int lo;                                // keys lo .. p_hi are seen by some row: their pages are held
+};
+// The run that starts at place `index` of the grid; false: none does.  Uniform.
+// (The blocks' first tokens come first, a token's kv heads side by side: every die gets as many of them.)
+__device__ __forceinline__ bool af_run(const AfArgs& a, int index, AfRun& run) {
+  const int full = 16 / (a.n_heads / a.n_kv), blocks = (a.n_tokens + full - 1) / full, place = index / a.n_kv;
+  if (place >= blocks * full) return false;
   const int t0 = place % blocks * full + place / blocks;
-  if (t0 >= n_tokens) return;
-  const int seq = seq_of_token[t0];
-  if (t0 % full && seq_of_token[t0 - 1] == seq) return;  // an earlier workgroup's run holds this token
-  int n_here = 1, p_lo = positions[t0], p_hi = p_lo;
-  for (; t0 + n_here < n_tokens && (t0 + n_here) % full && seq_of_token[t0 + n_here] == seq; ++n_here) {
-    const int p = positions[t0 + n_here];
-    p_lo = min(p_lo, p);
-    p_hi = max(p_hi, p);
+  if (t0 >= a.n_tokens) return false;
+  const int seq = a.seq_of_token[t0];
+  if (t0 % full && a.seq_of_token[t0 - 1] == seq) return false;  // an earlier run holds this token
+  run.t0 = t0, run.seq = seq, run.kvh = index % a.n_kv, run.n_here = 1;
+  run.p_lo = run.p_hi = a.positions[t0];
+  for (; t0 + run.n_here < a.n_tokens && (t0 + run.n_here) % full && a.seq_of_token[t0 + run.n_here] == seq; ++run.n_here) {
+    const int p = a.positions[t0 + run.n_here];
+    run.p_lo = min(run.p_lo, p);
+    run.p_hi = max(run.p_hi, p);
   }
-  const KvLayout lay(page_size, hd);
-  const size_t head_elems = (size_t)page_size * hd;
+  run.lo = first_key(run.p_lo, a.window);
+  return true;
+}
 
-  // this lane's row: a token of the block and one of its heads (rows behind the last repeat the last token)
-  const int mine = min(r / group, n_here - 1);
-  const bool live = r < n_here * group;
-  const int head = kvh * group + r % group, pos = positions[t0 + mine], first = first_key(pos, window);
-  const float d1 = dist ? dist[2 * head] : 0.f, d2 = dist ? dist[2 * head + 1] : 0.f;
-  for (int i = tid; i < DB * 4 * 16 * 4; i += AF_WAVES * FG_WAVE) {  // element by element: q may lie anywhere
-    const int d = i % (DB * 16), row = i / (DB * 16);
-    const int t = t0 + min(row / group, n_here - 1), h = kvh * group + row % group;
-    ((float*)&q_s[d / 4][row])[d % 4] = d < hd ? q[(size_t)t * q_stride + (size_t)h * hd + d] : 0.f;
+// Whether a wave alone takes the run.
+template <int DB>
+__device__ __forceinline__ bool af_alone(const AfArgs& a, const AfRun& run) {
+  const int tiles = run.p_hi / ATT_TILE - run.lo / ATT_TILE + 1;
+  return run.n_here * (a.n_heads / a.n_kv) <= AF_ALONE_ROWS && tiles <= AF_WAVES && a.few_runs >= af_alone_from(DB, tiles);
+}
+
+// Lane 16 g + r's row r: a token of the run and one of its heads (rows behind the last see no key and are not stored).
+struct AfRow {
+  int token, head, pos, first;
+  bool live;
+  float d1, d2;
+};
+__device__ __forceinline__ AfRow af_row(const AfArgs& a, const AfRun& run, int r) {
+  const int group = a.n_heads / a.n_kv;
+  AfRow row;
+  row.token = run.t0 + min(r / group, run.n_here - 1);
+  row.live = r < run.n_here * group;
+  row.head = run.kvh * group + r % group;
+  row.pos = a.positions[row.token];
+  row.first = first_key(row.pos, a.window);
+  row.d1 = a.dist ? a.dist[2 * row.head] : 0.f;
+  row.d2 = a.dist ? a.dist[2 * row.head + 1] : 0.f;
+  return row;
+}
+__device__ __forceinline__ bool af_sees(const AfRow& row, int key) { return row.live && key >= row.first && key <= row.pos; }
+
+// Query rows first, first + step, .. (below `rows`) of the run into LDS, q_s[4 dims][N rows], by a wave, element by element:
+// q may lie anywhere.
+template <int DB, int N>
+__device__ __forceinline__ void af_queries(const AfArgs& a, const AfRun& run, f32x4 (*q_s)[N], int first, int step, int rows,
+                                           int lane) {
+  const int group = a.n_heads / a.n_kv;
+  for (int row = first; row < rows; row += step) {  // uniform in the wave
+    const float* q = a.q + (size_t)(run.t0 + row / group) * a.q_stride + (size_t)(run.kvh * group + row % group) * a.hd;
+    float x[DB / 4];
+#pragma unroll
+    for (int k = 0; k < DB / 4; ++k) x[k] = q[min(lane + k * FG_WAVE, a.hd - 1)];
+#pragma unroll
+    for (int k = 0; k < DB / 4; ++k) {
+      const int d = lane + k * FG_WAVE;
+      ((float*)&q_s[d / 4][row])[d % 4] = d < a.hd ? x[k] : 0.f;
+    }
   }
+}
+
+// Scores of the tile's keys 16 b + 4 g + e with the lane's row (-infinity where the row does not see the key), and the
+// row's highest.
+template <int DB, int N>
+__device__ __forceinline__ float af_scores(const AfArgs& a, const AfRun& run, const AfRow& row, const KvLayout& lay, int tile,
+                                           const f32x4 (*q_s)[N], int q_row, int r, int g, f32x4 (&s)[4]) {
+  const int kb = tile * ATT_TILE;
+  const int* table = a.block_table + (size_t)run.seq * a.bt_stride;
+  const float* kp[4];
+#pragma unroll
+  for (int b = 0; b < 4; ++b) {  // (keys that no row sees are read as the nearest one that some row does)
+    const int key = min(max(kb + 16 * b + r, run.lo), run.p_hi);
+    kp[b] = a.k_pages + ((size_t)table[key / a.page_size] * a.n_kv + run.kvh) * ((size_t)a.page_size * a.hd) +
+            lay.k_off(key % a.page_size, 0);
+    s[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  const size_t chunk = (size_t)8 << lay.kb_shift;  // from 8 head dims of a key to the next 8
+  // The next block of 16 dims is asked for before this one is multiplied, and never conditionally: behind the head's dims
+  // its first ones, for zeros.
+  f32x4 kv[2][4];
+  auto load = [&](int i) {
+    const size_t at = 16 * i + 4 * g < a.hd ? chunk * (2 * i + g / 2) + g % 2 * 4 : 0;
+#pragma unroll
+    for (int b = 0; b < 4; ++b) kv[i % 2][b] = *(const f32x4*)(kp[b] + at);
+  };
+  load(0);
+#pragma unroll
+  for (int i = 0; i < DB; ++i) {
+    if (i + 1 < DB) load(i + 1);
+    __builtin_amdgcn_sched_barrier(0);
+    const f32x4 qv = q_s[4 * i + g][q_row];
+    const bool in = 16 * i + 4 * g < a.hd;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+        s[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? kv[i % 2][b][e] : 0.f, qv[e], s[b], 0, 0, 0);
+  }
+  float top = -INFINITY;
+#pragma unroll
+  for (int b = 0; b < 4; ++b)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int key = kb + 16 * b + 4 * g + e;
+      float v = s[b][e] * a.scale;
+      if (a.dist) v -= row.d1 * log1pf(row.d2 * (float)(row.pos - key));
+      asm("" : "+v"(v));  // rounded here in every use (a product fused with the maximum's subtraction would not be)
+      s[b][e] = af_sees(row, key) ? v : -INFINITY;
+      top = fmaxf(top, s[b][e]);
+    }
+  top = fmaxf(top, __shfl_xor(top, 16, FG_WAVE));
+  return fmaxf(top, __shfl_xor(top, 32, FG_WAVE));
+}
+
+// The tile's weights in the place of its scores, and the row's sum of them.
+__device__ __forceinline__ float af_weights(const AfRow& row, int tile, float m, int g, f32x4 (&s)[4]) {
+  float sum = 0.f;
+#pragma unroll
+  for (int b = 0; b < 4; ++b)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      s[b][e] = af_sees(row, tile * ATT_TILE + 16 * b + 4 * g + e) ? expf(s[b][e] - m) : 0.f;
+      sum += s[b][e];
+    }
+  sum += __shfl_xor(sum, 16, FG_WAVE);
+  return sum + __shfl_xor(sum, 32, FG_WAVE);
+}
+
+// done(i, start(i) + V^T P^T) for the blocks i of 16 head dims: lane 16 g + r gets dims 16 i + 4 g .. + 3 of row r.
+template <int DB, class Start, class Done>
+__device__ __forceinline__ void af_values(const AfArgs& a, const AfRun& run, const AfRow& row, const KvLayout& lay, int tile,
+                                          const f32x4 (&w)[4], int r, int g, Start start, Done done) {
+  const int kb = tile * ATT_TILE, lo = run.lo, hi = run.p_hi;
+  const int* table = a.block_table + (size_t)run.seq * a.bt_stride;
+  const float* vp[4];
+#pragma unroll
+  for (int b = 0; b < 4; ++b) {
+    const int four = min(max(kb + 16 * b + 4 * g, lo & ~3), hi & ~3), slot = lay.v_slot(four % a.page_size);
+    vp[b] = a.v_pages + ((size_t)table[four / a.page_size] * a.n_kv + run.kvh) * ((size_t)a.page_size * a.hd) + slot % 8 +
+            lay.v_chunk_off(slot / 8, 0);
+  }
+  // whether some key of the tile is seen by one row of the run and not by another
+  const bool mixed = run.p_lo != hi && (kb + ATT_TILE - 1 > run.p_lo || kb < first_key(hi, a.window));
+  f32x4 vv[2][4];
+  auto load = [&](int i) {
+    const size_t at = lay.v_chunk_off(0, 16 * i + r < a.hd ? 16 * i + r : 0);
+#pragma unroll
+    for (int b = 0; b < 4; ++b) vv[i % 2][b] = *(const f32x4*)(vp[b] + at);
+  };
+  load(0);
+#pragma unroll
+  for (int i = 0; i < DB; ++i) {
+    if (i + 1 < DB) load(i + 1);
+    __builtin_amdgcn_sched_barrier(0);
+    f32x4(&v)[4] = vv[i % 2];
+    // dims behind the head's, and keys that no row sees: their places may hold anything
+    const bool in = 16 * i + r < a.hd;
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int key = kb + 16 * b + 4 * g + e;
+        v[b][e] = in && key >= lo && key <= hi ? v[b][e] : 0.f;
+      }
+    bool bad = false;
+    if (mixed) {  // uniform
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) bad |= !(fabsf(v[b][e]) <= 3.402823466e38f);
+    }
+    f32x4 acc = start(i);
+    if (!__any(bad)) {
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(v[b][e], w[b][e], acc, 0, 0, 0);
+    } else {  // an infinity or NaN among the values: a weight of zero would not keep it from the rows before it
+      for (int other = 0; other < 16; ++other) {
+        const int p = __shfl(row.pos, other, FG_WAVE), f = __shfl(row.first, other, FG_WAVE);
+        f32x4 one = acc;
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int key = kb + 16 * b + 4 * g + e;
+            one = __builtin_amdgcn_mfma_f32_16x16x4f32(key >= f && key <= p ? v[b][e] : 0.f, w[b][e], one, 0, 0, 0);
+          }
+        if (r == other) acc = one;
+      }
+    }
+    done(i, acc);
+  }
+}
+
+// A part's share of a row whose highest score is `top`.
+__device__ __forceinline__ float af_factor(float m, float top) { return m == top ? 1.f : expf(m - top); }
+__device__ __forceinline__ f32x4 af_scaled(const f32x4 x, float f) {  // rounded, whatever is added to it
+  f32x4 y = x * f;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    float v = y[e];
+    asm("" : "+v"(v));
+    y[e] = v;
+  }
+  return y;
+}
+// A sink is one more term exp(sinks[h]) in the softmax's denominator, which brings no value.
+__device__ __forceinline__ float af_inverse(const AfArgs& a, const AfRow& row, float total, float top) {
+  if (a.sinks) total += expf(a.sinks[row.head] - top);
+  return 1.f / total;
+}
+__device__ __forceinline__ void af_store(const AfArgs& a, const AfRow& row, int d, const f32x4 o, float inv) {
+  if (!row.live) return;
+  float* at = a.out + (size_t)row.token * a.out_stride + (size_t)row.head * a.hd + d;
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    if (d + e < a.hd) at[e] = o[e] * inv;
+}
+
+// What a workgroup keeps in LDS for a run of its own, and what each of its waves does for one.
+template <int DB>
+struct AfShared {
+  static constexpr int MB = DB < 8 ? DB : 8;  // dim blocks merged at a time
+  f32x4 q_s[DB * 4][16];                      // [4 dims][row]
+  f32x4 o_s[AF_WAVES][MB][FG_WAVE];
+  float m_s[AF_WAVES][16], l_s[AF_WAVES][16];
+};
+template <int DB>
+struct AfAlone {
+  f32x4 q_s[DB * 4][AF_ALONE_ROWS];
+  f32x4 s_s[AF_WAVES][AF_ALONE_ROWS][ATT_TILE / 4];  // a part's scores
+  float m_s[AF_WAVES][AF_ALONE_ROWS];
+};
+
+// A run by a workgroup; ends in a barrier.
+template <int DB>
+__device__ __forceinline__ void af_together(const AfArgs& a, const AfRun& run, AfShared<DB>& lds, int wave, int lane) {
+  constexpr int MB = AfShared<DB>::MB;
+  const int r = lane % 16, g = lane / 16;
+  const KvLayout lay(a.page_size, a.hd);
+  const AfRow row = af_row(a, run, r);
+  af_queries<DB, 16>(a, run, lds.q_s, wave, AF_WAVES, run.n_here * (a.n_heads / a.n_kv), lane);
   __syncthreads();
-
-  const int* table = block_table + (size_t)seq * bt_stride;
-  const int lo = first_key(p_lo, window), hi = p_hi;  // the keys that some row of the run sees: their pages are held
-
   f32x4 acc[DB];
 #pragma unroll
   for (int i = 0; i < DB; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, l = 0.f;
-  for (int tile = lo / ATT_TILE + ((wave - lo / ATT_TILE) & (AF_WAVES - 1)); tile * ATT_TILE <= hi; tile += AF_WAVES) {
-    const int kb = tile * ATT_TILE;
-    const float* kp[4];
-    const float* vp[4];
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {  // (keys that no row sees are read as the nearest one that some row does)
-      const int key = min(max(kb + 16 * b + r, lo), hi);
-      kp[b] = k_pages + ((size_t)table[key / page_size] * n_kv + kvh) * head_elems + lay.k_off(key % page_size, 0);
-      const int four = min(max(kb + 16 * b + 4 * g, lo & ~3), hi & ~3), slot = lay.v_slot(four % page_size);
-      vp[b] = v_pages + ((size_t)table[four / page_size] * n_kv + kvh) * head_elems + slot % 8 +
-              lay.v_chunk_off(slot / 8, 0);
-    }
-    const size_t chunk = (size_t)8 << lay.kb_shift;  // from 8 head dims of a key to the next 8
+  const int t_lo = run.lo / ATT_TILE;
+  for (int tile = t_lo + ((wave - t_lo) & (AF_WAVES - 1)); tile * ATT_TILE <= run.p_hi; tile += AF_WAVES) {
     f32x4 s[4];
-#pragma unroll
-    for (int b = 0; b < 4; ++b) s[b] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int i = 0; i < DB; ++i) {
-      const f32x4 qv = q_s[4 * i + g][r];
-      f32x4 kv[4];
-      const bool in = 16 * i + 4 * g < hd;
-#pragma unroll
-      for (int b = 0; b < 4; ++b)
-        kv[b] = in ? *(const f32x4*)(kp[b] + chunk * (2 * i + g / 2) + g % 2 * 4) : f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) s[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[b][e], qv[e], s[b], 0, 0, 0);
-    }
-    float top = -INFINITY;
-#pragma unroll
-    for (int b = 0; b < 4; ++b)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int key = kb + 16 * b + 4 * g + e;
-        float v = s[b][e] * scale;
-        if (dist) v -= d1 * log1pf(d2 * (float)(pos - key));
-        s[b][e] = live && key >= first && key <= pos ? v : -INFINITY;
-        top = fmaxf(top, s[b][e]);
-      }
-    top = fmaxf(top, __shfl_xor(top, 16, FG_WAVE));
-    top = fmaxf(top, __shfl_xor(top, 32, FG_WAVE));
-    const float m_new = fmaxf(m, top);
+    const float m_new = fmaxf(m, af_scores<DB, 16>(a, run, row, lay, tile, lds.q_s, r, r, g, s));
     // a row that has seen no key yet, or sees none in this tile, stays as it is
-    const float alpha = m == m_new ? 1.f : expf(m - m_new);
-    float sum = 0.f;
-#pragma unroll
-    for (int b = 0; b < 4; ++b)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int key = kb + 16 * b + 4 * g + e;
-        s[b][e] = live && key >= first && key <= pos ? expf(s[b][e] - m_new) : 0.f;
-        sum += s[b][e];
-      }
-    sum += __shfl_xor(sum, 16, FG_WAVE);
-    sum += __shfl_xor(sum, 32, FG_WAVE);
-    l = l * alpha + sum;
+    const float alpha = af_factor(m, m_new);
+    l = l * alpha + af_weights(row, tile, m_new, g, s);
     m = m_new;
-    // whether some key of the tile is seen by one row of the run and not by another
-    const bool mixed = kb + ATT_TILE - 1 > p_lo || kb < first_key(p_hi, window);
-#pragma unroll
-    for (int i = 0; i < DB; ++i) {
-      acc[i] *= alpha;
-      const int d = 16 * i + r;
-      f32x4 vv[4];
-      const size_t at = lay.v_chunk_off(0, d);
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        vv[b] = d < hd ? *(const f32x4*)(vp[b] + at) : f32x4{0.f, 0.f, 0.f, 0.f};
-        // what lies behind the keys was never written and may be anything
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int key = kb + 16 * b + 4 * g + e;
-          if (key < lo || key > hi) vv[b][e] = 0.f;
-        }
-      }
-      bool bad = false;
-      if (mixed && p_lo != p_hi) {
-#pragma unroll
-        for (int b = 0; b < 4; ++b)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) bad |= !(fabsf(vv[b][e]) <= 3.402823466e38f);
-      }
-      if (!__any(bad)) {
-#pragma unroll
-        for (int b = 0; b < 4; ++b)
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[b][e], s[b][e], acc[i], 0, 0, 0);
-      } else {  // an infinity or NaN among the values: a weight of zero would not keep it from the rows before it
-        for (int row = 0; row < 16; ++row) {
-          const int p = __shfl(pos, row, FG_WAVE), f = __shfl(first, row, FG_WAVE);
-          f32x4 one = acc[i];
-#pragma unroll
-          for (int b = 0; b < 4; ++b)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const int key = kb + 16 * b + 4 * g + e;
-              one = __builtin_amdgcn_mfma_f32_16x16x4f32(key >= f && key <= p ? vv[b][e] : 0.f, s[b][e], one, 0, 0, 0);
-            }
-          if (r == row) acc[i] = one;
-        }
-      }
-    }
+    af_values<DB>(a, run, row, lay, tile, s, r, g, [&](int i) { return acc[i] * alpha; },
+                  [&](int i, const f32x4 x) { acc[i] = x; });
   }
-
-  // ---- the waves' results, in order
-  if (lane < 16) m_s[wave][r] = m, l_s[wave][r] = l;
+  // ---- the parts' results, in order
+  if (lane < 16) lds.m_s[wave][r] = m, lds.l_s[wave][r] = l;
   __syncthreads();
-  float top = m_s[0][r];
+  float top = lds.m_s[0][r];
 #pragma unroll
-  for (int w = 1; w < AF_WAVES; ++w) top = fmaxf(top, m_s[w][r]);
-  const float factor = m == top ? 1.f : expf(m - top);
+  for (int w = 1; w < AF_WAVES; ++w) top = fmaxf(top, lds.m_s[w][r]);
   float total = 0.f;
 #pragma unroll
-  for (int w = 0; w < AF_WAVES; ++w) total += l_s[w][r] * (m_s[w][r] == top ? 1.f : expf(m_s[w][r] - top));
-  // a sink: one more term exp(sinks[h]) in the softmax's denominator, which brings no value
-  if (sinks) total += expf(sinks[head] - top);
-  const float inv = 1.f / total;
+  for (int w = 0; w < AF_WAVES; ++w) total = fmaf(lds.l_s[w][r], af_factor(lds.m_s[w][r], top), total);
+  const float factor = af_factor(m, top), inv = af_inverse(a, row, total, top);
 #pragma unroll
   for (int i0 = 0; i0 < DB; i0 += MB) {
 #pragma unroll
-    for (int i = 0; i < MB; ++i) o_s[wave][i][lane] = acc[i0 + i] * factor;
+    for (int i = 0; i < MB; ++i) lds.o_s[wave][i][lane] = acc[i0 + i] * factor;
     __syncthreads();
     if (wave < MB) {  // (a thread's lane stands for the same row and dims as above, its wave for the dim block)
       f32x4 o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int w = 0; w < AF_WAVES; ++w) o += o_s[w][wave][lane];
-      const int d = 16 * (i0 + wave) + 4 * g;
-      if (live) {
-        float* at = out + (size_t)(t0 + mine) * out_stride + (size_t)head * hd + d;
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (d + e < hd) at[e] = o[e] * inv;
-      }
+      for (int w = 0; w < AF_WAVES; ++w) o += lds.o_s[w][wave][lane];
+      af_store(a, row, 16 * (i0 + wave) + 4 * g, o, inv);
     }
     __syncthreads();
   }
 }
 
+// A run of at most AF_ALONE_ROWS rows and AF_WAVES tiles by a wave: what `af_together` does, part after part.
+template <int DB>
+__device__ __forceinline__ void af_by_wave(const AfArgs& a, const AfRun& run, AfAlone<DB>& lds, int lane) {
+  const int r = lane % 16, g = lane / 16, q_row = min(r, AF_ALONE_ROWS - 1);
+  const bool keeps = r < AF_ALONE_ROWS;
+  const KvLayout lay(a.page_size, a.hd);
+  const AfRow row = af_row(a, run, r);
+  af_queries<DB, AF_ALONE_ROWS>(a, run, lds.q_s, 0, 1, run.n_here * (a.n_heads / a.n_kv), lane);
+  // (a wave's LDS operations are done in order; the fences keep the compiler to it)
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  const int t_lo = run.lo / ATT_TILE, t_hi = run.p_hi / ATT_TILE;
+  float top = -INFINITY;
+  for (int tile = t_lo; tile <= t_hi; ++tile) {
+    f32x4 s[4];
+    const float m = af_scores<DB, AF_ALONE_ROWS>(a, run, row, lay, tile, lds.q_s, q_row, r, g, s);
+    top = fmaxf(top, m);
+    if (keeps) {
+#pragma unroll
+      for (int b = 0; b < 4; ++b) lds.s_s[tile % AF_WAVES][r][4 * b + g] = s[b];
+      if (g == 0) lds.m_s[tile % AF_WAVES][r] = m;
+    }
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  f32x4 o[DB];
+#pragma unroll
+  for (int i = 0; i < DB; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float total = 0.f;
+  for (int part = 0; part < AF_WAVES; ++part) {
+    const int tile = t_lo + ((part - t_lo) & (AF_WAVES - 1));
+    if (tile > t_hi) continue;
+    f32x4 s[4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b) s[b] = lds.s_s[part][q_row][4 * b + g];
+    const float m = lds.m_s[part][q_row], l = af_weights(row, tile, m, g, s), factor = af_factor(m, top);
+    total = fmaf(l, factor, total);
+    af_values<DB>(a, run, row, lay, tile, s, r, g, [&](int) { return f32x4{0.f, 0.f, 0.f, 0.f}; },
+                  [&](int i, const f32x4 x) { o[i] += af_scaled(x, factor); });
+  }
+  const float inv = af_inverse(a, row, total, top);
+#pragma unroll
+  for (int i = 0; i < DB; ++i) af_store(a, row, 16 * i + 4 * g, o[i], inv);
+}
+
+// DB: head dims in blocks of 16, at least hd / 16 (hd is a multiple of 8).  ALONE: a wave alone takes what `af_alone` says.
+template <int DB, bool ALONE>
+__global__ __launch_bounds__(AF_WAVES* FG_WAVE) void attention_f32_kernel(const AfArgs a) {
+  const int lane = threadIdx.x % FG_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / FG_WAVE);
+  AfRun run;
+  if constexpr (!ALONE) {
+    __shared__ AfShared<DB> lds;
+    if (af_run(a, blockIdx.x, run)) af_together<DB>(a, run, lds, wave, lane);
+  } else {
+    __shared__ union {
+      AfShared<DB> together;
+      AfAlone<DB> alone[AF_WAVES];
+    } lds;
+    if (af_run(a, blockIdx.x, run) && !af_alone<DB>(a, run)) af_together<DB>(a, run, lds.together, wave, lane);
+    // (the first eighth of the grid looks after the others' runs, not every eighth workgroup: those are all on one die)
+    if (blockIdx.x < (gridDim.x + AF_WAVES - 1) / AF_WAVES && af_run(a, blockIdx.x * AF_WAVES + wave, run) &&
+        af_alone<DB>(a, run))
+      af_by_wave<DB>(a, run, lds.alone[wave], lane);
+  }
+}
+
 extern "C" int fg_paged_attention_general_sink(
     const void* q, int q_stride, void* out, int out_stride, const void* k_pages,
-    const void* v_pages, const int* block_table, int bt_stride, const int* seq_of_token,
+    const void* v_pages, const int* block_table, int bt_stride, int n_seqs, const int* seq_of_token,
     const int* positions, int n_tokens, int n_heads, int n_kv, int hd, int page_size,
     float scale, int window, const float* sinks, const float* dist, int dtype, hipStream_t stream) {
   if (n_tokens <= 0) return FG_OK;
@@ -367,10 +573,15 @@ extern "C" int fg_paged_attention_general_sink(
     const int full = 16 / group;
     const long long grid = (long long)((n_tokens + full - 1) / full * full) * n_kv;
     if (grid > 2147483647LL) return FG_ERR_ARG;
-#define ATTENTION_F32(DB)                                                                                           \
-  attention_f32_kernel<DB><<<(unsigned)grid, AF_WAVES * FG_WAVE, 0, stream>>>(                                                \
-      (const float*)q, q_stride, (float*)out, out_stride, (const float*)k_pages, (const float*)v_pages, block_table, \
-      bt_stride, seq_of_token, positions, n_tokens, n_heads, n_kv, hd, page_size, scale, window, sinks, dist)
+    const AfArgs a{(const float*)q, q_stride, (float*)out, out_stride, (const float*)k_pages, (const float*)v_pages, block_table,
+                   bt_stride, seq_of_token, positions, n_tokens, n_heads, n_kv, hd, page_size, scale, window, sinks, dist,
+                   (int)min((long long)min(n_seqs, n_tokens) * n_kv, 2147483647LL)};
+    const bool alone = group <= AF_ALONE_ROWS && a.few_runs >= (hd <= 64 ? af_alone_from(4, 1) : af_alone_from(8, 1));
+#define ATTENTION_F32(DB)                                                                                   \
+  do {                                                                                                      \
+    if (alone) attention_f32_kernel<DB, true><<<(unsigned)grid, AF_WAVES * FG_WAVE, 0, stream>>>(a);        \
+    else attention_f32_kernel<DB, false><<<(unsigned)grid, AF_WAVES * FG_WAVE, 0, stream>>>(a);             \
+  } while (0)
     if (hd <= 64) ATTENTION_F32(4);
     else if (hd <= 128) ATTENTION_F32(8);
     else if (hd <= 256) ATTENTION_F32(16);
@@ -395,14 +606,4 @@ extern "C" int fg_paged_attention_general_sink(
   else
     return FG_ERR_ARG;
   return fg_launch_status();
-}
-
-extern "C" int fg_paged_attention_general(
-    const void* q, int q_stride, void* out, int out_stride, const void* k_pages,
-    const void* v_pages, const int* block_table, int bt_stride, const int* seq_of_token,
-    const int* positions, int n_tokens, int n_heads, int n_kv, int hd, int page_size,
-    float scale, int window, int dtype, hipStream_t stream) {
-  return fg_paged_attention_general_sink(q, q_stride, out, out_stride, k_pages, v_pages, block_table, bt_stride,
-                                         seq_of_token, positions, n_tokens, n_heads, n_kv, hd, page_size, scale,
-                                         window, nullptr, nullptr, dtype, stream);
 }

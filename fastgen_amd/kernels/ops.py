@@ -544,7 +544,7 @@ def paged_attention_general(q: torch.Tensor, out: torch.Tensor, k_pages: torch.T
     _need(page_size % 8 == 0, f"page size {page_size} is not supported (multiple of 8)")
     st = _lib.load("attention").fg_paged_attention_general_sink(
         _ptr(q), q.stride(0), _ptr(out), out.stride(0), _ptr(k_pages), _ptr(v_pages), _ptr(block_table),
-        block_table.stride(0), _ptr(seq_of_token), _ptr(positions), T, n_heads, n_kv, hd, page_size,
+        block_table.stride(0), block_table.shape[0], _ptr(seq_of_token), _ptr(positions), T, n_heads, n_kv, hd, page_size,
         ctypes.c_float(scale), int(window or 0), _ptr(sinks), _ptr(distance), _code(q), _stream(q))
     _check(st, "paged_attention_general")
     return out

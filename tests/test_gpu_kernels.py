@@ -306,6 +306,34 @@ def test_paged_attention_f32_every_cut_gives_the_same_bits(ops, H, KV, hd, P, wi
     assert not torch.isfinite(got[sees][:, 0]).any()
 
 
+@pytest.mark.parametrize("H,KV,hd,P", [(16, 16, 64, 64), (24, 8, 128, 16), (8, 8, 24, 8), (8, 8, 136, 32), (16, 8, 256, 64),
+                                       (8, 8, 512, 64)])
+@pytest.mark.parametrize("window,more", [(0, False), (100, True), (500, False), (-96, False), (0, True)])
+def test_paged_attention_f32_runs_of_a_wave(ops, H, KV, hd, P, window, more):
+    """Many sequences of few keys, whose runs of up to 4 rows and 8 tiles are a wave's each, beside longer ones and a prompt:
+    the bits that each token's call of its own gives (a workgroup's run).  `more`: with sinks and a bias by distance."""
+    lens = [1, 2, 63, 64, 65, 128, 129, 511, 512, 513, 577, 640] + [(37 * i) % 70 + 1 for i in range(170)]
+    seqs = [(n - 1, 1) for n in lens[:100]] + [(130, 3), (0, 35)] + [(n - 1, 1) for n in lens[100:]]
+    case = _paged_case(torch.float32, seqs, H, KV, hd, P, seed=12)
+    sinks = torch.randn(H, device=DEV) if more else None
+    distance = torch.rand(H, 2, device=DEV) if more else None
+
+    def run(rows=slice(None), q=case["q"]):
+        out = torch.empty_like(q[rows])
+        return ops.paged_attention_general(q[rows], out, case["kp"], case["vp"], case["table"], case["seq_of"][rows],
+                                           case["pos"][rows], H, hd**-0.5, window, sinks, distance)
+
+    out = run()
+    assert torch.isfinite(out).all()
+    for t in [*range(14), *range(98, 145, 3), 200]:
+        assert torch.equal(run(slice(t, t + 1))[0], out[t]), t
+    wide = torch.zeros(len(out), H * hd + 3, device=DEV)  # rows of another stride, and not aligned
+    wide[:, 1:H * hd + 1] = case["q"]
+    assert torch.equal(run(q=wide[:, 1:H * hd + 1]), out)
+    if window >= 0 and not more:
+        assert torch.allclose(out[:12].cpu(), _plain_rows(case, seqs[:12], window or None), atol=2e-5, rtol=1e-5)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_paged_attention_far_key_stands_out(ops, dtype):
     """One key among hundreds, in an early page, gets nearly all the weight:
