@@ -23,6 +23,8 @@
 // again a step later.
 #include "common.h"
 
+#include <type_traits>
+
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -386,7 +388,7 @@ struct MoeOperand {
       base = w + ((size_t)expert * rows + min(row + lane % 16, rows - 1)) * ldw + 8 * (lane / 16);
     }
   }
-  // (behind k: any readable place; what stands there meets zeros of x)
+  // (behind k: any readable place; what stands there is replaced by zeros before it is multiplied)
   __device__ __forceinline__ bf16x8 load(int s, int K, int g) const {
     if constexpr (PACKED) return *(const bf16x8*)(base + (size_t)(32 * s < K ? s : 0) * 512);
     else return *(const bf16x8*)(base + moe_k_at(s, K, g));
@@ -410,15 +412,19 @@ __device__ __forceinline__ void moe_stream(const MoeOperand<PACKED> (&w)[NM], co
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb) b[set][i][mb] = *(const bf16x8*)(px[mb] + moe_k_at(s0 + i, K, g));
   };
-  auto multiply = [&](int s0, int set) {
+  // (where k ends inside the steps: zeros in both operands behind it, an infinity times a zero would be no number)
+  auto multiply = [&](int s0, int set, auto ends) {
 #pragma unroll
     for (int i = 0; i < U; ++i) {
-      const bool in = 32 * (s0 + i) + 8 * g < K;
+      const bool in = !ends.value || 32 * (s0 + i) + 8 * g < K;
+      bf16x8 av[NM];
+#pragma unroll
+      for (int m = 0; m < NM; ++m) av[m] = in ? a[set][i][m] : moe_zero8();
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb) {
         const bf16x8 bv = in ? b[set][i][mb] : moe_zero8();
 #pragma unroll
-        for (int m = 0; m < NM; ++m) acc[m][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[set][i][m], bv, acc[m][mb], 0, 0, 0);
+        for (int m = 0; m < NM; ++m) acc[m][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[m], bv, acc[m][mb], 0, 0, 0);
       }
     }
   };
@@ -428,13 +434,20 @@ __device__ __forceinline__ void moe_stream(const MoeOperand<PACKED> (&w)[NM], co
     for (int mb = 0; mb < MB; ++mb) acc[m][mb] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int steps = (K + 31) / 32;
   load(0, 0);
-  for (int s = 0; s < steps; s += 2 * U) {
+  int s = 0;
+  for (; 32 * (s + 2 * U) <= K; s += 2 * U) {
     load(s + U, 1);
     __builtin_amdgcn_sched_barrier(0);
-    multiply(s, 0);
+    multiply(s, 0, std::false_type());
     load(s + 2 * U, 0);
     __builtin_amdgcn_sched_barrier(0);
-    multiply(s + U, 1);
+    multiply(s + U, 1, std::false_type());
+  }
+  if (s < steps) {
+    load(s + U, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(s, 0, std::true_type());
+    multiply(s + U, 1, std::true_type());
   }
 }
 
@@ -569,7 +582,7 @@ __global__ __launch_bounds__(256 * WM, 2) void moe_tiled_kernel(
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) acc[mb][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // what step s needs: a chunk beyond k is any readable one and multiplied by a row of x of zeros
+  // what step s needs (a chunk beyond k is any readable one)
   auto load_x = [&](int s, bf16x8(&to)[2]) {
     const int at = moe_k_at(s, K, g);
 #pragma unroll
@@ -592,15 +605,20 @@ __global__ __launch_bounds__(256 * WM, 2) void moe_tiled_kernel(
   store_x(0, 0, xr[0]);
   __syncthreads();
   // Four steps a round, so that the register sets have fixed names, in one block of code: with an exit between them
-  // the compiler moves the loads behind it, to where their results are used.  (The last round's steps beyond k
-  // multiply by zeros.)
-  for (int i0 = 0; i0 < n_steps; i0 += 4) {
+  // the compiler moves the loads behind it, to where their results are used.  The last round, if k ends inside it, is
+  // code of its own, with zeros in both operands behind k (an infinity of the chunk read instead, times a zero of the
+  // other operand, would be no number).
+  auto round = [&](int i0, auto ends) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int i = i0 + u;
       load_x(i + 2, xr[u % 2]);
       load_w(i + 3, wr[(u + 3) % 4]);
       __builtin_amdgcn_sched_barrier(0);
+      if constexpr (ends.value) {
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) wr[u % 4][nb] = 32 * i + 8 * g < K ? wr[u % 4][nb] : moe_zero8();
+      }
 #pragma unroll
       for (int half = 0; half < 2; ++half) {
         bf16x8 b[4];
@@ -615,7 +633,10 @@ __global__ __launch_bounds__(256 * WM, 2) void moe_tiled_kernel(
       store_x(i + 1, (u + 1) % 2, xr[(u + 1) % 2]);
       __syncthreads();
     }
-  }
+  };
+  int i0 = 0;
+  for (; 32 * (i0 + 4) <= K; i0 += 4) round(i0, std::false_type());
+  if (i0 < n_steps) round(i0, std::true_type());
 
   // acc[mb][nb][i]: the tile's row 128 wm + 16 mb + r16, row 4 g + i of the matrix block nb
 #pragma unroll

@@ -334,3 +334,34 @@ def test_packed_experts_give_the_rows_bits(E, top, T, D, F, tile_rows):
         want[pair[at]] = act[at].float() @ wd[e].float().T
     torch.testing.assert_close(act.float(), torch.nn.functional.silu(gate) * up, rtol=2 ** -7, atol=1e-4)
     torch.testing.assert_close(y, want, rtol=1e-4, atol=1e-4)
+
+
+@pytest.mark.parametrize("E,top,T,D,F", [(3, 2, 40, 72, 40), (4, 2, 300, 296, 168)])
+@pytest.mark.parametrize("tile_rows", [16, 32, 64, 128, 256])
+@pytest.mark.parametrize("packed", [False, True])
+def test_routed_experts_infinite_weights_stay_infinite(E, top, T, D, F, tile_rows, packed):
+    """An infinity among an expert's weights, in the first k (which the kernels read again where a step ends behind k):
+    its output is infinite with the sign of what it meets, not a number that is none; every other output is finite."""
+    from fastgen_amd.kernels import ops
+
+    torch.manual_seed(D)
+    x = torch.randn(T, D, device="cuda").bfloat16()
+    wu, wd = torch.randn(E, F, D, device="cuda").bfloat16(), torch.randn(E, D, F, device="cuda").bfloat16()
+    wg = (torch.randn(E, F, D, device="cuda") / D ** 0.5).bfloat16()
+    wu[:, 5, 0] = float("inf")
+    wd[:, 7, 3] = float("inf")
+    stored = ops.pack_experts if packed else (lambda w: w)
+    choice = torch.stack([torch.randperm(E, device="cuda")[:top] for _ in range(T)]).int()
+    sorted_, tiles = ops.moe_sort(choice, E, tile_rows)
+    act = ops.moe_gate_up(x, stored(wg), stored(wu), sorted_, tiles, top, tile_rows)
+    assert torch.isinf(act[:, 5]).all()
+    other = torch.arange(F, device="cuda") != 5
+    assert torch.isfinite(act[:, other]).all()
+    clean = act.clone()
+    clean[:, 5] = 1
+    y = ops.moe_down(clean, stored(wd), sorted_, tiles, tile_rows)
+    met = torch.empty(T * top, device="cuda")
+    met[sorted_.long()] = clean[:, 3].float()
+    assert torch.equal(y[:, 7], met * float("inf"))
+    other = torch.arange(D, device="cuda") != 7
+    assert torch.isfinite(y[:, other]).all()
