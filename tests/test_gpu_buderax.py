@@ -365,3 +365,15 @@ def test_routed_experts_infinite_weights_stay_infinite(E, top, T, D, F, tile_row
     assert torch.equal(y[:, 7], met * float("inf"))
     other = torch.arange(D, device="cuda") != 7
     assert torch.isfinite(y[:, other]).all()
+
+
+@pytest.mark.parametrize("tile_rows", [128, 256])
+def test_packed_experts_wide_tiles_give_the_rows_bits(tile_rows):
+    """The same where the tiles through LDS are wide (128 x 256 a workgroup of a product, from 170 of them on), at sizes that
+    end inside a wave's columns (32 of gate and up, 64 of down), a step of 32 k and a round of four steps."""
+    from fastgen_amd.kernels import ops
+
+    E, top, T, D, F = 32, 4, 700, 1048, 520
+    tiles = ops.moe_max_tiles(T * top, E, tile_rows)
+    assert tiles * -(-F // 128) >= 170 and tiles * -(-D // 256) >= 170
+    test_packed_experts_give_the_rows_bits(E, top, T, D, F, tile_rows)
