@@ -1322,9 +1322,11 @@ def moe_gate_up(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, sorte
     _i32(tiles, "tiles")
     _need(tiles.dim() == 2 and tiles.shape[1] == 4 and tiles.data_ptr() % 16 == 0, "tiles must be [n, 4], 16-byte aligned")
     hidden, dim = w_gate.shape[1], w_gate.shape[2]
+    if not ldw and (x.data_ptr() % 16 or x.stride(0) % 8):
+        x = x.clone(memory_format=torch.contiguous_format)  # no other kernel reads packed experts
     mfma = _moe_mfma_ok(x, w_gate) and hidden % 8 == 0
     _need(tile_rows in MOE_TILE_ROWS and (mfma or tile_rows == 16), "tile_rows does not fit the kernel")
-    _need(mfma or ldw, "moe_gate_up: packed experts need x and sizes in multiples of 8, 16-byte aligned")
+    _need(mfma or ldw, "moe_gate_up: packed experts need sizes in multiples of 8")
     act = torch.empty((sorted_.numel(), hidden), dtype=x.dtype, device=x.device)
     st = _lib.load("moe").fg_moe_gate_up_act(_ptr(x), x.stride(0), gate, up, ldw, _ptr(sorted_), _ptr(tiles),
                                              tiles.shape[0], tile_rows, top, dim, hidden, _ptr(act), hidden, _code(x),
@@ -1348,7 +1350,7 @@ def moe_down(act: torch.Tensor, w_down: torch.Tensor, sorted_: torch.Tensor, til
     dim, hidden = w_down.shape[1], w_down.shape[2]
     mfma = _moe_mfma_ok(act, w_down)
     _need(tile_rows in MOE_TILE_ROWS and (mfma or tile_rows == 16), "tile_rows does not fit the kernel")
-    _need(mfma or ldw, "moe_down: packed experts need act in multiples of 8, 16-byte aligned")
+    _need(mfma or ldw, "moe_down: packed experts need sizes in multiples of 8, and act 16-byte aligned")
     y = torch.empty((act.shape[0], dim), dtype=torch.float32, device=act.device)
     st = _lib.load("moe").fg_moe_down(_ptr(act), hidden, down, ldw, _ptr(sorted_), _ptr(tiles), tiles.shape[0],
                                       tile_rows, dim, hidden, _ptr(y), _code(act), int(mfma), _stream(act))

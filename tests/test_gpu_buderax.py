@@ -336,6 +336,30 @@ def test_packed_experts_give_the_rows_bits(E, top, T, D, F, tile_rows):
     torch.testing.assert_close(y, want, rtol=1e-4, atol=1e-4)
 
 
+@pytest.mark.parametrize("T", [3, 200])
+def test_routed_experts_take_rows_anywhere(T):
+    """Rows of x whose stride is no multiple of 8: what the same rows give from memory of their own (the experts are packed,
+    and only the matrix-core kernels, which read x 16 bytes at a time, read them).  The router adds such rows' 64
+    products in another order, 64 roundings of 2^-24 each in its logits and so in the experts' weights."""
+    from fastgen_amd.config import PartSpec
+    from fastgen_amd.parts import build_part
+
+    D, E, top, F = 64, 4, 2, 40
+    config = {"width": D, "vocab": 8, "layers": [{"mixer": dict(heads=1, kv_heads=1, dim=8, vdim=8),
+                                                   "mlp": {"router": {"experts": E, "top": top}, "expert": {"ff": F}}}]}
+    part = build_part("feed_forward", PartSpec("moe", "l0.mlp", dict(
+        dim=D, hidden_dim=F, n_experts=E, top=top,
+        names={"router.weight": "router", "router.bias": "router.b", "expert": "e{}", "gate_proj.weight": "gate",
+               "up_proj.weight": "up", "down_proj.weight": "down"})))
+    part.load(plain_buderax_weights(config, 3), torch.bfloat16, DEV)
+    x = torch.randn(T, D).to(DEV, torch.bfloat16)
+    want = part.forward(x)
+    for wide in (D + 3, D + 4):
+        rows = torch.zeros(T, wide, dtype=torch.bfloat16, device=DEV)[:, :D]
+        rows.copy_(x)
+        torch.testing.assert_close(part.forward(rows), want, rtol=1e-5, atol=1e-5)
+
+
 @pytest.mark.parametrize("E,top,T,D,F", [(3, 2, 40, 72, 40), (4, 2, 300, 296, 168)])
 @pytest.mark.parametrize("tile_rows", [16, 32, 64, 128, 256])
 @pytest.mark.parametrize("packed", [False, True])
