@@ -666,14 +666,12 @@ __global__ __launch_bounds__(256, sizeof(TA) == 2 ? 2 : 1) void decay_chunk_outp
   }
 }
 
-extern "C" int fg_decay_chunk_tokens() { return DC; }
-
-// Chunk by chunk as above: d a multiple of 16 up to 128.  `state` [n_slots, H, d, e] is read and left at slot_ids.
+// Chunk by chunk as above: d a multiple of 16 up to 128, chunks of at most chunk_tokens = 64 tokens.  `state` [n_slots, H, d, e] is read and left at slot_ids.
 extern "C" int fg_decay_chunk_scan(const ChunkArgs* args, const int* slot_ids, const int* seq_chunk, float* state,
-                                   int n_chunks, int n_seqs, int act_dtype, hipStream_t stream) {
+                                   int n_chunks, int chunk_tokens, int n_seqs, int act_dtype, hipStream_t stream) {
   if (n_seqs <= 0 || n_chunks <= 0) return FG_OK;
   const ChunkArgs& a = *args;
-  if (a.H <= 0 || a.H > 65535 || a.d <= 0 || a.d % 16 || a.d > 128 || a.e <= 0 || (a.e + 127) / 128 > 65535 || !a.qkv ||
+  if (chunk_tokens != DC || a.H <= 0 || a.H > 65535 || a.d <= 0 || a.d % 16 || a.d > 128 || a.e <= 0 || (a.e + 127) / 128 > 65535 || !a.qkv ||
       !a.logs || !a.chunk_start || !a.states || !a.prod || !a.out)
     return FG_ERR_ARG;
   const dim3 grid(n_chunks, a.H, (a.e + 127) / 128);

@@ -16,6 +16,7 @@ from typing import Any, Dict, Hashable, List, Mapping, Optional, Sequence
 
 import torch
 
+from ..kernels.ops import gemm_f32_scratch
 from ..sampling import Sampler, SamplingParams
 from .context import StepEntry
 from .model import Model
@@ -42,15 +43,19 @@ def step_memory_estimate(model: Model, max_step_tokens: int, max_batch: int) -> 
     """Bytes that one step's intermediate tensors take at most: per token a few rows as wide as the
     widest matrix product of a layer (its output, the activation made from it, the fp32 partial sums
     of the product after it) and the fp32 residual stream; per request a row of fp32 logits, twice
-    (a captured step keeps its own).  (``fastgen/utils/tune.py:46-65`` budgets 1.2 x (4 dim + 4 ffn)
+    (a captured step keeps its own); and the most that a part takes beside that (the states of a recurrence's
+    chunks, the sums over k of a 32-bit product).  (``fastgen/utils/tune.py:46-65`` budgets 1.2 x (4 dim + 4 ffn)
     bytes a token for the same purpose.)"""
-    widest = model.layout.dim
+    widest, scratch = model.layout.dim, 0
     for part in model.parts.all_parts[1:-1]:  # the layers' parts; the embedding and the head are not per token
+        scratch = max(scratch, part.scratch_bytes(max_step_tokens, max_batch))
         for v in vars(part).values():
             shape = getattr(v, "shape", None)  # a tensor or a kernels.linear.StreamedMatrix
             if shape is not None and len(shape) == 2:
                 widest = max(widest, shape[0])
-    return int(max_step_tokens * 12 * widest + 3 * max_batch * model.vocab_size * 4)
+                if v.dtype == torch.float32:
+                    scratch = max(scratch, gemm_f32_scratch(max_step_tokens, *shape))
+    return int(max_step_tokens * 12 * widest + 3 * max_batch * model.vocab_size * 4) + scratch
 
 
 @dataclass

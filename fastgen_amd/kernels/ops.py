@@ -830,6 +830,12 @@ def gemm_f32_plan(M: int, N: int, K: int, cus: int) -> Tuple[int, int, bool]:
     return mb, nb, splits(mb, nb)
 
 
+def gemm_f32_scratch(M: int, N: int, K: int) -> int:
+    """Bytes of the groups' sums that :func:`gemm_nt` takes at most for up to ``M`` rows (see :func:`gemm_f32_plan`)."""
+    groups = -(-K // GEMM_F32_GROUP)
+    return min(groups * min(M, 4096) * N * 4, 256 << 20) if groups > 1 and M > 16 else 0
+
+
 def gemm_nt(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None,
             out_dtype: Optional[torch.dtype] = None) -> torch.Tensor:
     """``x @ w.T`` with ``w [N, K]``, by the engine's own kernels: float32 on the fp32 matrix cores, bfloat16 by
@@ -1797,7 +1803,23 @@ class _DecayChunkArgs(ctypes.Structure):
 
 
 SCAN_CHUNK = 128  # tokens of a chunk where long runs of tokens are scanned chunk by chunk, side by side
+DECAY_CHUNK = 64  # tokens of a chunk that goes through matrix products instead
 SCAN_CHUNKED_FROM = 256  # the shortest run of tokens of one sequence for which a step is scanned so
+
+
+def decay_scan_as_products(d: int) -> bool:
+    """Whether the chunks of long runs go through matrix products, by the key channels of a head."""
+    return d % 16 == 0 and d <= 128
+
+
+def decay_scan_scratch(n_tokens: int, n_seqs: int, H: int, d: int, e: int) -> int:
+    """Bytes that :func:`decay_scan` takes at most for ``n_tokens`` tokens of ``n_seqs`` sequences: the decays, and for
+    every chunk (each sequence's last one may be short) its state and the product of its decays."""
+    if n_tokens < SCAN_CHUNKED_FROM:
+        return 4 * n_tokens * H * d
+    chunk = DECAY_CHUNK if decay_scan_as_products(d) else SCAN_CHUNK
+    chunks = min(n_tokens, n_tokens // chunk + n_seqs)
+    return 4 * H * d * (n_tokens + chunks * (e + 1))
 
 
 def decay_scan(qkv: torch.Tensor, q_col: int, k_col: int, v_col: int, z: torch.Tensor, z_bias: Optional[torch.Tensor],
@@ -1832,7 +1854,7 @@ def decay_scan(qkv: torch.Tensor, q_col: int, k_col: int, v_col: int, z: torch.T
     lib = _lib.load("recurrence")
     lens = np.diff(np.asarray(q_start_host[: n_seqs + 1])) if q_start_host is not None else None
     chunked = lens is not None and len(lens) and int(lens.max()) >= SCAN_CHUNKED_FROM and not torch.cuda.is_current_stream_capturing()
-    products = chunked and d % 16 == 0 and d <= 128
+    products = chunked and decay_scan_as_products(d)
     # the decays of every token at once (exponentials and logarithms stay out of the chain of tokens), or their logarithms
     decay = torch.empty((T, H * d), dtype=torch.float32, device=z.device)
     st = lib.fg_decay_from_logits(_ptr(z), z.stride(0), _ptr(z_bias), ctypes.c_float(1.0 / tau), _ptr(decay), T, H * d,
@@ -1848,7 +1870,7 @@ def decay_scan(qkv: torch.Tensor, q_col: int, k_col: int, v_col: int, z: torch.T
         _check(st, "decay_scan")
         return out
     # chunk by chunk: the chunks' first tokens, and which chunks each sequence has
-    size = lib.fg_decay_chunk_tokens() if products else SCAN_CHUNK
+    size = DECAY_CHUNK if products else SCAN_CHUNK
     starts, seq_chunk = [], [0]
     for b in range(n_seqs):
         starts.extend(range(int(q_start_host[b]), int(q_start_host[b + 1]), size))
@@ -1863,7 +1885,7 @@ def decay_scan(qkv: torch.Tensor, q_col: int, k_col: int, v_col: int, z: torch.T
         chunks = torch.empty((n_chunks, H, d, e), dtype=torch.float32, device=qkv.device)
         c = _DecayChunkArgs(qkv.data_ptr(), qkv.stride(0), q_col, k_col, v_col, decay.data_ptr(), q_scale, chunk_start.data_ptr(),
                             chunks.data_ptr(), prod.data_ptr(), out.data_ptr(), H, d, e)
-        _check(lib.fg_decay_chunk_scan(ctypes.byref(c), _ptr(slot_ids), _ptr(seq_chunk_d), _ptr(state), n_chunks, int(n_seqs),
+        _check(lib.fg_decay_chunk_scan(ctypes.byref(c), _ptr(slot_ids), _ptr(seq_chunk_d), _ptr(state), n_chunks, size, int(n_seqs),
                                        _code(qkv), _stream(qkv)), "decay_scan (chunks as products)")
         return out
     chunks = torch.zeros((n_chunks, H, d, e), dtype=torch.float32, device=qkv.device)

@@ -117,6 +117,11 @@ class Part:
     def load(self, tensors: Mapping[str, torch.Tensor], dtype: torch.dtype, device: Any) -> None:
         pass
 
+    def scratch_bytes(self, n_tokens: int, n_requests: int) -> int:
+        """Bytes that ``forward`` takes at most, for a step of so many tokens of so many requests, beside a few rows a
+        token as wide as its products: what the room for the cache has to leave free."""
+        return 0
+
 
 class Mixer(Part):
     """A token mixer: rows in, rows out, with storage per token or per request.

@@ -68,6 +68,9 @@ class GatedLinearAttention(Mixer):
     def state_need(self) -> StateNeed:
         return StateNeed((self.n_heads, self.head_dim, self.v_head_dim), torch.float32)
 
+    def scratch_bytes(self, n_tokens: int, n_requests: int) -> int:
+        return ops.decay_scan_scratch(n_tokens, n_requests, self.n_heads, self.head_dim, self.v_head_dim)
+
     def forward(self, x: torch.Tensor, ctx: Any, store: LayerStore) -> torch.Tensor:
         H, d, e, low = self.n_heads, self.head_dim, self.v_head_dim, self.decay_rank
         T = x.shape[0]

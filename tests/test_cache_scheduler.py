@@ -633,3 +633,43 @@ def test_step_memory_estimate_sees_the_widest_product():
     widest = 2 * TINY_A["intermediate_size"]
     assert widest > TINY_A["hidden_size"]
     assert step_memory_estimate(model, 100, 4) == 100 * 12 * widest + 3 * 4 * TINY_A["vocab_size"] * 4
+
+
+def test_step_memory_estimate_counts_what_parts_take_beside_their_rows():
+    """The states of the chunks that a long prompt's recurrence goes through (64 tokens each where the head size lets them
+    be matrix products, else 128; every sequence's last one may be short), and the sums over k of 32-bit products that are
+    cut over workgroups (at most 256 MB; none where k is one group)."""
+    from types import SimpleNamespace
+
+    import torch
+
+    from fastgen_amd.config import PartSpec
+    from fastgen_amd.engine.engine import step_memory_estimate
+    from fastgen_amd.kernels import ops
+    from fastgen_amd.parts import build_part
+
+    def part(H, d, e):
+        return build_part("mixer", PartSpec("gated_linear_attention", "l0", dict(
+            dim=64, n_heads=H, head_dim=d, v_head_dim=e, tau=16.0, decay_rank=8, eps=1e-6)))
+
+    def estimate(*parts):
+        return step_memory_estimate(SimpleNamespace(layout=SimpleNamespace(dim=64), vocab_size=100, parts=SimpleNamespace(
+            all_parts=[None, *parts, None])), 8192, 4)
+
+    plain = 8192 * 12 * 64 + 3 * 4 * 100 * 4
+    assert estimate() == plain
+    for d, chunk in ((128, 64), (48, 64), (136, 128), (24, 128)):
+        chunks = sum(-(-n // chunk) for n in (8192 - 3 * 65, 65, 65, 65))  # what such a step takes
+        taken = 4 * 64 * d * (8192 + chunks * (256 + 1))
+        got = estimate(part(2, d, 8), part(64, d, 256)) - plain
+        assert taken <= got <= taken * 1.05
+    narrow, wide = torch.empty(64, 1024), torch.empty(64, 1025)
+    weights = lambda w: SimpleNamespace(w=w, scratch_bytes=lambda *_: 0)
+    assert estimate(weights(narrow)) == plain
+    assert estimate(weights(wide)) == plain + 2 * 4096 * 64 * 4
+    assert estimate(weights(wide.bfloat16())) == plain
+    cus = 256
+    for M in (17, 400, 2048, 4096, 4097, 8192):
+        for N, K in ((64, 1025), (3072, 8192), (16384, 3072), (28672, 8192)):
+            if ops.gemm_f32_plan(M, N, K, cus)[2]:
+                assert -(-K // ops.GEMM_F32_GROUP) * M * N * 4 <= ops.gemm_f32_scratch(8192, N, K)
