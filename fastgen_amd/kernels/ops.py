@@ -810,19 +810,23 @@ def gemm_f32_plan(M: int, N: int, K: int, cus: int) -> Tuple[int, int, bool]:
     """How the 32-bit product is cut: (tile rows / 32, tile columns / 32, whether every group of k has a workgroup
     of its own); (0, 0, False): the kernel of up to 16 rows.  Every cut gives the same bits.
 
-    Measured on 256 compute units (us; N x K 3072 x 3072, 16384 x 3072, 3072 x 8192).  Tiles of 64 x 64 while they
-    give 600 workgroups (2048 rows: 374, 1883, 975 against 401, 2098, 1051 with 64 x 32), smaller ones below (64 rows,
-    64 x 64 / 64 x 32 / 32 x 32: 40 / 36 / 33, 77 / 81 / 90, 60 / 51 / 54); 32 rows where the last tile of 64 would be
-    at least half empty (200 rows: 59, 247, 140 against 75, 252, 143).  A workgroup a group of k while whole ranges
-    would be fewer than 1536 workgroups (400 rows: 103 against 112, 239 against 289; 16384 x 3072, 3328
-    workgroups: 447 against 440), if the groups' sums stay under 256 MB."""
+    Measured on 256 compute units, matrices from memory (us; N x K 3072 x 3072, 16384 x 3072, 3072 x 8192).  The kernel of
+    up to 16 rows against tiles of 32 x 32 cut over k: 12 rows 19 / 58 / 40 against 31 / 55 / 39, 16 rows 20 / 62 / 43
+    against 31 / 55 / 39.  Tiles of 64 x 64 while they give 600 workgroups (2048 rows: 374, 1883, 975 against 401, 2098,
+    1051 with 64 x 32), smaller ones below (64 rows, 64 x 64 / 64 x 32 / 32 x 32: 40 / 36 / 33, 77 / 81 / 90, 60 / 51 /
+    54).  Tiles of 32 rows where the last one of 64 would be at least half empty, up to 640 rows, the better of each cut
+    over k or not (200 rows 63, 249, 145 against 77, 252, 147; 400: 105, 440, 238 against 97, 435, 245; 528: 125, 567,
+    305 against 136, 554, 303); not beyond (784: 175, 827, 439 against 177, 785, 424; 1040: 224, 1095, 568 against 220, 1018,
+    542; 2050: 438, 2124, 1151 against 427, 1957, 1135; 4110: 823, 4183, 2193 against 779, 3812, 2078).  A workgroup a
+    group of k while whole ranges would be fewer than 1536 workgroups (400 rows of 32: 105 against 116, 238 against 294;
+    16384 x 3072, 3328 workgroups: 453 against 440), if the groups' sums stay under 256 MB."""
     if M <= 16:
         return 0, 0, False
     groups = -(-K // GEMM_F32_GROUP)
     tiles = lambda mb, nb: -(-M // (32 * mb)) * -(-N // (32 * nb))
     splits = lambda mb, nb: groups > 1 and tiles(mb, nb) < 6 * cus and M <= 4096 and groups * M * N * 4 <= 256 << 20
     units = lambda mb, nb: tiles(mb, nb) * (groups if splits(mb, nb) else 1)
-    mb, nb = (1 if 0 < M % 64 <= 32 else 2), 2
+    mb, nb = (1 if 0 < M % 64 <= 32 and M <= 640 else 2), 2
     if units(mb, nb) < 600 * cus // 256:
         nb = 1
     if units(mb, nb) < 600 * cus // 256:

@@ -411,6 +411,16 @@ def test_gemm_f32_every_cut_gives_the_same_bits(ops, N, K):
         assert torch.equal(ops.gemm_nt(x[first:last], w), full[first:last]), (first, last)
 
 
+@pytest.mark.parametrize("N,K", [(130, 1100), (3072, 1028)])
+def test_gemm_f32_bits_around_the_line_of_the_narrow_tiles(ops, N, K):
+    """Up to 640 rows a last tile of at most 32 rows makes all tiles that narrow, beyond it does not: the same bits."""
+    torch.manual_seed(N)
+    x, w = torch.randn(720, K).to(DEV), torch.randn(N, K).to(DEV)
+    full = ops.gemm_nt(x, w)
+    for M in (16, 608, 609, 640, 641, 672, 673):
+        assert torch.equal(ops.gemm_nt(x[:M], w), full[:M]), M
+
+
 def test_gemm_f32_plan_is_bounded(ops):
     for M in (1, 16, 17, 64, 65, 400, 4096, 4097, 200000):
         for N in (1, 64, 3072, 128256):
