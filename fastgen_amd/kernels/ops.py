@@ -1304,14 +1304,16 @@ def _moe_mfma_ok(x: torch.Tensor, *weights) -> bool:
             and all(isinstance(w, PackedExperts) or (w.shape[2] % 8 == 0 and w.data_ptr() % 16 == 0) for w in weights))
 
 
+def _experts_data(w) -> torch.Tensor:
+    return w.data if isinstance(w, PackedExperts) else w
+
+
 def _experts_args(w, what: str):
     """C arguments (pointer, ldw) for the experts' matrices, contiguous ``[E, n, k]`` or :class:`PackedExperts` (ldw = 0)."""
     if isinstance(w, PackedExperts):
-        _gpu(w.data)
         _need(w.data.is_contiguous() and w.data.data_ptr() % 16 == 0
               and w.data.shape[1:] == (-(-w.n // 16), -(-w.k // 32), 64, 8), f"{what}: the packed experts do not fit their sizes")
         return _ptr(w.data), 0
-    _gpu(w)
     _need(w.dim() == 3 and w.is_contiguous(), f"{what}: the experts' matrices must be contiguous [E, n, k]")
     return _ptr(w), w.shape[2]
 
@@ -1323,7 +1325,7 @@ def moe_gate_up(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, sorte
     ``g * sigmoid(alpha * g) * (u + 1)``.
     ``w_gate``, ``w_up``: ``[E, hidden, dim]`` of ``x``'s dtype, or both :class:`PackedExperts`.  bfloat16 with sizes in
     multiples of 8 runs on the matrix cores; everything else the fp32-FMA kernel (tiles of 16 rows only)."""
-    _gpu(x, sorted_, tiles)
+    _gpu(x, _experts_data(w_gate), _experts_data(w_up), sorted_, tiles)
     (gate, ldw), (up, ldu) = _experts_args(w_gate, "moe_gate_up"), _experts_args(w_up, "moe_gate_up")
     _need(x.dim() == 2 and x.stride(1) == 1 and w_gate.shape == w_up.shape and w_gate.shape[2] == x.shape[1]
           and w_gate.dtype == x.dtype == w_up.dtype and ldw == ldu,
@@ -1350,7 +1352,7 @@ def moe_down(act: torch.Tensor, w_down: torch.Tensor, sorted_: torch.Tensor, til
              tile_rows: int) -> torch.Tensor:
     """``act_p W_down[e]^T`` for every pair as fp32 ``[T * top, dim]``, row = pair (not the sorted order).
     ``w_down``: ``[E, dim, hidden]`` of ``act``'s dtype, or :class:`PackedExperts`."""
-    _gpu(act, sorted_, tiles)
+    _gpu(act, _experts_data(w_down), sorted_, tiles)
     down, ldw = _experts_args(w_down, "moe_down")
     _need(act.dim() == 2 and act.is_contiguous() and w_down.shape[2] == act.shape[1] and w_down.dtype == act.dtype,
           "act contiguous [pairs, hidden], w_down [E, dim, hidden] of act's dtype")

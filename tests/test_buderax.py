@@ -112,3 +112,23 @@ def test_twins_of_the_routed_experts_are_the_plain_mixture():
     assert torch.allclose(plain_expert(n[:1], w["l1.mlp.e0.gate"], w["l1.mlp.e0.up"], w["l1.mlp.e0.down"]),
                           (torch.nn.functional.silu(n[:1] @ w["l1.mlp.e0.gate"].T) * (n[:1] @ w["l1.mlp.e0.up"].T))
                           @ w["l1.mlp.e0.down"].T)
+
+
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("elsewhere", ["gate", "up", "down"])
+def test_routed_products_refuse_experts_on_another_device(packed, elsewhere):
+    """The experts' matrices have to lie on the rows' device, however they are stored (stand-ins: one GPU or none is
+    enough, nothing is launched)."""
+    from types import SimpleNamespace
+
+    from fastgen_amd.kernels import ops
+
+    on = lambda device: SimpleNamespace(is_cuda=True, device=device, dtype=torch.bfloat16, dim=lambda: 5, shape=(2, 1, 1, 64, 8))
+    here, there = on("cuda:0"), on("cuda:1")
+    matrix = lambda which: ops.PackedExperts(there if which == elsewhere else here, 16, 32) if packed else (
+        there if which == elsewhere else here)
+    with pytest.raises(ops.KernelArgumentError, match="different devices"):
+        if elsewhere == "down":
+            ops.moe_down(here, matrix("down"), here, here, 16)
+        else:
+            ops.moe_gate_up(here, matrix("gate"), matrix("up"), here, here, 2, 16)
