@@ -9,7 +9,7 @@ is not on a GPU is refused.
 from __future__ import annotations
 
 import ctypes
-from dataclasses import dataclass
+from dataclasses import dataclass, field
 import os
 from typing import Dict, List, Optional, Sequence, Tuple
 
@@ -1266,7 +1266,7 @@ def moe_sort(choice: torch.Tensor, n_experts: int, tile_rows: int, n_identity: i
     return sorted_, tiles
 
 
-@dataclass
+@dataclass(frozen=True)
 class PackedExperts:
     """The experts' bfloat16 matrices ``[E, n, k]``, each in the order of :class:`PackedWeight`: ``data [E,
     ceil(n / 16), ceil(k / 32), 64, 8]``.  Every kernel that takes a bfloat16 expert reads this order, so it is
@@ -1275,14 +1275,15 @@ class PackedExperts:
     data: torch.Tensor
     n: int
     k: int
+    # the matrices' own, computed once: a step asks for them several times a layer
+    shape: torch.Size = field(init=False, repr=False)
+    dtype: torch.dtype = field(init=False, repr=False)
 
-    @property
-    def shape(self):
-        return torch.Size((self.data.shape[0], self.n, self.k))
-
-    @property
-    def dtype(self) -> torch.dtype:
-        return self.data.dtype
+    def __post_init__(self) -> None:
+        _need(self.data.dim() == 5 and self.data.shape[1:] == (-(-self.n // 16), -(-self.k // 32), 64, 8),
+              "the packed experts do not fit their sizes")
+        object.__setattr__(self, "shape", torch.Size((self.data.shape[0], self.n, self.k)))
+        object.__setattr__(self, "dtype", self.data.dtype)
 
 
 def pack_experts(w: torch.Tensor) -> PackedExperts:
@@ -1299,22 +1300,21 @@ def pack_experts(w: torch.Tensor) -> PackedExperts:
     return PackedExperts(data, n, k)
 
 
-def _moe_mfma_ok(x: torch.Tensor, *weights) -> bool:
+def _moe_mfma_ok(x: torch.Tensor, w) -> bool:
     return (x.dtype == torch.bfloat16 and x.shape[1] % 8 == 0 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
-            and all(isinstance(w, PackedExperts) or (w.shape[2] % 8 == 0 and w.data_ptr() % 16 == 0) for w in weights))
+            and (isinstance(w, PackedExperts) or (w.shape[2] % 8 == 0 and w.data_ptr() % 16 == 0)))
 
 
 def _experts_data(w) -> torch.Tensor:
     return w.data if isinstance(w, PackedExperts) else w
 
 
-def _experts_args(w, what: str):
+def _experts_args(w):
     """C arguments (pointer, ldw) for the experts' matrices, contiguous ``[E, n, k]`` or :class:`PackedExperts` (ldw = 0)."""
     if isinstance(w, PackedExperts):
-        _need(w.data.is_contiguous() and w.data.data_ptr() % 16 == 0
-              and w.data.shape[1:] == (-(-w.n // 16), -(-w.k // 32), 64, 8), f"{what}: the packed experts do not fit their sizes")
+        _need(w.data.is_contiguous() and w.data.data_ptr() % 16 == 0, "packed experts must be contiguous, 16-byte aligned")
         return _ptr(w.data), 0
-    _need(w.dim() == 3 and w.is_contiguous(), f"{what}: the experts' matrices must be contiguous [E, n, k]")
+    _need(w.dim() == 3 and w.is_contiguous(), "the experts' matrices must be contiguous [E, n, k]")
     return _ptr(w), w.shape[2]
 
 
@@ -1326,7 +1326,7 @@ def moe_gate_up(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, sorte
     ``w_gate``, ``w_up``: ``[E, hidden, dim]`` of ``x``'s dtype, or both :class:`PackedExperts`.  bfloat16 with sizes in
     multiples of 8 runs on the matrix cores; everything else the fp32-FMA kernel (tiles of 16 rows only)."""
     _gpu(x, _experts_data(w_gate), _experts_data(w_up), sorted_, tiles)
-    (gate, ldw), (up, ldu) = _experts_args(w_gate, "moe_gate_up"), _experts_args(w_up, "moe_gate_up")
+    (gate, ldw), (up, ldu) = _experts_args(w_gate), _experts_args(w_up)
     _need(x.dim() == 2 and x.stride(1) == 1 and w_gate.shape == w_up.shape and w_gate.shape[2] == x.shape[1]
           and w_gate.dtype == x.dtype == w_up.dtype and ldw == ldu,
           "x [T, dim], w_gate and w_up [E, hidden, dim] of x's dtype, stored alike")
@@ -1353,7 +1353,7 @@ def moe_down(act: torch.Tensor, w_down: torch.Tensor, sorted_: torch.Tensor, til
     """``act_p W_down[e]^T`` for every pair as fp32 ``[T * top, dim]``, row = pair (not the sorted order).
     ``w_down``: ``[E, dim, hidden]`` of ``act``'s dtype, or :class:`PackedExperts`."""
     _gpu(act, _experts_data(w_down), sorted_, tiles)
-    down, ldw = _experts_args(w_down, "moe_down")
+    down, ldw = _experts_args(w_down)
     _need(act.dim() == 2 and act.is_contiguous() and w_down.shape[2] == act.shape[1] and w_down.dtype == act.dtype,
           "act contiguous [pairs, hidden], w_down [E, dim, hidden] of act's dtype")
     _i32(sorted_, "sorted", act.shape[0])
