@@ -239,6 +239,7 @@ def _buderax_kernels(z: dict, rows: int) -> dict:
 
     from fastgen_amd.kernels import ops
     from fastgen_amd.kernels.linear import linear
+    from fastgen_amd.parts.moe import expert_tile_rows
 
     D, E, top, F = z["width"], z["experts"], z["top"], z["ff"]
     g = torch.Generator(device="cuda").manual_seed(rows)
@@ -246,8 +247,8 @@ def _buderax_kernels(z: dict, rows: int) -> dict:
     x = rnd(rows, D) * 20
     router, bias = rnd(E, D).float(), rnd(E).float()
     wg, wu, wd = rnd(E, F, D), rnd(E, F, D), rnd(E, D, F)
-    per_expert = rows * top / E
-    tile_rows = next((r for r, least in ((256, 768), (128, 96), (64, 48), (32, 24)) if per_expert >= least), 16)
+    tile_rows = expert_tile_rows(rows * top / E, min(D, F))
+    wg, wu, wd = (ops.pack_experts(w) for w in (wg, wu, wd))  # as a model keeps them
     choice, weight = ops.moe_route(x, router, bias, top)
     sorted_, tiles = ops.moe_sort(choice, E, tile_rows)
     act = ops.moe_gate_up(x, wg, wu, sorted_, tiles, top, tile_rows)
@@ -721,6 +722,7 @@ def _sodotar_kernels(z: dict, rows: int, context: int) -> dict:
     import torch
 
     from fastgen_amd.kernels import ops
+    from fastgen_amd.parts.moe import expert_tile_rows
 
     D, H, G, d, P, S = z["width"], z["heads"], z["kv_heads"], z["dim"], PAGE, z["streams"]
     Hd, Gd, e = H // 2, G // 2, 2 * d  # the differential layer: heads, key/value heads, value width
@@ -805,9 +807,9 @@ def _sodotar_kernels(z: dict, rows: int, context: int) -> dict:
     put("moe_route (buderax)", lambda: ops.moe_route(xr, r2, None, top), r2.numel() * 4 + rows * D * 2)
     # the experts' first product with the limited activation, beside the same with SiLU
     choice, _ = ops.moe_route(xr, r2, None, top)
-    tile_rows = 16 if decode else (128 if rows * top / E >= 96 else 64)
+    tile_rows = expert_tile_rows(rows * top / E, D)
     sorted_, tiles = ops.moe_sort(choice, E, tile_rows)
-    wg, wu = rnd(E, F, D), rnd(E, F, D)
+    wg, wu = ops.pack_experts(rnd(E, F, D)), ops.pack_experts(rnd(E, F, D))  # as a model keeps them
     used = min(E, rows * top)
     put("moe_gate_up (limited)", lambda: ops.moe_gate_up(xr, wg, wu, sorted_, tiles, top, tile_rows, 7.0, 1.702),
         used * 2 * F * D * 2, 2 * rows * top * 2 * F * D)

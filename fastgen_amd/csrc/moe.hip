@@ -20,7 +20,8 @@
 // The matrix-core kernels take the experts' matrices row by row or packed (ldw = 0): per expert blocks of 16 rows x
 // 32 k in operand order, [expert][ceil(rows / 16)][ceil(k / 32)][64 lanes][8], zeros behind the last row and k.  A
 // wave's load is then 1 KB of whole lines; from rows it is 16 halves of a line, and the other halves are asked for
-// again a step later.
+// again a step later.  A model keeps its experts packed and takes tiles of 16, 32 and 128 rows; matrices in rows and
+// tiles of 64 and 256 rows, nowhere the better ones, are there for callers of the products that hand them over so.
 #include "common.h"
 
 #include <type_traits>
@@ -537,8 +538,8 @@ __global__ __launch_bounds__(256) void moe_down_mfma_kernel(
 // matrix three; one barrier a step.  1897 tokens, 32 experts of 768 x 2048, top 4 (237 rows an expert, 48 + 24 GFLOP): 86 /
 // 67 us, 116 / 83 with the matrices in rows, 150 / 87 with tiles of 64 x 64 a wave; 6000 tokens 182 / 142 us against 344 /
 // 210, 0.83 / 0.53 PFLOP/s.  The tile's rows are gathered by token (gate_up) or are its sorted places (down);
-// for gate_up a block of 16 matrix rows is 8 gate rows and the 8 up rows of the same channels, so that silu(gate) * up is
-// applied to the accumulators.
+// for gate_up the first half of a wave's blocks of 16 matrix rows are gate rows and the second half the up rows of the
+// same channels, so that silu(gate) * up is applied to the accumulators.
 #define MT_GATE_UP 0
 #define MT_DOWN 1
 #define MT_RUN 4

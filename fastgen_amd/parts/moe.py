@@ -37,6 +37,19 @@ from ..config.layout import PartSpec
 from .base import MATRIX, VECTOR, FeedForward, TensorSpec, build_part, place, register_part
 
 
+def expert_tile_rows(per_expert: float, least_k: int) -> int:
+    """Rows of one expert a tile of the matrix-core kernels holds, by the rows an expert gets on average and the smaller
+    of the two products' k: 16 for few rows (decode: an expert's matrices are read once for its rows), 32 and 128
+    where the experts get so many rows each that their matrices would otherwise be read many times over; from 128 on
+    the rows of x go through LDS, k in steps of 32.  Measured (us, gate_up + down, packed, 32 experts of 768 x 2048, top 4;
+    tiles of 16 / 32 / 64 / 128 rows): 12 rows an expert 72 / 74 / 84 / -, 19: 95 / 81 / 91 / -, 25: 112 / 88 / 94 / 68,
+    50: 150 / 128 / 130 / 73, 237 (tiles of 256 rows 165): - / - / 434 / 153; 16 experts of 704 x 1024, top 2: 19: 37 / 28 /
+    31 / -, 25: 40 / 34 / 34 / 36, 50: 54 / 47 / 44 / 39."""
+    if per_expert >= 24 and least_k >= 32:
+        return 128
+    return 32 if per_expert >= 14 else 16
+
+
 class MoE(FeedForward):
     adds_to = True  # ``forward(x, plus=rows)`` returns plus + its own output, as fp32 [1, T, dim]
 
@@ -139,19 +152,9 @@ class MoE(FeedForward):
         self.w_gate, self.w_up, self.w_down = stored(gate), stored(up), stored(down)
 
     def tile_rows(self, n_rows: int) -> int:
-        """Rows of one expert a tile holds: 16 for few rows (decode: an expert's matrices are read once for its
-        rows), 32 and 128 where the experts get so many rows each that their matrices would otherwise be read many
-        times over; from 128 on the rows of x go through LDS (the matrix-core kernels only).  Measured (us, gate_up
-        + down, 32 experts of 768 x 2048, top 4; tiles of 16 / 32 / 64 / 128 rows): 12 rows an expert 72 / 74 / 84 / -,
-        19: 95 / 81 / 91 / -, 25: 112 / 88 / 94 / 68, 50: 150 / 128 / 130 / 73, 237 (tiles of 256 rows 165): - / - /
-        434 / 153; 16 experts of 704 x 1024, top 2: 19: 37 / 28 / 31 / -, 25: 40 / 34 / 34 / 36, 50: 54 / 47 / 44 / 39."""
         if self.w_gate.dtype != torch.bfloat16 or self.dim % 8:
             return 16
-        per_expert = n_rows * self.top / self.n_scored
-        lds_ok = min(self.dim, self.w_down.shape[2]) >= 32  # the tiles through LDS load k in steps of 32
-        if per_expert >= 24 and lds_ok:
-            return 128
-        return 32 if per_expert >= 14 else 16
+        return expert_tile_rows(n_rows * self.top / self.n_scored, min(self.dim, self.w_down.shape[2]))
 
     def forward(self, x: torch.Tensor, plus: Optional[torch.Tensor] = None) -> torch.Tensor:
         """fp32 ``[1, T, dim]``: the experts' weighted sum (plus ``plus``, rows that go to the
