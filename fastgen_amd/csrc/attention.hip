@@ -163,6 +163,18 @@ __global__ __launch_bounds__(ATT_WAVES* FG_WAVE) void paged_attention_general_ke
 // takes eight runs, one a wave, which keeps the scores of its tiles in LDS until it knows the rows' maxima and then does
 // what the eight waves' merge does, operation for operation: the same bits, so the choice is free to follow the load.
 //
+// A run of one tile (the first 64 places of a sequence) is where a workgroup of eight waves is most of it idle.  If there may
+// be many, a kernel of its own takes them, a wave a run of up to 16 rows: it needs no sums but a block's, so its loads are
+// 2 to 7 blocks of 16 dims ahead and several waves share a SIMD, and it leaves out the blocks of 16 keys behind the run's
+// last, which bring zeros.  The same operations otherwise, the same bits.  us, (token, head) by (token, head) / without
+// that kernel / with it, heads / kv heads x head size:
+//                            32/8x128          32/32x128         16/16x64         16/1x80          16/4x256         8/8x512
+//   64 prompts of 5      24 /  65 /  26    28 / 140 /  62    10 / 52 / 28    11 / 27 / 13    21 /  64 /  22    39 / 144 / 37
+//   8 of 37              34 /  51 /  29    35 /  81 /  54    14 / 36 / 28    17 / 28 / 20    32 /  50 /  36    60 / 109 / 55
+//   20 of 60            142 / 162 /  67   146 / 311 / 196    47 /103 / 71    61 / 66 / 29   134 / 127 /  62
+//   300 decoded, 9 keys  35 /  43 /  29    37 / 130 /  96    14 / 45 / 42    13 / 27 / 13    29 /  35 /  25    49 / 171 / 66
+// What is left to the first column is mostly the workgroups that find no run of theirs (9600 of 8 waves: 46 us).
+//
 // Bound by the latency of a tile's loads in each wave (the next block of 16 dims in flight while one is multiplied; more
 // of them in flight cost the registers) and, for long sequences, by the pages' reads.  Before: a wave a (token, head), a
 // lane a key (`paged_attention_general_kernel`).  us, before and now (heads / kv heads x head size):
@@ -198,25 +210,43 @@ struct AfArgs {
   float scale; int window;
   const float *sinks, *dist;
   int few_runs;  // how many runs of few rows there may be: one a sequence and kv head
+  int ones;      // whether runs of one tile are another kernel's
 };
 
 struct AfRun {
   int t0, n_here, seq, kvh, p_lo, p_hi;  // its tokens, and their lowest and highest position
   int lo;                                // keys lo .. p_hi are seen by some row: their pages are held
 };
-// The run that starts at place `index` of the grid; false: none does.  Uniform.
-// (The blocks' first tokens come first, a token's kv heads side by side: every die gets as many of them.)
-__device__ __forceinline__ bool af_run(const AfArgs& a, int index, AfRun& run) {
-  const int full = 16 / (a.n_heads / a.n_kv), blocks = (a.n_tokens + full - 1) / full, place = index / a.n_kv;
-  if (place >= blocks * full) return false;
-  const int t0 = place % blocks * full + place / blocks;
-  if (t0 >= a.n_tokens) return false;
-  const int seq = a.seq_of_token[t0];
-  if (t0 % full && a.seq_of_token[t0 - 1] == seq) return false;  // an earlier run holds this token
-  run.t0 = t0, run.seq = seq, run.kvh = index % a.n_kv, run.n_here = 1;
-  run.p_lo = run.p_hi = a.positions[t0];
-  for (; t0 + run.n_here < a.n_tokens && (t0 + run.n_here) % full && a.seq_of_token[t0 + run.n_here] == seq; ++run.n_here) {
-    const int p = a.positions[t0 + run.n_here];
+// A block's tokens, one a lane, and which of them start a run (bit i: token i).
+struct AfBlock {
+  int t0, n, seq, pos;
+  unsigned starts;
+};
+__device__ __forceinline__ AfBlock af_block(const AfArgs& a, int block, int lane) {
+  const int full = 16 / (a.n_heads / a.n_kv);
+  AfBlock k;
+  k.t0 = block * full;
+  k.n = min(full, a.n_tokens - k.t0);
+  const int t = k.t0 + min(lane, k.n - 1);
+  k.seq = a.seq_of_token[t];
+  k.pos = a.positions[t];
+  const int before = __shfl_up(k.seq, 1, FG_WAVE);
+  k.starts = (unsigned)__ballot(lane < k.n && (lane == 0 || before != k.seq));
+  return k;
+}
+// Run j of a block for a kv head; false: there are not so many.  Uniform.
+__device__ __forceinline__ bool af_run(const AfArgs& a, const AfBlock& k, int kvh, int j, AfRun& run) {
+  unsigned rest = k.starts;
+  for (; j > 0 && rest; --j) rest &= rest - 1;
+  if (!rest) return false;
+  const int at = __ffs(rest) - 1;
+  rest &= rest - 1;
+  const int end = rest ? __ffs(rest) - 1 : k.n;
+  run.t0 = k.t0 + at, run.n_here = end - at, run.kvh = kvh;
+  run.seq = __builtin_amdgcn_readlane(k.seq, at);
+  run.p_lo = run.p_hi = __builtin_amdgcn_readlane(k.pos, at);
+  for (int i = at + 1; i < end; ++i) {
+    const int p = __builtin_amdgcn_readlane(k.pos, i);
     run.p_lo = min(run.p_lo, p);
     run.p_hi = max(run.p_hi, p);
   }
@@ -224,11 +254,17 @@ __device__ __forceinline__ bool af_run(const AfArgs& a, int index, AfRun& run) {
   return true;
 }
 
-// Whether a wave alone takes the run.
+// Who takes a run: a workgroup, or a wave that keeps its scores in LDS; or, where that is launched, a wave of the kernel
+// for runs of one tile.
+enum { AF_TOGETHER, AF_ALONE, AF_ONE };
+// (at the largest head sizes the queries' room in LDS, and a wave's time for more keys, are too much)
+__host__ __device__ constexpr int af_one_rows(int db) { return db <= 16 ? 16 : 8; }
+__host__ __device__ constexpr int af_one_blocks(int db) { return db <= 16 ? 4 : 2; }  // of 16 keys
 template <int DB>
-__device__ __forceinline__ bool af_alone(const AfArgs& a, const AfRun& run) {
-  const int tiles = run.p_hi / ATT_TILE - run.lo / ATT_TILE + 1;
-  return run.n_here * (a.n_heads / a.n_kv) <= AF_ALONE_ROWS && tiles <= AF_WAVES && a.few_runs >= af_alone_from(DB, tiles);
+__device__ __forceinline__ int af_kind(const AfArgs& a, const AfRun& run) {
+  const int tiles = run.p_hi / ATT_TILE - run.lo / ATT_TILE + 1, rows = run.n_here * (a.n_heads / a.n_kv);
+  if (a.ones && tiles == 1 && rows <= af_one_rows(DB) && run.p_hi % ATT_TILE / 16 < af_one_blocks(DB)) return AF_ONE;
+  return rows <= AF_ALONE_ROWS && tiles <= AF_WAVES && a.few_runs >= af_alone_from(DB, tiles) ? AF_ALONE : AF_TOGETHER;
 }
 
 // Lane 16 g + r's row r: a token of the run and one of its heads (rows behind the last see no key and are not stored).
@@ -272,44 +308,45 @@ __device__ __forceinline__ void af_queries(const AfArgs& a, const AfRun& run, f3
 
 // Scores of the tile's keys 16 b + 4 g + e with the lane's row (-infinity where the row does not see the key), and the
 // row's highest.
-template <int DB, int N>
+template <int DB, int AHEAD, int N, int NB>
 __device__ __forceinline__ float af_scores(const AfArgs& a, const AfRun& run, const AfRow& row, const KvLayout& lay, int tile,
-                                           const f32x4 (*q_s)[N], int q_row, int r, int g, f32x4 (&s)[4]) {
+                                           const f32x4 (*q_s)[N], int q_row, int r, int g, f32x4 (&s)[NB]) {
   const int kb = tile * ATT_TILE;
   const int* table = a.block_table + (size_t)run.seq * a.bt_stride;
-  const float* kp[4];
+  const float* kp[NB];
 #pragma unroll
-  for (int b = 0; b < 4; ++b) {  // (keys that no row sees are read as the nearest one that some row does)
+  for (int b = 0; b < NB; ++b) {  // (keys that no row sees are read as the nearest one that some row does)
     const int key = min(max(kb + 16 * b + r, run.lo), run.p_hi);
     kp[b] = a.k_pages + ((size_t)table[key / a.page_size] * a.n_kv + run.kvh) * ((size_t)a.page_size * a.hd) +
             lay.k_off(key % a.page_size, 0);
     s[b] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
   const size_t chunk = (size_t)8 << lay.kb_shift;  // from 8 head dims of a key to the next 8
-  // The next block of 16 dims is asked for before this one is multiplied, and never conditionally: behind the head's dims
-  // its first ones, for zeros.
-  f32x4 kv[2][4];
+  // The next blocks of 16 dims are asked for before this one is multiplied, and never conditionally: behind the head's
+  // dims its first ones, for zeros.
+  f32x4 kv[AHEAD + 1][NB];
   auto load = [&](int i) {
     const size_t at = 16 * i + 4 * g < a.hd ? chunk * (2 * i + g / 2) + g % 2 * 4 : 0;
 #pragma unroll
-    for (int b = 0; b < 4; ++b) kv[i % 2][b] = *(const f32x4*)(kp[b] + at);
+    for (int b = 0; b < NB; ++b) kv[i % (AHEAD + 1)][b] = *(const f32x4*)(kp[b] + at);
   };
-  load(0);
+#pragma unroll
+  for (int i = 0; i < AHEAD && i < DB; ++i) load(i);
 #pragma unroll
   for (int i = 0; i < DB; ++i) {
-    if (i + 1 < DB) load(i + 1);
+    if (i + AHEAD < DB) load(i + AHEAD);
     __builtin_amdgcn_sched_barrier(0);
     const f32x4 qv = q_s[4 * i + g][q_row];
     const bool in = 16 * i + 4 * g < a.hd;
 #pragma unroll
     for (int e = 0; e < 4; ++e)
 #pragma unroll
-      for (int b = 0; b < 4; ++b)
-        s[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? kv[i % 2][b][e] : 0.f, qv[e], s[b], 0, 0, 0);
+      for (int b = 0; b < NB; ++b)
+        s[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? kv[i % (AHEAD + 1)][b][e] : 0.f, qv[e], s[b], 0, 0, 0);
   }
   float top = -INFINITY;
 #pragma unroll
-  for (int b = 0; b < 4; ++b)
+  for (int b = 0; b < NB; ++b)
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int key = kb + 16 * b + 4 * g + e;
@@ -324,10 +361,11 @@ __device__ __forceinline__ float af_scores(const AfArgs& a, const AfRun& run, co
 }
 
 // The tile's weights in the place of its scores, and the row's sum of them.
-__device__ __forceinline__ float af_weights(const AfRow& row, int tile, float m, int g, f32x4 (&s)[4]) {
+template <int NB>
+__device__ __forceinline__ float af_weights(const AfRow& row, int tile, float m, int g, f32x4 (&s)[NB]) {
   float sum = 0.f;
 #pragma unroll
-  for (int b = 0; b < 4; ++b)
+  for (int b = 0; b < NB; ++b)
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       s[b][e] = af_sees(row, tile * ATT_TILE + 16 * b + 4 * g + e) ? expf(s[b][e] - m) : 0.f;
@@ -338,36 +376,37 @@ __device__ __forceinline__ float af_weights(const AfRow& row, int tile, float m,
 }
 
 // done(i, start(i) + V^T P^T) for the blocks i of 16 head dims: lane 16 g + r gets dims 16 i + 4 g .. + 3 of row r.
-template <int DB, class Start, class Done>
+template <int DB, int AHEAD, int NB, class Start, class Done>
 __device__ __forceinline__ void af_values(const AfArgs& a, const AfRun& run, const AfRow& row, const KvLayout& lay, int tile,
-                                          const f32x4 (&w)[4], int r, int g, Start start, Done done) {
+                                          const f32x4 (&w)[NB], int r, int g, Start start, Done done) {
   const int kb = tile * ATT_TILE, lo = run.lo, hi = run.p_hi;
   const int* table = a.block_table + (size_t)run.seq * a.bt_stride;
-  const float* vp[4];
+  const float* vp[NB];
 #pragma unroll
-  for (int b = 0; b < 4; ++b) {
+  for (int b = 0; b < NB; ++b) {
     const int four = min(max(kb + 16 * b + 4 * g, lo & ~3), hi & ~3), slot = lay.v_slot(four % a.page_size);
     vp[b] = a.v_pages + ((size_t)table[four / a.page_size] * a.n_kv + run.kvh) * ((size_t)a.page_size * a.hd) + slot % 8 +
             lay.v_chunk_off(slot / 8, 0);
   }
   // whether some key of the tile is seen by one row of the run and not by another
   const bool mixed = run.p_lo != hi && (kb + ATT_TILE - 1 > run.p_lo || kb < first_key(hi, a.window));
-  f32x4 vv[2][4];
+  f32x4 vv[AHEAD + 1][NB];
   auto load = [&](int i) {
     const size_t at = lay.v_chunk_off(0, 16 * i + r < a.hd ? 16 * i + r : 0);
 #pragma unroll
-    for (int b = 0; b < 4; ++b) vv[i % 2][b] = *(const f32x4*)(vp[b] + at);
+    for (int b = 0; b < NB; ++b) vv[i % (AHEAD + 1)][b] = *(const f32x4*)(vp[b] + at);
   };
-  load(0);
+#pragma unroll
+  for (int i = 0; i < AHEAD && i < DB; ++i) load(i);
 #pragma unroll
   for (int i = 0; i < DB; ++i) {
-    if (i + 1 < DB) load(i + 1);
+    if (i + AHEAD < DB) load(i + AHEAD);
     __builtin_amdgcn_sched_barrier(0);
-    f32x4(&v)[4] = vv[i % 2];
+    f32x4(&v)[NB] = vv[i % (AHEAD + 1)];
     // dims behind the head's, and keys that no row sees: their places may hold anything
     const bool in = 16 * i + r < a.hd;
 #pragma unroll
-    for (int b = 0; b < 4; ++b)
+    for (int b = 0; b < NB; ++b)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int key = kb + 16 * b + 4 * g + e;
@@ -376,14 +415,14 @@ __device__ __forceinline__ void af_values(const AfArgs& a, const AfRun& run, con
     bool bad = false;
     if (mixed) {  // uniform
 #pragma unroll
-      for (int b = 0; b < 4; ++b)
+      for (int b = 0; b < NB; ++b)
 #pragma unroll
         for (int e = 0; e < 4; ++e) bad |= !(fabsf(v[b][e]) <= 3.402823466e38f);
     }
     f32x4 acc = start(i);
     if (!__any(bad)) {
 #pragma unroll
-      for (int b = 0; b < 4; ++b)
+      for (int b = 0; b < NB; ++b)
 #pragma unroll
         for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(v[b][e], w[b][e], acc, 0, 0, 0);
     } else {  // an infinity or NaN among the values: a weight of zero would not keep it from the rows before it
@@ -391,7 +430,7 @@ __device__ __forceinline__ void af_values(const AfArgs& a, const AfRun& run, con
         const int p = __shfl(row.pos, other, FG_WAVE), f = __shfl(row.first, other, FG_WAVE);
         f32x4 one = acc;
 #pragma unroll
-        for (int b = 0; b < 4; ++b)
+        for (int b = 0; b < NB; ++b)
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const int key = kb + 16 * b + 4 * g + e;
@@ -438,6 +477,10 @@ struct AfShared {
   float m_s[AF_WAVES][16], l_s[AF_WAVES][16];
 };
 template <int DB>
+struct AfOne {
+  f32x4 q_s[DB * 4][af_one_rows(DB)];
+};
+template <int DB>
 struct AfAlone {
   f32x4 q_s[DB * 4][AF_ALONE_ROWS];
   f32x4 s_s[AF_WAVES][AF_ALONE_ROWS][ATT_TILE / 4];  // a part's scores
@@ -460,12 +503,12 @@ __device__ __forceinline__ void af_together(const AfArgs& a, const AfRun& run, A
   const int t_lo = run.lo / ATT_TILE;
   for (int tile = t_lo + ((wave - t_lo) & (AF_WAVES - 1)); tile * ATT_TILE <= run.p_hi; tile += AF_WAVES) {
     f32x4 s[4];
-    const float m_new = fmaxf(m, af_scores<DB, 16>(a, run, row, lay, tile, lds.q_s, r, r, g, s));
+    const float m_new = fmaxf(m, af_scores<DB, 1>(a, run, row, lay, tile, lds.q_s, r, r, g, s));
     // a row that has seen no key yet, or sees none in this tile, stays as it is
     const float alpha = af_factor(m, m_new);
     l = l * alpha + af_weights(row, tile, m_new, g, s);
     m = m_new;
-    af_values<DB>(a, run, row, lay, tile, s, r, g, [&](int i) { return acc[i] * alpha; },
+    af_values<DB, 1>(a, run, row, lay, tile, s, r, g, [&](int i) { return acc[i] * alpha; },
                   [&](int i, const f32x4 x) { acc[i] = x; });
   }
   // ---- the parts' results, in order
@@ -508,7 +551,7 @@ __device__ __forceinline__ void af_by_wave(const AfArgs& a, const AfRun& run, Af
   float top = -INFINITY;
   for (int tile = t_lo; tile <= t_hi; ++tile) {
     f32x4 s[4];
-    const float m = af_scores<DB, AF_ALONE_ROWS>(a, run, row, lay, tile, lds.q_s, q_row, r, g, s);
+    const float m = af_scores<DB, 1>(a, run, row, lay, tile, lds.q_s, q_row, r, g, s);
     top = fmaxf(top, m);
     if (keeps) {
 #pragma unroll
@@ -530,7 +573,7 @@ __device__ __forceinline__ void af_by_wave(const AfArgs& a, const AfRun& run, Af
     for (int b = 0; b < 4; ++b) s[b] = lds.s_s[part][q_row][4 * b + g];
     const float m = lds.m_s[part][q_row], l = af_weights(row, tile, m, g, s), factor = af_factor(m, top);
     total = fmaf(l, factor, total);
-    af_values<DB>(a, run, row, lay, tile, s, r, g, [&](int) { return f32x4{0.f, 0.f, 0.f, 0.f}; },
+    af_values<DB, 1>(a, run, row, lay, tile, s, r, g, [&](int) { return f32x4{0.f, 0.f, 0.f, 0.f}; },
                   [&](int i, const f32x4 x) { o[i] += af_scaled(x, factor); });
   }
   const float inv = af_inverse(a, row, total, top);
@@ -538,25 +581,67 @@ __device__ __forceinline__ void af_by_wave(const AfArgs& a, const AfRun& run, Af
   for (int i = 0; i < DB; ++i) af_store(a, row, 16 * i + 4 * g, o[i], inv);
 }
 
-// DB: head dims in blocks of 16, at least hd / 16 (hd is a multiple of 8).  ALONE: a wave alone takes what `af_alone` says.
+// A run of one tile and at most af_one_rows rows by a wave, the tile's first NB blocks of 16 keys: the others are behind
+// every row's own place, so their weights are zeros, which change no sum.
+template <int DB, int NB>
+__device__ __forceinline__ void af_one_of(const AfArgs& a, const AfRun& run, const AfRow& row, const AfOne<DB>& lds, int r,
+                                              int g) {
+  constexpr int AHEAD = NB == 1 ? 7 : NB == 2 ? 3 : 2;  // (registers there are: a wave keeps no sums but a block's)
+  const KvLayout lay(a.page_size, a.hd);
+  const int tile = run.p_hi / ATT_TILE;
+  f32x4 s[NB];
+  const float top = af_scores<DB, AHEAD>(a, run, row, lay, tile, lds.q_s, min(r, af_one_rows(DB) - 1), r, g, s);
+  const float inv = af_inverse(a, row, af_weights(row, tile, top, g, s), top);
+  af_values<DB, AHEAD>(a, run, row, lay, tile, s, r, g, [&](int) { return f32x4{0.f, 0.f, 0.f, 0.f}; },
+                       [&](int i, const f32x4 x) { af_store(a, row, 16 * i + 4 * g, f32x4{0.f, 0.f, 0.f, 0.f} + x, inv); });
+}
+template <int DB>
+__device__ __forceinline__ void af_one(const AfArgs& a, const AfRun& run, AfOne<DB>& lds, int lane) {
+  const int r = lane % 16, g = lane / 16, blocks = run.p_hi % ATT_TILE / 16 + 1;
+  const AfRow row = af_row(a, run, r);
+  af_queries<DB, af_one_rows(DB)>(a, run, lds.q_s, 0, 1, run.n_here * (a.n_heads / a.n_kv), lane);
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  if (blocks == 1) return af_one_of<DB, 1>(a, run, row, lds, r, g);
+  if (blocks == 2) return af_one_of<DB, 2>(a, run, row, lds, r, g);
+  if constexpr (af_one_blocks(DB) > 2) af_one_of<DB, 4>(a, run, row, lds, r, g);
+}
+
+// The run at place `index` of a grid; false: none is.  Uniform.  (The blocks' first runs come first, a token's kv heads side
+// by side: every die gets as many of them.)
+__device__ __forceinline__ bool af_at(const AfArgs& a, int index, int lane, AfRun& run) {
+  const int full = 16 / (a.n_heads / a.n_kv), blocks = (a.n_tokens + full - 1) / full, place = index / a.n_kv;
+  return place < blocks * full && af_run(a, af_block(a, place % blocks, lane), index % a.n_kv, place / blocks, run);
+}
+
+// DB: head dims in blocks of 16, at least hd / 16 (hd is a multiple of 8).  ALONE: a wave alone takes what `af_kind` says.
 template <int DB, bool ALONE>
 __global__ __launch_bounds__(AF_WAVES* FG_WAVE) void attention_f32_kernel(const AfArgs a) {
   const int lane = threadIdx.x % FG_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / FG_WAVE);
   AfRun run;
   if constexpr (!ALONE) {
     __shared__ AfShared<DB> lds;
-    if (af_run(a, blockIdx.x, run)) af_together<DB>(a, run, lds, wave, lane);
+    if (af_at(a, blockIdx.x, lane, run) && af_kind<DB>(a, run) != AF_ONE) af_together<DB>(a, run, lds, wave, lane);
   } else {
     __shared__ union {
       AfShared<DB> together;
       AfAlone<DB> alone[AF_WAVES];
     } lds;
-    if (af_run(a, blockIdx.x, run) && !af_alone<DB>(a, run)) af_together<DB>(a, run, lds.together, wave, lane);
+    if (af_at(a, blockIdx.x, lane, run) && af_kind<DB>(a, run) == AF_TOGETHER) af_together<DB>(a, run, lds.together, wave, lane);
     // (the first eighth of the grid looks after the others' runs, not every eighth workgroup: those are all on one die)
-    if (blockIdx.x < (gridDim.x + AF_WAVES - 1) / AF_WAVES && af_run(a, blockIdx.x * AF_WAVES + wave, run) &&
-        af_alone<DB>(a, run))
+    if (blockIdx.x < (gridDim.x + AF_WAVES - 1) / AF_WAVES && af_at(a, blockIdx.x * AF_WAVES + wave, lane, run) &&
+        af_kind<DB>(a, run) == AF_ALONE)
       af_by_wave<DB>(a, run, lds.alone[wave], lane);
   }
+}
+
+// Runs of one tile and at most af_one_rows rows, a wave each.
+template <int DB>
+__global__ __launch_bounds__(4 * FG_WAVE) void attention_f32_one_kernel(const AfArgs a) {
+  const int lane = threadIdx.x % FG_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / FG_WAVE);
+  __shared__ AfOne<DB> lds[4];
+  AfRun run;
+  if (af_at(a, blockIdx.x * 4 + wave, lane, run) && af_kind<DB>(a, run) == AF_ONE) af_one<DB>(a, run, lds[wave], lane);
 }
 
 extern "C" int fg_paged_attention_general_sink(
@@ -573,12 +658,21 @@ extern "C" int fg_paged_attention_general_sink(
     const int full = 16 / group;
     const long long grid = (long long)((n_tokens + full - 1) / full * full) * n_kv;
     if (grid > 2147483647LL) return FG_ERR_ARG;
+    // The kernel for runs of one tile where there may be many: among prompts, from 2048 (token, head)s in the first 16 places
+    // of the sequences on (8 prompts of 37: 51 / 29 us without / with at 32 / 8 x 128, 50 / 36 at 16 / 4 x 256); with
+    // decoded tokens alone from 4096 on (64 of 60 keys, 32/32 x 128: 34 / 40; 300 of 9: 130 / 96; 200 of 100, which are none
+    // of them: 165 / 174).  Above head size 256, where a wave's run is long beside a workgroup's, among short sequences
+    // alone (8 / 8 x 512, 64 prompts of 5: 145 / 36, 300 of 9: 172 / 66; with 10 prompts of 100 beside 30 of 700: 362 / 402).
+    const bool decoded = n_tokens <= n_seqs, large = hd > 256;
+    const int ones = min((long long)n_tokens, 16LL * n_seqs) * n_heads >= (decoded && !large ? 4096 : 2048) &&
+                     (!large || n_tokens <= 16LL * n_seqs);
     const AfArgs a{(const float*)q, q_stride, (float*)out, out_stride, (const float*)k_pages, (const float*)v_pages, block_table,
                    bt_stride, seq_of_token, positions, n_tokens, n_heads, n_kv, hd, page_size, scale, window, sinks, dist,
-                   (int)min((long long)min(n_seqs, n_tokens) * n_kv, 2147483647LL)};
+                   (int)min((long long)min(n_seqs, n_tokens) * n_kv, 2147483647LL), ones};
     const bool alone = group <= AF_ALONE_ROWS && a.few_runs >= (hd <= 64 ? af_alone_from(4, 1) : af_alone_from(8, 1));
 #define ATTENTION_F32(DB)                                                                                   \
   do {                                                                                                      \
+    if (a.ones) attention_f32_one_kernel<DB><<<(unsigned)((grid + 3) / 4), 4 * FG_WAVE, 0, stream>>>(a);    \
     if (alone) attention_f32_kernel<DB, true><<<(unsigned)grid, AF_WAVES * FG_WAVE, 0, stream>>>(a);        \
     else attention_f32_kernel<DB, false><<<(unsigned)grid, AF_WAVES * FG_WAVE, 0, stream>>>(a);             \
   } while (0)

@@ -334,6 +334,37 @@ def test_paged_attention_f32_runs_of_a_wave(ops, H, KV, hd, P, window, more):
         assert torch.allclose(out[:12].cpu(), _plain_rows(case, seqs[:12], window or None), atol=2e-5, rtol=1e-5)
 
 
+@pytest.mark.parametrize("H,KV,hd,P", [(16, 16, 64, 64), (24, 8, 128, 16), (16, 1, 80, 32), (8, 8, 24, 8), (16, 4, 256, 64),
+                                       (16, 4, 320, 64), (8, 8, 512, 64)])
+@pytest.mark.parametrize("window,more", [(0, False), (20, True), (-48, False)])
+def test_paged_attention_f32_runs_of_one_tile(ops, H, KV, hd, P, window, more):
+    """Many short prompts, and decoded tokens of few keys, whose runs of one tile are another kernel's, a wave each, beside
+    runs of more: the bits that each sequence's call of its own gives, of which too few come for that kernel.  Lengths at the
+    ends of blocks of 16 keys and of tiles, runs cut by a sequence's end; what the pages hold beyond the last key is no
+    number."""
+    seqs = [(0, 5), (0, 1), (0, 16), (3, 14), (0, 17), (31, 1), (30, 4), (0, 33), (15, 1), (47, 2), (0, 64), (63, 1), (60, 9),
+            (64, 1), (0, 70), (200, 3)] + [(0, 1 + i % 11) for i in range(120)]
+    case = _paged_case(torch.float32, seqs, H, KV, hd, P, seed=13)
+    sinks = torch.randn(H, device=DEV) if more else None
+    distance = torch.rand(H, 2, device=DEV) if more else None
+
+    def run(at, rows, table):
+        out = torch.full_like(case["q"][at], float("nan"))
+        return ops.paged_attention_general(case["q"][at], out, case["kp"], case["vp"], table, rows, case["pos"][at], H, hd**-0.5,
+                                           window, sinks, distance)
+
+    out = run(slice(None), case["seq_of"], case["table"])
+    assert torch.isfinite(out).all()
+    t = 0
+    for i, (_, n) in enumerate(seqs[:40]):
+        here = slice(t, t + min(n, 8))  # (a call's own: 8 tokens of a sequence)
+        alone = run(here, torch.zeros_like(case["seq_of"][here]), case["table"][i : i + 1])
+        assert torch.equal(alone, out[here]), (i, seqs[i])
+        t += n
+    if window >= 0 and not more:
+        assert torch.allclose(out[:t].cpu(), _plain_rows(case, seqs[:40], window or None)[:t], atol=2e-5, rtol=1e-5)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_paged_attention_far_key_stands_out(ops, dtype):
     """One key among hundreds, in an early page, gets nearly all the weight:
