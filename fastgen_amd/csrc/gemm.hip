@@ -2,16 +2,25 @@
 // 470, 488-496, 513: F.linear): the engine's own matrix products without a
 // mode of reduced precision.
 //
-// float32 (the true 32-bit path) runs on v_mfma_f32_16x16x4_f32, whose
-// products and sums are fp32.  Every output element is summed in an order
-// fixed by K alone, whichever kernel takes the product: 32 k in a chain of
-// matrix instructions (instruction (s, j) adds the k = 16 s + 4 g + j of its
-// four lane groups g, one after the other), 4 chains into a segment's sum, 8
-// segments into a group's, the groups' into the total, each ascending.  A
-// row's result therefore does not depend on how many other rows the call
-// holds, and rounding grows with 32 + 4 + 8 + K/1024 additions (relative to
-// the product in 64 bits, random operands of K = 3072 / 8192 / 14336: 1.3 /
-// 1.4 / 1.4e-7; chains of 128 k: 2.1 / 2.2 / 2.2e-7).
+// float32 (the true 32-bit path) runs on v_mfma_f32_16x16x32_bf16, sixteen
+// times the rate of v_mfma_f32_16x16x4_f32: every operand is the exact sum of
+// three bf16 parts of 8 bits each (h = bf16(v), m = bf16(v - h), l = v - h -
+// m), a product of two is six instructions, and the parts' products left out
+// (m l, l m, l l) are below 2^-26 of the whole.  What rounding costs is the
+// sums', and the matrix core cuts off where it adds to its accumulator, so
+// the order is: h h over 128 k (4 instructions from zero) in one chain, the
+// five smaller products of the same k (20 instructions) in another, their sum
+// a segment's; 8 segments are a group's sum, the groups' sums the total, each
+// ascending in fp32.  An output's order is fixed by K alone, whichever kernel
+// takes the product, so a row's result does not depend on how many other rows
+// the call holds.  Error relative to the product in 64 bits, random operands
+// of K = 128 / 1024 / 3072 / 8192 / 14336: 0.7 / 0.9 / 0.9 / 1.0 / 1.1e-7
+// (the fp32 instructions with chains of 32 k: 1.1 / 1.2 / 1.3 / 1.4 / 1.4e-7);
+// with magnitudes spread over e^+-2 1.0 / 1.0 / 1.1 / 1.2 / 1.3e-7 (1.0 / 1.2 /
+// 1.2 / 1.4 / 1.5).  A part of an operand below 2^-109 may be too small for
+// bf16: such an operand counts with fewer bits.  Infinities (and what rounds to
+// one in bf16) have no such parts: an output that comes out as NaN is
+// computed again, one fp32 FMA a product (gf_again).
 //
 // Operands of bf16 with fp32 accumulation take the FMA kernel below, so that
 // any shape has a product when the tuned kernels refuse it.
@@ -117,9 +126,9 @@ extern "C" int fg_gemm_nt(const void* x, const void* w, void* y, int M, int N, i
 // ------------------------------------------------------------------ float32
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-#define GF_SEG 128    // k of a segment: 4 chains of matrix instructions
+#define GF_SEG 128    // k of a segment: 4 steps
 #define GF_GROUP 1024 // k of a group: 8 segments
-#define GF_STEP 32    // k of a chain; what the tiled kernel holds in LDS at a time
+#define GF_STEP 32    // k of a matrix instruction
 
 // Four elements of a row from k on, zeros behind K.  VEC: rows are 16-byte aligned and K is a multiple of 4.
 template <bool VEC>
@@ -135,11 +144,84 @@ __device__ __forceinline__ f32x4 gf_load4(const float* __restrict__ row, int k, 
   return v;
 }
 
-// Four instructions: 16 k.  A: 16 rows of W, B: 16 rows of x; lane 16 g + r ends with outputs 4 g .. 4 g + 3 of x row r.
-__device__ __forceinline__ f32x4 gf_mfma16(const f32x4 wv, const f32x4 xv, f32x4 acc) {
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+// The three parts of four numbers: v = part 0 + part 1 + part 2, the first rounded to nearest (so that the next has
+// either sign and what is left out no bias), the second cut off, the third the eight bits that are left.
+__device__ __forceinline__ void gf_parts4(const f32x4 v, bf16x4* p0, bf16x4* p1, bf16x4* p2) {
+  const unsigned top = 0xffff0000u;
+  unsigned p[3][2];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[j], xv[j], acc, 0, 0, 0);
-  return acc;
+  for (int e = 0; e < 2; ++e) {
+    const f32x2 pair = {v[2 * e], v[2 * e + 1]};
+    const unsigned h = __builtin_bit_cast(unsigned, __builtin_convertvector(pair, bf16x2));
+    const float r0 = pair[0] - __uint_as_float(h << 16), r1 = pair[1] - __uint_as_float(h & top);
+    const float l0 = r0 - __uint_as_float(__float_as_uint(r0) & top), l1 = r1 - __uint_as_float(__float_as_uint(r1) & top);
+    p[0][e] = h;  // (a permutation of bytes takes the upper halves of two words)
+    p[1][e] = __builtin_amdgcn_perm(__float_as_uint(r1), __float_as_uint(r0), 0x07060302u);
+    p[2][e] = __builtin_amdgcn_perm(__float_as_uint(l1), __float_as_uint(l0), 0x07060302u);
+  }
+  *p0 = __builtin_bit_cast(bf16x4, p[0]);
+  *p1 = __builtin_bit_cast(bf16x4, p[1]);
+  *p2 = __builtin_bit_cast(bf16x4, p[2]);
+}
+
+// An operand of the matrix instruction: lane 16 g + r holds of row r the k = 4 g .. 4 g + 3 and 16 + 4 g .. 19 + 4 g of
+// a step (the instruction sums over k, so any order will do that is the same for W and x; a load of this one takes
+// 64 bytes in a row).
+struct GfParts {
+  bf16x8 p[3];
+};
+
+__device__ __forceinline__ GfParts gf_parts(const f32x4 lo, const f32x4 hi) {
+  bf16x4 a[3], b[3];
+  gf_parts4(lo, &a[0], &a[1], &a[2]);
+  gf_parts4(hi, &b[0], &b[1], &b[2]);
+  GfParts s;
+#pragma unroll
+  for (int i = 0; i < 3; ++i) s.p[i] = __builtin_shufflevector(a[i], b[i], 0, 1, 2, 3, 4, 5, 6, 7);
+  return s;
+}
+
+template <bool VEC>
+__device__ __forceinline__ f32x4 gf_whole4(const float* p) {
+  if constexpr (VEC) return *(const f32x4*)p;
+  else return f32x4{p[0], p[1], p[2], p[3]};
+}
+
+#define GF_MFMA(A, B, C) __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, B, C, 0, 0, 0)
+
+// One step of one tile.  A: 16 rows of W, B: 16 rows of x; lane 16 g + r ends with outputs 4 g .. 4 g + 3 of x row r.
+__device__ __forceinline__ void gf_step(const GfParts& w, const bf16x8 x0, const bf16x8 x1, const bf16x8 x2,
+                                        f32x4& whole, f32x4& small) {
+  small = GF_MFMA(w.p[2], x0, small);
+  whole = GF_MFMA(w.p[0], x0, whole);
+  small = GF_MFMA(w.p[0], x2, small);
+  small = GF_MFMA(w.p[1], x1, small);
+  small = GF_MFMA(w.p[1], x0, small);
+  small = GF_MFMA(w.p[0], x1, small);
+}
+
+// An output whose sum came out as NaN: the operands may hold an infinity.
+__device__ __noinline__ float gf_again(const float* x, const float* w, int K) {
+  float sum = 0.f;
+  for (int k = 0; k < K && sum == sum; ++k) sum = fmaf(w[k], x[k], sum);
+  return sum;
+}
+
+__device__ __forceinline__ f32x4 gf_read4(const float* p, int n, int N, bool wide) {
+  f32x4 v = {0.f, 0.f, 0.f, 0.f};
+  if (wide && n + 4 <= N) {
+    v = *(const f32x4*)(p + n);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (n + e < N) v[e] = p[n + e];
+  }
+  return v;
 }
 
 __device__ __forceinline__ void gf_store4(float* __restrict__ y, int n, int N, bool wide, const f32x4 v) {
@@ -154,14 +236,17 @@ __device__ __forceinline__ void gf_store4(float* __restrict__ y, int n, int N, b
 
 // Up to 16 rows (decode): bound by reading W once.  A workgroup owns 16 outputs; a round is one group, a wave takes
 // one of its segments, so 64 KB of W (every wave's next segment) are in flight a workgroup while the current ones
-// are multiplied; the segments' sums meet in LDS and are added in order by one thread an output.  4 rows, N x K
-// 3072 x 3072 / 16384 x 3072 / 3072 x 8192: 16 / 50 / 35 us, 2.4 / 4.0 / 2.9 TB/s of W (FMA with a thread an output: 490
-// / 495 / 1250 us); at 16 rows the tiled kernel is level (31 / 54 / 38 against 20 / 61 / 45).
-template <bool VEC>
+// are multiplied; the segments' sums meet in LDS and are added in order by one thread an output.  N x K 3072 x 3072 /
+// 16384 x 3072 / 3072 x 8192: 13 / 44 / 32 us at 4 rows (4.6 TB/s of W at the largest), 18 / 60 / 41 at 16; with the fp32
+// instructions 14 / 48 / 32 and 18 / 60 / 41.
+// A wave cuts its segment of x into parts once: with FEW (up to 8 rows), each number in one lane, through LDS into
+// the operands' order; above, every lane the operand it needs.
+template <bool FEW, bool VEC>
 __global__ __launch_bounds__(512) void gemm_f32_few_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                            float* __restrict__ y, int M, int N, int K, int ldx,
                                                            int ldw, int ldy) {
   __shared__ f32x4 sums[2][8][FG_WAVE];
+  __shared__ bf16x4 parts[FEW ? 8 : 1][4][3][4][8][2];  // [wave][step][part][g][row][half]
   const int tid = threadIdx.x, lane = tid % FG_WAVE, wave = tid / FG_WAVE;
   const int r = lane % 16, g = lane / 16, n0 = blockIdx.x * 16;
   // rows behind the last repeat it: their outputs are not stored
@@ -177,24 +262,45 @@ __global__ __launch_bounds__(512) void gemm_f32_few_kernel(const float* __restri
   for (int s0 = 0, buf = 0; s0 < n_seg; s0 += 8, buf ^= 1) {
     const int seg = s0 + wave;
     if (seg < n_seg) {
+      if constexpr (FEW) {
+        const int c = lane % 32;  // four k of a row; the rows two apart
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        wv[i] = next[i];
-        xv[i] = gf_load4<VEC>(xrow, seg * GF_SEG + i * 16 + g * 4, K);
+        for (int i = 0; i < 4; ++i)
+          xv[i] = gf_load4<VEC>(x + (size_t)min(lane / 32 + 2 * i, M - 1) * ldx, seg * GF_SEG + c * 4, K);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) xv[i] = gf_load4<VEC>(xrow, seg * GF_SEG + i * 16 + g * 4, K);
       }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) wv[i] = next[i];
       if (seg + 8 < n_seg) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) next[i] = gf_load4<VEC>(wrow, (seg + 8) * GF_SEG + i * 16 + g * 4, K);
       }
-      f32x4 acc[4], sum = {0.f, 0.f, 0.f, 0.f};
+      if constexpr (FEW) {
+        const int c = lane % 32;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) acc[i] = gf_mfma16(wv[2 * i], xv[2 * i], f32x4{0.f, 0.f, 0.f, 0.f});
+        for (int i = 0; i < 4; ++i) {
+          const int row = lane / 32 + 2 * i;
+          bf16x4(*to)[4][8][2] = parts[wave][c / 8];
+          if (2 * i < M) gf_parts4(xv[i], &to[0][c % 4][row][c / 4 % 2], &to[1][c % 4][row][c / 4 % 2],
+                                   &to[2][c % 4][row][c / 4 % 2]);
+        }
+        __builtin_amdgcn_wave_barrier();  // (a wave reads only what it has written itself)
+      }
+      f32x4 whole = {0.f, 0.f, 0.f, 0.f}, small = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        acc[i] = gf_mfma16(wv[2 * i + 1], xv[2 * i + 1], acc[i]);
-        sum += acc[i];
+        GfParts xp;
+        if constexpr (FEW) {
+#pragma unroll
+          for (int p = 0; p < 3; ++p) xp.p[p] = *(const bf16x8*)&parts[wave][i][p][g][min(r, M - 1)][0];
+        } else {
+          xp = gf_parts(xv[2 * i], xv[2 * i + 1]);
+        }
+        gf_step(gf_parts(wv[2 * i], wv[2 * i + 1]), xp.p[0], xp.p[1], xp.p[2], whole, small);
       }
-      sums[buf][wave][lane] = sum;
+      sums[buf][wave][lane] = whole + small;
     }
     __syncthreads();  // (a round's sums are read before the round after next writes them: one barrier between)
     if (tid < 256) {
@@ -207,172 +313,243 @@ __global__ __launch_bounds__(512) void gemm_f32_few_kernel(const float* __restri
   // element tid of a wave's sums: lane tid / 4 = 16 g + r, output 4 g + tid % 4 of row r
   if (tid < 256) {
     const int m = (tid / 4) % 16, n = n0 + (tid / 64) * 4 + tid % 4;
-    if (m < M && n < N) y[(size_t)m * ldy + n] = total;
+    if (m < M && n < N) {
+      if (total != total) total = gf_again(x + (size_t)m * ldx, w + (size_t)n * ldw, K);
+      y[(size_t)m * ldy + n] = total;
+    }
   }
 }
 
-// Many rows: bound by the matrix cores (157 TFLOP/s of fp32).  Four waves own 32 MB rows x 32 NB outputs, both operands
-// go through registers into LDS, 32 k at a time in two buffers, in pieces of 4 k a row, piece-major with two pieces
-// of padding: a wave's operand reads are runs of 256 bytes, and 8 lanes load a whole line of a row (with 4 lanes a
-// row, half lines and LDS stores as contiguous as the reads: 5 % slower).  With `part` a workgroup takes one group of
-// k and stores its sum there ([groups][M][N]); the workgroups that read the same rows of W are neighbours on one die.
-// 400 rows of 16384 x 3072: 440 us, 92 TFLOP/s (FMA: 1206 us); 2048 rows: 1883 us, 109 TFLOP/s, 1592 without the
-// loads, so the rest is the matrix cores, the operand reads and the barrier of every 32 k.
-template <int MB, int NB, bool VEC>
-__global__ __launch_bounds__(256) void gemm_f32_tiled_kernel(const float* __restrict__ x, const float* __restrict__ w,
-                                                             float* __restrict__ y, float* __restrict__ part, int M,
-                                                             int N, int K, int ldx, int ldw, int ldy, int row_tiles,
-                                                             int col_tiles, int units, int wide) {
-  constexpr int TM = 32 * MB, TN = 32 * NB;
-  __shared__ f32x4 xs[2][8][TM + 2], ws[2][8][TN + 2];
+// Many rows: bound by the matrix cores at the clock they can hold.  NW waves own 16 MB rows x 16 NB NW outputs, each
+// all the rows and 16 NB outputs: a wave takes its rows of W from memory into registers itself, cuts them into parts
+// once and reads every x from LDS, where the workgroup has put its three parts in the operands' order, 32 k at a time
+// in two buffers.  The two waves of a SIMD cut W on either side of their matrix instructions (`late`), so that one's
+// vector work runs beside the other's products.  AHEAD: steps of W and x in flight, in registers; their loads stand
+// under no condition (with one the compiler copies what it has just loaded, that is, waits for it: 1.7 us a step
+// instead of 0.6 where the products take 0.1).  A group's sum is kept in LDS, which leaves the registers to the loads.
+// With `part` a workgroup takes one group of k and stores its sum there ([groups][M][N]); else it adds each group's to
+// y.  The workgroups that read the same rows of W are neighbours on one die.
+//
+// N x K 16384 x 3072 / 5120 x 3072 / 3072 x 8192, us: 400 rows 240 / 100 / 148 (433 / 153 / 240 with the fp32
+// instructions), 2048 rows 1163 / 418 / 667 (1891 / 605 / 981): 1.06 PFLOP/s of bf16 at the largest, against 1.4 that
+// a product of bf16 operands reaches.
+template <int MB, int NB, int NW, int AHEAD, bool VEC>
+__global__ __launch_bounds__(64 * NW, 2) void gemm_f32_tiled_kernel(
+    const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ y, float* __restrict__ part, int M,
+    int N, int K, int ldx, int ldw, int ldy, int row_tiles, int col_tiles, int units, int wide) {
+  constexpr int TM = 16 * MB, TN = 16 * NB * NW, XV = (TM * 8 + 64 * NW - 1) / (64 * NW);
+  static_assert(4 % AHEAD == 0, "a segment's steps use the sets of registers in turn");
+  __shared__ bf16x4 xs[2][MB][3][FG_WAVE][2];
+  __shared__ f32x4 mids[NW][MB * NB][FG_WAVE];
   const int unit = (blockIdx.x / 8 / row_tiles) * 8 + blockIdx.x % 8;
   if (unit >= units) return;
-  const int m0 = (blockIdx.x / 8 % row_tiles) * TM, n0 = (unit % col_tiles) * TN, group = unit / col_tiles;
-  const int tid = threadIdx.x, lane = tid % FG_WAVE, wave = tid / FG_WAVE;
-  const int r = lane % 16, g = lane / 16;
-  const int wm = (wave / 2) * 16 * MB, wn = (wave % 2) * 16 * NB;
-  const int piece = tid % 8, row = tid / 8;
-  const float* xr[MB];
-  const float* wr[NB];
-#pragma unroll
-  for (int i = 0; i < MB; ++i) xr[i] = x + (size_t)min(m0 + row + 32 * i, M - 1) * ldx;
-#pragma unroll
-  for (int i = 0; i < NB; ++i) wr[i] = w + (size_t)min(n0 + row + 32 * i, N - 1) * ldw;
+  const int m0 = (blockIdx.x / 8 % row_tiles) * TM, group = unit / col_tiles;
+  const int tid = threadIdx.x, lane = tid % FG_WAVE, wave = __builtin_amdgcn_readfirstlane(tid / FG_WAVE);
+  const int r = lane % 16, g = lane / 16, n0 = (unit % col_tiles) * TN + wave * 16 * NB;
+  const bool late = wave >= 4;
   const int k_begin = part ? group * GF_GROUP : 0, k_end = part ? min(K, k_begin + GF_GROUP) : K;
+  const int k_full = k_begin + (k_end - k_begin) / GF_SEG * GF_SEG;  // whole segments
+  // a lane's place behind the wave's (the tile's) first row; rows behind the last repeat it: their outputs are not stored
+  const float *wb = w + (size_t)min(n0, N - 1) * ldw, *xb = x + (size_t)m0 * ldx;
+  unsigned wo[NB], xo[XV];  // in bytes
+#pragma unroll
+  for (int j = 0; j < NB; ++j) wo[j] = 4 * (min(16 * j + r, max(N - 1 - n0, 0)) * ldw + 4 * g);
+  const int piece = tid % 8, row = tid / 8;  // of x: four k of a row, the rows 8 NW apart
+#pragma unroll
+  for (int i = 0; i < XV; ++i) xo[i] = 4 * (min(row + 8 * NW * i, M - 1 - m0) * ldx + 4 * piece);
 
-  f32x4 xv[MB], wv[NB], seg[MB][NB], mid[MB][NB], total[MB][NB];
+  f32x4 raw[AHEAD][NB][2], xv[AHEAD][XV], whole[MB][NB], small[MB][NB];
+  GfParts wp[NB];
+  // a whole step; what would be loaded ahead behind the last whole segment is its last step again
+  auto load_w = [&](int set, int k) {
+    const char* at = (const char*)(wb + min(k, k_full - GF_STEP));
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      raw[set][j][0] = gf_whole4<VEC>((const float*)(at + wo[j]));
+      raw[set][j][1] = gf_whole4<VEC>((const float*)(at + wo[j]) + 16);
+    }
+  };
+  auto load_x = [&](int set, int k) {
+    const char* at = (const char*)(xb + min(k, k_full - GF_STEP));
+#pragma unroll
+    for (int i = 0; i < XV; ++i) xv[set][i] = gf_whole4<VEC>((const float*)(at + xo[i]));
+  };
+  auto store_x = [&](int set, int buf) {
+#pragma unroll
+    for (int i = 0; i < XV; ++i) {
+      const int at = row + 8 * NW * i;
+      if (TM % (8 * NW) == 0 || at < TM) {
+        bf16x4(*to)[FG_WAVE][2] = xs[buf][at / 16];
+        const int l = (piece % 4) * 16 + at % 16, half = piece / 4;
+        gf_parts4(xv[set][i], &to[0][l][half], &to[1][l][half], &to[2][l][half]);
+      }
+    }
+  };
+  auto cut_w = [&](int set) {
+#pragma unroll
+    for (int j = 0; j < NB; ++j) wp[j] = gf_parts(raw[set][j][0], raw[set][j][1]);
+  };
+  auto multiply = [&](int buf) {
+#pragma unroll
+    for (int i = 0; i < MB; ++i) {
+      bf16x8 b[3];
+#pragma unroll
+      for (int p = 0; p < 3; ++p) b[p] = *(const bf16x8*)&xs[buf][i][p][lane][0];
+#pragma unroll
+      for (int j = 0; j < NB; ++j) gf_step(wp[j], b[0], b[1], b[2], whole[i][j], small[i][j]);
+    }
+  };
+  // the end of the segment from k0 on
+  auto close = [&](int k0) {
+    const int next = k0 + GF_SEG;
+    const bool first = k0 % GF_GROUP == 0, last = next % GF_GROUP == 0 || next >= k_end;
+#pragma unroll
+    for (int i = 0; i < MB; ++i) {
+      const int m = m0 + 16 * i + r;
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        f32x4 mid = first ? f32x4{0.f, 0.f, 0.f, 0.f} : mids[wave][i * NB + j][lane];
+        mid += whole[i][j] + small[i][j];
+        whole[i][j] = small[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (!last) {
+          mids[wave][i * NB + j][lane] = mid;
+        } else if (m < M) {
+          const int n = n0 + 16 * j + 4 * g;
+          if (part) {
+            gf_store4(part + ((size_t)group * M + m) * N, n, N, wide, mid);
+          } else {
+            float* out = y + (size_t)m * ldy;
+            if (k0 >= GF_GROUP) mid = gf_read4(out, n, N, wide) + mid;
+            if (next >= k_end) {
+#pragma unroll
+              for (int e = 0; e < 4; ++e)
+                if (mid[e] != mid[e] && n + e < N) mid[e] = gf_again(x + (size_t)m * ldx, w + (size_t)(n + e) * ldw, K);
+            }
+            gf_store4(out, n, N, wide, mid);
+          }
+        }
+      }
+    }
+  };
 #pragma unroll
   for (int i = 0; i < MB; ++i)
 #pragma unroll
-    for (int j = 0; j < NB; ++j) seg[i][j] = mid[i][j] = total[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < NB; ++j) whole[i][j] = small[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (k_begin < k_full) {
 #pragma unroll
-  for (int i = 0; i < MB; ++i) xs[0][piece][row + 32 * i] = gf_load4<VEC>(xr[i], k_begin + piece * 4, k_end);
-#pragma unroll
-  for (int i = 0; i < NB; ++i) ws[0][piece][row + 32 * i] = gf_load4<VEC>(wr[i], k_begin + piece * 4, k_end);
-  __syncthreads();
-  int buf = 0;
-  for (int k0 = k_begin; k0 < k_end; k0 += GF_STEP, buf ^= 1) {
-    const bool more = k0 + GF_STEP < k_end;
-    if (more) {
-#pragma unroll
-      for (int i = 0; i < MB; ++i) xv[i] = gf_load4<VEC>(xr[i], k0 + GF_STEP + piece * 4, k_end);
-#pragma unroll
-      for (int i = 0; i < NB; ++i) wv[i] = gf_load4<VEC>(wr[i], k0 + GF_STEP + piece * 4, k_end);
+    for (int a = 0; a < AHEAD; ++a) {
+      load_x(a, k_begin + a * GF_STEP);
+      load_w(a, k_begin + a * GF_STEP);
     }
-    f32x4 acc[MB][NB];
-#pragma unroll
-    for (int i = 0; i < MB; ++i)
-#pragma unroll
-      for (int j = 0; j < NB; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      f32x4 a[NB], b[MB];
-#pragma unroll
-      for (int j = 0; j < NB; ++j) a[j] = ws[buf][s * 4 + g][wn + 16 * j + r];
-#pragma unroll
-      for (int i = 0; i < MB; ++i) b[i] = xs[buf][s * 4 + g][wm + 16 * i + r];
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-#pragma unroll
-        for (int i = 0; i < MB; ++i)
-#pragma unroll
-          for (int j = 0; j < NB; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j][e], b[i][e], acc[i][j], 0, 0, 0);
-    }
-#pragma unroll
-    for (int i = 0; i < MB; ++i)
-#pragma unroll
-      for (int j = 0; j < NB; ++j) seg[i][j] += acc[i][j];
-    const int next_k = k0 + GF_STEP;
-    if (next_k % GF_SEG == 0 || !more) {
-#pragma unroll
-      for (int i = 0; i < MB; ++i)
-#pragma unroll
-        for (int j = 0; j < NB; ++j) {
-          mid[i][j] += seg[i][j];
-          seg[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-          if (next_k % GF_GROUP == 0 || !more) {
-            total[i][j] += mid[i][j];
-            mid[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-          }
-        }
-    }
-    if (more) {
-#pragma unroll
-      for (int i = 0; i < MB; ++i) xs[buf ^ 1][piece][row + 32 * i] = xv[i];
-#pragma unroll
-      for (int i = 0; i < NB; ++i) ws[buf ^ 1][piece][row + 32 * i] = wv[i];
-    }
+    store_x(0, 0);
+    if (late) cut_w(0);
     __syncthreads();
+    for (int k0 = k_begin; k0 < k_full; k0 += GF_SEG) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int k = k0 + q * GF_STEP, buf = q % 2;
+        load_x(q % AHEAD, k + AHEAD * GF_STEP);
+        if (!late) cut_w(q % AHEAD);
+        load_w(q % AHEAD, k + AHEAD * GF_STEP);
+        multiply(buf);
+        if (late) cut_w((q + 1) % AHEAD);
+        store_x((q + 1) % AHEAD, buf ^ 1);
+        __syncthreads();
+      }
+      close(k0);
+    }
   }
-  float* out = part ? part + (size_t)group * M * N : y;
-  const int ldo = part ? N : ldy;
+  if (k_full < k_end) {  // less than a segment at the end of the rows
+    for (int k = k_full; k < k_end; k += GF_STEP) {
 #pragma unroll
-  for (int i = 0; i < MB; ++i) {
-    const int m = m0 + wm + 16 * i + r;
-    if (m >= M) continue;
+      for (int i = 0; i < XV; ++i) xv[0][i] = gf_load4<VEC>(xb + xo[i] / 4 - 4 * piece, k + 4 * piece, k_end);
 #pragma unroll
-    for (int j = 0; j < NB; ++j)
-      gf_store4(out + (size_t)m * ldo, n0 + wn + 16 * j + 4 * g, N, wide, total[i][j]);
+      for (int j = 0; j < NB; ++j) {
+        raw[0][j][0] = gf_load4<VEC>(wb + wo[j] / 4 - 4 * g, k + 4 * g, k_end);
+        raw[0][j][1] = gf_load4<VEC>(wb + wo[j] / 4 - 4 * g, k + 16 + 4 * g, k_end);
+      }
+      store_x(0, 0);
+      cut_w(0);
+      __syncthreads();
+      multiply(0);
+      __syncthreads();
+    }
+    close(k_full);
   }
 }
 
 // The groups' sums, added in order.
 __global__ __launch_bounds__(256) void gemm_f32_sum_kernel(const float* __restrict__ part, float* __restrict__ y,
-                                                           int M, int N, int ldy, int groups, int wide) {
+                                                           const float* __restrict__ x, const float* __restrict__ w,
+                                                           int M, int N, int K, int ldx, int ldw, int ldy, int groups,
+                                                           int wide) {
   const int m = blockIdx.y, n = (blockIdx.x * 256 + threadIdx.x) * 4;
   if (n >= N) return;
   f32x4 total = {0.f, 0.f, 0.f, 0.f};
-  const float* p = part + (size_t)m * N + n;
-  for (int g = 0; g < groups; ++g, p += (size_t)M * N) {
-    f32x4 v = {0.f, 0.f, 0.f, 0.f};
-    if (wide && n + 4 <= N) {
-      v = *(const f32x4*)p;
-    } else {
+  for (int g = 0; g < groups; ++g) total += gf_read4(part + ((size_t)g * M + m) * N, n, N, wide);
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (n + e < N) v[e] = p[e];
-    }
-    total += v;
-  }
+  for (int e = 0; e < 4; ++e)
+    if (total[e] != total[e] && n + e < N) total[e] = gf_again(x + (size_t)m * ldx, w + (size_t)(n + e) * ldw, K);
   gf_store4(y + (size_t)m * ldy, n, N, wide, total);
 }
 
-// mb, nb: the tile of the many-rows kernel in units of 32 rows and 32 outputs (mb = 0: up to 16 rows, no tile).
+struct GfCall {
+  const float *x, *w;
+  float *y, *part;
+  int M, N, K, ldx, ldw, ldy, vec;
+  hipStream_t stream;
+};
+
+template <int MB, int NB, int NW>
+static int gf_launch(const GfCall& c) {
+  constexpr int AHEAD = MB <= 3 ? 4 : 2;
+  const int groups = (c.K + GF_GROUP - 1) / GF_GROUP;
+  const int wide = c.N % 4 == 0 && c.ldy % 4 == 0 && (uintptr_t)c.y % 16 == 0 && (uintptr_t)c.part % 16 == 0;
+  const int row_tiles = (c.M + 16 * MB - 1) / (16 * MB), col_tiles = (c.N + 16 * NB * NW - 1) / (16 * NB * NW);
+  const long long units = (long long)col_tiles * (c.part ? groups : 1);
+  const long long blocks = (units + 7) / 8 * 8 * row_tiles;
+  if (blocks > 2147483647LL || (c.part && c.M > 65535)) return FG_ERR_ARG;
+#define TILED(VEC)                                                                                            \
+  gemm_f32_tiled_kernel<MB, NB, NW, AHEAD, VEC><<<(unsigned)blocks, 64 * NW, 0, c.stream>>>(                  \
+      c.x, c.w, c.y, c.part, c.M, c.N, c.K, c.ldx, c.ldw, c.ldy, row_tiles, col_tiles, (int)units, wide)
+  if (c.vec) TILED(true);
+  else TILED(false);
+#undef TILED
+  if (c.part) {
+    gemm_f32_sum_kernel<<<dim3((c.N + 1023) / 1024, c.M), 256, 0, c.stream>>>(c.part, c.y, c.x, c.w, c.M, c.N, c.K,
+                                                                              c.ldx, c.ldw, c.ldy, groups, wide);
+  }
+  return fg_launch_status();
+}
+
+// mb, nw: the tile of the many-rows kernel, 16 mb rows (mb <= 5 with 4 waves, 7 with 8) and nw waves of 32 outputs
+// (mb = 0: up to 16 rows, no tile).
 // part: null, or fp32 [ceil(K / 1024)][M][N] for a workgroup a group of k.
 extern "C" int fg_gemm_f32(const float* x, const float* w, float* y, float* part, int M, int N, int K, int ldx,
-                           int ldw, int ldy, int mb, int nb, hipStream_t stream) {
+                           int ldw, int ldy, int mb, int nw, hipStream_t stream) {
   if (M <= 0 || N <= 0) return FG_OK;
   if (K <= 0 || ldx < K || ldw < K || ldy < N) return FG_ERR_ARG;
   const bool vec = K % 4 == 0 && ldx % 4 == 0 && ldw % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0;
   if (mb == 0) {
     if (M > 16 || part) return FG_ERR_ARG;
     const int blocks = (N + 15) / 16;
-    if (vec) gemm_f32_few_kernel<true><<<blocks, 512, 0, stream>>>(x, w, y, M, N, K, ldx, ldw, ldy);
-    else gemm_f32_few_kernel<false><<<blocks, 512, 0, stream>>>(x, w, y, M, N, K, ldx, ldw, ldy);
+#define FEW_ROWS(FEW, VEC) gemm_f32_few_kernel<FEW, VEC><<<blocks, 512, 0, stream>>>(x, w, y, M, N, K, ldx, ldw, ldy)
+    if (M <= 8) {
+      if (vec) FEW_ROWS(true, true);
+      else FEW_ROWS(true, false);
+    } else {
+      if (vec) FEW_ROWS(false, true);
+      else FEW_ROWS(false, false);
+    }
+#undef FEW_ROWS
     return fg_launch_status();
   }
-  const int groups = (K + GF_GROUP - 1) / GF_GROUP;
-  const int wide = N % 4 == 0 && ldy % 4 == 0 && (uintptr_t)y % 16 == 0 && (uintptr_t)part % 16 == 0;
-  const int row_tiles = (M + 32 * mb - 1) / (32 * mb), col_tiles = (N + 32 * nb - 1) / (32 * nb);
-  const long long units = (long long)col_tiles * (part ? groups : 1);
-  const long long blocks = (units + 7) / 8 * 8 * row_tiles;
-  if (blocks > 2147483647LL || (part && M > 65535)) return FG_ERR_ARG;
-#define TILED(MB, NB)                                                                                               \
-  do {                                                                                                              \
-    if (vec) gemm_f32_tiled_kernel<MB, NB, true><<<(unsigned)blocks, 256, 0, stream>>>(                             \
-        x, w, y, part, M, N, K, ldx, ldw, ldy, row_tiles, col_tiles, (int)units, wide);                             \
-    else gemm_f32_tiled_kernel<MB, NB, false><<<(unsigned)blocks, 256, 0, stream>>>(                                \
-        x, w, y, part, M, N, K, ldx, ldw, ldy, row_tiles, col_tiles, (int)units, wide);                             \
-  } while (0)
-  if (mb == 1 && nb == 1) TILED(1, 1);
-  else if (mb == 1 && nb == 2) TILED(1, 2);
-  else if (mb == 2 && nb == 1) TILED(2, 1);
-  else if (mb == 2 && nb == 2) TILED(2, 2);
-  else return FG_ERR_ARG;
-#undef TILED
-  if (part) {
-    gemm_f32_sum_kernel<<<dim3((N + 1023) / 1024, M), 256, 0, stream>>>(part, y, M, N, ldy, groups, wide);
-  }
-  return fg_launch_status();
+  const GfCall c = {x, w, y, part, M, N, K, ldx, ldw, ldy, vec, stream};
+  if (nw == 4 && mb > 5) return FG_ERR_ARG;
+#define CASE(MB)                                          \
+  if (mb == MB && nw == 8) return gf_launch<MB, 2, 8>(c); \
+  if (mb == MB && nw == 4) return gf_launch<MB < 6 ? MB : 5, 2, 4>(c);
+  CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7)
+#undef CASE
+  return FG_ERR_ARG;
 }

@@ -1,6 +1,6 @@
 """``y = x W^T`` for the two precisions of the engine.
 
-float32: the engine's own fused-multiply-add kernel (``gemm.hip``), a true
+float32: the engine's own matrix-core kernels (``gemm.hip``), a true
 32-bit product whose rows do not depend on one another.  bfloat16: several
 kernels can take a product (the engine's weight-streaming MFMA kernels of
 ``gemm_skinny.hip``, narrow and wide, with or without a cut of the k range, and

@@ -9,6 +9,7 @@ is not on a GPU is refused.
 from __future__ import annotations
 
 import ctypes
+import functools
 from dataclasses import dataclass, field
 import os
 from typing import Dict, List, Optional, Sequence, Tuple
@@ -806,32 +807,46 @@ def paged_attention(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v
 GEMM_F32_GROUP = 1024
 
 
-def gemm_f32_plan(M: int, N: int, K: int, cus: int) -> Tuple[int, int, bool]:
-    """How the 32-bit product is cut: (tile rows / 32, tile columns / 32, whether every group of k has a workgroup
-    of its own); (0, 0, False): the kernel of up to 16 rows.  Every cut gives the same bits.
+def gemm_f32_tile_blocks(M: int, mb: int, nb: int) -> int:
+    """Blocks of 16 rows in a tile of :func:`gemm_f32_plan`: at most 3 (mb = 1: more loads in flight), or 5 or 7 (what
+    the registers of 2 workgroups of 4 waves or one of 8 hold a compute unit), as even as they come."""
+    blocks, most = -(-M // 16), 3 if mb == 1 else 5 if nb == 1 else 7
+    return -(-blocks // -(-blocks // most))
 
-    Measured on 256 compute units, matrices from memory (us; N x K 3072 x 3072, 16384 x 3072, 3072 x 8192).  The kernel of
-    up to 16 rows against tiles of 32 x 32 cut over k: 12 rows 19 / 58 / 40 against 31 / 55 / 39, 16 rows 20 / 62 / 43
-    against 31 / 55 / 39.  Tiles of 64 x 64 while they give 600 workgroups (2048 rows: 374, 1883, 975 against 401, 2098,
-    1051 with 64 x 32), smaller ones below (64 rows, 64 x 64 / 64 x 32 / 32 x 32: 40 / 36 / 33, 77 / 81 / 90, 60 / 51 /
-    54).  Tiles of 32 rows where the last one of 64 would be at least half empty, up to 640 rows, the better of each cut
-    over k or not (200 rows 63, 249, 145 against 77, 252, 147; 400: 105, 440, 238 against 97, 435, 245; 528: 125, 567,
-    305 against 136, 554, 303); not beyond (784: 175, 827, 439 against 177, 785, 424; 1040: 224, 1095, 568 against 220, 1018,
-    542; 2050: 438, 2124, 1151 against 427, 1957, 1135; 4110: 823, 4183, 2193 against 779, 3812, 2078).  A workgroup a
-    group of k while whole ranges would be fewer than 1536 workgroups (400 rows of 32: 105 against 116, 238 against 294;
-    16384 x 3072, 3328 workgroups: 453 against 440), if the groups' sums stay under 256 MB."""
-    if M <= 16:
+
+@functools.lru_cache(maxsize=4096)
+def gemm_f32_plan(M: int, N: int, K: int, cus: int) -> Tuple[int, int, bool]:
+    """How the 32-bit product is cut: (short or tall tiles, 1 or 2, see :func:`gemm_f32_tile_blocks`; tile columns /
+    128, whether every group of k has a workgroup of its own); (0, 0, False): the kernel of up to 16 rows.  Every cut
+    gives the same bits.
+
+    The cut whose workgroups take the least time as counted here.  32 k of a tile of b blocks of rows take 0.85 + 0.2 b
+    us where a compute unit is full (8 waves in one workgroup or two; measured 1.0 / 1.24 / 1.76 / 2.3 for b = 1 / 3 / 5 /
+    7), 0.45 + 0.19 b with 4 waves alone (0.6 / 0.98 / 1.37); the groups' sums pass through memory twice; W itself
+    comes at 5 TB/s at best; and the kernel of up to 16 rows takes 4.6 us a group of k and block of 16 outputs a
+    compute unit (16 rows, N x K 3072 x 3072 / 5120 x 3072 / 16384 x 3072 / 3072 x 8192: 18 / 30 / 60 / 41 us against 25 / 26
+    / 53 / 31 in tiles; up to 8 rows it is the faster or level everywhere, 15 / 26 / 50 / 33 against 25 / 26 / 53 / 31).
+    Counted and measured (us): 400 rows 16384 x 3072 229 and 240, 5120 x 3072 91 and 100, 3072 x 8192 158 and 148; 64 rows
+    3072 x 3072 29 and 29.  A workgroup a group only if the sums stay under 256 MB."""
+    if M <= 8:
         return 0, 0, False
-    groups = -(-K // GEMM_F32_GROUP)
-    tiles = lambda mb, nb: -(-M // (32 * mb)) * -(-N // (32 * nb))
-    splits = lambda mb, nb: groups > 1 and tiles(mb, nb) < 6 * cus and M <= 4096 and groups * M * N * 4 <= 256 << 20
-    units = lambda mb, nb: tiles(mb, nb) * (groups if splits(mb, nb) else 1)
-    mb, nb = (1 if 0 < M % 64 <= 32 and M <= 640 else 2), 2
-    if units(mb, nb) < 600 * cus // 256:
-        nb = 1
-    if units(mb, nb) < 600 * cus // 256:
-        mb = 1
-    return mb, nb, splits(mb, nb)
+    groups, streaming = -(-K // GEMM_F32_GROUP), N * K * 4 / 5e6
+    best = (4 + 4.6 * groups * -(-N // (16 * cus)), (0, 0, False)) if M <= 16 else (float("inf"), None)
+    for mb in (2, 1):
+        for nb in (2, 1):
+            b = gemm_f32_tile_blocks(M, mb, nb)
+            tiles, full, alone = -(-M // (16 * b)) * -(-N // (128 * nb)), 0.85 + 0.2 * b, 0.45 + 0.19 * b
+            for split in (False, True):
+                if split and (groups == 1 or M > 4096 or groups * M * N * 4 > 256 << 20):
+                    continue
+                units = tiles * groups if split else tiles
+                rounds, rest = divmod(units, 2 * cus // nb)
+                time = rounds * full + (full if nb == 2 or rest > cus else alone if rest else 0)
+                time *= GEMM_F32_GROUP // 32 if split else -(-K // 32)
+                time = max(time, streaming) + (5 + groups * M * N * 4 / 2e6 if split else 0)
+                if time < best[0]:
+                    best = time, (mb, nb, split)
+    return best[1]
 
 
 def gemm_f32_scratch(M: int, N: int, K: int) -> int:
@@ -842,7 +857,7 @@ def gemm_f32_scratch(M: int, N: int, K: int) -> int:
 
 def gemm_nt(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None,
             out_dtype: Optional[torch.dtype] = None) -> torch.Tensor:
-    """``x @ w.T`` with ``w [N, K]``, by the engine's own kernels: float32 on the fp32 matrix cores, bfloat16 by
+    """``x @ w.T`` with ``w [N, K]``, by the engine's own kernels: float32 on the matrix cores, bfloat16 by
     fp32 FMA (sums over k in an order fixed by K; a row's result does not depend on the others)."""
     _gpu(x, w, out)
     _need(x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[1], "x [M,K] and w [N,K] must share K")
@@ -856,8 +871,10 @@ def gemm_nt(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None
     if x.dtype == torch.float32 and out.dtype == torch.float32:
         mb, nb, split = gemm_f32_plan(M, N, K, compute_units())
         part = torch.empty((-(-K // GEMM_F32_GROUP), M, N), dtype=torch.float32, device=x.device) if split else None
+        blocks = gemm_f32_tile_blocks(M, mb, nb) if mb else 0
         st = _lib.load("gemm").fg_gemm_f32(
-            _ptr(x), _ptr(w), _ptr(out), _ptr(part), M, N, K, x.stride(0), w.stride(0), out.stride(0), mb, nb, _stream(out))
+            _ptr(x), _ptr(w), _ptr(out), _ptr(part), M, N, K, x.stride(0), w.stride(0), out.stride(0), blocks, 4 * nb,
+            _stream(out))
         _check(st, "gemm_nt")
         return out
     for m0 in range(0, M, 65535 * 64):  # grid.y limit

@@ -452,6 +452,48 @@ def test_gemm_f32_bits_around_the_line_of_the_narrow_tiles(ops, N, K):
         assert torch.equal(ops.gemm_nt(x[:M], w), full[:M]), M
 
 
+@pytest.mark.parametrize("K", [24, 128, 156, 1056, 2200])
+@pytest.mark.parametrize("blocks,waves", [(b, w) for w in (4, 8) for b in range(1, 8 if w == 8 else 6)])
+def test_gemm_f32_every_tile_gives_the_bits_of_the_few_rows_kernel(ops, blocks, waves, K):
+    """Every tile of the many-rows kernel, with and without a workgroup a group of k: rows and outputs that end inside
+    a block, k inside a step, a segment and a group; within the longest chain of additions (4 instructions of 8
+    products at a time, 5 segments' parts, 8 segments, the groups)."""
+    from fastgen_amd.kernels import _lib
+
+    torch.manual_seed(100 * blocks + K)
+    M, N = 16 * blocks + 5, 32 * waves + 37  # two tiles each way, both last ones ragged
+    x, w = torch.randn(M, K).to(DEV), torch.randn(N, K).to(DEV)
+    few = torch.cat([ops.gemm_nt(x[m:m + 8], w) for m in range(0, M, 8)])
+    assert ops.gemm_f32_plan(8, N, K, 256) == (0, 0, False)
+    y, part = torch.full_like(few, 7.0), torch.empty(-(-K // 1024), M, N, device=DEV)
+    for p in (None, part):
+        st = _lib.load("gemm").fg_gemm_f32(ops._ptr(x), ops._ptr(w), ops._ptr(y), ops._ptr(p), M, N, K, K, K, N, blocks,
+                                           waves, ops._stream(y))
+        assert st == 0 and torch.equal(y, few)
+    bound = (32 + 8 + K / 1024 + 4) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    assert ((few.double() - x.double() @ w.double().T).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("M", [3, 12, 40, 300])
+def test_gemm_f32_infinities_and_scales(ops, M):
+    """Infinities and what rounds to one in 16 bits come out as in 32 bits; operands at far ends of the exponents lose
+    nothing (their products' parts stay above the smallest normal number)."""
+    torch.manual_seed(M)
+    N, K = 70, 1100
+    x, w = torch.randn(M, K).to(DEV), torch.randn(N, K).to(DEV)
+    x[0, 5], x[1, 1099], w[3, 7] = float("inf"), float("-inf"), float("inf")
+    x[2, :], x[2, 9] = 0.0, 3.4e38  # above the largest number of 16 bits
+    got, want = ops.gemm_nt(x, w), (x.double() @ w.double().T).float()
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    assert torch.equal(got[torch.isinf(want)], want[torch.isinf(want)])
+    ok = torch.isfinite(want[2])
+    assert torch.allclose(got[2][ok], want[2][ok], rtol=1e-6)
+    x, w = torch.randn(M, K).to(DEV), torch.randn(N, K).to(DEV)
+    plain = ops.gemm_nt(x, w)
+    for a, b in ((2.0 ** 100, 2.0 ** -80), (2.0 ** -80, 2.0 ** 60)):
+        assert torch.equal(ops.gemm_nt(x * a, w * b), plain * (a * b))
+
+
 def test_gemm_f32_plan_is_bounded(ops):
     for M in (1, 16, 17, 64, 65, 400, 4096, 4097, 200000):
         for N in (1, 64, 3072, 128256):
