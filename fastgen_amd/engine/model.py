@@ -172,6 +172,15 @@ class Model:
                         total += t.numel() * t.element_size()
         return total
 
+    def _reads_sums(self, i: int) -> bool:
+        """Whether what entry ``i`` of the order finds pending goes straight to a norm that adds up an
+        :class:`~fastgen_amd.kernels.ops.ExpertSum` (the final norm is handed tensors)."""
+        order = self.layout.order
+        if i == len(order):
+            return False
+        block = self.parts.blocks[order[i].layer]
+        return order[i].inject is None and getattr(block, "takes_sums", False) and getattr(block.mixer_norm, "takes_sums", False)
+
     # ------------------------------------------------------------- forward
     def forward(self, ctx: StepContext, stores: Sequence[LayerStore]) -> Optional[torch.Tensor]:
         """Run the step's tokens through every entry of the order; fp32
@@ -207,6 +216,8 @@ class Model:
                 after = blocks[order[i + 1].layer] if i + 1 < len(order) and order[i + 1].inject is None else None
                 next_norm = after.mixer_norm if getattr(after, "folds_norms", False) else None
                 pending = block.forward(h, pending, ctx, stores[i], next_norm=next_norm)
+            elif getattr(block, "leaves_sums", False) and h.dim() == 2 and self._reads_sums(i + 1):
+                pending = block.forward(h, None if isinstance(pending, ScaledRows) else pending, ctx, stores[i], sums=True)
             else:
                 pending = block.forward(h, None if isinstance(pending, ScaledRows) else pending, ctx, stores[i])
         if isinstance(pending, ScaledRows):

@@ -1439,6 +1439,56 @@ CONV_MAX_TAPS = 16
 class ConvInputs:
     """A causal convolution per channel that a kernel applies where it reads its rows: ``taps`` fp32 ``[C, K]`` (the
     last tap meets the token itself), and the state fp32 ``[n_slots, C, row_len]`` (slots and channels may have strides
+EXPERT_SUM_MAX_DIM = 4096
+
+
+@dataclass
+class ExpertSum:
+    """A routed feed-forward's output on its way into the residual stream, not yet added up: what :func:`moe_combine` takes
+    (without a gate and without identities).  A norm on the stream takes it where it takes rows."""
+
+    y: torch.Tensor
+    weight: torch.Tensor
+    plus: Optional[torch.Tensor]
+
+    def total(self) -> torch.Tensor:
+        """fp32 ``[1, T, dim]``."""
+        return moe_combine(self.y, self.weight, self.plus)
+
+    def add_norm(self, h: torch.Tensor, weight: torch.Tensor, eps: float, out: torch.Tensor,
+                 rows: Optional[torch.Tensor] = None) -> torch.Tensor:
+        """What :func:`add_rmsnorm` does with :meth:`total`, the same bits, in one kernel where it takes the sizes: rows
+        of up to 4,096 in eights, 16-byte aligned, in the types that a model's steps have."""
+        plus, T, top, dim = self.plus, *self.weight.shape, self.y.shape[1]
+        aligned = all(t is None or t.data_ptr() % 16 == 0 for t in (self.y, plus, h, weight, out))
+        strides = plus is None or (plus.stride(-1) == 1 and plus.stride(-2) % 8 == 0 and (plus.dim() == 2 or plus.stride(0) % 8 == 0))
+        types = out.dtype == torch.bfloat16 or (out.dtype == weight.dtype == torch.float32 and (plus is None or plus.dtype == torch.float32))
+        if dim % 8 or dim > EXPERT_SUM_MAX_DIM or not aligned or not strides or not types:
+            return add_rmsnorm(h, self.total(), weight, eps, out, rows)
+        _gpu(self.y, self.weight, plus, h, weight, out, rows)
+        _need(self.y.dtype == torch.float32 and self.y.shape[0] == T * top and self.y.is_contiguous()
+              and self.weight.dtype == torch.float32 and self.weight.is_contiguous(), "y float32 [T * top, dim], weight float32 [T, top]")
+        _need(h.dtype == torch.float32 and h.shape == (T, dim) and h.is_contiguous(), "h must be contiguous float32 [T, dim]")
+        n_rows = T if rows is None else rows.numel()
+        if rows is not None:
+            _i32(rows, "rows")
+        _need(weight.shape == (dim,) and weight.is_contiguous(), "weight must be [dim]")
+        _need(out.is_contiguous() and out.shape == (n_rows, dim), "out must be contiguous [rows, dim]")
+        ldp, n_plus, stride = dim, 0, 0
+        if plus is not None and plus.dim() == 3:
+            _need(plus.dtype == torch.float32 and plus.shape[1:] == (T, dim), "partial sums must be float32 [S, T, dim]")
+            ldp, n_plus, stride = plus.stride(1), plus.shape[0], plus.stride(0)
+        elif plus is not None:
+            _need(plus.shape == (T, dim), "plus must be [T, dim]")
+            ldp, n_plus = plus.stride(0), 1
+        st = _lib.load("moe").fg_moe_combine_norm(
+            _ptr(self.y), _ptr(self.weight), _ptr(plus), ldp, _code(plus) if plus is not None else F32, n_plus,
+            ctypes.c_longlong(stride), top, dim, _ptr(h), _ptr(weight), _code(weight), _ptr(out), _code(out), _ptr(rows), n_rows,
+            ctypes.c_float(eps), _stream(out))
+        _check(st, "moe_combine_norm")
+        return out
+
+
     of their own) whose rows hold the last ``K - 1`` inputs of earlier steps, oldest first, from column ``tail_off``
     on, with the step's vectors to find them.  ``moves``: every
     sequence of the step brings one token, and the kernel moves the tails on; else the caller does

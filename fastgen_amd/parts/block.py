@@ -111,10 +111,12 @@ class ParallelBlock:
     follows: it takes the layer before's output as ``pending`` and returns its own un-added.
 
     A feed-forward that can take the mixer's output into its last kernel (``adds_to``) returns the
-    sum as fp32 ``[1, T, dim]``; any other feed-forward's rows are added by a kernel of their own.
+    sum as fp32 ``[1, T, dim]``, or, with ``sums``, as what the norm that follows may add up itself;
+    any other feed-forward's rows are added by a kernel of their own.
     """
 
     folds_norms = False
+    leaves_sums = takes_sums = True  # ``sums``; ``pending`` goes to the mixer's norm as it is
 
     def __init__(self, mixer: Mixer, ffn: Optional[FeedForward], mixer_norm: Norm, ffn_norm: Optional[Norm] = None) -> None:
         if ffn_norm is not None:
@@ -122,13 +124,13 @@ class ParallelBlock:
         self.mixer, self.ffn, self.mixer_norm = mixer, ffn, mixer_norm
         _plain_outputs(mixer, ffn, "parallel")
 
-    def forward(self, h: torch.Tensor, pending, ctx: Any, store: LayerStore):
+    def forward(self, h: torch.Tensor, pending, ctx: Any, store: LayerStore, sums: bool = False):
         x = self.mixer_norm.forward(h, pending, ctx.act_dtype)
         mixed = self.mixer.forward(x, ctx, store)
         if self.ffn is None:
             return mixed
         if getattr(self.ffn, "adds_to", False):
-            return self.ffn.forward(x, plus=mixed)
+            return self.ffn.forward(x, plus=mixed, sums=True) if sums else self.ffn.forward(x, plus=mixed)
         fed = self.ffn.forward(x)
         if mixed.dim() == 3 or fed.dim() == 3:
             # fp32 partial sums (products whose k range was cut): all of them are the norm's to add

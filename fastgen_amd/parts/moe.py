@@ -156,9 +156,10 @@ class MoE(FeedForward):
             return 16
         return expert_tile_rows(n_rows * self.top / self.n_scored, min(self.dim, self.w_down.shape[2]))
 
-    def forward(self, x: torch.Tensor, plus: Optional[torch.Tensor] = None) -> torch.Tensor:
+    def forward(self, x: torch.Tensor, plus: Optional[torch.Tensor] = None, sums: bool = False):
         """fp32 ``[1, T, dim]``: the experts' weighted sum (plus ``plus``, rows that go to the
-        residual stream with it), for a norm to add."""
+        residual stream with it), for a norm to add.  With ``sums`` it may come as
+        :class:`~fastgen_amd.kernels.ops.ExpertSum`, for the norm to add up as well."""
         tile_rows = self.tile_rows(x.shape[0])
         if self.shared is not None:
             both = self.shared.forward(x)
@@ -173,6 +174,8 @@ class MoE(FeedForward):
         sorted_, tiles = ops.moe_sort(choice, self.n_scored, tile_rows, self.identity)
         act = ops.moe_gate_up(x, self.w_gate, self.w_up, sorted_, tiles, self.top, tile_rows, self.limit, self.alpha)
         y = ops.moe_down(act, self.w_down, sorted_, tiles, tile_rows)
+        if sums and not self.identity and not self.shared_gate:
+            return ops.ExpertSum(y, weight, plus)
         own = dict(choice=choice, n_tiled=self.n_experts, x=x) if self.identity else {}
         return ops.moe_combine(y, weight, plus, routed[2][:, 0] if self.shared_gate else None, **own)
 

@@ -15,6 +15,8 @@ class RMSNorm(Norm):
     ``unit_offset`` the checkpoint stores the weight around zero and ``1 + w`` is what multiplies
     (kept in fp32: the sum has more digits than bfloat16 holds)."""
 
+    takes_sums = True  # a routed feed-forward's output before it is added up
+
     def __init__(self, spec) -> None:
         super().__init__(spec)
         self.dim = int(spec.options["dim"])
@@ -39,7 +41,8 @@ class RMSNorm(Norm):
         """``delta`` may be :class:`~fastgen_amd.kernels.ops.PostNormed`: a sublayer's output that is normed
         itself before it is added (the norm behind a sublayer); one kernel does that norm, the addition and
         this norm.  :class:`~fastgen_amd.kernels.ops.ScaledDelta`: rows times a vector;
-        :class:`~fastgen_amd.kernels.ops.StreamTerms`: several sublayers' outputs.
+        :class:`~fastgen_amd.kernels.ops.StreamTerms`: several sublayers' outputs;
+        :class:`~fastgen_amd.kernels.ops.ExpertSum`: a routed feed-forward's, not yet added up.
         ``h`` may be several residual streams ``[S, T, dim]`` (``delta``: the
         :class:`~fastgen_amd.kernels.ops.StreamUpdate` still to be applied, or None): their sum is normed."""
         n = h.shape[-2] if rows is None else rows.numel()
@@ -52,6 +55,8 @@ class RMSNorm(Norm):
         if isinstance(delta, ops.StreamTerms):
             ops.stream_terms(h, delta, None, [(self.weight, out)], self.eps, rows)
             return out
+        if isinstance(delta, ops.ExpertSum):
+            return delta.add_norm(h, self.weight, self.eps, out, rows)
         if isinstance(delta, ops.ScaledDelta):
             return ops.add_rmsnorm(h, delta.rows, self.weight, self.eps, out, rows, delta_scale=delta.scale)
         return ops.add_rmsnorm(h, delta, self.weight, self.eps, out, rows)

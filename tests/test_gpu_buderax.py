@@ -401,3 +401,27 @@ def test_packed_experts_wide_tiles_give_the_rows_bits(tile_rows):
     tiles = ops.moe_max_tiles(T * top, E, tile_rows)
     assert tiles * -(-F // 128) >= 170 and tiles * -(-D // 256) >= 170
     test_packed_experts_give_the_rows_bits(E, top, T, D, F, tile_rows)
+
+
+@pytest.mark.parametrize("dim,top", [(8, 1), (264, 3), (2048, 4), (2056, 5), (4096, 9), (4104, 2), (100, 2)])
+@pytest.mark.parametrize("kind", ["bf16", "bf16 none", "bf16 sums", "fp32", "fp32 weight"])
+def test_expert_sum_inside_the_norm_gives_the_bits_of_the_two_kernels(dim, top, kind):
+    """A routed feed-forward's sum added up by the norm that follows it: every type a step has, whole and gathered rows
+    (which leave h as it is), sizes at the edges of a workgroup's share and beyond what the kernel takes."""
+    from fastgen_amd.kernels import ops
+    torch.manual_seed(dim + top)
+    T = 7
+    act = torch.float32 if kind.startswith("fp32") and kind != "fp32 weight" else torch.bfloat16
+    y, weight = torch.randn(T * top, dim, device="cuda"), torch.rand(T, top, device="cuda")
+    plus = None if kind == "bf16 none" else torch.randn(3, T, dim, device="cuda") if kind == "bf16 sums" else (
+        torch.randn(T, dim, device="cuda").to(act))
+    w = torch.randn(dim, device="cuda").to(torch.float32 if kind == "fp32 weight" else act)
+    h0 = torch.randn(T, dim, device="cuda")
+    pending = ops.ExpertSum(y, weight, plus)
+    for rows in (None, torch.tensor([6, 0, 6], dtype=torch.int32, device="cuda")):
+        n = T if rows is None else 3
+        h, want_h = h0.clone(), h0.clone()
+        out, want = torch.empty(n, dim, dtype=act, device="cuda"), torch.empty(n, dim, dtype=act, device="cuda")
+        pending.add_norm(h, w, 1e-6, out, rows)
+        ops.add_rmsnorm(want_h, pending.total(), w, 1e-6, want, rows)
+        assert torch.equal(out, want) and torch.equal(h, want_h)
