@@ -262,6 +262,48 @@ __device__ __forceinline__ void load_q(bf16x8 (&qop)[NKS], const bf16_t* qrow, b
   }
 }
 
+// An output gate [tokens, heads * HD] (g null: none): the attention's rounded output times it, or times its sigmoid, where
+// the output is stored: rounded, multiplied and rounded again, as a kernel of its own behind this one does it.  The
+// sigmoid takes the hardware's exponential and reciprocal (errors of 1e-7, far below the rounding that follows): the
+// library's, 64 a lane at the end of a prompt's workgroup, cost 5 us of the 10 that the other kernel took.
+struct OutGate {
+  const bf16_t* g;
+  int stride, sigmoid;
+};
+__device__ __forceinline__ float gated(float o, float g, int sigmoid) {
+  return (float)(__bf16)o * (sigmoid ? __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-g * LOG2E)) : g);
+}
+__device__ __forceinline__ bf16x4 out4(const f32x4 o) {
+  bf16x4 v;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[i] = (__bf16)o[i];
+  return v;
+}
+__device__ __forceinline__ bf16x4 gated4(const f32x4 o, const bf16x4 g, int sigmoid) {
+  bf16x4 v;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[i] = (__bf16)gated(o[i], (float)g[i], sigmoid);
+  return v;
+}
+// A row's blocks of 16 outputs, times inv, to token t's columns from c on (four a lane of each): the gate's loads all
+// in flight together (1897 tokens of 16 heads: 40.8 us without a gate, 42.6 with its sigmoid; the other
+// kernel takes 10.5).
+__device__ __forceinline__ void store_row(bf16_t* __restrict__ out, int out_stride, const f32x4 (&o)[NDB], float inv,
+                                          const OutGate& gate, int t, int c) {
+  bf16_t* to = out + (size_t)t * out_stride + c;
+  if (gate.g) {  // uniform
+    const bf16_t* from = gate.g + (size_t)t * gate.stride + c;
+    bf16x4 g[NDB];
+#pragma unroll
+    for (int db = 0; db < NDB; ++db) g[db] = *(const bf16x4*)(from + 16 * db);
+#pragma unroll
+    for (int db = 0; db < NDB; ++db) *(bf16x4*)(to + 16 * db) = gated4(o[db] * inv, g[db], gate.sigmoid);
+  } else {
+#pragma unroll
+    for (int db = 0; db < NDB; ++db) *(bf16x4*)(to + 16 * db) = out4(o[db] * inv);
+  }
+}
+
 // ------------------------------------------------------------------ split
 // The key ranges of the items are cut into chunks of the same number of tiles for every item, so that
 // a long sequence gives many workgroups and a short one few, each with about the same work; a plan
@@ -389,7 +431,8 @@ __global__ __launch_bounds__(256) void attn_split_kernel(
     const bf16_t* __restrict__ k_pages, const bf16_t* __restrict__ v_pages,
     const int* __restrict__ block_table, int bt_stride, const int* __restrict__ plan,
     float* __restrict__ part_o, float* __restrict__ part_ml, int n_heads, int n_kv, int page_size,
-    int page_shift, float scale, int window, const float* __restrict__ sinks, const float* __restrict__ dist) {
+    int page_shift, float scale, int window, const float* __restrict__ sinks, const float* __restrict__ dist,
+    const OutGate gate) {
   __shared__ float o_s[2][16][HD + 1];
   __shared__ float ml_s[2][16][2];
   const int lane = threadIdx.x % FG_WAVE, wave = threadIdx.x / FG_WAVE;
@@ -517,17 +560,9 @@ __global__ __launch_bounds__(256) void attn_split_kernel(
   if (r16 >= it.n_tok * G) return;
   const int t_out = it.tok0 + r16 / G, h_out = kvh * G + r16 % G;
   if (alone) {
-    bf16_t* orow = out + (size_t)t_out * out_stride + (size_t)h_out * HD;
     // a sink: one more term exp(sink) in the denominator (maxima are in base 2 and scaled), no value
     if (sinks) l += __builtin_amdgcn_exp2f(sinks[h_out] * LOG2E - m);
-    const float inv = 1.f / l;
-#pragma unroll
-    for (int db = 0; db < NDB; ++db) {
-      bf16x4 v;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = (__bf16)(o[db][i] * inv);
-      *(bf16x4*)(orow + 16 * db + 4 * g) = v;
-    }
+    store_row(out, out_stride, o, 1.f / l, gate, t_out, h_out * HD + 4 * g);
   } else {
     const size_t row = ((size_t)chunk * n_kv + kvh) * 16 + r16;
 #pragma unroll
@@ -550,7 +585,7 @@ __global__ __launch_bounds__(256) void attn_split_kernel(
 // wave, one chunk a lane, together with the first eight partial outputs.
 __global__ void attn_combine_rows_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
                                     const int* __restrict__ plan, bf16_t* __restrict__ out, int out_stride,
-                                    int n_heads, int n_kv, const float* __restrict__ sinks) {
+                                    int n_heads, int n_kv, const float* __restrict__ sinks, const OutGate gate) {
   __shared__ float f_s[COMBINE_MAX_SPLITS];  // weight of each chunk's partial output: 2^(m_s - M) / L
   const int r = blockIdx.x, kvh = blockIdx.y, chunk = blockIdx.z, d = threadIdx.x;
   const int G = n_heads / n_kv;
@@ -562,6 +597,8 @@ __global__ void attn_combine_rows_kernel(const float* __restrict__ part_o, const
   if (r >= it.n_tok * G) return;  // uniform: a row beyond the item, its partial results are never written
   const size_t row0 = ((size_t)chunk * n_kv + kvh) * 16 + r, step = (size_t)n_kv * 16;  // rows from chunk to chunk
   const int dc = min(d, HD - 1);
+  const int t = it.tok0 + r / G, h = kvh * G + r % G;
+  const float g = gate.g ? (float)gate.g[(size_t)t * gate.stride + (size_t)h * HD + dc] : 0.f;
   float first_o[8];
 #pragma unroll
   for (int u = 0; u < 8; ++u) first_o[u] = part_o[(row0 + (size_t)min(u, n_splits - 1) * step) * HD + dc];
@@ -603,8 +640,7 @@ __global__ void attn_combine_rows_kernel(const float* __restrict__ part_o, const
 #pragma unroll
     for (int u = 0; u < 8; ++u) O += s0 + u < n_splits ? f_s[s0 + u] * v[u] : 0.f;
   }
-  const int t = it.tok0 + r / G, h = kvh * G + r % G;
-  out[(size_t)t * out_stride + (size_t)h * HD + d] = (bf16_t)O;
+  out[(size_t)t * out_stride + (size_t)h * HD + d] = (bf16_t)(gate.g ? gated(O, g, gate.sigmoid) : O);
 }
 
 // For long chunk lists (many sequences; sixteen times fewer workgroups): grid (n_kv, max_chunks), 256
@@ -612,7 +648,8 @@ __global__ void attn_combine_rows_kernel(const float* __restrict__ part_o, const
 // lane; then every thread adds up four neighbouring head dimensions of a row (or of several rows).
 __global__ __launch_bounds__(256) void attn_combine_kernel(
     const float* __restrict__ part_o, const float* __restrict__ part_ml, const int* __restrict__ plan,
-    bf16_t* __restrict__ out, int out_stride, int n_heads, int n_kv, const float* __restrict__ sinks) {
+    bf16_t* __restrict__ out, int out_stride, int n_heads, int n_kv, const float* __restrict__ sinks,
+    const OutGate gate) {
   __shared__ float f_s[16][COMBINE_MAX_SPLITS];  // weight of each chunk's partial output: 2^(m_s - M) / L
   const int kvh = blockIdx.x, chunk = blockIdx.y, tid = threadIdx.x;
   const int lane = tid % FG_WAVE, wave = tid / FG_WAVE;
@@ -681,10 +718,9 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(
         if (s0 + u < n_splits) O += f_s[r][s0 + u] * v[u];
     }
     const int t = it.tok0 + r / G, h = kvh * G + r % G;
-    bf16x4 o4;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) o4[i] = (__bf16)O[i];
-    *(bf16x4*)(out + (size_t)t * out_stride + (size_t)h * HD + d) = o4;
+    const size_t c = (size_t)h * HD + d;
+    *(bf16x4*)(out + (size_t)t * out_stride + c) =
+        gate.g ? gated4(O, *(const bf16x4*)(gate.g + (size_t)t * gate.stride + c), gate.sigmoid) : out4(O);
   }
 }
 
@@ -707,19 +743,26 @@ extern "C" int fg_attn_plan(const int* items, int n_items, int window, int max_c
   return fg_launch_status();
 }
 
+static bool gate_ok(const void* gate, int stride, int n_heads) {
+  return !gate || (stride % 4 == 0 && (uintptr_t)gate % 8 == 0 && stride >= n_heads * HD);
+}
+
 // plan: what fg_attn_plan made of the items, with the same n_items, max_chunks and window.
 // max_rows: no item has more rows (tokens x heads of a kv head's group) than this, at most 16.
 // part_o: fp32 [max_chunks * n_kv * 16 * HD], part_ml: the same rows x 2.
 // dist: fp32 [n_heads, 2], in the build with FG_DIST_BIAS (null in the others).
 // sinks: fp32 [n_heads] or null: head h's softmax has one more term exp(sinks[h]) in its denominator, which
 // brings no value.
+// gate: bf16 rows of n_heads * hd, 8-byte aligned as are their strides, or null (see OutGate).
 extern "C" int fg_attn_split_sink(const void* q, int q_stride, void* out, int out_stride, const void* k_pages,
                                   const void* v_pages, const int* block_table, int bt_stride, const int* plan,
                                   int n_items, int max_chunks, int max_rows, float* part_o, float* part_ml,
                                   int n_heads, int n_kv, int hd, int page_size, float scale, int window,
-                                  const float* sinks, const float* dist, hipStream_t stream) {
+                                  const float* sinks, const float* dist, const void* gate, int gate_stride,
+                             int gate_sigmoid, hipStream_t stream) {
   if (n_items <= 0) return FG_OK;
-  if (DIST_BIAS != (dist != nullptr)) return FG_ERR_ARG;
+  if (DIST_BIAS != (dist != nullptr) || !gate_ok(gate, gate_stride, n_heads)) return FG_ERR_ARG;
+  const OutGate og{(const bf16_t*)gate, gate_stride, gate_sigmoid};
   if (hd != HD || n_kv <= 0 || n_heads % n_kv || n_heads / n_kv > 16 || page_size < 8 || page_size % 8 ||
       !(scale > 0.f) || max_chunks < 2 * n_items || max_chunks > 65535 || n_kv > 65535 ||
       q_stride % 8 || out_stride % 4 || !plan || !part_o || !part_ml || max_rows < 1 || max_rows > 16)
@@ -728,15 +771,15 @@ extern "C" int fg_attn_split_sink(const void* q, int q_stride, void* out, int ou
   attn_split_kernel<PERM><<<dim3(n_kv, max_chunks), 256, 0, stream>>>(                                         \
       (const bf16_t*)q, q_stride, (bf16_t*)out, out_stride, (const bf16_t*)k_pages, (const bf16_t*)v_pages,    \
       block_table, bt_stride, plan, part_o, part_ml, n_heads, n_kv, page_size,                                 \
-      page_shift_of(page_size), scale, window, sinks, dist)
+      page_shift_of(page_size), scale, window, sinks, dist, og)
   if (page_size % 32 == 0) LAUNCH(true); else LAUNCH(false);
 #undef LAUNCH
   if ((long long)max_chunks * n_kv * max_rows <= COMBINE_ROWS_MAX_GROUPS)
     attn_combine_rows_kernel<<<dim3(max_rows, n_kv, max_chunks), HD < 64 ? 64 : HD, 0, stream>>>(
-        part_o, part_ml, plan, (bf16_t*)out, out_stride, n_heads, n_kv, sinks);
+        part_o, part_ml, plan, (bf16_t*)out, out_stride, n_heads, n_kv, sinks, og);
   else
     attn_combine_kernel<<<dim3(n_kv, max_chunks), 256, 0, stream>>>(
-        part_o, part_ml, plan, (bf16_t*)out, out_stride, n_heads, n_kv, sinks);
+        part_o, part_ml, plan, (bf16_t*)out, out_stride, n_heads, n_kv, sinks, og);
   return fg_launch_status();
 }
 
@@ -747,7 +790,7 @@ extern "C" int fg_attn_split(const void* q, int q_stride, void* out, int out_str
                              hipStream_t stream) {
   return fg_attn_split_sink(q, q_stride, out, out_stride, k_pages, v_pages, block_table, bt_stride, plan, n_items,
                             max_chunks, max_rows, part_o, part_ml, n_heads, n_kv, hd, page_size, scale, window,
-                            nullptr, nullptr, stream);
+                            nullptr, nullptr, nullptr, 0, 0, stream);
 }
 
 // ----------------------------------------------------------- without allocation
@@ -863,7 +906,7 @@ __global__ __launch_bounds__(TILE_PAIR ? 512 : 256, TILE_PAIR ? 1 : 2) void attn
     const bf16_t* __restrict__ k_pages, const bf16_t* __restrict__ v_pages,
     const int* __restrict__ block_table, int bt_stride, const int* __restrict__ items, int n_heads, int n_kv,
     int page_size, int page_shift, float scale, int window, const float* __restrict__ sinks,
-    const float* __restrict__ dist) {
+    const float* __restrict__ dist, const OutGate gate) {
   constexpr bool PERM = PAGES >= PAGES_CHUNK, WHOLE = PAGES == PAGES_TILE;
   constexpr int TILE_RB = TILE_PAIR ? 2 : 1;  // row blocks a wave holds
   constexpr int TILE_THREADS = TILE_PAIR ? 512 : 256;
@@ -1133,16 +1176,9 @@ __global__ __launch_bounds__(TILE_PAIR ? 512 : 256, TILE_PAIR ? 1 : 2) void attn
     lsum += __shfl_xor(lsum, 32, FG_WAVE);
     const int row = (rg * RB + rb) * 16 + r16;
     if (row < it.n_tok * G) {
-      bf16_t* orow = out + (size_t)(it.tok0 + row / G) * out_stride + (size_t)(kvh * G + row % G) * HD;
+      const int t = it.tok0 + row / G, c = (kvh * G + row % G) * HD + 4 * g;
       if (sinks) lsum += __builtin_amdgcn_exp2f(sinks[kvh * G + row % G] * LOG2E - m[rb]);
-      const float inv = 1.f / lsum;
-#pragma unroll
-      for (int db = 0; db < NDB; ++db) {
-        bf16x4 v;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = (__bf16)(o[rb][db][i] * inv);
-        *(bf16x4*)(orow + 16 * db + 4 * g) = v;
-      }
+      store_row(out, out_stride, o[rb], 1.f / lsum, gate, t, c);
     }
   }
 }
@@ -1150,13 +1186,13 @@ __global__ __launch_bounds__(TILE_PAIR ? 512 : 256, TILE_PAIR ? 1 : 2) void attn
 struct TileArgs {
   const bf16_t* q; int q_stride; bf16_t* out; int out_stride; const bf16_t* k_pages; const bf16_t* v_pages;
   const int* block_table; int bt_stride; const int* items; int n_items, n_heads, n_kv, page_size; float scale;
-  int window; const float* sinks; const float* dist; hipStream_t stream;
+  int window; const float* sinks; const float* dist; OutGate gate; hipStream_t stream;
 };
 template <int PAGES, bool PAIR>
 static void launch_pages(const TileArgs& a) {
   attn_tile_kernel<PAGES, PAIR><<<a.n_items * a.n_kv, PAIR ? 512 : 256, 0, a.stream>>>(
       a.q, a.q_stride, a.out, a.out_stride, a.k_pages, a.v_pages, a.block_table, a.bt_stride, a.items, a.n_heads,
-      a.n_kv, a.page_size, page_shift_of(a.page_size), a.scale, a.window, a.sinks, a.dist);
+      a.n_kv, a.page_size, page_shift_of(a.page_size), a.scale, a.window, a.sinks, a.dist, a.gate);
 }
 template <bool PAIR>
 static void launch_tile(const TileArgs& a) {
@@ -1174,16 +1210,17 @@ template <> struct PairForm<false> { static void go(const TileArgs&) {} };
 extern "C" int fg_attn_tile_sink(const void* q, int q_stride, void* out, int out_stride, const void* k_pages,
                                  const void* v_pages, const int* block_table, int bt_stride, const int* items,
                                  int n_items, int item_rows, int n_heads, int n_kv, int hd, int page_size,
-                                 float scale, int window, const float* sinks, const float* dist,
-                                 hipStream_t stream) {
+                                 float scale, int window, const float* sinks, const float* dist, const void* gate,
+                                 int gate_stride, int gate_sigmoid, hipStream_t stream) {
   if (n_items <= 0) return FG_OK;
-  if (DIST_BIAS != (dist != nullptr)) return FG_ERR_ARG;
+  if (DIST_BIAS != (dist != nullptr) || !gate_ok(gate, gate_stride, n_heads)) return FG_ERR_ARG;
   if (hd != HD || !(scale > 0.f) || n_kv <= 0 || n_heads % n_kv || n_heads / n_kv > item_rows || page_size < 8 || page_size % 8 ||
       (long long)n_items * n_kv > 2147483647LL || q_stride % 8 || out_stride % 4 ||
       (item_rows != TILE_ROWS && item_rows != TILE_ROWS_SMALL))
     return FG_ERR_ARG;
   const TileArgs a{(const bf16_t*)q, q_stride, (bf16_t*)out, out_stride, (const bf16_t*)k_pages, (const bf16_t*)v_pages,
-                   block_table, bt_stride, items, n_items, n_heads, n_kv, page_size, scale, window, sinks, dist, stream};
+                   block_table, bt_stride, items, n_items, n_heads, n_kv, page_size, scale, window, sinks, dist,
+                   OutGate{(const bf16_t*)gate, gate_stride, gate_sigmoid}, stream};
   if (TILE_PAIR_OK && item_rows == TILE_ROWS) PairForm<TILE_PAIR_OK>::go(a);
   else launch_tile<false>(a);
   return fg_launch_status();
@@ -1194,7 +1231,7 @@ extern "C" int fg_attn_tile(const void* q, int q_stride, void* out, int out_stri
                             int n_items, int item_rows, int n_heads, int n_kv, int hd, int page_size, float scale,
                             int window, hipStream_t stream) {
   return fg_attn_tile_sink(q, q_stride, out, out_stride, k_pages, v_pages, block_table, bt_stride, items, n_items,
-                           item_rows, n_heads, n_kv, hd, page_size, scale, window, nullptr, nullptr, stream);
+                           item_rows, n_heads, n_kv, hd, page_size, scale, window, nullptr, nullptr, nullptr, 0, 0, stream);
 }
 
 // query rows (tokens x heads of a kv head's group) of one item of fg_attn_tile: of the larger form, or

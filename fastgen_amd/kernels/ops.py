@@ -668,7 +668,8 @@ def paged_attention_mfma(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tens
                          plan: Optional[torch.Tensor] = None, max_chunks: Optional[int] = None,
                          min_tiles: int = 4, max_rows: int = 16, tile_rows: Optional[int] = None,
                          exact_weights: bool = False, sinks: Optional[torch.Tensor] = None,
-                         distance: Optional[torch.Tensor] = None) -> torch.Tensor:
+                         distance: Optional[torch.Tensor] = None, gate: Optional[torch.Tensor] = None,
+                         gate_sigmoid: bool = True) -> torch.Tensor:
     """bf16 attention on the matrix cores.  ``small_items`` / ``big_items`` are
     device int32 ``[n, 4]`` lists from :func:`attention_items` (16-byte aligned);
     every query token of the step must be covered by exactly one item.
@@ -680,8 +681,17 @@ def paged_attention_mfma(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tens
     the current stream waits for it before this returns (not while a graph is captured, not with
     ``FG_ONE_STREAM=1``).  ``exact_weights``: the build of the kernels in which the softmax weights enter
     the product with the values as two bfloat16 terms (16 significant bits).  ``sinks`` and ``distance``: as
-    :func:`paged_attention_general` (a build of the kernels with exact weights takes the distance bias)."""
-    _gpu(q, out, k_pages, v_pages, block_table, small_items, big_items, plan, sinks, distance)
+    :func:`paged_attention_general` (a build of the kernels with exact weights takes the distance bias).  ``gate`` and
+    ``gate_sigmoid``: what :func:`gate_mul` does with them behind the attention, done where the output is stored (the
+    same bits), for bfloat16 rows that can be read in fours; else by that kernel."""
+    _gpu(q, out, k_pages, v_pages, block_table, small_items, big_items, plan, sinks, distance, gate)
+    if gate is not None and (gate.dtype != torch.bfloat16 or gate.data_ptr() % 8 or gate.stride(0) % 4):
+        return gate_mul(paged_attention_mfma(q, out, k_pages, v_pages, block_table, small_items, big_items, n_heads, scale,
+                                             window, plan, max_chunks, min_tiles, max_rows, tile_rows, exact_weights, sinks,
+                                             distance), gate, gate_sigmoid)
+    _need(gate is None or (gate.dim() == 2 and gate.shape[0] == q.shape[0] and gate.shape[1] >= out.shape[1]
+                           and gate.stride(1) == 1), "gate must be [T, >= H*hd] with unit column stride")
+    gate_args = (_ptr(gate), gate.stride(0) if gate is not None else 0, int(gate_sigmoid))
     _sinks_ok(sinks, n_heads)
     _distance_ok(distance, n_heads)
     dist = distance is not None
@@ -726,7 +736,7 @@ def paged_attention_mfma(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tens
         st = lib.fg_attn_split_sink(
             _ptr(q), q.stride(0), _ptr(out), out.stride(0), _ptr(k_pages), _ptr(v_pages), _ptr(block_table),
             block_table.stride(0), _ptr(plan), n, max_chunks, max_rows, _ptr(part_o), _ptr(part_ml), n_heads, n_kv, hd,
-            page_size, ctypes.c_float(scale), int(window or 0), _ptr(sinks), _ptr(distance), _stream(q))
+            page_size, ctypes.c_float(scale), int(window or 0), _ptr(sinks), _ptr(distance), *gate_args, _stream(q))
         _check(st, "attn_split")
     if big_items is not None and big_items.numel():
         tile_rows = attention_tile_rows(hd, False, exact_weights, dist) if tile_rows is None else int(tile_rows)
@@ -738,7 +748,7 @@ def paged_attention_mfma(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tens
         st = lib.fg_attn_tile_sink(
             _ptr(q), q.stride(0), _ptr(out), out.stride(0), _ptr(k_pages), _ptr(v_pages), _ptr(block_table),
             block_table.stride(0), _ptr(big_items), big_items.numel() // 4, tile_rows, n_heads, n_kv, hd, page_size,
-            ctypes.c_float(scale), int(window or 0), _ptr(sinks), _ptr(distance),
+            ctypes.c_float(scale), int(window or 0), _ptr(sinks), _ptr(distance), *gate_args,
             ctypes.c_void_p(beside.cuda_stream) if beside else _stream(q))
         _check(st, "attn_tile")
         if beside is not None:
@@ -749,9 +759,11 @@ def paged_attention_mfma(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tens
 def paged_attention(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor,
                     group, ctx, n_heads: int, scale: float, window: int = 0,
                     exact_weights: bool = False, sinks: Optional[torch.Tensor] = None,
-                    distance: Optional[torch.Tensor] = None) -> torch.Tensor:
+                    distance: Optional[torch.Tensor] = None, gate: Optional[torch.Tensor] = None,
+                    gate_sigmoid: bool = True) -> torch.Tensor:
     """Attention for one step: picks the kernel for the step's dtype and shape.
     ``exact_weights``: see :func:`paged_attention_mfma` (the general kernel's weights are fp32 anyway).
+    ``gate``, ``gate_sigmoid``: an output gate as :func:`gate_mul` takes it.
 
     ``group`` carries the block table of the layer's cache group, ``ctx`` the
     step's per-token vectors (``fastgen_amd.engine.context``).  bfloat16 with a
@@ -762,8 +774,9 @@ def paged_attention(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v
     n_kv, hd = k_pages.shape[1], k_pages.shape[3]
     G = n_heads // n_kv
     if q.dtype != torch.bfloat16 or hd % 16 or hd > MFMA_MAX_HEAD_DIM or G > 16:
-        return paged_attention_general(q, out, k_pages, v_pages, group.block_table, ctx.seq_of_token,
-                                       ctx.positions, n_heads, scale, window, sinks, distance)
+        paged_attention_general(q, out, k_pages, v_pages, group.block_table, ctx.seq_of_token,
+                                ctx.positions, n_heads, scale, window, sinks, distance)
+        return out if gate is None else gate_mul(out, gate, gate_sigmoid)
     dist = distance is not None
     items_key = ("attention_items", G, hd, n_kv)  # (how a step is cut into items depends on all three)
     plan = ctx.scratch.get(items_key)
@@ -799,7 +812,8 @@ def paged_attention(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v
     rows = G * int(ctx.q_lens.max()) if big_d is None else 16
     return paged_attention_mfma(q, out, k_pages, v_pages, group.block_table, small_d, big_d, n_heads, scale,
                                 window, split_plan, chunks, max_rows=min(16, rows), tile_rows=tile_rows,
-                                exact_weights=exact_weights, sinks=sinks, distance=distance)
+                                exact_weights=exact_weights, sinks=sinks, distance=distance, gate=gate,
+                                gate_sigmoid=gate_sigmoid)
 
 
 # ----------------------------------------------------------------------- gemm
@@ -1425,20 +1439,6 @@ def moe_combine(y: torch.Tensor, weight: torch.Tensor, plus: Optional[torch.Tens
     return out
 
 
-class _ConvIn(ctypes.Structure):
-    _fields_ = [("w", ctypes.c_void_p), ("taps", ctypes.c_int), ("state", ctypes.c_void_p),
-                ("slot_stride", ctypes.c_longlong), ("channels", ctypes.c_int), ("row_len", ctypes.c_int),
-                ("tail_off", ctypes.c_int), ("slot_ids", ctypes.c_void_p), ("seq_of_token", ctypes.c_void_p),
-                ("q_start", ctypes.c_void_p), ("move", ctypes.c_int)]
-
-
-CONV_MAX_TAPS = 16
-
-
-@dataclass
-class ConvInputs:
-    """A causal convolution per channel that a kernel applies where it reads its rows: ``taps`` fp32 ``[C, K]`` (the
-    last tap meets the token itself), and the state fp32 ``[n_slots, C, row_len]`` (slots and channels may have strides
 EXPERT_SUM_MAX_DIM = 4096
 
 
@@ -1489,6 +1489,20 @@ class ExpertSum:
         return out
 
 
+class _ConvIn(ctypes.Structure):
+    _fields_ = [("w", ctypes.c_void_p), ("taps", ctypes.c_int), ("state", ctypes.c_void_p),
+                ("slot_stride", ctypes.c_longlong), ("channels", ctypes.c_int), ("row_len", ctypes.c_int),
+                ("tail_off", ctypes.c_int), ("slot_ids", ctypes.c_void_p), ("seq_of_token", ctypes.c_void_p),
+                ("q_start", ctypes.c_void_p), ("move", ctypes.c_int)]
+
+
+CONV_MAX_TAPS = 16
+
+
+@dataclass
+class ConvInputs:
+    """A causal convolution per channel that a kernel applies where it reads its rows: ``taps`` fp32 ``[C, K]`` (the
+    last tap meets the token itself), and the state fp32 ``[n_slots, C, row_len]`` (slots and channels may have strides
     of their own) whose rows hold the last ``K - 1`` inputs of earlier steps, oldest first, from column ``tail_off``
     on, with the step's vectors to find them.  ``moves``: every
     sequence of the step brings one token, and the kernel moves the tails on; else the caller does

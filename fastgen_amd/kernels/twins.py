@@ -258,7 +258,8 @@ def paged_attention_mfma(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tens
                          plan=None, max_chunks=None, min_tiles: int = 4, max_rows: int = 16,
                          tile_rows=None, exact_weights: bool = False,
                          sinks: Optional[torch.Tensor] = None,
-                         distance: Optional[torch.Tensor] = None) -> torch.Tensor:
+                         distance: Optional[torch.Tensor] = None, gate: Optional[torch.Tensor] = None,
+                         gate_sigmoid: bool = True) -> torch.Tensor:
     """The same attention for tokens listed as items (sequence, first flat token, tokens, position of the
     first token).  How the kernels cut the work (``plan`` and what follows it) does not change the result;
     ``exact_weights`` only says how many digits of the softmax weights the kernel keeps (here: all)."""
@@ -270,18 +271,21 @@ def paged_attention_mfma(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tens
         for b, first, n, pos in items.reshape(-1, 4).tolist():
             seq_of_token[first : first + n] = b
             positions[first : first + n] = torch.arange(pos, pos + n, dtype=torch.int32)
-    return paged_attention_general(q, out, k_pages, v_pages, block_table, seq_of_token, positions, n_heads, scale,
-                                   window, sinks, distance)
+    paged_attention_general(q, out, k_pages, v_pages, block_table, seq_of_token, positions, n_heads, scale,
+                            window, sinks, distance)
+    return out if gate is None else gate_mul(out, gate, gate_sigmoid)
 
 
 def paged_attention(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor,
                     group, ctx, n_heads: int, scale: float, window: int = 0,
                     exact_weights: bool = False, sinks: Optional[torch.Tensor] = None,
-                    distance: Optional[torch.Tensor] = None) -> torch.Tensor:
+                    distance: Optional[torch.Tensor] = None, gate: Optional[torch.Tensor] = None,
+                    gate_sigmoid: bool = True) -> torch.Tensor:
     """Attention of one step: the block table from the layer's cache group, sequences and positions of the
     tokens from the step's context."""
-    return paged_attention_general(q, out, k_pages, v_pages, group.block_table, ctx.seq_of_token, ctx.positions,
-                                   n_heads, scale, window, sinks, distance)
+    paged_attention_general(q, out, k_pages, v_pages, group.block_table, ctx.seq_of_token, ctx.positions,
+                            n_heads, scale, window, sinks, distance)
+    return out if gate is None else gate_mul(out, gate, gate_sigmoid)
 
 
 def gemm_nt(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None,

@@ -228,9 +228,8 @@ class Attention(RowsMixer):
             gate_done = False
         out = torch.empty((rows.shape[0], q_width), dtype=rows.dtype, device=rows.device)
         ops.paged_attention(qkv, out, store.k_pages, store.v_pages, group, ctx, self.n_heads, self.scale,
-                            self.window or 0, exact_weights=self.exact_weights, sinks=self.sinks, distance=self.distance)
-        if gate is not None:
-            ops.gate_mul(out, gate, sigmoid=not gate_done)
+                            self.window or 0, exact_weights=self.exact_weights, sinks=self.sinks, distance=self.distance,
+                            gate=gate, gate_sigmoid=not gate_done)
         return linear(out, self.wo, partials_ok=True, residual=then)
 
     def _rope_table(self, ctx: Any):

@@ -425,3 +425,43 @@ def test_expert_sum_inside_the_norm_gives_the_bits_of_the_two_kernels(dim, top, 
         pending.add_norm(h, w, 1e-6, out, rows)
         ops.add_rmsnorm(want_h, pending.total(), w, 1e-6, want, rows)
         assert torch.equal(out, want) and torch.equal(h, want_h)
+
+
+@pytest.mark.parametrize("hd", [16, 80, 128, 192, 256])
+@pytest.mark.parametrize("lens", [[1, 1, 1], [1, 300, 2], [130]])  # split alone and in chunks; beside tiles; tiles
+def test_output_gate_inside_the_attention(hd, lens):
+    """Both forms of the gate, rows with strides of their own, one that cannot be read in fours: what the two kernels give,
+    the same bits where the gate is taken as it is; its sigmoid within errors of 1e-6 that may move the last rounding
+    (one unit in the last of 8 bits)."""
+    from types import SimpleNamespace
+
+    import numpy as np
+
+    from fastgen_amd.kernels import ops
+    torch.manual_seed(hd + sum(lens))
+    H, KV, P, cached = 6, 2, 16, [20, 700, 1500][: len(lens)]
+    pages = [-(-(n + c) // P) for n, c in zip(lens, cached)]
+    table = torch.zeros(len(lens), max(pages), dtype=torch.int32)
+    order = torch.randperm(sum(pages)).int()
+    for i, n in enumerate(pages):
+        table[i, :n], order = order[:n], order[n:]
+    k = torch.randn(sum(pages), KV, P, hd, device="cuda").bfloat16()
+    v = torch.randn(sum(pages), KV, hd, P, device="cuda").bfloat16()
+    T = sum(lens)
+    q = torch.randn(T, H * hd, device="cuda").bfloat16()
+    wide = torch.randn(T, H * hd + 12, device="cuda").bfloat16()
+    starts = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+
+    def run(**gate):
+        ctx = SimpleNamespace(scratch={}, seq_records=None, q_lens=np.array(lens, dtype=np.int32), q_start_host=starts,
+                              n_cached=np.array(cached, dtype=np.int32), graph_capacity=0)
+        return ops.paged_attention(q, torch.empty_like(q), k, v, SimpleNamespace(block_table=table.cuda()), ctx, H,
+                                   hd ** -0.5, **gate)
+
+    plain = run()
+    for gate in (wide[:, 8:], wide[:, : H * hd], wide[:, 3 : 3 + H * hd], wide[:, : H * hd].float()):
+        for sigmoid in (True, False):
+            got, want = run(gate=gate, gate_sigmoid=sigmoid).float(), ops.gate_mul(plain.clone(), gate, sigmoid).float()
+            if not sigmoid:
+                assert torch.equal(got, want)
+            assert ((got - want).abs() <= 2.0 ** -7 * want.abs()).all() and (got != want).float().mean() < 1e-3
