@@ -31,11 +31,11 @@ typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // ------------------------------------------------------------------- route
-// A workgroup one token (few tokens: decode) or four.  Logits: the WAVES waves take the experts in turns of EPW (a wave
+// A workgroup one token, four or eight.  Logits: the WAVES waves take the experts in turns of EPW (a wave
 // reads the rows of x once for its EPW experts, eight elements a lane and round, and an expert's row of the router once
-// for its tokens; the lanes' partial sums are added by the wave in a fixed order), into LDS.  Few tokens get 16 waves and
-// 2 experts a turn, so that the router's rows are asked for by many waves at once; many tokens 4 waves, 4 experts a turn and
-// 4 tokens, or the router would be read from the L2 once a token.  From there on a wave a token: the `top` largest (ties:
+// for its tokens; the lanes' partial sums are added by the wave in a fixed order, the same in every form), into LDS.  A
+// turn is a chain of reads from the L2, so many waves of two experts each; several tokens, or the router would be read
+// from the L2 once a token.  From there on a wave a token: the `top` largest (ties:
 // the lower expert) by a wave-wide argmax repeated `top` times, and the softmax over them.  LDS, per token: n_experts +
 // n_extra logits, then `top` chosen values, then n_experts scores, then n_groups ranks.
 //
@@ -237,15 +237,25 @@ extern "C" int fg_moe_route_mode(const void* x, int ldx, int dtype, const float*
 #define GO(T, WAVES, EPW, TOK)                                                                                        \
   moe_route_kernel<T, WAVES, EPW, TOK><<<(n_tokens + TOK - 1) / TOK, 64 * WAVES, TOK * lds, stream>>>(                 \
       (const T*)x, ldx, wr, bias, n_tokens, dim, n_experts, top, choice, weight, mode)
-  // (many tokens: four a workgroup from where that still leaves a workgroup for every compute unit)
-  const int form = n_tokens <= 64 ? 0 : n_tokens < 1024 || 4 * lds > 60000 ? 1 : 2;
-  if (dtype == FG_F32) {
-    if (form == 0) GO(float, 16, 2, 1); else if (form == 1) GO(float, 4, 4, 1); else GO(float, 4, 4, 4);
-  } else if (dtype == FG_BF16) {
-    if (form == 0) GO(bf16_t, 16, 2, 1); else if (form == 1) GO(bf16_t, 4, 4, 1); else GO(bf16_t, 4, 4, 4);
-  } else {
-    return FG_ERR_ARG;
-  }
+  // Tokens a workgroup: one while every token's workgroup has a place at once, then four, then eight, as their logits fit.
+  // Waves: 16 of two rows a turn, or 8 where the router has no more than 16 rows.  bf16, router in the caches, us, 32
+  // experts of 2048 with 4 waves of four rows before: 65 / 300 / 700 / 1024 / 1897 / 6000 tokens 6.6 / 9.8 / 10.2 / 11.1 / 13.9
+  // / 36.5 against 10.0 / 10.7 / 12.4 / 15.6 / 17.0 / 38.3; 128 of 4096 25.7 / 41 / 48 / 55 / 74 / 206 against 49 / 52 / 61 / 74 /
+  // 100 / 274; 16 of 1024 4.2 / 5.7 / 5.8 / 5.9 / 7.3 / 14.1 against 5.1 / 5.3 / 5.8 / 7.4 / 7.8 / 15.0.
+  const int tok = n_tokens <= 256 || 4 * lds > 60000 ? 1 : n_tokens <= 1280 || 8 * lds > 60000 ? 4 : 8;
+  const bool few_rows = n_experts + n_extra <= 16;
+#define FORMS(T)                                                   \
+  do {                                                             \
+    if (tok == 1) GO(T, 16, 2, 1);                                 \
+    else if (tok == 4 && few_rows) GO(T, 8, 2, 4);                 \
+    else if (tok == 4) GO(T, 16, 2, 4);                            \
+    else if (few_rows) GO(T, 8, 2, 8);                             \
+    else GO(T, 16, 2, 8);                                          \
+  } while (0)
+  if (dtype == FG_F32) FORMS(float);
+  else if (dtype == FG_BF16) FORMS(bf16_t);
+  else return FG_ERR_ARG;
+#undef FORMS
 #undef GO
   return fg_launch_status();
 }
