@@ -310,11 +310,16 @@ __device__ __forceinline__ void store_row(bf16_t* __restrict__ out, int out_stri
 // kernel does the cutting on the device from the items alone, so that a captured step cuts anew
 // for the lengths of every replay.
 //
-// plan: int32 [4 + 8 * max_chunks]
+// plan: int32 [4 + 8 * max_chunks], or with the second list [4 + 16 * max_chunks]
 //   [0] tiles per chunk, [1] chunks in use;
 //   from [4] on, 8 ints a chunk, the chunks of an item one after the other: the item's record
 //   (sequence, first flat token, tokens, first position), first tile, end tile, chunks of the item
-//   (0: this chunk is not in use), number of this chunk among its item's.
+//   (0: this chunk is not in use), number of this chunk among its item's;
+//   from [4 + 8 * max_chunks] on the same chunks, longest first, with their place in the first list instead of that
+//   number: the order in which the split kernel takes them.  Chunks of items of many lengths are of many lengths too, and
+//   with more workgroups than places a long one begun last is what the kernel ends with: 64 sequences of 100 to 2,400
+//   keys, 8 kv heads, 760 workgroups on 512 places: 74 us a layer
+//   in the items' order, 66 so.
 #define COMBINE_MAX_SPLITS 256
 #define COMBINE_ROWS_MAX_GROUPS 8192  // up to this many workgroups the combine takes a workgroup a row
 constexpr int PLAN_HEAD = 4;
@@ -333,9 +338,10 @@ __device__ __forceinline__ void item_tiles(const Item& it, int window, int& t_lo
 // that this gives the longest item, as even as they can be (33 tiles in chunks of 12, 12, 9, not 16,
 // 16, 1: sequences of one length are the common case), if the chunks of all items still fit.
 __global__ __launch_bounds__(256) void attn_plan_kernel(const int* __restrict__ items, int n_items, int window,
-                                                        int max_chunks, int min_tiles, int* __restrict__ plan) {
+                                                        int max_chunks, int min_tiles, int ordered,
+                                                        int* __restrict__ plan) {
   __shared__ int red_s[256], red_m[256];
-  __shared__ int carry;
+  __shared__ int carry, place[64];
   const int tid = threadIdx.x;
   int tot = 0, mx = 0;
   for (int i = tid; i < n_items; i += 256) {
@@ -420,6 +426,36 @@ __global__ __launch_bounds__(256) void attn_plan_kernel(const int* __restrict__ 
     plan[0] = ts;
     plan[1] = used;
   }
+  if (!ordered) return;  // uniform
+  // The second list: by length in 64 steps, longest first (a chunk has at most ts tiles).
+  int* list = chunks + (size_t)max_chunks * 8;
+  auto step_of = [&](const int4 b) { return (int)((long long)(ts - (b.y - b.x)) * 64 / ts); };  // 0 .. 63
+  if (tid < 64) place[tid] = 0;
+  __syncthreads();  // (and the records of the first list are there for all threads)
+  for (int j = tid; j < used; j += 256) atomicAdd(&place[step_of(*(const int4*)(chunks + (size_t)j * 8 + 4))], 1);
+  __syncthreads();
+  if (tid < 64) {
+    const int n = place[tid];
+    int sum = n;
+    for (int w = 1; w < 64; w <<= 1) {
+      const int add = __shfl_up(sum, w, FG_WAVE);
+      sum += tid >= w ? add : 0;
+    }
+    place[tid] = sum - n;
+  }
+  __syncthreads();
+  for (int j = tid; j < max_chunks; j += 256) {
+    int4 a{0, 0, 0, 0}, b{0, 0, 0, 0};
+    int at = j;
+    if (j < used) {
+      a = *(const int4*)(chunks + (size_t)j * 8);
+      b = *(const int4*)(chunks + (size_t)j * 8 + 4);
+      at = atomicAdd(&place[step_of(b)], 1);
+      b.w = j;
+    }
+    *(int4*)(list + (size_t)at * 8) = a;
+    *(int4*)(list + (size_t)at * 8 + 4) = b;
+  }
 }
 
 // grid (n_kv, max_chunks), 256 threads: one chunk of one item (a run of at most 16 rows:
@@ -429,18 +465,19 @@ template <bool PERM /* the page's value slots are permuted: page_size % 32 == 0 
 __global__ __launch_bounds__(256) void attn_split_kernel(
     const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, int out_stride,
     const bf16_t* __restrict__ k_pages, const bf16_t* __restrict__ v_pages,
-    const int* __restrict__ block_table, int bt_stride, const int* __restrict__ plan,
+    const int* __restrict__ block_table, int bt_stride, const int* __restrict__ list,
     float* __restrict__ part_o, float* __restrict__ part_ml, int n_heads, int n_kv, int page_size,
     int page_shift, float scale, int window, const float* __restrict__ sinks, const float* __restrict__ dist,
-    const OutGate gate) {
+    const OutGate gate, int ordered) {
   __shared__ float o_s[2][16][HD + 1];
   __shared__ float ml_s[2][16][2];
   const int lane = threadIdx.x % FG_WAVE, wave = threadIdx.x / FG_WAVE;
   const int r16 = lane & 15, g = lane >> 4;
-  const int kvh = blockIdx.x, chunk = blockIdx.y;
+  const int kvh = blockIdx.x;
   const int G = n_heads / n_kv;
-  const int* rec = plan + PLAN_HEAD + (size_t)chunk * 8;
+  const int* rec = list + (size_t)blockIdx.y * 8;
   const int4 rec_a = *(const int4*)rec, rec_b = *(const int4*)(rec + 4);
+  const int chunk = ordered ? rec_b.w : blockIdx.y;
   if (rec_b.z == 0) return;  // uniform: a chunk that is not in use
   const Item it{rec_a.x, rec_a.y, rec_a.z, rec_a.w};
   const int t_begin = rec_b.x, t_end = rec_b.y;
@@ -731,23 +768,30 @@ static int page_shift_of(int page_size) {
 }
 
 // ints of a plan of max_chunks chunks
-extern "C" long long fg_attn_plan_ints(int max_chunks) { return PLAN_HEAD + 8LL * max_chunks; }
+extern "C" long long fg_attn_plan_ints(int max_chunks) { return PLAN_HEAD + 16LL * max_chunks; }
 
 // Cuts the items (int32 [n_items][4], 16-byte aligned) into chunks: see the layout of `plan` above.
-// max_chunks >= 2 * n_items; min_tiles: a chunk's tiles are a multiple of it (4: one tile a wave).
-extern "C" int fg_attn_plan(const int* items, int n_items, int window, int max_chunks, int min_tiles, int* plan,
-                            hipStream_t stream) {
+// max_chunks >= 2 * n_items; min_tiles: a chunk's tiles are a multiple of it (4: one tile a wave).  ordered: with the
+// second list.
+extern "C" int fg_attn_plan_ordered(const int* items, int n_items, int window, int max_chunks, int min_tiles, int ordered,
+                                    int* plan, hipStream_t stream) {
   if (n_items <= 0) return FG_OK;
   if (!items || !plan || max_chunks < 2 * n_items || min_tiles < 1) return FG_ERR_ARG;
-  attn_plan_kernel<<<1, 256, 0, stream>>>(items, n_items, window, max_chunks, min_tiles, plan);
+  attn_plan_kernel<<<1, 256, 0, stream>>>(items, n_items, window, max_chunks, min_tiles, ordered, plan);
   return fg_launch_status();
+}
+
+// The first list only: int32 [4 + 8 * max_chunks].
+extern "C" int fg_attn_plan(const int* items, int n_items, int window, int max_chunks, int min_tiles, int* plan,
+                            hipStream_t stream) {
+  return fg_attn_plan_ordered(items, n_items, window, max_chunks, min_tiles, 0, plan, stream);
 }
 
 static bool gate_ok(const void* gate, int stride, int n_heads) {
   return !gate || (stride % 4 == 0 && (uintptr_t)gate % 8 == 0 && stride >= n_heads * HD);
 }
 
-// plan: what fg_attn_plan made of the items, with the same n_items, max_chunks and window.
+// plan: what fg_attn_plan_ordered made of the items, with the same n_items, max_chunks, window and `ordered`.
 // max_rows: no item has more rows (tokens x heads of a kv head's group) than this, at most 16.
 // part_o: fp32 [max_chunks * n_kv * 16 * HD], part_ml: the same rows x 2.
 // dist: fp32 [n_heads, 2], in the build with FG_DIST_BIAS (null in the others).
@@ -759,7 +803,7 @@ extern "C" int fg_attn_split_sink(const void* q, int q_stride, void* out, int ou
                                   int n_items, int max_chunks, int max_rows, float* part_o, float* part_ml,
                                   int n_heads, int n_kv, int hd, int page_size, float scale, int window,
                                   const float* sinks, const float* dist, const void* gate, int gate_stride,
-                             int gate_sigmoid, hipStream_t stream) {
+                             int gate_sigmoid, int ordered, hipStream_t stream) {
   if (n_items <= 0) return FG_OK;
   if (DIST_BIAS != (dist != nullptr) || !gate_ok(gate, gate_stride, n_heads)) return FG_ERR_ARG;
   const OutGate og{(const bf16_t*)gate, gate_stride, gate_sigmoid};
@@ -770,8 +814,9 @@ extern "C" int fg_attn_split_sink(const void* q, int q_stride, void* out, int ou
 #define LAUNCH(PERM)                                                                                           \
   attn_split_kernel<PERM><<<dim3(n_kv, max_chunks), 256, 0, stream>>>(                                         \
       (const bf16_t*)q, q_stride, (bf16_t*)out, out_stride, (const bf16_t*)k_pages, (const bf16_t*)v_pages,    \
-      block_table, bt_stride, plan, part_o, part_ml, n_heads, n_kv, page_size,                                 \
-      page_shift_of(page_size), scale, window, sinks, dist, og)
+      block_table, bt_stride, plan + PLAN_HEAD + (ordered ? 8LL * max_chunks : 0), part_o, part_ml, n_heads,   \
+      n_kv, page_size,                                                                                         \
+      page_shift_of(page_size), scale, window, sinks, dist, og, ordered)
   if (page_size % 32 == 0) LAUNCH(true); else LAUNCH(false);
 #undef LAUNCH
   if ((long long)max_chunks * n_kv * max_rows <= COMBINE_ROWS_MAX_GROUPS)
@@ -790,7 +835,7 @@ extern "C" int fg_attn_split(const void* q, int q_stride, void* out, int out_str
                              hipStream_t stream) {
   return fg_attn_split_sink(q, q_stride, out, out_stride, k_pages, v_pages, block_table, bt_stride, plan, n_items,
                             max_chunks, max_rows, part_o, part_ml, n_heads, n_kv, hd, page_size, scale, window,
-                            nullptr, nullptr, nullptr, 0, 0, stream);
+                            nullptr, nullptr, nullptr, 0, 0, 0, stream);
 }
 
 // ----------------------------------------------------------- without allocation

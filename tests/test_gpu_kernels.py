@@ -1096,6 +1096,25 @@ def test_paged_attention_mfma_many_decoding_sequences(ops, n_items, cut):
 
 
 @pytest.mark.parametrize("n_items,window,max_chunks,min_tiles", [
+    (17, 0, 34, 4), (17, 0, 128, 4), (64, 0, 128, 4), (300, 777, 1024, 1), (513, 0, 4096, 2)])
+def test_attention_plan_lists_the_longest_chunks_first(ops, n_items, window, max_chunks, min_tiles):
+    """The order in which the split kernel takes the chunks: every chunk in use once, with its place, lengths that do not
+    grow by more than a 64th of the longest, and nothing behind them."""
+    import numpy as np
+
+    rng = np.random.default_rng(n_items)
+    pos0 = rng.integers(0, 6000, n_items)
+    items = np.stack([np.arange(n_items), np.arange(n_items), np.ones(n_items), pos0], axis=1).astype(np.int32)
+    plan = ops.attention_plan(torch.from_numpy(items.reshape(-1)).to(DEV), n_items, max_chunks, 128, window, min_tiles).cpu().numpy()
+    ts, used = int(plan[0]), int(plan[1])
+    chunks, taken = plan[4: 4 + 16 * max_chunks].reshape(2, max_chunks, 8)
+    assert sorted(taken[:used, 7]) == list(range(used)) and (taken[used:] == 0).all()
+    assert (taken[:used, :7] == chunks[taken[:used, 7], :7]).all()
+    length = taken[:used, 5] - taken[:used, 4]
+    assert (length[1:] <= length[:-1] + -(-ts // 64)).all()
+
+
+@pytest.mark.parametrize("n_items,window,max_chunks,min_tiles", [
     (1, 0, 2, 4), (7, 0, 128, 4), (7, 100, 14, 1), (300, 0, 600, 4), (300, 777, 1024, 1), (513, 0, 4096, 2),
     (8, 0, 40, 4), (12, 0, 44, 4), (40, 0, 81, 2),
 ])
