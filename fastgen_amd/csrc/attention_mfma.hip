@@ -288,21 +288,23 @@ __device__ __forceinline__ bf16x4 gated4(const f32x4 o, const bf16x4 g, int sigm
 // A row's blocks of 16 outputs, times inv, to token t's columns from c on (four a lane of each): the gate's loads all
 // in flight together (1897 tokens of 16 heads: 40.8 us without a gate, 42.6 with its sigmoid; the other
 // kernel takes 10.5).
-__device__ __forceinline__ void store_row(bf16_t* __restrict__ out, int out_stride, const f32x4 (&o)[NDB], float inv,
-                                          const OutGate& gate, int t, int c) {
+__device__ __forceinline__ void store_row(bf16_t* __restrict__ out, int out_stride, const f32x4 (&o)[NDB], float inv, int t,
+                                          int c, const OutGate gate) {
   bf16_t* to = out + (size_t)t * out_stride + c;
-  if (gate.g) {  // uniform
-    const bf16_t* from = gate.g + (size_t)t * gate.stride + c;
-    bf16x4 g[NDB];
+  const bf16_t* from = gate.g + (size_t)t * gate.stride + c;
+  bf16x4 g[NDB];
 #pragma unroll
-    for (int db = 0; db < NDB; ++db) g[db] = *(const bf16x4*)(from + 16 * db);
+  for (int db = 0; db < NDB; ++db) g[db] = *(const bf16x4*)(from + 16 * db);
 #pragma unroll
-    for (int db = 0; db < NDB; ++db) *(bf16x4*)(to + 16 * db) = gated4(o[db] * inv, g[db], gate.sigmoid);
-  } else {
-#pragma unroll
-    for (int db = 0; db < NDB; ++db) *(bf16x4*)(to + 16 * db) = out4(o[db] * inv);
-  }
+  for (int db = 0; db < NDB; ++db) *(bf16x4*)(to + 16 * db) = gated4(o[db] * inv, g[db], gate.sigmoid);
 }
+__device__ __forceinline__ void store_row(bf16_t* __restrict__ out, int out_stride, const f32x4 (&o)[NDB], float inv, int t,
+                                          int c) {
+  bf16_t* to = out + (size_t)t * out_stride + c;
+#pragma unroll
+  for (int db = 0; db < NDB; ++db) *(bf16x4*)(to + 16 * db) = out4(o[db] * inv);
+}
+__device__ __forceinline__ const OutGate& the_gate(const OutGate& gate) { return gate; }
 
 // ------------------------------------------------------------------ split
 // The key ranges of the items are cut into chunks of the same number of tiles for every item, so that
@@ -461,14 +463,20 @@ __global__ __launch_bounds__(256) void attn_plan_kernel(const int* __restrict__ 
 // grid (n_kv, max_chunks), 256 threads: one chunk of one item (a run of at most 16 rows:
 // n_tok * (H / KV) <= 16) for one kv head.  An item of one chunk writes its output rows; of more, the
 // chunk's (max, sum, O) go to part_o / part_ml at row (chunk * n_kv + kv head) * 16 + row.
-template <bool PERM /* the page's value slots are permuted: page_size % 32 == 0 */>
+// The gate, where there is one, is one more argument, and `ordered` rides on page_shift: the others are 128 bytes, two
+// cache lines of arguments, and a third, which every workgroup would wait for, costs a launch 0.4 us.  (So in the
+// combine kernels, whose arguments without a gate are one line.)
+#define SHIFT_ORDERED 64  // added to page_shift (-1 .. 30): the list is the ordered one
+template <bool PERM /* the page's value slots are permuted: page_size % 32 == 0 */, class... GATE>
 __global__ __launch_bounds__(256) void attn_split_kernel(
     const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, int out_stride,
     const bf16_t* __restrict__ k_pages, const bf16_t* __restrict__ v_pages,
     const int* __restrict__ block_table, int bt_stride, const int* __restrict__ list,
     float* __restrict__ part_o, float* __restrict__ part_ml, int n_heads, int n_kv, int page_size,
-    int page_shift, float scale, int window, const float* __restrict__ sinks, const float* __restrict__ dist,
-    const OutGate gate, int ordered) {
+    int shift_ordered, float scale, int window, const float* __restrict__ sinks, const float* __restrict__ dist,
+    const GATE... gate) {
+  const bool ordered = shift_ordered >= SHIFT_ORDERED - 1;
+  const int page_shift = ordered ? shift_ordered - SHIFT_ORDERED : shift_ordered;
   __shared__ float o_s[2][16][HD + 1];
   __shared__ float ml_s[2][16][2];
   const int lane = threadIdx.x % FG_WAVE, wave = threadIdx.x / FG_WAVE;
@@ -599,7 +607,7 @@ __global__ __launch_bounds__(256) void attn_split_kernel(
   if (alone) {
     // a sink: one more term exp(sink) in the denominator (maxima are in base 2 and scaled), no value
     if (sinks) l += __builtin_amdgcn_exp2f(sinks[h_out] * LOG2E - m);
-    store_row(out, out_stride, o, 1.f / l, gate, t_out, h_out * HD + 4 * g);
+    store_row(out, out_stride, o, 1.f / l, t_out, h_out * HD + 4 * g, gate...);
   } else {
     const size_t row = ((size_t)chunk * n_kv + kvh) * 16 + r16;
 #pragma unroll
@@ -620,9 +628,10 @@ __global__ __launch_bounds__(256) void attn_split_kernel(
 // For short chunk lists (a few sequences): grid (16 rows, n_kv, max_chunks), one thread per head
 // dimension (at least one wave), a workgroup a row.  The chunks' maxima and sums are read by the first
 // wave, one chunk a lane, together with the first eight partial outputs.
+template <class... GATE>
 __global__ void attn_combine_rows_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
                                     const int* __restrict__ plan, bf16_t* __restrict__ out, int out_stride,
-                                    int n_heads, int n_kv, const float* __restrict__ sinks, const OutGate gate) {
+                                    int n_heads, int n_kv, const float* __restrict__ sinks, const GATE... gate) {
   __shared__ float f_s[COMBINE_MAX_SPLITS];  // weight of each chunk's partial output: 2^(m_s - M) / L
   const int r = blockIdx.x, kvh = blockIdx.y, chunk = blockIdx.z, d = threadIdx.x;
   const int G = n_heads / n_kv;
@@ -635,7 +644,11 @@ __global__ void attn_combine_rows_kernel(const float* __restrict__ part_o, const
   const size_t row0 = ((size_t)chunk * n_kv + kvh) * 16 + r, step = (size_t)n_kv * 16;  // rows from chunk to chunk
   const int dc = min(d, HD - 1);
   const int t = it.tok0 + r / G, h = kvh * G + r % G;
-  const float g = gate.g ? (float)gate.g[(size_t)t * gate.stride + (size_t)h * HD + dc] : 0.f;
+  float g = 0.f;
+  if constexpr (sizeof...(GATE)) {
+    const OutGate& og = the_gate(gate...);
+    g = (float)og.g[(size_t)t * og.stride + (size_t)h * HD + dc];
+  }
   float first_o[8];
 #pragma unroll
   for (int u = 0; u < 8; ++u) first_o[u] = part_o[(row0 + (size_t)min(u, n_splits - 1) * step) * HD + dc];
@@ -677,16 +690,18 @@ __global__ void attn_combine_rows_kernel(const float* __restrict__ part_o, const
 #pragma unroll
     for (int u = 0; u < 8; ++u) O += s0 + u < n_splits ? f_s[s0 + u] * v[u] : 0.f;
   }
-  out[(size_t)t * out_stride + (size_t)h * HD + d] = (bf16_t)(gate.g ? gated(O, g, gate.sigmoid) : O);
+  if constexpr (sizeof...(GATE)) O = gated(O, g, the_gate(gate...).sigmoid);
+  out[(size_t)t * out_stride + (size_t)h * HD + d] = (bf16_t)O;
 }
 
 // For long chunk lists (many sequences; sixteen times fewer workgroups): grid (n_kv, max_chunks), 256
 // threads, a workgroup for the 16 rows x HD of a kv head.  Wave w weighs rows 4w .. 4w+3, one chunk a
 // lane; then every thread adds up four neighbouring head dimensions of a row (or of several rows).
+template <class... GATE>
 __global__ __launch_bounds__(256) void attn_combine_kernel(
     const float* __restrict__ part_o, const float* __restrict__ part_ml, const int* __restrict__ plan,
     bf16_t* __restrict__ out, int out_stride, int n_heads, int n_kv, const float* __restrict__ sinks,
-    const OutGate gate) {
+    const GATE... gate) {
   __shared__ float f_s[16][COMBINE_MAX_SPLITS];  // weight of each chunk's partial output: 2^(m_s - M) / L
   const int kvh = blockIdx.x, chunk = blockIdx.y, tid = threadIdx.x;
   const int lane = tid % FG_WAVE, wave = tid / FG_WAVE;
@@ -756,8 +771,13 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(
     }
     const int t = it.tok0 + r / G, h = kvh * G + r % G;
     const size_t c = (size_t)h * HD + d;
-    *(bf16x4*)(out + (size_t)t * out_stride + c) =
-        gate.g ? gated4(O, *(const bf16x4*)(gate.g + (size_t)t * gate.stride + c), gate.sigmoid) : out4(O);
+    bf16x4* to = (bf16x4*)(out + (size_t)t * out_stride + c);
+    if constexpr (sizeof...(GATE)) {
+      const OutGate& og = the_gate(gate...);
+      *to = gated4(O, *(const bf16x4*)(og.g + (size_t)t * og.stride + c), og.sigmoid);
+    } else {
+      *to = out4(O);
+    }
   }
 }
 
@@ -797,13 +817,14 @@ static bool gate_ok(const void* gate, int stride, int n_heads) {
 // dist: fp32 [n_heads, 2], in the build with FG_DIST_BIAS (null in the others).
 // sinks: fp32 [n_heads] or null: head h's softmax has one more term exp(sinks[h]) in its denominator, which
 // brings no value.
+// merge 0: items of several chunks are left as their partial results.
 // gate: bf16 rows of n_heads * hd, 8-byte aligned as are their strides, or null (see OutGate).
 extern "C" int fg_attn_split_sink(const void* q, int q_stride, void* out, int out_stride, const void* k_pages,
                                   const void* v_pages, const int* block_table, int bt_stride, const int* plan,
                                   int n_items, int max_chunks, int max_rows, float* part_o, float* part_ml,
                                   int n_heads, int n_kv, int hd, int page_size, float scale, int window,
                                   const float* sinks, const float* dist, const void* gate, int gate_stride,
-                             int gate_sigmoid, int ordered, hipStream_t stream) {
+                             int gate_sigmoid, int ordered, int merge, hipStream_t stream) {
   if (n_items <= 0) return FG_OK;
   if (DIST_BIAS != (dist != nullptr) || !gate_ok(gate, gate_stride, n_heads)) return FG_ERR_ARG;
   const OutGate og{(const bf16_t*)gate, gate_stride, gate_sigmoid};
@@ -811,20 +832,33 @@ extern "C" int fg_attn_split_sink(const void* q, int q_stride, void* out, int ou
       !(scale > 0.f) || max_chunks < 2 * n_items || max_chunks > 65535 || n_kv > 65535 ||
       q_stride % 8 || out_stride % 4 || !plan || !part_o || !part_ml || max_rows < 1 || max_rows > 16)
     return FG_ERR_ARG;
-#define LAUNCH(PERM)                                                                                           \
-  attn_split_kernel<PERM><<<dim3(n_kv, max_chunks), 256, 0, stream>>>(                                         \
-      (const bf16_t*)q, q_stride, (bf16_t*)out, out_stride, (const bf16_t*)k_pages, (const bf16_t*)v_pages,    \
-      block_table, bt_stride, plan + PLAN_HEAD + (ordered ? 8LL * max_chunks : 0), part_o, part_ml, n_heads,   \
-      n_kv, page_size,                                                                                         \
-      page_shift_of(page_size), scale, window, sinks, dist, og, ordered)
-  if (page_size % 32 == 0) LAUNCH(true); else LAUNCH(false);
+  const int shift = page_shift_of(page_size) + (ordered ? SHIFT_ORDERED : 0);
+  const int* list = plan + PLAN_HEAD + (ordered ? 8LL * max_chunks : 0);
+#define LAUNCH(PERM, ...)                                                                                        \
+  attn_split_kernel<PERM><<<dim3(n_kv, max_chunks), 256, 0, stream>>>(                                           \
+      (const bf16_t*)q, q_stride, (bf16_t*)out, out_stride, (const bf16_t*)k_pages, (const bf16_t*)v_pages,      \
+      block_table, bt_stride, list, part_o, part_ml, n_heads, n_kv, page_size, shift, scale, window, sinks, dist \
+      __VA_ARGS__)
+#define COMMA ,
+  if (page_size % 32 == 0) {
+    if (gate) LAUNCH(true, COMMA og); else LAUNCH(true);
+  } else {
+    if (gate) LAUNCH(false, COMMA og); else LAUNCH(false);
+  }
 #undef LAUNCH
-  if ((long long)max_chunks * n_kv * max_rows <= COMBINE_ROWS_MAX_GROUPS)
-    attn_combine_rows_kernel<<<dim3(max_rows, n_kv, max_chunks), HD < 64 ? 64 : HD, 0, stream>>>(
-        part_o, part_ml, plan, (bf16_t*)out, out_stride, n_heads, n_kv, sinks, og);
-  else
-    attn_combine_kernel<<<dim3(n_kv, max_chunks), 256, 0, stream>>>(
-        part_o, part_ml, plan, (bf16_t*)out, out_stride, n_heads, n_kv, sinks, og);
+  if (!merge) return fg_launch_status();
+#define COMBINE(...)                                                                                             \
+  do {                                                                                                           \
+    if ((long long)max_chunks * n_kv * max_rows <= COMBINE_ROWS_MAX_GROUPS)                                      \
+      attn_combine_rows_kernel<<<dim3(max_rows, n_kv, max_chunks), HD < 64 ? 64 : HD, 0, stream>>>(              \
+          part_o, part_ml, plan, (bf16_t*)out, out_stride, n_heads, n_kv, sinks __VA_ARGS__);                    \
+    else                                                                                                         \
+      attn_combine_kernel<<<dim3(n_kv, max_chunks), 256, 0, stream>>>(                                           \
+          part_o, part_ml, plan, (bf16_t*)out, out_stride, n_heads, n_kv, sinks __VA_ARGS__);                    \
+  } while (0)
+  if (gate) COMBINE(COMMA og); else COMBINE();
+#undef COMBINE
+#undef COMMA
   return fg_launch_status();
 }
 
@@ -835,7 +869,7 @@ extern "C" int fg_attn_split(const void* q, int q_stride, void* out, int out_str
                              hipStream_t stream) {
   return fg_attn_split_sink(q, q_stride, out, out_stride, k_pages, v_pages, block_table, bt_stride, plan, n_items,
                             max_chunks, max_rows, part_o, part_ml, n_heads, n_kv, hd, page_size, scale, window,
-                            nullptr, nullptr, nullptr, 0, 0, 0, stream);
+                            nullptr, nullptr, nullptr, 0, 0, 0, 1, stream);
 }
 
 // ----------------------------------------------------------- without allocation
@@ -1223,7 +1257,8 @@ __global__ __launch_bounds__(TILE_PAIR ? 512 : 256, TILE_PAIR ? 1 : 2) void attn
     if (row < it.n_tok * G) {
       const int t = it.tok0 + row / G, c = (kvh * G + row % G) * HD + 4 * g;
       if (sinks) lsum += __builtin_amdgcn_exp2f(sinks[kvh * G + row % G] * LOG2E - m[rb]);
-      store_row(out, out_stride, o[rb], 1.f / lsum, gate, t, c);
+      if (gate.g) store_row(out, out_stride, o[rb], 1.f / lsum, t, c, gate);  // uniform
+      else store_row(out, out_stride, o[rb], 1.f / lsum, t, c);
     }
   }
 }

@@ -491,6 +491,118 @@ __global__ __launch_bounds__(256, MB <= 4 ? 3 : 2) void gemm_skinny64_kernel(
   }
 }
 
+// One row, the output projection of an attention whose chunks' partial results nobody has merged yet (AttnParts): every
+// workgroup merges them into the row it multiplies by, while its first loads of W are in flight, which spares the merge a
+// kernel of its own.  The row is summed and rounded as that kernel does it (a head's weights are added chunk by chunk
+// instead of over a wave's lanes).  An attention of one chunk has stored the row itself.  It pays while the partial
+// results, which every workgroup reads, are few: see the caller's rule.
+#define MERGE_MAX_CHUNKS 16
+#define MERGE_MAX_HEADS 128
+#define MERGE_MAX_K 8192
+struct AttnParts {
+  const float* part_o;   // [chunk][n_kv][16][hd], of a chunk the rows of a kv head's query heads
+  const float* part_ml;  // [chunk][n_kv][16][2]: their maxima (in base 2) and sums
+  const int* n_chunks;   // on the device
+  const float* sinks;    // [n_heads] or null: one more term of a head's sum
+  int n_heads, n_kv, hd;
+};
+template <int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void gemm_skinny_attn_kernel(const bf16_t* __restrict__ x, const AttnParts at,
+                                                                      const bf16_t* __restrict__ w, int ldw, int N,
+                                                                      Residual rs) {  // (128 bytes of arguments)
+  const int K = at.n_heads * at.hd;
+  constexpr int U = 8, FLY = 4;  // k steps in flight; chunks in flight
+  __shared__ float red[WAVES][256];
+  __shared__ float rscale[16];
+  __shared__ float f_s[MERGE_MAX_HEADS][MERGE_MAX_CHUNKS];  // weight of each chunk's partial output
+  __shared__ __attribute__((aligned(16))) bf16_t xs[MERGE_MAX_K];
+  const ResidualRegs pre = residual_begin(rs, blockIdx.x * 16, 1, N);
+  const int tid = threadIdx.x, lane = tid % FG_WAVE, wave = tid / FG_WAVE, g = lane >> 4, r16 = lane & 15;
+  const int n0 = blockIdx.x * 16;
+  const WSrc ws = w_src(w, ldw, n0, N, K, lane);
+  const int kw = ((K + WAVES * 32 - 1) / (WAVES * 32)) * 32;  // k per wave
+  const int k_begin = min(K, wave * kw), k_end = min(K, k_begin + kw);
+  bf16x8 a[U];
+  auto load_w = [&](int kk) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const bool in = kk + 32 * u + 8 * g < k_end;
+      const bf16x8 av = *ws.at(kk + 32 * u, in);
+      a[u] = in ? av : gs_zero8();
+    }
+  };
+  // asked for before n is known (looked at with one chunk), and before W, whose loads it would wait for behind them
+  const bf16x8 own = *(const bf16x8*)(x + min(8 * tid, K - 8));
+  __builtin_amdgcn_sched_barrier(0);
+  load_w(k_begin);
+  const int n = min(*at.n_chunks, MERGE_MAX_CHUNKS), G = at.n_heads / at.n_kv;
+  const size_t step = (size_t)at.n_kv * 16;  // rows from chunk to chunk
+  if (tid < 16) rscale[tid] = 1.f;
+  if (n > 1) {  // uniform
+    auto part_row = [&](int h) { return (size_t)(h / G) * 16 + h % G; };
+    if (tid < at.n_heads) {
+      const float* ml = at.part_ml + part_row(tid) * 2;
+      float m[MERGE_MAX_CHUNKS], l[MERGE_MAX_CHUNKS], M = -INFINITY, L = 0.f;
+#pragma unroll
+      for (int s = 0; s < MERGE_MAX_CHUNKS; ++s) {
+        const float2 v = *(const float2*)(ml + (size_t)min(s, n - 1) * step * 2);
+        m[s] = s < n ? v.x : -INFINITY;
+        l[s] = v.y;
+      }
+#pragma unroll
+      for (int s = 0; s < MERGE_MAX_CHUNKS; ++s) M = fmaxf(M, m[s]);
+#pragma unroll
+      for (int s = 0; s < MERGE_MAX_CHUNKS; ++s) {
+        m[s] = m[s] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m[s] - M);
+        L += m[s] * l[s];
+      }
+      if (at.sinks) L += __builtin_amdgcn_exp2f(at.sinks[tid] * 1.4426950408889634f - M);
+      const float inv = 1.f / L;
+#pragma unroll
+      for (int s = 0; s < MERGE_MAX_CHUNKS; ++s) f_s[tid][s] = m[s] * inv;
+    }
+    bool ready = false;
+    for (int c = tid; c < (K + 7) / 8 || !ready; c += WAVES * 64) {  // (all threads meet the barrier once)
+      const int e = min(8 * c, K - 8), h = e / at.hd;
+      const float* o = at.part_o + part_row(h) * at.hd + e % at.hd;
+      float sum[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) sum[i] = 0.f;
+      for (int s0 = 0; s0 < n; s0 += FLY) {
+        float v[FLY][8];
+#pragma unroll
+        for (int u = 0; u < FLY; ++u) load8<float>(o + (size_t)min(s0 + u, n - 1) * step * at.hd, v[u]);
+        if (!ready) __syncthreads();  // the weights
+        ready = true;
+#pragma unroll
+        for (int u = 0; u < FLY; ++u)
+          if (s0 + u < n) {  // uniform
+            const float f = f_s[h][s0 + u];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) sum[i] = fmaf(f, v[u][i], sum[i]);
+          }
+      }
+      if (8 * c < K) store8<bf16_t>(xs + 8 * c, sum);
+    }
+  } else {
+    if (8 * tid < K) *(bf16x8*)(xs + 8 * tid) = own;
+    for (int c = tid + WAVES * 64; 8 * c < K; c += WAVES * 64) *(bf16x8*)(xs + 8 * c) = *(const bf16x8*)(x + 8 * c);
+  }
+  __syncthreads();
+  f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int kk = k_begin; kk < k_end; kk += 32 * U) {
+    if (kk != k_begin) load_w(kk);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {  // (a chunk behind the range meets zeros of W: any that is there)
+      const int k = kk + 32 * u + 8 * g;
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], *(const bf16x8*)(xs + (k < k_end ? k : k_begin)), acc, 0, 0, 0);
+    }
+  }
+  *(f32x4*)(&red[wave][r16 * 16 + 4 * g]) = acc;
+  __syncthreads();
+  residual_epilogue<WAVES>(red, rscale, rs, pre, n0, 1, N);
+}
+
 template <int MB, int EPI, class TY>
 static void launch_skinny(const void* x, int ldx, const void* w, int ldw, void* y, int ldy, int M, int N,
                           int K, const RowScale& sc, const Residual& rs, hipStream_t stream) {
@@ -572,6 +684,29 @@ extern "C" int fg_gemm_skinny_fused(const void* x, int ldx, const void* w, int l
   else if (epilogue == EPI_GELU_MUL) launch_skinny<1, EPI_GELU_MUL, bf16_t>(x, ldx, w, ldw, y, ldy, M, N, K, sc, rs, stream);
   else if (epilogue == EPI_RESIDUAL) launch_skinny<1, EPI_RESIDUAL, bf16_t>(x, ldx, w, ldw, y, ldy, M, N, K, sc, rs, stream);
   else return FG_ERR_ARG;
+  return fg_launch_status();
+}
+
+// The residual product of the one row that an attention's parts make (see gemm_skinny_attn_kernel): w [N, K] with K =
+// n_heads * hd; x [K]: the row where there is one chunk; n_chunks: an int on the device, at most 16.
+extern "C" int fg_gemm_skinny_attn(const void* x, const float* part_o, const float* part_ml, const int* n_chunks,
+                                   const float* sinks, int n_heads, int n_kv, int hd, const void* w, int ldw, int N,
+                                   float* h, const void* norm_w, int norm_w_dtype, void* x_out, float* ssq_out,
+                                   hipStream_t stream) {
+  if (N <= 0) return FG_OK;
+  if (n_heads <= 0 || n_kv <= 0 || n_heads % n_kv || n_heads / n_kv > 16 || n_heads > MERGE_MAX_HEADS || hd <= 0 || hd % 8 ||
+      (long long)n_heads * hd > MERGE_MAX_K)
+    return FG_ERR_ARG;
+  const int K = n_heads * hd, blocks = (N + 15) / 16;
+  if (ldw % 8 || (ldw && ldw < K) || !x || !part_o || !part_ml || !n_chunks || !h || !norm_w || !x_out || !ssq_out ||
+      ((uintptr_t)x | (uintptr_t)part_o) % 16 || (uintptr_t)part_ml % 8 || (norm_w_dtype != FG_F32 && norm_w_dtype != FG_BF16))
+    return FG_ERR_ARG;
+  const AttnParts at{part_o, part_ml, n_chunks, sinks, n_heads, n_kv, hd};
+  const Residual rs{h, N, norm_w, norm_w_dtype == FG_F32, (bf16_t*)x_out, N, ssq_out};
+  if (blocks >= 1024)
+    gemm_skinny_attn_kernel<4><<<blocks, 256, 0, stream>>>((const bf16_t*)x, at, (const bf16_t*)w, ldw, N, rs);
+  else
+    gemm_skinny_attn_kernel<8><<<blocks, 512, 0, stream>>>((const bf16_t*)x, at, (const bf16_t*)w, ldw, N, rs);
   return fg_launch_status();
 }
 

@@ -669,6 +669,52 @@ def _second_stream(device) -> "torch.cuda.Stream":
     return _second[index]
 
 
+# the row that an output projection may merge itself: chunks and keys at most, heads and values at most
+MERGE_MAX_CHUNKS, MERGE_MAX_KEYS, MERGE_MAX_HEADS, MERGE_MAX_K = 16, 1024, 128, 8192
+
+
+@dataclass
+class AttentionParts:
+    """The attention of one token whose chunks are not merged: ``out [1, H*hd]`` holds it where there is one chunk (the
+    first int of ``n_chunks``, on the device), the partial results else.  :meth:`project` merges them inside the product
+    that reads them."""
+
+    out: torch.Tensor
+    part_o: torch.Tensor
+    part_ml: torch.Tensor
+    n_chunks: torch.Tensor
+    sinks: Optional[torch.Tensor]
+    n_heads: int
+    n_kv: int
+
+    def project(self, w, h: torch.Tensor, norm_weight: torch.Tensor, eps: float) -> "ScaledRows":
+        """What :func:`gemm_skinny_residual` does with the merged row."""
+        K, N = self.out.shape[1], w.shape[0]
+        _gpu(self.out, h, norm_weight)
+        w_ptr, ldw = _weight_args(w, K, "attention's output projection")
+        _need(h.dtype == torch.float32 and h.shape == (1, N) and h.is_contiguous(), "h must be float32 [1, N]")
+        _need(norm_weight.shape == (N,) and norm_weight.is_contiguous()
+              and norm_weight.dtype in (torch.float32, torch.bfloat16), "norm_weight must be [N], float32 or bfloat16")
+        x_out = torch.empty((1, N), dtype=torch.bfloat16, device=h.device)
+        ssq_out = torch.empty((1, -(-N // 16)), dtype=torch.float32, device=h.device)
+        st = _lib.load("gemm_skinny").fg_gemm_skinny_attn(
+            _ptr(self.out), _ptr(self.part_o), _ptr(self.part_ml), _ptr(self.n_chunks), _ptr(self.sinks), self.n_heads, self.n_kv,
+            K // self.n_heads, w_ptr, ldw, N, _ptr(h), _ptr(norm_weight), _code(norm_weight), _ptr(x_out), _ptr(ssq_out),
+            _stream(h))
+        _check(st, "attention's output projection")
+        return ScaledRows(x_out, ssq_out, N, float(eps))
+
+
+def attention_parts_fit(n_tokens: int, n_heads: int, head_dim: int, n_kv: int, max_keys: int) -> bool:
+    """Whether a step's attention may be left as :class:`AttentionParts`: one token with at most ``max_keys`` keys, whose
+    parts every workgroup of the projection then reads (5 chunks of 12 KB for 24 heads at 1,024 keys).  One request through
+    28 layers of 24 heads with the merge inside the product and as a kernel of its own, us a step: 100 keys 1685 and 1726,
+    300 keys 1755 and 1788, 950 keys 1762 and 1793."""
+    return (n_tokens == 1 and max_keys <= MERGE_MAX_KEYS and -(-(max_keys // 64 + 1) // _SPLIT_MIN_TILES) <= MERGE_MAX_CHUNKS
+            and n_heads <= MERGE_MAX_HEADS and n_heads * head_dim <= MERGE_MAX_K and n_heads // n_kv <= 16
+            and head_dim % 16 == 0 and head_dim <= MFMA_MAX_HEAD_DIM)
+
+
 def paged_attention_mfma(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor,
                          block_table: torch.Tensor, small_items: Optional[torch.Tensor],
                          big_items: Optional[torch.Tensor], n_heads: int, scale: float, window: int = 0,
@@ -676,7 +722,7 @@ def paged_attention_mfma(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tens
                          min_tiles: int = 4, max_rows: int = 16, tile_rows: Optional[int] = None,
                          exact_weights: bool = False, sinks: Optional[torch.Tensor] = None,
                          distance: Optional[torch.Tensor] = None, gate: Optional[torch.Tensor] = None,
-                         gate_sigmoid: bool = True) -> torch.Tensor:
+                         gate_sigmoid: bool = True, leave_parts: bool = False) -> torch.Tensor:
     """bf16 attention on the matrix cores.  ``small_items`` / ``big_items`` are
     device int32 ``[n, 4]`` lists from :func:`attention_items` (16-byte aligned);
     every query token of the step must be covered by exactly one item.
@@ -690,7 +736,9 @@ def paged_attention_mfma(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tens
     the product with the values as two bfloat16 terms (16 significant bits).  ``sinks`` and ``distance``: as
     :func:`paged_attention_general` (a build of the kernels with exact weights takes the distance bias).  ``gate`` and
     ``gate_sigmoid``: what :func:`gate_mul` does with them behind the attention, done where the output is stored (the
-    same bits), for bfloat16 rows that can be read in fours; else by that kernel."""
+    same bits), for bfloat16 rows that can be read in fours; else by that kernel.  ``leave_parts``: one token without a
+    gate comes as :class:`AttentionParts` (the caller has asked :func:`attention_parts_fit`)."""
+    leave_parts = leave_parts and gate is None and q.shape[0] == 1 and (big_items is None or not big_items.numel())
     _gpu(q, out, k_pages, v_pages, block_table, small_items, big_items, plan, sinks, distance, gate)
     if gate is not None and (gate.dtype != torch.bfloat16 or gate.data_ptr() % 8 or gate.stride(0) % 4):
         return gate_mul(paged_attention_mfma(q, out, k_pages, v_pages, block_table, small_items, big_items, n_heads, scale,
@@ -743,8 +791,11 @@ def paged_attention_mfma(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tens
         st = lib.fg_attn_split_sink(
             _ptr(q), q.stride(0), _ptr(out), out.stride(0), _ptr(k_pages), _ptr(v_pages), _ptr(block_table),
             block_table.stride(0), _ptr(plan), n, max_chunks, max_rows, _ptr(part_o), _ptr(part_ml), n_heads, n_kv, hd,
-            page_size, ctypes.c_float(scale), int(window or 0), _ptr(sinks), _ptr(distance), *gate_args, _plan_ordered(n), _stream(q))
+            page_size, ctypes.c_float(scale), int(window or 0), _ptr(sinks), _ptr(distance), *gate_args, _plan_ordered(n),
+            int(not leave_parts), _stream(q))
         _check(st, "attn_split")
+        if leave_parts:
+            return AttentionParts(out, part_o, part_ml, plan[10:], sinks, n_heads, n_kv)
     if big_items is not None and big_items.numel():
         tile_rows = attention_tile_rows(hd, False, exact_weights, dist) if tile_rows is None else int(tile_rows)
         _need(tile_rows in (attention_tile_rows(hd, False, exact_weights, dist), attention_tile_rows(hd, True, exact_weights, dist)),
@@ -767,10 +818,11 @@ def paged_attention(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v
                     group, ctx, n_heads: int, scale: float, window: int = 0,
                     exact_weights: bool = False, sinks: Optional[torch.Tensor] = None,
                     distance: Optional[torch.Tensor] = None, gate: Optional[torch.Tensor] = None,
-                    gate_sigmoid: bool = True) -> torch.Tensor:
+                    gate_sigmoid: bool = True, leave_parts: bool = False) -> torch.Tensor:
     """Attention for one step: picks the kernel for the step's dtype and shape.
     ``exact_weights``: see :func:`paged_attention_mfma` (the general kernel's weights are fp32 anyway).
-    ``gate``, ``gate_sigmoid``: an output gate as :func:`gate_mul` takes it.
+    ``gate``, ``gate_sigmoid``: an output gate as :func:`gate_mul` takes it.  ``leave_parts``: the result may be
+    :class:`AttentionParts` where the step has one token with few keys.
 
     ``group`` carries the block table of the layer's cache group, ``ctx`` the
     step's per-token vectors (``fastgen_amd.engine.context``).  bfloat16 with a
@@ -820,7 +872,8 @@ def paged_attention(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v
     return paged_attention_mfma(q, out, k_pages, v_pages, group.block_table, small_d, big_d, n_heads, scale,
                                 window, split_plan, chunks, max_rows=min(16, rows), tile_rows=tile_rows,
                                 exact_weights=exact_weights, sinks=sinks, distance=distance, gate=gate,
-                                gate_sigmoid=gate_sigmoid)
+                                gate_sigmoid=gate_sigmoid, leave_parts=leave_parts and attention_parts_fit(
+                                    q.shape[0], n_heads, hd, n_kv, group.block_table.shape[1] * k_pages.shape[2]))
 
 
 # ----------------------------------------------------------------------- gemm

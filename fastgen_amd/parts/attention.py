@@ -227,9 +227,13 @@ class Attention(RowsMixer):
             gate = qkv[:, gate_col:] if self.output_gate else None
             gate_done = False
         out = torch.empty((rows.shape[0], q_width), dtype=rows.dtype, device=rows.device)
-        ops.paged_attention(qkv, out, store.k_pages, store.v_pages, group, ctx, self.n_heads, self.scale,
-                            self.window or 0, exact_weights=self.exact_weights, sinks=self.sinks, distance=self.distance,
-                            gate=gate, gate_sigmoid=not gate_done)
+        # one token whose output projection folds the norm behind it: that product may merge the attention's chunks itself
+        leave = then is not None and out.dtype == torch.bfloat16 and skinny_ok(out, self.wo)
+        done = ops.paged_attention(qkv, out, store.k_pages, store.v_pages, group, ctx, self.n_heads, self.scale,
+                                   self.window or 0, exact_weights=self.exact_weights, sinks=self.sinks, distance=self.distance,
+                                   gate=gate, gate_sigmoid=not gate_done, leave_parts=leave)
+        if isinstance(done, ops.AttentionParts):
+            return done.project(self.wo.streaming, *then)
         return linear(out, self.wo, partials_ok=True, residual=then)
 
     def _rope_table(self, ctx: Any):

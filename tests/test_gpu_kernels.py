@@ -1158,3 +1158,31 @@ def test_attention_plan_cuts_every_item_into_equal_chunks(ops, n_items, window, 
     if even < want and int((-(-tiles // even)).sum()) <= max_chunks:
         want = even
     assert ts == want
+
+
+@pytest.mark.parametrize("H,KV,hd", [(24, 8, 128), (32, 8, 128), (4, 4, 16), (6, 2, 80), (128, 8, 64), (16, 1, 256)])
+@pytest.mark.parametrize("n_keys", [1, 256, 257, 600, 1024])
+@pytest.mark.parametrize("sink", [False, True])
+def test_output_projection_merges_the_chunks_of_one_token(ops, H, KV, hd, n_keys, sink):
+    """One chunk to five, against the merge and the product as kernels of their own: the row differs at most by its last
+    rounding to bfloat16 (the weights are summed in another order), so the stream by less than that of its products."""
+    torch.manual_seed(H + n_keys)
+    case = _paged_case(torch.bfloat16, [(n_keys - 1, 1)], H, KV, hd, 16, seed=n_keys)
+    N = 48
+    w = (torch.randn(N, H * hd) * 0.1).bfloat16().to(DEV)
+    sinks = torch.randn(H).to(DEV) if sink else None
+    norm_w, h0 = torch.randn(N).to(DEV), torch.randn(1, N).to(DEV)
+    items = torch.tensor([0, 0, 1, n_keys - 1], dtype=torch.int32, device=DEV)
+    assert ops.attention_parts_fit(1, H, hd, KV, 1024)
+    args = (case["kp"], case["vp"], case["table"], items, None, H, hd ** -0.5)
+    run = lambda **kw: ops.paged_attention_mfma(case["q"], torch.empty_like(case["q"][:, : H * hd]), *args, max_rows=H // KV,
+                                                sinks=sinks, **kw)
+    row, parts = run(), run(leave_parts=True)
+    assert isinstance(parts, ops.AttentionParts) and int(parts.n_chunks[0]) == -(-(-(-n_keys // 64)) // 4)
+    for weight in (w, ops.pack_weight(w)):
+        h, want_h = h0.clone(), h0.clone()
+        got, want = parts.project(weight, h, norm_w, 1e-5), ops.gemm_skinny_residual(row, weight, want_h, norm_w, 1e-5)
+        bound = 2.0 ** -8 * (row.double().abs() @ w.double().abs().T) + 1e-6 * want_h.abs()
+        assert ((h - want_h).abs() <= bound).all()
+        if n_keys <= 256:
+            assert torch.equal(h, want_h) and torch.equal(got.rows, want.rows) and torch.equal(got.ssq, want.ssq)
