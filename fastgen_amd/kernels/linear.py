@@ -7,10 +7,10 @@ kernels can take a product (the engine's weight-streaming MFMA kernels of
 the vendor library's product through ``torch``, which the reference uses for
 all of them: cuBLAS through ``F.linear``, ``fastgen/forward.py:433-513``).
 Which one is the fastest depends on the matrix and on the number of rows, so
-it is measured: the first time a product of some shape ``(N, K)`` meets some
+it is measured: the first few times a product of some shape ``(N, K)`` meets some
 number of rows, the kernels that can take it are timed on the operands at hand
 (the caches emptied before each run) and the winner is kept in one table (``choices``) for every later product of
-that shape and row bucket.  No size of any model stands here or in the parts.
+that shape and row bucket; times that are close are a tie, which a fixed order decides.  No size of any model stands here or in the parts.
 
 A part hands ``linear`` its matrix as a :class:`StreamedMatrix` (made by :func:`streamed` when the part
 loads): the matrix row by row and, where a model's weights fit the GPU twice over, a second copy in the order
@@ -161,12 +161,20 @@ def k_splits_for(n_out: int, k: int, rows: int = 0) -> int:
 # ------------------------------------------------------------------ the table
 # (what is asked for, N, K, row bucket) -> name of the kernel that measured fastest
 choices: Dict[Tuple[str, int, int, int], str] = {}
-# the same keys -> what each candidate took when it was measured (milliseconds, the consumer's cost included)
+# the same keys -> what each candidate took when it was measured (milliseconds on average, the consumer's cost included)
 timings: Dict[Tuple[str, int, int, int], Dict[str, float]] = {}
+_samples: Dict[Tuple[str, int, int, int], List[Dict[str, float]]] = {}  # of the keys met so far, at most _SAMPLES each
 # set to a candidate's name to take that kernel wherever it is among the candidates (tests run the
 # engine once under each name, so that every kernel that may be chosen is compared with the plain run)
 force: Optional[str] = None
-_TIMED_RUNS = 4
+_TIMED_RUNS = 2  # of every candidate, each of the _SAMPLES times
+# How long a product takes depends on where its matrix happens to lie (64 rows of 28,672 x 4,096: the library's takes 49 to
+# 51 us on one layer's matrix and 59 to 63 on the next ones, in every process; the wide kernel 52 to 57 on all of them), so
+# the candidates are measured at the first calls that ask for a product, in a model one layer's matrix after the other.
+_SAMPLES = 3
+# A lead smaller than this decides nothing: the same program would take one kernel today and another tomorrow, and their
+# results differ by a rounding.
+_TIE = 0.04
 # Before each timed run this many bytes are read, so that a candidate finds the weights where a model's step
 # finds them: in memory, not in the caches (a memory-side cache of 256 MB and the L2s; a decode step streams
 # gigabytes of other weights between two uses of a matrix).  Timed warm, the wide kernel looks faster than the
@@ -197,14 +205,21 @@ def _capturing() -> bool:
     return torch.cuda.is_current_stream_capturing()
 
 
+def _winner(best: Dict[str, float], order: List[str]) -> str:
+    """Of the candidates whose time is within ``_TIE`` of the shortest the first in ``order``."""
+    limit = (1 + _TIE) * min(best.values())
+    return next(name for name in order if best[name] <= limit)
+
+
 def _choose(what: str, n: int, k: int, rows: int, candidates: List[Tuple[str, Callable[[], torch.Tensor]]],
-            handicap: Optional[Dict[str, float]] = None) -> str:
-    """The candidate to run: the forced one, the one the table holds, or the one that is fastest now.
+            handicap: Optional[Dict[str, float]] = None, order: Optional[List[str]] = None) -> str:
+    """The candidate to run: the forced one, the one the table holds, or, at the first calls, the fastest so far.
     Timing needs the device to itself (events and a wait for them), so a product that is first met while
     a step is being recorded runs the first candidate, unrecorded in the table; the engine runs every
     step once, unrecorded, before it records it.  The candidates are timed in turn on the same
     operands, each run behind a sweep of memory that empties the caches.  ``handicap``: milliseconds added to a candidate's time
-    for what its result costs the consumer (partial sums that are still to be added)."""
+    for what its result costs the consumer (partial sums that are still to be added).  ``order``: who takes a tie
+    (default: the candidates' own order)."""
     names = [c[0] for c in candidates]
     if force in names:
         return force
@@ -212,13 +227,28 @@ def _choose(what: str, n: int, k: int, rows: int, candidates: List[Tuple[str, Ca
         return names[0]
     key = (what, n, k, row_bucket(rows))
     got = choices.get(key)
-    if got in names:
+    seen = _samples.get(key, [])
+    settled = not seen or len(seen) >= _SAMPLES  # (a choice without samples was put there from outside)
+    if got in names and (settled or _capturing()):
         return got
     if _capturing():
         return names[0]
+    if got not in names:
+        seen = []
+    seen = seen + [_measure(candidates, handicap or {}, first=not seen)]
+    timings[key] = {name: sum(t[name] for t in seen) / len(seen) for name in names}
+    choices[key] = _winner(timings[key], order or names)
+    _samples[key] = seen
+    return choices[key]
+
+
+def _measure(candidates: List[Tuple[str, Callable[[], torch.Tensor]]], handicap: Dict[str, float],
+             first: bool) -> Dict[str, float]:
+    """What each candidate takes on the operands at hand, in milliseconds."""
     best: Dict[str, float] = {}
-    for fn in (c[1] for c in candidates):  # once each, unmeasured: libraries load, the library picks its kernel
-        fn()
+    if first:  # once each, unmeasured: libraries load, the library picks its kernel
+        for _, fn in candidates:
+            fn()
     try:
         flush = torch.zeros(_FLUSH_BYTES // 4, dtype=torch.int32, device=torch.cuda.current_device())
         torch.cuda.current_stream().synchronize()  # (its zeros are in memory before anything is timed)
@@ -235,12 +265,9 @@ def _choose(what: str, n: int, k: int, rows: int, candidates: List[Tuple[str, Ca
             ev[r][1].record()
     torch.cuda.current_stream().synchronize()
     del flush
-    for ev, name in zip(events, names):
-        best[name] = min(a.elapsed_time(b) for a, b in ev) + (handicap or {}).get(name, 0.0)
-    winner = min(names, key=lambda nm: best[nm])
-    choices[key] = winner
-    timings[key] = best
-    return winner
+    for ev, (name, _) in zip(events, candidates):
+        best[name] = min(a.elapsed_time(b) for a, b in ev) + handicap.get(name, 0.0)
+    return best
 
 
 def linear(x, w, out_dtype: Optional[torch.dtype] = None,
@@ -338,5 +365,10 @@ def linear(x, w, out_dtype: Optional[torch.dtype] = None,
     what = (epilogue if silu else "store") + ("+partials" if partials_ok and rows > SKINNY_ROWS else "") + (
         "+f32" if out_dtype == torch.float32 else "") + ("+scaled" if scaled is not None else "") + (
         "+packed" if sw is not w else "")
-    name = _choose(what, N, K, rows, candidates, handicap)
+    # Ties: the kernel with the epilogue in it, and with few rows the narrow one, both the least launches; a plain
+    # product of more rows goes to the library, whose result is whole (no partial sums to add).
+    order = [c[0] for c in candidates]
+    if not silu and rows > SKINNY_ROWS:
+        order.sort(key=lambda name: name != "library")
+    name = _choose(what, N, K, rows, candidates, handicap, order)
     return dict(candidates)[name]()
