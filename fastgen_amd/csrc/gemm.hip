@@ -24,6 +24,8 @@
 //
 // Operands of bf16 with fp32 accumulation take the FMA kernel below, so that
 // any shape has a product when the tuned kernels refuse it.
+#include <type_traits>
+
 #include "common.h"
 
 #define GT_M 64
@@ -333,7 +335,9 @@ __global__ __launch_bounds__(512) void gemm_f32_few_kernel(const float* __restri
 // N x K 16384 x 3072 / 5120 x 3072 / 3072 x 8192, us: 400 rows 240 / 100 / 148 (433 / 153 / 240 with the fp32
 // instructions), 2048 rows 1163 / 418 / 667 (1891 / 605 / 981): 1.06 PFLOP/s of bf16 at the largest, against 1.4 that
 // a product of bf16 operands reaches.
-template <int MB, int NB, int NW, int AHEAD, bool VEC>
+// FAR: rows so far apart that a tile spans 4 GB, with offsets of 64 bits (of 32, a load is one register of offset behind
+// a uniform base).
+template <int MB, int NB, int NW, int AHEAD, bool VEC, bool FAR>
 __global__ __launch_bounds__(64 * NW, 2) void gemm_f32_tiled_kernel(
     const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ y, float* __restrict__ part, int M,
     int N, int K, int ldx, int ldw, int ldy, int row_tiles, int col_tiles, int units, int wide) {
@@ -351,12 +355,13 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_f32_tiled_kernel(
   const int k_full = k_begin + (k_end - k_begin) / GF_SEG * GF_SEG;  // whole segments
   // a lane's place behind the wave's (the tile's) first row; rows behind the last repeat it: their outputs are not stored
   const float *wb = w + (size_t)min(n0, N - 1) * ldw, *xb = x + (size_t)m0 * ldx;
-  unsigned wo[NB], xo[XV];  // in bytes
+  using Offset = std::conditional_t<FAR, size_t, unsigned>;
+  Offset wo[NB], xo[XV];  // in bytes
 #pragma unroll
-  for (int j = 0; j < NB; ++j) wo[j] = 4 * (min(16 * j + r, max(N - 1 - n0, 0)) * ldw + 4 * g);
+  for (int j = 0; j < NB; ++j) wo[j] = 4 * ((Offset)min(16 * j + r, max(N - 1 - n0, 0)) * ldw + 4 * g);
   const int piece = tid % 8, row = tid / 8;  // of x: four k of a row, the rows 8 NW apart
 #pragma unroll
-  for (int i = 0; i < XV; ++i) xo[i] = 4 * (min(row + 8 * NW * i, M - 1 - m0) * ldx + 4 * piece);
+  for (int i = 0; i < XV; ++i) xo[i] = 4 * ((Offset)min(row + 8 * NW * i, M - 1 - m0) * ldx + 4 * piece);
 
   f32x4 raw[AHEAD][NB][2], xv[AHEAD][XV], whole[MB][NB], small[MB][NB];
   GfParts wp[NB];
@@ -500,7 +505,7 @@ struct GfCall {
   hipStream_t stream;
 };
 
-template <int MB, int NB, int NW>
+template <int MB, int NB, int NW, bool FAR = false>
 static int gf_launch(const GfCall& c) {
   constexpr int AHEAD = MB <= 3 ? 4 : 2;
   const int groups = (c.K + GF_GROUP - 1) / GF_GROUP;
@@ -510,7 +515,7 @@ static int gf_launch(const GfCall& c) {
   const long long blocks = (units + 7) / 8 * 8 * row_tiles;
   if (blocks > 2147483647LL || (c.part && c.M > 65535)) return FG_ERR_ARG;
 #define TILED(VEC)                                                                                            \
-  gemm_f32_tiled_kernel<MB, NB, NW, AHEAD, VEC><<<(unsigned)blocks, 64 * NW, 0, c.stream>>>(                  \
+  gemm_f32_tiled_kernel<MB, NB, NW, AHEAD, VEC, FAR><<<(unsigned)blocks, 64 * NW, 0, c.stream>>>(                  \
       c.x, c.w, c.y, c.part, c.M, c.N, c.K, c.ldx, c.ldw, c.ldy, row_tiles, col_tiles, (int)units, wide)
   if (c.vec) TILED(true);
   else TILED(false);
@@ -545,7 +550,11 @@ extern "C" int fg_gemm_f32(const float* x, const float* w, float* y, float* part
     return fg_launch_status();
   }
   const GfCall c = {x, w, y, part, M, N, K, ldx, ldw, ldy, vec, stream};
-  if (nw == 4 && mb > 5) return FG_ERR_ARG;
+  if (mb < 1 || mb > 7 || (nw == 4 && mb > 5) || (nw != 4 && nw != 8)) return FG_ERR_ARG;
+  // What a tile's rows span, of x and of a wave's 32 of W: any strides are taken, beyond 32 bits of bytes by the smallest
+  // tile (every cut gives the same bits).
+  const long long span = max((long long)(min(16 * mb, M) - 1) * ldx, (long long)(min(32, N) - 1) * ldw);
+  if (4 * (span + 32) > 0xffffffffLL) return gf_launch<1, 2, 8, true>(c);
 #define CASE(MB)                                          \
   if (mb == MB && nw == 8) return gf_launch<MB, 2, 8>(c); \
   if (mb == MB && nw == 4) return gf_launch<MB < 6 ? MB : 5, 2, 4>(c);

@@ -442,6 +442,23 @@ def test_gemm_f32_every_cut_gives_the_same_bits(ops, N, K):
         assert torch.equal(ops.gemm_nt(x[first:last], w), full[first:last]), (first, last)
 
 
+@pytest.mark.parametrize("M,N,K,ldx,ldw", [
+    (113, 40, 136, 4_800_001, 136),  # a tile's rows of x span more than 2^31 bytes, unaligned
+    (113, 300, 136, 9_800_000, 136),  # more than 2^32
+    (70, 33, 1100, 1100, 34_700_000),  # a wave's rows of W
+    (20, 33, 41, 16_000_001, 34_700_001)])  # both, the scalar loads
+def test_gemm_f32_rows_far_apart(ops, M, N, K, ldx, ldw):
+    """Rows of any stride: what the same rows side by side give, the same bits."""
+    torch.manual_seed(M + K)
+    x, w = torch.randn(M, K).to(DEV), torch.randn(N, K).to(DEV)
+    far = []
+    for t, ld in ((x, ldx), (w, ldw)):
+        rows = torch.empty((t.shape[0] - 1) * ld + K, device=DEV).as_strided(t.shape, (ld, 1))
+        rows.copy_(t)
+        far.append(rows)
+    assert torch.equal(ops.gemm_nt(*far), ops.gemm_nt(x, w))
+
+
 @pytest.mark.parametrize("N,K", [(130, 1100), (3072, 1028)])
 def test_gemm_f32_bits_around_the_line_of_the_narrow_tiles(ops, N, K):
     """Up to 640 rows a last tile of at most 32 rows makes all tiles that narrow, beyond it does not: the same bits."""
