@@ -4,23 +4,33 @@
 //
 // float32 (the true 32-bit path) runs on v_mfma_f32_16x16x32_bf16, sixteen
 // times the rate of v_mfma_f32_16x16x4_f32: every operand is the exact sum of
-// three bf16 parts of 8 bits each (h = bf16(v), m = bf16(v - h), l = v - h -
-// m), a product of two is six instructions, and the parts' products left out
-// (m l, l m, l l) are below 2^-26 of the whole.  What rounding costs is the
-// sums', and the matrix core cuts off where it adds to its accumulator, so
-// the order is: h h over 128 k (4 instructions from zero) in one chain, the
-// five smaller products of the same k (20 instructions) in another, their sum
-// a segment's; 8 segments are a group's sum, the groups' sums the total, each
-// ascending in fp32.  An output's order is fixed by K alone, whichever kernel
-// takes the product, so a row's result does not depend on how many other rows
-// the call holds.  Error relative to the product in 64 bits, random operands
-// of K = 128 / 1024 / 3072 / 8192 / 14336: 0.7 / 0.9 / 0.9 / 1.0 / 1.1e-7
-// (the fp32 instructions with chains of 32 k: 1.1 / 1.2 / 1.3 / 1.4 / 1.4e-7);
-// with magnitudes spread over e^+-2 1.0 / 1.0 / 1.1 / 1.2 / 1.3e-7 (1.0 / 1.2 /
-// 1.2 / 1.4 / 1.5).  A part of an operand below 2^-109 may be too small for
-// bf16: such an operand counts with fewer bits.  Infinities (and what rounds to
-// one in bf16) have no such parts: an output that comes out as NaN is
-// computed again, one fp32 FMA a product (gf_again).
+// three bf16 parts of 8 bits each (h = bf16(v), m = bf16(v - h), l = v - h - m;
+// m and l scaled up, so that small operands keep all bits too), and a product of
+// two is six instructions: h h, then h m + m h, then h l + l h + m m.  m is up to
+// 2^-8 of an operand's leading bit and l up to 2^-17, so the products left out
+// (m l, l m; l l) are at most 2^-24 of the whole, half a unit of its last place,
+// and of either sign.  Each of the three kinds is summed over the 32 k of an
+// instruction from zero and added to the segment's sum by the vector units,
+// rounded to nearest (the matrix core cuts off where it adds to its
+// accumulator): 4 steps are a segment's sum, 8 segments a group's, the groups'
+// sums the total, each ascending.  An output's order is fixed by K alone,
+// whichever kernel takes the product, so a row's result does not depend on how
+// many other rows the call holds.
+//
+// Error relative to the product in 64 bits (2-norms, units of 1e-7), in brackets
+// that of the fp32 instructions with chains of 32 k; K = 128 / 1024 / 3072 / 14336:
+//   random signs           0.57 / 0.79 / 0.87 / 1.08  (1.10 / 1.24 / 1.29 / 1.43)
+//   magnitudes of those    0.43 / 0.52 / 0.43 / 0.62  (0.58 / 0.54 / 0.43 / 0.63)
+//   uniform in [0, 1)      0.43 / 0.49 / 0.43 / 0.57  (0.57 / 0.50 / 0.44 / 0.57)
+//   constant rows          0.25 / 0.64 / 0.47 / 1.07  (2.28 / 2.52 / 2.40 / 2.85)
+//   e^N(0,2), one sign     0.91 / 1.67 / 0.92 / 0.90  (0.70 / 1.52 / 0.69 / 0.70)
+//   the same, both signs   0.58 / 0.78 / 0.84 / 1.24  (0.68 / 0.85 / 1.11 / 1.21)
+// The fifth line is where it is not the better one: inside an instruction eight
+// products are cut off below the largest of them.  Magnitudes down to the
+// smallest normal number change nothing; of an operand below it up to 3/4 of its
+// last place is left out.  Infinities (and what rounds to one in
+// bf16) have no such parts: an output that comes out as NaN is computed again,
+// one fp32 FMA a product (gf_again).
 //
 // Operands of bf16 with fp32 accumulation take the FMA kernel below, so that
 // any shape has a product when the tuned kernels refuse it.
@@ -131,6 +141,8 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 #define GF_SEG 128    // k of a segment: 4 steps
 #define GF_GROUP 1024 // k of a group: 8 segments
 #define GF_STEP 32    // k of a matrix instruction
+#define GF_STEP_UP 256.f         // a part's scale against the part before it
+#define GF_STEP_DOWN 0.00390625f
 
 // Four elements of a row from k on, zeros behind K.  VEC: rows are 16-byte aligned and K is a multiple of 4.
 template <bool VEC>
@@ -151,8 +163,10 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
-// The three parts of four numbers: v = part 0 + part 1 + part 2, the first rounded to nearest (so that the next has
-// either sign and what is left out no bias), the second cut off, the third the eight bits that are left.
+// The three parts of four numbers: v = part 0 + 2^-8 part 1 + 2^-16 part 2, exactly, whatever v is (down to the smallest
+// number: the parts that are of 2^-9 and 2^-17 of it are kept 2^8 and 2^16 times as large, so that 8 bits with the
+// smallest exponent of bf16 hold all of them).  The first two are rounded to nearest, so that what follows has either
+// sign; the third is what is left, at most 7 bits.
 __device__ __forceinline__ void gf_parts4(const f32x4 v, bf16x4* p0, bf16x4* p1, bf16x4* p2) {
   const unsigned top = 0xffff0000u;
   unsigned p[3][2];
@@ -160,10 +174,11 @@ __device__ __forceinline__ void gf_parts4(const f32x4 v, bf16x4* p0, bf16x4* p1,
   for (int e = 0; e < 2; ++e) {
     const f32x2 pair = {v[2 * e], v[2 * e + 1]};
     const unsigned h = __builtin_bit_cast(unsigned, __builtin_convertvector(pair, bf16x2));
-    const float r0 = pair[0] - __uint_as_float(h << 16), r1 = pair[1] - __uint_as_float(h & top);
-    const float l0 = r0 - __uint_as_float(__float_as_uint(r0) & top), l1 = r1 - __uint_as_float(__float_as_uint(r1) & top);
-    p[0][e] = h;  // (a permutation of bytes takes the upper halves of two words)
-    p[1][e] = __builtin_amdgcn_perm(__float_as_uint(r1), __float_as_uint(r0), 0x07060302u);
+    const float r0 = GF_STEP_UP * (pair[0] - __uint_as_float(h << 16)), r1 = GF_STEP_UP * (pair[1] - __uint_as_float(h & top));
+    const unsigned m = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{r0, r1}), bf16x2));
+    const float l0 = GF_STEP_UP * (r0 - __uint_as_float(m << 16)), l1 = GF_STEP_UP * (r1 - __uint_as_float(m & top));
+    p[0][e] = h;
+    p[1][e] = m;  // (a permutation of bytes takes the upper halves of two words)
     p[2][e] = __builtin_amdgcn_perm(__float_as_uint(l1), __float_as_uint(l0), 0x07060302u);
   }
   *p0 = __builtin_bit_cast(bf16x4, p[0]);
@@ -196,15 +211,30 @@ __device__ __forceinline__ f32x4 gf_whole4(const float* p) {
 
 #define GF_MFMA(A, B, C) __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, B, C, 0, 0, 0)
 
-// One step of one tile.  A: 16 rows of W, B: 16 rows of x; lane 16 g + r ends with outputs 4 g .. 4 g + 3 of x row r.
-__device__ __forceinline__ void gf_step(const GfParts& w, const bf16x8 x0, const bf16x8 x1, const bf16x8 x2,
-                                        f32x4& whole, f32x4& small) {
-  small = GF_MFMA(w.p[2], x0, small);
-  whole = GF_MFMA(w.p[0], x0, whole);
-  small = GF_MFMA(w.p[0], x2, small);
-  small = GF_MFMA(w.p[1], x1, small);
-  small = GF_MFMA(w.p[1], x0, small);
-  small = GF_MFMA(w.p[0], x1, small);
+// One step of one tile: the products of the parts by size, each kind from zero.  A: 16 rows of W, B: 16 rows of x; lane
+// 16 g + r ends with outputs 4 g .. 4 g + 3 of x row r.
+struct GfTerms {
+  f32x4 whole, middle, small;
+};
+
+__device__ __forceinline__ GfTerms gf_step(const GfParts& w, const bf16x8 x0, const bf16x8 x1, const bf16x8 x2) {
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  GfTerms t;
+  t.small = GF_MFMA(w.p[2], x0, zero);
+  t.whole = GF_MFMA(w.p[0], x0, zero);
+  t.middle = GF_MFMA(w.p[1], x0, zero);
+  t.small = GF_MFMA(w.p[0], x2, t.small);
+  t.middle = GF_MFMA(w.p[0], x1, t.middle);
+  t.small = GF_MFMA(w.p[1], x1, t.small);
+  return t;
+}
+
+// A step's products into its segment's sum, rounded to nearest (the matrix core cuts off where it adds).
+__device__ __forceinline__ void gf_fold(f32x4& sum, const GfTerms& t) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    sum[i] += fmaf(fmaf(t.small[i], GF_STEP_DOWN, t.middle[i]), GF_STEP_DOWN, t.whole[i]);
+  asm volatile("" : "+v"(sum));  // here, or the compiler keeps every step's terms up to the segment's end, in scratch memory
 }
 
 // An output whose sum came out as NaN: the operands may hold an infinity.
@@ -239,8 +269,8 @@ __device__ __forceinline__ void gf_store4(float* __restrict__ y, int n, int N, b
 // Up to 16 rows (decode): bound by reading W once.  A workgroup owns 16 outputs; a round is one group, a wave takes
 // one of its segments, so 64 KB of W (every wave's next segment) are in flight a workgroup while the current ones
 // are multiplied; the segments' sums meet in LDS and are added in order by one thread an output.  N x K 3072 x 3072 /
-// 16384 x 3072 / 3072 x 8192: 13 / 44 / 32 us at 4 rows (4.6 TB/s of W at the largest), 18 / 60 / 41 at 16; with the fp32
-// instructions 14 / 48 / 32 and 18 / 60 / 41.
+// 16384 x 3072 / 3072 x 8192: 14 / 46 / 33 us at 4 rows (4.4 TB/s of W at the largest), 18 / 56 / 41 at 16; with the fp32
+// instructions 14 / 48 / 33 and 17 / 60 / 41.
 // A wave cuts its segment of x into parts once: with FEW (up to 8 rows), each number in one lane, through LDS into
 // the operands' order; above, every lane the operand it needs.
 template <bool FEW, bool VEC>
@@ -290,7 +320,7 @@ __global__ __launch_bounds__(512) void gemm_f32_few_kernel(const float* __restri
         }
         __builtin_amdgcn_wave_barrier();  // (a wave reads only what it has written itself)
       }
-      f32x4 whole = {0.f, 0.f, 0.f, 0.f}, small = {0.f, 0.f, 0.f, 0.f};
+      f32x4 sum = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         GfParts xp;
@@ -300,9 +330,9 @@ __global__ __launch_bounds__(512) void gemm_f32_few_kernel(const float* __restri
         } else {
           xp = gf_parts(xv[2 * i], xv[2 * i + 1]);
         }
-        gf_step(gf_parts(wv[2 * i], wv[2 * i + 1]), xp.p[0], xp.p[1], xp.p[2], whole, small);
+        gf_fold(sum, gf_step(gf_parts(wv[2 * i], wv[2 * i + 1]), xp.p[0], xp.p[1], xp.p[2]));
       }
-      sums[buf][wave][lane] = whole + small;
+      sums[buf][wave][lane] = sum;
     }
     __syncthreads();  // (a round's sums are read before the round after next writes them: one barrier between)
     if (tid < 256) {
@@ -332,9 +362,9 @@ __global__ __launch_bounds__(512) void gemm_f32_few_kernel(const float* __restri
 // With `part` a workgroup takes one group of k and stores its sum there ([groups][M][N]); else it adds each group's to
 // y.  The workgroups that read the same rows of W are neighbours on one die.
 //
-// N x K 16384 x 3072 / 5120 x 3072 / 3072 x 8192, us: 400 rows 240 / 100 / 148 (433 / 153 / 240 with the fp32
-// instructions), 2048 rows 1163 / 418 / 667 (1891 / 605 / 981): 1.06 PFLOP/s of bf16 at the largest, against 1.4 that
-// a product of bf16 operands reaches.
+// N x K 16384 x 3072 / 5120 x 3072 / 3072 x 8192, us: 400 rows 290 / 105 / 159 (459 / 167 / 256 with the fp32
+// instructions), 2048 rows 1326 / 468 / 748 (1900 / 622 / 982): 0.93 PFLOP/s of bf16 at the largest, against 1.4 that
+// a product of bf16 operands reaches; with the sums on the matrix core itself, cut off there, 12 % less.
 // FAR: rows so far apart that a tile spans 4 GB, with offsets of 64 bits (of 32, a load is one register of offset behind
 // a uniform base).
 template <int MB, int NB, int NW, int AHEAD, bool VEC, bool FAR>
@@ -363,7 +393,7 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_f32_tiled_kernel(
 #pragma unroll
   for (int i = 0; i < XV; ++i) xo[i] = 4 * ((Offset)min(row + 8 * NW * i, M - 1 - m0) * ldx + 4 * piece);
 
-  f32x4 raw[AHEAD][NB][2], xv[AHEAD][XV], whole[MB][NB], small[MB][NB];
+  f32x4 raw[AHEAD][NB][2], xv[AHEAD][XV], sum[MB][NB];
   GfParts wp[NB];
   // a whole step; what would be loaded ahead behind the last whole segment is its last step again
   auto load_w = [&](int set, int k) {
@@ -395,14 +425,21 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_f32_tiled_kernel(
     for (int j = 0; j < NB; ++j) wp[j] = gf_parts(raw[set][j][0], raw[set][j][1]);
   };
   auto multiply = [&](int buf) {
+    GfTerms terms[2][NB];  // a row of blocks is added up behind the next one's products
 #pragma unroll
     for (int i = 0; i < MB; ++i) {
       bf16x8 b[3];
 #pragma unroll
       for (int p = 0; p < 3; ++p) b[p] = *(const bf16x8*)&xs[buf][i][p][lane][0];
 #pragma unroll
-      for (int j = 0; j < NB; ++j) gf_step(wp[j], b[0], b[1], b[2], whole[i][j], small[i][j]);
+      for (int j = 0; j < NB; ++j) terms[i % 2][j] = gf_step(wp[j], b[0], b[1], b[2]);
+      if (i > 0) {
+#pragma unroll
+        for (int j = 0; j < NB; ++j) gf_fold(sum[i - 1][j], terms[(i - 1) % 2][j]);
+      }
     }
+#pragma unroll
+    for (int j = 0; j < NB; ++j) gf_fold(sum[MB - 1][j], terms[(MB - 1) % 2][j]);
   };
   // the end of the segment from k0 on
   auto close = [&](int k0) {
@@ -414,8 +451,8 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_f32_tiled_kernel(
 #pragma unroll
       for (int j = 0; j < NB; ++j) {
         f32x4 mid = first ? f32x4{0.f, 0.f, 0.f, 0.f} : mids[wave][i * NB + j][lane];
-        mid += whole[i][j] + small[i][j];
-        whole[i][j] = small[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        mid += sum[i][j];
+        sum[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
         if (!last) {
           mids[wave][i * NB + j][lane] = mid;
         } else if (m < M) {
@@ -439,7 +476,7 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_f32_tiled_kernel(
 #pragma unroll
   for (int i = 0; i < MB; ++i)
 #pragma unroll
-    for (int j = 0; j < NB; ++j) whole[i][j] = small[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < NB; ++j) sum[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   if (k_begin < k_full) {
 #pragma unroll
     for (int a = 0; a < AHEAD; ++a) {

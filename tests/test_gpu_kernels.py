@@ -491,6 +491,60 @@ def test_gemm_f32_every_tile_gives_the_bits_of_the_few_rows_kernel(ops, blocks, 
     assert ((few.double() - x.double() @ w.double().T).abs() <= bound).all()
 
 
+def _f32_operands(kind, rows, K):
+    """Operands whose products' parts round in different ways."""
+    one = lambda n: (torch.rand(n, 1) + 1).expand(n, K)
+    signs = lambda n: (torch.rand(n, K) < 0.5).float() * 2 - 1
+    return {"normal": lambda n: torch.randn(n, K), "one sign": lambda n: torch.randn(n, K).abs(), "uniform": lambda n: torch.rand(n, K),
+            "constant": one, "edge of a part": lambda n: (1 + 2.0 ** -8 - 2.0 ** -23) * signs(n)}[kind](rows).contiguous().to(DEV)
+
+
+@pytest.mark.parametrize("M", [8, 40])
+@pytest.mark.parametrize("K", [128, 1056, 3000, 14336])
+@pytest.mark.parametrize("kind", ["normal", "one sign", "uniform", "constant", "edge of a part"])
+def test_gemm_f32_error_against_64_bits(ops, kind, K, M):
+    """Every part of every product is there, over all of k: the error's 2-norm against what roundings of the sums make.  A
+    rounding is 0.4 x 2^-24 of a sum on average and the squares add up, over a chain of n sums to (n + 1) / 2: chains of 4
+    steps, 8 segments and the groups, and 3 roundings of a step's terms; twice that is allowed (constant rows round alike).
+    A part left out anywhere is 2^-18 of the result or more."""
+    torch.manual_seed(K + M)
+    x, w = _f32_operands(kind, M, K), _f32_operands(kind, 200, K)
+    want = x.double() @ w.double().T
+    bound = 2 * 0.4 * 2.0 ** -24 * (5 / 2 + 9 / 2 + (-(-K // 1024) + 1) / 2 + 3) ** 0.5
+    assert (ops.gemm_nt(x, w).double() - want).norm() <= bound * want.norm()
+
+
+@pytest.mark.parametrize("M", [8, 40])
+def test_gemm_f32_products_of_few_terms_are_rounded_once(ops, M):
+    """Eight equal products: their sum is off by its own rounding and what a product leaves out, at most 2^-24 each."""
+    for v, left_out in ((1 + 2.0 ** -8 - 2.0 ** -23, 2.0 ** -30), (1 + 2.0 ** -8 - 2.0 ** -17, 2.0 ** -24), (1.5 + 2.0 ** -23, 2.0 ** -30)):
+        x, w = torch.full((M, 8), v, device=DEV), torch.full((33, 8), v, device=DEV)
+        want = x.double() @ w.double().T
+        assert ((ops.gemm_nt(x, w).double() - want).abs() <= (2.0 ** -24 + left_out) * 1.001 * want).all(), v
+
+
+@pytest.mark.parametrize("M", [8, 40])
+@pytest.mark.parametrize("exponent", [-100, -109, -115, -120, -126, -135])
+def test_gemm_f32_small_operands_keep_their_bits(ops, M, exponent):
+    """Operands down to the smallest normal number and below: what larger ones give, scaled, as long as no part's last bits
+    are bf16's smallest (the parts' sum is exact there too, but cut elsewhere), and always as close to the 64 bits: below the
+    smallest normal number within 3/4 of an operand's last place, since the first part ends at 2^-133 and the second at
+    2^-141 there (at most 2^-134 times 2^-17 and 2^-142 times 2^-8 of the other operand are left out)."""
+    torch.manual_seed(M)
+    x, w = torch.rand(M, 300).to(DEV) + 1, torch.randn(70, 300).to(DEV)
+    scale, up = 2.0 ** exponent, 2.0 ** 100
+    small = (x * 2.0 ** -100) * (scale * up)
+    want, bound = small.double() @ (w * up).double().T, 4e-7 * (small.double().abs() @ (w * up).double().abs().T)
+    if exponent < -126:
+        bound += 0.75 * 2.0 ** -149 * (w * up).double().abs().sum(1)
+    got = ops.gemm_nt(small, w * up)
+    if exponent >= -115:
+        assert torch.equal(got, ops.gemm_nt(x, w) * 2.0 ** (exponent + 100))
+    # the longest way of a term through the sums: 4 steps' terms of two roundings, 3 segments, half a unit each
+    assert ((got.double() - want).abs() <= bound).all()
+    assert ((ops.gemm_nt(w * up, small).double() - want.T).abs() <= bound.T).all()  # small ones in the other operand
+
+
 @pytest.mark.parametrize("M", [3, 12, 40, 300])
 def test_gemm_f32_infinities_and_scales(ops, M):
     """Infinities and what rounds to one in 16 bits come out as in 32 bits; operands at far ends of the exponents lose
