@@ -266,7 +266,7 @@ __device__ __forceinline__ void gf_store4(float* __restrict__ y, int n, int N, b
   }
 }
 
-// Up to 16 rows (decode): bound by reading W once.  A workgroup owns 16 outputs; a round is one group, a wave takes
+// 16 rows (decode, and outputs too few for tiles): bound by reading W.  A workgroup owns 16 outputs of 16 rows; a round is one group, a wave takes
 // one of its segments, so 64 KB of W (every wave's next segment) are in flight a workgroup while the current ones
 // are multiplied; the segments' sums meet in LDS and are added in order by one thread an output.  N x K 3072 x 3072 /
 // 16384 x 3072 / 3072 x 8192: 14 / 46 / 33 us at 4 rows (4.4 TB/s of W at the largest), 18 / 56 / 41 at 16; with the fp32
@@ -281,6 +281,9 @@ __global__ __launch_bounds__(512) void gemm_f32_few_kernel(const float* __restri
   __shared__ bf16x4 parts[FEW ? 8 : 1][4][3][4][8][2];  // [wave][step][part][g][row][half]
   const int tid = threadIdx.x, lane = tid % FG_WAVE, wave = tid / FG_WAVE;
   const int r = lane % 16, g = lane / 16, n0 = blockIdx.x * 16;
+  x += (size_t)blockIdx.y * 16 * ldx;
+  y += (size_t)blockIdx.y * 16 * ldy;
+  M = min(M - (int)blockIdx.y * 16, 16);
   // rows behind the last repeat it: their outputs are not stored
   const float* wrow = w + (size_t)min(n0 + r, N - 1) * ldw;
   const float* xrow = x + (size_t)min(r, M - 1) * ldx;
@@ -360,10 +363,10 @@ __global__ __launch_bounds__(512) void gemm_f32_few_kernel(const float* __restri
 // under no condition (with one the compiler copies what it has just loaded, that is, waits for it: 1.7 us a step
 // instead of 0.6 where the products take 0.1).  A group's sum is kept in LDS, which leaves the registers to the loads.
 // With `part` a workgroup takes one group of k and stores its sum there ([groups][M][N]); else it adds each group's to
-// y.  The workgroups that read the same rows of W are neighbours on one die.
+// y.  A die's workgroups are an eighth of the tiles, those that read the same rows of W one after the other.
 //
 // N x K 16384 x 3072 / 5120 x 3072 / 3072 x 8192, us: 400 rows 290 / 105 / 159 (459 / 167 / 256 with the fp32
-// instructions), 2048 rows 1326 / 468 / 748 (1900 / 622 / 982): 0.93 PFLOP/s of bf16 at the largest, against 1.4 that
+// instructions), 2048 rows 1326 / 483 / 702 (1900 / 622 / 1000): 0.93 PFLOP/s of bf16 at the largest, against 1.4 that
 // a product of bf16 operands reaches; with the sums on the matrix core itself, cut off there, 12 % less.
 // FAR: rows so far apart that a tile spans 4 GB, with offsets of 64 bits (of 32, a load is one register of offset behind
 // a uniform base).
@@ -375,9 +378,9 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_f32_tiled_kernel(
   static_assert(4 % AHEAD == 0, "a segment's steps use the sets of registers in turn");
   __shared__ bf16x4 xs[2][MB][3][FG_WAVE][2];
   __shared__ f32x4 mids[NW][MB * NB][FG_WAVE];
-  const int unit = (blockIdx.x / 8 / row_tiles) * 8 + blockIdx.x % 8;
-  if (unit >= units) return;
-  const int m0 = (blockIdx.x / 8 % row_tiles) * TM, group = unit / col_tiles;
+  const int tile = blockIdx.x % 8 * (gridDim.x / 8) + blockIdx.x / 8;  // (workgroup i runs on die i % 8)
+  if (tile >= units * row_tiles) return;
+  const int unit = tile / row_tiles, m0 = tile % row_tiles * TM, group = unit / col_tiles;
   const int tid = threadIdx.x, lane = tid % FG_WAVE, wave = __builtin_amdgcn_readfirstlane(tid / FG_WAVE);
   const int r = lane % 16, g = lane / 16, n0 = (unit % col_tiles) * TN + wave * 16 * NB;
   const bool late = wave >= 4;
@@ -549,7 +552,7 @@ static int gf_launch(const GfCall& c) {
   const int wide = c.N % 4 == 0 && c.ldy % 4 == 0 && (uintptr_t)c.y % 16 == 0 && (uintptr_t)c.part % 16 == 0;
   const int row_tiles = (c.M + 16 * MB - 1) / (16 * MB), col_tiles = (c.N + 16 * NB * NW - 1) / (16 * NB * NW);
   const long long units = (long long)col_tiles * (c.part ? groups : 1);
-  const long long blocks = (units + 7) / 8 * 8 * row_tiles;
+  const long long blocks = (units * row_tiles + 7) / 8 * 8;
   if (blocks > 2147483647LL || (c.part && c.M > 65535)) return FG_ERR_ARG;
 #define TILED(VEC)                                                                                            \
   gemm_f32_tiled_kernel<MB, NB, NW, AHEAD, VEC, FAR><<<(unsigned)blocks, 64 * NW, 0, c.stream>>>(                  \
@@ -565,7 +568,7 @@ static int gf_launch(const GfCall& c) {
 }
 
 // mb, nw: the tile of the many-rows kernel, 16 mb rows (mb <= 5 with 4 waves, 7 with 8) and nw waves of 32 outputs
-// (mb = 0: up to 16 rows, no tile).
+// (mb = 0: the kernel of 16 rows).
 // part: null, or fp32 [ceil(K / 1024)][M][N] for a workgroup a group of k.
 extern "C" int fg_gemm_f32(const float* x, const float* w, float* y, float* part, int M, int N, int K, int ldx,
                            int ldw, int ldy, int mb, int nw, hipStream_t stream) {
@@ -573,8 +576,8 @@ extern "C" int fg_gemm_f32(const float* x, const float* w, float* y, float* part
   if (K <= 0 || ldx < K || ldw < K || ldy < N) return FG_ERR_ARG;
   const bool vec = K % 4 == 0 && ldx % 4 == 0 && ldw % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0;
   if (mb == 0) {
-    if (M > 16 || part) return FG_ERR_ARG;
-    const int blocks = (N + 15) / 16;
+    if (M > 16 * 65535 || part) return FG_ERR_ARG;
+    const dim3 blocks((N + 15) / 16, (M + 15) / 16);
 #define FEW_ROWS(FEW, VEC) gemm_f32_few_kernel<FEW, VEC><<<blocks, 512, 0, stream>>>(x, w, y, M, N, K, ldx, ldw, ldy)
     if (M <= 8) {
       if (vec) FEW_ROWS(true, true);

@@ -881,52 +881,55 @@ def paged_attention(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v
 GEMM_F32_GROUP = 1024
 
 
-def gemm_f32_tile_blocks(M: int, mb: int, nb: int) -> int:
-    """Blocks of 16 rows in a tile of :func:`gemm_f32_plan`: at most 3 (mb = 1: more loads in flight), or 5 or 7 (what
-    the registers of 2 workgroups of 4 waves or one of 8 hold a compute unit), as even as they come."""
-    blocks, most = -(-M // 16), 3 if mb == 1 else 5 if nb == 1 else 7
-    return -(-blocks // -(-blocks // most))
+# Up to this many rows the 32-bit product's kernel of 16 rows takes any size without scratch memory; the largest sums of
+# groups that other cuts put into memory, in bytes and in rows
+GEMM_F32_FEW_ROWS, GEMM_F32_MAX_SUMS, GEMM_F32_MAX_SPLIT_ROWS = 8, 256 << 20, 4096
 
 
 @functools.lru_cache(maxsize=4096)
 def gemm_f32_plan(M: int, N: int, K: int, cus: int) -> Tuple[int, int, bool]:
-    """How the 32-bit product is cut: (short or tall tiles, 1 or 2, see :func:`gemm_f32_tile_blocks`; tile columns /
-    128, whether every group of k has a workgroup of its own); (0, 0, False): the kernel of up to 16 rows.  Every cut
-    gives the same bits.
+    """How the 32-bit product is cut: (blocks of 16 rows in a tile, waves of 32 outputs in a tile, whether every group of k
+    has a workgroup of its own); (0, 0, False): the kernel of 16 rows and 16 outputs.  Every cut gives the same bits.
 
-    The cut whose workgroups take the least time as counted here.  32 k of a tile of b blocks of rows take 0.85 + 0.2 b
-    us where a compute unit is full (8 waves in one workgroup or two; measured 1.0 / 1.24 / 1.76 / 2.3 for b = 1 / 3 / 5 /
-    7), 0.45 + 0.19 b with 4 waves alone (0.6 / 0.98 / 1.37); the groups' sums pass through memory twice; W itself
-    comes at 5 TB/s at best; and the kernel of up to 16 rows takes 4.6 us a group of k and block of 16 outputs a
-    compute unit (16 rows, N x K 3072 x 3072 / 5120 x 3072 / 16384 x 3072 / 3072 x 8192: 18 / 30 / 60 / 41 us against 25 / 26
-    / 53 / 31 in tiles; up to 8 rows it is the faster or level everywhere, 15 / 26 / 50 / 33 against 25 / 26 / 53 / 31).
-    Counted and measured (us): 400 rows 16384 x 3072 229 and 240, 5120 x 3072 91 and 100, 3072 x 8192 158 and 148; 64 rows
-    3072 x 3072 29 and 29.  A workgroup a group only if the sums stay under 256 MB."""
-    if M <= 8:
+    The cut whose workgroups take the least time as counted here (244 sizes of 9 to 4,096 rows, N 64 to 28,672, K 512 to
+    14,336, every cut measured: 0.7 % above the best on average).  32 k of a tile of b blocks take 0.61 + 0.29 b us where a
+    compute unit is full (8 waves in one workgroup or two), 0.44 + 0.2 b with 4 waves alone; a die has an eighth of the
+    tiles; the groups' sums pass through memory twice, at 6 TB/s and with 2 us for their kernel; a group of k takes the
+    kernel of 16 rows 4.8 us with one workgroup a unit and 10 with two, its last segments alone a third of that; W itself
+    comes at 5 TB/s at best.  Counted and measured (us): 400 rows 16384 x 3072 281 and 290, 5120 x 3072 102 and 105,
+    2048 x 2048 44 and 45; 64 rows 512 x 2048 12 and 12.  (On the fp32 matrix instructions, 32 x 32 outputs a workgroup,
+    products that fill the chip took 1.3 to 1.7 times as long, and some below 30 us that do not 3 to 8 us less.)"""
+    if M <= GEMM_F32_FEW_ROWS:
         return 0, 0, False
-    groups, streaming = -(-K // GEMM_F32_GROUP), N * K * 4 / 5e6
-    best = (4 + 4.6 * groups * -(-N // (16 * cus)), (0, 0, False)) if M <= 16 else (float("inf"), None)
-    for mb in (2, 1):
-        for nb in (2, 1):
-            b = gemm_f32_tile_blocks(M, mb, nb)
-            tiles, full, alone = -(-M // (16 * b)) * -(-N // (128 * nb)), 0.85 + 0.2 * b, 0.45 + 0.19 * b
+    groups, blocks, streaming = -(-K // GEMM_F32_GROUP), -(-M // 16), N * K * 4 / 5e6
+    part = K % GEMM_F32_GROUP / GEMM_F32_GROUP
+    whole = K // GEMM_F32_GROUP + (0.35 + 0.65 * part if part else 0)
+    wgs = -(-N // 16) * blocks
+    best = 2 + max(whole * (4.8 if wgs <= cus else 10 * -(-wgs // (2 * cus))), streaming), (0, 0, False)
+    for waves, tallest in ((8, 7), (4, 5)):  # (what the registers hold)
+        for b in range(1, tallest + 1):
+            row_tiles = -(-blocks // b)
+            if b > 1 and -(-blocks // (b - 1)) == row_tiles:
+                continue  # as few tiles with shorter ones
+            full, alone = 0.61 + 0.29 * b, 0.44 + 0.2 * b
             for split in (False, True):
-                if split and (groups == 1 or M > 4096 or groups * M * N * 4 > 256 << 20):
+                if split and (groups == 1 or M > GEMM_F32_MAX_SPLIT_ROWS or groups * M * N * 4 > GEMM_F32_MAX_SUMS):
                     continue
-                units = tiles * groups if split else tiles
-                rounds, rest = divmod(units, 2 * cus // nb)
-                time = rounds * full + (full if nb == 2 or rest > cus else alone if rest else 0)
-                time *= GEMM_F32_GROUP // 32 if split else -(-K // 32)
-                time = max(time, streaming) + (5 + groups * M * N * 4 / 2e6 if split else 0)
+                die = -(-row_tiles * -(-N // (32 * waves)) * (groups if split else 1) // 8)
+                rounds, rest = divmod(die, cus // 8 * (8 // waves))
+                time = rounds * full + (0 if not rest else alone if waves == 4 and rest <= cus // 8 else full)
+                time = max(time * (GEMM_F32_GROUP // 32 if split else -(-K // 32)), streaming)
+                time += 5 + (2 + groups * M * N * 8 / 6e6 if split else 0)
                 if time < best[0]:
-                    best = time, (mb, nb, split)
+                    best = time, (b, waves, split)
     return best[1]
 
 
 def gemm_f32_scratch(M: int, N: int, K: int) -> int:
     """Bytes of the groups' sums that :func:`gemm_nt` takes at most for up to ``M`` rows (see :func:`gemm_f32_plan`)."""
     groups = -(-K // GEMM_F32_GROUP)
-    return min(groups * min(M, 4096) * N * 4, 256 << 20) if groups > 1 and M > 16 else 0
+    sums = min(groups * min(M, GEMM_F32_MAX_SPLIT_ROWS) * N * 4, GEMM_F32_MAX_SUMS)
+    return sums if groups > 1 and M > 16 else 0
 
 
 def gemm_nt(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None,
@@ -943,11 +946,10 @@ def gemm_nt(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None
         out = torch.empty((M, N), dtype=out_dtype or x.dtype, device=x.device)
     _need(out.shape == (M, N) and out.stride(1) == 1, "out must be [M, N]")
     if x.dtype == torch.float32 and out.dtype == torch.float32:
-        mb, nb, split = gemm_f32_plan(M, N, K, compute_units())
+        blocks, waves, split = gemm_f32_plan(M, N, K, compute_units())
         part = torch.empty((-(-K // GEMM_F32_GROUP), M, N), dtype=torch.float32, device=x.device) if split else None
-        blocks = gemm_f32_tile_blocks(M, mb, nb) if mb else 0
         st = _lib.load("gemm").fg_gemm_f32(
-            _ptr(x), _ptr(w), _ptr(out), _ptr(part), M, N, K, x.stride(0), w.stride(0), out.stride(0), blocks, 4 * nb,
+            _ptr(x), _ptr(w), _ptr(out), _ptr(part), M, N, K, x.stride(0), w.stride(0), out.stride(0), blocks, waves,
             _stream(out))
         _check(st, "gemm_nt")
         return out

@@ -426,7 +426,8 @@ def test_gemm_rows_do_not_depend_on_the_batch(ops):
 def test_gemm_f32_every_cut_gives_the_same_bits(ops, N, K):
     """The 32-bit product at the edges of its tiles, segments of 128 k and groups of 1024: the rows of a call, alone or
     beside others, in rows of another stride (unaligned: the scalar loads), within the bound of the longest chain of
-    additions (32 in a chain of instructions, 4 chains, 8 segments, K / 1024 groups) of the double product."""
+    additions (32 k of an instruction, 4 steps, 8 segments, K / 1024 groups) of the double product; the parts of products:
+    test_gemm_f32_error_against_64_bits."""
     torch.manual_seed(N + K)
     x, w = torch.randn(203, K).to(DEV), torch.randn(N, K).to(DEV)
     x[7, K // 2] = float("nan")  # its row and no other
@@ -459,22 +460,41 @@ def test_gemm_f32_rows_far_apart(ops, M, N, K, ldx, ldw):
     assert torch.equal(ops.gemm_nt(*far), ops.gemm_nt(x, w))
 
 
-@pytest.mark.parametrize("N,K", [(130, 1100), (3072, 1028)])
-def test_gemm_f32_bits_around_the_line_of_the_narrow_tiles(ops, N, K):
-    """Up to 640 rows a last tile of at most 32 rows makes all tiles that narrow, beyond it does not: the same bits."""
+@pytest.mark.parametrize("N,K", [(1030, 1100), (3072, 1028), (515, 2049)])
+def test_gemm_f32_bits_around_the_lines_of_the_plan(ops, N, K):
+    """The last number of rows that is cut in one way and the first one that is cut in another: the same bits."""
     torch.manual_seed(N)
     x, w = torch.randn(720, K).to(DEV), torch.randn(N, K).to(DEV)
     full = ops.gemm_nt(x, w)
-    for M in (16, 608, 609, 640, 641, 672, 673):
-        assert torch.equal(ops.gemm_nt(x[:M], w), full[:M]), M
+    plan = lambda M: ops.gemm_f32_plan(M, N, K, ops.compute_units())
+    lines = [M for M in range(1, 720) if plan(M) != plan(M + 1)]
+    assert len(lines) >= 2 and lines[0] >= 8
+    for M in sorted({1, 8, 9, 16, 17, *lines, *(M + 1 for M in lines)}):
+        assert torch.equal(ops.gemm_nt(x[:M], w), full[:M]), (M, plan(M))
 
 
-@pytest.mark.parametrize("K", [24, 128, 156, 1056, 2200])
+@pytest.mark.parametrize("M,N,K", [(9, 40, 17), (16, 130, 1031), (17, 64, 129), (100, 515, 2048), (203, 33, 41)])
+def test_gemm_f32_kernel_of_16_rows_at_any_number_of_rows(ops, M, N, K):
+    """Sixteen rows a workgroup, the last one's fewer; rows that can and cannot be read in fours."""
+    from fastgen_amd.kernels import _lib
+
+    torch.manual_seed(M)
+    wide = torch.randn(M, K + 3).to(DEV)
+    w = torch.randn(N, K).to(DEV)
+    for x in (wide[:, 3:], wide[:, :K].contiguous()):
+        y = torch.full((M, N), 7.0, device=DEV)
+        st = _lib.load("gemm").fg_gemm_f32(ops._ptr(x), ops._ptr(w), ops._ptr(y), None, M, N, K, x.stride(0), K, N, 0, 0,
+                                           ops._stream(y))
+        few = torch.cat([ops.gemm_nt(x[m:m + 8], w) for m in range(0, M, 8)])
+        assert st == 0 and torch.equal(y, few)
+
+
+@pytest.mark.parametrize("K", [24, 37, 128, 156, 1056, 1151, 2200])
 @pytest.mark.parametrize("blocks,waves", [(b, w) for w in (4, 8) for b in range(1, 8 if w == 8 else 6)])
 def test_gemm_f32_every_tile_gives_the_bits_of_the_few_rows_kernel(ops, blocks, waves, K):
     """Every tile of the many-rows kernel, with and without a workgroup a group of k: rows and outputs that end inside
-    a block, k inside a step, a segment and a group; within the longest chain of additions (4 instructions of 8
-    products at a time, 5 segments' parts, 8 segments, the groups)."""
+    a block, k inside a step, a segment and a group, rows that cannot be read in fours; within the longest chain of
+    additions (32 k of an instruction, 2 of a step's terms, 4 steps, 8 segments, the groups)."""
     from fastgen_amd.kernels import _lib
 
     torch.manual_seed(100 * blocks + K)
@@ -483,11 +503,14 @@ def test_gemm_f32_every_tile_gives_the_bits_of_the_few_rows_kernel(ops, blocks, 
     few = torch.cat([ops.gemm_nt(x[m:m + 8], w) for m in range(0, M, 8)])
     assert ops.gemm_f32_plan(8, N, K, 256) == (0, 0, False)
     y, part = torch.full_like(few, 7.0), torch.empty(-(-K // 1024), M, N, device=DEV)
+    odd = torch.empty(M, K + 1, device=DEV)[:, 1:].copy_(x)
     for p in (None, part):
-        st = _lib.load("gemm").fg_gemm_f32(ops._ptr(x), ops._ptr(w), ops._ptr(y), ops._ptr(p), M, N, K, K, K, N, blocks,
-                                           waves, ops._stream(y))
-        assert st == 0 and torch.equal(y, few)
-    bound = (32 + 8 + K / 1024 + 4) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+        for rows in (x, odd):
+            y.fill_(7.0)
+            st = _lib.load("gemm").fg_gemm_f32(ops._ptr(rows), ops._ptr(w), ops._ptr(y), ops._ptr(p), M, N, K, rows.stride(0),
+                                               K, N, blocks, waves, ops._stream(y))
+            assert st == 0 and torch.equal(y, few)
+    bound = (32 + 2 + 4 + 8 + K / 1024) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
     assert ((few.double() - x.double() @ w.double().T).abs() <= bound).all()
 
 
@@ -569,8 +592,8 @@ def test_gemm_f32_plan_is_bounded(ops):
     for M in (1, 16, 17, 64, 65, 400, 4096, 4097, 200000):
         for N in (1, 64, 3072, 128256):
             for K in (8, 1024, 1025, 3072, 28672):
-                mb, nb, split = ops.gemm_f32_plan(M, N, K, 256)
-                assert (mb, nb) in ((0, 0), (1, 1), (1, 2), (2, 1), (2, 2)) and (mb > 0 or M <= 16)
+                blocks, waves, split = ops.gemm_f32_plan(M, N, K, 256)
+                assert 1 <= blocks <= {4: 5, 8: 7}[waves] if waves else (blocks, split) == (0, False) and M <= 65535 * 16
                 assert not split or (M <= 65535 and -(-K // 1024) * M * N * 4 <= 256 << 20)
 
 
