@@ -929,7 +929,7 @@ def gemm_f32_scratch(M: int, N: int, K: int) -> int:
     """Bytes of the groups' sums that :func:`gemm_nt` takes at most for up to ``M`` rows (see :func:`gemm_f32_plan`)."""
     groups = -(-K // GEMM_F32_GROUP)
     sums = min(groups * min(M, GEMM_F32_MAX_SPLIT_ROWS) * N * 4, GEMM_F32_MAX_SUMS)
-    return sums if groups > 1 and M > 16 else 0
+    return sums if groups > 1 and M > GEMM_F32_FEW_ROWS else 0
 
 
 def gemm_nt(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None,

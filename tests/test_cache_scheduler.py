@@ -673,3 +673,8 @@ def test_step_memory_estimate_counts_what_parts_take_beside_their_rows():
         for N, K in ((64, 1025), (3072, 8192), (16384, 3072), (28672, 8192)):
             if ops.gemm_f32_plan(M, N, K, cus)[2]:
                 assert -(-K // ops.GEMM_F32_GROUP) * M * N * 4 <= ops.gemm_f32_scratch(8192, N, K)
+    for M in range(1, 65):  # an engine of few tokens a step: its largest step counts
+        for N, K in ((5120, 3072), (16384, 3072), (3072, 8192), (4096, 14336), (1000, 1100)):
+            taken = max((-(-K // ops.GEMM_F32_GROUP) * m * N * 4 for m in range(1, M + 1)
+                         if ops.gemm_f32_plan(m, N, K, cus)[2]), default=0)
+            assert taken <= ops.gemm_f32_scratch(M, N, K), (M, N, K)
