@@ -29,8 +29,9 @@
 // products are cut off below the largest of them.  Magnitudes down to the
 // smallest normal number change nothing; of an operand below it up to 3/4 of its
 // last place is left out.  Infinities (and what rounds to one in
-// bf16) have no such parts: an output that comes out as NaN is computed again,
-// one fp32 FMA a product (gf_again).
+// bf16) have no such parts, and a part's product may be one where the whole one
+// is not: an output that comes out as no number is computed again, one fp32 FMA
+// a product (gf_again).
 //
 // Operands of bf16 with fp32 accumulation take the FMA kernel below, so that
 // any shape has a product when the tuned kernels refuse it.
@@ -237,7 +238,9 @@ __device__ __forceinline__ void gf_fold(f32x4& sum, const GfTerms& t) {
   asm volatile("" : "+v"(sum));  // here, or the compiler keeps every step's terms up to the segment's end, in scratch memory
 }
 
-// An output whose sum came out as NaN: the operands may hold an infinity.
+// An output whose sum is no number: the operands may hold an infinity, or a part's product have rounded up to one where
+// the whole product is just below the largest number.
+__device__ __forceinline__ bool gf_lost(float sum) { return !(fabsf(sum) <= 3.402823466e38f); }
 __device__ __noinline__ float gf_again(const float* x, const float* w, int K) {
   float sum = 0.f;
   for (int k = 0; k < K && sum == sum; ++k) sum = fmaf(w[k], x[k], sum);
@@ -349,7 +352,7 @@ __global__ __launch_bounds__(512) void gemm_f32_few_kernel(const float* __restri
   if (tid < 256) {
     const int m = (tid / 4) % 16, n = n0 + (tid / 64) * 4 + tid % 4;
     if (m < M && n < N) {
-      if (total != total) total = gf_again(x + (size_t)m * ldx, w + (size_t)n * ldw, K);
+      if (gf_lost(total)) total = gf_again(x + (size_t)m * ldx, w + (size_t)n * ldw, K);
       y[(size_t)m * ldy + n] = total;
     }
   }
@@ -468,7 +471,7 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_f32_tiled_kernel(
             if (next >= k_end) {
 #pragma unroll
               for (int e = 0; e < 4; ++e)
-                if (mid[e] != mid[e] && n + e < N) mid[e] = gf_again(x + (size_t)m * ldx, w + (size_t)(n + e) * ldw, K);
+                if (gf_lost(mid[e]) && n + e < N) mid[e] = gf_again(x + (size_t)m * ldx, w + (size_t)(n + e) * ldw, K);
             }
             gf_store4(out, n, N, wide, mid);
           }
@@ -534,7 +537,7 @@ __global__ __launch_bounds__(256) void gemm_f32_sum_kernel(const float* __restri
   for (int g = 0; g < groups; ++g) total += gf_read4(part + ((size_t)g * M + m) * N, n, N, wide);
 #pragma unroll
   for (int e = 0; e < 4; ++e)
-    if (total[e] != total[e] && n + e < N) total[e] = gf_again(x + (size_t)m * ldx, w + (size_t)(n + e) * ldw, K);
+    if (gf_lost(total[e]) && n + e < N) total[e] = gf_again(x + (size_t)m * ldx, w + (size_t)(n + e) * ldw, K);
   gf_store4(y + (size_t)m * ldy, n, N, wide, total);
 }
 

@@ -588,6 +588,29 @@ def test_gemm_f32_infinities_and_scales(ops, M):
         assert torch.equal(ops.gemm_nt(x * a, w * b), plain * (a * b))
 
 
+@pytest.mark.parametrize("M", [3, 12, 40])
+def test_gemm_f32_just_below_the_largest_number(ops, M):
+    """Products whose first parts' product is an infinity and whose value is not, alone and at the end of a row of groups of k
+    (tiles with and without a workgroup a group); what is too large is an infinity."""
+    from fastgen_amd.kernels import _lib
+
+    a = 2.0 ** 64 * (1 - 2.0 ** -12)
+    for K in (1, 1100, 3000):
+        x, w = torch.zeros(M, K, device=DEV), torch.zeros(300, K, device=DEV)
+        x[:, K - 1], w[:, K - 1] = a, a
+        x[1, K - 1], w[7, K - 1] = 2.0 ** 64, -a
+        w[9, K - 1] = -(2.0 ** 64)
+        want = (x.double() @ w.double().T).float()
+        assert torch.isfinite(want[0, 0]) and torch.isinf(want[1, 9])
+        assert torch.equal(ops.gemm_nt(x, w), want), K
+        if M > 16:
+            for part in (None, torch.empty(-(-K // 1024), M, 300, device=DEV)):
+                y = torch.empty(M, 300, device=DEV)
+                st = _lib.load("gemm").fg_gemm_f32(ops._ptr(x), ops._ptr(w), ops._ptr(y), ops._ptr(part), M, 300, K, K, K, 300, 2, 4,
+                                                   ops._stream(y))
+                assert st == 0 and torch.equal(y, want), K
+
+
 def test_gemm_f32_plan_is_bounded(ops):
     for M in (1, 16, 17, 64, 65, 400, 4096, 4097, 200000):
         for N in (1, 64, 3072, 128256):
