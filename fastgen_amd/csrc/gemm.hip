@@ -274,10 +274,11 @@ __device__ __forceinline__ void gf_store4(float* __restrict__ y, int n, int N, b
 // are multiplied; the segments' sums meet in LDS and are added in order by one thread an output.  N x K 3072 x 3072 /
 // 16384 x 3072 / 3072 x 8192: 14 / 46 / 33 us at 4 rows (4.4 TB/s of W at the largest), 18 / 56 / 41 at 16; with the fp32
 // instructions 14 / 48 / 33 and 17 / 60 / 41.
+// Two workgroups a compute unit (at most 128 registers): 441 workgroups of two groups 13 us, 15.7 with one.
 // A wave cuts its segment of x into parts once: with FEW (up to 8 rows), each number in one lane, through LDS into
 // the operands' order; above, every lane the operand it needs.
 template <bool FEW, bool VEC>
-__global__ __launch_bounds__(512) void gemm_f32_few_kernel(const float* __restrict__ x, const float* __restrict__ w,
+__global__ __launch_bounds__(512, 4) void gemm_f32_few_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                            float* __restrict__ y, int M, int N, int K, int ldx,
                                                            int ldw, int ldy) {
   __shared__ f32x4 sums[2][8][FG_WAVE];

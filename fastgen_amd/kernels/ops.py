@@ -891,21 +891,22 @@ def gemm_f32_plan(M: int, N: int, K: int, cus: int) -> Tuple[int, int, bool]:
     """How the 32-bit product is cut: (blocks of 16 rows in a tile, waves of 32 outputs in a tile, whether every group of k
     has a workgroup of its own); (0, 0, False): the kernel of 16 rows and 16 outputs.  Every cut gives the same bits.
 
-    The cut whose workgroups take the least time as counted here (244 sizes of 9 to 4,096 rows, N 64 to 28,672, K 512 to
-    14,336, every cut measured: 0.7 % above the best on average).  32 k of a tile of b blocks take 0.61 + 0.29 b us where a
+    The cut whose workgroups take the least time as counted here (257 sizes of 4 to 4,096 rows, N 64 to 28,672, K 512 to
+    14,336, every cut measured: 0.3 % above the best on average).  32 k of a tile of b blocks take 0.61 + 0.29 b us where a
     compute unit is full (8 waves in one workgroup or two), 0.44 + 0.2 b with 4 waves alone; a die has an eighth of the
     tiles; the groups' sums pass through memory twice, at 6 TB/s and with 2 us for their kernel; a group of k takes the
-    kernel of 16 rows 4.8 us with one workgroup a unit and 10 with two, its last segments alone a third of that; W itself
-    comes at 5 TB/s at best.  Counted and measured (us): 400 rows 16384 x 3072 281 and 290, 5120 x 3072 102 and 105,
-    2048 x 2048 44 and 45; 64 rows 512 x 2048 12 and 12.  (On the fp32 matrix instructions, 32 x 32 outputs a workgroup,
-    products that fill the chip took 1.3 to 1.7 times as long, and some below 30 us that do not 3 to 8 us less.)"""
+    kernel of 16 rows 4.8 us with at most one workgroup a unit and 1.6 + 4 a unit's worth beyond, 9 at least, a part of a
+    group as much less as it is shorter; W itself comes at 5 TB/s at best.  Counted and measured (us): 400 rows 16384 x 3072
+    281 and 290, 5120 x 3072 102 and 105, 2048 x 2048 44 and 45; 64 rows 512 x 2048 12 and 12.  (On the fp32 matrix
+    instructions, 32 x 32 outputs a workgroup, products that fill the chip took 1.3 to 1.7 times as long, and some below 30
+    us that do not 1 to 6 us less.)"""
     if M <= GEMM_F32_FEW_ROWS:
         return 0, 0, False
     groups, blocks, streaming = -(-K // GEMM_F32_GROUP), -(-M // 16), N * K * 4 / 5e6
     part = K % GEMM_F32_GROUP / GEMM_F32_GROUP
-    whole = K // GEMM_F32_GROUP + (0.35 + 0.65 * part if part else 0)
+    whole = K // GEMM_F32_GROUP + (max(0.4, part) if part else 0)
     wgs = -(-N // 16) * blocks
-    best = 2 + max(whole * (4.8 if wgs <= cus else 10 * -(-wgs // (2 * cus))), streaming), (0, 0, False)
+    best = 2 + max(whole * (4.8 if wgs <= cus else max(9, 1.6 + 4 * wgs / cus)), streaming), (0, 0, False)
     for waves, tallest in ((8, 7), (4, 5)):  # (what the registers hold)
         for b in range(1, tallest + 1):
             row_tiles = -(-blocks // b)
