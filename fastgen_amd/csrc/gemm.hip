@@ -325,7 +325,9 @@ __global__ __launch_bounds__(512, 4) void gemm_f32_few_kernel(const float* __res
           if (2 * i < M) gf_parts4(xv[i], &to[0][c % 4][row][c / 4 % 2], &to[1][c % 4][row][c / 4 % 2],
                                    &to[2][c % 4][row][c / 4 % 2]);
         }
-        __builtin_amdgcn_wave_barrier();  // (a wave reads only what it has written itself)
+        // a wave reads only what it has written itself, but a lane what others have: behind their stores
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_wave_barrier();
       }
       f32x4 sum = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
