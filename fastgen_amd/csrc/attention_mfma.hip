@@ -263,15 +263,15 @@ __device__ __forceinline__ void load_q(bf16x8 (&qop)[NKS], const bf16_t* qrow, b
 }
 
 // An output gate [tokens, heads * HD] (g null: none): the attention's rounded output times it, or times its sigmoid, where
-// the output is stored: rounded, multiplied and rounded again, as a kernel of its own behind this one does it.  The
-// sigmoid takes the hardware's exponential and reciprocal (errors of 1e-7, far below the rounding that follows): the
-// library's, 64 a lane at the end of a prompt's workgroup, cost 5 us of the 10 that the other kernel took.
+// the output is stored: rounded, multiplied and rounded again, as a kernel of its own behind this one does it, the same
+// bits (so the sigmoid is the library's: the hardware's exponential and reciprocal are 3 us a layer of a prompt faster and
+// may move the last rounding).
 struct OutGate {
   const bf16_t* g;
   int stride, sigmoid;
 };
 __device__ __forceinline__ float gated(float o, float g, int sigmoid) {
-  return (float)(__bf16)o * (sigmoid ? __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-g * LOG2E)) : g);
+  return (float)(__bf16)o * (sigmoid ? 1.f / (1.f + expf(-g)) : g);
 }
 __device__ __forceinline__ bf16x4 out4(const f32x4 o) {
   bf16x4 v;
@@ -286,7 +286,7 @@ __device__ __forceinline__ bf16x4 gated4(const f32x4 o, const bf16x4 g, int sigm
   return v;
 }
 // A row's blocks of 16 outputs, times inv, to token t's columns from c on (four a lane of each): the gate's loads all
-// in flight together (1897 tokens of 16 heads: 40.8 us without a gate, 42.6 with its sigmoid; the other
+// in flight together (1897 tokens of 16 heads: 40.8 us without a gate, 45.8 with its sigmoid; the other
 // kernel takes 10.5).
 __device__ __forceinline__ void store_row(bf16_t* __restrict__ out, int out_stride, const f32x4 (&o)[NDB], float inv, int t,
                                           int c, const OutGate gate) {
