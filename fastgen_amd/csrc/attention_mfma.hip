@@ -319,9 +319,8 @@ __device__ __forceinline__ const OutGate& the_gate(const OutGate& gate) { return
 //   (0: this chunk is not in use), number of this chunk among its item's;
 //   from [4 + 8 * max_chunks] on the same chunks, longest first, with their place in the first list instead of that
 //   number: the order in which the split kernel takes them.  Chunks of items of many lengths are of many lengths too, and
-//   with more workgroups than places a long one begun last is what the kernel ends with: 64 sequences of 100 to 2,400
-//   keys, 8 kv heads, 760 workgroups on 512 places: 74 us a layer
-//   in the items' order, 66 so.
+//   with more workgroups than compute units a long one begun last, or beside another long one, is what the kernel ends
+//   with: 64 sequences of 100 to 2,400 keys, 8 kv heads, 760 workgroups: 77.2 us a layer in the items' order, 68.1 so.
 #define COMBINE_MAX_SPLITS 256
 #define COMBINE_ROWS_MAX_GROUPS 8192  // up to this many workgroups the combine takes a workgroup a row
 constexpr int PLAN_HEAD = 4;
@@ -787,8 +786,8 @@ static int page_shift_of(int page_size) {
   return -1;
 }
 
-// ints of a plan of max_chunks chunks
-extern "C" long long fg_attn_plan_ints(int max_chunks) { return PLAN_HEAD + 16LL * max_chunks; }
+// ints of a plan of max_chunks chunks; the second list takes 8 * max_chunks more
+extern "C" long long fg_attn_plan_ints(int max_chunks) { return PLAN_HEAD + 8LL * max_chunks; }
 
 // Cuts the items (int32 [n_items][4], 16-byte aligned) into chunks: see the layout of `plan` above.
 // max_chunks >= 2 * n_items; min_tiles: a chunk's tiles are a multiple of it (4: one tile a wave).  ordered: with the

@@ -628,30 +628,33 @@ def attention_chunks_for(n_items: int, n_kv: int) -> int:
     return max(-(-_split_target_blocks() // n_kv) + n_items, 2 * n_items)
 
 
-def _plan_ordered(n_items: int) -> int:
-    """Whether the split kernel takes the chunks longest first: not for up to 16 items, whose chunks but the last ones are of
-    one length (the second list costs the plan 3 us, a decode step of one request 0.5 % with it for nothing)."""
-    return int(n_items > 16)
+def _plan_ordered(n_items: int, n_kv: int) -> bool:
+    """Whether the split kernel takes the chunks longest first: not for up to 16 items (the second list costs the plan 3 us, a
+    decode step of one request 0.5 % with it for nothing)."""
+    return n_items > 16
 
 
-def _plan_ints(lib, max_chunks: int) -> int:
+def _plan_ints(lib, max_chunks: int, ordered: bool) -> int:
     lib.fg_attn_plan_ints.restype = ctypes.c_longlong
-    return int(lib.fg_attn_plan_ints(max_chunks))
+    return int(lib.fg_attn_plan_ints(max_chunks)) + (8 * max_chunks if ordered else 0)
 
 
 def attention_plan(items: torch.Tensor, n_items: int, max_chunks: int, head_dim: int, window: int = 0,
-                   min_tiles: int = 4, exact: bool = False, dist: bool = False) -> torch.Tensor:
+                   min_tiles: int = 4, exact: bool = False, dist: bool = False,
+                   ordered: Optional[bool] = None) -> torch.Tensor:
     """Cuts the key ranges of ``items`` (device int32 ``[n_items, 4]``, 16-byte aligned) into chunks of
     the same number of 64-key tiles, a multiple of ``min_tiles``, on the device: a captured step cuts
-    anew for the lengths of every replay.  The int32 plan that :func:`paged_attention_mfma` takes."""
+    anew for the lengths of every replay.  The int32 plan that :func:`paged_attention_mfma` takes, which sees
+    from its size whether it lists the chunks a second time, longest first (``ordered``; default: with more than
+    16 items)."""
     _gpu(items)
     _i32(items, "items")
     _need(items.data_ptr() % 16 == 0 and items.numel() >= 4 * n_items > 0, "items must be [n, 4], 16-byte aligned")
     _need(max_chunks >= 2 * n_items and min_tiles >= 1, "max_chunks must be at least twice the number of items")
     lib = _mfma_attention(head_dim, exact, dist)  # the plan is the same for every head size and build
-    plan = torch.empty(_plan_ints(lib, max_chunks), dtype=torch.int32, device=items.device)
-    _check(lib.fg_attn_plan_ordered(_ptr(items), n_items, int(window or 0), max_chunks, min_tiles, _plan_ordered(n_items),
-                                    _ptr(plan),
+    ordered = n_items > 16 if ordered is None else bool(ordered)
+    plan = torch.empty(_plan_ints(lib, max_chunks, ordered), dtype=torch.int32, device=items.device)
+    _check(lib.fg_attn_plan_ordered(_ptr(items), n_items, int(window or 0), max_chunks, min_tiles, int(ordered), _ptr(plan),
                                     _stream(items)), "attn_plan")
     return plan
 
@@ -783,15 +786,17 @@ def paged_attention_mfma(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tens
             max_chunks = attention_chunks_for(n, n_kv)
         _need(2 * n <= max_chunks <= 65535, "the chunk list holds at least two chunks an item and at most 65535")
         if plan is None:
-            plan = attention_plan(small_items, n, max_chunks, hd, window, min_tiles, exact_weights, dist)
-        _need(plan.dtype == torch.int32 and plan.numel() == _plan_ints(lib, max_chunks),
+            plan = attention_plan(small_items, n, max_chunks, hd, window, min_tiles, exact_weights, dist,
+                                  _plan_ordered(n, n_kv))
+        ordered = plan.numel() == _plan_ints(lib, max_chunks, True)
+        _need(plan.dtype == torch.int32 and (ordered or plan.numel() == _plan_ints(lib, max_chunks, False)),
               "the plan does not fit the items and max_chunks")
         part_o = torch.empty((max_chunks * n_kv * 16, hd), dtype=torch.float32, device=q.device)
         part_ml = torch.empty((max_chunks * n_kv * 16, 2), dtype=torch.float32, device=q.device)
         st = lib.fg_attn_split_sink(
             _ptr(q), q.stride(0), _ptr(out), out.stride(0), _ptr(k_pages), _ptr(v_pages), _ptr(block_table),
             block_table.stride(0), _ptr(plan), n, max_chunks, max_rows, _ptr(part_o), _ptr(part_ml), n_heads, n_kv, hd,
-            page_size, ctypes.c_float(scale), int(window or 0), _ptr(sinks), _ptr(distance), *gate_args, _plan_ordered(n),
+            page_size, ctypes.c_float(scale), int(window or 0), _ptr(sinks), _ptr(distance), *gate_args, int(ordered),
             int(not leave_parts), _stream(q))
         _check(st, "attn_split")
         if leave_parts:
@@ -866,7 +871,7 @@ def paged_attention(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v
         split_plan = ctx.scratch.get(key)
         if split_plan is None:
             split_plan = ctx.scratch[key] = attention_plan(small_d, n_small, chunks, hd, window, _SPLIT_MIN_TILES,
-                                                           exact_weights, dist)
+                                                           exact_weights, dist, _plan_ordered(n_small, n_kv))
     # rows of the largest small item: one token a sequence in a decode step (also a captured one)
     rows = G * int(ctx.q_lens.max()) if big_d is None else 16
     return paged_attention_mfma(q, out, k_pages, v_pages, group.block_table, small_d, big_d, n_heads, scale,

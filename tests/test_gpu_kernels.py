@@ -1212,6 +1212,28 @@ def test_paged_attention_mfma_many_decoding_sequences(ops, n_items, cut):
     assert torch.allclose(out.cpu().float(), _plain_rows(case, seqs), atol=1.5e-2, rtol=2e-2)
 
 
+@pytest.mark.parametrize("listed,planned", [(20, 12), (17, 16), (40, 17), (20, 20), (12, 12)])
+def test_attention_takes_the_plan_that_it_is_given(ops, listed, planned):
+    """A plan of the first of the listed items, with and without the second list: those items' rows, the same bits, and no
+    others (the attention goes by the plan, not by how many items it sees)."""
+    H, KV, hd = 8, 2, 64
+    seqs = [(97 * i % 900, 1) for i in range(listed)]
+    case = _paged_case(torch.bfloat16, seqs, H, KV, hd, 32, seed=listed)
+    items = torch.tensor([(i, i, 1, n0) for i, (n0, _) in enumerate(seqs)], dtype=torch.int32, device=DEV).reshape(-1)
+    chunks = ops.attention_chunks_for(listed, KV)
+    outs = []
+    for ordered in (None, False, True):
+        plan = ops.attention_plan(items, planned, chunks, hd, ordered=ordered)
+        out = torch.full((listed, H * hd), 7.0, dtype=torch.bfloat16, device=DEV)
+        outs.append(ops.paged_attention_mfma(case["q"], out, case["kp"], case["vp"], case["table"], items, None, H, hd ** -0.5,
+                                             plan=plan, max_chunks=chunks, max_rows=H // KV))
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2]) and (outs[0][planned:] == 7.0).all()
+    assert torch.allclose(outs[0][:planned].cpu().float(), _plain_rows(case, seqs)[:planned], atol=1.5e-2, rtol=2e-2)
+    with pytest.raises(ops.KernelArgumentError):
+        ops.paged_attention_mfma(case["q"], outs[0], case["kp"], case["vp"], case["table"], items, None, H, hd ** -0.5,
+                                 plan=plan[:-8], max_chunks=chunks, max_rows=H // KV)
+
+
 @pytest.mark.parametrize("n_items,window,max_chunks,min_tiles", [
     (17, 0, 34, 4), (17, 0, 128, 4), (64, 0, 128, 4), (300, 777, 1024, 1), (513, 0, 4096, 2)])
 def test_attention_plan_lists_the_longest_chunks_first(ops, n_items, window, max_chunks, min_tiles):
