@@ -629,9 +629,14 @@ def attention_chunks_for(n_items: int, n_kv: int) -> int:
 
 
 def _plan_ordered(n_items: int, n_kv: int) -> bool:
-    """Whether the split kernel takes the chunks longest first: not for up to 16 items (the second list costs the plan 3 us, a
-    decode step of one request 0.5 % with it for nothing)."""
-    return n_items > 16
+    """Whether the split kernel takes the chunks longest first.  That pays where there are more workgroups than compute
+    units, of which the host knows that there are between ``n_items * n_kv`` and as many more as there are units; the
+    second list costs the plan 2 to 3 us a step.  Eight layers with the plan, 256 units, us without and with it, sequences of
+    100 to 2,400 keys: 8 kv heads, 17 / 24 / 32 / 48 / 64 / 100 sequences 240 / 266 / 356 / 457 / 618 / 850 and 205 / 265 / 323 /
+    423 / 545 / 803; 4 kv heads 144 / 186 / 238 / 297 / 339 / 482 and 147 / 164 / 201 / 257 / 317 / 436; 2 kv heads, 24 / 40 / 48 /
+    64 / 100 115 / 150 / 186 / 236 / 301 and 116 / 152 / 167 / 200 / 265: a third of the units is where it begins to pay.  All of
+    one length: level or up to 10 % less.  (Up to 16 items: a decode step of one request 0.5 % more for nothing.)"""
+    return n_items > 16 and 3 * n_items * n_kv > compute_units()
 
 
 def _plan_ints(lib, max_chunks: int, ordered: bool) -> int:
