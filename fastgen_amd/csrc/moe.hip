@@ -936,17 +936,16 @@ extern "C" int fg_moe_combine(const float* y, const float* weight, const void* p
 
 // The combine inside the norm that follows it: h[t] += plus[t] + sum_j weight[t][j] * y[t * top + j], out = norm(h) * w, the
 // same sums in the same order (the bits of the two kernels), for rows without identities and without a gate of plus.
-// Row r of the output is row rows[r] with `rows` (h stays as it is), else row r.  A workgroup a row, all of a row's loads
+// A workgroup a row, all of a row's loads
 // in flight before anything is added; bound by them (1897 tokens of 2048, top 4: 19.5 us, 5.4 TB/s, against 15.2 + 13.8 for
 // the kernels apart, whose sums went through memory; 12 tokens 5.4 against 4.8 + 4.6, and a launch less).
 template <class TP, class TA, class TW, int NIT>
 __global__ __launch_bounds__(256) void moe_combine_norm_kernel(
     const float* __restrict__ y, const float* __restrict__ weight, const TP* __restrict__ plus, int ldp, int n_plus,
     size_t plus_stride, int top, int dim, float* __restrict__ h, const TW* __restrict__ w, TA* __restrict__ out,
-    const int* __restrict__ rows, float eps) {
+    float eps) {
   __shared__ float red[16];
-  const int r = blockIdx.x;
-  const size_t t = rows ? (size_t)rows[r] : (size_t)r;
+  const size_t t = blockIdx.x;
   float* hrow = h + t * dim;
   int e[NIT], ec[NIT];  // a thread whose share lies behind the row reads its last 8 and stores nothing
 #pragma unroll
@@ -1003,14 +1002,14 @@ __global__ __launch_bounds__(256) void moe_combine_norm_kernel(
 #pragma unroll
     for (int i = 0; i < 8; ++i) v[it][i] += s[it][i];
     if (e[it] < dim) {
-      if (!rows) store8<float>(hrow + e[it], v[it]);
+      store8<float>(hrow + e[it], v[it]);
 #pragma unroll
       for (int i = 0; i < 8; ++i) ss += v[it][i] * v[it][i];
     }
   }
   ss = block_sum(ss, red);
   const float rstd = rsqrtf(ss / (float)dim + eps);
-  TA* orow = out + (size_t)r * dim;
+  TA* orow = out + t * dim;
 #pragma unroll
   for (int it = 0; it < NIT; ++it) {
     if (e[it] < dim) {
@@ -1024,7 +1023,7 @@ __global__ __launch_bounds__(256) void moe_combine_norm_kernel(
 
 extern "C" int fg_moe_combine_norm(const float* y, const float* weight, const void* plus, int ldp, int plus_dtype, int n_plus,
                                    long long plus_stride, int top, int dim, float* h, const void* w, int w_dtype,
-                                   void* out, int out_dtype, const int* rows, int n_rows, float eps, hipStream_t stream) {
+                                   void* out, int out_dtype, int n_rows, float eps, hipStream_t stream) {
   if (n_rows <= 0) return FG_OK;
   if (top <= 0 || dim <= 0 || dim % 8 || dim > 4096 || (plus && (ldp < dim || ldp % 8 || n_plus < 1 || plus_stride % 8)) ||
       (n_plus > 1 && plus_dtype != FG_F32))
@@ -1033,7 +1032,7 @@ extern "C" int fg_moe_combine_norm(const float* y, const float* weight, const vo
 #define GO_AS(TP, TA, TW, NIT)                                                                                          \
   moe_combine_norm_kernel<TP, TA, TW, NIT><<<n_rows, 256, 0, stream>>>(y, weight, (const TP*)plus, ldp, n_plus,         \
                                                                        (size_t)plus_stride, top, dim, h, (const TW*)w,  \
-                                                                       (TA*)out, rows, eps)
+                                                                       (TA*)out, eps)
 #define GO(TP, TA, TW)                        \
   do {                                        \
     if (dim <= 2048) GO_AS(TP, TA, TW, 1);    \

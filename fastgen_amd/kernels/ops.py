@@ -1531,22 +1531,19 @@ class ExpertSum:
     def add_norm(self, h: torch.Tensor, weight: torch.Tensor, eps: float, out: torch.Tensor,
                  rows: Optional[torch.Tensor] = None) -> torch.Tensor:
         """What :func:`add_rmsnorm` does with :meth:`total`, the same bits, in one kernel where it takes the sizes: rows
-        of up to 4,096 in eights, 16-byte aligned, in the types that a model's steps have."""
+        of up to 4,096 in eights, 16-byte aligned, in the types that a model's steps have, all of them (not ``rows``)."""
         plus, T, top, dim = self.plus, *self.weight.shape, self.y.shape[1]
         aligned = all(t is None or t.data_ptr() % 16 == 0 for t in (self.y, plus, h, weight, out))
         strides = plus is None or (plus.stride(-1) == 1 and plus.stride(-2) % 8 == 0 and (plus.dim() == 2 or plus.stride(0) % 8 == 0))
         types = out.dtype == torch.bfloat16 or (out.dtype == weight.dtype == torch.float32 and (plus is None or plus.dtype == torch.float32))
-        if dim % 8 or dim > EXPERT_SUM_MAX_DIM or not aligned or not strides or not types:
+        if rows is not None or dim % 8 or dim > EXPERT_SUM_MAX_DIM or not aligned or not strides or not types:
             return add_rmsnorm(h, self.total(), weight, eps, out, rows)
-        _gpu(self.y, self.weight, plus, h, weight, out, rows)
+        _gpu(self.y, self.weight, plus, h, weight, out)
         _need(self.y.dtype == torch.float32 and self.y.shape[0] == T * top and self.y.is_contiguous()
               and self.weight.dtype == torch.float32 and self.weight.is_contiguous(), "y float32 [T * top, dim], weight float32 [T, top]")
         _need(h.dtype == torch.float32 and h.shape == (T, dim) and h.is_contiguous(), "h must be contiguous float32 [T, dim]")
-        n_rows = T if rows is None else rows.numel()
-        if rows is not None:
-            _i32(rows, "rows")
         _need(weight.shape == (dim,) and weight.is_contiguous(), "weight must be [dim]")
-        _need(out.is_contiguous() and out.shape == (n_rows, dim), "out must be contiguous [rows, dim]")
+        _need(out.is_contiguous() and out.shape == (T, dim), "out must be contiguous [T, dim]")
         ldp, n_plus, stride = dim, 0, 0
         if plus is not None and plus.dim() == 3:
             _need(plus.dtype == torch.float32 and plus.shape[1:] == (T, dim), "partial sums must be float32 [S, T, dim]")
@@ -1556,7 +1553,7 @@ class ExpertSum:
             ldp, n_plus = plus.stride(0), 1
         st = _lib.load("moe").fg_moe_combine_norm(
             _ptr(self.y), _ptr(self.weight), _ptr(plus), ldp, _code(plus) if plus is not None else F32, n_plus,
-            ctypes.c_longlong(stride), top, dim, _ptr(h), _ptr(weight), _code(weight), _ptr(out), _code(out), _ptr(rows), n_rows,
+            ctypes.c_longlong(stride), top, dim, _ptr(h), _ptr(weight), _code(weight), _ptr(out), _code(out), T,
             ctypes.c_float(eps), _stream(out))
         _check(st, "moe_combine_norm")
         return out
