@@ -238,15 +238,17 @@ extern "C" int fg_moe_route_mode(const void* x, int ldx, int dtype, const float*
   moe_route_kernel<T, WAVES, EPW, TOK><<<(n_tokens + TOK - 1) / TOK, 64 * WAVES, TOK * lds, stream>>>(                 \
       (const T*)x, ldx, wr, bias, n_tokens, dim, n_experts, top, choice, weight, mode)
   // Tokens a workgroup: one while every token's workgroup has a place at once, then four, then eight, as their logits fit.
-  // Waves: 16 of two rows a turn, or 8 where the router has no more than 16 rows.  bf16, router in the caches, us, 32
+  // Waves: 16 of two rows a turn, or 8 where the router has no more than 16 rows, twice as many of which have a place.  bf16, router in the caches, us, 32
   // experts of 2048 with 4 waves of four rows before: 65 / 300 / 700 / 1024 / 1897 / 6000 tokens 6.6 / 9.8 / 10.2 / 11.1 / 13.9
   // / 36.5 against 10.0 / 10.7 / 12.4 / 15.6 / 17.0 / 38.3; 128 of 4096 25.7 / 41 / 48 / 55 / 74 / 206 against 49 / 52 / 61 / 74 /
-  // 100 / 274; 16 of 1024 4.2 / 5.7 / 5.8 / 5.9 / 7.3 / 14.1 against 5.1 / 5.3 / 5.8 / 7.4 / 7.8 / 15.0.
-  const int tok = n_tokens <= 256 || 4 * lds > 60000 ? 1 : n_tokens <= 1280 || 8 * lds > 60000 ? 4 : 8;
+  // 100 / 274; 16 of 1024 4.0 / 4.7 / 5.7 / 5.9 / 7.3 / 14.1 against 4.9 / 5.1 / 5.6 / 6.2 / 7.8 / 15.0 (512 tokens: one a
+  // workgroup 5.1, four 5.5; 700: both 5.7).
   const bool few_rows = n_experts + n_extra <= 16;
+  const int tok = n_tokens <= (few_rows ? 512 : 256) || 4 * lds > 60000 ? 1 : n_tokens <= 1280 || 8 * lds > 60000 ? 4 : 8;
 #define FORMS(T)                                                   \
   do {                                                             \
-    if (tok == 1) GO(T, 16, 2, 1);                                 \
+    if (tok == 1 && few_rows) GO(T, 8, 2, 1);                      \
+    else if (tok == 1) GO(T, 16, 2, 1);                            \
     else if (tok == 4 && few_rows) GO(T, 8, 2, 4);                 \
     else if (tok == 4) GO(T, 16, 2, 4);                            \
     else if (few_rows) GO(T, 8, 2, 8);                             \

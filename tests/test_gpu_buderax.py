@@ -467,13 +467,13 @@ def test_output_gate_inside_the_attention(hd, lens):
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("E,dim,extra", [(5, 40, 0), (16, 264, 0), (16, 512, 1), (33, 2048, 0), (130, 1000, 2)])
 def test_route_forms_give_the_same_bits(E, dim, extra, dtype):
-    """A token's experts and weights beside 1, 256, 257, 1280, 1281 tokens (workgroups of one token, four, eight; the last
-    ones partly filled)."""
+    """A token's experts and weights beside 1, 256, 257, 512, 513, 1280, 1281 tokens (workgroups of one token, four, eight;
+    the last ones partly filled)."""
     from fastgen_amd.kernels import ops
     torch.manual_seed(E + dim)
     x = torch.randn(1299, dim, device="cuda").to(dtype)
     router, bias = torch.randn(E + extra, dim, device="cuda"), torch.randn(E, device="cuda")
     whole = ops.moe_route(x, router, bias, 3, n_extra=extra)
-    for n in (1, 255, 256, 257, 1279, 1280, 1281):
+    for n in (1, 255, 256, 257, 511, 512, 513, 1279, 1280, 1281):
         for got, want in zip(ops.moe_route(x[:n], router, bias, 3, n_extra=extra), whole):
             assert torch.equal(got, want[:n])
