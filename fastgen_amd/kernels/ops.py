@@ -715,11 +715,13 @@ class AttentionParts:
 
 def attention_parts_fit(n_tokens: int, n_heads: int, head_dim: int, n_kv: int, max_keys: int) -> bool:
     """Whether a step's attention may be left as :class:`AttentionParts`: one token with at most ``max_keys`` keys, whose
-    parts every workgroup of the projection then reads (5 chunks of 12 KB for 24 heads at 1,024 keys).  One request through
-    28 layers of 24 heads with the merge inside the product and as a kernel of its own, us a step: 100 keys 1685 and 1726,
-    300 keys 1755 and 1788, 950 keys 1762 and 1793."""
-    return (n_tokens == 1 and max_keys <= MERGE_MAX_KEYS and -(-(max_keys // 64 + 1) // _SPLIT_MIN_TILES) <= MERGE_MAX_CHUNKS
-            and n_heads <= MERGE_MAX_HEADS and n_heads * head_dim <= MERGE_MAX_K and n_heads // n_kv <= 16
+    parts every workgroup of the projection then reads (5 chunks of 12 KB for 24 heads at 1,024 keys; with so few keys no
+    plan cuts more than ``MERGE_MAX_CHUNKS``).  One request through 28 layers of 24 heads with the merge inside the product
+    and as a kernel of its own, us a step: 100 keys 1685 and 1726, 300 keys 1755 and 1788, 950 keys 1762 and 1793.  Attention
+    and projection of a layer, us, at 100 / 500 / 1,024 keys, in heads x kv heads x head size: 24 x 8 x 128 13.5 / 16.1 / 16.3
+    and 15.1 / 17.4 / 17.5, 64 x 8 x 128 33.8 / 35.8 / 36.5 and 36.0 / 37.3 / 37.4, 128 x 8 x 64 33.0 / 34.6 / 34.8 and 35.3 / 35.5
+    / 35.6, 64 x 64 x 128 34.1 / 37.4 / 40.1 and 35.6 / 37.7 / 40.0: level at the widest, which is where the limits lie."""
+    return (n_tokens == 1 and max_keys <= MERGE_MAX_KEYS <= 64 * MERGE_MAX_CHUNKS and n_heads <= MERGE_MAX_HEADS and n_heads * head_dim <= MERGE_MAX_K and n_heads // n_kv <= 16
             and head_dim % 16 == 0 and head_dim <= MFMA_MAX_HEAD_DIM)
 
 
@@ -730,7 +732,7 @@ def paged_attention_mfma(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tens
                          min_tiles: int = 4, max_rows: int = 16, tile_rows: Optional[int] = None,
                          exact_weights: bool = False, sinks: Optional[torch.Tensor] = None,
                          distance: Optional[torch.Tensor] = None, gate: Optional[torch.Tensor] = None,
-                         gate_sigmoid: bool = True, leave_parts: bool = False) -> torch.Tensor:
+                         gate_sigmoid: bool = True, leave_parts: bool = False) -> "torch.Tensor | AttentionParts":
     """bf16 attention on the matrix cores.  ``small_items`` / ``big_items`` are
     device int32 ``[n, 4]`` lists from :func:`attention_items` (16-byte aligned);
     every query token of the step must be covered by exactly one item.
@@ -745,8 +747,9 @@ def paged_attention_mfma(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tens
     :func:`paged_attention_general` (a build of the kernels with exact weights takes the distance bias).  ``gate`` and
     ``gate_sigmoid``: what :func:`gate_mul` does with them behind the attention, done where the output is stored (the
     same bits), for bfloat16 rows that can be read in fours; else by that kernel.  ``leave_parts``: one token without a
-    gate comes as :class:`AttentionParts` (the caller has asked :func:`attention_parts_fit`)."""
-    leave_parts = leave_parts and gate is None and q.shape[0] == 1 and (big_items is None or not big_items.numel())
+    gate comes as :class:`AttentionParts` where :func:`attention_parts_fit` the cache's pages."""
+    leave_parts = (leave_parts and gate is None and (big_items is None or not big_items.numel()) and attention_parts_fit(
+        q.shape[0], n_heads, k_pages.shape[3], k_pages.shape[1], block_table.shape[1] * k_pages.shape[2]))
     _gpu(q, out, k_pages, v_pages, block_table, small_items, big_items, plan, sinks, distance, gate)
     if gate is not None and (gate.dtype != torch.bfloat16 or gate.data_ptr() % 8 or gate.stride(0) % 4):
         return gate_mul(paged_attention_mfma(q, out, k_pages, v_pages, block_table, small_items, big_items, n_heads, scale,
@@ -828,7 +831,7 @@ def paged_attention(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v
                     group, ctx, n_heads: int, scale: float, window: int = 0,
                     exact_weights: bool = False, sinks: Optional[torch.Tensor] = None,
                     distance: Optional[torch.Tensor] = None, gate: Optional[torch.Tensor] = None,
-                    gate_sigmoid: bool = True, leave_parts: bool = False) -> torch.Tensor:
+                    gate_sigmoid: bool = True, leave_parts: bool = False) -> "torch.Tensor | AttentionParts":
     """Attention for one step: picks the kernel for the step's dtype and shape.
     ``exact_weights``: see :func:`paged_attention_mfma` (the general kernel's weights are fp32 anyway).
     ``gate``, ``gate_sigmoid``: an output gate as :func:`gate_mul` takes it.  ``leave_parts``: the result may be
@@ -882,8 +885,7 @@ def paged_attention(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v
     return paged_attention_mfma(q, out, k_pages, v_pages, group.block_table, small_d, big_d, n_heads, scale,
                                 window, split_plan, chunks, max_rows=min(16, rows), tile_rows=tile_rows,
                                 exact_weights=exact_weights, sinks=sinks, distance=distance, gate=gate,
-                                gate_sigmoid=gate_sigmoid, leave_parts=leave_parts and attention_parts_fit(
-                                    q.shape[0], n_heads, hd, n_kv, group.block_table.shape[1] * k_pages.shape[2]))
+                                gate_sigmoid=gate_sigmoid, leave_parts=leave_parts)
 
 
 # ----------------------------------------------------------------------- gemm

@@ -1325,3 +1325,24 @@ def test_output_projection_merges_the_chunks_of_one_token(ops, H, KV, hd, n_keys
         assert ((h - want_h).abs() <= bound).all()
         if n_keys <= 256:
             assert torch.equal(h, want_h) and torch.equal(got.rows, want.rows) and torch.equal(got.ssq, want.ssq)
+
+
+@pytest.mark.parametrize("n_keys,min_tiles,left", [(1024, 1, True), (1025, 4, False), (6000, 4, False)])
+def test_parts_are_left_only_where_the_projection_takes_all_of_them(ops, n_keys, min_tiles, left):
+    """At the last key in as many chunks as a plan can cut (16), beyond it as the merged row, however many chunks."""
+    H, KV, hd, N = 6, 2, 64, 32
+    torch.manual_seed(n_keys)
+    case = _paged_case(torch.bfloat16, [(n_keys - 1, 1)], H, KV, hd, 16, seed=n_keys)
+    w, norm_w, h = torch.randn(N, H * hd).bfloat16().to(DEV), torch.randn(N).to(DEV), torch.randn(1, N).to(DEV)
+    items = torch.tensor([0, 0, 1, n_keys - 1], dtype=torch.int32, device=DEV)
+    plan = ops.attention_plan(items, 1, 40, hd, min_tiles=min_tiles)
+    run = lambda **kw: ops.paged_attention_mfma(case["q"], torch.empty_like(case["q"][:, : H * hd]), case["kp"], case["vp"], case["table"],
+                                                items, None, H, hd ** -0.5, plan=plan, max_chunks=40, max_rows=H // KV, **kw)
+    row, got = run(), run(leave_parts=True)
+    if left:
+        assert int(got.n_chunks[0]) == 16
+        want_h, h0 = h.clone(), h.clone()
+        got.project(w, h, norm_w, 1e-5), ops.gemm_skinny_residual(row, w, want_h, norm_w, 1e-5)
+        assert ((h - want_h).abs() <= 2.0 ** -8 * (row.double().abs() @ w.double().abs().T) + 1e-6 * h0.abs()).all()
+    else:
+        assert int(plan[10]) == -(-(-(-n_keys // 64)) // min_tiles) and torch.equal(got, row)
