@@ -212,32 +212,31 @@ def _winner(best: Dict[str, float], order: List[str]) -> str:
 
 
 def _choose(what: str, n: int, k: int, rows: int, candidates: List[Tuple[str, Callable[[], torch.Tensor]]],
-            handicap: Optional[Dict[str, float]] = None, order: Optional[List[str]] = None) -> str:
+            handicap: Optional[Dict[str, float]] = None, library_ties: bool = False) -> str:
     """The candidate to run: the forced one, the one the table holds, or, at the first calls, the fastest so far.
     Timing needs the device to itself (events and a wait for them), so a product that is first met while
     a step is being recorded runs the first candidate, unrecorded in the table; the engine runs every
     step once, unrecorded, before it records it.  The candidates are timed in turn on the same
     operands, each run behind a sweep of memory that empties the caches.  ``handicap``: milliseconds added to a candidate's time
-    for what its result costs the consumer (partial sums that are still to be added).  ``order``: who takes a tie
-    (default: the candidates' own order)."""
+    for what its result costs the consumer (partial sums that are still to be added).  ``library_ties``: the library
+    takes a tie, else the earlier candidate does."""
     names = [c[0] for c in candidates]
     if force in names:
         return force
     if len(candidates) == 1:
         return names[0]
     key = (what, n, k, row_bucket(rows))
-    got = choices.get(key)
-    seen = _samples.get(key, [])
-    settled = not seen or len(seen) >= _SAMPLES  # (a choice without samples was put there from outside)
-    if got in names and (settled or _capturing()):
+    got, seen = choices.get(key), _samples.get(key)
+    known = got in names
+    if known and (seen is None or len(seen) >= _SAMPLES):  # (a choice without samples was put there from outside)
         return got
     if _capturing():
-        return names[0]
-    if got not in names:
-        seen = []
+        return got if known else names[0]
+    seen = seen if known else []
+    order = sorted(names, key=lambda name: name != "library") if library_ties else names
     seen = seen + [_measure(candidates, handicap or {}, first=not seen)]
     timings[key] = {name: sum(t[name] for t in seen) / len(seen) for name in names}
-    choices[key] = _winner(timings[key], order or names)
+    choices[key] = _winner(timings[key], order)
     _samples[key] = seen
     return choices[key]
 
@@ -367,8 +366,5 @@ def linear(x, w, out_dtype: Optional[torch.dtype] = None,
         "+packed" if sw is not w else "")
     # Ties: the kernel with the epilogue in it, and with few rows the narrow one, both the least launches; a plain
     # product of more rows goes to the library, whose result is whole (no partial sums to add).
-    order = [c[0] for c in candidates]
-    if not silu and rows > SKINNY_ROWS:
-        order.sort(key=lambda name: name != "library")
-    name = _choose(what, N, K, rows, candidates, handicap, order)
+    name = _choose(what, N, K, rows, candidates, handicap, library_ties=not silu and rows > SKINNY_ROWS)
     return dict(candidates)[name]()

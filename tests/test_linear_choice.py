@@ -14,7 +14,7 @@ def ask(monkeypatch):
     recording = [False]
     monkeypatch.setattr(linear, "_capturing", lambda: recording[0])
 
-    def run(names, measured=None, capturing=False, order=None):
+    def run(names, measured=None, capturing=False, library_ties=False):
         recording[0] = capturing
 
         def measure(candidates, handicap, first):
@@ -22,7 +22,7 @@ def ask(monkeypatch):
             return dict(zip(names, measured))
 
         monkeypatch.setattr(linear, "_measure", measure)
-        return linear._choose("silu_mul", 28672, 4096, 64, [(n, None) for n in names], order=order)
+        return linear._choose("silu_mul", 28672, 4096, 64, [(n, None) for n in names], library_ties=library_ties)
 
     return run
 
@@ -40,7 +40,9 @@ def test_near_ties_go_to_the_same_kernel_in_every_process(ask, wide, library):
     """The times that different processes measured for one product: its kernel, and so its bits, must not depend on them."""
     for _ in range(4):
         assert ask(["wide", "library"], (wide, library)) == "wide"
-    assert linear._winner({"wide": library, "library": wide}, ["library", "wide"]) == "library"
+    linear.choices.clear(), linear._samples.clear()
+    for _ in range(4):
+        assert ask(["wide", "library"], (library, wide), library_ties=True) == "library"
 
 
 def test_a_lead_beyond_a_tie_decides_and_is_kept(ask):
