@@ -6,7 +6,9 @@
 // times the rate of v_mfma_f32_16x16x4_f32: every operand is the exact sum of
 // three bf16 parts of 8 bits each (h = bf16(v), m = bf16(v - h), l = v - h - m;
 // m and l scaled up, so that small operands keep all bits too), and a product of
-// two is six instructions: h h, then h m + m h, then h l + l h + m m.  m is up to
+// two is six instructions: h h, then h m + m h, then h l + l h + m m (Henry, Tang
+// and Heinecke, "Leveraging the bfloat16 artificial intelligence datatype for
+// higher-precision computations", ARITH 2019, name the split).  m is up to
 // 2^-8 of an operand's leading bit and l up to 2^-17, so the products left out
 // (m l, l m; l l) are at most 2^-24 of the whole, half a unit of its last place,
 // and of either sign.  Each of the three kinds is summed over the 32 k of an
@@ -269,9 +271,9 @@ __device__ __forceinline__ void gf_store4(float* __restrict__ y, int n, int N, b
   }
 }
 
-// 16 rows (decode, and outputs too few for tiles): bound by reading W.  A workgroup owns 16 outputs of 16 rows; a round is one group, a wave takes
-// one of its segments, so 64 KB of W (every wave's next segment) are in flight a workgroup while the current ones
-// are multiplied; the segments' sums meet in LDS and are added in order by one thread an output.  N x K 3072 x 3072 /
+// 16 rows (decode, and outputs too few for tiles): bound by reading W.  A workgroup owns 16 outputs of 16 rows; a round is
+// one group, a wave takes one of its segments, so 64 KB of W (every wave's next segment) are in flight a workgroup while
+// the current ones are multiplied; the segments' sums meet in LDS and are added in order by one thread an output.  N x K 3072 x 3072 /
 // 16384 x 3072 / 3072 x 8192: 14 / 46 / 33 us at 4 rows (4.4 TB/s of W at the largest), 18 / 56 / 41 at 16; with the fp32
 // instructions 14 / 48 / 33 and 17 / 60 / 41.
 // Two workgroups a compute unit (at most 128 registers): 441 workgroups of two groups 13 us, 15.7 with one.
