@@ -273,9 +273,9 @@ __device__ __forceinline__ void gf_store4(float* __restrict__ y, int n, int N, b
 
 // 16 rows (decode, and outputs too few for tiles): bound by reading W.  A workgroup owns 16 outputs of 16 rows; a round is
 // one group, a wave takes one of its segments, so 64 KB of W (every wave's next segment) are in flight a workgroup while
-// the current ones are multiplied; the segments' sums meet in LDS and are added in order by one thread an output.  N x K 3072 x 3072 /
-// 16384 x 3072 / 3072 x 8192: 14 / 46 / 33 us at 4 rows (4.4 TB/s of W at the largest), 18 / 56 / 41 at 16; with the fp32
-// instructions 14 / 48 / 33 and 17 / 60 / 41.
+// the current ones are multiplied; the segments' sums meet in LDS and are added in order by one thread an output.
+// N x K 3072 x 3072 / 16384 x 3072 / 3072 x 8192: 13 / 45 / 31 us at 4 rows (4.5 TB/s of W at the largest), 18 / 60 / 43 at
+// 16 (in tiles 25 / 54 / 32); with the fp32 instructions 14 / 47 / 31 and 18 / 60 / 40.
 // Two workgroups a compute unit (at most 128 registers): 441 workgroups of two groups 13 us, 15.7 with one.
 // A wave cuts its segment of x into parts once: with FEW (up to 8 rows), each number in one lane, through LDS into
 // the operands' order; above, every lane the operand it needs.
