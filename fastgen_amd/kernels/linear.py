@@ -163,15 +163,16 @@ def k_splits_for(n_out: int, k: int, rows: int = 0) -> int:
 choices: Dict[Tuple[str, int, int, int], str] = {}
 # the same keys -> what each candidate took when it was measured (milliseconds on average, the consumer's cost included)
 timings: Dict[Tuple[str, int, int, int], Dict[str, float]] = {}
-_samples: Dict[Tuple[str, int, int, int], List[Dict[str, float]]] = {}  # of the keys met so far, at most _SAMPLES each
+_samples: Dict[Tuple[str, int, int, int], List[Dict[str, float]]] = {}  # of the keys that are still measured
 # set to a candidate's name to take that kernel wherever it is among the candidates (tests run the
 # engine once under each name, so that every kernel that may be chosen is compared with the plain run)
 force: Optional[str] = None
 _TIMED_RUNS = 2  # of every candidate, each of the _SAMPLES times
 # How long a product takes depends on where its matrix happens to lie (64 rows of 28,672 x 4,096: the library's takes 49 to
 # 51 us on one layer's matrix and 59 to 63 on the next ones, in every process; the wide kernel 52 to 57 on all of them), so
-# the candidates are measured at the first calls that ask for a product, in a model one layer's matrix after the other.
-_SAMPLES = 3
+# the candidates are measured at the first calls that ask for a product, in a model one layer's matrix after the other; not
+# again where one of them leads by more than that.
+_SAMPLES, _CLEAR = 3, 0.25
 # A lead smaller than this decides nothing: the same program would take one kernel today and another tomorrow, and their
 # results differ by a rounding.
 _TIE = 0.04
@@ -228,17 +229,21 @@ def _choose(what: str, n: int, k: int, rows: int, candidates: List[Tuple[str, Ca
     key = (what, n, k, row_bucket(rows))
     got, seen = choices.get(key), _samples.get(key)
     known = got in names
-    if known and (seen is None or len(seen) >= _SAMPLES):  # (a choice without samples was put there from outside)
+    if known and seen is None:  # settled, or put there from outside
         return got
     if _capturing():
         return got if known else names[0]
-    seen = seen if known else []
+    seen = seen if known and seen else []
     order = sorted(names, key=lambda name: name != "library") if library_ties else names
     seen = seen + [_measure(candidates, handicap or {}, first=not seen)]
     timings[key] = {name: sum(t[name] for t in seen) / len(seen) for name in names}
-    choices[key] = _winner(timings[key], order)
-    _samples[key] = seen
-    return choices[key]
+    choices[key] = winner = _winner(timings[key], order)
+    clear = (1 + _CLEAR) * timings[key][winner]
+    if len(seen) < _SAMPLES and any(timings[key][name] <= clear for name in names if name != winner):
+        _samples[key] = seen
+    else:
+        _samples.pop(key, None)
+    return winner
 
 
 def _measure(candidates: List[Tuple[str, Callable[[], torch.Tensor]]], handicap: Dict[str, float],

@@ -47,8 +47,18 @@ def test_near_ties_go_to_the_same_kernel_in_every_process(ask, wide, library):
 
 def test_a_lead_beyond_a_tie_decides_and_is_kept(ask):
     for _ in range(3):
-        assert ask(["wide", "library"], (33.9, 19.8)) == "library"
-    assert ask(["wide", "library"]) == "library"
+        assert ask(["wide", "library"], (23.9, 19.8)) == "library"
+    assert ask(["wide", "library"]) == "library" and not linear._samples
+
+
+def test_a_clear_lead_is_not_measured_again(ask):
+    assert ask(["wide", "library", "tiled"], (33.9, 19.8, 26.0)) == "library"
+    assert ask(["wide", "library", "tiled"]) == "library" and not linear._samples
+    assert ask(["wide", "tiled"], (33.9, 26.0)) == "tiled"  # the winner is not among the candidates: from the start
+    assert ask(["wide", "tiled"]) == "tiled"
+
+
+def test_the_fastest_of_several_wins(ask):
     assert linear._winner({"library": 50.0, "wide": 34.0, "tiled": 34.5}, ["library", "wide", "tiled"]) == "wide"
 
 
