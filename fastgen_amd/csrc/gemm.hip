@@ -599,9 +599,10 @@ extern "C" int fg_gemm_f32(const float* x, const float* w, float* y, float* part
   }
   const GfCall c = {x, w, y, part, M, N, K, ldx, ldw, ldy, vec, stream};
   if (mb < 1 || mb > 7 || (nw == 4 && mb > 5) || (nw != 4 && nw != 8)) return FG_ERR_ARG;
-  // What a tile's rows span, of x and of a wave's 32 of W: any strides are taken, beyond 32 bits of bytes by the smallest
-  // tile (every cut gives the same bits).
-  const long long span = max((long long)(min(16 * mb, M) - 1) * ldx, (long long)(min(32, N) - 1) * ldw);
+  // What the rows that a tile loads span, of x (8 a wave at a time) and of a wave's 32 of W: any strides are taken, beyond 32
+  // bits of bytes by the smallest tile (every cut gives the same bits).
+  const int loaded = (16 * mb + 8 * nw - 1) / (8 * nw) * 8 * nw;
+  const long long span = max((long long)(min(loaded, M) - 1) * ldx, (long long)(min(32, N) - 1) * ldw);
   if (4 * (span + 32) > 0xffffffffLL) return gf_launch<1, 2, 8, true>(c);
 #define CASE(MB)                                          \
   if (mb == MB && nw == 8) return gf_launch<MB, 2, 8>(c); \
