@@ -35,6 +35,9 @@ HIPCC_FLAGS = [
 ]
 HEADERS = ["common.h", "kv_layout.h", "attention_static.h", "conv_inputs.h"]
 
+# headers of single sources
+OWN_HEADERS = {"gemm_large.hip": ("tile_product.h",), "moe.hip": ("tile_product.h",)}
+
 # library name -> source file
 LIBRARIES: Dict[str, str] = {
     "rows": "rows.hip",
@@ -43,6 +46,7 @@ LIBRARIES: Dict[str, str] = {
     "gemm": "gemm.hip",
     "gemm_skinny": "gemm_skinny.hip",
     "gemm_tiled": "gemm_tiled.hip",
+    "gemm_large": "gemm_large.hip",
     "sampling": "sampling.hip",
     "moe": "moe.hip",
     "heads": "heads.hip",
@@ -103,7 +107,7 @@ def _split_variant(name: str):
 def _source_hash(name: str) -> str:
     src, defines, _ = _split_variant(name)
     h = hashlib.sha256()
-    for f in [src, *HEADERS]:
+    for f in [src, *HEADERS, *OWN_HEADERS.get(src, ())]:
         h.update(f.encode())
         h.update((CSRC / f).read_bytes())
     h.update(" ".join(HIPCC_FLAGS + defines).encode())

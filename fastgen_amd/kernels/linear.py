@@ -3,7 +3,8 @@
 float32: the engine's own matrix-core kernels (``gemm.hip``), a true
 32-bit product whose rows do not depend on one another.  bfloat16: several
 kernels can take a product (the engine's weight-streaming MFMA kernels of
-``gemm_skinny.hip``, narrow and wide, with or without a cut of the k range, and
+``gemm_skinny.hip``, narrow and wide, with or without a cut of the k range, its
+large tiles of ``gemm_large.hip`` for prompts, and
 the vendor library's product through ``torch``, which the reference uses for
 all of them: cuBLAS through ``F.linear``, ``fastgen/forward.py:433-513``).
 Which one is the fastest depends on the matrix and on the number of rows, so
@@ -51,8 +52,19 @@ def _library_mm_f32_out(x: torch.Tensor, w: torch.Tensor) -> Optional[torch.Tens
 SKINNY_ROWS = 16  # one 16-row block of x: the narrow kernel (16 output columns a workgroup) and every folded epilogue
 WIDE_ROWS = ops.SKINNY_MAX_ROWS  # the wide kernel (64 columns a workgroup): up to eight blocks of x
 # the tiled kernel takes any number of rows; it is offered where it has been seen to win or come close (from the
-# wide kernel's range up to a few hundred rows; beyond, the library's large tiles are twice as fast)
+# wide kernel's range up to a few hundred rows; beyond, the library's large tiles are twice as fast), for a matrix without
+# a packed copy: with one the large tiles are never the slower ones (us at 192 rows, o and down of 4,096 x 4,096 and x 14,336:
+# 17 / 43 against 24 / 54)
 TILED_MIN_ROWS, TILED_MAX_ROWS = 65, 512
+# The large tiles (:func:`~fastgen_amd.kernels.ops.gemm_large`) take any number of rows of a packed matrix.  Up to this
+# many they are measured against the others, under the name of the tiled kernel; beyond, they run without being measured: of 132 products of 520 to 4,096 rows
+# (1,024 to 28,672 columns, 768 to 14,336 of k) they are faster than the library in 110, 1.17 times on average (gated
+# 1.09 to 1.5: the gate and up rows do not go through memory), and slower by up to 10 % where the library's tiles happen to fill the
+# chip (squares of 4,096).
+LARGE_MEASURED_ROWS = TILED_MAX_ROWS
+# Fewer rows than a tile has: where the output alone gives every compute unit a tile (gate and up of 28,672 x 4,096 at 64
+# rows 46 us against the wide kernel's 52; logits of 128,256 x 3,072 158 against the library's 192), else from 65 rows on.
+LARGE_MIN_ROWS = 65
 
 
 # ------------------------------------------------------- a weight, stored for its readers
@@ -336,7 +348,12 @@ def linear(x, w, out_dtype: Optional[torch.dtype] = None,
 
     candidates: List[Tuple[str, Callable[[], torch.Tensor]]] = []
     handicap: Dict[str, float] = {}
-    tiled_ok = own and TILED_MIN_ROWS <= rows <= TILED_MAX_ROWS
+    large_ok = (own and sw is not w and K % 64 == 0 and scaled is None and (not silu or (N % 16 == 0 and out_dtype == torch.bfloat16))
+                and ops.gemm_large_takes(x, N))
+    if large_ok and rows > LARGE_MEASURED_ROWS and force in (None, "tiled"):
+        tile, splits = ops.large_plan(rows, N, K, silu, partials_ok and out_dtype == torch.bfloat16)
+        return ops.gemm_large(x, sw, out_dtype, gated if silu else False, splits, tile)
+    tiled_ok = own and sw is w and TILED_MIN_ROWS <= rows <= TILED_MAX_ROWS
 
     def sums_cost(splits: int) -> float:
         """Milliseconds the consumer takes to read the partial sums beyond the first (at 4 TB/s)."""
@@ -364,6 +381,10 @@ def linear(x, w, out_dtype: Optional[torch.dtype] = None,
                 candidates.append((name, lambda tile_rows=tile_rows, s_t=s_t: ops.gemm_tiled(
                     x, sw, out_dtype, k_splits=s_t, tile_rows=tile_rows)))
                 handicap[name] = sums_cost(s_t)
+    if large_ok and rows > SKINNY_ROWS and (rows >= LARGE_MIN_ROWS or ((silu or out_dtype == torch.float32) and N >= 64 * ops.compute_units())):
+        tile, splits = ops.large_plan(rows, N, K, silu, partials_ok and out_dtype == torch.bfloat16)
+        candidates.append(("tiled", lambda: ops.gemm_large(x, sw, out_dtype, gated if silu else False, splits, tile)))
+        handicap["tiled"] = sums_cost(splits)
     if scaled is None or not candidates:
         candidates.append(("library", library))
     what = (epilogue if silu else "store") + ("+partials" if partials_ok and rows > SKINNY_ROWS else "") + (

@@ -1214,6 +1214,86 @@ def gemm_tiled(x: torch.Tensor, w, out_dtype: Optional[torch.dtype] = None,
     return y
 
 
+# rows and columns of x and of the output that a workgroup of gemm_large takes (1,000 * rows + columns)
+LARGE_TILES = (256256, 256192, 128256, 128192, 128128)
+# Microseconds that a tile takes on a compute unit of its own, for every 64 of k and beside them, and, of the tiles that fit
+# twice, two at a time.  Fitted to 1,600 products (130 to 4,096 rows, 1,024 to 28,672 columns, 768 to 14,336 of k, 1 to 4
+# splits); the plan that is the fastest by them takes 1.5 % longer on average than the fastest one.
+_LARGE_COST = {256256: (1.117, 7.7, 0.0, 0.0), 256192: (0.862, 9.0, 0.0, 0.0), 128256: (0.646, 7.0, 1.313, 13.3),
+               128192: (0.531, 5.9, 1.051, 10.8), 128128: (0.357, 6.0, 0.877, 7.0)}
+_LARGE_SPLITS = 4
+
+
+def large_cost(tile: int, M: int, N: int, K: int, splits: int = 1) -> float:
+    """About how long :func:`gemm_large` takes with a tile, in microseconds, and its consumer for the partial sums: rounds over the
+    compute units."""
+    one, rest, two, rest_two = _LARGE_COST[tile]
+    steps, units = -(-(K // 64) // splits), compute_units()
+    tiles = -(-M // (tile // 1000)) * -(-N // (tile % 1000)) * splits
+    sums = 1.0 + 1.5 * (4 * splits - 2) * M * N / 4e6 if splits > 1 else 0.0  # written and read at 4 TB/s, and half as much
+    if not two:
+        return -(-tiles // units) * (steps * one + rest) + sums
+    rounds, left = divmod(tiles, 2 * units)
+    last = 0.0 if not left else steps * one + rest if left <= units else steps * two + rest_two
+    return rounds * (steps * two + rest_two) + last + sums
+
+
+@functools.lru_cache(maxsize=4096)
+def large_plan(M: int, N: int, K: int, gated: bool = False, partials: bool = False) -> Tuple[int, int]:
+    """The tile that :func:`gemm_large` is fastest with, and, where its result may be partial sums, the splits of k: each of
+    512 at least, none empty, and no more workgroups than have a place at once."""
+    plans = [(t, 1) for t in LARGE_TILES if not gated or t % 1000 != 192]
+    if partials:
+        steps, places = K // 64, 2 * compute_units()
+        plans += [(t, s) for t in LARGE_TILES if _LARGE_COST[t][2] for s in range(2, _LARGE_SPLITS + 1)
+                  if steps // s >= 8 and -(-steps // s) * (s - 1) < steps
+                  and -(-M // (t // 1000)) * -(-N // (t % 1000)) * s <= places]
+    return min(plans, key=lambda p: large_cost(p[0], M, N, K, p[1]))
+
+
+def gemm_large_takes(x: torch.Tensor, N: int) -> bool:
+    """Whether offsets within a tile of :func:`gemm_large` fit 32 bits, and its tiles the grid."""
+    return (x.stride(0) >= x.shape[1] and 512 * x.stride(0) + 2 * x.shape[1] <= 4_000_000_000 and x.shape[1] <= 30_000_000
+            and -(-x.shape[0] // 128) * -(-N // 128) <= 1 << 27)
+
+
+def gemm_large_scratch(M: int, N: int) -> int:
+    """Bytes of the partial sums that :func:`gemm_large` writes at most for up to ``M`` rows as :func:`large_plan` plans it."""
+    return min(_LARGE_SPLITS * M * N * 4, 2 * compute_units() * 128 * 256 * 4)
+
+
+def gemm_large(x: torch.Tensor, w: "PackedWeight", out_dtype: Optional[torch.dtype] = None, silu_mul_epilogue: bool = False,
+               k_splits: int = 1, tile: Optional[int] = None) -> torch.Tensor:
+    """``x @ w.T`` for the many rows of a prompt, bf16 ``x [M, K]`` (``K`` a multiple of 64) and a packed ``w``, by the
+    engine's large tiles (``tile``: one of ``LARGE_TILES``, default the one that suits the sizes); with
+    ``silu_mul_epilogue`` as :func:`gemm_skinny`; with ``k_splits > 1`` fp32 ``[k_splits, M, N]`` partial sums over the k ranges
+    ``[s * ceil(K / 64 / k_splits) * 64, ...)``."""
+    _gpu(x)
+    _need(x.dtype == torch.bfloat16 and x.dim() == 2 and isinstance(w, PackedWeight), "gemm_large takes bfloat16 x [M, K], w packed")
+    M, K = x.shape
+    N = w.shape[0]
+    _need(M > 0 and K % 64 == 0 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.stride(0) >= K and x.data_ptr() % 16 == 0,
+          "K must be a multiple of 64, rows 16-byte aligned")
+    w_ptr, _ = _weight_args(w, K, "gemm_large")
+    out_dtype = out_dtype or torch.bfloat16
+    if silu_mul_epilogue:
+        _need(N % 16 == 0 and out_dtype == torch.bfloat16 and k_splits == 1,
+              "the gate/up epilogue needs N % 16 == 0, bf16 output and one split")
+    _need(1 <= k_splits <= 64 and -(-(K // 64) // k_splits) * (k_splits - 1) < K // 64, "a split of k would be empty")
+    if k_splits > 1:
+        out_dtype = torch.float32
+    if tile is None:
+        tile = large_plan(M, N, K, bool(silu_mul_epilogue))[0]
+    _need(tile in LARGE_TILES, f"tile must be one of {LARGE_TILES}")
+    cols = N // 2 if silu_mul_epilogue else N
+    y = torch.empty((k_splits, M, cols) if k_splits > 1 else (M, cols), dtype=out_dtype, device=x.device)
+    st = _lib.load("gemm_large").fg_gemm_large(
+        _ptr(x), x.stride(0), w_ptr, _ptr(y), cols, ctypes.c_longlong(M * cols), k_splits, M, N, K, _code(y),
+        _gated_code(silu_mul_epilogue), int(tile), _stream(x))
+    _check(st, "gemm_large")
+    return y
+
+
 def gemm_skinny_qkv(x, wqkv, table: Optional[torch.Tensor], slots: torch.Tensor,
                     k_pages: torch.Tensor, v_pages: torch.Tensor, n_heads: int, n_kv: int, head_dim: int,
                     rotary_dim: int, value_from_key: bool = False, gate: bool = False) -> torch.Tensor:

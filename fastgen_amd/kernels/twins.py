@@ -340,6 +340,20 @@ def gemm_skinny(x, w, out_dtype: Optional[torch.dtype] = None, silu_mul_epilogue
     return y.to(out_dtype or torch.bfloat16)
 
 
+def gemm_large(x: torch.Tensor, w, out_dtype: Optional[torch.dtype] = None, silu_mul_epilogue: bool = False,
+               k_splits: int = 1, tile: Optional[int] = None) -> torch.Tensor:
+    """``x @ w.T``; with ``silu_mul_epilogue`` as :func:`gemm_skinny`; with ``k_splits > 1`` fp32 ``[S, M, N]`` partial sums over
+    the k ranges ``[s * ceil(K / 64 / S) * 64, ...)``.  ``tile`` only picks a tile."""
+    xf, wf = x.float(), _matrix(w)
+    if k_splits > 1:
+        step = -(-(wf.shape[1] // 64) // k_splits) * 64
+        return torch.stack([xf[:, s * step : (s + 1) * step] @ wf[:, s * step : (s + 1) * step].T for s in range(k_splits)])
+    y = xf @ wf.T
+    if silu_mul_epilogue:
+        y = _gated(y, silu_mul_epilogue)
+    return y.to(out_dtype or torch.bfloat16)
+
+
 def gemm_tiled(x: torch.Tensor, w, out_dtype: Optional[torch.dtype] = None,
                silu_mul_epilogue: bool = False, k_splits: int = 1, tile_rows: int = 128) -> torch.Tensor:
     """``x @ w.T``; with ``silu_mul_epilogue`` as :func:`gemm_skinny`; with ``k_splits > 1`` fp32 ``[S, M, N]``

@@ -726,6 +726,58 @@ def test_products_of_few_columns_do_not_look_behind_their_operands(ops, K):
                 assert (got.cpu().double() - want).abs().max() <= 1e-4 * want.abs().max() + 1e-6
 
 
+@pytest.mark.parametrize("tile", [256256, 256192, 128256, 128192, 128128])
+@pytest.mark.parametrize("M,N,K,S", [(1, 8, 64, 1), (127, 272, 128, 1), (129, 515, 320, 2), (257, 1040, 704, 3), (513, 264, 1024, 4),
+                                     (2100, 2064, 192, 1)])
+def test_gemm_large(ops, tile, M, N, K, S):
+    """The large tiles at every shape: rows and columns beyond a tile, stages that are no multiple of a round of the loop, splits
+    of k whose last is shorter, rows of x apart from one another with NaN between and behind them."""
+    torch.manual_seed(M + N)
+    room = torch.full((M + 2, K + 64), float("nan"), dtype=torch.bfloat16)
+    room[:M, :K] = torch.randn(M, K)
+    w = (torch.randn(N, K) * K**-0.5).bfloat16()
+    want = room[:M, :K].double() @ w.double().T
+    x, pw = room.to(DEV)[:M, :K], ops.pack_weight(w.to(DEV))
+    y32 = ops.gemm_large(x, pw, torch.float32, tile=tile)
+    assert y32.dtype == torch.float32 and (y32.cpu().double() - want).abs().max() <= 1e-4 * want.abs().max() + 1e-6
+    # bfloat16 is the same sums, rounded once
+    assert torch.equal(ops.gemm_large(x, pw, tile=tile), y32.to(torch.bfloat16))
+    if S > 1:
+        got, step = ops.gemm_large(x, pw, k_splits=S, tile=tile), -(-(K // 64) // S) * 64
+        assert got.shape == (S, M, N) and got.dtype == torch.float32
+        for s in range(S):
+            part = room[:M, s * step:(s + 1) * step][:, :max(0, K - s * step)].double() @ w[:, s * step:(s + 1) * step].double().T
+            assert (got[s].cpu().double() - part).abs().max() <= 1e-4 * want.abs().max() + 1e-6
+    if N % 16 == 0 and tile % 1000 != 192:
+        F = N // 2
+        both = want.float()
+        for epilogue, act in ((True, torch.nn.functional.silu), ("gelu_tanh", lambda g: torch.nn.functional.gelu(g, approximate="tanh"))):
+            got = ops.gemm_large(x, pw, None, epilogue, tile=tile).cpu().float()
+            gate, up = both.view(M, -1, 2, 8)[:, :, 0].reshape(M, F), both.view(M, -1, 2, 8)[:, :, 1].reshape(M, F)
+            # (the result's rounding to bfloat16, 2^-9, and what the sums' 1e-4 becomes in the product of two)
+            assert (got - act(gate) * up).abs().max() <= 5e-3 * (act(gate) * up).abs().max() + 1e-3
+
+
+def test_gemm_large_plans_and_refusals(ops):
+    from fastgen_amd.kernels import KernelArgumentError
+
+    for M, N, K in [(65, 1024, 64), (513, 2048, 5632), (700, 4096, 14336), (1300, 3072, 8192), (8192, 512, 1024), (100, 48, 640)]:
+        for gated in (False, True):
+            for partials in (False, True):
+                tile, splits = ops.large_plan(M, N, K, gated, partials)
+                assert tile in ops.LARGE_TILES and (not gated or tile % 1000 != 192) and (splits == 1 or partials)
+                assert -(-(K // 64) // splits) * (splits - 1) < K // 64
+                assert splits == 1 or splits * M * N * 4 <= ops.gemm_large_scratch(M, N)
+    x, w = torch.zeros(70, 128, dtype=torch.bfloat16, device=DEV), torch.zeros(32, 128, dtype=torch.bfloat16, device=DEV)
+    pw = ops.pack_weight(w)
+    for bad in (lambda: ops.gemm_large(x, w), lambda: ops.gemm_large(x[:, :72], ops.pack_weight(w[:, :72].contiguous())),
+                lambda: ops.gemm_large(x.float(), pw), lambda: ops.gemm_large(x, pw, k_splits=3),
+                lambda: ops.gemm_large(x[:, ::2], ops.pack_weight(w[:, :64].contiguous())),
+                lambda: ops.gemm_large(x, pw, tile=128129)):
+        with pytest.raises(KernelArgumentError):
+            bad()
+
+
 @pytest.mark.parametrize("M,F,K", [(129, 328, 240), (256, 14336, 4096), (70, 8, 64)])
 def test_gemm_tiled_gate_up_epilogue(ops, M, F, K):
     torch.manual_seed(F)

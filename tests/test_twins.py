@@ -23,7 +23,7 @@ from plain_llama import plain_attention, plain_rmsnorm, plain_rope_interleaved, 
 # functions of ops that launch a kernel (the others plan work, build arguments or pick a kernel)
 KERNEL_OPS = ["embed", "add_rmsnorm", "rmsnorm", "silu_mul", "rope_table", "rope_kv_write", "paged_attention_general",
               "paged_attention_mfma", "paged_attention", "gemm_nt", "scale_rows", "gemm_skinny_residual", "gemm_skinny",
-              "gemm_skinny_qkv", "gemm_tiled", "sample", "logprob", "stream_add", "add_rows", "gate_mul", "moe_route",
+              "gemm_skinny_qkv", "gemm_tiled", "gemm_large", "sample", "logprob", "stream_add", "add_rows", "gate_mul", "moe_route",
               "moe_sort", "moe_gate_up", "moe_down", "moe_combine", "gelu_mul", "post_add_rmsnorm", "softcap",
               "heads_prepare", "head_linear", "head_norm_gate", "decay_scan", "gated_mul", "causal_conv", "selective_scan",
               "sigmoid_attention", "scale_logits", "head_diff_norm", "streams_spread", "streams_step", "conv_tail",
