@@ -20,15 +20,11 @@
 // The matrix-core kernels take the experts' matrices row by row or packed (ldw = 0): per expert blocks of 16 rows x
 // 32 k in operand order, [expert][ceil(rows / 16)][ceil(k / 32)][64 lanes][8], zeros behind the last row and k.  A
 // wave's load is then 1 KB of whole lines; from rows it is 16 halves of a line, and the other halves are asked for
-// again a step later.  A model keeps its experts packed and takes tiles of 16, 32 and 128 rows; matrices in rows and
-// tiles of 64 and 256 rows, nowhere the better ones, are there for callers of the products that hand them over so.
-#include "common.h"
+// again a step later.  A model keeps its experts packed; matrices in rows and tiles of 64 rows, nowhere the better ones, are
+// there for callers of the products that hand them over so.
+#include "tile_product.h"
 
 #include <type_traits>
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // ------------------------------------------------------------------- route
 // A workgroup one token, four or eight.  Logits: the WAVES waves take the experts in turns of EPW (a wave
@@ -714,11 +710,176 @@ static int launch_moe_tiled(const void* x, int ldx, const void* w0, const void* 
   return launch_moe_tiled_as<WM, 4, EPI>(x, ldx, w0, w1, ldw, y, ldy, sorted, tiles, max_tiles, top, N, K, fn, stream);
 }
 
+// The same with packed matrices and k in multiples of 64: tile_product.h, 256 columns of the matrix a workgroup.  A tile of up to 64,
+// of up to 128 rows is a product of that many, so an expert's last tile costs no more than it holds.  Bound by the matrices, which
+// reach a die once, and by what a tile takes beside its product (14 us: the launch, its first loads, its last stores).  2,048
+// tokens, 32 experts of 768 x 2048, top 4 (256 rows an expert; 201 and 101 MB of matrices, 48 + 24 GFLOP): 72 / 57 us with tiles of
+// 256 rows, 79 / 61 of 128, 85 / 71 in the kernel above; 1,024 tokens 59 / 38 against 78 / 51; 4,096 117 / 97 against 148 / 106; 130
+// tokens 40 / 22.5 against 47 / 26 with tiles of 32 rows and no LDS.
+template <int MB, int NB, int NST, int WS, bool ONE_WAVE, int EPI>
+__device__ __forceinline__ void moe_large_tile(bf16_t* lds, const bf16_t* x, unsigned x_bytes, int ldx, const bf16_t* w0,
+                                               const bf16_t* w1, void* y, int ldy, const int* sorted, const int4 tile, int ct,
+                                               int top, int N, int K, const GatedAct fn) {
+#ifdef __HIP_DEVICE_COMPILE__
+  typedef TileProduct<MB, NB, NST, WS, ONE_WAVE> Product;
+  constexpr int WAVE_N = EPI == MT_GATE_UP ? 8 * NB : 16 * NB;
+  const int lane = threadIdx.x % FG_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / FG_WAVE);
+  const int r16 = lane & 15, g = lane >> 4;
+  const int n_base = (ct * 4 + wave) * WAVE_N, blocks = (N + 15) / 16, block = n_base / 16;
+  TileOperands op;
+  op.x = EPI == MT_GATE_UP ? (const void*)x : (const void*)(x + (size_t)tile.y * ldx);
+  op.x_bytes = EPI == MT_GATE_UP ? x_bytes : 2u * (unsigned)((tile.z - 1) * ldx + K);
+  op.w_row = (unsigned)K * 32u;
+  const size_t at = ((size_t)tile.x * blocks + block) * op.w_row;
+  if constexpr (EPI == MT_GATE_UP) {
+    op.w[0] = (const char*)w0 + at;
+    op.w[1] = (const char*)w1 + at;
+    op.w_bytes[0] = op.w_bytes[1] = (unsigned)max(0, min(NB / 2, blocks - block)) * op.w_row;
+  } else {
+    op.w[0] = (const char*)w0 + at;
+    op.w[1] = (const char*)w0 + at + (size_t)Product::HALF * op.w_row;
+    op.w_bytes[0] = (unsigned)max(0, min(Product::HALF, blocks - block)) * op.w_row;
+    op.w_bytes[1] = (unsigned)max(0, min(NB - Product::HALF, blocks - block - Product::HALF)) * op.w_row;
+  }
+  unsigned xo[Product::XL];
+#pragma unroll
+  for (int j = 0; j < Product::XL; ++j) {
+    const int row = Product::row_of(wave, j, lane);
+    const int from = EPI == MT_GATE_UP ? sorted[tile.y + min(row, tile.z - 1)] / top : row;
+    xo[j] = row < tile.z ? 2u * (unsigned)from * (unsigned)ldx + Product::chunk_of(lane) : TP_NOWHERE;
+  }
+  f32x4 acc[MB][NB];
+  Product::run(lds, op, xo, wave, lane, 0, K / 64, K / 64, acc);
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb) {
+    const int ml = 16 * mb + r16;
+    const bool there = ml < tile.z;
+    const int pos = tile.y + ml;
+    if constexpr (EPI == MT_DOWN) {
+      float* row = (float*)y + (size_t)(there ? sorted[pos] : 0) * ldy;
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
+        const f32x4 sum = Product::sums(acc[mb][nb]);
+        const int n = n_base + 16 * nb + 4 * g;
+        if (there && n + 3 < N && (ldy & 3) == 0) {
+          *(f32x4*)(row + n) = sum;
+        } else if (there) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (n + i < N) row[n + i] = sum[i];
+        }
+      }
+    } else {
+#pragma unroll
+      for (int nb = 0; nb < NB / 2; ++nb) {
+        const f32x4 gate = Product::sums(acc[mb][nb]), up = Product::sums(acc[mb][nb + NB / 2]);
+        const int n = n_base + 16 * nb + 4 * g;
+        bf16x4 v;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = (__bf16)gated_act<true>(gate[i], up[i], fn);
+        if (there && n < N) *(bf16x4*)((bf16_t*)y + (size_t)pos * ldy + n) = v;  // (N is a multiple of 8)
+      }
+    }
+  }
+#endif
+}
+
+// What workgroup `place` of die `die` does: a tile (rows 0: nothing) and a block of columns.
+// Up to 64 tiles, which a wave sees at once: those of more than 128 rows come first and those of up to 64 last, so that no long one
+// begins when the others end.  An expert's tiles, in runs of up to MT_RUN, and one block of columns are one die's, whose L2 that part of the
+// matrix is read into once; runs and blocks of columns are dealt to the dies in turn, and a die's workgroups are counted
+// without gaps (with places left free a quarter of the compute units got all of the work: 77 us against 40 for 130 tokens).
+// More tiles: a run of any MT_RUN tiles and one block of columns, so that nobody looks for its tile through all of them.
+__device__ __forceinline__ int moe_lane(int v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
+__device__ __forceinline__ int4 moe_task(const int* tiles, int max_tiles, int cols, int die, int place, int& ct) {
+  if (max_tiles > FG_WAVE) {
+    const int run = place / MT_RUN * 8 + die, ti = run / cols * MT_RUN + place % MT_RUN;
+    ct = run % cols;
+    return ti < max_tiles ? *(const int4*)(tiles + 4 * (size_t)ti) : make_int4(0, 0, 0, 0);
+  }
+  const int lane = threadIdx.x % FG_WAVE;
+  const int4 tile = lane < max_tiles ? *(const int4*)(tiles + 4 * (size_t)lane) : make_int4(0, 0, 0, 0);
+  const bool there = tile.z > 0;
+  const uint64_t upto = (2ull << lane) - 1, below = upto >> 1;
+  const int before = __builtin_amdgcn_update_dpp(-1, tile.x, 0x138 /* wave_shr:1 */, 0xf, 0xf, false);
+  const uint64_t firsts = __ballot(there && tile.x != before) & upto;  // experts' first tiles
+  const int within = firsts ? lane - (63 - __clzll(firsts)) : 0;       // which of its expert's tiles
+  const int run = __popcll(__ballot(there && within % MT_RUN == 0) & upto) - 1;
+  const int col0 = (die - run * cols) & 7, each = cols / 8;  // this tile's blocks of columns on this die: col0, col0 + 8, ..
+  const bool one_more = col0 < cols % 8;
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    const bool in = there && (tile.z > 128 ? 0 : tile.z > 64 ? 1 : 2) == c;
+    const uint64_t all = __ballot(in), more = __ballot(in && one_more);
+    const int total = each * __popcll(all) + __popcll(more);
+    if (place < total) {
+      const int first = each * __popcll(all & below) + __popcll(more & below);
+      const int at = __builtin_ctzll(__ballot(in && place >= first && place < first + each + (one_more ? 1 : 0)));
+      ct = moe_lane(col0, at) + 8 * (place - moe_lane(first, at));
+      return make_int4(moe_lane(tile.x, at), moe_lane(tile.y, at), moe_lane(tile.z, at), 0);
+    }
+    place -= total;
+  }
+  ct = 0;
+  return make_int4(0, 0, 0, 0);
+}
+
+template <int MB, int NB, int NST, int WS, int OCC, int EPI>
+__global__ __launch_bounds__(256, OCC) void moe_large_kernel(const bf16_t* x, unsigned x_bytes, int ldx, const bf16_t* w0,
+                                                             const bf16_t* w1, void* y, int ldy, const int* sorted,
+                                                             const int* tiles, int max_tiles, int top, int N, int K, const GatedAct fn) {
+  constexpr int COLS = (EPI == MT_GATE_UP ? 32 : 64) * NB;
+  extern __shared__ __attribute__((aligned(16))) bf16_t large_lds[];
+  int ct;
+  int4 tile = moe_task(tiles, max_tiles, (N + COLS - 1) / COLS, blockIdx.x % 8, blockIdx.x / 8, ct);
+  if (tile.z <= 0) return;  // (the whole workgroup)
+  tile = make_int4(__builtin_amdgcn_readfirstlane(tile.x), __builtin_amdgcn_readfirstlane(tile.y), __builtin_amdgcn_readfirstlane(tile.z), 0);
+#define GO(ROWS) \
+  moe_large_tile<ROWS, NB, NST, WS, OCC == 1, EPI>(large_lds, x, x_bytes, ldx, w0, w1, y, ldy, sorted, tile, ct, top, N, K, fn)
+  if (tile.z <= 64) GO(4);
+  else if (MB == 8 || tile.z <= 128) GO(8);
+  else if constexpr (MB == 16) GO(16);
+#undef GO
+}
+
+template <int MB, int NB, int NST, int WS, int OCC, int EPI>
+static int launch_moe_large(const void* x, unsigned x_bytes, int ldx, const void* w0, const void* w1, void* y, int ldy,
+                            const int* sorted, const int* tiles, int max_tiles, int n_experts, int top, int N, int K,
+                            const GatedAct fn, hipStream_t stream) {
+  constexpr int COLS = (EPI == MT_GATE_UP ? 32 : 64) * NB, lds = NST * MB * 2048;
+  static_assert(OCC * lds <= 160 * 1024, "LDS of a compute unit");
+  // (every expert's last run may be a part of one)
+  const long long runs = (long long)(max_tiles / MT_RUN + (n_experts < max_tiles ? n_experts : max_tiles)) * ((N + COLS - 1) / COLS);
+  const long long grid = (runs + 7) / 8 * 8 * MT_RUN;
+  if (grid > 2147483647LL) return FG_ERR_ARG;
+  static uint64_t raised = 0;  // devices that were asked for more than 64 KB of dynamic LDS, a bit each (asking twice does no harm)
+  auto kernel = moe_large_kernel<MB, NB, NST, WS, OCC, EPI>;
+  int device = 0;
+  if (hipGetDevice(&device) != hipSuccess) return FG_ERR_LAUNCH;
+  if (device >= 64 || !(__atomic_load_n(&raised, __ATOMIC_RELAXED) >> device & 1)) {
+    if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return FG_ERR_LAUNCH;
+    if (device < 64) __atomic_fetch_or(&raised, (uint64_t)1 << device, __ATOMIC_RELAXED);
+  }
+  kernel<<<(unsigned)grid, 256, lds, stream>>>((const bf16_t*)x, x_bytes, ldx, (const bf16_t*)w0, (const bf16_t*)w1, y, ldy, sorted, tiles,
+                                               max_tiles, top, N, K, fn);
+  return fg_launch_status();
+}
+
+// Whether wide tiles would leave a third of the compute units without a workgroup (see launch_moe_tiled).
+static bool moe_few(int max_tiles, int N, int cols) { return (long long)max_tiles * ((N + cols - 1) / cols) < 170; }
+
+// Whether the large tiles take it: packed matrices, k in steps of 64, 32-bit offsets within the rows of x and 64 rows of a matrix.
+static bool moe_large_ok(const void* x, long long rows, int ldx, const void* w0, const void* w1, int ldw, int K, int tile_rows) {
+  return ldw == 0 && K % 64 == 0 && (tile_rows == 128 || tile_rows == 256) && rows > 0 && rows * ldx * 2 <= 4000000000LL &&
+         (long long)K * 128 <= 4000000000LL && !(((uintptr_t)x | (uintptr_t)w0 | (uintptr_t)w1) & 15);
+}
+
 // x [T, dim] rows gathered by token; wg, wu [E, hidden, ldw], act [n_pairs, lda] in the sorted order.
 // mfma: bf16 with dim % 8 == 0, ldx % 8 == 0, ldw % 8 == 0 (16-byte loads); tile_rows = 16 * MB, MB in 1, 2, 4,
 // or 128 / 256: the tiles that go through LDS.
 // act_kind, limit, alpha: the gated activation (GatedAct in common.h).
-extern "C" int fg_moe_gate_up_act(const void* x, int ldx, const void* wg, const void* wu, int ldw, const int* sorted,
+// n_tokens, n_experts: the rows of x and the experts that tiles may name (0: not known, no large tiles).
+extern "C" int fg_moe_gate_up_act(const void* x, int n_tokens, int n_experts, int ldx, const void* wg, const void* wu, int ldw, const int* sorted,
                                   const int* tiles, int max_tiles, int tile_rows, int top, int dim, int hidden, void* act,
                                   int lda, int dtype, int mfma, int act_kind, float limit, float alpha,
                                   hipStream_t stream) {
@@ -730,6 +891,15 @@ extern "C" int fg_moe_gate_up_act(const void* x, int ldx, const void* wg, const 
     if (dtype != FG_BF16 || dim % 8 || ldx % 8 || ldw % 8 || lda % 4) return FG_ERR_ARG;
     if (tile_rows == 128 || tile_rows == 256) {
       if (hidden % 8 || dim < 32) return FG_ERR_ARG;  // (a lane's stand-in load reads the row's first 32 k)
+      if (n_experts > 0 && moe_large_ok(x, n_tokens, ldx, wg, wu, ldw, dim, tile_rows)) {
+        const unsigned bytes = 2u * ((unsigned)(n_tokens - 1) * (unsigned)ldx + (unsigned)dim);
+#define GO(MB, NB, NST, WS, OCC) \
+  return launch_moe_large<MB, NB, NST, WS, OCC, MT_GATE_UP>(x, bytes, ldx, wg, wu, act, lda, sorted, tiles, max_tiles, n_experts, top, hidden, dim, fn, stream)
+        if (tile_rows == 256) GO(16, 4, 5, 8, 1);
+        if (moe_few(max_tiles, hidden, 128)) GO(8, 2, 5, 8, 2);
+        GO(8, 4, 5, 4, 2);
+#undef GO
+      }
       return tile_rows == 128
                  ? launch_moe_tiled<1, MT_GATE_UP>(x, ldx, wg, wu, ldw, act, lda, sorted, tiles, max_tiles, top, hidden, dim, fn, stream)
                  : launch_moe_tiled<2, MT_GATE_UP>(x, ldx, wg, wu, ldw, act, lda, sorted, tiles, max_tiles, top, hidden, dim, fn, stream);
@@ -770,12 +940,12 @@ extern "C" int fg_moe_gate_up_act(const void* x, int ldx, const void* wg, const 
 extern "C" int fg_moe_gate_up(const void* x, int ldx, const void* wg, const void* wu, int ldw, const int* sorted,
                               const int* tiles, int max_tiles, int tile_rows, int top, int dim, int hidden, void* act,
                               int lda, int dtype, int mfma, hipStream_t stream) {
-  return fg_moe_gate_up_act(x, ldx, wg, wu, ldw, sorted, tiles, max_tiles, tile_rows, top, dim, hidden, act, lda, dtype,
+  return fg_moe_gate_up_act(x, 0, 0, ldx, wg, wu, ldw, sorted, tiles, max_tiles, tile_rows, top, dim, hidden, act, lda, dtype,
                             mfma, FG_ACT_SILU, 0.f, 1.f, stream);
 }
 
 // act [n_pairs, lda] in the sorted order; wd [E, dim, ldw]; y fp32 [n_pairs, dim], row = pair.
-extern "C" int fg_moe_down(const void* act, int lda, const void* wd, int ldw, const int* sorted, const int* tiles,
+extern "C" int fg_moe_down(const void* act, int n_experts, int lda, const void* wd, int ldw, const int* sorted, const int* tiles,
                            int max_tiles, int tile_rows, int dim, int hidden, float* y, int dtype, int mfma,
                            hipStream_t stream) {
   if (max_tiles <= 0) return FG_OK;
@@ -783,6 +953,15 @@ extern "C" int fg_moe_down(const void* act, int lda, const void* wd, int ldw, co
   if (mfma) {
     if (dtype != FG_BF16 || hidden % 8 || lda % 8 || ldw % 8) return FG_ERR_ARG;
     if ((tile_rows == 128 || tile_rows == 256) && hidden < 32) return FG_ERR_ARG;
+    if (n_experts > 0 && moe_large_ok(act, tile_rows, lda, wd, nullptr, ldw, hidden, tile_rows)) {
+#define GO(MB, NB, NST, WS, OCC)                                                                                               \
+  return launch_moe_large<MB, NB, NST, WS, OCC, MT_DOWN>(act, 0, lda, wd, nullptr, y, dim, sorted, tiles, max_tiles, n_experts, 1, dim, hidden, \
+                                                         GatedAct{0, 0.f, 1.f}, stream)
+      if (tile_rows == 256) GO(16, 4, 5, 8, 1);
+      if (moe_few(max_tiles, dim, 256)) GO(8, 2, 5, 8, 2);
+      GO(8, 4, 5, 4, 2);
+#undef GO
+    }
     if (tile_rows == 128 || tile_rows == 256)
       return tile_rows == 128
                  ? launch_moe_tiled<1, MT_DOWN>(act, lda, wd, nullptr, ldw, y, dim, sorted, tiles, max_tiles, 1, dim, hidden, GatedAct{0, 0.f, 1.f}, stream)

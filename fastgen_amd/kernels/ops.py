@@ -1526,7 +1526,7 @@ def moe_gate_up(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, sorte
     _need(tile_rows in MOE_TILE_ROWS and (mfma or tile_rows == 16), "tile_rows does not fit the kernel")
     _need(mfma or ldw, "moe_gate_up: packed experts need sizes in multiples of 8")
     act = torch.empty((sorted_.numel(), hidden), dtype=x.dtype, device=x.device)
-    st = _lib.load("moe").fg_moe_gate_up_act(_ptr(x), x.stride(0), gate, up, ldw, _ptr(sorted_), _ptr(tiles),
+    st = _lib.load("moe").fg_moe_gate_up_act(_ptr(x), x.shape[0], w_gate.shape[0], x.stride(0), gate, up, ldw, _ptr(sorted_), _ptr(tiles),
                                              tiles.shape[0], tile_rows, top, dim, hidden, _ptr(act), hidden, _code(x),
                                              int(mfma), ACT_LIMITED if limit > 0 else 0, ctypes.c_float(limit),
                                              ctypes.c_float(alpha), _stream(x))
@@ -1550,7 +1550,7 @@ def moe_down(act: torch.Tensor, w_down: torch.Tensor, sorted_: torch.Tensor, til
     _need(tile_rows in MOE_TILE_ROWS and (mfma or tile_rows == 16), "tile_rows does not fit the kernel")
     _need(mfma or ldw, "moe_down: packed experts need sizes in multiples of 8, and act 16-byte aligned")
     y = torch.empty((act.shape[0], dim), dtype=torch.float32, device=act.device)
-    st = _lib.load("moe").fg_moe_down(_ptr(act), hidden, down, ldw, _ptr(sorted_), _ptr(tiles), tiles.shape[0],
+    st = _lib.load("moe").fg_moe_down(_ptr(act), w_down.shape[0], hidden, down, ldw, _ptr(sorted_), _ptr(tiles), tiles.shape[0],
                                       tile_rows, dim, hidden, _ptr(y), _code(act), int(mfma), _stream(act))
     _check(st, "moe_down")
     return y

@@ -37,17 +37,25 @@ from ..config.layout import PartSpec
 from .base import MATRIX, VECTOR, FeedForward, TensorSpec, build_part, place, register_part
 
 
-def expert_tile_rows(per_expert: float, least_k: int) -> int:
+def expert_tile_rows(per_expert: float, least_k: int, large: int = 0) -> int:
     """Rows of one expert a tile of the matrix-core kernels holds, by the rows an expert gets on average and the smaller
     of the two products' k: 16 for few rows (decode: an expert's matrices are read once for its rows), 32 and 128
     where the experts get so many rows each that their matrices would otherwise be read many times over; from 128 on
-    the rows of x go through LDS, k in steps of 32.  Measured (us, gate_up + down, packed, 32 experts of 768 x 2048, top 4;
-    tiles of 16 / 32 / 64 / 128 rows): 12 rows an expert 72 / 74 / 84 / -, 19: 95 / 81 / 91 / -, 25: 112 / 88 / 94 / 68,
-    50: 150 / 128 / 130 / 73, 237 (tiles of 256 rows 165): - / - / 434 / 153; 16 experts of 704 x 1024, top 2: 19: 37 / 28 /
-    31 / -, 25: 40 / 34 / 34 / 36, 50: 54 / 47 / 44 / 39."""
+    the rows of x go through LDS.  ``large``: where packed matrices have sizes in multiples of 64, the workgroups of 128 channels
+    that one tile of every expert makes; those go to the large tiles (``csrc/tile_product.h``), which take a tile of up to 64
+    and of up to 128 rows as one of that many, so 128 from 10 rows an expert on, and 256 while most experts then have one tile and
+    there are workgroups for most compute units.
+
+    Measured (us, gate_up + down, packed, 32 experts of 768 x 2048, top 4; tiles of 16 / 32 / 128 / 256 rows): 8 rows an
+    expert 63 / 66 / 64 / 68, 12: 67 / 68 / 64 / 67, 16: 84 / 73 / 64 / 67, 128: - / - / 101 / 98, 187: - / - / 107 / 107,
+    256: - / - / 140 / 128, 512: - / - / 220 / 214, 1,024: - / - / 393 / 416; 64 of 1,408 x 2048, top 6, 140: 343 / 307 (128 / 256),
+    768: 957 / 962; 16 of 704 x 1024, top 2 (96 workgroups), 8: 17.8 / 18.1 / 20.0 / 24.2, 12: 21.2 / 21.1 / 20.1 / 24.3, 128: 36 / 61
+    (128 / 256).  Other sizes (16 / 32 / 128): 12 rows an expert 72 / 74 / -, 19: 95 / 81 / -, 25: 112 / 88 / 68, 50: 150 / 128 / 73."""
+    if large and per_expert >= 10:
+        return 256 if 112 <= per_expert <= 640 and large >= 170 else 128
     if per_expert >= 24 and least_k >= 32:
         return 128
-    return 32 if per_expert >= 14 else 16
+    return 32 if per_expert >= 14 and not large else 16
 
 
 class MoE(FeedForward):
@@ -154,7 +162,9 @@ class MoE(FeedForward):
     def tile_rows(self, n_rows: int) -> int:
         if self.w_gate.dtype != torch.bfloat16 or self.dim % 8:
             return 16
-        return expert_tile_rows(n_rows * self.top / self.n_scored, min(self.dim, self.w_down.shape[2]))
+        hidden = self.w_down.shape[2]
+        large = self.n_experts * -(-hidden // 128) if self.dim % 64 == 0 and hidden % 64 == 0 else 0
+        return expert_tile_rows(n_rows * self.top / self.n_scored, min(self.dim, hidden), large)
 
     def forward(self, x: torch.Tensor, plus: Optional[torch.Tensor] = None, sums: bool = False):
         """fp32 ``[1, T, dim]``: the experts' weighted sum (plus ``plus``, rows that go to the

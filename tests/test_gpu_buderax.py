@@ -299,6 +299,28 @@ def test_command_lines(cases, tmp_path):
     assert chat.returncode == 0, chat.stderr[-2000:]
 
 
+@pytest.mark.parametrize("counts,D,F", [((0, 64, 65, 128, 129, 256, 300, 1, 513), 192, 72 * 8), ((700,), 64, 64), ((3,) * 70 + (260,), 128, 136 * 8),
+                                        ((1,) * 9, 320, 64)])
+@pytest.mark.parametrize("tile_rows", [128, 256])
+def test_large_tiles_of_experts_give_the_rows_bits(counts, D, F, tile_rows):
+    """Packed experts with sizes in multiples of 64 (the large tiles) against matrices stored row by row, where experts have as
+    many rows as a tile of 64, 128 or 256, one more, none, more than one tile, and where there are more than 64 tiles."""
+    from fastgen_amd.kernels import ops
+
+    E, T = len(counts), sum(counts)
+    torch.manual_seed(T)
+    x = torch.full((T, D + 8), float("nan"), device="cuda").bfloat16()[:, :D]  # (the rows lie apart, with NaN between)
+    x.copy_(torch.randn(T, D))
+    wg, wu = ((torch.randn(E, F, D, device="cuda") / D ** 0.5).bfloat16() for _ in range(2))
+    wd = (torch.randn(E, D, F, device="cuda") / F ** 0.5).bfloat16()
+    choice = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(T)].int()[:, None].cuda()
+    sorted_, tiles = ops.moe_sort(choice, E, tile_rows)
+    act = ops.moe_gate_up(x, wg, wu, sorted_, tiles, 1, tile_rows)
+    assert torch.equal(ops.moe_gate_up(x, ops.pack_experts(wg), ops.pack_experts(wu), sorted_, tiles, 1, tile_rows), act)
+    assert torch.equal(ops.moe_down(act, ops.pack_experts(wd), sorted_, tiles, tile_rows),
+                       ops.moe_down(act, wd, sorted_, tiles, tile_rows))
+
+
 @pytest.mark.parametrize("E,top,T,D,F", [(3, 2, 40, 40, 24), (5, 1, 700, 2048, 136), (4, 3, 300, 104, 520), (32, 4, 257, 64, 32)])
 @pytest.mark.parametrize("tile_rows", [16, 32, 64, 128, 256])
 def test_packed_experts_give_the_rows_bits(E, top, T, D, F, tile_rows):
