@@ -41,30 +41,19 @@ __device__ __forceinline__ uint32_t gl_pair(float a, float b) {
   return __builtin_bit_cast(uint32_t, p);
 }
 
-template <int MB, int NB, int NST, int WS, int OCC, int EPI, class TY>
-__global__ __launch_bounds__(256, OCC) void gemm_large_kernel(const bf16_t* x, int ldx, const bf16_t* w, TY* y,
-                                                                        int ldy, long long part_stride, int M, int N, int K,
-                                                                        int row_tiles, int col_tiles, int split_stages) {
+// A tile: 16 MB rows from m0 on, 64 NB columns from 64 NB ct on.
+template <int MB, int NB, int NST, int WS, bool ONE_WAVE, int EPI, class TY>
+__device__ __forceinline__ void gemm_large_tile(bf16_t* lds, const bf16_t* x, int ldx, const bf16_t* w, TY* y, int ldy, int M, int N,
+                                                int K, int m0, int ct, int first, int n_stages) {
 #ifdef __HIP_DEVICE_COMPILE__
-  typedef TileProduct<MB, NB, NST, WS, OCC == 1> Product;
-  extern __shared__ __attribute__((aligned(16))) bf16_t lds[];
-  // A die (blockIdx % 8) takes a run of tiles, by bands of 2,048 rows, in a band column after column: its compute units
-  // work on about as many rows of x as of W at a time, each of which its L2 reads once.
-  constexpr int BAND = 2048 / (16 * MB);
-  const int tiles = row_tiles * col_tiles, id = blockIdx.x % 8 * ((tiles + 7) / 8) + blockIdx.x / 8;
-  if (id >= tiles || (int)(blockIdx.x / 8) >= (tiles + 7) / 8) return;
-  const int band = id / (BAND * col_tiles), rows_here = min(BAND, row_tiles - band * BAND), at = id - band * BAND * col_tiles;
-  const int ct = at / rows_here, rt = band * BAND + at % rows_here;
+  typedef TileProduct<MB, NB, NST, WS, ONE_WAVE> Product;
   const int lane = threadIdx.x % FG_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / FG_WAVE);
   const int r16 = lane & 15, g = lane >> 4;
-  const int m0 = rt * 16 * MB, n0 = (ct * 4 + wave) * 16 * NB;
-  const int n_all = K / 64, first = blockIdx.y * split_stages, n_stages = min(split_stages, n_all - first);
-  y += blockIdx.y * part_stride;
-
+  const int n0 = (ct * 4 + wave) * 16 * NB;
   TileOperands op;
   op.x = x + (size_t)m0 * ldx;
   op.x_bytes = 2u * (unsigned)((min(16 * MB, M - m0) - 1) * ldx + K);
-  op.w_row = n_all * 2048u;
+  op.w_row = (unsigned)K * 32u;
   const int blocks = max(0, min(NB, (N + 15) / 16 - n0 / 16));  // of 16 rows of W that are there
   op.w[0] = (const char*)w + (size_t)(n0 / 16) * op.w_row;
   op.w[1] = (const char*)op.w[0] + (size_t)Product::HALF * op.w_row;
@@ -153,9 +142,42 @@ __global__ __launch_bounds__(256, OCC) void gemm_large_kernel(const bf16_t* x, i
 #endif
 }
 
+// Tiles of 256 rows: the first `whole` of them whole, the others in halves of 128 rows.  Where the last round of whole tiles would leave
+// half of the compute units without one or more, halves take half of its time: 2,048 x 28,672 x 4,096 (896 tiles, three rounds and
+// 128).
+template <int MB, int NB, int NST, int WS, int OCC, int EPI, class TY>
+__global__ __launch_bounds__(256, OCC) void gemm_large_kernel(const bf16_t* x, int ldx, const bf16_t* w, TY* y, int ldy,
+                                                              long long part_stride, int M, int N, int K, int row_tiles,
+                                                              int col_tiles, int whole, int split_stages) {
+  extern __shared__ __attribute__((aligned(16))) bf16_t large_lds[];
+  // A die (blockIdx % 8) takes a run of tiles, by bands of 2,048 rows, in a band column after column: its compute units
+  // work on about as many rows of x as of W at a time, each of which its L2 reads once.
+  constexpr int BAND = 2048 / (16 * MB);
+  const int tiles = row_tiles * col_tiles, die = blockIdx.x % 8, place = blockIdx.x / 8, each = (whole + 7) / 8;
+  int id = die * each + place, half = -1;
+  if (place >= each) {
+    const int halves = 2 * (tiles - whole), of_die = (halves + 7) / 8, h = die * of_die + place - each;
+    if (place - each >= of_die || h >= halves) return;
+    id = whole + h / 2;
+    half = h % 2;
+  } else if (id >= whole) {
+    return;
+  }
+  const int band = id / (BAND * col_tiles), rows_here = min(BAND, row_tiles - band * BAND), at = id - band * BAND * col_tiles;
+  const int ct = at / rows_here, m0 = (band * BAND + at % rows_here) * 16 * MB;
+  const int first = blockIdx.y * split_stages, n_stages = min(split_stages, K / 64 - first);
+  y += blockIdx.y * part_stride;
+  if (MB != 16 || half < 0) {
+    gemm_large_tile<MB, NB, NST, WS, OCC == 1, EPI, TY>(large_lds, x, ldx, w, y, ldy, M, N, K, m0, ct, first, n_stages);
+  } else if constexpr (MB == 16) {
+    if (m0 + 128 * half < M)
+      gemm_large_tile<8, NB, NST, WS, OCC == 1, EPI, TY>(large_lds, x, ldx, w, y, ldy, M, N, K, m0 + 128 * half, ct, first, n_stages);
+  }
+}
+
 template <int MB, int NB, int NST, int WS, int OCC, int EPI, class TY>
 static int launch_large(const void* x, int ldx, const void* w, void* y, int ldy, long long part_stride, int splits, int M, int N,
-                        int K, hipStream_t stream) {
+                        int K, int whole_tiles, hipStream_t stream) {
   constexpr int lds = NST * MB * 2048;
   static_assert(OCC * lds <= 160 * 1024, "LDS of a compute unit");
   static uint64_t raised = 0;  // devices that were asked for more than 64 KB of dynamic LDS, a bit each (asking twice does no harm)
@@ -169,18 +191,21 @@ static int launch_large(const void* x, int ldx, const void* w, void* y, int ldy,
   const long long rt = ((long long)M + 16 * MB - 1) / (16 * MB), ct = ((long long)N + 64 * NB - 1) / (64 * NB);
   if (rt * ct > 1 << 27) return FG_ERR_ARG;
   const int split_stages = (K / 64 + splits - 1) / splits;
-  kernel<<<dim3((unsigned)((rt * ct + 7) / 8 * 8), splits), 256, lds, stream>>>((const bf16_t*)x, ldx, (const bf16_t*)w, (TY*)y, ldy, part_stride,
-                                                                                M, N, K, (int)rt, (int)ct, split_stages);
+  const long long whole = whole_tiles > 0 && MB == 16 && whole_tiles < rt * ct ? whole_tiles : rt * ct;
+  const long long blocks = (whole + 7) / 8 * 8 + (2 * (rt * ct - whole) + 7) / 8 * 8;
+  kernel<<<dim3((unsigned)blocks, splits), 256, lds, stream>>>((const bf16_t*)x, ldx, (const bf16_t*)w, (TY*)y, ldy, part_stride, M, N, K,
+                                                               (int)rt, (int)ct, (int)whole, split_stages);
   return fg_launch_status();
 }
 
 // x [M, K] bf16 (K % 64 == 0, rows 16-byte aligned), w packed [N, K].  tile: 256256, 256192, 128256, 128192 or 128128 (rows and
 // columns of a workgroup's tile).  epilogue 0: y [M, N] of out_dtype (splits > 1: fp32 [splits, M, N], part_stride elements
 // apart, sums over ceil(K / 64 / splits) * 64 of k each; no split may be empty); 1 and 4: gate and up rows interleaved (N % 16 == 0), y [M, N / 2]
-// bf16, one split.
+// bf16, one split.  whole_tiles: 0, or of the tiles of 256 rows those that are not cut into halves (a multiple of 8).
 extern "C" int fg_gemm_large(const void* x, int ldx, const void* w, void* y, int ldy, long long part_stride, int splits, int M,
-                             int N, int K, int out_dtype, int epilogue, int tile, hipStream_t stream) {
+                             int N, int K, int out_dtype, int epilogue, int tile, int whole_tiles, hipStream_t stream) {
   if (M <= 0 || N <= 0) return FG_OK;
+  if (whole_tiles < 0 || whole_tiles % 8) return FG_ERR_ARG;
   if (K <= 0 || K % 64 || ldx % 8 || ldx < K || (((uintptr_t)x | (uintptr_t)w | (uintptr_t)y) & 15)) return FG_ERR_ARG;
   // offsets within a tile's rows, and within 16 x 4 packed rows, are 32-bit
   if ((long long)ldx * 512 + 2ll * K > 4000000000LL || (long long)K * 32 * 4 > 4000000000LL) return FG_ERR_ARG;
@@ -190,7 +215,7 @@ extern "C" int fg_gemm_large(const void* x, int ldx, const void* w, void* y, int
   if (EPI_IS_GATED(epilogue) ? (N % 16 || ldy < N / 2 || ldy % 8 || out_dtype != FG_BF16 || splits != 1) : (epilogue != EPI_STORE || ldy < N))
     return FG_ERR_ARG;
 #define GO(MB, NB, NST, WS, OCC, EPI, TY) \
-  return launch_large<MB, NB, NST, WS, OCC, EPI, TY>(x, ldx, w, y, ldy, part_stride, splits, M, N, K, stream)
+  return launch_large<MB, NB, NST, WS, OCC, EPI, TY>(x, ldx, w, y, ldy, part_stride, splits, M, N, K, whole_tiles, stream)
 #define STORE(...)                                                \
   do {                                                            \
     if (out_dtype == FG_BF16) GO(__VA_ARGS__, EPI_STORE, bf16_t); \

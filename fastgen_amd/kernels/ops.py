@@ -1216,26 +1216,42 @@ def gemm_tiled(x: torch.Tensor, w, out_dtype: Optional[torch.dtype] = None,
 
 # rows and columns of x and of the output that a workgroup of gemm_large takes (1,000 * rows + columns)
 LARGE_TILES = (256256, 256192, 128256, 128192, 128128)
-# Microseconds that a tile takes on a compute unit of its own, for every 64 of k and beside them, and, of the tiles that fit
-# twice, two at a time.  Fitted to 1,600 products (130 to 4,096 rows, 1,024 to 28,672 columns, 768 to 14,336 of k, 1 to 4
-# splits); the plan that is the fastest by them takes 1.5 % longer on average than the fastest one.
-_LARGE_COST = {256256: (1.117, 7.7, 0.0, 0.0), 256192: (0.862, 9.0, 0.0, 0.0), 128256: (0.646, 7.0, 1.313, 13.3),
-               128192: (0.531, 5.9, 1.051, 10.8), 128128: (0.357, 6.0, 0.877, 7.0)}
+# What a round of tiles takes, in microseconds: for every 64 of k, as much more for every 64 of k times the share of the
+# places that have a tile, and beside k.  First: one tile a compute unit; second: two (of the tiles that fit twice), or the halves
+# behind the last round.  Fitted to 1,739 products (130 to 4,096 rows, 1,024 to 28,672 columns, 768 to 14,336 of k, 1 to 4 splits) with
+# 3 to 9 % about them; the plan that is the fastest by them takes 0.6 % longer than the fastest one on average.  (8 us of the halves' rest
+# are added: in a model, 28 layers of other matrices between, 1,278 x 16,384 x 3,072 and 2,000 x 11,264 x 2,048 in halves made the
+# step 0.8 and 2 % longer than tiles of 128 rows, where they measured alike by themselves.)
+_LARGE_COST = {256256: ((0.936, 0.405, 8.3), (0.605, 0.24, 11.7)), 256192: ((0.723, 0.288, 9.6), (0.356, 0.265, 14.2)),
+               128256: ((0.468, 0.348, 7.0), (0.643, 0.865, 13.3)), 128192: ((0.385, 0.273, 5.9), (0.607, 0.591, 10.2)),
+               128128: ((0.296, 0.177, 4.3), (0.476, 0.459, 6.9))}
+_LARGE_GATED = 0.92  # of tiles that fit twice, against those that do not: one's activations run beside the other's products
 _LARGE_SPLITS = 4
 
 
-def large_cost(tile: int, M: int, N: int, K: int, splits: int = 1) -> float:
-    """About how long :func:`gemm_large` takes with a tile, in microseconds, and its consumer for the partial sums: rounds over the
-    compute units."""
-    one, rest, two, rest_two = _LARGE_COST[tile]
+def large_whole_tiles(tile: int, M: int, N: int) -> int:
+    """Of the tiles of 256 rows those that :func:`gemm_large` does not cut into halves of 128 rows: what is left behind their last
+    whole round, if that is at most half a round, is (0: all are whole)."""
+    units = compute_units()
+    rounds, left = divmod(-(-M // (tile // 1000)) * -(-N // (tile % 1000)), units)
+    return rounds * units if tile >= 256000 and rounds and 0 < 2 * left <= units and units % 8 == 0 else 0
+
+
+def large_cost(tile: int, M: int, N: int, K: int, splits: int = 1, gated: bool = False) -> float:
+    """About how long :func:`gemm_large` takes with a tile, in microseconds, and its consumer for the partial sums."""
+    one, two = _LARGE_COST[tile]
     steps, units = -(-(K // 64) // splits), compute_units()
     tiles = -(-M // (tile // 1000)) * -(-N // (tile % 1000)) * splits
+    took = lambda cost, fill: steps * (cost[0] + cost[1] * fill) + cost[2]
     sums = 1.0 + 1.5 * (4 * splits - 2) * M * N / 4e6 if splits > 1 else 0.0  # written and read at 4 TB/s, and half as much
-    if not two:
-        return -(-tiles // units) * (steps * one + rest) + sums
+    if tile >= 256000:
+        whole = large_whole_tiles(tile, M, N)
+        rounds, left = divmod(whole or tiles, units)
+        last = took(two, 2 * (tiles - whole) / units) if whole else took(one, left / units) if left else 0.0
+        return rounds * took(one, 1.0) + last + sums
     rounds, left = divmod(tiles, 2 * units)
-    last = 0.0 if not left else steps * one + rest if left <= units else steps * two + rest_two
-    return rounds * (steps * two + rest_two) + last + sums
+    last = 0.0 if not left else took(one, left / units) if left <= units else took(two, left / (2 * units))
+    return (rounds * took(two, 1.0) + last) * (_LARGE_GATED if gated else 1.0) + sums
 
 
 @functools.lru_cache(maxsize=4096)
@@ -1243,12 +1259,12 @@ def large_plan(M: int, N: int, K: int, gated: bool = False, partials: bool = Fal
     """The tile that :func:`gemm_large` is fastest with, and, where its result may be partial sums, the splits of k: each of
     512 at least, none empty, and no more workgroups than have a place at once."""
     plans = [(t, 1) for t in LARGE_TILES if not gated or t % 1000 != 192]
-    if partials:
+    if partials and not gated:
         steps, places = K // 64, 2 * compute_units()
-        plans += [(t, s) for t in LARGE_TILES if _LARGE_COST[t][2] for s in range(2, _LARGE_SPLITS + 1)
+        plans += [(t, s) for t in LARGE_TILES if t < 256000 for s in range(2, _LARGE_SPLITS + 1)
                   if steps // s >= 8 and -(-steps // s) * (s - 1) < steps
                   and -(-M // (t // 1000)) * -(-N // (t % 1000)) * s <= places]
-    return min(plans, key=lambda p: large_cost(p[0], M, N, K, p[1]))
+    return min(plans, key=lambda p: large_cost(p[0], M, N, K, p[1], gated))
 
 
 def gemm_large_takes(x: torch.Tensor, N: int) -> bool:
@@ -1289,7 +1305,7 @@ def gemm_large(x: torch.Tensor, w: "PackedWeight", out_dtype: Optional[torch.dty
     y = torch.empty((k_splits, M, cols) if k_splits > 1 else (M, cols), dtype=out_dtype, device=x.device)
     st = _lib.load("gemm_large").fg_gemm_large(
         _ptr(x), x.stride(0), w_ptr, _ptr(y), cols, ctypes.c_longlong(M * cols), k_splits, M, N, K, _code(y),
-        _gated_code(silu_mul_epilogue), int(tile), _stream(x))
+        _gated_code(silu_mul_epilogue), int(tile), large_whole_tiles(tile, M, N), _stream(x))
     _check(st, "gemm_large")
     return y
 

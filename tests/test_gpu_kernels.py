@@ -728,9 +728,9 @@ def test_products_of_few_columns_do_not_look_behind_their_operands(ops, K):
 
 @pytest.mark.parametrize("tile", [256256, 256192, 128256, 128192, 128128])
 @pytest.mark.parametrize("M,N,K,S", [(1, 8, 64, 1), (127, 272, 128, 1), (129, 515, 320, 2), (257, 1040, 704, 3), (513, 264, 1024, 4),
-                                     (2100, 2064, 192, 1)])
+                                     (2100, 2064, 192, 1), (2049, 8272, 128, 1)])
 def test_gemm_large(ops, tile, M, N, K, S):
-    """The large tiles at every shape: rows and columns beyond a tile, stages that are no multiple of a round of the loop, splits
+    """The large tiles at every shape: rows and columns beyond a tile, more than a round of tiles of 256 rows (the rest in halves), stages that are no multiple of a round of the loop, splits
     of k whose last is shorter, rows of x apart from one another with NaN between and behind them."""
     torch.manual_seed(M + N)
     room = torch.full((M + 2, K + 64), float("nan"), dtype=torch.bfloat16)
