@@ -154,6 +154,23 @@ def test_heads_prepare_kernel(dtype, H, G, d, e, hc, rot, P):
                 _close(torch.nan_to_num(got), torch.nan_to_num(want), dtype, "pages")
 
 
+@pytest.mark.parametrize("T,H,N,K,tail,pad", [(1, 2, 64, 128, 0, 0), (65, 3, 128, 160, 8, 8), (130, 1, 200, 264, 16, 24), (63, 2, 72, 40, 5, 3)])
+@pytest.mark.parametrize("out", [torch.bfloat16, torch.float32])
+def test_head_linear_stores_whole_lines_or_elements(T, H, N, K, tail, pad, out):
+    """Channels in whole blocks of 64, beyond them, rows of the output aligned to 16 bytes or not, columns copied behind them."""
+    from fastgen_amd.kernels import ops, twins
+
+    torch.manual_seed(N)
+    xs, ys = K + -(-tail // 8) * 8, N + tail + pad
+    x, w = torch.randn(T, H * xs).bfloat16(), (torch.randn(H, N, K) * K**-0.5).bfloat16()
+    yc, yg = torch.full((T, H * ys), 3.0).to(out), torch.full((T, H * ys), 3.0, device=DEV).to(out)
+    bias = torch.randn(H, N)
+    twins.head_linear(x, xs, w, yc, ys, tail, bias=bias)
+    ops.head_linear(x.to(DEV), xs, w.to(DEV), yg, ys, tail, bias=bias.to(DEV))
+    # products of K terms of about 1 in fp32 (1e-5), and one rounding to bfloat16 (2^-9 of values up to 8)
+    assert (yg.cpu().float() - yc.float()).abs().max() <= (2e-2 if out == torch.bfloat16 else 1e-4)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("T,H,N,K,tail,pad", [(5, 3, 7, 6, 2, 3), (70, 6, 128, 32, 32, 0), (130, 2, 40, 136, 0, 8),
                                               (1, 16, 24, 48, 8, 0), (9, 1, 200, 1024, 0, 0)])
