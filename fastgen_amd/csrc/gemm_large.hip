@@ -3,6 +3,11 @@
 // takes, and what becomes of the sums: bf16 or fp32 rows, or silu(gate) * up of a matrix whose rows are gate and up
 // interleaved in groups of 8 (the tanh form of GELU in SiLU's place), so that the gate/up rows never go through memory.
 //
+// Up to 64 rows (a batch that decodes) it is bound by reading W, and what the tile brings is how W is read: a wave 1 KB at a time in whole
+// lines, seven steps of 32 k ahead, and no barrier between W and the products.  28,672 x 4,096 with its activation at 64 rows 44.5 us = 5.3 TB/s
+// (the wide kernel of gemm_skinny.hip 51), 4,096 x 14,336 in eight splits with the sums read back 26.3 (32), 4,096 x 4,096 12.1 (13.7),
+// 3,072 x 8,192 15.7 (19.1), 2,048 x 2,048 6.6 (9.8).
+//
 // Where the tiles are few and k long, k is cut over workgroups (blockIdx.y) into fp32 partial sums that the norm kernel behind
 // adds in order.  Sums run over k in ascending order (within a split), whatever the batch holds.
 #include "tile_product.h"
@@ -198,7 +203,7 @@ static int launch_large(const void* x, int ldx, const void* w, void* y, int ldy,
   return fg_launch_status();
 }
 
-// x [M, K] bf16 (K % 64 == 0, rows 16-byte aligned), w packed [N, K].  tile: 256256, 256192, 128256, 128192 or 128128 (rows and
+// x [M, K] bf16 (K % 64 == 0, rows 16-byte aligned), w packed [N, K].  tile: 256256, 256192, 128256, 128192, 128128 or 64128 (rows and
 // columns of a workgroup's tile).  epilogue 0: y [M, N] of out_dtype (splits > 1: fp32 [splits, M, N], part_stride elements
 // apart, sums over ceil(K / 64 / splits) * 64 of k each; no split may be empty); 1 and 4: gate and up rows interleaved (N % 16 == 0), y [M, N / 2]
 // bf16, one split.  whole_tiles: 0, or of the tiles of 256 rows those that are not cut into halves (a multiple of 8).
@@ -231,6 +236,7 @@ extern "C" int fg_gemm_large(const void* x, int ldx, const void* w, void* y, int
     case 256256: PICK(16, 4, 5, 4, 1);
     case 128256: PICK(8, 4, 5, 4, 2);
     case 128128: PICK(8, 2, 5, 8, 2);
+    case 64128: PICK(4, 2, 5, 8, 3);
     case 256192: if (epilogue == EPI_STORE) STORE(16, 3, 5, 4, 1); return FG_ERR_ARG;
     case 128192: if (epilogue == EPI_STORE) STORE(8, 3, 5, 4, 2); return FG_ERR_ARG;
   }

@@ -52,19 +52,21 @@ def _library_mm_f32_out(x: torch.Tensor, w: torch.Tensor) -> Optional[torch.Tens
 SKINNY_ROWS = 16  # one 16-row block of x: the narrow kernel (16 output columns a workgroup) and every folded epilogue
 WIDE_ROWS = ops.SKINNY_MAX_ROWS  # the wide kernel (64 columns a workgroup): up to eight blocks of x
 # the tiled kernel takes any number of rows; it is offered where it has been seen to win or come close (from the
-# wide kernel's range up to a few hundred rows; beyond, the library's large tiles are twice as fast), for a matrix without
-# a packed copy: with one the large tiles are never the slower ones (us at 192 rows, o and down of 4,096 x 4,096 and x 14,336:
-# 17 / 43 against 24 / 54)
+# wide kernel's range up to a few hundred rows; beyond, the library's large tiles are twice as fast), where the large tiles below do
+# not take the matrix (us at 192 rows, o and down of 4,096 x 4,096 and x 14,336: 24 / 54 against 17 / 43)
 TILED_MIN_ROWS, TILED_MAX_ROWS = 65, 512
-# The large tiles (:func:`~fastgen_amd.kernels.ops.gemm_large`) take any number of rows of a packed matrix.  Up to this
-# many they are measured against the others, under the name of the tiled kernel; beyond, they run without being measured: of 132 products of 520 to 4,096 rows
-# (1,024 to 28,672 columns, 768 to 14,336 of k) they are faster than the library in 110, 1.17 times on average (gated
-# 1.09 to 1.5: the gate and up rows do not go through memory), and slower by up to 10 % where the library's tiles happen to fill the
-# chip (squares of 4,096).
-LARGE_MEASURED_ROWS = TILED_MAX_ROWS
-# Fewer rows than a tile has: where the output alone gives every compute unit a tile (gate and up of 28,672 x 4,096 at 64
-# rows 46 us against the wide kernel's 52; logits of 128,256 x 3,072 158 against the library's 192), else from 65 rows on.
-LARGE_MIN_ROWS = 65
+# The large tiles (:func:`~fastgen_amd.kernels.ops.gemm_large`) take any number of rows of a packed matrix and run without being
+# measured, so that a first step takes no longer and every process takes the same kernel, where they are the faster ones (us):
+# * beyond this many rows: of 130 products of 520 to 4,096 rows (1,024 to 28,672 columns, 768 to 14,336 of k) in 110, 1.2 times on
+#   average (gated 1.04 to 1.6: the gate and up rows do not go through memory), and slower by up to 10 % where the library's tiles happen
+#   to fill the chip (squares of 4,096);
+# * from 17 rows on gated products (28,672 x 4,096 at 64 rows 44.5 against 51 of the wide kernel and 55 of the library; 16,384 x 3,072
+#   at 17 to 128 rows 23 to 34 against 24 to 31, at 160 to 512 29 to 47 against 35 to 61), products that may leave partial sums (4,096 x
+#   14,336 at 17 / 64 / 192 rows 23.1 / 26.3 / 43 against 23.5 / 32 / 54; 2,048 x 2,048 at 256 10.6 against 9.9 is where it is not so), and
+#   wide fp32 outputs (logits of 128,256 x 4,096 at 64 rows 218 against 224).
+# A plain product of fewer rows has no splits to fill the chip with and goes the other ways (6,144 x 4,096 at 65 rows 34 against
+# 23 of the library, at 320 36 against 30).
+LARGE_ROWS = TILED_MAX_ROWS
 
 
 # ------------------------------------------------------- a weight, stored for its readers
@@ -350,10 +352,12 @@ def linear(x, w, out_dtype: Optional[torch.dtype] = None,
     handicap: Dict[str, float] = {}
     large_ok = (own and sw is not w and K % 64 == 0 and scaled is None and (not silu or (N % 16 == 0 and out_dtype == torch.bfloat16))
                 and ops.gemm_large_takes(x, N))
-    if large_ok and rows > LARGE_MEASURED_ROWS and force in (None, "tiled"):
-        tile, splits = ops.large_plan(rows, N, K, silu, partials_ok and out_dtype == torch.bfloat16)
-        return ops.gemm_large(x, sw, out_dtype, gated if silu else False, splits, tile)
-    tiled_ok = own and sw is w and TILED_MIN_ROWS <= rows <= TILED_MAX_ROWS
+    if large_ok and rows > SKINNY_ROWS and force in (None, "tiled") and (
+            rows > LARGE_ROWS or silu or (partials_ok and out_dtype == torch.bfloat16)
+            or (out_dtype == torch.float32 and N >= 64 * ops.compute_units())):
+        tile, l_splits = ops.large_plan(rows, N, K, silu, partials_ok and out_dtype == torch.bfloat16)
+        return ops.gemm_large(x, sw, out_dtype, gated if silu else False, l_splits, tile)
+    tiled_ok = own and not large_ok and TILED_MIN_ROWS <= rows <= TILED_MAX_ROWS
 
     def sums_cost(splits: int) -> float:
         """Milliseconds the consumer takes to read the partial sums beyond the first (at 4 TB/s)."""
@@ -381,10 +385,6 @@ def linear(x, w, out_dtype: Optional[torch.dtype] = None,
                 candidates.append((name, lambda tile_rows=tile_rows, s_t=s_t: ops.gemm_tiled(
                     x, sw, out_dtype, k_splits=s_t, tile_rows=tile_rows)))
                 handicap[name] = sums_cost(s_t)
-    if large_ok and rows > SKINNY_ROWS and (rows >= LARGE_MIN_ROWS or ((silu or out_dtype == torch.float32) and N >= 64 * ops.compute_units())):
-        tile, splits = ops.large_plan(rows, N, K, silu, partials_ok and out_dtype == torch.bfloat16)
-        candidates.append(("tiled", lambda: ops.gemm_large(x, sw, out_dtype, gated if silu else False, splits, tile)))
-        handicap["tiled"] = sums_cost(splits)
     if scaled is None or not candidates:
         candidates.append(("library", library))
     what = (epilogue if silu else "store") + ("+partials" if partials_ok and rows > SKINNY_ROWS else "") + (

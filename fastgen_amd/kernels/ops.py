@@ -1215,7 +1215,7 @@ def gemm_tiled(x: torch.Tensor, w, out_dtype: Optional[torch.dtype] = None,
 
 
 # rows and columns of x and of the output that a workgroup of gemm_large takes (1,000 * rows + columns)
-LARGE_TILES = (256256, 256192, 128256, 128192, 128128)
+LARGE_TILES = (256256, 256192, 128256, 128192, 128128, 64128)
 # What a round of tiles takes, in microseconds: for every 64 of k, as much more for every 64 of k times the share of the
 # places that have a tile, and beside k.  First: one tile a compute unit; second: two (of the tiles that fit twice), or the halves
 # behind the last round.  Fitted to 1,739 products (130 to 4,096 rows, 1,024 to 28,672 columns, 768 to 14,336 of k, 1 to 4 splits) with
@@ -1226,7 +1226,7 @@ _LARGE_COST = {256256: ((0.936, 0.405, 8.3), (0.605, 0.24, 11.7)), 256192: ((0.7
                128256: ((0.468, 0.348, 7.0), (0.643, 0.865, 13.3)), 128192: ((0.385, 0.273, 5.9), (0.607, 0.591, 10.2)),
                128128: ((0.296, 0.177, 4.3), (0.476, 0.459, 6.9))}
 _LARGE_GATED = 0.92  # of tiles that fit twice, against those that do not: one's activations run beside the other's products
-_LARGE_SPLITS = 4
+_LARGE_SPLITS = 8
 
 
 def large_whole_tiles(tile: int, M: int, N: int) -> int:
@@ -1257,13 +1257,15 @@ def large_cost(tile: int, M: int, N: int, K: int, splits: int = 1, gated: bool =
 @functools.lru_cache(maxsize=4096)
 def large_plan(M: int, N: int, K: int, gated: bool = False, partials: bool = False) -> Tuple[int, int]:
     """The tile that :func:`gemm_large` is fastest with, and, where its result may be partial sums, the splits of k: each of
-    512 at least, none empty, and no more workgroups than have a place at once."""
-    plans = [(t, 1) for t in LARGE_TILES if not gated or t % 1000 != 192]
-    if partials and not gated:
-        steps, places = K // 64, 2 * compute_units()
-        plans += [(t, s) for t in LARGE_TILES if t < 256000 for s in range(2, _LARGE_SPLITS + 1)
-                  if steps // s >= 8 and -(-steps // s) * (s - 1) < steps
-                  and -(-M // (t // 1000)) * -(-N // (t % 1000)) * s <= places]
+    512 at least, none empty, and no more workgroups than have a place at once.  Up to 64 rows the tile of as many, and as many splits up
+    to 8 as there may be (us at 64 rows with 4 and 8, the sums read back: 4,096 x 14,336 30 / 26.3, 4,096 x 4,096 12.8 / 12.1; with 16 31.3)."""
+    steps, places = K // 64, 2 * compute_units()
+    may = [s for s in (2, 3, 4, 6, 8) if partials and not gated and steps // s >= 8 and -(-steps // s) * (s - 1) < steps]
+    fits = lambda t, s: -(-M // (t // 1000)) * -(-N // (t % 1000)) * s <= places
+    if M <= 64:
+        return 64128, max((s for s in may if s in (2, 4, 8) and fits(64128, s)), default=1)
+    plans = [(t, 1) for t in _LARGE_COST if not gated or t % 1000 != 192]
+    plans += [(t, s) for t in _LARGE_COST if t < 256000 for s in may if fits(t, s)]
     return min(plans, key=lambda p: large_cost(p[0], M, N, K, p[1], gated))
 
 

@@ -726,7 +726,7 @@ def test_products_of_few_columns_do_not_look_behind_their_operands(ops, K):
                 assert (got.cpu().double() - want).abs().max() <= 1e-4 * want.abs().max() + 1e-6
 
 
-@pytest.mark.parametrize("tile", [256256, 256192, 128256, 128192, 128128])
+@pytest.mark.parametrize("tile", [256256, 256192, 128256, 128192, 128128, 64128])
 @pytest.mark.parametrize("M,N,K,S", [(1, 8, 64, 1), (127, 272, 128, 1), (129, 515, 320, 2), (257, 1040, 704, 3), (513, 264, 1024, 4),
                                      (2100, 2064, 192, 1), (2049, 8272, 128, 1)])
 def test_gemm_large(ops, tile, M, N, K, S):
@@ -761,7 +761,7 @@ def test_gemm_large(ops, tile, M, N, K, S):
 def test_gemm_large_plans_and_refusals(ops):
     from fastgen_amd.kernels import KernelArgumentError
 
-    for M, N, K in [(65, 1024, 64), (513, 2048, 5632), (700, 4096, 14336), (1300, 3072, 8192), (8192, 512, 1024), (100, 48, 640)]:
+    for M, N, K in [(17, 4096, 14336), (64, 48, 192), (65, 1024, 64), (513, 2048, 5632), (700, 4096, 14336), (1300, 3072, 8192), (8192, 512, 1024), (100, 48, 640)]:
         for gated in (False, True):
             for partials in (False, True):
                 tile, splits = ops.large_plan(M, N, K, gated, partials)
