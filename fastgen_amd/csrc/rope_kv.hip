@@ -195,3 +195,81 @@ extern "C" int fg_rope_kv_write(void* qkv, int row_stride, const int* positions,
 #undef LAUNCH
   return fg_launch_status();
 }
+
+// The same from a product's fp32 partial sums [n_parts, n_tokens, width]: they are added in order, rotated and rounded once; the
+// queries go to q_out [n_tokens, n_heads * hd], keys and values into their pages.  With this behind it the q/k/v product of a
+// decoding batch may cut k over workgroups, which it needs to fill the chip (6,144 outputs are 48 tiles of 128).
+// Bound by latency: a thread's chunk of 8 columns, U parts in flight, and as many workgroups as 128 threads make of the columns, so that
+// a few tokens are a few hundred waves.  64 tokens of 6,144 x 4,096: product and this kernel 18.6 us, the library's product with the
+// kernel above 23.5.  value_from_key: there are no v columns, the values are the keys before the rotation.
+#define ROPE_PARTS_THREADS 128
+template <int U>
+__global__ __launch_bounds__(ROPE_PARTS_THREADS) void rope_kv_parts_kernel(
+    const float* __restrict__ parts, size_t part_elems, int n_parts, bf16_t* __restrict__ q_out, const float* __restrict__ table,
+    const int* __restrict__ slots, bf16_t* __restrict__ k_pages, bf16_t* __restrict__ v_pages, int n_heads, int n_kv, int hd,
+    int rotary_dim, int page_size, int value_from_key) {
+  const int t = blockIdx.x;
+  const int cph = hd / 8;  // chunks per head
+  const int heads = n_heads + (value_from_key ? n_kv : 2 * n_kv);
+  const int w = blockIdx.y * ROPE_PARTS_THREADS + threadIdx.x;
+  if (w >= heads * cph) return;
+  const int head = w / cph, c = w % cph;
+  const int slot = slots[t];
+  if (head >= n_heads && slot < 0) return;
+  const float* src = parts + (size_t)t * heads * hd + 8 * w;
+  float v[8] = {};
+  for (int s = 0; s < n_parts; s += U) {
+    float p[U][8];
+#pragma unroll
+    for (int u = 0; u < U; ++u) load8<float>(src + (s + u) * part_elems, p[u]);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] += p[u][j];
+  }
+  const KvLayout lay(page_size, hd);
+  const size_t head_elems = (size_t)page_size * hd;
+  const int page = slot >= 0 ? slot / page_size : 0, off = slot >= 0 ? slot % page_size : 0;
+  const int kvh = head < n_heads ? 0 : (head - n_heads) % n_kv;
+  const size_t place = ((size_t)page * n_kv + kvh) * head_elems;
+  const bool is_v = head >= n_heads + n_kv;
+  if (is_v || (value_from_key && head >= n_heads)) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v_pages[place + lay.v_off(off, 8 * c + j)] = from_f<bf16_t>(v[j]);
+  }
+  if (is_v) return;
+  if (8 * c < rotary_dim) {
+    float cs4[8];  // cos, sin of the chunk's four pairs
+    load8<float>(table + ((size_t)t * (rotary_dim / 2) + 4 * c) * 2, cs4);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float cs = cs4[2 * j], sn = cs4[2 * j + 1];
+      const float a = v[2 * j], b = v[2 * j + 1];
+      v[2 * j] = a * cs - b * sn;
+      v[2 * j + 1] = b * cs + a * sn;
+    }
+  }
+  store8<bf16_t>(head < n_heads ? q_out + (size_t)t * n_heads * hd + 8 * w : k_pages + place + lay.k_off(off, 8 * c), v);
+}
+
+extern "C" int fg_rope_kv_parts(const float* parts, int n_parts, void* q_out, const float* table, const int* slots, void* k_pages,
+                                void* v_pages, int n_tokens, int n_heads, int n_kv, int hd, int rotary_dim, int page_size,
+                                int value_from_key, hipStream_t stream) {
+  if (n_tokens <= 0) return FG_OK;
+  if (n_parts <= 0 || hd <= 0 || hd % 8 || rotary_dim < 0 || rotary_dim > hd || rotary_dim % 8 || page_size <= 0 || page_size % 8 ||
+      n_heads <= 0 || n_kv <= 0 || (rotary_dim && !table))
+    return FG_ERR_ARG;
+  const long long chunks = (long long)(n_heads + (value_from_key ? 1 : 2) * n_kv) * (hd / 8);
+  const long long groups = (chunks + ROPE_PARTS_THREADS - 1) / ROPE_PARTS_THREADS;
+  if (groups > 65535) return FG_ERR_ARG;
+  const dim3 grid(n_tokens, (unsigned)groups);
+#define LAUNCH(U)                                                                                                          \
+  rope_kv_parts_kernel<U><<<grid, ROPE_PARTS_THREADS, 0, stream>>>(parts, (size_t)n_tokens * chunks * 8, n_parts,          \
+      (bf16_t*)q_out, table, slots, (bf16_t*)k_pages, (bf16_t*)v_pages, n_heads, n_kv, hd, rotary_dim, page_size, value_from_key)
+  if (n_parts % 8 == 0) LAUNCH(8);
+  else if (n_parts % 4 == 0) LAUNCH(4);
+  else if (n_parts % 2 == 0) LAUNCH(2);
+  else LAUNCH(1);
+#undef LAUNCH
+  return fg_launch_status();
+}

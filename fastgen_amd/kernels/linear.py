@@ -67,6 +67,12 @@ TILED_MIN_ROWS, TILED_MAX_ROWS = 65, 512
 # A plain product of fewer rows has no splits to fill the chip with and goes the other ways (6,144 x 4,096 at 65 rows 34 against
 # 23 of the library, at 320 36 against 30).
 LARGE_ROWS = TILED_MAX_ROWS
+# The q/k/v product of up to this many rows leaves partial sums to the kernel that rotates and writes the cache; both together, us,
+# against the library's product and that kernel on its rows: 6,144 x 4,096 at 17 / 64 / 128 rows 15.7 / 18.6 / 23.1 against 20.3 /
+# 23.5 / 31.4, 5,120 x 3,072 11.7 / 14.0 / 18.5 against 14.9 / 18.4 / 24.7, 12,288 x 4,096 25.1 / 29.7 / 37.9 against 30.2 / 33.9 /
+# 41.7, 2,048 x 1,536 8.5 / 9.8 / 10.9 against 10.4 / 11.2 / 11.0.  Beyond, small matrices lose (at 192 rows 2,048 x 1,536 12.2
+# against 11.7), and the sums' bytes grow with the rows where W's do not.
+QKV_PARTS_ROWS = 128
 
 
 # ------------------------------------------------------- a weight, stored for its readers
@@ -286,6 +292,17 @@ def _measure(candidates: List[Tuple[str, Callable[[], torch.Tensor]]], handicap:
     for ev, (name, _) in zip(events, candidates):
         best[name] = min(a.elapsed_time(b) for a, b in ev) + handicap.get(name, 0.0)
     return best
+
+
+def qkv_parts(x: torch.Tensor, w) -> Optional[torch.Tensor]:
+    """The q/k/v product of a decoding batch as fp32 partial sums ``[S, M, N]`` for
+    :func:`~fastgen_amd.kernels.ops.rope_kv_parts`, or None where they are not the way (``QKV_PARTS_ROWS``)."""
+    if not (force in (None, "tiled") and isinstance(w, StreamedMatrix) and w.packed is not None and x.dtype == torch.bfloat16
+            and w.dtype == torch.bfloat16 and SKINNY_ROWS < x.shape[0] <= QKV_PARTS_ROWS and w.shape[1] % 64 == 0
+            and _aligned(x, w.rows) and ops.gemm_large_takes(x, w.shape[0])):
+        return None
+    tile, splits = ops.parts_plan(x.shape[0], *w.shape)
+    return ops.gemm_large(x, w.packed, k_splits=splits, tile=tile) if splits > 1 else None
 
 
 def linear(x, w, out_dtype: Optional[torch.dtype] = None,

@@ -496,6 +496,36 @@ def rope_kv_write(qkv: torch.Tensor, positions: torch.Tensor, freqs: Optional[to
     _check(st, "rope_kv_write")
 
 
+def rope_kv_parts(parts: torch.Tensor, table: Optional[torch.Tensor], slots: torch.Tensor, k_pages: torch.Tensor,
+                  v_pages: torch.Tensor, n_heads: int, n_kv: int, head_dim: int, rotary_dim: int,
+                  value_from_key: bool = False) -> torch.Tensor:
+    """:func:`rope_kv_write` from the q/k/v product's fp32 partial sums ``parts [S, T, (H+2KV)*hd]``, added in order: returns the
+    rotated queries ``[T, H*hd]`` in bfloat16; keys and values go into their pages.  ``value_from_key``: there are no v
+    columns, a token's value is its key before the rotation."""
+    _gpu(parts, table, slots, k_pages, v_pages)
+    _need(parts.dim() == 3 and parts.dtype == torch.float32 and parts.is_contiguous()
+          and parts.shape[2] == (n_heads + (1 if value_from_key else 2) * n_kv) * head_dim,
+          "parts must be contiguous float32 [S, T, columns of q, k and v]")
+    T = parts.shape[1]
+    _need(parts.shape[0] > 0 and n_kv > 0 and head_dim % 8 == 0 and rotary_dim % 8 == 0 and 0 <= rotary_dim <= head_dim
+          and parts.data_ptr() % 16 == 0, "head_dim and rotary_dim must be multiples of 8 and rotary_dim <= head_dim")
+    _i32(slots, "slots", T)
+    if rotary_dim:
+        _need(table is not None and table.dtype == torch.float32 and table.is_contiguous()
+              and table.shape == (T, rotary_dim // 2, 2), "table must be float32 [T, rotary_dim/2, 2]")
+    _need(k_pages.dim() == 4 and k_pages.is_contiguous() and k_pages.dtype == torch.bfloat16
+          and k_pages.shape[1] == n_kv and k_pages.shape[3] == head_dim, "k_pages must be contiguous bfloat16 [n_pages, KV, P, hd]")
+    _need(v_pages.is_contiguous() and v_pages.dtype == torch.bfloat16
+          and v_pages.shape == (k_pages.shape[0], n_kv, head_dim, k_pages.shape[2]),
+          "v_pages must be contiguous bfloat16 [n_pages, KV, hd, P]")
+    q = torch.empty((T, n_heads * head_dim), dtype=torch.bfloat16, device=parts.device)
+    st = _lib.load("rope_kv").fg_rope_kv_parts(
+        _ptr(parts), parts.shape[0], _ptr(q), _ptr(table if rotary_dim else None), _ptr(slots), _ptr(k_pages), _ptr(v_pages),
+        T, n_heads, n_kv, head_dim, rotary_dim, k_pages.shape[2], int(value_from_key), _stream(parts))
+    _check(st, "rope_kv_parts")
+    return q
+
+
 # ------------------------------------------------------------------ attention
 def _distance_ok(distance: Optional[torch.Tensor], n_heads: int) -> None:
     if distance is not None:
@@ -1267,6 +1297,19 @@ def large_plan(M: int, N: int, K: int, gated: bool = False, partials: bool = Fal
     plans = [(t, 1) for t in _LARGE_COST if not gated or t % 1000 != 192]
     plans += [(t, s) for t in _LARGE_COST if t < 256000 for s in may if fits(t, s)]
     return min(plans, key=lambda p: large_cost(p[0], M, N, K, p[1], gated))
+
+
+@functools.lru_cache(maxsize=4096)
+def parts_plan(M: int, N: int, K: int) -> Tuple[int, int]:
+    """Tile and splits of k for up to 128 rows whose partial sums :func:`rope_kv_parts` adds up: as many of 4, 3 or 2 splits as leave a
+    workgroup a compute unit, each of 6 steps at least (more only add sums to read: 6,144 x 4,096 at 64 rows with 2 / 4 / 8 splits 24.4 /
+    18.6 / 22.1 us), 1 where none do.  Beyond 64 rows tiles of 64 rows where four splits of two of them fit (3,072 x 2,048 at 96 rows
+    11.9 against 13.2 of 128 rows), else of 128 (6,144 x 4,096 21.4 against 23.1)."""
+    steps, cols, places = K // 64, -(-N // 128), compute_units()
+    small = M <= 64 or -(-M // 64) * cols * 4 <= places
+    wgs = cols * (-(-M // 64) if small else -(-M // 128))
+    splits = (s for s in (4, 3, 2) if wgs * s <= places and steps // s >= 6 and -(-steps // s) * (s - 1) < steps)
+    return (64128 if small else 128128), next(splits, 1)
 
 
 def gemm_large_takes(x: torch.Tensor, N: int) -> bool:

@@ -386,7 +386,18 @@ def gemm_skinny_qkv(x, wqkv, table: Optional[torch.Tensor], slots: torch.Tensor,
     bfloat16; the rotated keys and the values go into the pages.  ``value_from_key``: there are no v rows,
     the values are the keys before the rotation.  ``gate``: ``H * hd`` more rows, whose sigmoid is returned
     behind the queries."""
-    qkv = _rows(x) @ _matrix(wqkv).T
+    return _qkv_rows(_rows(x) @ _matrix(wqkv).T, table, slots, k_pages, v_pages, n_heads, n_kv, head_dim, rotary_dim,
+                     value_from_key, gate)
+
+
+def rope_kv_parts(parts: torch.Tensor, table: Optional[torch.Tensor], slots: torch.Tensor, k_pages: torch.Tensor,
+                  v_pages: torch.Tensor, n_heads: int, n_kv: int, head_dim: int, rotary_dim: int,
+                  value_from_key: bool = False) -> torch.Tensor:
+    """:func:`gemm_skinny_qkv` from the product's partial sums ``[S, T, columns]``."""
+    return _qkv_rows(parts.sum(0), table, slots, k_pages, v_pages, n_heads, n_kv, head_dim, rotary_dim, value_from_key, False)
+
+
+def _qkv_rows(qkv, table, slots, k_pages, v_pages, n_heads, n_kv, head_dim, rotary_dim, value_from_key, gate) -> torch.Tensor:
     T, q_cols, kv_cols = qkv.shape[0], n_heads * head_dim, n_kv * head_dim
     q = _rotate(qkv[:, :q_cols].view(T, n_heads, head_dim), table, rotary_dim)
     k_raw = qkv[:, q_cols : q_cols + kv_cols].view(T, n_kv, head_dim)

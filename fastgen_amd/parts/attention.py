@@ -33,7 +33,7 @@ from typing import Any, List, Mapping, Optional
 import torch
 
 from ..kernels import ops
-from ..kernels.linear import StreamedMatrix, linear, skinny_ok, streamed
+from ..kernels.linear import StreamedMatrix, linear, qkv_parts, skinny_ok, streamed
 from .base import LayerStore, PagedNeed, StateNeed, TensorSpec, build_part, place, register_part, MATRIX, VECTOR
 from .rows_mixer import RowsMixer
 
@@ -218,12 +218,18 @@ class Attention(RowsMixer):
         else:
             # an entry that reads another entry's cache needs its queries only (and its gate)
             own_rows = self.wqkv if store.owns or self.output_gate else self.wqkv.first_rows(q_width)
-            qkv = linear(x, own_rows)
-            ops.rope_kv_write(
-                qkv, ctx.positions, self.freqs, group.slots, store.k_pages, store.v_pages,
-                self.n_heads, self.n_kv_heads, self.head_dim, self.position.rotary_dim, write_kv=store.owns,
-                table=table, v_col=v_col,
-            )
+            plain = store.owns and not self.output_gate and self.head_dim % 8 == 0 and self.position.rotary_dim % 8 == 0
+            parts = qkv_parts(x, own_rows) if plain else None
+            if parts is not None:
+                qkv = ops.rope_kv_parts(parts, table, group.slots, store.k_pages, store.v_pages, self.n_heads, self.n_kv_heads,
+                                        self.head_dim, self.position.rotary_dim, value_from_key=self.value_from_key)
+            else:
+                qkv = linear(x, own_rows)
+                ops.rope_kv_write(
+                    qkv, ctx.positions, self.freqs, group.slots, store.k_pages, store.v_pages,
+                    self.n_heads, self.n_kv_heads, self.head_dim, self.position.rotary_dim, write_kv=store.owns,
+                    table=table, v_col=v_col,
+                )
             gate = qkv[:, gate_col:] if self.output_gate else None
             gate_done = False
         out = torch.empty((rows.shape[0], q_width), dtype=rows.dtype, device=rows.device)

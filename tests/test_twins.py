@@ -23,7 +23,7 @@ from plain_llama import plain_attention, plain_rmsnorm, plain_rope_interleaved, 
 # functions of ops that launch a kernel (the others plan work, build arguments or pick a kernel)
 KERNEL_OPS = ["embed", "add_rmsnorm", "rmsnorm", "silu_mul", "rope_table", "rope_kv_write", "paged_attention_general",
               "paged_attention_mfma", "paged_attention", "gemm_nt", "scale_rows", "gemm_skinny_residual", "gemm_skinny",
-              "gemm_skinny_qkv", "gemm_tiled", "gemm_large", "sample", "logprob", "stream_add", "add_rows", "gate_mul", "moe_route",
+              "gemm_skinny_qkv", "rope_kv_parts", "gemm_tiled", "gemm_large", "sample", "logprob", "stream_add", "add_rows", "gate_mul", "moe_route",
               "moe_sort", "moe_gate_up", "moe_down", "moe_combine", "gelu_mul", "post_add_rmsnorm", "softcap",
               "heads_prepare", "head_linear", "head_norm_gate", "decay_scan", "gated_mul", "causal_conv", "selective_scan",
               "sigmoid_attention", "scale_logits", "head_diff_norm", "streams_spread", "streams_step", "conv_tail",
@@ -243,6 +243,30 @@ def test_rope_kv_write_twin(ops, dtype, H, KV, hd, rot, P):
         for i in (0, 4, 5):  # q (and the untouched k, v columns), the K pages, the V pages
             _close(dev[i], cpu[i], dtype)
     _both("rope_kv_write", make, compare, ops)
+
+
+@gpu
+@pytest.mark.parametrize("S,T,H,KV,hd,rot,P,from_key", [(2, 17, 6, 2, 48, 48, 16, False), (8, 64, 32, 8, 128, 128, 64, False),
+                                                        (3, 1, 5, 1, 80, 32, 8, False), (4, 33, 4, 4, 64, 0, 16, False),
+                                                        (16, 20, 16, 3, 40, 24, 32, True)])
+def test_rope_kv_parts_twin(ops, S, T, H, KV, hd, rot, P, from_key):
+    """The sums of 2 to 16 parts (all in flight, or in rounds), columns that fill no workgroup, a token without a place.  The sums
+    differ by fp32 rounding only, so a bfloat16 result by one step of it at most (2^-8 of the value; near zero, after a
+    rotation, S + 2 roundings of sums of up to S * 6)."""
+    torch.manual_seed(hd)
+    pos = torch.randint(0, 5000, (T,), dtype=torch.int32)
+    slots = torch.randperm(12 * P)[:T].to(torch.int32)
+    slots[T // 2] = -1
+    table = twins.rope_table(pos, 1.0 / 500000.0 ** (torch.arange(0, rot, 2).float() / rot)) if rot else None
+    make = lambda: (torch.randn(S, T, (H + (1 if from_key else 2) * KV) * hd), table, slots, torch.full((12, KV, P, hd), 7.0).bfloat16(),
+                    torch.full((12, KV, hd, P), 7.0).bfloat16(), H, KV, hd, rot, from_key)
+
+    def compare(got, want, dev, cpu):
+        for g, w in ((got, want), (dev[3], cpu[3]), (dev[4], cpu[4])):
+            torch.testing.assert_close(g.float().cpu(), w.float(), rtol=2.0**-7, atol=(S + 2) * S * 6 * 2.0**-24)
+    _both("rope_kv_parts", make, compare, ops)
+    with pytest.raises(ops.KernelArgumentError):
+        ops.rope_kv_parts(*[a.cuda() if isinstance(a, torch.Tensor) else a for a in (make()[0][:, :, :-8].contiguous(), *make()[1:])])
 
 
 def _attention_case(dtype, H, KV, hd, P, lens, seed):
