@@ -8,9 +8,9 @@ large tiles of ``gemm_large.hip`` for prompts, and
 the vendor library's product through ``torch``, which the reference uses for
 all of them: cuBLAS through ``F.linear``, ``fastgen/forward.py:433-513``).
 Which one is the fastest depends on the matrix and on the number of rows, so
-it is measured: the first few times a product of some shape ``(N, K)`` meets some
-number of rows, the kernels that can take it are timed on the operands at hand
-(the caches emptied before each run) and the winner is kept in one table (``choices``) for every later product of
+it is measured: the first time a product of some shape ``(N, K)`` meets some
+number of rows, the kernels that can take it are timed on the model's matrices of that shape
+(the caches emptied before each run) and the winner is kept in one table (``choices``) for this and every later product of
 that shape and row bucket; times that are close are a tie, which a fixed order decides.  No size of any model stands here or in the parts.
 
 A part hands ``linear`` its matrix as a :class:`StreamedMatrix` (made by :func:`streamed` when the part
@@ -20,10 +20,12 @@ in which the streaming kernels read it, which those kernels take.
 
 from __future__ import annotations
 
+import itertools
 import os
+import weakref
 from contextlib import contextmanager
 from dataclasses import dataclass
-from typing import Callable, Dict, List, Optional, Tuple
+from typing import Callable, Dict, List, Optional, Sequence, Tuple
 
 import torch
 
@@ -86,6 +88,7 @@ class StreamedMatrix:
 
     rows: torch.Tensor
     packed: Optional[ops.PackedWeight] = None
+    part_of: Optional["StreamedMatrix"] = None  # the matrix whose first rows these are
 
     @property
     def shape(self):
@@ -103,11 +106,26 @@ class StreamedMatrix:
     def first_rows(self, n: int) -> "StreamedMatrix":
         """The matrix of the first ``n`` rows (views; the packed copy only if ``n`` is a multiple of 16)."""
         keep = self.packed is not None and (n % 16 == 0 or n == self.rows.shape[0])
-        return StreamedMatrix(self.rows[:n], self.packed.first_rows(n) if keep else None)
+        return StreamedMatrix(self.rows[:n], self.packed.first_rows(n) if keep else None, self)
+
+    def alike(self) -> List["StreamedMatrix"]:
+        """This matrix and the others of its kind, other layers' as a rule: what a measurement is made on."""
+        if self.part_of is not None:
+            return [self] + [m.first_rows(self.rows.shape[0]) for m in self.part_of.alike()[1:]]
+        others = (ref() for ref in _stored.get(_kind(self), ()))
+        return [self] + [m for m in others if m is not None and m is not self]
 
     def nbytes(self) -> int:
         return self.rows.numel() * self.rows.element_size() + (
             self.packed.data.numel() * self.packed.data.element_size() if self.packed is not None else 0)
+
+
+# the stored matrices of a kind, as long as their parts hold them
+_stored: Dict[tuple, List["weakref.ref[StreamedMatrix]"]] = {}
+
+
+def _kind(m: StreamedMatrix) -> tuple:
+    return tuple(m.rows.shape), m.rows.stride(), m.rows.dtype, m.rows.device, m.rows.data_ptr() % 16, m.packed is not None
 
 
 # whether `streamed` makes the second copy: set for the time a model loads (`packing`)
@@ -142,9 +160,11 @@ def packing_fits(matrix_bytes: int, device, budget_bytes: Optional[int] = None) 
 
 def streamed(w: torch.Tensor) -> StreamedMatrix:
     """A part's weight matrix, placed on the device, as the products take it."""
-    if _pack_now and w.is_cuda and w.dtype == torch.bfloat16 and w.dim() == 2:
-        return StreamedMatrix(w, ops.pack_weight(w))
-    return StreamedMatrix(w)
+    pack = _pack_now and w.is_cuda and w.dtype == torch.bfloat16 and w.dim() == 2
+    m = StreamedMatrix(w, ops.pack_weight(w) if pack else None)
+    if w.dtype == torch.bfloat16:  # (a 32-bit product is not measured)
+        _stored[_kind(m)] = [ref for ref in _stored.get(_kind(m), ()) if ref() is not None] + [weakref.ref(m)]
+    return m
 
 
 def _rows_of(w) -> torch.Tensor:
@@ -190,8 +210,8 @@ force: Optional[str] = None
 _TIMED_RUNS = 2  # of every candidate, each of the _SAMPLES times
 # How long a product takes depends on where its matrix happens to lie (64 rows of 28,672 x 4,096: the library's takes 49 to
 # 51 us on one layer's matrix and 59 to 63 on the next ones, in every process; the wide kernel 52 to 57 on all of them), so
-# the candidates are measured at the first calls that ask for a product, in a model one layer's matrix after the other; not
-# again where one of them leads by more than that.
+# the candidates are measured on as many of the model's matrices, one layer's after the other's; not again where one of them
+# leads by more than that.
 _SAMPLES, _CLEAR = 3, 0.25
 # A lead smaller than this decides nothing: the same program would take one kernel today and another tomorrow, and their
 # results differ by a rounding.
@@ -234,7 +254,7 @@ def _winner(best: Dict[str, float], order: List[str]) -> str:
 
 def _choose(what: str, n: int, k: int, rows: int, candidates: List[Tuple[str, Callable[[], torch.Tensor]]],
             handicap: Optional[Dict[str, float]] = None, library_ties: bool = False) -> str:
-    """The candidate to run: the forced one, the one the table holds, or, at the first calls, the fastest so far.
+    """The candidate to run: the forced one, the one the table holds, or, measured once more, the fastest so far.
     Timing needs the device to itself (events and a wait for them), so a product that is first met while
     a step is being recorded runs the first candidate, unrecorded in the table; the engine runs every
     step once, unrecorded, before it records it.  The candidates are timed in turn on the same
@@ -264,6 +284,20 @@ def _choose(what: str, n: int, k: int, rows: int, candidates: List[Tuple[str, Ca
     else:
         _samples.pop(key, None)
     return winner
+
+
+def _settle(what: str, n: int, k: int, rows: int, candidates: List[Tuple[str, Callable]], matrices: Callable[[], Sequence],
+            handicap: Optional[Dict[str, float]] = None, library_ties: bool = False) -> str:
+    """:func:`_choose` until the table's entry stays, before anything is computed by it: with the best so far, a step that
+    is recorded after one warm-up would keep a kernel that the next engine of the process does not take, and their results would
+    differ by a rounding.  ``candidates``: functions of a matrix; ``matrices()``: the matrices that they are timed on in turn."""
+    key = (what, n, k, row_bucket(rows))
+    if choices.get(key) in (c[0] for c in candidates) and key not in _samples and force is None:
+        return choices[key]
+    for m in itertools.cycle(matrices()):
+        name = _choose(what, n, k, rows, [(c, lambda fn=fn: fn(m)) for c, fn in candidates], handicap, library_ties)
+        if key not in _samples or _capturing():
+            return name
 
 
 def _measure(candidates: List[Tuple[str, Callable[[], torch.Tensor]]], handicap: Dict[str, float],
@@ -328,8 +362,8 @@ def linear(x, w, out_dtype: Optional[torch.dtype] = None,
         raise ops.KernelArgumentError(f"linear: unknown epilogue {epilogue!r}")
     gated = "gelu_tanh" if epilogue == "gelu_tanh_mul" else True  # what the kernels' epilogue argument takes
     act_mul = ops.gelu_mul if epilogue == "gelu_tanh_mul" else ops.silu_mul
-    sw = w.streaming if isinstance(w, StreamedMatrix) else w  # what the streaming kernels read
-    w = _rows_of(w)
+    matrix = w if isinstance(w, StreamedMatrix) else StreamedMatrix(w)
+    sw, w = matrix.streaming, matrix.rows  # what the streaming kernels read, and the library
     scaled = x if isinstance(x, ops.ScaledRows) else None
     if scaled is not None:
         if not fold_ok(scaled.rows, w) or out_dtype not in (None, torch.bfloat16):
@@ -355,17 +389,17 @@ def linear(x, w, out_dtype: Optional[torch.dtype] = None,
         if h.dtype == torch.float32 and h.is_contiguous() and h.shape == (rows, N):
             return ops.gemm_skinny_residual(src, sw, h, norm_w, eps)
 
-    def library() -> torch.Tensor:
+    def library(m: StreamedMatrix) -> torch.Tensor:
         xin = scaled.materialize() if scaled is not None else x
         if out_dtype == torch.bfloat16:
-            y = torch.nn.functional.linear(xin, w)
+            y = torch.nn.functional.linear(xin, m.rows)
         else:
-            y = _library_mm_f32_out(xin, w)
+            y = _library_mm_f32_out(xin, m.rows)
             if y is None:
-                y = ops.gemm_nt(xin, w, out_dtype=torch.float32)
+                y = ops.gemm_nt(xin, m.rows, out_dtype=torch.float32)
         return act_mul(y) if silu else y
 
-    candidates: List[Tuple[str, Callable[[], torch.Tensor]]] = []
+    candidates: List[Tuple[str, Callable[[StreamedMatrix], torch.Tensor]]] = []
     handicap: Dict[str, float] = {}
     large_ok = (own and sw is not w and K % 64 == 0 and scaled is None and (not silu or (N % 16 == 0 and out_dtype == torch.bfloat16))
                 and ops.gemm_large_takes(x, N))
@@ -382,25 +416,25 @@ def linear(x, w, out_dtype: Optional[torch.dtype] = None,
 
     if own and silu and out_dtype == torch.bfloat16 and N % 16 == 0:
         if rows <= SKINNY_ROWS:
-            candidates.append(("narrow", lambda: ops.gemm_skinny(src, sw, silu_mul_epilogue=gated, wide=False)))
+            candidates.append(("narrow", lambda m: ops.gemm_skinny(src, m.streaming, silu_mul_epilogue=gated, wide=False)))
         if rows <= WIDE_ROWS:
-            candidates.append(("wide", lambda: ops.gemm_skinny(src, sw, silu_mul_epilogue=gated, wide=True)))
+            candidates.append(("wide", lambda m: ops.gemm_skinny(src, m.streaming, silu_mul_epilogue=gated, wide=True)))
         if tiled_ok:
-            candidates.append(("tiled256", lambda: ops.gemm_tiled(x, sw, silu_mul_epilogue=gated, tile_rows=256)))
+            candidates.append(("tiled256", lambda m: ops.gemm_tiled(x, m.streaming, silu_mul_epilogue=gated, tile_rows=256)))
     elif own and not silu:
         if rows <= SKINNY_ROWS:
-            candidates.append(("narrow", lambda: ops.gemm_skinny(src, sw, out_dtype, wide=False)))
+            candidates.append(("narrow", lambda m: ops.gemm_skinny(src, m.streaming, out_dtype, wide=False)))
         elif rows <= WIDE_ROWS and partials_ok:
             splits = k_splits_for(N, K, rows)
-            candidates.append(("wide", lambda: ops.gemm_skinny(x, sw, out_dtype, k_splits=splits, wide=True)))
+            candidates.append(("wide", lambda m: ops.gemm_skinny(x, m.streaming, out_dtype, k_splits=splits, wide=True)))
             handicap["wide"] = sums_cost(splits)
         elif rows <= 64:
-            candidates.append(("wide", lambda: ops.gemm_skinny(x, sw, out_dtype, wide=True)))
+            candidates.append(("wide", lambda m: ops.gemm_skinny(x, m.streaming, out_dtype, wide=True)))
         if tiled_ok and partials_ok and out_dtype == torch.bfloat16:
             for name, tile_rows in zip(("tiled", "tiled256"), ops.TILED_TILE_ROWS):
                 s_t = tiled_splits(N, K, rows, tile_rows)
-                candidates.append((name, lambda tile_rows=tile_rows, s_t=s_t: ops.gemm_tiled(
-                    x, sw, out_dtype, k_splits=s_t, tile_rows=tile_rows)))
+                candidates.append((name, lambda m, tile_rows=tile_rows, s_t=s_t: ops.gemm_tiled(
+                    x, m.streaming, out_dtype, k_splits=s_t, tile_rows=tile_rows)))
                 handicap[name] = sums_cost(s_t)
     if scaled is None or not candidates:
         candidates.append(("library", library))
@@ -409,5 +443,5 @@ def linear(x, w, out_dtype: Optional[torch.dtype] = None,
         "+packed" if sw is not w else "")
     # Ties: the kernel with the epilogue in it, and with few rows the narrow one, both the least launches; a plain
     # product of more rows goes to the library, whose result is whole (no partial sums to add).
-    name = _choose(what, N, K, rows, candidates, handicap, library_ties=not silu and rows > SKINNY_ROWS)
-    return dict(candidates)[name]()
+    name = _settle(what, N, K, rows, candidates, matrix.alike, handicap, library_ties=not silu and rows > SKINNY_ROWS)
+    return dict(candidates)[name](matrix)

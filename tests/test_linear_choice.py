@@ -1,6 +1,7 @@
 """Which kernel the table of measured products takes."""
 
 import pytest
+import torch
 
 from fastgen_amd.kernels import linear
 
@@ -69,3 +70,55 @@ def test_nothing_is_measured_while_a_step_is_recorded(ask):
     linear.choices.clear(), linear._samples.clear()
     linear.choices[("silu_mul", 28672, 4096, 64)] = "library"  # put there by a caller
     assert ask(["wide", "library"]) == "library"
+
+
+@pytest.mark.parametrize("times,winner", [([(54.9, 48.6), (53.8, 60.1), (54.0, 61.0)], "wide"),  # the first matrix lies well
+                                          ([(50.0, 40.0), (50.0, 49.0), (50.0, 40.0)], "library")])
+@pytest.mark.parametrize("n_matrices", [1, 2, 3, 5])
+def test_a_product_is_settled_before_it_is_used(ask, monkeypatch, times, winner, n_matrices):
+    """The first pass takes the kernel that later ones take, whatever it is and however few matrices a model has: a step that is
+    recorded after one warm-up (two layers, one head) and the next engine's have the same bits.  The samples are of
+    one matrix after the other."""
+    ask(["wide"])  # (installs the fixture's table)
+    left, on = list(times), []
+    run = [("wide", lambda m: on.append(m)), ("library", lambda m: None)]
+
+    def measure(candidates, handicap, first):
+        candidates[0][1]()
+        return dict(zip(("wide", "library"), left.pop(0)))
+
+    monkeypatch.setattr(linear, "_measure", measure)
+    settle = lambda: linear._settle("silu_mul", 28672, 4096, 64, run, lambda: list(range(n_matrices)))
+    assert settle() == winner and not left and not linear._samples
+    assert on == [i % n_matrices for i in range(3)]
+    monkeypatch.setattr(linear, "_capturing", lambda: True)
+    assert settle() == winner
+    monkeypatch.setattr(linear, "_capturing", lambda: False)
+    assert settle() == winner
+
+
+def test_settling_ends_where_nothing_is_measured(ask, monkeypatch):
+    ask(["wide"])
+    two = [("wide", lambda m: None), ("library", lambda m: None)]
+    settle = lambda names: linear._settle("silu_mul", 28672, 4096, 64, names, lambda: [0])
+    assert settle(two[:1]) == "wide" and not linear.choices  # one candidate
+    monkeypatch.setattr(linear, "force", "library")
+    assert settle(two) == "library" and not linear.choices
+    monkeypatch.setattr(linear, "force", None)
+    monkeypatch.setattr(linear, "_capturing", lambda: True)
+    assert settle(two) == "wide" and not linear.choices  # first met inside a recording
+
+
+def test_matrices_that_are_measured_for_one_another():
+    """The stored matrices of one shape, layout and alignment, as long as somebody holds them; of a part of a matrix the
+    same parts."""
+    make = lambda *shape: linear.streamed(torch.zeros(*shape, dtype=torch.bfloat16))
+    a, b, other = make(48, 64), make(48, 64), make(64, 48)
+    c = linear.StreamedMatrix(torch.zeros(48, 64, dtype=torch.bfloat16))  # stored by nobody
+    assert [m is x for m, x in zip(a.alike(), (a, b))] == [True, True] and len(a.alike()) == 2
+    assert other.alike() == [other] and len(c.alike()) == 3 and c.alike()[0] is c
+    part = b.first_rows(16).alike()
+    assert [m.rows.data_ptr() for m in part] == [b.rows.data_ptr(), a.rows.data_ptr()] and all(m.shape == (16, 64) for m in part)
+    del a, part
+    assert len(b.alike()) == 1
+    assert len(linear._stored[linear._kind(make(48, 64))]) <= 2  # what is gone is not kept
