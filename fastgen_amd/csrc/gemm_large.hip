@@ -59,16 +59,13 @@ __device__ __forceinline__ void gemm_large_tile(bf16_t* lds, const bf16_t* x, in
   op.x = x + (size_t)m0 * ldx;
   op.x_bytes = 2u * (unsigned)((min(16 * MB, M - m0) - 1) * ldx + K);
   op.w_row = (unsigned)K * 32u;
-  const int blocks = max(0, min(NB, (N + 15) / 16 - n0 / 16));  // of 16 rows of W that are there
-  op.w[0] = (const char*)w + (size_t)(n0 / 16) * op.w_row;
-  op.w[1] = (const char*)op.w[0] + (size_t)Product::HALF * op.w_row;
-  op.w_bytes[0] = min(blocks, Product::HALF) * op.w_row;
-  op.w_bytes[1] = max(blocks - Product::HALF, 0) * op.w_row;
+  op.set_w(0, w, n0 / 16, (N + 15) / 16, Product::HALF);
+  op.set_w(1, w, n0 / 16 + Product::HALF, (N + 15) / 16, NB - Product::HALF);
   unsigned xo[Product::XL];
 #pragma unroll
   for (int j = 0; j < Product::XL; ++j) {
     const int row = Product::row_of(wave, j, lane);
-    xo[j] = m0 + row < M ? 2u * (unsigned)(row * ldx) + Product::chunk_of(lane) : TP_NOWHERE;
+    xo[j] = op.row_offset(m0 + row < M, row, ldx, Product::chunk_of(lane));
   }
   f32x4 acc[MB][NB];
   Product::run(lds, op, xo, wave, lane, first, n_stages, n_stages, acc);

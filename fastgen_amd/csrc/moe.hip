@@ -730,23 +730,16 @@ __device__ __forceinline__ void moe_large_tile(bf16_t* lds, const bf16_t* x, uns
   op.x = EPI == MT_GATE_UP ? (const void*)x : (const void*)(x + (size_t)tile.y * ldx);
   op.x_bytes = EPI == MT_GATE_UP ? x_bytes : 2u * (unsigned)((tile.z - 1) * ldx + K);
   op.w_row = (unsigned)K * 32u;
-  const size_t at = ((size_t)tile.x * blocks + block) * op.w_row;
-  if constexpr (EPI == MT_GATE_UP) {
-    op.w[0] = (const char*)w0 + at;
-    op.w[1] = (const char*)w1 + at;
-    op.w_bytes[0] = op.w_bytes[1] = (unsigned)max(0, min(NB / 2, blocks - block)) * op.w_row;
-  } else {
-    op.w[0] = (const char*)w0 + at;
-    op.w[1] = (const char*)w0 + at + (size_t)Product::HALF * op.w_row;
-    op.w_bytes[0] = (unsigned)max(0, min(Product::HALF, blocks - block)) * op.w_row;
-    op.w_bytes[1] = (unsigned)max(0, min(NB - Product::HALF, blocks - block - Product::HALF)) * op.w_row;
-  }
+  const size_t expert = (size_t)tile.x * blocks * op.w_row;
+  op.set_w(0, (const char*)w0 + expert, block, blocks, Product::HALF);
+  if constexpr (EPI == MT_GATE_UP) op.set_w(1, (const char*)w1 + expert, block, blocks, NB - Product::HALF);
+  else op.set_w(1, (const char*)w0 + expert, block + Product::HALF, blocks, NB - Product::HALF);
   unsigned xo[Product::XL];
 #pragma unroll
   for (int j = 0; j < Product::XL; ++j) {
     const int row = Product::row_of(wave, j, lane);
     const int from = EPI == MT_GATE_UP ? sorted[tile.y + min(row, tile.z - 1)] / top : row;
-    xo[j] = row < tile.z ? 2u * (unsigned)from * (unsigned)ldx + Product::chunk_of(lane) : TP_NOWHERE;
+    xo[j] = op.row_offset(row < tile.z, from, ldx, Product::chunk_of(lane));
   }
   f32x4 acc[MB][NB];
   Product::run(lds, op, xo, wave, lane, 0, K / 64, K / 64, acc);

@@ -20,7 +20,10 @@
 // (22 k of its 178 k clocks it waits at barriers and for its first loads); 14,336 of k 314 us = 1.53.  Without the order
 // within a stage 329, and with eight waves of 128 x 64 and rows of x through registers 473 against 359 (28,672 x 4,096, gated).
 //
-// Rows of x beyond the tile, and stages beyond the k range, are loads behind the end of their buffer: zeros, and no access.
+// Rows of x beyond the tile and stages beyond the k range are loads behind the end of their buffer: zeros, and no access.  Whether and
+// how a load's scalar offset takes part in that check must not matter for where it reads: a row that is not there has a lane's offset
+// (TP_NOWHERE) that is behind any buffer and stays so with the scalar offset added, a stage that is not there has a size of 0,
+// and a block of the matrix that is not there is the last one that is: its sums are not stored.
 #pragma once
 
 #include "common.h"
@@ -29,8 +32,9 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-// An offset behind the end of any buffer: the load gives zeros.
-#define TP_NOWHERE 0xfffffff0u
+// A lane's offset behind the end of any buffer (they have up to 4,000,000,000 bytes, of which a row's 2 K are at most 62,500,000): the
+// load gives zeros.
+#define TP_NOWHERE 0xf0000000u
 
 struct TileOperands {
   const void* x;     // first byte that an offset of a row counts from
@@ -38,6 +42,23 @@ struct TileOperands {
   const void* w[2];  // packed rows of the wave's first (NB + 1) / 2 blocks of 16, and of the others
   unsigned w_bytes[2];
   unsigned w_row;    // bytes of 16 packed rows
+  unsigned w_step[2];  // from a part's first block to its second: 0 where there is none
+
+  // w[part]: `most` blocks from block `block` on of a matrix of `blocks`, those that are there.
+  __host__ __device__ __forceinline__ void set_w(int part, const void* matrix, int block, int blocks, int most) {
+    const int there = max(0, min(most, blocks - block));
+    w[part] = (const char*)matrix + (there ? (size_t)block * w_row : 0);
+    w_bytes[part] = there * w_row;
+    w_step[part] = there > 1 ? w_row : 0;
+  }
+  __host__ __device__ __forceinline__ unsigned row_offset(bool there, int row, int ldx, unsigned chunk) const {
+    return there ? 2u * (unsigned)row * (unsigned)ldx + chunk : TP_NOWHERE;
+  }
+};
+
+// What a load's buffer holds, and the scalar part of its offset.
+struct TileLoad {
+  unsigned bytes, at;
 };
 
 template <int MB, int NB, int NST, int WS, bool ONE_WAVE>
@@ -49,7 +70,17 @@ struct TileProduct {
   static constexpr int LA = NST - 2;                 // stages asked for ahead
   static constexpr int U = WS / 2;                   // stages a round of the loop
   static constexpr int HALF = (NB + 1) / 2;
-  static_assert(MB % RB == 0 && MB % 4 == 0 && WS % 2 == 0 && NST >= 4, "tile");
+  static_assert(MB % RB == 0 && MB % 4 == 0 && NB <= 4 && WS % 2 == 0 && NST >= 4, "tile");
+
+  // The loads of stage s of the range's n_stages, and of block nb and step t of 32 k.  (HALF is at most 2.)
+  __host__ __device__ static __forceinline__ TileLoad x_load(const TileOperands& op, int s, int first, int n_stages) {
+    return {s < n_stages ? op.x_bytes : 0u, 128u * (unsigned)(first + s)};
+  }
+  __host__ __device__ static __forceinline__ TileLoad w_load(const TileOperands& op, int nb, int t, int first, int n_stages) {
+    const int part = nb < HALF ? 0 : 1;
+    return {t < 2 * n_stages ? op.w_bytes[part] : 0u,
+            (nb - part * HALF) * op.w_step[part] + 1024u * (unsigned)(2 * first + t)};
+  }
 
 #ifdef __HIP_DEVICE_COMPILE__
   template <int N>
@@ -98,16 +129,16 @@ struct TileProduct {
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb) acc[mb][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
     auto load_x = [&](int s, int slot, int j) {
-      const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)op.x, 0, s < n_stages ? op.x_bytes : 0u, 0x20000);
+      const TileLoad load = x_load(op, s, first, n_stages);
+      const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)op.x, 0, load.bytes, 0x20000);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(ring + slot * STAGE + (wave + 4 * j) * 512),
-                                               16, xo[j], 128 * (first + s), 0, 0);
+                                               16, xo[j], load.at, 0, 0);
     };
     const unsigned wo = lane * 16;
     auto load_w = [&](int t, int set, int nb) {
-      const int part = nb < HALF ? 0 : 1;
-      const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)op.w[part], 0, t < 2 * n_stages ? op.w_bytes[part] : 0u, 0x20000);
-      wr[set][nb] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(
-          rs, wo, (nb - part * HALF) * op.w_row + 1024u * (unsigned)(2 * first + t), 0));
+      const TileLoad load = w_load(op, nb, t, first, n_stages);
+      const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)op.w[nb < HALF ? 0 : 1], 0, load.bytes, 0x20000);
+      wr[set][nb] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rs, wo, load.at, 0));
     };
     const int r16 = lane & 15, g = lane >> 4, row8 = r16 % 8;
     int off[2];  // this lane's place in a block of 16 rows, for the first and the second 32 k of a stage
