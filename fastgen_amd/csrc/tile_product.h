@@ -150,6 +150,9 @@ struct TileProduct {
     for (int s = 0; s < LA; ++s)
 #pragma unroll
       for (int j = 0; j < XL; ++j) load_x(s, s, j);
+    // the count below is of loads behind these: all of x before the first of the matrix
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int t = 0; t < WS - 1; ++t)
 #pragma unroll

@@ -1,5 +1,7 @@
-"""The offsets of the large tiles' loads (csrc/tile_product.h), worked out by the kernels' own functions on the CPU."""
+"""The large tiles' product (csrc/tile_product.h) as far as it shows without a GPU: the offsets of its loads, worked out by the
+kernels' own functions, and the order in which the compiler leaves the first ones."""
 
+import re
 import shutil
 import subprocess
 
@@ -121,3 +123,36 @@ def test_loads_stay_inside_whichever_way_the_scalar_offset_is_checked(hipcc, tmp
                     str(tmp_path / "loads")], check=True, timeout=120)
     run = subprocess.run([str(tmp_path / "loads")], capture_output=True, text=True, timeout=100)
     assert run.returncode == 0, run.stdout
+
+
+def first_loads(listing):
+    """The buffer loads in front of a product's first barrier, one string per product: x to LDS, W to registers."""
+    found, here = [], ""
+    for line in listing.splitlines():
+        if "s_barrier" in line and len(here) > 8:  # in a product there are fewer between two matrix instructions
+            found.append(here)
+        if "v_mfma" in line or "s_barrier" in line or "s_nop 15" in line:  # (which end a product)
+            here = ""
+        elif "buffer_load_dwordx4" in line:
+            here += "x" if re.search(r"\blds\b", line) else "W"
+    return found
+
+
+@pytest.mark.parametrize("source", ["gemm_large", "moe"])
+def test_first_loads_are_in_the_order_that_the_wait_counts(hipcc, tmp_path, source):
+    """The wait in front of a product's first barrier lets a number of loads be on their way: it is right only if all of x was
+    asked for before the first of W."""
+    flags = [f for f in _lib.HIPCC_FLAGS if f not in ("-shared", "-fPIC")]
+    subprocess.run([hipcc, *flags, "-S", "--offload-device-only", f"-I{_lib.CSRC}", str(_lib.CSRC / f"{source}.hip"), "-o",
+                    str(tmp_path / "listing")], check=True, capture_output=True, timeout=300)
+    n_products = 0
+    for name, body in re.findall(r"^(_Z\d+(?:gemm|moe)_large_kernel\w+):(.*?)^\.Lfunc_end", (tmp_path / "listing").read_text(), re.S | re.M):
+        mb, nb, nst, ws = (int(n) for n in re.findall(r"Li(\d+)E", name)[:4])
+        products = first_loads(body)
+        # tiles of 256 rows also go in halves; the experts' as products of 64 rows on
+        rows = [m for m in (16, 8, 4) if m == mb or (m < mb and (source == "moe" or m == 8))]
+        assert sorted(products) == sorted("x" * ((nst - 2) * m // 2) + "W" * ((ws - 1) * nb) for m in rows), name
+        n_products += len(products)
+    assert n_products >= 14
+    assert first_loads("buffer_load_dwordx4 v1, s[0:3], 0 offen lds\n" * 4 + "buffer_load_dwordx4 v[0:3], v1, s[0:3], 0 offen\n" * 5
+                       + "buffer_load_dwordx4 v1, s[0:3], 0 offen lds\n" * 2 + "s_barrier\n") == ["xxxxWWWWWxx"]
