@@ -1329,8 +1329,8 @@ def gemm_large(x: torch.Tensor, w: "PackedWeight", out_dtype: Optional[torch.dty
     engine's large tiles (``tile``: one of ``LARGE_TILES``, default the one that suits the sizes); with
     ``silu_mul_epilogue`` as :func:`gemm_skinny`; with ``k_splits > 1`` fp32 ``[k_splits, M, N]`` partial sums over the k ranges
     ``[s * ceil(K / 64 / k_splits) * 64, ...)``."""
-    _gpu(x)
-    _need(x.dtype == torch.bfloat16 and x.dim() == 2 and isinstance(w, PackedWeight), "gemm_large takes bfloat16 x [M, K], w packed")
+    _need(isinstance(w, PackedWeight) and x.dtype == torch.bfloat16 and x.dim() == 2, "gemm_large takes bfloat16 x [M, K], w packed")
+    _gpu(x, w.data)
     M, K = x.shape
     N = w.shape[0]
     _need(M > 0 and K % 64 == 0 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.stride(0) >= K and x.data_ptr() % 16 == 0,
