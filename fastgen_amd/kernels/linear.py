@@ -204,7 +204,8 @@ choices: Dict[Tuple[str, int, int, int], str] = {}
 # the same keys -> what each candidate took when it was measured (milliseconds on average, the consumer's cost included)
 timings: Dict[Tuple[str, int, int, int], Dict[str, float]] = {}
 _samples: Dict[Tuple[str, int, int, int], List[Dict[str, float]]] = {}  # of the keys that are still measured
-# set to a candidate's name to take that kernel wherever it is among the candidates (tests run the
+# set to a candidate's name to take that kernel wherever it is among the candidates, to "large" for the large tiles
+# wherever they can take a product of more than 16 rows, under any other name not by their rule (tests run the
 # engine once under each name, so that every kernel that may be chosen is compared with the plain run)
 force: Optional[str] = None
 _TIMED_RUNS = 2  # of every candidate, each of the _SAMPLES times
@@ -331,7 +332,7 @@ def _measure(candidates: List[Tuple[str, Callable[[], torch.Tensor]]], handicap:
 def qkv_parts(x: torch.Tensor, w) -> Optional[torch.Tensor]:
     """The q/k/v product of a decoding batch as fp32 partial sums ``[S, M, N]`` for
     :func:`~fastgen_amd.kernels.ops.rope_kv_parts`, or None where they are not the way (``QKV_PARTS_ROWS``)."""
-    if not (force in (None, "tiled") and isinstance(w, StreamedMatrix) and w.packed is not None and x.dtype == torch.bfloat16
+    if not (force in (None, "large") and isinstance(w, StreamedMatrix) and w.packed is not None and x.dtype == torch.bfloat16
             and w.dtype == torch.bfloat16 and SKINNY_ROWS < x.shape[0] <= QKV_PARTS_ROWS and w.shape[1] % 64 == 0
             and _aligned(x, w.rows) and ops.gemm_large_takes(x, w.shape[0])):
         return None
@@ -403,12 +404,12 @@ def linear(x, w, out_dtype: Optional[torch.dtype] = None,
     handicap: Dict[str, float] = {}
     large_ok = (own and sw is not w and K % 64 == 0 and scaled is None and (not silu or (N % 16 == 0 and out_dtype == torch.bfloat16))
                 and ops.gemm_large_takes(x, N))
-    if large_ok and rows > SKINNY_ROWS and force in (None, "tiled") and (
+    if large_ok and rows > SKINNY_ROWS and (force == "large" or force is None and (
             rows > LARGE_ROWS or silu or (partials_ok and out_dtype == torch.bfloat16)
-            or (out_dtype == torch.float32 and N >= 64 * ops.compute_units())):
+            or (out_dtype == torch.float32 and N >= 64 * ops.compute_units()))):
         tile, l_splits = ops.large_plan(rows, N, K, silu, partials_ok and out_dtype == torch.bfloat16)
         return ops.gemm_large(x, sw, out_dtype, gated if silu else False, l_splits, tile)
-    tiled_ok = own and not large_ok and TILED_MIN_ROWS <= rows <= TILED_MAX_ROWS
+    tiled_ok = own and (not large_ok or force in ("tiled", "tiled256")) and TILED_MIN_ROWS <= rows <= TILED_MAX_ROWS
 
     def sums_cost(splits: int) -> float:
         """Milliseconds the consumer takes to read the partial sums beyond the first (at 4 TB/s)."""

@@ -282,22 +282,28 @@ def test_many_requests_decode_together_bfloat16(n_live, captured, tmp_path):
                  plain_logits(weights, cfg, tokens, torch.bfloat16), f"{n_live} live")
 
 
-@pytest.mark.parametrize("forced,packed", [("narrow", True), ("narrow", False), ("wide", True), ("wide", False),
-                                           ("tiled", True), ("tiled256", False), ("library", True), (None, True),
-                                           (None, False)])
-def test_every_kernel_that_may_be_chosen_gives_the_plain_logits(forced, packed, tmp_path, monkeypatch):
+@pytest.mark.parametrize("forced,packed,cfg", [("narrow", True, TINY_B), ("narrow", False, TINY_B), ("wide", True, TINY_B),
+                                               ("wide", False, TINY_B), ("tiled", True, TINY_B), ("tiled256", False, TINY_B),
+                                               ("library", True, TINY_B), (None, True, TINY_B), (None, False, TINY_B),
+                                               ("large", True, TINY_B), ("tiled", True, TINY_C), ("tiled256", True, TINY_C),
+                                               (None, True, TINY_C)])
+def test_every_kernel_that_may_be_chosen_gives_the_plain_logits(forced, packed, cfg, tmp_path, monkeypatch):
     """Which kernel takes a matrix product is measured at run time (``fastgen_amd.kernels.linear``), so which
     one an engine test meets depends on the machine.  Here the engine runs once under each kernel's name
     (taken wherever it is among the candidates of a product) and once as measured: whole prompts (up to 150
     rows), mixed steps, and 20 requests decoding together (17..32 rows), every position against the plain
     implementation.  ``packed``: with and without the second copy of the matrices in the streaming kernels'
-    order (a model too large for two copies runs without)."""
-    from fastgen_amd.kernels import linear
+    order (a model too large for two copies runs without).  TINY_B's k are multiples of 64, which the large tiles need,
+    TINY_C's are none."""
+    from fastgen_amd.kernels import linear, ops
 
     monkeypatch.setattr(linear, "force", forced)
     monkeypatch.setattr(linear, "choices", {})
     monkeypatch.setenv("FG_PACKED_WEIGHTS", "1" if packed else "0")
-    cfg = TINY_B
+    taken = set()
+    for name in ("gemm_tiled", "gemm_large"):
+        run = getattr(ops, name)
+        monkeypatch.setattr(ops, name, lambda *a, name=name, run=run, **k: taken.add(name) or run(*a, **k))
     weights = sharpen(plain_random_weights(cfg, 9))
     weights = {k: v.to(torch.bfloat16).float() for k, v in weights.items()}
     folder = save_model_folder(tmp_path / "forced", cfg, weights)
@@ -320,5 +326,7 @@ def test_every_kernel_that_may_be_chosen_gives_the_plain_logits(forced, packed, 
     got = run_trace(runner, trace, tokens)
     assert_close(got, plain_logits(weights, cfg, tokens), torch.bfloat16,
                  plain_logits(weights, cfg, tokens, torch.bfloat16), f"forced {forced}, 20 live")
+    large = packed and cfg is TINY_B and forced in (None, "large")
+    assert ("gemm_large" in taken) == large and (forced not in ("tiled", "tiled256") or taken == {"gemm_tiled"})
     if forced is None:
         assert linear.choices and set(linear.choices.values()) <= {"narrow", "wide", "tiled", "tiled256", "library"}
