@@ -20,6 +20,7 @@ in which the streaming kernels read it, which those kernels take.
 
 from __future__ import annotations
 
+import functools
 import itertools
 import os
 import weakref
@@ -329,15 +330,35 @@ def _measure(candidates: List[Tuple[str, Callable[[], torch.Tensor]]], handicap:
     return best
 
 
+@functools.lru_cache(maxsize=4096)
+def _large_way(M: int, N: int, K: int, ldx: int, gated: bool, partials: bool, wide_out: bool, forced: bool) -> Optional[Tuple[int, int]]:
+    """Tile and splits of k of a product that goes to the large tiles (``LARGE_ROWS``; ``forced``: wherever they can take it), or
+    None.  ``wide_out``: fp32 output."""
+    if M <= SKINNY_ROWS or not ops.gemm_large_takes(M, N, K, ldx) or (gated and (N % 16 or wide_out)):
+        return None
+    if not (forced or M > LARGE_ROWS or gated or partials or (wide_out and N >= 64 * ops.compute_units())):
+        return None
+    return ops.large_plan(M, N, K, gated, partials)
+
+
+@functools.lru_cache(maxsize=4096)
+def _qkv_way(M: int, N: int, K: int, ldx: int) -> Optional[Tuple[int, int]]:
+    """Tile and splits of a q/k/v product that leaves partial sums (``QKV_PARTS_ROWS``), or None."""
+    if not SKINNY_ROWS < M <= QKV_PARTS_ROWS or not ops.gemm_large_takes(M, N, K, ldx):
+        return None
+    tile, splits = ops.parts_plan(M, N, K)
+    return (tile, splits) if splits > 1 else None
+
+
 def qkv_parts(x: torch.Tensor, w) -> Optional[torch.Tensor]:
     """The q/k/v product of a decoding batch as fp32 partial sums ``[S, M, N]`` for
     :func:`~fastgen_amd.kernels.ops.rope_kv_parts`, or None where they are not the way (``QKV_PARTS_ROWS``)."""
-    if not (force in (None, "large") and isinstance(w, StreamedMatrix) and w.packed is not None and x.dtype == torch.bfloat16
-            and w.dtype == torch.bfloat16 and SKINNY_ROWS < x.shape[0] <= QKV_PARTS_ROWS and w.shape[1] % 64 == 0
-            and _aligned(x, w.rows) and ops.gemm_large_takes(x, w.shape[0])):
+    if force not in (None, "large") or not isinstance(w, StreamedMatrix) or w.packed is None:
         return None
-    tile, splits = ops.parts_plan(x.shape[0], *w.shape)
-    return ops.gemm_large(x, w.packed, k_splits=splits, tile=tile) if splits > 1 else None
+    way = _qkv_way(x.shape[0], *w.rows.shape, x.stride(0))
+    if way is None or not _aligned(x, w.rows):
+        return None
+    return ops.gemm_large(x, w.packed, k_splits=way[1], tile=way[0])
 
 
 def linear(x, w, out_dtype: Optional[torch.dtype] = None,
@@ -390,6 +411,12 @@ def linear(x, w, out_dtype: Optional[torch.dtype] = None,
         if h.dtype == torch.float32 and h.is_contiguous() and h.shape == (rows, N):
             return ops.gemm_skinny_residual(src, sw, h, norm_w, eps)
 
+    if own and rows > SKINNY_ROWS and sw is not w and force in (None, "large"):  # (no open norm: those have few rows)
+        way = _large_way(rows, N, K, x.stride(0), silu, partials_ok and out_dtype == torch.bfloat16, out_dtype == torch.float32,
+                         force is not None)
+        if way is not None:
+            return ops.gemm_large(x, sw, out_dtype, gated if silu else False, way[1], way[0])
+
     def library(m: StreamedMatrix) -> torch.Tensor:
         xin = scaled.materialize() if scaled is not None else x
         if out_dtype == torch.bfloat16:
@@ -402,14 +429,8 @@ def linear(x, w, out_dtype: Optional[torch.dtype] = None,
 
     candidates: List[Tuple[str, Callable[[StreamedMatrix], torch.Tensor]]] = []
     handicap: Dict[str, float] = {}
-    large_ok = (own and sw is not w and K % 64 == 0 and scaled is None and (not silu or (N % 16 == 0 and out_dtype == torch.bfloat16))
-                and ops.gemm_large_takes(x, N))
-    if large_ok and rows > SKINNY_ROWS and (force == "large" or force is None and (
-            rows > LARGE_ROWS or silu or (partials_ok and out_dtype == torch.bfloat16)
-            or (out_dtype == torch.float32 and N >= 64 * ops.compute_units()))):
-        tile, l_splits = ops.large_plan(rows, N, K, silu, partials_ok and out_dtype == torch.bfloat16)
-        return ops.gemm_large(x, sw, out_dtype, gated if silu else False, l_splits, tile)
-    tiled_ok = own and (not large_ok or force in ("tiled", "tiled256")) and TILED_MIN_ROWS <= rows <= TILED_MAX_ROWS
+    tiled_ok = own and TILED_MIN_ROWS <= rows <= TILED_MAX_ROWS and (
+        force in ("tiled", "tiled256") or sw is w or not ops.gemm_large_takes(rows, N, K, x.stride(0)))
 
     def sums_cost(splits: int) -> float:
         """Milliseconds the consumer takes to read the partial sums beyond the first (at 4 TB/s)."""

@@ -1312,15 +1312,32 @@ def parts_plan(M: int, N: int, K: int) -> Tuple[int, int]:
     return (64128 if small else 128128), next(splits, 1)
 
 
-def gemm_large_takes(x: torch.Tensor, N: int) -> bool:
-    """Whether offsets within a tile of :func:`gemm_large` fit 32 bits, and its tiles the grid."""
-    return (x.stride(0) >= x.shape[1] and 512 * x.stride(0) + 2 * x.shape[1] <= 4_000_000_000 and x.shape[1] <= 30_000_000
-            and -(-x.shape[0] // 128) * -(-N // 128) <= 1 << 27)
+@functools.lru_cache(maxsize=4096)
+def gemm_large_takes(M: int, N: int, K: int, ldx: int) -> bool:
+    """Whether :func:`gemm_large` takes ``x [M, K]`` of row stride ``ldx`` and a packed ``[N, K]``: whole steps of 64 k, offsets within a
+    tile that fit 32 bits, tiles that fit the grid."""
+    return (M > 0 and K > 0 and K % 64 == 0 and ldx >= K and ldx % 8 == 0 and 512 * ldx + 2 * K <= 4_000_000_000 and K <= 30_000_000
+            and -(-M // 128) * -(-N // 128) <= 1 << 27)
 
 
 def gemm_large_scratch(M: int, N: int) -> int:
     """Bytes of the partial sums that :func:`gemm_large` writes at most for up to ``M`` rows as :func:`large_plan` plans it."""
     return min(_LARGE_SPLITS * M * N * 4, 2 * compute_units() * 128 * 256 * 4)
+
+
+@functools.lru_cache(maxsize=4096)
+def _large_sizes(M: int, N: int, K: int, ldx: int, gated: bool, out_dtype: torch.dtype, k_splits: int, tile: Optional[int]) -> Tuple[int, int]:
+    """The tile of a product of :func:`gemm_large` and those that are not cut; other sizes are refused.  What depends on the
+    sizes alone is worked out once for them: a step of a few dozen rows waits for the host."""
+    _need(gemm_large_takes(M, N, K, ldx), "K must be a multiple of 64, rows 16-byte aligned, offsets of 32 bits")
+    if gated:
+        _need(N % 16 == 0 and out_dtype == torch.bfloat16 and k_splits == 1,
+              "the gate/up epilogue needs N % 16 == 0, bf16 output and one split")
+    _need(1 <= k_splits <= 64 and -(-(K // 64) // k_splits) * (k_splits - 1) < K // 64, "a split of k would be empty")
+    if tile is None:
+        tile = large_plan(M, N, K, gated)[0]
+    _need(tile in LARGE_TILES, f"tile must be one of {LARGE_TILES}")
+    return int(tile), large_whole_tiles(tile, M, N)
 
 
 def gemm_large(x: torch.Tensor, w: "PackedWeight", out_dtype: Optional[torch.dtype] = None, silu_mul_epilogue: bool = False,
@@ -1331,26 +1348,18 @@ def gemm_large(x: torch.Tensor, w: "PackedWeight", out_dtype: Optional[torch.dty
     ``[s * ceil(K / 64 / k_splits) * 64, ...)``."""
     _need(isinstance(w, PackedWeight) and x.dtype == torch.bfloat16 and x.dim() == 2, "gemm_large takes bfloat16 x [M, K], w packed")
     _gpu(x, w.data)
-    M, K = x.shape
-    N = w.shape[0]
-    _need(M > 0 and K % 64 == 0 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.stride(0) >= K and x.data_ptr() % 16 == 0,
-          "K must be a multiple of 64, rows 16-byte aligned")
+    (M, K), (ldx, unit), N, x_ptr = x.shape, x.stride(), w.n, x.data_ptr()
+    _need(unit == 1 and x_ptr % 16 == 0, "gemm_large: rows 16-byte aligned")
     w_ptr, _ = _weight_args(w, K, "gemm_large")
+    gated = bool(silu_mul_epilogue)
     out_dtype = out_dtype or torch.bfloat16
-    if silu_mul_epilogue:
-        _need(N % 16 == 0 and out_dtype == torch.bfloat16 and k_splits == 1,
-              "the gate/up epilogue needs N % 16 == 0, bf16 output and one split")
-    _need(1 <= k_splits <= 64 and -(-(K // 64) // k_splits) * (k_splits - 1) < K // 64, "a split of k would be empty")
-    if k_splits > 1:
-        out_dtype = torch.float32
-    if tile is None:
-        tile = large_plan(M, N, K, bool(silu_mul_epilogue))[0]
-    _need(tile in LARGE_TILES, f"tile must be one of {LARGE_TILES}")
-    cols = N // 2 if silu_mul_epilogue else N
-    y = torch.empty((k_splits, M, cols) if k_splits > 1 else (M, cols), dtype=out_dtype, device=x.device)
+    tile, whole = _large_sizes(M, N, K, ldx, gated, out_dtype, k_splits, tile)
+    cols = N // 2 if gated else N
+    shape, out_dtype = ((M, cols), out_dtype) if k_splits == 1 else ((k_splits, M, cols), torch.float32)
+    y = torch.empty(shape, dtype=out_dtype, device=x.device)
     st = _lib.load("gemm_large").fg_gemm_large(
-        _ptr(x), x.stride(0), w_ptr, _ptr(y), cols, ctypes.c_longlong(M * cols), k_splits, M, N, K, _code(y),
-        _gated_code(silu_mul_epilogue), int(tile), large_whole_tiles(tile, M, N), _stream(x))
+        ctypes.c_void_p(x_ptr), ldx, w_ptr, _ptr(y), cols, ctypes.c_longlong(M * cols), k_splits, M, N, K, _code(y),
+        _gated_code(silu_mul_epilogue), tile, whole, _stream(x))
     _check(st, "gemm_large")
     return y
 
