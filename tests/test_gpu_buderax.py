@@ -300,7 +300,7 @@ def test_command_lines(cases, tmp_path):
 
 
 @pytest.mark.parametrize("counts,D,F", [((0, 64, 65, 128, 129, 256, 300, 1, 513), 192, 72 * 8), ((700,), 64, 64), ((3,) * 70 + (260,), 128, 136 * 8),
-                                        ((1,) * 9, 320, 64)])
+                                        ((1,) * 9, 320, 64), ((5,) * 3 + (0, 128) * 9 + (64, 1), 64, 136 * 8)])
 @pytest.mark.parametrize("tile_rows", [128, 256])
 def test_large_tiles_of_experts_give_the_rows_bits(counts, D, F, tile_rows):
     """Packed experts with sizes in multiples of 64 (the large tiles) against matrices stored row by row, where experts have as
