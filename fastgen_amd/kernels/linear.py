@@ -59,15 +59,19 @@ WIDE_ROWS = ops.SKINNY_MAX_ROWS  # the wide kernel (64 columns a workgroup): up 
 # not take the matrix (us at 192 rows, o and down of 4,096 x 4,096 and x 14,336: 24 / 54 against 17 / 43)
 TILED_MIN_ROWS, TILED_MAX_ROWS = 65, 512
 # The large tiles (:func:`~fastgen_amd.kernels.ops.gemm_large`) take any number of rows of a packed matrix and run without being
-# measured, so that a first step takes no longer and every process takes the same kernel, where they are the faster ones (us):
-# * beyond this many rows: of 130 products of 520 to 4,096 rows (1,024 to 28,672 columns, 768 to 14,336 of k) in 110, 1.2 times on
-#   average (gated 1.04 to 1.6: the gate and up rows do not go through memory), and slower by up to 10 % where the library's tiles happen
-#   to fill the chip (squares of 4,096);
-# * from 17 rows on gated products (28,672 x 4,096 at 64 rows 44.5 against 51 of the wide kernel and 55 of the library; 16,384 x 3,072
-#   at 17 to 128 rows 23 to 34 against 24 to 31, at 160 to 512 29 to 47 against 35 to 61), products that may leave partial sums (4,096 x
-#   14,336 at 17 / 64 / 192 rows 23.1 / 26.3 / 43 against 23.5 / 32 / 54; 2,048 x 2,048 at 256 10.6 against 9.9 is where it is not so), and
-#   wide fp32 outputs (logits of 128,256 x 4,096 at 64 rows 218 against 224).
-# A plain product of fewer rows has no splits to fill the chip with and goes the other ways (6,144 x 4,096 at 65 rows 34 against
+# measured, so that a first step takes no longer and every process takes the same kernel, where they are the faster ones (`_large_way`).
+# Times against the kernel that is measured to be the fastest otherwise, of 44 matrices (512 to 128,256 columns, 512 to 14,336 of k) at 17 to 4,096 rows, with the
+# norm behind where the result may be partial sums:
+# * gated products: 0.45 to 1.0 beyond 64 rows (1.02 to 1.1 in 28 of 260, where the library's tiles happen to fill the chip).  Up to 64 rows they are
+#   bound by how many workgroups read the matrix, 64 rows x 128 columns each: from 80 columns a compute unit on 0.91 to 1.0; fewer 1.05 to
+#   1.17 (the wide kernel's workgroups are twice as many, and it takes them), but for short k beyond 32 rows (k = 1,024: 0.78 to 1.02);
+# * products that may leave partial sums: 0.4 to 1.0 at 33 to 512 rows (1.02 to 1.1 in 22 of 300).  Up to 32 rows 0.91 to 1.04 from 2^24
+#   elements of the matrix on, with fewer 1.0 to 1.17 (the wide kernel's);
+# * wide fp32 outputs (logits) 0.7 to 1.02 from 96 columns a compute unit on; 16,384 x 2,048 is 1.1 to 1.19 up to 64 rows, and at 129 to 384 rows, where
+#   the library has tiles of 160 and 192 rows, 32,000 columns are 0.8 to 1.17, 50,304 and more 0.74 to 1.05;
+# * beyond LARGE_ROWS plain products and partial sums too: 0.65 to 1.1, 0.96 on average.  Where k is long and one round of tiles leaves a fifth of the compute
+#   units or more without one, the library, which cuts k there, is 1.09 times as fast (1.21 at 3,000 x 2,048 x 8,192, 192 tiles).
+# A plain product of fewer rows has no splits to fill the chip with and goes the other ways (6,144 x 4,096 at 65 rows 34 us against
 # 23 of the library, at 320 36 against 30).
 LARGE_ROWS = TILED_MAX_ROWS
 # The q/k/v product of up to this many rows leaves partial sums to the kernel that rotates and writes the cache; both together, us,
@@ -332,13 +336,27 @@ def _measure(candidates: List[Tuple[str, Callable[[], torch.Tensor]]], handicap:
 
 @functools.lru_cache(maxsize=4096)
 def _large_way(M: int, N: int, K: int, ldx: int, gated: bool, partials: bool, wide_out: bool, forced: bool) -> Optional[Tuple[int, int]]:
-    """Tile and splits of k of a product that goes to the large tiles (``LARGE_ROWS``; ``forced``: wherever they can take it), or
-    None.  ``wide_out``: fp32 output."""
+    """Tile and splits of k of a product that goes to the large tiles (``LARGE_ROWS``; ``forced``: wherever they can take it), ``(0,
+    splits)`` for the wide kernel, or None: one of those that are measured.  ``wide_out``: fp32 output."""
     if M <= SKINNY_ROWS or not ops.gemm_large_takes(M, N, K, ldx) or (gated and (N % 16 or wide_out)):
         return None
-    if not (forced or M > LARGE_ROWS or gated or partials or (wide_out and N >= 64 * ops.compute_units())):
-        return None
-    return ops.large_plan(M, N, K, gated, partials)
+    units = ops.compute_units()
+    if forced or M > LARGE_ROWS:
+        takes = True
+    elif gated:
+        takes = M > 64 or N >= 80 * units or (M > 32 and K <= 1024)
+    elif partials:
+        takes = M > 32 or N * K >= 1 << 24
+    else:
+        takes = wide_out and N >= (192 if 128 < M <= 384 else 96) * units
+    if not takes:
+        return (0, k_splits_for(N, K, M) if partials else 1) if gated or partials else None
+    tile, splits = ops.large_plan(M, N, K, gated, partials)
+    if M > LARGE_ROWS and not (forced or gated or wide_out) and K >= 4096 * splits:
+        tiles = -(-M // (tile // 1000)) * -(-N // (tile % 1000)) * splits
+        if tiles <= 0.8 * units:
+            return None
+    return tile, splits
 
 
 @functools.lru_cache(maxsize=4096)
@@ -414,8 +432,10 @@ def linear(x, w, out_dtype: Optional[torch.dtype] = None,
     if own and rows > SKINNY_ROWS and sw is not w and force in (None, "large"):  # (no open norm: those have few rows)
         way = _large_way(rows, N, K, x.stride(0), silu, partials_ok and out_dtype == torch.bfloat16, out_dtype == torch.float32,
                          force is not None)
-        if way is not None:
+        if way is not None and way[0]:
             return ops.gemm_large(x, sw, out_dtype, gated if silu else False, way[1], way[0])
+        if way is not None:
+            return ops.gemm_skinny(x, sw, out_dtype, gated if silu else False, way[1], wide=True)
 
     def library(m: StreamedMatrix) -> torch.Tensor:
         xin = scaled.materialize() if scaled is not None else x

@@ -1246,16 +1246,23 @@ def gemm_tiled(x: torch.Tensor, w, out_dtype: Optional[torch.dtype] = None,
 
 # rows and columns of x and of the output that a workgroup of gemm_large takes (1,000 * rows + columns)
 LARGE_TILES = (256256, 256192, 128256, 128192, 128128, 64128)
-# What a round of tiles takes, in microseconds: for every 64 of k, as much more for every 64 of k times the share of the
-# places that have a tile, and beside k.  First: one tile a compute unit; second: two (of the tiles that fit twice), or the halves
-# behind the last round.  Fitted to 1,739 products (130 to 4,096 rows, 1,024 to 28,672 columns, 768 to 14,336 of k, 1 to 4 splits) with
-# 3 to 9 % about them; the plan that is the fastest by them takes 0.6 % longer than the fastest one on average.  (8 us of the halves' rest
-# are added: in a model, 28 layers of other matrices between, 1,278 x 16,384 x 3,072 and 2,000 x 11,264 x 2,048 in halves made the
-# step 0.8 and 2 % longer than tiles of 128 rows, where they measured alike by themselves.)
-_LARGE_COST = {256256: ((0.936, 0.405, 8.3), (0.605, 0.24, 11.7)), 256192: ((0.723, 0.288, 9.6), (0.356, 0.265, 14.2)),
-               128256: ((0.468, 0.348, 7.0), (0.643, 0.865, 13.3)), 128192: ((0.385, 0.273, 5.9), (0.607, 0.591, 10.2)),
-               128128: ((0.296, 0.177, 4.3), (0.476, 0.459, 6.9))}
-_LARGE_GATED = 0.92  # of tiles that fit twice, against those that do not: one's activations run beside the other's products
+# What a round of tiles takes, in microseconds: for every 64 of k, as much more for every 64 of k times the share of the places that have a
+# tile, and beside k.  One entry for as many workgroups a compute unit as there are at once (tiles of 256 rows one, of 128 rows two, of 64
+# rows three); then with an activation, whose tiles of 128 and 64 rows run beside another's products (more than one a compute unit: as if 0.9 of the
+# places had one at least, 320 x 28,672 x 4,096 with its 336 tiles of 128 x 256 takes 110 us, not 84).  Fitted to 7,547 products (65 to 4,096 rows, 512
+# to 32,768 columns, 512 to 16,384 of k, 1 to 8 splits); the plan that is the fastest by them takes longer than the fastest one by 0.3 and 1.5 % on
+# average with an activation (up to 512 rows and beyond), 0.4 and 1.3 % plain, 1.8 and 2.6 % with splits.  Without the tiles of 64 rows it was 16 %, 23 and 8 %, 15 and 7 %: a small
+# product has too few larger tiles (us, with the norm behind, without / with them / library: 100 x 1,024 x 2,816 12.9 / 10.2 / 12.6,
+# 400 x 512 x 1,408 12.6 / 9.9 / 10.1, 512 x 2,048 x 2,048 19.9 / 17.2 / 17.3, 640 x 3,072 x 2,048 21.6 / 16.8 / 16.9).
+_LARGE_COST = {256256: ((0.933, 0.437, 10.6),), 256192: ((0.757, 0.324, 9.4),), 128256: ((0.642, 0.227, 5.5), (0.699, 0.96, 16.2)),
+               128192: ((0.563, 0.207, 4.7), (0.712, 0.605, 13.5)), 128128: ((0.388, 0.211, 4.7), (0.469, 0.579, 11.0)),
+               64128: ((0.287, 0.185, 2.9), (0.361, 0.48, 6.1), (0.469, 0.678, 8.8))}
+_LARGE_COST_GATED = {256256: ((0.972, 0.387, 10.2),), 128256: ((0.633, 0.258, 4.8), (0.661, 0.979, 8.5)),
+                     128128: ((0.361, 0.237, 3.9), (0.44, 0.583, 6.6)), 64128: ((0.259, 0.189, 2.8), (0.289, 0.528, 4.6), (0.511, 0.572, 5.2))}
+# The halves behind the last round of tiles of 256 rows.  (8 us of the rest are added: in a model, 28 layers of other matrices between,
+# 1,278 x 16,384 x 3,072 and 2,000 x 11,264 x 2,048 in halves made the step 0.8 and 2 % longer than tiles of 128 rows, where they measured alike by
+# themselves.)
+_LARGE_HALVES = {256256: (0.605, 0.24, 11.7), 256192: (0.356, 0.265, 14.2)}
 _LARGE_SPLITS = 8
 
 
@@ -1269,28 +1276,30 @@ def large_whole_tiles(tile: int, M: int, N: int) -> int:
 
 def large_cost(tile: int, M: int, N: int, K: int, splits: int = 1, gated: bool = False) -> float:
     """About how long :func:`gemm_large` takes with a tile, in microseconds, and its consumer for the partial sums."""
-    one, two = _LARGE_COST[tile]
+    costs = (_LARGE_COST_GATED if gated else _LARGE_COST)[tile]
     steps, units = -(-(K // 64) // splits), compute_units()
     tiles = -(-M // (tile // 1000)) * -(-N // (tile % 1000)) * splits
     took = lambda cost, fill: steps * (cost[0] + cost[1] * fill) + cost[2]
-    sums = 1.0 + 1.5 * (4 * splits - 2) * M * N / 4e6 if splits > 1 else 0.0  # written and read at 4 TB/s, and half as much
-    if tile >= 256000:
-        whole = large_whole_tiles(tile, M, N)
-        rounds, left = divmod(whole or tiles, units)
-        last = took(two, 2 * (tiles - whole) / units) if whole else took(one, left / units) if left else 0.0
-        return rounds * took(one, 1.0) + last + sums
-    rounds, left = divmod(tiles, 2 * units)
-    last = 0.0 if not left else took(one, left / units) if left <= units else took(two, left / (2 * units))
-    return (rounds * took(two, 1.0) + last) * (_LARGE_GATED if gated else 1.0) + sums
+    sums = 1.0 + 2.0 * (4 * splits - 2) * M * N / 4e6 if splits > 1 else 0.0  # written and read at 4 TB/s, and as much again
+    whole = large_whole_tiles(tile, M, N)
+    rounds, left = divmod(whole or tiles, len(costs) * units)
+    last = 0.0
+    if whole:
+        last = took(_LARGE_HALVES[tile], 2 * (tiles - whole) / units)
+    elif left:
+        each = -(-left // units)  # workgroups a compute unit in the last round
+        last = took(costs[each - 1], max(left / (each * units), 0.9 if gated and each > 1 else 0.0))
+    return rounds * took(costs[-1], 1.0) + last + sums
 
 
 @functools.lru_cache(maxsize=4096)
 def large_plan(M: int, N: int, K: int, gated: bool = False, partials: bool = False) -> Tuple[int, int]:
-    """The tile that :func:`gemm_large` is fastest with, and, where its result may be partial sums, the splits of k: each of
-    512 at least, none empty, and no more workgroups than have a place at once.  Up to 64 rows the tile of as many, and as many splits up
-    to 8 as there may be (us at 64 rows with 4 and 8, the sums read back: 4,096 x 14,336 30 / 26.3, 4,096 x 4,096 12.8 / 12.1; with 16 31.3)."""
+    """The tile that :func:`gemm_large` is fastest with, and, where its result may be partial sums, the splits of k: none empty, each of
+    320 at least (a small product's few tiles are bound by the steps of one), and no more workgroups than have a place at once.  Up to 64 rows the
+    tile of as many, and as many splits up to 8, of 512 at least, as there may be (us at 64 rows with 4 and 8, the sums read back: 4,096 x 14,336 30 / 26.3, 4,096 x 4,096 12.8 / 12.1; with 16 31.3)."""
     steps, places = K // 64, 2 * compute_units()
-    may = [s for s in (2, 3, 4, 6, 8) if partials and not gated and steps // s >= 8 and -(-steps // s) * (s - 1) < steps]
+    least = 8 if M <= 64 else 5
+    may = [s for s in (2, 3, 4, 6, 8) if partials and not gated and steps // s >= least and -(-steps // s) * (s - 1) < steps]
     fits = lambda t, s: -(-M // (t // 1000)) * -(-N // (t % 1000)) * s <= places
     if M <= 64:
         return 64128, max((s for s in may if s in (2, 4, 8) and fits(64128, s)), default=1)
@@ -1317,7 +1326,7 @@ def gemm_large_takes(M: int, N: int, K: int, ldx: int) -> bool:
     """Whether :func:`gemm_large` takes ``x [M, K]`` of row stride ``ldx`` and a packed ``[N, K]``: whole steps of 64 k, offsets within a
     tile that fit 32 bits, tiles that fit the grid."""
     return (M > 0 and K > 0 and K % 64 == 0 and ldx >= K and ldx % 8 == 0 and 512 * ldx + 2 * K <= 4_000_000_000 and K <= 30_000_000
-            and -(-M // 128) * -(-N // 128) <= 1 << 27)
+            and -(-M // 64) * -(-N // 128) <= 1 << 27)
 
 
 def gemm_large_scratch(M: int, N: int) -> int:

@@ -77,34 +77,40 @@ def test_sizes_are_worked_out_once(calls, monkeypatch):
     for name in ("large_whole_tiles", "large_plan", "parts_plan"):
         work = getattr(ops, name)
         monkeypatch.setattr(ops, name, lambda *a, name=name, work=work: asked.append(name) or work(*a))
-    x, w = on_gpu(45, 1088), linear.StreamedMatrix(on_gpu(1040, 1088), packed(1040, 1088))
+    x, w = on_gpu(70, 1088), linear.StreamedMatrix(on_gpu(1040, 1088), packed(1040, 1088))
     for _ in range(3):
         linear.linear(x, w, partials_ok=True)
         linear.linear(x, w, epilogue="silu_mul")
         linear.qkv_parts(x, w)
+        first = list(asked) if not calls[3:] else first
     assert names(calls) == {"fg_gemm_large"} and len(calls) == 9
-    assert sorted(asked) == ["large_plan"] * 2 + ["large_whole_tiles"] * 2 + ["parts_plan"]  # (two of the three are one tile and split)
+    assert set(asked) == {"large_whole_tiles", "large_plan", "parts_plan"} and asked == first
 
 
-def test_what_goes_to_the_large_tiles(calls, monkeypatch):
-    """Rows, k, strides, alignment and epilogues that they take, and those that go other ways or are refused as before."""
+def test_which_kernel_takes_a_product(calls, monkeypatch):
+    """Rows, k, strides, alignment and epilogues that the large tiles and the wide kernel take without a measurement, and those that go
+    other ways or are refused."""
     monkeypatch.setattr(linear, "_settle", lambda what, n, k, rows, candidates, *a, **b: candidates[-1][0])
     monkeypatch.setattr(torch.nn.functional, "linear", lambda x, w: on_gpu(x.shape[0], w.shape[0]))
 
-    def large(M, N, K, more, ldx=0, matrix=None):
+    def took(M, N, K, more, ldx=0, matrix=None):
         calls.clear()
         x = on_gpu(M, ldx or K)[:, :K].as_subclass(OnGpu)
         linear.linear(x, linear.StreamedMatrix(on_gpu(N, K), packed(N, K)) if matrix is None else matrix, **more)
-        return "fg_gemm_large" in names(calls)
+        entries = [entry for entry in names(calls) if entry in (large, wide)]
+        return entries[0] if entries else False
 
+    large, wide = "fg_gemm_large", "fg_gemm_skinny64"
     parts, gated, f32 = {"partials_ok": True}, {"epilogue": "gelu_tanh_mul"}, {"out_dtype": torch.float32}
-    for M, N, K, more, want in [(16, 64, 64, gated, False), (17, 64, 64, gated, True), (17, 64, 72, gated, False),
-                                (17, 64, 72, parts, False), (17, 40, 128, parts, True), (512, 64, 64, {}, False), (513, 64, 64, {}, True),
-                                (513, 64, 96, {}, False), (40, 16384, 64, f32, True), (40, 16383, 64, f32, False), (513, 64, 64, f32, True),
-                                (40, 64, 64, dict(parts, **f32), False)]:
-        assert large(M, N, K, more) == want, (M, N, K, more)
-    assert large(20, 64, 64, gated, ldx=72) and not large(20, 64, 64, gated, ldx=68)
-    assert not large(20, 64, 64, gated, matrix=on_gpu(64, 64))  # no packed copy
+    for M, N, K, more, want in [(16, 64, 64, gated, False), (32, 64, 64, gated, wide), (33, 64, 64, gated, large), (17, 20480, 64, gated, large),
+                                (64, 64, 1088, gated, wide), (65, 64, 1088, gated, large), (40, 64, 72, gated, False),
+                                (33, 64, 72, parts, False), (33, 40, 128, parts, large), (32, 40, 128, parts, wide), (17, 4096, 4096, parts, large),
+                                (512, 64, 64, {}, False), (513, 64, 64, {}, large), (513, 64, 96, {}, False), (513, 64, 4096, {}, False),
+                                (513, 64, 4096, f32, large), (40, 24576, 64, f32, large), (40, 24575, 64, f32, False), (129, 24576, 64, f32, False),
+                                (385, 24576, 64, f32, large), (129, 49152, 64, f32, large), (513, 64, 64, f32, large), (40, 64, 64, dict(parts, **f32), False)]:
+        assert took(M, N, K, more) == want, (M, N, K, more)
+    assert took(40, 64, 64, gated, ldx=72) == large and not took(40, 64, 64, gated, ldx=68)
+    assert not took(40, 64, 64, gated, matrix=on_gpu(64, 64))  # no packed copy
     x = on_gpu(20, 64 + 8)
     for bad in (lambda: ops.gemm_large(x[:, :40], packed(64, 40)), lambda: ops.gemm_large(x[:, 1:65], packed(64, 64)),
                 lambda: ops.gemm_large(x[:, :64], packed(64, 64), k_splits=2), lambda: ops.gemm_large(x[:, :64], packed(72, 64), None, True),
@@ -130,3 +136,21 @@ def test_parts_plan_leaves_whole_splits_and_a_workgroup_a_unit(monkeypatch):
                 assert splits == 1 or (wgs * splits <= 256 and steps // splits >= 6 and -(-steps // splits) * (splits - 1) < steps)
                 cut += splits > 1
     assert cut > 100
+
+
+@pytest.mark.parametrize("gated,partials", [(False, False), (False, True), (True, False)])
+def test_large_plan_fits(monkeypatch, gated, partials):
+    """Whatever the sizes: a tile that the kernel has, no empty split of k, no more workgroups than places where k is cut, and
+    partial sums within the room that is kept for them; more than 64 rows of a small product go to tiles of 64 rows."""
+    monkeypatch.setattr(ops, "_n_cus", 256)
+    small = 0
+    for M in (17, 64, 65, 100, 128, 129, 300, 512, 513, 1000, 2049, 4096, 16384):
+        for N in (16, 512, 1040, 2048, 4096, 11264, 28672):
+            for K in (64, 320, 704, 1408, 2048, 4096, 14336):
+                tile, splits = ops.large_plan(M, N, K, gated, partials)
+                assert tile in ops.LARGE_TILES and (not gated or tile % 1000 != 192)
+                steps, tiles = K // 64, -(-M // (tile // 1000)) * -(-N // (tile % 1000))
+                assert splits == 1 or (partials and -(-steps // splits) * (splits - 1) < steps and tiles * splits <= 512 and steps // splits >= 5
+                                       and splits * M * N * 4 <= ops.gemm_large_scratch(M, N))
+                small += M > 64 and tile == 64128
+    assert small > 50
