@@ -247,7 +247,7 @@ def _buderax_kernels(z: dict, rows: int) -> dict:
     x = rnd(rows, D) * 20
     router, bias = rnd(E, D).float(), rnd(E).float()
     wg, wu, wd = rnd(E, F, D), rnd(E, F, D), rnd(E, D, F)
-    tile_rows = expert_tile_rows(rows * top / E, min(D, F), E * -(-F // 128) if D % 64 == F % 64 == 0 else 0)
+    tile_rows = expert_tile_rows(rows * top / E, E, D, F)
     wg, wu, wd = (ops.pack_experts(w) for w in (wg, wu, wd))  # as a model keeps them
     choice, weight = ops.moe_route(x, router, bias, top)
     sorted_, tiles = ops.moe_sort(choice, E, tile_rows)
@@ -807,7 +807,7 @@ def _sodotar_kernels(z: dict, rows: int, context: int) -> dict:
     put("moe_route (buderax)", lambda: ops.moe_route(xr, r2, None, top), r2.numel() * 4 + rows * D * 2)
     # the experts' first product with the limited activation, beside the same with SiLU
     choice, _ = ops.moe_route(xr, r2, None, top)
-    tile_rows = expert_tile_rows(rows * top / E, D, E * -(-F // 128) if D % 64 == F % 64 == 0 else 0)
+    tile_rows = expert_tile_rows(rows * top / E, E, D, F)
     sorted_, tiles = ops.moe_sort(choice, E, tile_rows)
     wg, wu = ops.pack_experts(rnd(E, F, D)), ops.pack_experts(rnd(E, F, D))  # as a model keeps them
     used = min(E, rows * top)

@@ -37,25 +37,29 @@ from ..config.layout import PartSpec
 from .base import MATRIX, VECTOR, FeedForward, TensorSpec, build_part, place, register_part
 
 
-def expert_tile_rows(per_expert: float, least_k: int, large: int = 0) -> int:
-    """Rows of one expert a tile of the matrix-core kernels holds, by the rows an expert gets on average and the smaller
-    of the two products' k: 16 for few rows (decode: an expert's matrices are read once for its rows), 32 and 128
-    where the experts get so many rows each that their matrices would otherwise be read many times over; from 128 on
-    the rows of x go through LDS.  ``large``: where packed matrices have sizes in multiples of 64, the workgroups of 128 channels
-    that one tile of every expert makes; those go to the large tiles (``csrc/tile_product.h``), which take a tile of up to 64
-    and of up to 128 rows as one of that many, so 128 from 10 rows an expert on, and 256 while most experts then have one tile and
-    there are workgroups for most compute units.
+def expert_tile_rows(per_expert: float, n_experts: int, dim: int, hidden: int) -> int:
+    """Rows of one expert a tile of the matrix-core kernels holds, by the rows an expert gets on average: 16 for few rows (decode: an
+    expert's matrices are read once for its rows), 32 and 128 where the experts get so many rows each that their matrices would
+    otherwise be read many times over; from 128 on the rows of x go through LDS.  Matrices with sizes in multiples of 64 go to the
+    large tiles (``csrc/tile_product.h``), which take a tile of up to 64 and of up to 128 rows as one of that many, so 128 from 14 rows an
+    expert on, with many experts from 10; and 256 while most experts have one or two such tiles, if there are workgroups for most compute units and k is
+    long enough for a compute unit's only workgroup.
 
-    Measured (us, gate_up + down, packed, 32 experts of 768 x 2048, top 4; tiles of 16 / 32 / 128 / 256 rows): 8 rows an
-    expert 63 / 66 / 64 / 68, 12: 67 / 68 / 64 / 67, 16: 84 / 73 / 64 / 67, 128: - / - / 101 / 98, 187: - / - / 107 / 107,
-    256: - / - / 140 / 128, 512: - / - / 220 / 214, 1,024: - / - / 393 / 416; 64 of 1,408 x 2048, top 6, 140: 343 / 307 (128 / 256),
-    768: 957 / 962; 16 of 704 x 1024, top 2 (96 workgroups), 8: 17.8 / 18.1 / 20.0 / 24.2, 12: 21.2 / 21.1 / 20.1 / 24.3, 128: 36 / 61
-    (128 / 256).  Other sizes (16 / 32 / 128): 12 rows an expert 72 / 74 / -, 19: 95 / 81 / -, 25: 112 / 88 / 68, 50: 150 / 128 / 73."""
-    if large and per_expert >= 10:
-        return 256 if 112 <= per_expert <= 640 and large >= 170 else 128
-    if per_expert >= 24 and least_k >= 32:
+    Measured (us, sort, gate_up and down, packed, rows dealt by a random router), tiles of 16 / 32 / 128 rows at 10 and at 14 rows an expert: 32 experts of 768 x
+    2048 68 / 70 / 64, 70 / 72 / 66; 60 of 1,408 x 2048 199 / 207 / 190, 220 / 217 / 193; 128 of 768 x 2048 237 / 238 / 219, 263 / 247 / 222; 8 of 3,584 x
+    2048 74 / 78 / 80, 93 / 80 / 80; 16 of 2,048 x 4096 151 / 153 / 164, 172 / 158 / 165; 16 of 704 x 1024 24 / 22 / 24, 25 / 22 / 23; 8 of 1,024 x 1024
+    19 / 21 / 20, 20 / 22 / 21; 32 of 2,048 x 1024 84 / 81 / 93, 88 / 84 / 93.
+    Tiles of 128 / 256 rows at 128, 200, 256 and 320 rows: 32 of 768 x 2048 107 / 102, 121 / 116, 144 / 144 (rows dealt evenly 140 / 128), 168 / 193; 16 of 2,048 x 4096 236 /
+    189, 236 / 216, 320 / 314, 313 / 404; 60 of 1,408 x 2048 298 / 294, 330 / 343, 412 / 419, 460 / 596; 32 of 2,048 x 1024 131 / 141, 131 / 161, 175 / 197,
+    188 / 249; 8 of 3,584 x 2048 114 / 134, 114 / 148, 143 / 167, 159 / 197.  Sizes that are no multiples of 64 (16 / 32 / 128): 12 rows 72 / 74 / -,
+    19: 95 / 81 / -, 25: 112 / 88 / 68, 50: 150 / 128 / 73."""
+    if dim % 64 == 0 and hidden % 64 == 0:
+        if 112 <= per_expert <= 288 and n_experts >= 16 and n_experts * -(-hidden // 128) >= 170 and dim >= 2048:
+            return 256
+        return 128 if per_expert >= (10 if n_experts >= 32 else 14) else 16
+    if per_expert >= 24 and min(dim, hidden) >= 32:
         return 128
-    return 32 if per_expert >= 14 and not large else 16
+    return 32 if per_expert >= 14 else 16
 
 
 class MoE(FeedForward):
@@ -162,9 +166,7 @@ class MoE(FeedForward):
     def tile_rows(self, n_rows: int) -> int:
         if self.w_gate.dtype != torch.bfloat16 or self.dim % 8:
             return 16
-        hidden = self.w_down.shape[2]
-        large = self.n_experts * -(-hidden // 128) if self.dim % 64 == 0 and hidden % 64 == 0 else 0
-        return expert_tile_rows(n_rows * self.top / self.n_scored, min(self.dim, hidden), large)
+        return expert_tile_rows(n_rows * self.top / self.n_scored, self.n_experts, self.dim, self.w_down.shape[2])
 
     def forward(self, x: torch.Tensor, plus: Optional[torch.Tensor] = None, sums: bool = False):
         """fp32 ``[1, T, dim]``: the experts' weighted sum (plus ``plus``, rows that go to the

@@ -154,3 +154,15 @@ def test_large_plan_fits(monkeypatch, gated, partials):
                                        and splits * M * N * 4 <= ops.gemm_large_scratch(M, N))
                 small += M > 64 and tile == 64128
     assert small > 50
+
+
+def test_expert_tile_rows():
+    """Tiles of few rows while the experts get few, of 64 to 128 rows beyond, of 256 for one or two a expert where enough workgroups with a
+    long k are left; sizes that the large tiles do not take keep their tiles."""
+    from fastgen_amd.parts.moe import expert_tile_rows
+
+    for per, E, D, F, want in [(9.9, 32, 2048, 768, 16), (10, 32, 2048, 768, 128), (111, 32, 2048, 768, 128), (112, 32, 2048, 768, 256),
+                               (288, 32, 2048, 768, 256), (289, 32, 2048, 768, 128), (13, 8, 2048, 3584, 16), (14, 8, 2048, 3584, 128),
+                               (150, 8, 2048, 3584, 128), (150, 32, 1024, 2048, 128), (150, 16, 4096, 2048, 256), (150, 16, 2048, 704, 128),
+                               (13, 4, 96, 100, 16), (14, 4, 96, 100, 32), (24, 4, 96, 100, 128), (24, 4, 96, 24, 32)]:
+        assert expert_tile_rows(per, E, D, F) == want, (per, E, D, F)
