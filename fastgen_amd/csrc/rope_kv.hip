@@ -266,8 +266,7 @@ extern "C" int fg_rope_kv_parts(const float* parts, int n_parts, void* q_out, co
 #define LAUNCH(U)                                                                                                          \
   rope_kv_parts_kernel<U><<<grid, ROPE_PARTS_THREADS, 0, stream>>>(parts, (size_t)n_tokens * chunks * 8, n_parts,          \
       (bf16_t*)q_out, table, slots, (bf16_t*)k_pages, (bf16_t*)v_pages, n_heads, n_kv, hd, rotary_dim, page_size, value_from_key)
-  if (n_parts % 8 == 0) LAUNCH(8);
-  else if (n_parts % 4 == 0) LAUNCH(4);
+  if (n_parts % 4 == 0) LAUNCH(4);  // (the plan of the product before gives 2 to 4 parts)
   else if (n_parts % 2 == 0) LAUNCH(2);
   else LAUNCH(1);
 #undef LAUNCH

@@ -72,18 +72,25 @@ def test_family_shape_under_every_cut(family, dtype):
 
 
 @pytest.mark.parametrize("n_live", [24, 61, 75, 100])
-def test_family_shape_many_requests_decode_together(family, n_live):
+def test_family_shape_many_requests_decode_together(family, n_live, monkeypatch):
     """The benchmark's decode path at its layer sizes: dozens of live requests of different lengths,
     prompts fed in portions, then 40 decode steps of all together, eagerly and from captured steps
-    (61 requests in a step recorded for 64, 75 in one for 80, 100 in one for 128): the wide products with k splits at
-    17..64 rows and, for o and down, at 65..128 (gate/up with its activation up to 80), the library's q/k/v product with the rotation kernel,
-    split attention with dozens of items and both combine kernels.  Every position against the plain implementation, which for this many tokens
+    (61 requests in a step recorded for 64, 75 in one for 80, 100 in one for some more): the large tiles at 17..128 rows (gate/up with its
+    activation, o and down with k splits, q/k/v with k splits and the kernel that adds the sums up and rotates), split attention with
+    dozens of items and both combine kernels.  Every position against the plain implementation, which for this many tokens
     runs its torch operations on the GPU; the fixture pins such a run to the CPU run on one request."""
     import numpy as np
 
+    from fastgen_amd.kernels import ops
+
+    rows_of = {"gemm_large": set(), "rope_kv_parts": set()}  # of x, of the parts
+    for name in rows_of:
+        run = getattr(ops, name)
+        monkeypatch.setattr(ops, name, lambda a, *b, name=name, run=run, **k: rows_of[name].add(a.shape[-2]) or run(a, *b, **k))
+
     FAMILY = family["config"]
     if FAMILY["hidden_size"] != 4096 and n_live not in (61, 100):
-        pytest.skip("the other widths take the two sizes that cover the wide products and the library's")
+        pytest.skip("the other widths take the two sizes that cover tiles of 64 and of 128 rows")
     w_gpu = {k: v.to("cuda:0") for k, v in family["weights"].items()}
     rng = np.random.default_rng(n_live)
     n_decode = 40
@@ -103,4 +110,7 @@ def test_family_shape_many_requests_decode_together(family, n_live):
         got = run_trace(runner, trace, tokens)
         assert bool(runner.graphs) == captured
         assert_close(got, want, torch.bfloat16, noise, f"{n_live} live, captured={captured}")
+        for name, met in rows_of.items():
+            assert {c for c, _ in runner.graphs} <= met if captured else n_live in met, (name, met)
+            met.clear()
         del runner
