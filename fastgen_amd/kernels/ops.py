@@ -1259,10 +1259,10 @@ _LARGE_COST = {256256: ((0.933, 0.437, 10.6),), 256192: ((0.757, 0.324, 9.4),), 
                64128: ((0.287, 0.185, 2.9), (0.361, 0.48, 6.1), (0.469, 0.678, 8.8))}
 _LARGE_COST_GATED = {256256: ((0.972, 0.387, 10.2),), 128256: ((0.633, 0.258, 4.8), (0.661, 0.979, 8.5)),
                      128128: ((0.361, 0.237, 3.9), (0.44, 0.583, 6.6)), 64128: ((0.259, 0.189, 2.8), (0.289, 0.528, 4.6), (0.511, 0.572, 5.2))}
-# The halves behind the last round of tiles of 256 rows.  (8 us of the rest are added: in a model, 28 layers of other matrices between,
-# 1,278 x 16,384 x 3,072 and 2,000 x 11,264 x 2,048 in halves made the step 0.8 and 2 % longer than tiles of 128 rows, where they measured alike by
-# themselves.)
-_LARGE_HALVES = {256256: (0.605, 0.24, 11.7), 256192: (0.356, 0.265, 14.2)}
+# The halves behind the last round of tiles of 256 rows.  (16 us of the rest are added: in a model, layers of other matrices between, 1,278 x
+# 16,384 x 3,072 and 2,000 x 11,264 x 2,048 in halves made the step 0.8 and 2 % longer than tiles of 128 rows, where they measured
+# alike by themselves.)
+_LARGE_HALVES = {256256: (0.605, 0.24, 19.7), 256192: (0.356, 0.265, 22.2)}
 _LARGE_SPLITS = 8
 
 
