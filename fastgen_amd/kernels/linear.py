@@ -62,15 +62,17 @@ TILED_MIN_ROWS, TILED_MAX_ROWS = 65, 512
 # measured, so that a first step takes no longer and every process takes the same kernel, where they are the faster ones (`_large_way`).
 # Times against the kernel that is measured to be the fastest otherwise, of 44 matrices (512 to 128,256 columns, 512 to 14,336 of k) at 17 to 4,096 rows, with the
 # norm behind where the result may be partial sums:
-# * gated products: 0.45 to 1.0 beyond 64 rows (1.02 to 1.1 in 28 of 260, where the library's tiles happen to fill the chip).  Up to 64 rows they are
-#   bound by how many workgroups read the matrix, 64 rows x 128 columns each: from 80 columns a compute unit on 0.91 to 1.0; fewer 1.05 to
-#   1.17 (the wide kernel's workgroups are twice as many, and it takes them), but for short k beyond 32 rows (k = 1,024: 0.78 to 1.02);
-# * products that may leave partial sums: 0.4 to 1.0 at 33 to 512 rows (1.02 to 1.1 in 22 of 300).  Up to 32 rows 0.91 to 1.04 from 2^24
-#   elements of the matrix on, with fewer 1.0 to 1.17 (the wide kernel's);
-# * wide fp32 outputs (logits) 0.7 to 1.02 from 96 columns a compute unit on; 16,384 x 2,048 is 1.1 to 1.19 up to 64 rows, and at 129 to 384 rows, where
-#   the library has tiles of 160 and 192 rows, 32,000 columns are 0.8 to 1.17, 50,304 and more 0.74 to 1.05;
-# * beyond LARGE_ROWS plain products and partial sums too: 0.65 to 1.1, 0.96 on average.  Where k is long and one round of tiles leaves a fifth of the compute
-#   units or more without one, the library, which cuts k there, is 1.09 times as fast (1.21 at 3,000 x 2,048 x 8,192, 192 tiles).
+# * gated products: 0.45 to 1.11 beyond 64 rows, 0.78 on average (above 1.02 in 16 of 250, where the library's tiles happen to fill the chip). Up to 64
+#   rows they are bound by how many workgroups read the matrix, 64 rows x 128 columns each: from 80 columns a compute unit on 0.91 to 1.0; fewer 0.97
+#   to 1.17, 1.09 on average (the wide kernel's workgroups are twice as many, and it takes them), but for short k beyond 32 rows (k = 1,024
+#   and less: 0.78 to 1.02);
+# * products that may leave partial sums: 0.40 to 1.10 at 33 to 512 rows, 0.87 on average (above 1.02 in 20 of 342).  Up to 32 rows 0.91 to 1.04 from 2^24
+#   elements of the matrix on, with fewer 0.87 to 1.17, 1.06 on average (the wide kernel's);
+# * wide fp32 outputs (logits) 0.75 to 1.05 from 96 columns a compute unit on; 16,384 x 2,048 is 1.1 to 1.19 up to 64 rows, and at 129 to 384
+#   rows, which fill tiles of 128 and 256 badly, 32,000 columns are 0.81 to 1.17, 50,304 and more 0.75 to 1.05;
+# * beyond LARGE_ROWS plain products and partial sums too: 0.62 to 1.18, 0.93 on average (above 1.02 in 41 of 256).  Where k is long and one round of tiles leaves a
+#   fifth of the compute units or more without one, the library is 1.09 times as fast (0.93 to 1.21 at 19 sizes, the most at
+#   3,000 x 2,048 x 8,192, 192 tiles).
 # A plain product of fewer rows has no splits to fill the chip with and goes the other ways (6,144 x 4,096 at 65 rows 34 us against
 # 23 of the library, at 320 36 against 30).
 LARGE_ROWS = TILED_MAX_ROWS

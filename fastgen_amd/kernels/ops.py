@@ -1252,8 +1252,8 @@ LARGE_TILES = (256256, 256192, 128256, 128192, 128128, 64128)
 # places had one at least, 320 x 28,672 x 4,096 with its 336 tiles of 128 x 256 takes 110 us, not 84).  Fitted to 7,547 products (65 to 4,096 rows, 512
 # to 32,768 columns, 512 to 16,384 of k, 1 to 8 splits); the plan that is the fastest by them takes longer than the fastest one by 0.3 and 1.5 % on
 # average with an activation (up to 512 rows and beyond), 0.4 and 1.3 % plain, 1.8 and 2.6 % with splits.  Without the tiles of 64 rows it was 16 %, 23 and 8 %, 15 and 7 %: a small
-# product has too few larger tiles (us, with the norm behind, without / with them / library: 100 x 1,024 x 2,816 12.9 / 10.2 / 12.6,
-# 400 x 512 x 1,408 12.6 / 9.9 / 10.1, 512 x 2,048 x 2,048 19.9 / 17.2 / 17.3, 640 x 3,072 x 2,048 21.6 / 16.8 / 16.9).
+# product has too few larger tiles (us, with the norm behind, without / with them / library: 100 x 1,024 x 2,816 12.9 / 11.2 / 12.4,
+# 400 x 512 x 1,408 12.6 / 10.4 / 10.0, 512 x 2,048 x 2,048 19.9 / 17.2 / 17.1, 640 x 3,072 x 2,048 21.6 / 16.8 / 16.6).
 _LARGE_COST = {256256: ((0.933, 0.437, 10.6),), 256192: ((0.757, 0.324, 9.4),), 128256: ((0.642, 0.227, 5.5), (0.699, 0.96, 16.2)),
                128192: ((0.563, 0.207, 4.7), (0.712, 0.605, 13.5)), 128128: ((0.388, 0.211, 4.7), (0.469, 0.579, 11.0)),
                64128: ((0.287, 0.185, 2.9), (0.361, 0.48, 6.1), (0.469, 0.678, 8.8))}
