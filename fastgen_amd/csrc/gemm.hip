@@ -40,6 +40,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "kv_layout.h"
 
 #define GT_M 64
 #define GT_N 64
@@ -271,36 +272,48 @@ __device__ __forceinline__ void gf_store4(float* __restrict__ y, int n, int N, b
   }
 }
 
+// What fg_silu_mul and fg_gelu_mul (rows.hip) give in fp32: the epilogue codes of the bf16 products.
+#define GF_SILU 1
+#define GF_GELU 4
+__device__ __forceinline__ float gf_gated(float gate, float up, int act) {
+  if (act == GF_GELU) return 0.5f * gate * (1.f + tanhf(0.7978845608028654f * (gate + 0.044715f * gate * gate * gate))) * up;
+  return gate / (1.f + expf(-gate)) * up;
+}
+
 // 16 rows (decode, and outputs too few for tiles): bound by reading W.  A workgroup owns 16 outputs of 16 rows; a round is
 // one group, a wave takes one of its segments, so 64 KB of W (every wave's next segment) are in flight a workgroup while
 // the current ones are multiplied; the segments' sums meet in LDS and are added in order by one thread an output.
 // N x K 3072 x 3072 / 16384 x 3072 / 3072 x 8192: 13 / 45 / 31 us at 4 rows (4.5 TB/s of W at the largest), 18 / 60 / 43 at
 // 16 (in tiles 25 / 54 / 32); with the fp32 instructions 14 / 47 / 31 and 18 / 60 / 40.
 // Two workgroups a compute unit (at most 128 registers): 441 workgroups of two groups 13 us, 15.7 with one.
+// With `part` a workgroup takes one group of k (blockIdx.z) and stores its sum, as the kernel of tiles below: what few outputs need to
+// have a workgroup for every compute unit.  With `act` the outputs are a gate and an up matrix interleaved in groups of eight, which
+// are these 16, and silu(gate) * up is stored (the tanh form of GELU).
 // A wave cuts its segment of x into parts once: with FEW (up to 8 rows), each number in one lane, through LDS into
 // the operands' order; above, every lane the operand it needs.
 template <bool FEW, bool VEC>
 __global__ __launch_bounds__(512, 4) void gemm_f32_few_kernel(const float* __restrict__ x, const float* __restrict__ w,
-                                                           float* __restrict__ y, int M, int N, int K, int ldx,
-                                                           int ldw, int ldy) {
+                                                           float* __restrict__ y, float* __restrict__ part, int M, int N,
+                                                           int K, int ldx, int ldw, int ldy, int act) {
   __shared__ f32x4 sums[2][8][FG_WAVE];
   __shared__ bf16x4 parts[FEW ? 8 : 1][4][3][4][8][2];  // [wave][step][part][g][row][half]
   const int tid = threadIdx.x, lane = tid % FG_WAVE, wave = tid / FG_WAVE;
   const int r = lane % 16, g = lane / 16, n0 = blockIdx.x * 16;
   x += (size_t)blockIdx.y * 16 * ldx;
   y += (size_t)blockIdx.y * 16 * ldy;
+  if (part) part += ((size_t)blockIdx.z * M + blockIdx.y * 16) * N;
   M = min(M - (int)blockIdx.y * 16, 16);
   // rows behind the last repeat it: their outputs are not stored
   const float* wrow = w + (size_t)min(n0 + r, N - 1) * ldw;
   const float* xrow = x + (size_t)min(r, M - 1) * ldx;
-  const int n_seg = (K + GF_SEG - 1) / GF_SEG;
+  const int s_begin = part ? 8 * blockIdx.z : 0, n_seg = min((K + GF_SEG - 1) / GF_SEG, part ? s_begin + 8 : 0x7fffffff);
   f32x4 wv[8], next[8], xv[8];
-  if (wave < n_seg) {
+  if (s_begin + wave < n_seg) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) next[i] = gf_load4<VEC>(wrow, wave * GF_SEG + i * 16 + g * 4, K);
+    for (int i = 0; i < 8; ++i) next[i] = gf_load4<VEC>(wrow, (s_begin + wave) * GF_SEG + i * 16 + g * 4, K);
   }
   float total = 0.f;
-  for (int s0 = 0, buf = 0; s0 < n_seg; s0 += 8, buf ^= 1) {
+  for (int s0 = s_begin, buf = 0; s0 < n_seg; s0 += 8, buf ^= 1) {
     const int seg = s0 + wave;
     if (seg < n_seg) {
       if constexpr (FEW) {
@@ -354,13 +367,23 @@ __global__ __launch_bounds__(512, 4) void gemm_f32_few_kernel(const float* __res
     }
   }
   // element tid of a wave's sums: lane tid / 4 = 16 g + r, output 4 g + tid % 4 of row r
-  if (tid < 256) {
-    const int m = (tid / 4) % 16, n = n0 + (tid / 64) * 4 + tid % 4;
-    if (m < M && n < N) {
-      if (gf_lost(total)) total = gf_again(x + (size_t)m * ldx, w + (size_t)n * ldw, K);
-      y[(size_t)m * ldy + n] = total;
-    }
+  const int m = (tid / 4) % 16, n = n0 + (tid / 64) * 4 + tid % 4;
+  const bool mine = tid < 256 && m < M && n < N;
+  if (part) {
+    if (mine) part[(size_t)m * N + n] = total;
+    return;
   }
+  if (mine && gf_lost(total)) total = gf_again(x + (size_t)m * ldx, w + (size_t)n * ldw, K);
+  if (!act) {
+    if (mine) y[(size_t)m * ldy + n] = total;
+    return;
+  }
+  // the outputs are eight gates and the ups of their channels (N % 16 == 0)
+  float* ups = (float*)sums;  // (behind a round's sums at the earliest: what is read there is read before the barrier)
+  __syncthreads();
+  if (tid >= 128 && tid < 256) ups[tid - 128] = total;
+  __syncthreads();
+  if (tid < 128 && m < M) y[(size_t)m * ldy + n0 / 2 + (tid / 64) * 4 + tid % 4] = gf_gated(total, ups[tid], act);
 }
 
 // Many rows: bound by the matrix cores at the clock they can hold.  NW waves own 16 MB rows x 16 NB NW outputs, each
@@ -531,19 +554,138 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_f32_tiled_kernel(
   }
 }
 
-// The groups' sums, added in order.
-__global__ __launch_bounds__(256) void gemm_f32_sum_kernel(const float* __restrict__ part, float* __restrict__ y,
-                                                           const float* __restrict__ x, const float* __restrict__ w,
-                                                           int M, int N, int K, int ldx, int ldw, int ldy, int groups,
-                                                           int wide) {
-  const int m = blockIdx.y, n = (blockIdx.x * 256 + threadIdx.x) * 4;
-  if (n >= N) return;
-  f32x4 total = {0.f, 0.f, 0.f, 0.f};
-  for (int g = 0; g < groups; ++g) total += gf_read4(part + ((size_t)g * M + m) * N, n, N, wide);
+// What a product leaves where every group of k has a workgroup of its own: fp32 [groups][M][N], to be added in order.  An
+// output that comes out as no number is computed again from the operands.
+struct GfSums {
+  const float *part, *x, *w;
+  int M, N, K, ldx, ldw, groups;
+};
+
+// Outputs n[v] .. n[v] + 3 of row m.  U: groups whose sums are in flight together: behind a product of few rows the kernels below are a
+// chain of memory's latencies (3,072 outputs of 8 groups, 4 rows, with the norm: 8 us four by four, 4 at once).
+template <int NV, int U>
+__device__ __forceinline__ void gf_totals(const GfSums& s, int m, const int (&n)[NV], bool wide, f32x4 (&total)[NV]) {
 #pragma unroll
-  for (int e = 0; e < 4; ++e)
-    if (gf_lost(total[e]) && n + e < N) total[e] = gf_again(x + (size_t)m * ldx, w + (size_t)(n + e) * ldw, K);
-  gf_store4(y + (size_t)m * ldy, n, N, wide, total);
+  for (int v = 0; v < NV; ++v) total[v] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int g0 = 0; g0 < s.groups; g0 += U) {
+    f32x4 p[U][NV];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int v = 0; v < NV; ++v) p[u][v] = gf_read4(s.part + ((size_t)min(g0 + u, s.groups - 1) * s.M + m) * s.N, n[v], s.N, wide);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (g0 + u < s.groups) {  // uniform
+#pragma unroll
+        for (int v = 0; v < NV; ++v) total[v] += p[u][v];
+      }
+  }
+#pragma unroll
+  for (int v = 0; v < NV; ++v)
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (gf_lost(total[v][e]) && n[v] + e < s.N) total[v][e] = gf_again(s.x + (size_t)m * s.ldx, s.w + (size_t)(n[v] + e) * s.ldw, s.K);
+}
+
+__global__ __launch_bounds__(256) void gemm_f32_sum_kernel(const GfSums s, float* __restrict__ y, int ldy, int wide) {
+  const int m = blockIdx.y, n = (blockIdx.x * 256 + threadIdx.x) * 4;
+  if (n >= s.N) return;
+  const int at[1] = {n};
+  f32x4 total[1];
+  gf_totals<1, 4>(s, m, at, wide, total);
+  gf_store4(y + (size_t)m * ldy, n, s.N, wide, total[0]);
+}
+
+// The sums of a gate and an up matrix interleaved in groups of eight, and the activation: four channels a thread.
+// (N % 16 == 0, y [M][N / 2].)
+__global__ __launch_bounds__(256) void gemm_f32_sum_act_kernel(const GfSums s, float* __restrict__ y, int act) {
+  const int m = blockIdx.y, c = (blockIdx.x * 256 + threadIdx.x) * 4;
+  if (c >= s.N / 2) return;
+  const int n[2] = {c / 8 * 16 + c % 8, c / 8 * 16 + c % 8 + 8};  // gates, ups
+  f32x4 total[2], v;
+  gf_totals<2, 4>(s, m, n, true, total);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = gf_gated(total[0][e], total[1][e], act);
+  *(f32x4*)(y + (size_t)m * (s.N / 2) + c) = v;
+}
+
+// The sums, added to the residual stream, and the norm behind: fg_add_rmsnorm (rows.hip) on the product's rows, in its order and with
+// its bits.  A workgroup a row, eight elements a thread and round, in registers.  N % 8 == 0, N <= 2048 NIT.
+template <int NIT>
+__global__ __launch_bounds__(256) void gemm_f32_sum_norm_kernel(const GfSums s, float* __restrict__ h, const float* __restrict__ weight,
+                                                                float* __restrict__ out, float eps) {
+  __shared__ float red[16];
+  const int m = blockIdx.x;
+  float* hrow = h + (size_t)m * s.N;
+  f32x4 v[2 * NIT], wv[2 * NIT], total[2 * NIT];
+  int n[2 * NIT];  // (a thread whose share lies behind the row reads its last elements and stores nothing)
+#pragma unroll
+  for (int i = 0; i < 2 * NIT; ++i) {
+    n[i] = min((int)(threadIdx.x + i / 2 * 256) * 8, s.N - 8) + 4 * (i % 2);
+    v[i] = *(const f32x4*)(hrow + n[i]);
+    wv[i] = *(const f32x4*)(weight + n[i]);
+  }
+  gf_totals<2 * NIT, NIT <= 2 ? 8 : 4>(s, m, n, true, total);
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < 2 * NIT; ++i) {
+    v[i] += total[i];
+    if ((int)(threadIdx.x + i / 2 * 256) * 8 < s.N) {
+      *(f32x4*)(hrow + n[i]) = v[i];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) ss += v[i][e] * v[i][e];
+    }
+  }
+  ss = block_sum(ss, red);
+  const float rstd = rsqrtf(ss / (float)s.N + eps);
+#pragma unroll
+  for (int i = 0; i < 2 * NIT; ++i) {
+    f32x4 o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = v[i][e] * rstd * wv[i][e];
+    if ((int)(threadIdx.x + i / 2 * 256) * 8 < s.N) *(f32x4*)(out + (size_t)m * s.N + n[i]) = o;
+  }
+}
+
+// The sums of a q/k/v product, rotated, keys and values into their pages: fg_rope_kv_write (rope_kv.hip) on the product's rows, the
+// same bits, the queries to q_out [M][n_heads * hd].  A chunk of 8 columns a thread.
+__global__ __launch_bounds__(128) void gemm_f32_sum_rope_kernel(const GfSums s, float* __restrict__ q_out, const float* __restrict__ table,
+                                                                const int* __restrict__ slots, float* __restrict__ k_pages,
+                                                                float* __restrict__ v_pages, int n_heads, int n_kv, int hd,
+                                                                int rotary_dim, int page_size, int value_from_key) {
+  const int t = blockIdx.x, cph = hd / 8, c8 = blockIdx.y * 128 + threadIdx.x;
+  if (c8 * 8 >= s.N) return;
+  const int head = c8 / cph, c = c8 % cph, slot = slots[t];
+  if (head >= n_heads && slot < 0) return;
+  const int n[2] = {8 * c8, 8 * c8 + 4};
+  f32x4 total[2];
+  gf_totals<2, 4>(s, t, n, true, total);
+  float v[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) v[j] = total[j / 4][j % 4];
+  const KvLayout lay(page_size, hd);
+  const size_t head_elems = (size_t)page_size * hd;
+  const int page = slot >= 0 ? slot / page_size : 0, off = slot >= 0 ? slot % page_size : 0;
+  const int kvh = head < n_heads ? 0 : (head - n_heads) % n_kv;
+  const size_t place = ((size_t)page * n_kv + kvh) * head_elems;
+  const bool is_v = head >= n_heads + n_kv;
+  if (is_v || (value_from_key && head >= n_heads)) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v_pages[place + lay.v_off(off, 8 * c + j)] = v[j];
+  }
+  if (is_v) return;
+  if (8 * c < rotary_dim) {
+    float cs4[8];  // cos, sin of the chunk's four pairs
+    load8<float>(table + ((size_t)t * (rotary_dim / 2) + 4 * c) * 2, cs4);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float cs = cs4[2 * j], sn = cs4[2 * j + 1];
+      const float a = v[2 * j], b = v[2 * j + 1];
+      v[2 * j] = a * cs - b * sn;
+      v[2 * j + 1] = b * cs + a * sn;
+    }
+  }
+  store8<float>(head < n_heads ? q_out + (size_t)t * n_heads * hd + 8 * c8 : k_pages + place + lay.k_off(off, 8 * c), v);
 }
 
 struct GfCall {
@@ -553,11 +695,24 @@ struct GfCall {
   hipStream_t stream;
 };
 
+static int gf_wide(const GfCall& c) {
+  return c.N % 4 == 0 && c.ldy % 4 == 0 && (uintptr_t)c.y % 16 == 0 && (uintptr_t)c.part % 16 == 0;
+}
+
+// The groups' sums to y, where there are any and somebody wants them added up.
+static int gf_sum(const GfCall& c) {
+  if (c.part && c.y) {
+    const GfSums s = {c.part, c.x, c.w, c.M, c.N, c.K, c.ldx, c.ldw, (c.K + GF_GROUP - 1) / GF_GROUP};
+    gemm_f32_sum_kernel<<<dim3((c.N + 1023) / 1024, c.M), 256, 0, c.stream>>>(s, c.y, c.ldy, gf_wide(c));
+  }
+  return fg_launch_status();
+}
+
 template <int MB, int NB, int NW, bool FAR = false>
 static int gf_launch(const GfCall& c) {
   constexpr int AHEAD = MB <= 3 ? 4 : 2;
   const int groups = (c.K + GF_GROUP - 1) / GF_GROUP;
-  const int wide = c.N % 4 == 0 && c.ldy % 4 == 0 && (uintptr_t)c.y % 16 == 0 && (uintptr_t)c.part % 16 == 0;
+  const int wide = gf_wide(c);
   const int row_tiles = (c.M + 16 * MB - 1) / (16 * MB), col_tiles = (c.N + 16 * NB * NW - 1) / (16 * NB * NW);
   const long long units = (long long)col_tiles * (c.part ? groups : 1);
   const long long blocks = (units * row_tiles + 7) / 8 * 8;
@@ -568,25 +723,24 @@ static int gf_launch(const GfCall& c) {
   if (c.vec) TILED(true);
   else TILED(false);
 #undef TILED
-  if (c.part) {
-    gemm_f32_sum_kernel<<<dim3((c.N + 1023) / 1024, c.M), 256, 0, c.stream>>>(c.part, c.y, c.x, c.w, c.M, c.N, c.K,
-                                                                              c.ldx, c.ldw, c.ldy, groups, wide);
-  }
-  return fg_launch_status();
+  return gf_sum(c);
 }
 
 // mb, nw: the tile of the many-rows kernel, 16 mb rows (mb <= 5 with 4 waves, 7 with 8) and nw waves of 32 outputs
 // (mb = 0: the kernel of 16 rows).
-// part: null, or fp32 [ceil(K / 1024)][M][N] for a workgroup a group of k.
-extern "C" int fg_gemm_f32(const float* x, const float* w, float* y, float* part, int M, int N, int K, int ldx,
-                           int ldw, int ldy, int mb, int nw, hipStream_t stream) {
+// part: null, or fp32 [ceil(K / 1024)][M][N] for a workgroup a group of k; with y null the sums stay there.
+// act: 0, or (mb = 0 without part, N % 16 == 0) GF_SILU or GF_GELU: y is [M][N / 2].
+extern "C" int fg_gemm_f32_act(const float* x, const float* w, float* y, float* part, int M, int N, int K, int ldx, int ldw, int ldy,
+                               int mb, int nw, int act, hipStream_t stream) {
   if (M <= 0 || N <= 0) return FG_OK;
-  if (K <= 0 || ldx < K || ldw < K || ldy < N) return FG_ERR_ARG;
+  if (K <= 0 || ldx < K || ldw < K || (y && ldy < (act ? N / 2 : N)) || (!y && !part)) return FG_ERR_ARG;
+  if (act && ((act != GF_SILU && act != GF_GELU) || mb || part || N % 16)) return FG_ERR_ARG;
   const bool vec = K % 4 == 0 && ldx % 4 == 0 && ldw % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0;
   if (mb == 0) {
-    if (M > 16 * 65535 || part) return FG_ERR_ARG;
-    const dim3 blocks((N + 15) / 16, (M + 15) / 16);
-#define FEW_ROWS(FEW, VEC) gemm_f32_few_kernel<FEW, VEC><<<blocks, 512, 0, stream>>>(x, w, y, M, N, K, ldx, ldw, ldy)
+    const int groups = (K + GF_GROUP - 1) / GF_GROUP;
+    if (M > 16 * 65535 || (part && (M > 65535 || groups > 65535))) return FG_ERR_ARG;
+    const dim3 blocks((N + 15) / 16, (M + 15) / 16, part ? groups : 1);
+#define FEW_ROWS(FEW, VEC) gemm_f32_few_kernel<FEW, VEC><<<blocks, 512, 0, stream>>>(x, w, y, part, M, N, K, ldx, ldw, ldy, act)
     if (M <= 8) {
       if (vec) FEW_ROWS(true, true);
       else FEW_ROWS(true, false);
@@ -595,7 +749,7 @@ extern "C" int fg_gemm_f32(const float* x, const float* w, float* y, float* part
       else FEW_ROWS(false, false);
     }
 #undef FEW_ROWS
-    return fg_launch_status();
+    return gf_sum({x, w, y, part, M, N, K, ldx, ldw, ldy, vec, stream});
   }
   const GfCall c = {x, w, y, part, M, N, K, ldx, ldw, ldy, vec, stream};
   if (mb < 1 || mb > 7 || (nw == 4 && mb > 5) || (nw != 4 && nw != 8)) return FG_ERR_ARG;
@@ -611,3 +765,52 @@ extern "C" int fg_gemm_f32(const float* x, const float* w, float* y, float* part
 #undef CASE
   return FG_ERR_ARG;
 }
+
+extern "C" int fg_gemm_f32(const float* x, const float* w, float* y, float* part, int M, int N, int K, int ldx,
+                           int ldw, int ldy, int mb, int nw, hipStream_t stream) {
+  return y || M <= 0 || N <= 0 ? fg_gemm_f32_act(x, w, y, part, M, N, K, ldx, ldw, ldy, mb, nw, 0, stream) : FG_ERR_ARG;
+}
+
+// The groups' sums `part` of x [M, K] and w [N, K] (what fg_gemm_f32_act left) and what comes behind the product.  All rows 16-byte aligned.
+#define GF_SUMS const GfSums s = {part, x, w, M, N, K, ldx, ldw, (K + GF_GROUP - 1) / GF_GROUP}
+static bool gf_sums_ok(const float* part, int M, int N, int K, const void* out) {
+  return part && K > 0 && N % 8 == 0 && M <= 65535 && (uintptr_t)part % 16 == 0 && (uintptr_t)out % 16 == 0;
+}
+
+// silu(gate) * up (act GF_SILU) or the tanh form of GELU in its place (GF_GELU) of interleaved columns: y [M, N / 2].
+extern "C" int fg_gemm_f32_sum_act(const float* part, const float* x, const float* w, float* y, int M, int N, int K, int ldx, int ldw,
+                                   int act, hipStream_t stream) {
+  if (M <= 0 || N <= 0) return FG_OK;
+  if (!gf_sums_ok(part, M, N, K, y) || N % 16 || (act != GF_SILU && act != GF_GELU)) return FG_ERR_ARG;
+  GF_SUMS;
+  gemm_f32_sum_act_kernel<<<dim3((N / 2 + 1023) / 1024, M), 256, 0, stream>>>(s, y, act);
+  return fg_launch_status();
+}
+
+// h [M, N] += the product, out = rmsnorm(h) * weight.  N <= 8192.
+extern "C" int fg_gemm_f32_sum_norm(const float* part, const float* x, const float* w, float* h, const float* weight, float* out, int M,
+                                    int N, int K, int ldx, int ldw, float eps, hipStream_t stream) {
+  if (M <= 0 || N <= 0) return FG_OK;
+  if (!gf_sums_ok(part, M, N, K, out) || N > 8192 || ((uintptr_t)h | (uintptr_t)weight) % 16) return FG_ERR_ARG;
+  GF_SUMS;
+  if (N <= 2048) gemm_f32_sum_norm_kernel<1><<<M, 256, 0, stream>>>(s, h, weight, out, eps);
+  else if (N <= 4096) gemm_f32_sum_norm_kernel<2><<<M, 256, 0, stream>>>(s, h, weight, out, eps);
+  else gemm_f32_sum_norm_kernel<4><<<M, 256, 0, stream>>>(s, h, weight, out, eps);
+  return fg_launch_status();
+}
+
+// The rotated queries to q_out [M, n_heads * hd], keys and values into their pages (see fg_rope_kv_parts in rope_kv.hip).
+extern "C" int fg_gemm_f32_sum_rope(const float* part, const float* x, const float* w, float* q_out, const float* table, const int* slots,
+                                    float* k_pages, float* v_pages, int M, int N, int K, int ldx, int ldw, int n_heads, int n_kv, int hd,
+                                    int rotary_dim, int page_size, int value_from_key, hipStream_t stream) {
+  if (M <= 0 || N <= 0) return FG_OK;
+  if (!gf_sums_ok(part, M, N, K, q_out) || hd <= 0 || hd % 8 || rotary_dim < 0 || rotary_dim > hd || rotary_dim % 8 || page_size <= 0 ||
+      page_size % 8 || n_heads <= 0 || n_kv <= 0 || (rotary_dim && (!table || (uintptr_t)table % 16)) || (uintptr_t)k_pages % 16 ||
+      N != (n_heads + (value_from_key ? 1 : 2) * n_kv) * hd)
+    return FG_ERR_ARG;
+  GF_SUMS;
+  gemm_f32_sum_rope_kernel<<<dim3(M, (N / 8 + 127) / 128), 128, 0, stream>>>(s, q_out, table, slots, k_pages, v_pages, n_heads, n_kv, hd,
+                                                                            rotary_dim, page_size, value_from_key);
+  return fg_launch_status();
+}
+#undef GF_SUMS

@@ -398,7 +398,7 @@ def linear(x, w, out_dtype: Optional[torch.dtype] = None,
     eps) asks for more than the product: add it to the fp32 residual stream ``h`` and prepare the
     RMSNorm that follows.  Where that can be folded into the product's kernel (few rows, bfloat16)
     the result is ``ScaledRows`` and ``h`` is updated; where not, the plain product comes back and
-    adding and norming are the caller's."""
+    adding and norming are the caller's.  A float32 product with ``residual`` is finished, :class:`~fastgen_amd.kernels.ops.NormedRows`."""
     silu = epilogue in ("silu_mul", "gelu_tanh_mul")  # a gated epilogue: act(gate) * up
     if epilogue not in (None, "silu_mul", "gelu_tanh_mul"):
         raise ops.KernelArgumentError(f"linear: unknown epilogue {epilogue!r}")
@@ -417,8 +417,11 @@ def linear(x, w, out_dtype: Optional[torch.dtype] = None,
     if x.dtype == torch.float32:
         if out_dtype not in (None, torch.float32):
             raise ops.KernelArgumentError("a float32 product has float32 output")
-        y = ops.gemm_nt(x, w)
-        return act_mul(y) if silu else y
+        if silu:
+            return ops.gemm_f32_gated(x, w, "gelu_tanh" if gated == "gelu_tanh" else "silu")
+        if residual is not None and ops.gemm_f32_norm_ok(x, w, residual[0], residual[1]):
+            return ops.NormedRows(ops.gemm_f32_norm(x, w, *residual))
+        return ops.gemm_nt(x, w)
     if x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
         raise ops.KernelArgumentError(f"linear: unsupported dtypes {x.dtype}, {w.dtype}")
     out_dtype = out_dtype or torch.bfloat16

@@ -929,7 +929,7 @@ GEMM_F32_FEW_ROWS, GEMM_F32_MAX_SUMS, GEMM_F32_MAX_SPLIT_ROWS = 8, 256 << 20, 40
 
 
 @functools.lru_cache(maxsize=4096)
-def gemm_f32_plan(M: int, N: int, K: int, cus: int) -> Tuple[int, int, bool]:
+def gemm_f32_plan(M: int, N: int, K: int, cus: int, behind: bool = False) -> Tuple[int, int, bool]:
     """How the 32-bit product is cut: (blocks of 16 rows in a tile, waves of 32 outputs in a tile, whether every group of k
     has a workgroup of its own); (0, 0, False): the kernel of 16 rows and 16 outputs.  Every cut gives the same bits.
 
@@ -941,14 +941,26 @@ def gemm_f32_plan(M: int, N: int, K: int, cus: int) -> Tuple[int, int, bool]:
     group as much less as it is shorter; W itself comes at 5 TB/s at best.  Counted and measured (us): 400 rows 16384 x 3072
     281 and 290, 5120 x 3072 102 and 105, 2048 x 2048 44 and 45; 64 rows 512 x 2048 12 and 12.  (On the fp32 matrix
     instructions, 32 x 32 outputs a workgroup, products that fill the chip took 1.3 to 1.7 times as long, and some below 30
-    us that do not 1 to 6 us less.)"""
-    if M <= GEMM_F32_FEW_ROWS:
+    us that do not 1 to 6 us less.)
+
+    ``behind``: the groups' sums are added up by the kernel that follows the product anyway (a norm, an activation, a rotation).  Up
+    to 16 rows the kernel of 16 rows may then be cut too: a round of 1,024 k of its workgroups takes 3.5 us a workgroup and compute unit,
+    3.8 at least; cut, all of W comes at 5.1 TB/s behind 7.5 us, 2 % more a row beyond four, and the sums cost the kernel behind 1 us and
+    0.35 a group.  Measured at 4 rows, uncut and cut, with the kernel behind: 5,120 x 3,072 (320 workgroups) 31 and 25, 3,072 x 8,192 38.1 and 35.2,
+    3,072 x 3,072 19.8 and 20.6, 4,096 x 14,336 61.0 and 62.8."""
+    if M <= GEMM_F32_FEW_ROWS and not behind:
         return 0, 0, False
     groups, blocks, streaming = -(-K // GEMM_F32_GROUP), -(-M // 16), N * K * 4 / 5e6
     part = K % GEMM_F32_GROUP / GEMM_F32_GROUP
     whole = K // GEMM_F32_GROUP + (max(0.4, part) if part else 0)
     wgs = -(-N // 16) * blocks
     best = 2 + max(whole * (4.8 if wgs <= cus else max(9, 1.6 + 4 * wgs / cus)), streaming), (0, 0, False)
+    if behind and M <= 16 and groups > 1:
+        uncut = 4 + whole * max(3.8, 3.5 * -(-wgs // cus))
+        cut = (7.5 + N * K * 4 / 5.1e6) * (1 + 0.02 * max(0, M - 4)) + 1 + 0.35 * groups
+        best = min(best if M > GEMM_F32_FEW_ROWS else (uncut, (0, 0, False)), (cut, (0, 0, True)))
+    if M <= GEMM_F32_FEW_ROWS:
+        return best[1]
     for waves, tallest in ((8, 7), (4, 5)):  # (what the registers hold)
         for b in range(1, tallest + 1):
             row_tiles = -(-blocks // b)
@@ -962,7 +974,9 @@ def gemm_f32_plan(M: int, N: int, K: int, cus: int) -> Tuple[int, int, bool]:
                 rounds, rest = divmod(die, cus // 8 * (8 // waves))
                 time = rounds * full + (0 if not rest else alone if waves == 4 and rest <= cus // 8 else full)
                 time = max(time * (GEMM_F32_GROUP // 32 if split else -(-K // 32)), streaming)
-                time += 5 + (2 + groups * M * N * 8 / 6e6 if split else 0)
+                if split:
+                    time += 1 + 0.35 * groups + groups * M * N * 4 / 6e6 if behind else 2 + groups * M * N * 8 / 6e6
+                time += 5
                 if time < best[0]:
                     best = time, (b, waves, split)
     return best[1]
@@ -972,7 +986,7 @@ def gemm_f32_scratch(M: int, N: int, K: int) -> int:
     """Bytes of the groups' sums that :func:`gemm_nt` takes at most for up to ``M`` rows (see :func:`gemm_f32_plan`)."""
     groups = -(-K // GEMM_F32_GROUP)
     sums = min(groups * min(M, GEMM_F32_MAX_SPLIT_ROWS) * N * 4, GEMM_F32_MAX_SUMS)
-    return sums if groups > 1 and M > GEMM_F32_FEW_ROWS else 0
+    return sums if groups > 1 else 0
 
 
 def gemm_nt(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None,
@@ -1003,6 +1017,97 @@ def gemm_nt(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None
             _code(x), _code(out), _stream(out))
         _check(st, "gemm_nt")
     return out
+
+
+def _f32_product(x: torch.Tensor, w: torch.Tensor, what: str, act: int = 0) -> Tuple[torch.Tensor, bool]:
+    """The 32-bit product with a kernel behind it that adds the groups' sums up: ``(y [M, N], False)``, or ``(sums [groups, M, N],
+    True)``.  ``act``: an epilogue code; the kernel of 16 rows stores the activation's ``[M, N / 2]`` itself."""
+    _need(x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[1] and x.dtype == w.dtype == torch.float32
+          and x.stride(1) == 1 and w.stride(1) == 1, f"{what}: x [M, K] and w [N, K] must be float32 with unit column stride")
+    (M, K), N = x.shape, w.shape[0]
+    blocks, waves, split = gemm_f32_plan(M, N, K, compute_units(), True)
+    act = 0 if split or blocks else act
+    shape = (-(-K // GEMM_F32_GROUP), M, N) if split else (M, N // 2 if act else N)
+    y = torch.empty(shape, dtype=torch.float32, device=x.device)
+    st = _lib.load("gemm").fg_gemm_f32_act(_ptr(x), _ptr(w), _ptr(None if split else y), _ptr(y if split else None), M, N, K, x.stride(0),
+                                           w.stride(0), shape[-1], blocks, waves, act, _stream(x))
+    _check(st, what)
+    return y, split
+
+
+def _f32_sums_args(parts: torch.Tensor, x: torch.Tensor, w: torch.Tensor):
+    return _ptr(parts), _ptr(x), _ptr(w)
+
+
+def gemm_f32_gated(x: torch.Tensor, w: torch.Tensor, epilogue="silu") -> torch.Tensor:
+    """``act(gate) * up`` in float32 of the product with a gate and an up matrix interleaved by :func:`interleave_gate_up` (``"silu"`` or
+    ``"gelu_tanh"``), with the bits of :func:`gemm_nt` and :func:`silu_mul` or :func:`gelu_mul` behind it."""
+    _gpu(x, w)
+    act, N = _gated_code(epilogue), w.shape[0]
+    _need(act != 0 and N % 16 == 0, "gemm_f32_gated: a gated epilogue, N % 16 == 0")
+    y, split = _f32_product(x, w, "gemm_f32_gated", act)
+    if not split:
+        return y if y.shape[1] == N // 2 else gelu_mul(y) if act == 4 else silu_mul(y)
+    (M, K), out = x.shape, torch.empty((x.shape[0], N // 2), dtype=torch.float32, device=x.device)
+    st = _lib.load("gemm").fg_gemm_f32_sum_act(*_f32_sums_args(y, x, w), _ptr(out), M, N, K, x.stride(0), w.stride(0), act, _stream(x))
+    _check(st, "gemm_f32_gated")
+    return out
+
+
+def gemm_f32_norm_ok(x: torch.Tensor, w: torch.Tensor, h: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether :func:`gemm_f32_norm` takes the norm behind a float32 product."""
+    N = w.shape[0]
+    return (N % 8 == 0 and N <= 8192 and x.shape[0] <= 65535 and h.dtype == torch.float32 and h.shape == (x.shape[0], N) and h.is_contiguous()
+            and weight.dtype == torch.float32 and weight.shape == (N,) and weight.is_contiguous()
+            and h.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
+
+
+def gemm_f32_norm(x: torch.Tensor, w: torch.Tensor, h: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
+    """``h += x @ w.T`` in float32, and ``rmsnorm(h) * weight``, with the bits of :func:`gemm_nt` and :func:`add_rmsnorm` behind it."""
+    _gpu(x, w, h, weight)
+    _need(gemm_f32_norm_ok(x, w, h, weight), "gemm_f32_norm: h [M, N] and weight [N] float32, N a multiple of 8 up to 8,192")
+    (M, K), N = x.shape, w.shape[0]
+    y, split = _f32_product(x, w, "gemm_f32_norm")
+    out = torch.empty((M, N), dtype=torch.float32, device=x.device)
+    if not split:
+        return add_rmsnorm(h, y, weight, eps, out)
+    st = _lib.load("gemm").fg_gemm_f32_sum_norm(*_f32_sums_args(y, x, w), _ptr(h), _ptr(weight), _ptr(out), M, N, K, x.stride(0), w.stride(0),
+                                                ctypes.c_float(eps), _stream(x))
+    _check(st, "gemm_f32_norm")
+    return out
+
+
+def gemm_f32_qkv(x: torch.Tensor, wqkv: torch.Tensor, table: Optional[torch.Tensor], positions: torch.Tensor, slots: torch.Tensor,
+                 k_pages: torch.Tensor, v_pages: torch.Tensor, n_heads: int, n_kv: int, head_dim: int, rotary_dim: int,
+                 value_from_key: bool = False) -> torch.Tensor:
+    """The float32 q, k, v projections with :func:`rope_kv_write` behind them, the same bits: rows that begin with the rotated queries
+    ``[M, >= H*hd]``; the rotated keys and the values go into their pages.  ``value_from_key``: ``wqkv`` has no v rows, a token's
+    value is its key before the rotation."""
+    _gpu(x, wqkv, table, positions, slots, k_pages, v_pages)
+    (M, K), N = x.shape, wqkv.shape[0]
+    _need(N == (n_heads + (1 if value_from_key else 2) * n_kv) * head_dim, "wqkv must have the rows of q, k and v")
+    y, split = _f32_product(x, wqkv, "gemm_f32_qkv")
+    if not split or head_dim % 8 or rotary_dim % 8 or M > 65535:
+        if split:
+            y = gemm_nt(x, wqkv)
+        rope_kv_write(y, positions, None, slots, k_pages, v_pages, n_heads, n_kv, head_dim, rotary_dim, table=table,
+                      v_col=n_heads * head_dim if value_from_key else None)
+        return y
+    _i32(slots, "slots", M)
+    if rotary_dim:
+        _need(table is not None and table.dtype == torch.float32 and table.is_contiguous()
+              and table.shape == (M, rotary_dim // 2, 2), "table must be float32 [M, rotary_dim/2, 2]")
+    _need(k_pages.dim() == 4 and k_pages.is_contiguous() and k_pages.dtype == torch.float32
+          and k_pages.shape[1] == n_kv and k_pages.shape[3] == head_dim, "k_pages must be contiguous float32 [n_pages, KV, P, hd]")
+    _need(v_pages.is_contiguous() and v_pages.dtype == torch.float32
+          and v_pages.shape == (k_pages.shape[0], n_kv, head_dim, k_pages.shape[2]),
+          "v_pages must be contiguous float32 [n_pages, KV, hd, P]")
+    q = torch.empty((M, n_heads * head_dim), dtype=torch.float32, device=x.device)
+    st = _lib.load("gemm").fg_gemm_f32_sum_rope(
+        *_f32_sums_args(y, x, wqkv), _ptr(q), _ptr(table if rotary_dim else None), _ptr(slots), _ptr(k_pages), _ptr(v_pages), M, N, K,
+        x.stride(0), wqkv.stride(0), n_heads, n_kv, head_dim, rotary_dim, k_pages.shape[2], int(value_from_key), _stream(x))
+    _check(st, "gemm_f32_qkv")
+    return q
 
 
 SKINNY_MAX_ROWS = 128
@@ -1101,6 +1206,16 @@ class ScaledRows:
     def materialize(self) -> torch.Tensor:
         """The rows themselves (a kernel of its own: for a consumer that does not take the pair)."""
         return scale_rows(self.rows, self.ssq, self.dim, self.eps)
+
+
+class NormedRows(ScaledRows):
+    """Rows whose norm is done: what a product leaves that added itself to the residual stream and normed it."""
+
+    def __init__(self, rows: torch.Tensor) -> None:
+        super().__init__(rows, None, rows.shape[1], 0.0)
+
+    def materialize(self) -> torch.Tensor:
+        return self.rows
 
 
 def _row_scale_args(x, M: int):

@@ -219,8 +219,11 @@ class Attention(RowsMixer):
             # an entry that reads another entry's cache needs its queries only (and its gate)
             own_rows = self.wqkv if store.owns or self.output_gate else self.wqkv.first_rows(q_width)
             plain = store.owns and not self.output_gate and self.head_dim % 8 == 0 and self.position.rotary_dim % 8 == 0
-            parts = qkv_parts(x, own_rows) if plain else None
-            if parts is not None:
+            parts = qkv_parts(x, own_rows) if plain and x.dtype == torch.bfloat16 else None
+            if plain and x.dtype == torch.float32:
+                qkv = ops.gemm_f32_qkv(x, own_rows.rows, table, ctx.positions, group.slots, store.k_pages, store.v_pages, self.n_heads,
+                                       self.n_kv_heads, self.head_dim, self.position.rotary_dim, value_from_key=self.value_from_key)
+            elif parts is not None:
                 qkv = ops.rope_kv_parts(parts, table, group.slots, store.k_pages, store.v_pages, self.n_heads, self.n_kv_heads,
                                         self.head_dim, self.position.rotary_dim, value_from_key=self.value_from_key)
             else:

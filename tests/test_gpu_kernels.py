@@ -1398,3 +1398,36 @@ def test_parts_are_left_only_where_the_projection_takes_all_of_them(ops, n_keys,
         assert ((h - want_h).abs() <= 2.0 ** -8 * (row.double().abs() @ w.double().abs().T) + 1e-6 * h0.abs()).all()
     else:
         assert int(plan[10]) == -(-(-(-n_keys // 64)) // min_tiles) and torch.equal(got, row)
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 5120, 3072), (8, 3072, 8192), (9, 640, 2100), (16, 5120, 3072), (33, 1536, 4096), (70, 8192, 1100),
+                                   (130, 2048, 1000), (300, 1040, 2048)])
+def test_gemm_f32_with_what_is_behind_has_the_bits_of_both(ops, M, N, K):
+    """The sums of the groups of k added up by the activation, the norm or the rotation behind the product (cut and uncut), the
+    activation in the kernel of few rows, against the product and those kernels one after the other: bit for bit, and an output
+    that comes out as no number computed again there too."""
+    torch.manual_seed(N)
+    x, w = torch.randn(M, K).to(DEV), torch.randn(N, K).to(DEV)
+    x[M // 2, K - 1], w[5, 3] = float("inf"), 3.4e38  # (an infinity's parts' products, and what rounds to one in 16 bits)
+    h, weight = torch.randn(M, N).to(DEV), torch.randn(N).to(DEV)
+    same = lambda a, b: torch.equal(a[~b.isnan()], b[~b.isnan()]) and torch.equal(a.isnan(), b.isnan())
+    y = ops.gemm_nt(x, w)
+    assert same(ops.gemm_f32_gated(x, w), ops.silu_mul(y)) and same(ops.gemm_f32_gated(x, w, "gelu_tanh"), ops.gelu_mul(y))
+    h1, h2 = h.clone(), h.clone()
+    want = ops.add_rmsnorm(h2, y, weight, 1e-5, torch.empty_like(h))
+    assert same(ops.gemm_f32_norm(x, w, h1, weight, 1e-5), want) and same(h1, h2)
+    wide = torch.randn(M, K + 4, device=DEV)[:, :K]  # rows further apart
+    wide.copy_(x)
+    assert same(ops.gemm_f32_norm(wide, w, h.clone(), weight, 1e-5), want)
+    hd, n_kv, P = 16, 4, 16
+    for from_key in (False, True):
+        H, rot = N // hd - (1 if from_key else 2) * n_kv, 8
+        pos = torch.arange(M, dtype=torch.int32, device=DEV) * 3
+        table = ops.rope_table(pos, torch.rand(rot // 2, device=DEV))
+        slots = torch.randperm(M + 20)[:M].to(torch.int32).to(DEV)
+        slots[M // 3] = -1
+        pages = [torch.full((M // P + 2, n_kv, *s), 7.0, device=DEV) for s in ((P, hd), (hd, P)) * 2]
+        q = ops.gemm_f32_qkv(x, w, table, pos, slots, *pages[:2], H, n_kv, hd, rot, from_key)
+        rows = y.clone()
+        ops.rope_kv_write(rows, pos, None, slots, *pages[2:], H, n_kv, hd, rot, table=table, v_col=H * hd if from_key else None)
+        assert same(q[:, :H * hd], rows[:, :H * hd]) and same(pages[0], pages[2]) and same(pages[1], pages[3])
