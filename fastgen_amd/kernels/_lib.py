@@ -14,6 +14,7 @@ from __future__ import annotations
 import ctypes
 import hashlib
 import os
+import re
 import shutil
 import subprocess
 import sys
@@ -73,12 +74,44 @@ VARIANT_LIBRARIES: Dict[str, tuple] = {
     "sigmoid_attention_mfma": ("sigmoid_attention_mfma.hip", "FG_HD", tuple(range(16, 257, 16)), ()),
 }
 
-_loaded: Dict[str, ctypes.CDLL] = {}
+_loaded: Dict[str, "Library"] = {}
 _lock = threading.Lock()
 
 
 class KernelBuildError(RuntimeError):
     pass
+
+
+_ENTRY = re.compile(r'extern "C"\s+([\w ]+?[\s*]+)(fg_\w+)\s*\(([^)]*)\)')
+_C_TYPES = {"int": ctypes.c_int, "long long": ctypes.c_longlong, "float": ctypes.c_float, "hipStream_t": ctypes.c_void_p}
+
+
+def entry_types(source: str) -> Dict[str, tuple]:
+    """The C entries that a kernel source defines: name -> (result type, argument types) for ``ctypes``."""
+    def of(decl: str):
+        decl = " ".join(decl.split())
+        if "*" in decl:
+            return ctypes.c_char_p if decl == "const char*" else ctypes.c_void_p
+        return _C_TYPES[decl]
+
+    return {name: (of(result), [of(a if "*" in a else a.rsplit(None, 1)[0]) for a in args.split(",") if a.strip()])
+            for result, name, args in _ENTRY.findall(source)}
+
+
+class Library:
+    """A loaded kernel library.  Its entries take plain integers for pointers and streams (and None), plain numbers for the
+    rest: their argument types stand in the source, and a step that has a few hundred launches makes no ``ctypes`` object for any."""
+
+    def __init__(self, path: Path, source: str) -> None:
+        self._dll, self._types = ctypes.CDLL(str(path)), entry_types(source)
+
+    def __getattr__(self, name: str):
+        if name not in self.__dict__.get("_types", ()):
+            raise AttributeError(f"no kernel entry {name!r}")
+        fn = getattr(self._dll, name)
+        fn.restype, fn.argtypes = self._types[name]
+        self.__dict__[name] = fn  # looked up once
+        return fn
 
 
 def _hipcc() -> str:
@@ -202,7 +235,7 @@ def build_all(*, force: bool = True, verbose: bool = True, jobs: int = 8) -> Dic
     return out  # type: ignore[return-value]
 
 
-def load(name: str) -> ctypes.CDLL:
+def load(name: str) -> Library:
     """The loaded library ``name``; found, or compiled at this first call."""
     lib = _loaded.get(name)
     if lib is not None:
@@ -215,7 +248,7 @@ def load(name: str) -> ctypes.CDLL:
             raise KeyError(f"no kernel library named {name!r}")
         path = find_built(name) or compile_library(name)
         try:
-            lib = ctypes.CDLL(str(path))
+            lib = Library(path, (CSRC / _split_variant(name)[0]).read_text())
         except OSError as e:
             raise KernelBuildError(f"cannot load {path}: {e}") from e
         _loaded[name] = lib

@@ -180,9 +180,10 @@ def _rows_of(w) -> torch.Tensor:
 
 def _aligned(x: torch.Tensor, w) -> bool:
     w = _rows_of(w)
+    (ldx, unit_x), (ldw, unit_w) = x.stride(), w.stride()
     return (x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.shape[1] % 8 == 0
-            and x.stride(1) == 1 and w.stride(1) == 1 and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0
-            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+            and unit_x == 1 and unit_w == 1 and ldx % 8 == 0 and ldw % 8 == 0
+            and (x.data_ptr() | w.data_ptr()) % 16 == 0)
 
 
 def skinny_ok(x: torch.Tensor, w) -> bool:
@@ -434,12 +435,12 @@ def linear(x, w, out_dtype: Optional[torch.dtype] = None,
         if h.dtype == torch.float32 and h.is_contiguous() and h.shape == (rows, N):
             return ops.gemm_skinny_residual(src, sw, h, norm_w, eps)
 
-    if own and rows > SKINNY_ROWS and sw is not w and force in (None, "large"):  # (no open norm: those have few rows)
+    if own and rows > SKINNY_ROWS and sw is not w and (force is None or force == "large"):  # (no open norm: those have few rows)
         way = _large_way(rows, N, K, x.stride(0), silu, partials_ok and out_dtype == torch.bfloat16, out_dtype == torch.float32,
                          force is not None)
-        if way is not None and way[0]:
-            return ops.gemm_large(x, sw, out_dtype, gated if silu else False, way[1], way[0])
         if way is not None:
+            if way[0]:
+                return ops.gemm_large(x, sw, out_dtype, gated if silu else False, way[1], way[0])
             return ops.gemm_skinny(x, sw, out_dtype, gated if silu else False, way[1], wide=True)
 
     def library(m: StreamedMatrix) -> torch.Tensor:

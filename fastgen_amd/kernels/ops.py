@@ -40,28 +40,37 @@ def _need(cond: bool, msg: str) -> None:
         raise KernelArgumentError(msg)
 
 
+def _refuse(msg: str) -> bool:
+    """``ok or _refuse(f"...")``: a message that is put together only where it is needed."""
+    raise KernelArgumentError(msg)
+
+
 def _gpu(*tensors: Optional[torch.Tensor]) -> None:
     dev = None
     for t in tensors:
         if t is None:
             continue
-        _need(t.is_cuda, "fastgen_amd kernels run on the GPU only; got a tensor on " + str(t.device))
-        dev = dev or t.device
-        _need(t.device == dev, "operands live on different devices")
+        if not t.is_cuda:
+            raise KernelArgumentError("fastgen_amd kernels run on the GPU only; got a tensor on " + str(t.device))
+        d = t.device
+        if dev is None:
+            dev = d
+        elif d != dev:
+            raise KernelArgumentError("operands live on different devices")
 
 
-def _ptr(t: Optional[torch.Tensor]) -> ctypes.c_void_p:
-    return ctypes.c_void_p(t.data_ptr() if t is not None else 0)
+def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
+    return t.data_ptr() if t is not None else None
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)  # the stream's handle without a Stream object
 
 
-def _stream(t: torch.Tensor) -> ctypes.c_void_p:
+def _stream(t: torch.Tensor) -> int:
     """The device's current stream (a few hundred launches a step ask for it)."""
     if _raw_stream is not None:
-        return ctypes.c_void_p(_raw_stream(t.device.index if t.device.index is not None else torch.cuda.current_device()))
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+        return _raw_stream(t.get_device())
+    return torch.cuda.current_stream(t.device).cuda_stream
 
 
 def upload(values, dtype: torch.dtype, device: torch.device | str) -> torch.Tensor:
@@ -85,9 +94,9 @@ def _check(status: int, what: str) -> None:
 
 
 def _i32(t: torch.Tensor, name: str, n: Optional[int] = None) -> None:
-    _need(t.dtype == torch.int32 and t.is_contiguous(), f"{name} must be contiguous int32")
+    (t.dtype == torch.int32 and t.is_contiguous()) or _refuse(f"{name} must be contiguous int32")
     if n is not None:
-        _need(t.numel() >= n, f"{name} holds {t.numel()} entries, {n} are needed")
+        t.numel() >= n or _refuse(f"{name} holds {t.numel()} entries, {n} are needed")
 
 
 # --------------------------------------------------------------------- rows
@@ -101,7 +110,7 @@ def embed(table: torch.Tensor, tokens: torch.Tensor, out: torch.Tensor, scale: f
           "out must be contiguous float32 [n_tokens, dim]")
     st = _lib.load("rows").fg_embed(
         _ptr(table), _code(table), _ptr(tokens), _ptr(out), n, table.shape[1], table.shape[0],
-        ctypes.c_float(scale), _stream(out))
+        float(scale), _stream(out))
     _check(st, "embed")
     return out
 
@@ -146,8 +155,8 @@ def add_rmsnorm(h: torch.Tensor, delta: Optional[torch.Tensor], weight: torch.Te
         _need(delta.shape == h.shape and delta.is_contiguous() and delta.dtype == out.dtype,
               "delta must be contiguous, shaped like h, of out's dtype")
     st = _lib.load("rows").fg_add_rmsnorm(
-        _ptr(h), _ptr(delta), _ptr(parts), n_parts, ctypes.c_longlong(part_stride), _ptr(delta_scale), _ptr(weight),
-        _ptr(out), _ptr(rows), n_rows, dim, ctypes.c_float(eps), _code(out), _code(weight), _stream(out))
+        _ptr(h), _ptr(delta), _ptr(parts), n_parts, part_stride, _ptr(delta_scale), _ptr(weight),
+        _ptr(out), _ptr(rows), n_rows, dim, float(eps), _code(out), _code(weight), _stream(out))
     _check(st, "add_rmsnorm")
     return out
 
@@ -156,13 +165,13 @@ def _delta_args(h: torch.Tensor, delta: Optional[torch.Tensor], what: str):
     """C arguments (delta, dtype code, parts, n_parts, part stride) for what is to be added to the fp32
     stream ``h``: nothing, rows ``[T, dim]``, or fp32 partial sums ``[S, T, dim]``."""
     if delta is None:
-        return _ptr(None), F32, _ptr(None), 0, ctypes.c_longlong(0)
+        return None, F32, None, 0, 0
     if delta.dim() == 3:
-        _need(delta.dtype == torch.float32 and delta.shape[1:] == h.shape and delta.stride(2) == 1
-              and delta.stride(1) == h.shape[1], f"{what}: partial sums must be float32 [S, T, dim] with contiguous rows")
-        return _ptr(None), F32, _ptr(delta), delta.shape[0], ctypes.c_longlong(delta.stride(0))
-    _need(delta.shape == h.shape and delta.is_contiguous(), f"{what}: delta must be contiguous and shaped like h")
-    return _ptr(delta), _code(delta), _ptr(None), 0, ctypes.c_longlong(0)
+        (delta.dtype == torch.float32 and delta.shape[1:] == h.shape and delta.stride(2) == 1
+              and delta.stride(1) == h.shape[1]) or _refuse(f"{what}: partial sums must be float32 [S, T, dim] with contiguous rows")
+        return None, F32, delta.data_ptr(), delta.shape[0], delta.stride(0)
+    (delta.shape == h.shape and delta.is_contiguous()) or _refuse(f"{what}: delta must be contiguous and shaped like h")
+    return delta.data_ptr(), _code(delta), None, 0, 0
 
 
 def stream_add(h: torch.Tensor, delta: Optional[torch.Tensor], again: Optional[torch.Tensor],
@@ -192,7 +201,7 @@ def add_rows(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     _need(a.dim() == 2 and a.shape == b.shape and a.dtype == b.dtype and a.is_contiguous() and b.is_contiguous(),
           "a and b must be contiguous [T, dim] of one dtype")
     out = torch.empty((1, *a.shape), dtype=torch.float32, device=a.device)
-    st = _lib.load("rows").fg_add_rows(_ptr(a), _ptr(b), _ptr(out), ctypes.c_longlong(a.numel()), _code(a), _stream(a))
+    st = _lib.load("rows").fg_add_rows(_ptr(a), _ptr(b), _ptr(out), a.numel(), _code(a), _stream(a))
     _check(st, "add_rows")
     return out
 
@@ -219,7 +228,7 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float, out: Optional[tor
     _need(out.shape == x.shape and out.dtype == x.dtype and out.is_contiguous(), "out must match x")
     _need(weight.shape == (dim,) and weight.is_contiguous(), "weight must be [dim]")
     st = _lib.load("rows").fg_rmsnorm(
-        _ptr(x), _ptr(weight), _ptr(out), x.numel() // dim, dim, ctypes.c_float(eps), _code(x),
+        _ptr(x), _ptr(weight), _ptr(out), x.numel() // dim, dim, float(eps), _code(x),
         _code(weight), _stream(out))
     _check(st, "rmsnorm")
     return out
@@ -232,8 +241,7 @@ def interleave_gate_up(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
     16-row tile of a product with it holds both halves of 8 channels, so
     ``silu(gate) * up`` can be applied where the tile is stored."""
     hidden, dim = gate.shape
-    _need(up.shape == gate.shape and hidden % 8 == 0,
-          f"gate and up must have the same shape and a row count that is a multiple of 8 (got {hidden})")
+    (up.shape == gate.shape and hidden % 8 == 0) or _refuse(f"gate and up must have the same shape and a row count that is a multiple of 8 (got {hidden})")
     return torch.stack([gate.reshape(hidden // 8, 8, dim), up.reshape(hidden // 8, 8, dim)], dim=1).reshape(
         2 * hidden, dim)
 
@@ -312,8 +320,8 @@ def post_add_rmsnorm(h: torch.Tensor, delta: Optional[torch.Tensor], post_weight
         _need(delta.dtype == act, "delta must have out's dtype")
     w_any = post_weight if post_weight is not None else weight
     st = _lib.load("rows").fg_post_add_rmsnorm(
-        _ptr(h), d_ptr, parts, n_parts, part_stride, _ptr(post_weight), ctypes.c_float(post_eps), _ptr(weight),
-        _ptr(out), _ptr(rows), n_rows, dim, ctypes.c_float(eps), _DTYPE_CODE[act],
+        _ptr(h), d_ptr, parts, n_parts, part_stride, _ptr(post_weight), float(post_eps), _ptr(weight),
+        _ptr(out), _ptr(rows), n_rows, dim, float(eps), _DTYPE_CODE[act],
         _code(w_any) if w_any is not None else F32, _ptr(delta_bias), _stream(h))
     _check(st, "post_add_rmsnorm")
     return out
@@ -424,7 +432,7 @@ def softcap(x: torch.Tensor, cap: float) -> torch.Tensor:
     """``x = cap * tanh(x / cap)`` in place on contiguous fp32."""
     _gpu(x)
     _need(x.dtype == torch.float32 and x.is_contiguous() and cap > 0, "x must be contiguous float32, cap positive")
-    st = _lib.load("rows").fg_softcap(_ptr(x), ctypes.c_longlong(x.numel()), ctypes.c_float(cap), _stream(x))
+    st = _lib.load("rows").fg_softcap(_ptr(x), x.numel(), float(cap), _stream(x))
     _check(st, "softcap")
     return x
 
@@ -434,7 +442,7 @@ def scale_logits(x: torch.Tensor, factor: float) -> torch.Tensor:
     """``x *= factor`` in place on contiguous fp32."""
     _gpu(x)
     _need(x.dtype == torch.float32 and x.is_contiguous(), "x must be contiguous float32")
-    _check(_lib.load("rows").fg_scale(_ptr(x), ctypes.c_longlong(x.numel()), ctypes.c_float(factor), _stream(x)), "scale_logits")
+    _check(_lib.load("rows").fg_scale(_ptr(x), x.numel(), float(factor), _stream(x)), "scale_logits")
     return x
 
 
@@ -467,7 +475,7 @@ def rope_kv_write(qkv: torch.Tensor, positions: torch.Tensor, freqs: Optional[to
     T = qkv.shape[0]
     v_col = (n_heads + n_kv) * head_dim if v_col is None else int(v_col)
     width = max((n_heads + n_kv) * head_dim, v_col + n_kv * head_dim) if write_kv else n_heads * head_dim
-    _need(qkv.shape[1] >= width, f"qkv rows hold {qkv.shape[1]} elements, {width} are needed")
+    (qkv.shape[1] >= width) or _refuse(f"qkv rows hold {qkv.shape[1]} elements, {width} are needed")
     _need(v_col >= n_heads * head_dim and v_col % 8 == 0, "the values begin behind the queries, at a multiple of 8")
     _i32(positions, "positions", T)
     _need(head_dim % 2 == 0 and 0 <= rotary_dim <= head_dim and rotary_dim % 2 == 0,
@@ -571,12 +579,12 @@ def paged_attention_general(q: torch.Tensor, out: torch.Tensor, k_pages: torch.T
     _i32(seq_of_token, "seq_of_token", T)
     _i32(positions, "positions", T)
     _need(n_heads % n_kv == 0, "the number of heads must be a multiple of the number of kv heads")
-    _need(hd % 8 == 0 and hd <= 512, f"head size {hd} is not supported (multiple of 8, at most 512)")
-    _need(page_size % 8 == 0, f"page size {page_size} is not supported (multiple of 8)")
+    (hd % 8 == 0 and hd <= 512) or _refuse(f"head size {hd} is not supported (multiple of 8, at most 512)")
+    (page_size % 8 == 0) or _refuse(f"page size {page_size} is not supported (multiple of 8)")
     st = _lib.load("attention").fg_paged_attention_general_sink(
         _ptr(q), q.stride(0), _ptr(out), out.stride(0), _ptr(k_pages), _ptr(v_pages), _ptr(block_table),
         block_table.stride(0), block_table.shape[0], _ptr(seq_of_token), _ptr(positions), T, n_heads, n_kv, hd, page_size,
-        ctypes.c_float(scale), int(window or 0), _ptr(sinks), _ptr(distance), _code(q), _stream(q))
+        float(scale), int(window or 0), _ptr(sinks), _ptr(distance), _code(q), _stream(q))
     _check(st, "paged_attention_general")
     return out
 
@@ -622,6 +630,7 @@ def _mfma_attention(head_dim: int, exact: bool = False, dist: bool = False):
     return _lib.load(f"attention_mfma_exact@{head_dim}" if exact else f"attention_mfma@{head_dim}")
 
 
+@functools.lru_cache(maxsize=256)
 def attention_tile_rows(head_dim: int, small: bool = False, exact: bool = False, dist: bool = False) -> int:
     """Query rows of one item of the tile kernel for this head size: of its larger form (128 rows up to
     head size 128), or of the form with ``small`` items (64 rows, more and lighter workgroups)."""
@@ -670,7 +679,6 @@ def _plan_ordered(n_items: int, n_kv: int) -> bool:
 
 
 def _plan_ints(lib, max_chunks: int, ordered: bool) -> int:
-    lib.fg_attn_plan_ints.restype = ctypes.c_longlong
     return int(lib.fg_attn_plan_ints(max_chunks)) + (8 * max_chunks if ordered else 0)
 
 
@@ -696,6 +704,14 @@ def attention_plan(items: torch.Tensor, n_items: int, max_chunks: int, head_dim:
 
 _ONE_STREAM = bool(os.environ.get("FG_ONE_STREAM"))  # no kernel runs beside another
 _second: Dict[int, "torch.cuda.Stream"] = {}
+
+
+def _tiles_beside(n_workgroups: int) -> bool:
+    """Whether the tile kernel goes to the second stream.  Its two waits take the host 40 us a layer, which a step of short prompt
+    portions waits for: 32 requests decoding beside portions of 100 and 500 tokens, one stream and two, us: Buderax's layers
+    1,608 and 2,021, Gisodra's 8 requests 1,728 and 2,206, Llama 3B's 5,722 and 5,939.  From about a workgroup for every compute unit on (portions of 1,000 to
+    2,000 tokens) the two are level, 0.3 % for one stream to 0.8 % for two, and steps of more prompt tokens gain 1 %."""
+    return not _ONE_STREAM and 8 * n_workgroups >= 7 * compute_units()
 
 
 def _second_stream(device) -> "torch.cuda.Stream":
@@ -770,8 +786,8 @@ def paged_attention_mfma(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tens
     and ``window`` (made here if not given).  ``max_rows``: no small item has
     more rows (tokens times query heads per kv head) than this.  ``tile_rows``: the
     rows the big items were cut for (:func:`attention_tile_rows`; default: the larger form's).
-    With items of both kinds the tile kernel runs on a second stream beside the split kernel and
-    the current stream waits for it before this returns (not while a graph is captured, not with
+    With items of both kinds, and enough of the big ones to fill the GPU, the tile kernel runs on a second stream beside
+    the split kernel and the current stream waits for it before this returns (not while a graph is captured, not with
     ``FG_ONE_STREAM=1``).  ``exact_weights``: the build of the kernels in which the softmax weights enter
     the product with the values as two bfloat16 terms (16 significant bits).  ``sinks`` and ``distance``: as
     :func:`paged_attention_general` (a build of the kernels with exact weights takes the distance bias).  ``gate`` and
@@ -794,7 +810,7 @@ def paged_attention_mfma(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tens
     n_pages, n_kv, page_size, hd = k_pages.shape
     _need(q.dtype == torch.bfloat16 and out.dtype == torch.bfloat16 and k_pages.dtype == torch.bfloat16
           and v_pages.dtype == torch.bfloat16, "the MFMA attention kernels take bfloat16")
-    _need(hd % 16 == 0 and hd <= MFMA_MAX_HEAD_DIM, f"head size {hd}: multiples of 16 up to {MFMA_MAX_HEAD_DIM}")
+    (hd % 16 == 0 and hd <= MFMA_MAX_HEAD_DIM) or _refuse(f"head size {hd}: multiples of 16 up to {MFMA_MAX_HEAD_DIM}")
     _need(k_pages.is_contiguous() and v_pages.is_contiguous() and v_pages.shape == (n_pages, n_kv, hd, page_size),
           "k_pages [n_pages, KV, P, hd] and v_pages [n_pages, KV, hd, P] must be contiguous")
     _need(n_heads % n_kv == 0 and page_size % 8 == 0, "heads must be a multiple of kv heads, pages of 8 tokens")
@@ -808,11 +824,11 @@ def paged_attention_mfma(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tens
     lib = _mfma_attention(hd, exact_weights, dist)
     G = n_heads // n_kv
     beside = None
-    if (small_items is not None and small_items.numel() and big_items is not None and big_items.numel()
-            and not _ONE_STREAM and not torch.cuda.is_current_stream_capturing()):
+    if (small_items is not None and big_items is not None and small_items.numel() and big_items.numel()
+            and _tiles_beside(big_items.numel() // 4 * n_kv) and not torch.cuda.is_current_stream_capturing()):
         # a step with both kinds of items (prompt portions beside decoded tokens): the two kernels write
         # different rows of `out`, one is bound by the matrix cores and one by memory, so the tile kernel
-        # runs on a second stream beside the split kernel (3 % of a continuous-batching run)
+        # runs on a second stream beside the split kernel
         beside = _second_stream(q.device)
         beside.wait_event(torch.cuda.current_stream(q.device).record_event())
     if small_items is not None and small_items.numel():
@@ -826,15 +842,15 @@ def paged_attention_mfma(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tens
         if plan is None:
             plan = attention_plan(small_items, n, max_chunks, hd, window, min_tiles, exact_weights, dist,
                                   _plan_ordered(n, n_kv))
-        ordered = plan.numel() == _plan_ints(lib, max_chunks, True)
-        _need(plan.dtype == torch.int32 and (ordered or plan.numel() == _plan_ints(lib, max_chunks, False)),
-              "the plan does not fit the items and max_chunks")
+        more = plan.numel() - _plan_ints(lib, max_chunks, False)
+        ordered = more == 8 * max_chunks
+        _need(plan.dtype == torch.int32 and (ordered or more == 0), "the plan does not fit the items and max_chunks")
         part_o = torch.empty((max_chunks * n_kv * 16, hd), dtype=torch.float32, device=q.device)
         part_ml = torch.empty((max_chunks * n_kv * 16, 2), dtype=torch.float32, device=q.device)
         st = lib.fg_attn_split_sink(
             _ptr(q), q.stride(0), _ptr(out), out.stride(0), _ptr(k_pages), _ptr(v_pages), _ptr(block_table),
             block_table.stride(0), _ptr(plan), n, max_chunks, max_rows, _ptr(part_o), _ptr(part_ml), n_heads, n_kv, hd,
-            page_size, ctypes.c_float(scale), int(window or 0), _ptr(sinks), _ptr(distance), *gate_args, int(ordered),
+            page_size, float(scale), int(window or 0), _ptr(sinks), _ptr(distance), *gate_args, int(ordered),
             int(not leave_parts), _stream(q))
         _check(st, "attn_split")
         if leave_parts:
@@ -849,8 +865,8 @@ def paged_attention_mfma(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tens
         st = lib.fg_attn_tile_sink(
             _ptr(q), q.stride(0), _ptr(out), out.stride(0), _ptr(k_pages), _ptr(v_pages), _ptr(block_table),
             block_table.stride(0), _ptr(big_items), big_items.numel() // 4, tile_rows, n_heads, n_kv, hd, page_size,
-            ctypes.c_float(scale), int(window or 0), _ptr(sinks), _ptr(distance), *gate_args,
-            ctypes.c_void_p(beside.cuda_stream) if beside else _stream(q))
+            float(scale), int(window or 0), _ptr(sinks), _ptr(distance), *gate_args,
+            beside.cuda_stream if beside else _stream(q))
         _check(st, "attn_tile")
         if beside is not None:
             torch.cuda.current_stream(q.device).wait_event(beside.record_event())
@@ -886,7 +902,7 @@ def paged_attention(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v
         if ctx.seq_records is not None and int(ctx.q_lens.max()) * G <= 16:
             # every sequence is one item of the split kernel: its records are in the step's buffer
             # already (and are refreshed with it when the step is a replayed graph)
-            plan = (ctx.seq_records, None, ctx.n_seqs, None)
+            plan = (ctx.seq_records, None, ctx.n_seqs, None, min(16, G * int(ctx.q_lens.max())))
         else:
             tile_rows = attention_tile_rows(hd, False, exact_weights, dist)
             small, big = attention_items(ctx.q_lens, ctx.q_start_host, ctx.n_cached, G, tile_rows)
@@ -898,9 +914,9 @@ def paged_attention(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v
                 small, big = attention_items(ctx.q_lens, ctx.q_start_host, ctx.n_cached, G, tile_rows)
             both = upload(np.concatenate([small, big]).reshape(-1), torch.int32, q.device)
             plan = (both[: small.size] if small.size else None, both[small.size:] if big.size else None, len(small),
-                    tile_rows)
+                    tile_rows, 16 if big.size else min(16, G * int(ctx.q_lens.max())))
         ctx.scratch[items_key] = plan
-    small_d, big_d, n_small, tile_rows = plan
+    small_d, big_d, n_small, tile_rows, max_rows = plan  # rows of the largest small item: one token a sequence in a decode step
     chunks = split_plan = None
     if n_small:
         # how the items' key ranges are cut depends on the window: layers with the same one share the cut
@@ -910,10 +926,8 @@ def paged_attention(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v
         if split_plan is None:
             split_plan = ctx.scratch[key] = attention_plan(small_d, n_small, chunks, hd, window, _SPLIT_MIN_TILES,
                                                            exact_weights, dist, _plan_ordered(n_small, n_kv))
-    # rows of the largest small item: one token a sequence in a decode step (also a captured one)
-    rows = G * int(ctx.q_lens.max()) if big_d is None else 16
     return paged_attention_mfma(q, out, k_pages, v_pages, group.block_table, small_d, big_d, n_heads, scale,
-                                window, split_plan, chunks, max_rows=min(16, rows), tile_rows=tile_rows,
+                                window, split_plan, chunks, max_rows=max_rows, tile_rows=tile_rows,
                                 exact_weights=exact_weights, sinks=sinks, distance=distance, gate=gate,
                                 gate_sigmoid=gate_sigmoid, leave_parts=leave_parts)
 
@@ -1022,8 +1036,8 @@ def gemm_nt(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None
 def _f32_product(x: torch.Tensor, w: torch.Tensor, what: str, act: int = 0) -> Tuple[torch.Tensor, bool]:
     """The 32-bit product with a kernel behind it that adds the groups' sums up: ``(y [M, N], False)``, or ``(sums [groups, M, N],
     True)``.  ``act``: an epilogue code; the kernel of 16 rows stores the activation's ``[M, N / 2]`` itself."""
-    _need(x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[1] and x.dtype == w.dtype == torch.float32
-          and x.stride(1) == 1 and w.stride(1) == 1, f"{what}: x [M, K] and w [N, K] must be float32 with unit column stride")
+    (x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[1] and x.dtype == w.dtype == torch.float32
+          and x.stride(1) == 1 and w.stride(1) == 1) or _refuse(f"{what}: x [M, K] and w [N, K] must be float32 with unit column stride")
     (M, K), N = x.shape, w.shape[0]
     blocks, waves, split = gemm_f32_plan(M, N, K, compute_units(), True)
     act = 0 if split or blocks else act
@@ -1072,7 +1086,7 @@ def gemm_f32_norm(x: torch.Tensor, w: torch.Tensor, h: torch.Tensor, weight: tor
     if not split:
         return add_rmsnorm(h, y, weight, eps, out)
     st = _lib.load("gemm").fg_gemm_f32_sum_norm(*_f32_sums_args(y, x, w), _ptr(h), _ptr(weight), _ptr(out), M, N, K, x.stride(0), w.stride(0),
-                                                ctypes.c_float(eps), _stream(x))
+                                                float(eps), _stream(x))
     _check(st, "gemm_f32_norm")
     return out
 
@@ -1175,14 +1189,15 @@ def _weight_args(w, K: int, what: str):
     """C arguments (pointer, ldw) for the weight of a streaming product, a matrix or :class:`PackedWeight`
     (ldw = 0), checked against the k of x."""
     if isinstance(w, PackedWeight):
-        _gpu(w.data)
-        _need(w.data.dtype == torch.bfloat16 and w.data.is_contiguous() and w.k == K
-              and w.data.shape == (-(-w.n // 16), -(-w.k // 32), 64, 8) and w.data.data_ptr() % 16 == 0,
-              f"{what}: the packed weight does not fit x [M, {K}]")
-        return _ptr(w.data), 0
+        data, n = w.data, w.n
+        _gpu(data)
+        ptr = data.data_ptr()
+        (data.dtype == torch.bfloat16 and data.is_contiguous() and w.k == K and ptr % 16 == 0
+         and data.shape == ((n + 15) // 16, (K + 31) // 32, 64, 8)) or _refuse(f"{what}: the packed weight does not fit x [M, {K}]")
+        return ptr, 0
     _gpu(w)
-    _need(w.dim() == 2 and w.dtype == torch.bfloat16 and w.shape[1] == K, f"{what}: w must be bfloat16 [N, {K}]")
-    _need(w.stride(1) == 1 and w.stride(0) % 8 == 0 and w.data_ptr() % 16 == 0, f"{what}: w needs 16-byte aligned rows")
+    (w.dim() == 2 and w.dtype == torch.bfloat16 and w.shape[1] == K) or _refuse(f"{what}: w must be bfloat16 [N, {K}]")
+    (w.stride(1) == 1 and w.stride(0) % 8 == 0 and w.data_ptr() % 16 == 0) or _refuse(f"{what}: w needs 16-byte aligned rows")
     return _ptr(w), w.stride(0)
 
 
@@ -1221,12 +1236,12 @@ class NormedRows(ScaledRows):
 def _row_scale_args(x, M: int):
     """C arguments (ssq, n_parts, dim, eps) for ``x`` a tensor or :class:`ScaledRows`."""
     if not isinstance(x, ScaledRows):
-        return ctypes.c_void_p(0), 0, 0, ctypes.c_float(0.0)
+        return None, 0, 0, 0.0
     ssq = x.ssq
     _need(ssq.dtype == torch.float32 and ssq.is_contiguous() and ssq.dim() == 2 and ssq.shape[0] == M
           and ssq.is_cuda, "ssq must be contiguous float32 [M, n_parts] on the GPU")
     _need(x.dim > 0 and x.eps >= 0, "ScaledRows needs dim > 0 and eps >= 0")
-    return _ptr(ssq), ssq.shape[1], int(x.dim), ctypes.c_float(x.eps)
+    return _ptr(ssq), ssq.shape[1], int(x.dim), float(x.eps)
 
 
 def scale_rows(rows: torch.Tensor, ssq: torch.Tensor, dim: int, eps: float) -> torch.Tensor:
@@ -1236,7 +1251,7 @@ def scale_rows(rows: torch.Tensor, ssq: torch.Tensor, dim: int, eps: float) -> t
           and ssq.dtype == torch.float32 and ssq.shape[0] == rows.shape[0], "rows [T, D], ssq float32 [T, n_parts]")
     out = torch.empty_like(rows)
     st = _lib.load("rows").fg_scale_rows(_ptr(rows), _ptr(ssq), _ptr(out), rows.shape[0], rows.shape[1],
-                                         ssq.shape[1], int(dim), ctypes.c_float(eps), _code(rows), _stream(rows))
+                                         ssq.shape[1], int(dim), float(eps), _code(rows), _stream(rows))
     _check(st, "scale_rows")
     return out
 
@@ -1263,7 +1278,7 @@ def gemm_skinny_residual(x: torch.Tensor, w, h: torch.Tensor, norm_weight: torch
     ssq_out = torch.empty((M, n_parts), dtype=torch.float32, device=rows.device)
     sc = _row_scale_args(x, M)
     st = _lib.load("gemm_skinny").fg_gemm_skinny_fused(
-        _ptr(rows), rows.stride(0), w_ptr, ldw, ctypes.c_void_p(0), 0, M, N, K, 3, *sc,
+        _ptr(rows), rows.stride(0), w_ptr, ldw, None, 0, M, N, K, 3, *sc,
         _ptr(h), h.stride(0), _ptr(norm_weight), _code(norm_weight), _ptr(x_out), x_out.stride(0), _ptr(ssq_out),
         _stream(rows))
     _check(st, "gemm_skinny_residual")
@@ -1288,7 +1303,7 @@ def gemm_skinny(x, w, out_dtype: Optional[torch.dtype] = None,
     _need(x.dtype == torch.bfloat16 and x.dim() == 2, "gemm_skinny takes bfloat16 x [M, K]")
     M, K = x.shape
     N = w.shape[0]
-    _need(0 < M <= SKINNY_MAX_ROWS, f"gemm_skinny takes 1..{SKINNY_MAX_ROWS} rows, got {M}")
+    (0 < M <= SKINNY_MAX_ROWS) or _refuse(f"gemm_skinny takes 1..{SKINNY_MAX_ROWS} rows, got {M}")
     _need(K % 8 == 0 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0,
           "K must be a multiple of 8, rows 16-byte aligned")
     w_ptr, ldw = _weight_args(w, K, "gemm_skinny")
@@ -1306,17 +1321,17 @@ def gemm_skinny(x, w, out_dtype: Optional[torch.dtype] = None,
     if scaled is not None and wide:
         _need(M <= 16 and k_splits == 1 and out_dtype == torch.bfloat16, "scaled rows: at most 16 rows, bfloat16 out")
         st = lib.fg_gemm_skinny64(
-            _ptr(x), x.stride(0), w_ptr, ldw, _ptr(y), cols, ctypes.c_longlong(M * cols), 1, M, N,
+            _ptr(x), x.stride(0), w_ptr, ldw, _ptr(y), cols, M * cols, 1, M, N,
             K, _code(y), _gated_code(silu_mul_epilogue), *_row_scale_args(scaled, M), _stream(x))
     elif scaled is not None:
         _need(M <= 16 and out_dtype == torch.bfloat16, "scaled rows: at most 16 rows, bfloat16 out")
         st = lib.fg_gemm_skinny_fused(
             _ptr(x), x.stride(0), w_ptr, ldw, _ptr(y), y.stride(0), M, N, K, _gated_code(silu_mul_epilogue),
-            *_row_scale_args(scaled, M), ctypes.c_void_p(0), 0, ctypes.c_void_p(0), 0, ctypes.c_void_p(0), 0,
-            ctypes.c_void_p(0), _stream(x))
+            *_row_scale_args(scaled, M), None, 0, None, 0, None, 0,
+            None, _stream(x))
     elif wide:
         st = lib.fg_gemm_skinny64(
-            _ptr(x), x.stride(0), w_ptr, ldw, _ptr(y), cols, ctypes.c_longlong(M * cols), k_splits, M, N,
+            _ptr(x), x.stride(0), w_ptr, ldw, _ptr(y), cols, M * cols, k_splits, M, N,
             K, _code(y), _gated_code(silu_mul_epilogue), *_row_scale_args(None, M), _stream(x))
     else:
         st = lib.fg_gemm_skinny(
@@ -1342,7 +1357,7 @@ def gemm_tiled(x: torch.Tensor, w, out_dtype: Optional[torch.dtype] = None,
     _need(M > 0 and K % 8 == 0 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0,
           "K must be a multiple of 8, rows 16-byte aligned")
     w_ptr, ldw = _weight_args(w, K, "gemm_tiled")
-    _need(tile_rows in TILED_TILE_ROWS, f"tile_rows must be one of {TILED_TILE_ROWS}")
+    (tile_rows in TILED_TILE_ROWS) or _refuse(f"tile_rows must be one of {TILED_TILE_ROWS}")
     out_dtype = out_dtype or torch.bfloat16
     if silu_mul_epilogue:
         _need(N % 16 == 0 and out_dtype == torch.bfloat16 and k_splits == 1,
@@ -1353,7 +1368,7 @@ def gemm_tiled(x: torch.Tensor, w, out_dtype: Optional[torch.dtype] = None,
     cols = N // 2 if silu_mul_epilogue else N
     y = torch.empty((k_splits, M, cols) if k_splits > 1 else (M, cols), dtype=out_dtype, device=x.device)
     st = _lib.load("gemm_tiled").fg_gemm_tiled(
-        _ptr(x), x.stride(0), w_ptr, ldw, _ptr(y), cols, ctypes.c_longlong(M * cols), k_splits, M, N, K,
+        _ptr(x), x.stride(0), w_ptr, ldw, _ptr(y), cols, M * cols, k_splits, M, N, K,
         _code(y), _gated_code(silu_mul_epilogue), int(tile_rows), _stream(x))
     _check(st, "gemm_tiled")
     return y
@@ -1460,7 +1475,7 @@ def _large_sizes(M: int, N: int, K: int, ldx: int, gated: bool, out_dtype: torch
     _need(1 <= k_splits <= 64 and -(-(K // 64) // k_splits) * (k_splits - 1) < K // 64, "a split of k would be empty")
     if tile is None:
         tile = large_plan(M, N, K, gated)[0]
-    _need(tile in LARGE_TILES, f"tile must be one of {LARGE_TILES}")
+    (tile in LARGE_TILES) or _refuse(f"tile must be one of {LARGE_TILES}")
     return int(tile), large_whole_tiles(tile, M, N)
 
 
@@ -1479,12 +1494,15 @@ def gemm_large(x: torch.Tensor, w: "PackedWeight", out_dtype: Optional[torch.dty
     out_dtype = out_dtype or torch.bfloat16
     tile, whole = _large_sizes(M, N, K, ldx, gated, out_dtype, k_splits, tile)
     cols = N // 2 if gated else N
-    shape, out_dtype = ((M, cols), out_dtype) if k_splits == 1 else ((k_splits, M, cols), torch.float32)
-    y = torch.empty(shape, dtype=out_dtype, device=x.device)
+    if k_splits == 1:
+        y = torch.empty((M, cols), dtype=out_dtype, device=x.device)
+    else:
+        y = torch.empty((k_splits, M, cols), dtype=torch.float32, device=x.device)
     st = _lib.load("gemm_large").fg_gemm_large(
-        ctypes.c_void_p(x_ptr), ldx, w_ptr, _ptr(y), cols, ctypes.c_longlong(M * cols), k_splits, M, N, K, _code(y),
-        _gated_code(silu_mul_epilogue), tile, whole, _stream(x))
-    _check(st, "gemm_large")
+        x_ptr, ldx, w_ptr, y.data_ptr(), cols, M * cols, k_splits, M, N, K, _DTYPE_CODE[y.dtype],
+        _gated_code(silu_mul_epilogue) if gated else 0, tile, whole, _stream(x))
+    if st:
+        _check(st, "gemm_large")
     return y
 
 
@@ -1508,7 +1526,7 @@ def gemm_skinny_qkv(x, wqkv, table: Optional[torch.Tensor], slots: torch.Tensor,
     w_ptr, ldw = _weight_args(wqkv, K, "gemm_skinny_qkv")
     gate_cols = n_heads * head_dim if gate else 0
     n_rows = (n_heads + (1 if value_from_key else 2) * n_kv) * head_dim + gate_cols
-    _need(0 < M <= 16 and tuple(wqkv.shape) == (n_rows, K), f"x [M<=16, K], wqkv [{n_rows}, K]")
+    (0 < M <= 16 and tuple(wqkv.shape) == (n_rows, K)) or _refuse(f"x [M<=16, K], wqkv [{n_rows}, K]")
     _need(K % 8 == 0 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0,
           "K must be a multiple of 8, rows 16-byte aligned")
     _need(head_dim % 16 == 0, "head size must be a multiple of 16")
@@ -1546,10 +1564,10 @@ def sample(logits: torch.Tensor, temperature: Optional[torch.Tensor] = None,
     _i32(out, "out", n)
     for name, t in (("temperature", temperature), ("top_p", top_p)):
         if t is not None:
-            _need(t.dtype == torch.float32 and t.is_contiguous() and t.numel() >= n, f"{name} must be float32 [n]")
+            (t.dtype == torch.float32 and t.is_contiguous() and t.numel() >= n) or _refuse(f"{name} must be float32 [n]")
     for name, t in (("seeds", seeds), ("counters", counters)):
         if t is not None:
-            _need(t.dtype == torch.int64 and t.is_contiguous() and t.numel() >= n, f"{name} must be int64 [n]")
+            (t.dtype == torch.int64 and t.is_contiguous() and t.numel() >= n) or _refuse(f"{name} must be int64 [n]")
     if temperature is not None:
         _need(seeds is not None and counters is not None, "sampling needs seeds and counters")
     st = _lib.load("sampling").fg_sample(
@@ -1603,7 +1621,7 @@ def moe_route(x: torch.Tensor, router: torch.Tensor, bias: Optional[torch.Tensor
           "router must be contiguous float32 [E + n_extra, dim]")
     if bias is not None:
         _need(bias.dtype == torch.float32 and bias.shape == (E,) and bias.is_contiguous(), "bias must be float32 [E]")
-    _need(1 <= top <= E, f"top={top} must be between 1 and the {E} experts")
+    (1 <= top <= E) or _refuse(f"top={top} must be between 1 and the {E} experts")
     choice = torch.empty((T, top), dtype=torch.int32, device=x.device)
     weight = torch.empty((T, top), dtype=torch.float32, device=x.device)
     _f32_vec(correction, E, "correction")
@@ -1611,12 +1629,11 @@ def moe_route(x: torch.Tensor, router: torch.Tensor, bias: Optional[torch.Tensor
     _need(scored or not (group_max or raw_weights), "group_max and raw_weights go with sigmoid or softmax scores")
     _need(scored or (correction is None and n_groups == 1), "correction and groups go with sigmoid or softmax scores")
     extra = torch.empty((T, n_extra), dtype=torch.float32, device=x.device) if n_extra else None
-    _need(n_groups >= 1 and E % n_groups == 0 and 1 <= keep_groups <= n_groups and top <= keep_groups * (E // n_groups),
-          f"{n_groups} groups of which {keep_groups} stay do not fit {E} experts and top={top}")
+    (n_groups >= 1 and E % n_groups == 0 and 1 <= keep_groups <= n_groups and top <= keep_groups * (E // n_groups)) or _refuse(f"{n_groups} groups of which {keep_groups} stay do not fit {E} experts and top={top}")
     st = _lib.load("moe").fg_moe_route_mode(_ptr(x), x.stride(0), _code(x), _ptr(router), _ptr(bias), T, dim, E, top,
                                             _ptr(choice), _ptr(weight), 2 if softmax_scores else int(bool(sigmoid_scores)),
                                             _ptr(correction), int(n_groups), int(keep_groups),
-                                            ctypes.c_float(weight_scale), int(n_extra), _ptr(extra), int(bool(group_max)),
+                                            float(weight_scale), int(n_extra), _ptr(extra), int(bool(group_max)),
                                             int(bool(raw_weights)), _stream(x))
     _check(st, "moe_route")
     return (choice, weight, extra) if n_extra else (choice, weight)
@@ -1722,8 +1739,8 @@ def moe_gate_up(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, sorte
     act = torch.empty((sorted_.numel(), hidden), dtype=x.dtype, device=x.device)
     st = _lib.load("moe").fg_moe_gate_up_act(_ptr(x), x.shape[0], w_gate.shape[0], x.stride(0), gate, up, ldw, _ptr(sorted_), _ptr(tiles),
                                              tiles.shape[0], tile_rows, top, dim, hidden, _ptr(act), hidden, _code(x),
-                                             int(mfma), ACT_LIMITED if limit > 0 else 0, ctypes.c_float(limit),
-                                             ctypes.c_float(alpha), _stream(x))
+                                             int(mfma), ACT_LIMITED if limit > 0 else 0, float(limit),
+                                             float(alpha), _stream(x))
     _check(st, "moe_gate_up")
     return act
 
@@ -1781,7 +1798,7 @@ def moe_combine(y: torch.Tensor, weight: torch.Tensor, plus: Optional[torch.Tens
             _need(x.dtype == torch.bfloat16, "bfloat16 rows are added to outputs of a bfloat16 x")
     out = torch.empty((1, T, dim), dtype=torch.float32, device=y.device)
     st = _lib.load("moe").fg_moe_combine_identity(_ptr(y), _ptr(weight), _ptr(plus), ldp, _code(plus) if plus is not None else F32,
-                                               n_plus, ctypes.c_longlong(stride), T, top, dim, _ptr(out), _ptr(plus_gate),
+                                               n_plus, stride, T, top, dim, _ptr(out), _ptr(plus_gate),
                                                plus_gate.stride(0) if plus_gate is not None else 0, _ptr(choice), int(n_tiled), _ptr(x),
                                                x.stride(0) if x is not None else 0, _code(x) if x is not None else F32, _stream(y))
     _check(st, "moe_combine")
@@ -1829,8 +1846,8 @@ class ExpertSum:
             ldp, n_plus = plus.stride(0), 1
         st = _lib.load("moe").fg_moe_combine_norm(
             _ptr(self.y), _ptr(self.weight), _ptr(plus), ldp, _code(plus) if plus is not None else F32, n_plus,
-            ctypes.c_longlong(stride), top, dim, _ptr(h), _ptr(weight), _code(weight), _ptr(out), _code(out), T,
-            ctypes.c_float(eps), _stream(out))
+            stride, top, dim, _ptr(h), _ptr(weight), _code(weight), _ptr(out), _code(out), T,
+            float(eps), _stream(out))
         _check(st, "moe_combine_norm")
         return out
 
@@ -1865,12 +1882,10 @@ class ConvInputs:
     def check(self, T: int, what: str) -> None:
         C, K = self.taps.shape
         _gpu(self.taps, self.state, self.slot_ids, self.seq_of_token, self.q_start)
-        _need(self.taps.dtype == torch.float32 and self.taps.is_contiguous() and 1 <= K <= CONV_MAX_TAPS,
-              f"{what}: taps must be contiguous float32 [C, 1..{CONV_MAX_TAPS}]")
-        _need(self.state.dtype == torch.float32 and self.state.dim() == 3 and self.state.shape[1] == C
+        (self.taps.dtype == torch.float32 and self.taps.is_contiguous() and 1 <= K <= CONV_MAX_TAPS) or _refuse(f"{what}: taps must be contiguous float32 [C, 1..{CONV_MAX_TAPS}]")
+        (self.state.dtype == torch.float32 and self.state.dim() == 3 and self.state.shape[1] == C
               and (self.state.stride(2) == 1 or self.state.shape[2] <= 1) and self.tail_off >= 0
-              and self.tail_off + K - 1 <= self.state.shape[2],
-              f"{what}: the state must be float32 [n_slots, C, >= tail_off + K - 1], rows contiguous")
+              and self.tail_off + K - 1 <= self.state.shape[2]) or _refuse(f"{what}: the state must be float32 [n_slots, C, >= tail_off + K - 1], rows contiguous")
         _i32(self.seq_of_token, "seq_of_token", T)
         _i32(self.slot_ids, "slot_ids")
         _i32(self.q_start, "q_start")
@@ -1919,7 +1934,7 @@ class _PrepareArgs(ctypes.Structure):
 
 def _f32_vec(t: Optional[torch.Tensor], n: int, name: str) -> None:
     if t is not None:
-        _need(t.dtype == torch.float32 and t.is_contiguous() and t.numel() >= n, f"{name} must be contiguous float32 [{n}]")
+        (t.dtype == torch.float32 and t.is_contiguous() and t.numel() >= n) or _refuse(f"{name} must be contiguous float32 [{n}]")
 
 
 def heads_prepare(src: torch.Tensor, bias: Optional[torch.Tensor], eps: float,
@@ -2084,7 +2099,7 @@ def head_norm_gate(x: torch.Tensor, weight: torch.Tensor, eps: float, gate: torc
     _need(gate.dim() == 2 and gate.stride(1) == 1 and gate.shape[0] == T and gate.shape[1] >= n_heads * e
           and gate.dtype in (out.dtype, torch.float32), "gate must be [T, >= H*e] of out's dtype or float32")
     st = _lib.load("heads").fg_head_norm_gate(_ptr(x), _ptr(weight), _ptr(gate), gate.stride(0), _ptr(out), out.stride(0),
-                                              T, n_heads, e, ctypes.c_float(eps), ctypes.c_float(out_scale), int(bool(sigmoid)), _code(out),
+                                              T, n_heads, e, float(eps), float(out_scale), int(bool(sigmoid)), _code(out),
                                               _code(gate), _stream(out))
     _check(st, "head_norm_gate")
     return out
@@ -2102,7 +2117,7 @@ def row_norm_gate(x: torch.Tensor, weight: torch.Tensor, eps: float, gate: torch
     _rows_of_width(out, T, W, "out")
     _need(gate.dtype == torch.float32 and W <= 16384, "gate must be float32, rows of at most 16384")
     st = _lib.load("heads").fg_row_norm_gate(_ptr(x), _ptr(weight), _ptr(gate), gate.stride(0), _ptr(out), out.stride(0), T, W,
-                                             ctypes.c_float(eps), ctypes.c_float(out_scale), _code(out), _stream(out))
+                                             float(eps), float(out_scale), _code(out), _stream(out))
     _check(st, "row_norm_gate")
     return out
 
@@ -2123,8 +2138,8 @@ def head_diff_norm(att: torch.Tensor, head_width: int, out: torch.Tensor, n_head
           and out.dtype == att.dtype, "out must be [T, >= H * v_width] of att's dtype")
     _need(group >= 1 and n_heads % group == 0 and v_width <= 1024, "heads in whole groups, of at most 1024 values")
     st = _lib.load("heads").fg_head_diff_norm(_ptr(att), att.stride(0), head_width, _ptr(out), out.stride(0), T, n_heads,
-                                              group, v_width, ctypes.c_float(lam), ctypes.c_float(eps),
-                                              ctypes.c_float(out_scale), _code(att), _stream(att))
+                                              group, v_width, float(lam), float(eps),
+                                              float(out_scale), _code(att), _stream(att))
     _check(st, "head_diff_norm")
     return out
 
@@ -2156,10 +2171,9 @@ STREAMS_MAX = 16
 def streams_spread(h: torch.Tensor, n_streams: int) -> torch.Tensor:
     """fp32 ``[S, T, dim]``: ``h [T, dim]`` copied into every one of ``n_streams`` residual streams."""
     _gpu(h)
-    _need(h.dtype == torch.float32 and h.dim() == 2 and h.is_contiguous() and 1 <= n_streams <= STREAMS_MAX,
-          f"h must be contiguous float32 [T, dim], at most {STREAMS_MAX} streams")
+    (h.dtype == torch.float32 and h.dim() == 2 and h.is_contiguous() and 1 <= n_streams <= STREAMS_MAX) or _refuse(f"h must be contiguous float32 [T, dim], at most {STREAMS_MAX} streams")
     x = torch.empty((n_streams, *h.shape), dtype=torch.float32, device=h.device)
-    _check(_lib.load("streams").fg_streams_spread(_ptr(h), _ptr(x), ctypes.c_longlong(h.numel()), n_streams, _stream(h)),
+    _check(_lib.load("streams").fg_streams_spread(_ptr(h), _ptr(x), h.numel(), n_streams, _stream(h)),
            "streams_spread")
     return x
 
@@ -2173,8 +2187,7 @@ def streams_step(x: torch.Tensor, update: Optional[StreamUpdate], in_weights: Op
     and/or ``u_out = u`` in fp32.  With ``rows`` only those tokens are computed, into consecutive rows, and ``x`` is
     left as it was."""
     _gpu(x, in_weights, norm_weight, out, rows, u_out, *(() if update is None else (update.rows, update.mix, update.out)))
-    _need(x.dtype == torch.float32 and x.dim() == 3 and x.is_contiguous() and 1 <= x.shape[0] <= STREAMS_MAX,
-          f"x must be contiguous float32 [S, T, dim], at most {STREAMS_MAX} streams")
+    (x.dtype == torch.float32 and x.dim() == 3 and x.is_contiguous() and 1 <= x.shape[0] <= STREAMS_MAX) or _refuse(f"x must be contiguous float32 [S, T, dim], at most {STREAMS_MAX} streams")
     S, T, dim = x.shape
     _need(dim <= 8192, "rows of at most 8192 elements")
     n_rows = T if rows is None else rows.numel()
@@ -2290,7 +2303,7 @@ def decay_scan(qkv: torch.Tensor, q_col: int, k_col: int, v_col: int, z: torch.T
     products = chunked and decay_scan_as_products(d)
     # the decays of every token at once (exponentials and logarithms stay out of the chain of tokens), or their logarithms
     decay = torch.empty((T, H * d), dtype=torch.float32, device=z.device)
-    st = lib.fg_decay_from_logits(_ptr(z), z.stride(0), _ptr(z_bias), ctypes.c_float(1.0 / tau), _ptr(decay), T, H * d,
+    st = lib.fg_decay_from_logits(_ptr(z), z.stride(0), _ptr(z_bias), float(1.0 / tau), _ptr(decay), T, H * d,
                                   int(products), _stream(z))
     _check(st, "decay_from_logits")
     a = _ScanArgs()
@@ -2346,7 +2359,7 @@ def gated_mul(gate_up: torch.Tensor, bias: Optional[torch.Tensor], activation: s
     ``gelu_tanh``, ``relu``, or ``limited``: ``g = min(gate, limit)``, ``u = clamp(up, -limit, limit)``,
     ``g * sigmoid(alpha * g) * (u + 1)``.  All of it in fp32, one rounding to ``out_dtype``."""
     _gpu(gate_up, bias, out)
-    _need(activation in _ACT_CODE, f"activation {activation!r} is not supported ({sorted(_ACT_CODE)})")
+    (activation in _ACT_CODE) or _refuse(f"activation {activation!r} is not supported ({sorted(_ACT_CODE)})")
     _need(gate_up.dim() == 2 and gate_up.is_contiguous() and gate_up.shape[1] % 16 == 0,
           "gate_up must be contiguous [T, 2 * hidden], hidden a multiple of 8")
     T, hidden = gate_up.shape[0], gate_up.shape[1] // 2
@@ -2357,7 +2370,7 @@ def gated_mul(gate_up: torch.Tensor, bias: Optional[torch.Tensor], activation: s
     _need(out.shape == (T, hidden) and out.is_contiguous() and out.dtype == out_dtype, "out must be contiguous [T, hidden]")
     _need(activation != "limited" or limit > 0, "the limited activation needs a positive limit")
     st = _lib.load("rows").fg_gated_mul_act(_ptr(gate_up), _ptr(bias), _ptr(out), T, hidden, _ACT_CODE[activation],
-                                            ctypes.c_float(limit), ctypes.c_float(alpha), _code(gate_up), _code(out),
+                                            float(limit), float(alpha), _code(gate_up), _code(out),
                                             _stream(out))
     _check(st, "gated_mul")
     return out
@@ -2370,7 +2383,7 @@ def bias_act(x: torch.Tensor, bias: Optional[torch.Tensor], activation: str, out
     """``act(x + bias)`` for contiguous ``x [T, hidden]`` (fp32, or ``out_dtype``; ``hidden`` a multiple of 8) and fp32 ``bias
     [hidden]`` or None; ``activation`` one of ``relu2`` (the square of ReLU), ``relu``, ``silu``, ``gelu_tanh``."""
     _gpu(x, bias)
-    _need(activation in _PLAIN_ACT_CODE, f"activation {activation!r} is not supported ({sorted(_PLAIN_ACT_CODE)})")
+    (activation in _PLAIN_ACT_CODE) or _refuse(f"activation {activation!r} is not supported ({sorted(_PLAIN_ACT_CODE)})")
     _need(x.dim() == 2 and x.is_contiguous() and x.shape[1] % 8 == 0, "x must be contiguous [T, hidden], hidden a multiple of 8")
     _need(x.dtype == torch.float32 or x.dtype == out_dtype, "x must be float32 or of the result's dtype")
     _f32_vec(bias, x.shape[1], "bias")
@@ -2398,8 +2411,7 @@ SELECTIVE_CHUNKED_FROM = 96  # the shortest run of tokens of one sequence for wh
 
 
 def _rows_of_width(t: torch.Tensor, T: int, width: int, name: str) -> None:
-    _need(t.dim() == 2 and t.stride(1) == 1 and t.shape[0] == T and t.shape[1] >= width,
-          f"{name} must be [T, >= {width}] with unit column stride")
+    (t.dim() == 2 and t.stride(1) == 1 and t.shape[0] == T and t.shape[1] >= width) or _refuse(f"{name} must be [T, >= {width}] with unit column stride")
 
 
 def causal_conv(x: torch.Tensor, taps: torch.Tensor, bias: Optional[torch.Tensor], state: torch.Tensor, tail_off: int,
