@@ -386,28 +386,51 @@ __global__ __launch_bounds__(512, 4) void gemm_f32_few_kernel(const float* __res
   if (tid < 128 && m < M) y[(size_t)m * ldy + n0 / 2 + (tid / 64) * 4 + tid % 4] = gf_gated(total, ups[tid], act);
 }
 
+// Rows cut beforehand: [ceil(n / 16)][K / 32][3][64][8], a block's three parts of a step in operand order (K a multiple of 32; rows that are
+// not there are zeros).  A wave takes a step of 16 rows.
+__global__ __launch_bounds__(256) void gemm_f32_cut_kernel(const float* __restrict__ rows, int ld, int n, int K, bf16x8* __restrict__ out) {
+  const int lane = threadIdx.x % FG_WAVE, steps = K / GF_STEP, step = blockIdx.y * 4 + threadIdx.x / FG_WAVE;
+  const int row = blockIdx.x * 16 + lane % 16;
+  if (step >= steps) return;
+  f32x4 lo = {0.f, 0.f, 0.f, 0.f}, hi = lo;
+  if (row < n) {
+    const float* from = rows + (size_t)row * ld + step * GF_STEP + lane / 16 * 4;
+    lo = *(const f32x4*)from;
+    hi = *(const f32x4*)(from + 16);
+  }
+  const GfParts c = gf_parts(lo, hi);
+  bf16x8* to = out + ((size_t)blockIdx.x * steps + step) * 192 + lane;
+#pragma unroll
+  for (int p = 0; p < 3; ++p) to[64 * p] = c.p[p];
+}
+
 // Many rows: bound by the matrix cores at the clock they can hold.  NW waves own 16 MB rows x 16 NB NW outputs, each
-// all the rows and 16 NB outputs: a wave takes its rows of W from memory into registers itself, cuts them into parts
-// once and reads every x from LDS, where the workgroup has put its three parts in the operands' order, 32 k at a time
-// in two buffers.  The two waves of a SIMD cut W on either side of their matrix instructions (`late`), so that one's
-// vector work runs beside the other's products.  AHEAD: steps of W and x in flight, in registers; their loads stand
+// all the rows and 16 NB outputs: a wave takes its rows of W from memory into registers itself and reads every x from LDS, where the
+// workgroup has put its three parts in the operands' order, 32 k at a time in two buffers.
+// Operands as they are: a wave cuts W into parts once, and the two waves of a SIMD do it on either side of their matrix instructions
+// (`late`), so that one's vector work runs beside the other's products.
+// CUT, operands cut beforehand (xp, wp; K a multiple of 128): two fifths of the vector work are gone, and what is left, the sums, fits between
+// the matrix instructions, two behind each.  Half as many bytes of W again, so not for a few rows.
+// AHEAD: steps of W and x in flight, in registers; their loads stand
 // under no condition (with one the compiler copies what it has just loaded, that is, waits for it: 1.7 us a step
 // instead of 0.6 where the products take 0.1).  A group's sum is kept in LDS, which leaves the registers to the loads.
 // With `part` a workgroup takes one group of k and stores its sum there ([groups][M][N]); else it adds each group's to
 // y.  A die's workgroups are an eighth of the tiles, those that read the same rows of W one after the other.
 //
-// N x K 16384 x 3072 / 5120 x 3072 / 3072 x 8192, us: 400 rows 290 / 105 / 159 (459 / 167 / 256 with the fp32
-// instructions), 2048 rows 1326 / 483 / 702 (1900 / 622 / 1000): 0.93 PFLOP/s of bf16 at the largest, against 1.4 that
+// N x K 16384 x 3072 / 5120 x 3072 / 3072 x 8192, us: 400 rows 283 / 105 / 160, cut 237 / 89 / 129 (459 / 167 / 256 with the fp32
+// instructions), 2000 rows 1300 / 412 / 641, cut 1103 / 344 / 543: 1.1 PFLOP/s of bf16, against 1.4 that
 // a product of bf16 operands reaches; with the sums on the matrix core itself, cut off there, 12 % less.
 // FAR: rows so far apart that a tile spans 4 GB, with offsets of 64 bits (of 32, a load is one register of offset behind
 // a uniform base).
-template <int MB, int NB, int NW, int AHEAD, bool VEC, bool FAR>
+template <int MB, int NB, int NW, int AHEAD, bool VEC, bool FAR, bool CUT>
 __global__ __launch_bounds__(64 * NW, 2) void gemm_f32_tiled_kernel(
-    const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ y, float* __restrict__ part, int M,
-    int N, int K, int ldx, int ldw, int ldy, int row_tiles, int col_tiles, int units, int wide) {
-  constexpr int TM = 16 * MB, TN = 16 * NB * NW, XV = (TM * 8 + 64 * NW - 1) / (64 * NW);
+    const float* __restrict__ x, const float* __restrict__ w, const bf16x8* __restrict__ xp, const bf16x8* __restrict__ wp,
+    float* __restrict__ y, float* __restrict__ part, int M, int N, int K, int ldx, int ldw, int ldy, int row_tiles, int col_tiles, int units,
+    int wide) {
+  // pieces of x that a thread brings a step: four k of a row, or eight of a part
+  constexpr int TM = 16 * MB, TN = 16 * NB * NW, XV = ((CUT ? MB * 192 : TM * 8) + 64 * NW - 1) / (64 * NW);
   static_assert(4 % AHEAD == 0, "a segment's steps use the sets of registers in turn");
-  __shared__ bf16x4 xs[2][MB][3][FG_WAVE][2];
+  __shared__ bf16x8 xs[2][CUT ? XV * 64 * NW : MB * 192];  // [block][part][lane]
   __shared__ f32x4 mids[NW][MB * NB][FG_WAVE];
   const int tile = blockIdx.x % 8 * (gridDim.x / 8) + blockIdx.x / 8;  // (workgroup i runs on die i % 8)
   if (tile >= units * row_tiles) return;
@@ -421,55 +444,92 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_f32_tiled_kernel(
   const float *wb = w + (size_t)min(n0, N - 1) * ldw, *xb = x + (size_t)m0 * ldx;
   using Offset = std::conditional_t<FAR, size_t, unsigned>;
   Offset wo[NB], xo[XV];  // in bytes
+  const int steps = K / GF_STEP, piece = tid % 8, row = tid / 8;  // of x as it is: the rows 8 NW apart
+  const char *wc = nullptr, *xc = nullptr;
+  if constexpr (CUT) {
+    const int last = (N + 15) / 16 - 1, first = min(n0 / 16, last);
+    wc = (const char*)(wp + (size_t)first * steps * 192);
+    xc = (const char*)(xp + (size_t)(m0 / 16) * steps * 192);
 #pragma unroll
-  for (int j = 0; j < NB; ++j) wo[j] = 4 * ((Offset)min(16 * j + r, max(N - 1 - n0, 0)) * ldw + 4 * g);
-  const int piece = tid % 8, row = tid / 8;  // of x: four k of a row, the rows 8 NW apart
+    for (int j = 0; j < NB; ++j) wo[j] = 16 * ((unsigned)min(j, last - first) * steps * 192 + lane);
 #pragma unroll
-  for (int i = 0; i < XV; ++i) xo[i] = 4 * ((Offset)min(row + 8 * NW * i, M - 1 - m0) * ldx + 4 * piece);
+    for (int i = 0; i < XV; ++i) {
+      const int c = tid + 64 * NW * i, block = min(c / 192, min(MB, (M - m0 + 15) / 16) - 1);
+      xo[i] = 16 * ((unsigned)block * steps * 192 + c % 192);
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < NB; ++j) wo[j] = 4 * ((Offset)min(16 * j + r, max(N - 1 - n0, 0)) * ldw + 4 * g);
+#pragma unroll
+    for (int i = 0; i < XV; ++i) xo[i] = 4 * ((Offset)min(row + 8 * NW * i, M - 1 - m0) * ldx + 4 * piece);
+  }
 
-  f32x4 raw[AHEAD][NB][2], xv[AHEAD][XV], sum[MB][NB];
-  GfParts wp[NB];
+  f32x4 raw[CUT ? 1 : AHEAD][NB][2], xv[CUT ? 1 : AHEAD][XV], sum[MB][NB];
+  bf16x8 xcut[CUT ? AHEAD : 1][XV];
+  GfParts wpart[CUT ? AHEAD : 1][NB];
   // a whole step; what would be loaded ahead behind the last whole segment is its last step again
   auto load_w = [&](int set, int k) {
-    const char* at = (const char*)(wb + min(k, k_full - GF_STEP));
+    k = min(k, k_full - GF_STEP);
+    if constexpr (CUT) {
 #pragma unroll
-    for (int j = 0; j < NB; ++j) {
-      raw[set][j][0] = gf_whole4<VEC>((const float*)(at + wo[j]));
-      raw[set][j][1] = gf_whole4<VEC>((const float*)(at + wo[j]) + 16);
+      for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int p = 0; p < 3; ++p) wpart[set][j].p[p] = *(const bf16x8*)(wc + (size_t)(k / GF_STEP) * 3072 + wo[j] + 1024 * p);
+    } else {
+      const char* at = (const char*)(wb + k);
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        raw[set][j][0] = gf_whole4<VEC>((const float*)(at + wo[j]));
+        raw[set][j][1] = gf_whole4<VEC>((const float*)(at + wo[j]) + 16);
+      }
     }
   };
   auto load_x = [&](int set, int k) {
-    const char* at = (const char*)(xb + min(k, k_full - GF_STEP));
+    k = min(k, k_full - GF_STEP);
 #pragma unroll
-    for (int i = 0; i < XV; ++i) xv[set][i] = gf_whole4<VEC>((const float*)(at + xo[i]));
+    for (int i = 0; i < XV; ++i) {
+      if constexpr (CUT) xcut[set][i] = *(const bf16x8*)(xc + (size_t)(k / GF_STEP) * 3072 + xo[i]);
+      else xv[set][i] = gf_whole4<VEC>((const float*)((const char*)(xb + k) + xo[i]));
+    }
   };
   auto store_x = [&](int set, int buf) {
 #pragma unroll
     for (int i = 0; i < XV; ++i) {
-      const int at = row + 8 * NW * i;
-      if (TM % (8 * NW) == 0 || at < TM) {
-        bf16x4(*to)[FG_WAVE][2] = xs[buf][at / 16];
-        const int l = (piece % 4) * 16 + at % 16, half = piece / 4;
-        gf_parts4(xv[set][i], &to[0][l][half], &to[1][l][half], &to[2][l][half]);
+      if constexpr (CUT) {
+        xs[buf][tid + 64 * NW * i] = xcut[set][i];
+      } else {
+        const int at = row + 8 * NW * i;
+        if (TM % (8 * NW) == 0 || at < TM) {
+          bf16x8* to = xs[buf] + at / 16 * 192 + (piece % 4) * 16 + at % 16;
+          const int half = piece / 4;
+          gf_parts4(xv[set][i], (bf16x4*)to + half, (bf16x4*)(to + 64) + half, (bf16x4*)(to + 128) + half);
+        }
       }
     }
   };
   auto cut_w = [&](int set) {
 #pragma unroll
-    for (int j = 0; j < NB; ++j) wp[j] = gf_parts(raw[set][j][0], raw[set][j][1]);
+    for (int j = 0; j < NB; ++j) wpart[0][j] = gf_parts(raw[set][j][0], raw[set][j][1]);
   };
-  auto multiply = [&](int buf) {
+  auto multiply = [&](int buf, int set) {
     GfTerms terms[2][NB];  // a row of blocks is added up behind the next one's products
 #pragma unroll
     for (int i = 0; i < MB; ++i) {
       bf16x8 b[3];
 #pragma unroll
-      for (int p = 0; p < 3; ++p) b[p] = *(const bf16x8*)&xs[buf][i][p][lane][0];
+      for (int p = 0; p < 3; ++p) b[p] = xs[buf][(3 * i + p) * 64 + lane];
 #pragma unroll
-      for (int j = 0; j < NB; ++j) terms[i % 2][j] = gf_step(wp[j], b[0], b[1], b[2]);
+      for (int j = 0; j < NB; ++j) terms[i % 2][j] = gf_step(wpart[set][j], b[0], b[1], b[2]);
       if (i > 0) {
 #pragma unroll
         for (int j = 0; j < NB; ++j) gf_fold(sum[i - 1][j], terms[(i - 1) % 2][j]);
+        if constexpr (CUT && MB > 5) {  // (in smaller tiles the compiler's own order is as good)
+#pragma unroll
+          for (int z = 0; z < 6 * NB; ++z) {
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);  // a matrix instruction
+            __builtin_amdgcn_sched_group_barrier(0x2, 2, 0);  // two vector instructions
+          }
+        }
       }
     }
 #pragma unroll
@@ -518,39 +578,47 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_f32_tiled_kernel(
       load_w(a, k_begin + a * GF_STEP);
     }
     store_x(0, 0);
-    if (late) cut_w(0);
+    if (!CUT && late) cut_w(0);
     __syncthreads();
     for (int k0 = k_begin; k0 < k_full; k0 += GF_SEG) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int k = k0 + q * GF_STEP, buf = q % 2;
         load_x(q % AHEAD, k + AHEAD * GF_STEP);
-        if (!late) cut_w(q % AHEAD);
-        load_w(q % AHEAD, k + AHEAD * GF_STEP);
-        multiply(buf);
-        if (late) cut_w((q + 1) % AHEAD);
-        store_x((q + 1) % AHEAD, buf ^ 1);
+        if constexpr (CUT) {
+          store_x((q + 1) % AHEAD, buf ^ 1);
+          multiply(buf, q % AHEAD);
+          load_w(q % AHEAD, k + AHEAD * GF_STEP);
+        } else {
+          if (!late) cut_w(q % AHEAD);
+          load_w(q % AHEAD, k + AHEAD * GF_STEP);
+          multiply(buf, 0);
+          if (late) cut_w((q + 1) % AHEAD);
+          store_x((q + 1) % AHEAD, buf ^ 1);
+        }
         __syncthreads();
       }
       close(k0);
     }
   }
-  if (k_full < k_end) {  // less than a segment at the end of the rows
-    for (int k = k_full; k < k_end; k += GF_STEP) {
+  if constexpr (!CUT) {
+    if (k_full < k_end) {  // less than a segment at the end of the rows
+      for (int k = k_full; k < k_end; k += GF_STEP) {
 #pragma unroll
-      for (int i = 0; i < XV; ++i) xv[0][i] = gf_load4<VEC>(xb + xo[i] / 4 - 4 * piece, k + 4 * piece, k_end);
+        for (int i = 0; i < XV; ++i) xv[0][i] = gf_load4<VEC>(xb + xo[i] / 4 - 4 * piece, k + 4 * piece, k_end);
 #pragma unroll
-      for (int j = 0; j < NB; ++j) {
-        raw[0][j][0] = gf_load4<VEC>(wb + wo[j] / 4 - 4 * g, k + 4 * g, k_end);
-        raw[0][j][1] = gf_load4<VEC>(wb + wo[j] / 4 - 4 * g, k + 16 + 4 * g, k_end);
+        for (int j = 0; j < NB; ++j) {
+          raw[0][j][0] = gf_load4<VEC>(wb + wo[j] / 4 - 4 * g, k + 4 * g, k_end);
+          raw[0][j][1] = gf_load4<VEC>(wb + wo[j] / 4 - 4 * g, k + 16 + 4 * g, k_end);
+        }
+        store_x(0, 0);
+        cut_w(0);
+        __syncthreads();
+        multiply(0, 0);
+        __syncthreads();
       }
-      store_x(0, 0);
-      cut_w(0);
-      __syncthreads();
-      multiply(0);
-      __syncthreads();
+      close(k_full);
     }
-    close(k_full);
   }
 }
 
@@ -693,6 +761,7 @@ struct GfCall {
   float *y, *part;
   int M, N, K, ldx, ldw, ldy, vec;
   hipStream_t stream;
+  const bf16x8 *xp, *wp;  // the operands cut beforehand, or null
 };
 
 static int gf_wide(const GfCall& c) {
@@ -708,7 +777,7 @@ static int gf_sum(const GfCall& c) {
   return fg_launch_status();
 }
 
-template <int MB, int NB, int NW, bool FAR = false>
+template <int MB, int NB, int NW, bool FAR = false, bool CUT = false>
 static int gf_launch(const GfCall& c) {
   constexpr int AHEAD = MB <= 3 ? 4 : 2;
   const int groups = (c.K + GF_GROUP - 1) / GF_GROUP;
@@ -718,9 +787,10 @@ static int gf_launch(const GfCall& c) {
   const long long blocks = (units * row_tiles + 7) / 8 * 8;
   if (blocks > 2147483647LL || (c.part && c.M > 65535)) return FG_ERR_ARG;
 #define TILED(VEC)                                                                                            \
-  gemm_f32_tiled_kernel<MB, NB, NW, AHEAD, VEC, FAR><<<(unsigned)blocks, 64 * NW, 0, c.stream>>>(                  \
-      c.x, c.w, c.y, c.part, c.M, c.N, c.K, c.ldx, c.ldw, c.ldy, row_tiles, col_tiles, (int)units, wide)
-  if (c.vec) TILED(true);
+  gemm_f32_tiled_kernel<MB, NB, NW, AHEAD, VEC, FAR, CUT><<<(unsigned)blocks, 64 * NW, 0, c.stream>>>(             \
+      c.x, c.w, c.xp, c.wp, c.y, c.part, c.M, c.N, c.K, c.ldx, c.ldw, c.ldy, row_tiles, col_tiles, (int)units, wide)
+  if constexpr (CUT) TILED(true);
+  else if (c.vec) TILED(true);
   else TILED(false);
 #undef TILED
   return gf_sum(c);
@@ -749,9 +819,9 @@ extern "C" int fg_gemm_f32_act(const float* x, const float* w, float* y, float* 
       else FEW_ROWS(false, false);
     }
 #undef FEW_ROWS
-    return gf_sum({x, w, y, part, M, N, K, ldx, ldw, ldy, vec, stream});
+    return gf_sum({x, w, y, part, M, N, K, ldx, ldw, ldy, vec, stream, nullptr, nullptr});
   }
-  const GfCall c = {x, w, y, part, M, N, K, ldx, ldw, ldy, vec, stream};
+  const GfCall c = {x, w, y, part, M, N, K, ldx, ldw, ldy, vec, stream, nullptr, nullptr};
   if (mb < 1 || mb > 7 || (nw == 4 && mb > 5) || (nw != 4 && nw != 8)) return FG_ERR_ARG;
   // What the rows that a tile loads span, of x (8 a wave at a time) and of a wave's 32 of W: any strides are taken, beyond 32
   // bits of bytes by the smallest tile (every cut gives the same bits).
@@ -761,6 +831,31 @@ extern "C" int fg_gemm_f32_act(const float* x, const float* w, float* y, float* 
 #define CASE(MB)                                          \
   if (mb == MB && nw == 8) return gf_launch<MB, 2, 8>(c); \
   if (mb == MB && nw == 4) return gf_launch<MB < 6 ? MB : 5, 2, 4>(c);
+  CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7)
+#undef CASE
+  return FG_ERR_ARG;
+}
+
+// Rows [n, K] in their three parts: out bf16 [ceil(n / 16)][K / 32][3][64][8].
+extern "C" int fg_gemm_f32_cut(const float* rows, int ld, int n, int K, void* out, hipStream_t stream) {
+  if (n <= 0) return FG_OK;
+  if (K <= 0 || K % GF_STEP || ld < K || ld % 4 || ((uintptr_t)rows | (uintptr_t)out) % 16 || K / GF_STEP > 4 * 65535) return FG_ERR_ARG;
+  gemm_f32_cut_kernel<<<dim3((n + 15) / 16, (K / GF_STEP + 3) / 4), 256, 0, stream>>>(rows, ld, n, K, (bf16x8*)out);
+  return fg_launch_status();
+}
+
+// fg_gemm_f32_act's tiles (mb > 0, act 0) with the operands cut beforehand, xp and wp from fg_gemm_f32_cut; K a multiple of 128.
+extern "C" int fg_gemm_f32_parts(const void* xp, const void* wp, const float* x, const float* w, float* y, float* part, int M, int N, int K,
+                                 int ldx, int ldw, int ldy, int mb, int nw, hipStream_t stream) {
+  if (M <= 0 || N <= 0) return FG_OK;
+  if (!xp || !wp || ((uintptr_t)xp | (uintptr_t)wp) % 16 || K <= 0 || K % GF_SEG || K > 1 << 20 || ldx < K || ldw < K || (y && ldy < N) ||
+      (!y && !part))
+    return FG_ERR_ARG;
+  if (mb < 1 || mb > 7 || (nw == 4 && mb > 5) || (nw != 4 && nw != 8)) return FG_ERR_ARG;
+  const GfCall c = {x, w, y, part, M, N, K, ldx, ldw, ldy, 1, stream, (const bf16x8*)xp, (const bf16x8*)wp};
+#define CASE(MB)                                                       \
+  if (mb == MB && nw == 8) return gf_launch<MB, 2, 8, false, true>(c); \
+  if (mb == MB && nw == 4) return gf_launch<MB < 6 ? MB : 5, 2, 4, false, true>(c);
   CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7)
 #undef CASE
   return FG_ERR_ARG;

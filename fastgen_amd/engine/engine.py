@@ -54,7 +54,8 @@ def step_memory_estimate(model: Model, max_step_tokens: int, max_batch: int) -> 
             if shape is not None and len(shape) == 2:
                 widest = max(widest, shape[0])
                 if v.dtype == torch.float32:
-                    scratch = max(scratch, gemm_f32_scratch(max_step_tokens, *shape))
+                    cut = 6 * max_step_tokens * shape[1] if getattr(v, "cut", None) is not None else 0  # x in its parts
+                    scratch = max(scratch, gemm_f32_scratch(max_step_tokens, *shape) + cut)
                 elif getattr(v, "packed", None) is not None:
                     scratch = max(scratch, gemm_large_scratch(max_step_tokens, shape[0]))
     return int(max_step_tokens * 12 * widest + 3 * max_batch * model.vocab_size * 4) + scratch

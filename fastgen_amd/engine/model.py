@@ -73,8 +73,8 @@ class Model:
     def __init__(self, layout: ModelLayout, dtype: torch.dtype, device: torch.device | str, args: Any = None,
                  architecture: Optional[str] = None, packed_weights: Optional[bool] = None,
                  memory_budget: Optional[int] = None) -> None:
-        """``packed_weights``: whether the bfloat16 matrices get a second copy in the order in which the
-        products of few rows read them (``kernels.linear.StreamedMatrix``); None: if the weights twice
+        """``packed_weights``: whether the matrices get a second copy, bfloat16 ones in the order in which the products of few rows
+        read them, float32 ones in the parts that the products of many rows multiply (``kernels.linear.StreamedMatrix``); None: if the weights twice
         leave half of ``memory_budget`` (bytes for the model and its cache; default: the GPU's memory) free
         (``kernels.linear.packing_fits``)."""
         if dtype not in (torch.float32, torch.bfloat16):
@@ -125,9 +125,10 @@ class Model:
         check_against_specs(source, specs, self.parts.duplicates())
         pack = self.packed_weights
         if pack is None:
-            matrix_bytes = sum(math.prod(s.shape) for s in specs if s.role == MATRIX) * 2
-            pack = self.dtype == torch.bfloat16 and packing_fits(matrix_bytes, self.device, self.memory_budget)
-        with packing(pack and self.dtype == torch.bfloat16):
+            # (a float32 matrix and its parts are 10 bytes an element, a bfloat16 one twice 4)
+            matrix_bytes = sum(math.prod(s.shape) for s in specs if s.role == MATRIX) * (2 if self.dtype == torch.bfloat16 else 5)
+            pack = packing_fits(matrix_bytes, self.device, self.memory_budget)
+        with packing(pack):
             for part in self.parts.all_parts:
                 tensors = {s.name: source.get(s.name) for s in part.tensor_specs()}
                 part.load(tensors, self.dtype, self.device)
@@ -164,7 +165,7 @@ class Model:
         seen, total = set(), 0
         for p in self.parts.all_parts:
             for v in vars(p).values():
-                held = [v.rows, v.packed.data if v.packed is not None else None] if isinstance(v, StreamedMatrix) else (
+                held = v.tensors() if isinstance(v, StreamedMatrix) else (
                     [v.data] if isinstance(v, PackedExperts) else [v])
                 for t in held:
                     if isinstance(t, torch.Tensor) and t.data_ptr() not in seen:

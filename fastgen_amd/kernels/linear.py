@@ -96,6 +96,7 @@ class StreamedMatrix:
     rows: torch.Tensor
     packed: Optional[ops.PackedWeight] = None
     part_of: Optional["StreamedMatrix"] = None  # the matrix whose first rows these are
+    cut: Optional[ops.CutWeight] = None  # of a float32 matrix: its parts, for products of many rows
 
     @property
     def shape(self):
@@ -113,7 +114,8 @@ class StreamedMatrix:
     def first_rows(self, n: int) -> "StreamedMatrix":
         """The matrix of the first ``n`` rows (views; the packed copy only if ``n`` is a multiple of 16)."""
         keep = self.packed is not None and (n % 16 == 0 or n == self.rows.shape[0])
-        return StreamedMatrix(self.rows[:n], self.packed.first_rows(n) if keep else None, self)
+        cut = self.cut.first_rows(n) if self.cut is not None and (n % 16 == 0 or n == self.rows.shape[0]) else None
+        return StreamedMatrix(self.rows[:n], self.packed.first_rows(n) if keep else None, self, cut)
 
     def alike(self) -> List["StreamedMatrix"]:
         """This matrix and the others of its kind, other layers' as a rule: what a measurement is made on."""
@@ -123,8 +125,11 @@ class StreamedMatrix:
         return [self] + [m for m in others if m is not None and m is not self]
 
     def nbytes(self) -> int:
-        return self.rows.numel() * self.rows.element_size() + (
-            self.packed.data.numel() * self.packed.data.element_size() if self.packed is not None else 0)
+        return sum(t.numel() * t.element_size() for t in self.tensors())
+
+    def tensors(self) -> List[torch.Tensor]:
+        """The matrix and its second copy."""
+        return [self.rows] + [copy.data for copy in (self.packed, self.cut) if copy is not None]
 
 
 # the stored matrices of a kind, as long as their parts hold them
@@ -165,10 +170,12 @@ def packing_fits(matrix_bytes: int, device, budget_bytes: Optional[int] = None) 
     return 2 * matrix_bytes <= budget_bytes // 2
 
 
-def streamed(w: torch.Tensor) -> StreamedMatrix:
-    """A part's weight matrix, placed on the device, as the products take it."""
+def streamed(w: torch.Tensor, many_rows: bool = True) -> StreamedMatrix:
+    """A part's weight matrix, placed on the device, as the products take it.  ``many_rows``: whether a step's tokens go through it (not
+    only the rows that logits are wanted of): a float32 matrix's second copy serves those."""
     pack = _pack_now and w.is_cuda and w.dtype == torch.bfloat16 and w.dim() == 2
-    m = StreamedMatrix(w, ops.pack_weight(w) if pack else None)
+    m = StreamedMatrix(w, ops.pack_weight(w) if pack else None, None,
+                       ops.cut_weight(w) if _pack_now and many_rows and ops.cut_weight_ok(w) else None)
     if w.dtype == torch.bfloat16:  # (a 32-bit product is not measured)
         _stored[_kind(m)] = [ref for ref in _stored.get(_kind(m), ()) if ref() is not None] + [weakref.ref(m)]
     return m
@@ -419,10 +426,10 @@ def linear(x, w, out_dtype: Optional[torch.dtype] = None,
         if out_dtype not in (None, torch.float32):
             raise ops.KernelArgumentError("a float32 product has float32 output")
         if silu:
-            return ops.gemm_f32_gated(x, w, "gelu_tanh" if gated == "gelu_tanh" else "silu")
+            return ops.gemm_f32_gated(x, w, "gelu_tanh" if gated == "gelu_tanh" else "silu", matrix.cut)
         if residual is not None and ops.gemm_f32_norm_ok(x, w, residual[0], residual[1]):
-            return ops.NormedRows(ops.gemm_f32_norm(x, w, *residual))
-        return ops.gemm_nt(x, w)
+            return ops.NormedRows(ops.gemm_f32_norm(x, w, *residual, matrix.cut))
+        return ops.gemm_f32(x, w, matrix.cut)
     if x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
         raise ops.KernelArgumentError(f"linear: unsupported dtypes {x.dtype}, {w.dtype}")
     out_dtype = out_dtype or torch.bfloat16

@@ -942,7 +942,6 @@ GEMM_F32_GROUP = 1024
 GEMM_F32_FEW_ROWS, GEMM_F32_MAX_SUMS, GEMM_F32_MAX_SPLIT_ROWS = 8, 256 << 20, 4096
 
 
-@functools.lru_cache(maxsize=4096)
 def gemm_f32_plan(M: int, N: int, K: int, cus: int, behind: bool = False) -> Tuple[int, int, bool]:
     """How the 32-bit product is cut: (blocks of 16 rows in a tile, waves of 32 outputs in a tile, whether every group of k
     has a workgroup of its own); (0, 0, False): the kernel of 16 rows and 16 outputs.  Every cut gives the same bits.
@@ -962,25 +961,35 @@ def gemm_f32_plan(M: int, N: int, K: int, cus: int, behind: bool = False) -> Tup
     3.8 at least; cut, all of W comes at 5.1 TB/s behind 7.5 us, 2 % more a row beyond four, and the sums cost the kernel behind 1 us and
     0.35 a group.  Measured at 4 rows, uncut and cut, with the kernel behind: 5,120 x 3,072 (320 workgroups) 31 and 25, 3,072 x 8,192 38.1 and 35.2,
     3,072 x 3,072 19.8 and 20.6, 4,096 x 14,336 61.0 and 62.8."""
+    return _f32_plan(M, N, K, cus, behind, False)[1]
+
+
+@functools.lru_cache(maxsize=4096)
+def _f32_plan(M: int, N: int, K: int, cus: int, behind: bool, cut: bool) -> Tuple[float, Tuple[int, int, bool]]:
+    """The microseconds of a cut as :func:`gemm_f32_plan` counts them (of no use up to 8 rows), and the cut.  ``cut``: tiles of operands cut
+    into their parts beforehand, whose steps take 0.83 of the time and whose W is half as many bytes again, and the kernel that
+    cuts x (3 us; 4 bytes of an element read and 6 written)."""
     if M <= GEMM_F32_FEW_ROWS and not behind:
-        return 0, 0, False
-    groups, blocks, streaming = -(-K // GEMM_F32_GROUP), -(-M // 16), N * K * 4 / 5e6
+        return 0.0, (0, 0, False)
+    groups, blocks, streaming = -(-K // GEMM_F32_GROUP), -(-M // 16), N * K * (6 if cut else 4) / 5e6
     part = K % GEMM_F32_GROUP / GEMM_F32_GROUP
     whole = K // GEMM_F32_GROUP + (max(0.4, part) if part else 0)
     wgs = -(-N // 16) * blocks
     best = 2 + max(whole * (4.8 if wgs <= cus else max(9, 1.6 + 4 * wgs / cus)), streaming), (0, 0, False)
     if behind and M <= 16 and groups > 1:
         uncut = 4 + whole * max(3.8, 3.5 * -(-wgs // cus))
-        cut = (7.5 + N * K * 4 / 5.1e6) * (1 + 0.02 * max(0, M - 4)) + 1 + 0.35 * groups
-        best = min(best if M > GEMM_F32_FEW_ROWS else (uncut, (0, 0, False)), (cut, (0, 0, True)))
+        by_groups = (7.5 + N * K * 4 / 5.1e6) * (1 + 0.02 * max(0, M - 4)) + 1 + 0.35 * groups
+        best = min(best if M > GEMM_F32_FEW_ROWS else (uncut, (0, 0, False)), (by_groups, (0, 0, True)))
     if M <= GEMM_F32_FEW_ROWS:
-        return best[1]
+        return best
+    if cut:
+        best = float("inf"), best[1]
     for waves, tallest in ((8, 7), (4, 5)):  # (what the registers hold)
         for b in range(1, tallest + 1):
             row_tiles = -(-blocks // b)
             if b > 1 and -(-blocks // (b - 1)) == row_tiles:
                 continue  # as few tiles with shorter ones
-            full, alone = 0.61 + 0.29 * b, 0.44 + 0.2 * b
+            full, alone = (0.83 if cut else 1.0) * (0.61 + 0.29 * b), (0.83 if cut else 1.0) * (0.44 + 0.2 * b)
             for split in (False, True):
                 if split and (groups == 1 or M > GEMM_F32_MAX_SPLIT_ROWS or groups * M * N * 4 > GEMM_F32_MAX_SUMS):
                     continue
@@ -990,10 +999,10 @@ def gemm_f32_plan(M: int, N: int, K: int, cus: int, behind: bool = False) -> Tup
                 time = max(time * (GEMM_F32_GROUP // 32 if split else -(-K // 32)), streaming)
                 if split:
                     time += 1 + 0.35 * groups + groups * M * N * 4 / 6e6 if behind else 2 + groups * M * N * 8 / 6e6
-                time += 5
+                time += 5 + (3 + M * K * 10 / 5e6 if cut else 0)
                 if time < best[0]:
                     best = time, (b, waves, split)
-    return best[1]
+    return best
 
 
 def gemm_f32_scratch(M: int, N: int, K: int) -> int:
@@ -1033,33 +1042,87 @@ def gemm_nt(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None
     return out
 
 
-def _f32_product(x: torch.Tensor, w: torch.Tensor, what: str, act: int = 0) -> Tuple[torch.Tensor, bool]:
+@dataclass
+class CutWeight:
+    """A float32 matrix ``[n, k]`` (``k`` a multiple of 128) in the three bfloat16 parts that its products of many rows multiply
+    (:func:`cut_weight`), in the operands' order: ``data [ceil(n / 16), k / 32, 3, 64, 8]``.  A second copy, of half as many bytes again: the matrix
+    itself is what products of few rows read, and what a lost output is computed from."""
+
+    data: torch.Tensor
+    n: int
+    k: int
+
+    def first_rows(self, n: int) -> "CutWeight":
+        """The matrix of the first ``n`` rows (a multiple of 16, or all): a view."""
+        _need(0 < n <= self.n and (n % 16 == 0 or n == self.n), "a cut matrix is cut at multiples of 16 rows")
+        return CutWeight(self.data[: -(-n // 16)], n, self.k)
+
+
+def _cut_rows(x: torch.Tensor) -> torch.Tensor:
+    """The three parts of float32 rows (``fg_gemm_f32_cut``)."""
+    n, k = x.shape
+    out = torch.empty((-(-n // 16), k // 32, 3, 64, 8), dtype=torch.bfloat16, device=x.device)
+    _check(_lib.load("gemm").fg_gemm_f32_cut(_ptr(x), x.stride(0), n, k, _ptr(out), _stream(x)), "cut of float32 rows")
+    return out
+
+
+def cut_weight_ok(w: torch.Tensor) -> bool:
+    """Whether :func:`cut_weight` takes a matrix."""
+    return (w.dim() == 2 and w.dtype == torch.float32 and w.is_cuda and w.shape[0] > 0 and 0 < w.shape[1] <= 1 << 20 and w.shape[1] % 128 == 0
+            and w.stride(1) == 1 and w.stride(0) % 4 == 0 and w.data_ptr() % 16 == 0)
+
+
+def cut_weight(w: torch.Tensor) -> CutWeight:
+    """``w [n, k]`` (float32, ``k`` a multiple of 128, rows 16-byte aligned) as :class:`CutWeight`, on the device of ``w``."""
+    _need(cut_weight_ok(w), "cut_weight takes a float32 matrix on the GPU, k a multiple of 128, rows 16-byte aligned")
+    return CutWeight(_cut_rows(w), *w.shape)
+
+
+def _f32_product(x: torch.Tensor, w: torch.Tensor, cut: Optional[CutWeight], what: str, act: int = 0, behind: bool = True) -> Tuple[torch.Tensor, bool]:
     """The 32-bit product with a kernel behind it that adds the groups' sums up: ``(y [M, N], False)``, or ``(sums [groups, M, N],
-    True)``.  ``act``: an epilogue code; the kernel of 16 rows stores the activation's ``[M, N / 2]`` itself."""
-    (x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[1] and x.dtype == w.dtype == torch.float32
-          and x.stride(1) == 1 and w.stride(1) == 1) or _refuse(f"{what}: x [M, K] and w [N, K] must be float32 with unit column stride")
+    True)``; without ``behind`` always the former.  ``act``: an epilogue code; the kernel of 16 rows stores the activation's ``[M, N / 2]`` itself.
+    ``cut``: the same matrix's parts, which take the product where that is the shorter way."""
+    _need(x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[1] and x.dtype == w.dtype == torch.float32
+          and x.stride(1) == 1 and w.stride(1) == 1, "a float32 product: x [M, K] and w [N, K] of unit column stride")
     (M, K), N = x.shape, w.shape[0]
-    blocks, waves, split = gemm_f32_plan(M, N, K, compute_units(), True)
+    took, (blocks, waves, split) = _f32_plan(M, N, K, compute_units(), behind, False)
+    parts = None
+    if cut is not None and M > 16 and x.stride(0) % 4 == 0 and x.data_ptr() % 16 == 0:
+        (cut.n == N and cut.k == K and cut.data.dtype == torch.bfloat16 and cut.data.is_contiguous()
+         and cut.data.shape == (-(-N // 16), K // 32, 3, 64, 8) and cut.data.device == w.device) or _refuse(f"{what}: the parts do not fit w")
+        shorter, plan = _f32_plan(M, N, K, compute_units(), behind, True)
+        if shorter < took:
+            parts, (blocks, waves, split) = _cut_rows(x), plan
     act = 0 if split or blocks else act
-    shape = (-(-K // GEMM_F32_GROUP), M, N) if split else (M, N // 2 if act else N)
-    y = torch.empty(shape, dtype=torch.float32, device=x.device)
-    st = _lib.load("gemm").fg_gemm_f32_act(_ptr(x), _ptr(w), _ptr(None if split else y), _ptr(y if split else None), M, N, K, x.stride(0),
-                                           w.stride(0), shape[-1], blocks, waves, act, _stream(x))
+    y = torch.empty((M, N // 2 if act else N), dtype=torch.float32, device=x.device) if not (split and behind) else None
+    sums = torch.empty((-(-K // GEMM_F32_GROUP), M, N), dtype=torch.float32, device=x.device) if split else None
+    sizes = M, N, K, x.stride(0), w.stride(0), N // 2 if act else N, blocks, waves
+    lib = _lib.load("gemm")
+    if parts is not None:
+        st = lib.fg_gemm_f32_parts(_ptr(parts), _ptr(cut.data), _ptr(x), _ptr(w), _ptr(y), _ptr(sums), *sizes, _stream(x))
+    else:
+        st = lib.fg_gemm_f32_act(_ptr(x), _ptr(w), _ptr(y), _ptr(sums), *sizes, act, _stream(x))
     _check(st, what)
-    return y, split
+    return (sums, True) if y is None else (y, False)
+
+
+def gemm_f32(x: torch.Tensor, w: torch.Tensor, cut: Optional[CutWeight] = None) -> torch.Tensor:
+    """:func:`gemm_nt` of float32 operands; ``cut``: the parts of ``w``, the same bits in less time for many rows."""
+    _gpu(x, w)
+    return _f32_product(x, w, cut, "gemm_f32", 0, False)[0]
 
 
 def _f32_sums_args(parts: torch.Tensor, x: torch.Tensor, w: torch.Tensor):
     return _ptr(parts), _ptr(x), _ptr(w)
 
 
-def gemm_f32_gated(x: torch.Tensor, w: torch.Tensor, epilogue="silu") -> torch.Tensor:
+def gemm_f32_gated(x: torch.Tensor, w: torch.Tensor, epilogue="silu", cut: Optional[CutWeight] = None) -> torch.Tensor:
     """``act(gate) * up`` in float32 of the product with a gate and an up matrix interleaved by :func:`interleave_gate_up` (``"silu"`` or
     ``"gelu_tanh"``), with the bits of :func:`gemm_nt` and :func:`silu_mul` or :func:`gelu_mul` behind it."""
     _gpu(x, w)
     act, N = _gated_code(epilogue), w.shape[0]
     _need(act != 0 and N % 16 == 0, "gemm_f32_gated: a gated epilogue, N % 16 == 0")
-    y, split = _f32_product(x, w, "gemm_f32_gated", act)
+    y, split = _f32_product(x, w, cut, "gemm_f32_gated", act)
     if not split:
         return y if y.shape[1] == N // 2 else gelu_mul(y) if act == 4 else silu_mul(y)
     (M, K), out = x.shape, torch.empty((x.shape[0], N // 2), dtype=torch.float32, device=x.device)
@@ -1076,12 +1139,13 @@ def gemm_f32_norm_ok(x: torch.Tensor, w: torch.Tensor, h: torch.Tensor, weight: 
             and h.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
 
 
-def gemm_f32_norm(x: torch.Tensor, w: torch.Tensor, h: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
+def gemm_f32_norm(x: torch.Tensor, w: torch.Tensor, h: torch.Tensor, weight: torch.Tensor, eps: float,
+                  cut: Optional[CutWeight] = None) -> torch.Tensor:
     """``h += x @ w.T`` in float32, and ``rmsnorm(h) * weight``, with the bits of :func:`gemm_nt` and :func:`add_rmsnorm` behind it."""
     _gpu(x, w, h, weight)
     _need(gemm_f32_norm_ok(x, w, h, weight), "gemm_f32_norm: h [M, N] and weight [N] float32, N a multiple of 8 up to 8,192")
     (M, K), N = x.shape, w.shape[0]
-    y, split = _f32_product(x, w, "gemm_f32_norm")
+    y, split = _f32_product(x, w, cut, "gemm_f32_norm")
     out = torch.empty((M, N), dtype=torch.float32, device=x.device)
     if not split:
         return add_rmsnorm(h, y, weight, eps, out)
@@ -1093,17 +1157,16 @@ def gemm_f32_norm(x: torch.Tensor, w: torch.Tensor, h: torch.Tensor, weight: tor
 
 def gemm_f32_qkv(x: torch.Tensor, wqkv: torch.Tensor, table: Optional[torch.Tensor], positions: torch.Tensor, slots: torch.Tensor,
                  k_pages: torch.Tensor, v_pages: torch.Tensor, n_heads: int, n_kv: int, head_dim: int, rotary_dim: int,
-                 value_from_key: bool = False) -> torch.Tensor:
+                 value_from_key: bool = False, cut: Optional[CutWeight] = None) -> torch.Tensor:
     """The float32 q, k, v projections with :func:`rope_kv_write` behind them, the same bits: rows that begin with the rotated queries
     ``[M, >= H*hd]``; the rotated keys and the values go into their pages.  ``value_from_key``: ``wqkv`` has no v rows, a token's
     value is its key before the rotation."""
     _gpu(x, wqkv, table, positions, slots, k_pages, v_pages)
     (M, K), N = x.shape, wqkv.shape[0]
     _need(N == (n_heads + (1 if value_from_key else 2) * n_kv) * head_dim, "wqkv must have the rows of q, k and v")
-    y, split = _f32_product(x, wqkv, "gemm_f32_qkv")
-    if not split or head_dim % 8 or rotary_dim % 8 or M > 65535:
-        if split:
-            y = gemm_nt(x, wqkv)
+    fused = head_dim % 8 == 0 and rotary_dim % 8 == 0 and M <= 65535
+    y, split = _f32_product(x, wqkv, cut, "gemm_f32_qkv", 0, fused)
+    if not split:
         rope_kv_write(y, positions, None, slots, k_pages, v_pages, n_heads, n_kv, head_dim, rotary_dim, table=table,
                       v_col=n_heads * head_dim if value_from_key else None)
         return y

@@ -298,19 +298,24 @@ def gemm_nt(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None
     return out
 
 
-def gemm_f32_gated(x: torch.Tensor, w: torch.Tensor, epilogue="silu") -> torch.Tensor:
+def gemm_f32(x: torch.Tensor, w: torch.Tensor, cut=None) -> torch.Tensor:
+    """``x @ w.T``; ``cut`` is ``w`` again."""
+    return x @ w.T
+
+
+def gemm_f32_gated(x: torch.Tensor, w: torch.Tensor, epilogue="silu", cut=None) -> torch.Tensor:
     """``act(gate) * up`` of ``x @ w.T`` whose columns are interleaved in turns of 8."""
     return _gated(x @ w.T, epilogue)
 
 
-def gemm_f32_norm(x: torch.Tensor, w: torch.Tensor, h: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
+def gemm_f32_norm(x: torch.Tensor, w: torch.Tensor, h: torch.Tensor, weight: torch.Tensor, eps: float, cut=None) -> torch.Tensor:
     """``h += x @ w.T``; ``h * rsqrt(mean(h^2) + eps) * weight``."""
     return add_rmsnorm(h, x @ w.T, weight, eps, torch.empty_like(h))
 
 
 def gemm_f32_qkv(x: torch.Tensor, wqkv: torch.Tensor, table: Optional[torch.Tensor], positions: torch.Tensor, slots: torch.Tensor,
                  k_pages: torch.Tensor, v_pages: torch.Tensor, n_heads: int, n_kv: int, head_dim: int, rotary_dim: int,
-                 value_from_key: bool = False) -> torch.Tensor:
+                 value_from_key: bool = False, cut=None) -> torch.Tensor:
     """The q, k, v projections, rotated; keys and values into their pages: rows that begin with the queries."""
     return rope_kv_write(x @ wqkv.T, positions, None, slots, k_pages, v_pages, n_heads, n_kv, head_dim, rotary_dim, table=table,
                          v_col=n_heads * head_dim if value_from_key else None)

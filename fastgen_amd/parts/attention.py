@@ -222,7 +222,7 @@ class Attention(RowsMixer):
             parts = qkv_parts(x, own_rows) if plain and x.dtype == torch.bfloat16 else None
             if plain and x.dtype == torch.float32:
                 qkv = ops.gemm_f32_qkv(x, own_rows.rows, table, ctx.positions, group.slots, store.k_pages, store.v_pages, self.n_heads,
-                                       self.n_kv_heads, self.head_dim, self.position.rotary_dim, value_from_key=self.value_from_key)
+                                       self.n_kv_heads, self.head_dim, self.position.rotary_dim, value_from_key=self.value_from_key, cut=own_rows.cut)
             elif parts is not None:
                 qkv = ops.rope_kv_parts(parts, table, group.slots, store.k_pages, store.v_pages, self.n_heads, self.n_kv_heads,
                                         self.head_dim, self.position.rotary_dim, value_from_key=self.value_from_key)

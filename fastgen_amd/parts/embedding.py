@@ -60,10 +60,10 @@ class LMHead(Part):
 
     def load(self, tensors: Mapping[str, torch.Tensor], dtype: torch.dtype, device: Any) -> None:
         if not self.tied_to:
-            self.weight = streamed(place(tensors[self._name("weight")], MATRIX, dtype, device))
+            self.weight = streamed(place(tensors[self._name("weight")], MATRIX, dtype, device), many_rows=False)
 
     def tie(self, table: torch.Tensor) -> None:
-        self.weight = streamed(table)  # the table itself row by row; a packed copy of it if copies are made
+        self.weight = streamed(table, many_rows=False)  # the table itself row by row; a packed copy of it if copies are made
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         logits = linear(x, self.weight, out_dtype=torch.float32)

@@ -1431,3 +1431,38 @@ def test_gemm_f32_with_what_is_behind_has_the_bits_of_both(ops, M, N, K):
         rows = y.clone()
         ops.rope_kv_write(rows, pos, None, slots, *pages[2:], H, n_kv, hd, rot, table=table, v_col=H * hd if from_key else None)
         assert same(q[:, :H * hd], rows[:, :H * hd]) and same(pages[0], pages[2]) and same(pages[1], pages[3])
+
+
+@pytest.mark.parametrize("M,N,K", [(17, 48, 128), (100, 1000, 1152), (112, 272, 2048), (113, 3072, 1024), (250, 515, 3072), (400, 2048, 256)])
+def test_gemm_f32_of_operands_cut_beforehand_has_the_same_bits(ops, M, N, K):
+    """Every tile, with and without a workgroup a group of k, rows and outputs that fill none, against the operands as they are; infinities
+    and what rounds to one in 16 bits."""
+    from fastgen_amd.kernels import _lib
+
+    torch.manual_seed(K)
+    x, w = torch.randn(M, K, device=DEV), torch.randn(N, K, device=DEV)
+    x[M // 2, K - 1], w[5, 3], x[1] = float("inf"), 3.4e38, x[1] * 2.0 ** -100
+    same = lambda a, b: torch.equal(a[~b.isnan()], b[~b.isnan()]) and torch.equal(a.isnan(), b.isnan())
+    want, cut = ops.gemm_nt(x, w), ops.cut_weight(w)
+    wide = torch.randn(M, K + 8, device=DEV)[:, 4:K + 4]
+    wide.copy_(x)
+    for rows in (x, wide):
+        xp = ops._cut_rows(rows)
+        parts = xp.view(-(-M // 16), K // 32, 3, 4, 16, 2, 4).double()  # [block, step, part, g, row, half, 4]
+        back = (parts[:, :, 0] + parts[:, :, 1] * 2.0 ** -8 + parts[:, :, 2] * 2.0 ** -16).permute(0, 3, 1, 4, 2, 5).reshape(-1, K)
+        finite = torch.arange(back.shape[0], device=DEV) != M // 2
+        assert torch.equal(back[finite], torch.nn.functional.pad(x, (0, 0, 0, -M % 16)).double()[finite])  # the parts are the number
+        for waves, tallest in ((8, 7), (4, 5)):
+            for blocks in range(1, tallest + 1):
+                for sums in (None, torch.empty(-(-K // 1024), M, N, device=DEV)):
+                    y = torch.empty(M, N, device=DEV)
+                    st = _lib.load("gemm").fg_gemm_f32_parts(xp.data_ptr(), cut.data.data_ptr(), rows.data_ptr(), w.data_ptr(), y.data_ptr(), ops._ptr(sums),
+                                                             M, N, K, rows.stride(0), K, N, blocks, waves, ops._stream(y))
+                    assert st == 0 and same(y, want), (blocks, waves, sums is None)
+    assert same(ops.gemm_f32(x, w, cut), want)
+    if N >= 48:
+        assert same(ops.gemm_f32(x, w[:32], cut.first_rows(32)), want[:, :32])
+    with pytest.raises(ops.KernelArgumentError):
+        ops.gemm_f32(x, w[:16], cut)
+    with pytest.raises(ops.KernelArgumentError):
+        ops.cut_weight(w[:, :K - 4])
