@@ -24,6 +24,7 @@
 //    (max, sum, O) go to scratch and a combine kernel merges them.
 //  * fg_attn_tile (prompt portions, up to 128 rows an item): K and V tiles are
 //    staged in LDS and shared by the workgroup's waves.
+//  * fg_attn_both: items of both kinds in one launch.
 //
 // Semantics as in attention.hip (fastgen/forward.py:176-258).
 #include "common.h"
@@ -466,26 +467,20 @@ __global__ __launch_bounds__(256) void attn_plan_kernel(const int* __restrict__ 
 // cache lines of arguments, and a third, which every workgroup would wait for, costs a launch 0.4 us.  (So in the
 // combine kernels, whose arguments without a gate are one line.)
 #define SHIFT_ORDERED 64  // added to page_shift (-1 .. 30): the list is the ordered one
-template <bool PERM /* the page's value slots are permuted: page_size % 32 == 0 */, class... GATE>
-__global__ __launch_bounds__(256) void attn_split_kernel(
-    const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, int out_stride,
-    const bf16_t* __restrict__ k_pages, const bf16_t* __restrict__ v_pages,
-    const int* __restrict__ block_table, int bt_stride, const int* __restrict__ list,
-    float* __restrict__ part_o, float* __restrict__ part_ml, int n_heads, int n_kv, int page_size,
-    int shift_ordered, float scale, int window, const float* __restrict__ sinks, const float* __restrict__ dist,
-    const GATE... gate) {
-  const bool ordered = shift_ordered >= SHIFT_ORDERED - 1;
-  const int page_shift = ordered ? shift_ordered - SHIFT_ORDERED : shift_ordered;
-  __shared__ float o_s[2][16][HD + 1];
-  __shared__ float ml_s[2][16][2];
-  const int lane = threadIdx.x % FG_WAVE, wave = threadIdx.x / FG_WAVE;
+
+// A chunk for one kv head by four waves of the workgroup, `wave` among them.  Every wave of the workgroup comes through
+// the barriers in here as often, a chunk that is not in use too.  o_s, ml_s: the four waves' LDS.  store(o, 1 / sum, token, column) stores a row.
+typedef float SplitO[16][HD + 1];
+typedef float SplitMl[16][2];
+template <bool PERM /* the page's value slots are permuted: page_size % 32 == 0 */, class STORE>
+__device__ __forceinline__ void split_chunk(const int4 rec_a, const int4 rec_b, int chunk, int kvh, int wave, SplitO* o_s, SplitMl* ml_s,
+    const bf16_t* __restrict__ q, int q_stride, const bf16_t* __restrict__ k_pages, const bf16_t* __restrict__ v_pages,
+    const int* __restrict__ block_table, int bt_stride, float* __restrict__ part_o, float* __restrict__ part_ml,
+    int n_heads, int n_kv, int page_size, int page_shift, float scale, int window, const float* __restrict__ sinks,
+    const float* __restrict__ dist, STORE store) {
+  const int lane = threadIdx.x % FG_WAVE;
   const int r16 = lane & 15, g = lane >> 4;
-  const int kvh = blockIdx.x;
   const int G = n_heads / n_kv;
-  const int* rec = list + (size_t)blockIdx.y * 8;
-  const int4 rec_a = *(const int4*)rec, rec_b = *(const int4*)(rec + 4);
-  const int chunk = ordered ? rec_b.w : blockIdx.y;
-  if (rec_b.z == 0) return;  // uniform: a chunk that is not in use
   const Item it{rec_a.x, rec_a.y, rec_a.z, rec_a.w};
   const int t_begin = rec_b.x, t_end = rec_b.y;
   const bool alone = rec_b.z == 1;  // the item's only chunk
@@ -606,7 +601,7 @@ __global__ __launch_bounds__(256) void attn_split_kernel(
   if (alone) {
     // a sink: one more term exp(sink) in the denominator (maxima are in base 2 and scaled), no value
     if (sinks) l += __builtin_amdgcn_exp2f(sinks[h_out] * LOG2E - m);
-    store_row(out, out_stride, o, 1.f / l, t_out, h_out * HD + 4 * g, gate...);
+    store(o, 1.f / l, t_out, h_out * HD + 4 * g);
   } else {
     const size_t row = ((size_t)chunk * n_kv + kvh) * 16 + r16;
 #pragma unroll
@@ -616,6 +611,26 @@ __global__ __launch_bounds__(256) void attn_split_kernel(
       part_ml[row * 2 + 1] = l;
     }
   }
+}
+
+template <bool PERM, class... GATE>
+__global__ __launch_bounds__(256) void attn_split_kernel(
+    const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, int out_stride,
+    const bf16_t* __restrict__ k_pages, const bf16_t* __restrict__ v_pages,
+    const int* __restrict__ block_table, int bt_stride, const int* __restrict__ list,
+    float* __restrict__ part_o, float* __restrict__ part_ml, int n_heads, int n_kv, int page_size,
+    int shift_ordered, float scale, int window, const float* __restrict__ sinks, const float* __restrict__ dist,
+    const GATE... gate) {
+  const bool ordered = shift_ordered >= SHIFT_ORDERED - 1;
+  __shared__ SplitO o_s[2];
+  __shared__ SplitMl ml_s[2];
+  const int* rec = list + (size_t)blockIdx.y * 8;
+  const int4 rec_a = *(const int4*)rec, rec_b = *(const int4*)(rec + 4);
+  if (rec_b.z == 0) return;  // uniform: a chunk that is not in use
+  split_chunk<PERM>(rec_a, rec_b, ordered ? rec_b.w : blockIdx.y, blockIdx.x, threadIdx.x / FG_WAVE, o_s, ml_s, q, q_stride,
+                    k_pages, v_pages, block_table, bt_stride, part_o, part_ml, n_heads, n_kv, page_size,
+                    ordered ? shift_ordered - SHIFT_ORDERED : shift_ordered, scale, window, sinks, dist,
+                    [&](const f32x4(&o)[NDB], float inv, int t, int c) { store_row(out, out_stride, o, inv, t, c, gate...); });
 }
 
 // Two kernels add up the chunks of the items that have several, in chunk order: the workgroups of an
@@ -810,6 +825,20 @@ static bool gate_ok(const void* gate, int stride, int n_heads) {
   return !gate || (stride % 4 == 0 && (uintptr_t)gate % 8 == 0 && stride >= n_heads * HD);
 }
 
+static void launch_combine(const float* part_o, const float* part_ml, const int* plan, bf16_t* out, int out_stride, int max_chunks,
+                           int max_rows, int n_heads, int n_kv, const float* sinks, const OutGate& og, hipStream_t stream) {
+  const bool rows = (long long)max_chunks * n_kv * max_rows <= COMBINE_ROWS_MAX_GROUPS;
+  auto go = [&](auto... gate) {
+    if (rows)
+      attn_combine_rows_kernel<<<dim3(max_rows, n_kv, max_chunks), HD < 64 ? 64 : HD, 0, stream>>>(
+          part_o, part_ml, plan, out, out_stride, n_heads, n_kv, sinks, gate...);
+    else
+      attn_combine_kernel<<<dim3(n_kv, max_chunks), 256, 0, stream>>>(part_o, part_ml, plan, out, out_stride, n_heads, n_kv, sinks,
+                                                                      gate...);
+  };
+  if (og.g) go(og); else go();
+}
+
 // plan: what fg_attn_plan_ordered made of the items, with the same n_items, max_chunks, window and `ordered`.
 // max_rows: no item has more rows (tokens x heads of a kv head's group) than this, at most 16.
 // part_o: fp32 [max_chunks * n_kv * 16 * HD], part_ml: the same rows x 2.
@@ -845,19 +874,8 @@ extern "C" int fg_attn_split_sink(const void* q, int q_stride, void* out, int ou
     if (gate) LAUNCH(false, COMMA og); else LAUNCH(false);
   }
 #undef LAUNCH
-  if (!merge) return fg_launch_status();
-#define COMBINE(...)                                                                                             \
-  do {                                                                                                           \
-    if ((long long)max_chunks * n_kv * max_rows <= COMBINE_ROWS_MAX_GROUPS)                                      \
-      attn_combine_rows_kernel<<<dim3(max_rows, n_kv, max_chunks), HD < 64 ? 64 : HD, 0, stream>>>(              \
-          part_o, part_ml, plan, (bf16_t*)out, out_stride, n_heads, n_kv, sinks __VA_ARGS__);                    \
-    else                                                                                                         \
-      attn_combine_kernel<<<dim3(n_kv, max_chunks), 256, 0, stream>>>(                                           \
-          part_o, part_ml, plan, (bf16_t*)out, out_stride, n_heads, n_kv, sinks __VA_ARGS__);                    \
-  } while (0)
-  if (gate) COMBINE(COMMA og); else COMBINE();
-#undef COMBINE
 #undef COMMA
+  if (merge) launch_combine(part_o, part_ml, plan, (bf16_t*)out, out_stride, max_chunks, max_rows, n_heads, n_kv, sinks, og, stream);
   return fg_launch_status();
 }
 
@@ -978,13 +996,27 @@ constexpr int TILE_ROWS_SMALL = 64;                // of the second form
 // such an end: 64 / 300 / 2000 tokens at head size 128 with it 7.2 / 12.0 / 49.2 us, without 6.1 / 10.8 / 48.3.
 enum { PAGES_ANY = 0, PAGES_CHUNK = 1, PAGES_TILE = 2 };  // multiples of 8, 32, 64
 
-template <int PAGES, bool TILE_PAIR>
+// In a step that has both kinds of items one launch takes both (SPLIT): prompt portions are bound by the matrix cores and by as
+// long as the longest item is, decoded tokens by memory, and neither needs the other.  A workgroup is then an item of the
+// tiles or as many chunks of the split list as it has groups of four waves; eight neighbouring
+// workgroups, one a die, are of one kind, and the kinds alternate while there are both, each in its own order: long items
+// and long chunks first, with the heads on the dies where the kernels alone have them.  The same bits as two launches.
+// Llama 3B's layer, prompts of 380 and 874 tokens beside 24 requests of 100 to 1,500: two launches on two streams took 58 us from
+// the cache's write to the next product (34 the tiles, 22 the split under them, 10 the combine kernel, and 17 of waits between the
+// streams), one launch 38 and the combine kernel, whose grid counts a decoded token's rows and not 16, 5.
+struct SplitPart {
+  const int* list;  // the plan's first or second list
+  float *part_o, *part_ml;
+  int max_chunks, ordered, tile_groups /* workgroups with an item of the tiles */;
+};
+__device__ __forceinline__ const SplitPart& the_split(const SplitPart& s) { return s; }
+template <int PAGES, bool TILE_PAIR, class... SPLIT>
 __global__ __launch_bounds__(TILE_PAIR ? 512 : 256, TILE_PAIR ? 1 : 2) void attn_tile_kernel(
     const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, int out_stride,
     const bf16_t* __restrict__ k_pages, const bf16_t* __restrict__ v_pages,
     const int* __restrict__ block_table, int bt_stride, const int* __restrict__ items, int n_heads, int n_kv,
     int page_size, int page_shift, float scale, int window, const float* __restrict__ sinks,
-    const float* __restrict__ dist, const OutGate gate) {
+    const float* __restrict__ dist, const OutGate gate, const SPLIT... split) {
   constexpr bool PERM = PAGES >= PAGES_CHUNK, WHOLE = PAGES == PAGES_TILE;
   constexpr int TILE_RB = TILE_PAIR ? 2 : 1;  // row blocks a wave holds
   constexpr int TILE_THREADS = TILE_PAIR ? 512 : 256;
@@ -995,11 +1027,45 @@ __global__ __launch_bounds__(TILE_PAIR ? 512 : 256, TILE_PAIR ? 1 : 2) void attn
   constexpr int NSLOT = TILE_PAIR ? 4 : 1;
   __shared__ __attribute__((aligned(16))) bf16_t k_lds[NSLOT][TILE * HD];
   __shared__ __attribute__((aligned(16))) bf16_t v_lds[NSLOT][TILE * HD];
+  int block = blockIdx.x;
+  if constexpr (sizeof...(SPLIT)) {
+    const SplitPart& sp = the_split(split...);
+    const int split_groups = gridDim.x - sp.tile_groups, both = min(sp.tile_groups, split_groups) / 8;  // eights of each kind that alternate
+    int at;  // among the workgroups of its kind
+    bool is_split;
+    if (block < 16 * both) {
+      at = block / 16 * 8 + block % 8;
+      is_split = block / 8 % 2;
+    } else {
+      at = block - 8 * both;
+      is_split = at >= sp.tile_groups;
+      if (is_split) at -= sp.tile_groups - 8 * both;
+    }
+    if (is_split) {  // uniform
+      constexpr int HALVES = NT / 256, HALF = 2 * (sizeof(SplitO) + sizeof(SplitMl));  // groups of four waves, bytes of each
+      constexpr bool FITS = HALVES * HALF <= (int)sizeof(k_lds);  // (where tiles come in pairs)
+      __shared__ __attribute__((aligned(16))) char own_lds[FITS ? 16 : HALVES * HALF];
+      const int half = threadIdx.x / 256, first = at / n_kv * HALVES, mine = min(first + half, sp.max_chunks - 1);
+      if (sp.list[(size_t)first * 8 + 6] == 0) return;  // uniform: not in use, and so none behind it
+      int4 rec_a = *(const int4*)(sp.list + (size_t)mine * 8), rec_b = *(const int4*)(sp.list + (size_t)mine * 8 + 4);
+      if (first + half > mine) rec_a = rec_b = int4{0, 0, 0, 0};
+      char* const at_lds = (FITS ? (char*)&k_lds[0][0] : own_lds) + half * HALF;
+      split_chunk<PERM>(rec_a, rec_b, sp.ordered ? rec_b.w : mine, at % n_kv, threadIdx.x / FG_WAVE % 4, (SplitO*)at_lds,
+                        (SplitMl*)(at_lds + 2 * sizeof(SplitO)), q, q_stride, k_pages, v_pages, block_table, bt_stride,
+                        sp.part_o, sp.part_ml, n_heads, n_kv, page_size, page_shift, scale, window, sinks, dist,
+                        [&](const f32x4(&o)[NDB], float inv, int t, int c) {
+                          if (gate.g) store_row(out, out_stride, o, inv, t, c, gate);  // uniform
+                          else store_row(out, out_stride, o, inv, t, c);
+                        });
+      return;
+    }
+    block = at;
+  }
   const int lane = threadIdx.x % FG_WAVE, wave = threadIdx.x / FG_WAVE;
   const int r16 = lane & 15, g = lane >> 4;
   const int rg = wave & 3;    // row group
   const int par = wave >> 2;  // which tile of a pair this wave takes (0 when tiles come one at a time)
-  const int item = blockIdx.x / n_kv, kvh = blockIdx.x % n_kv;
+  const int item = block / n_kv, kvh = block % n_kv;
   const int G = n_heads / n_kv;
   const Item it = load_item(items, item);
   const Pager pager{block_table + (size_t)it.seq * bt_stride, page_size, page_shift};
@@ -1267,11 +1333,13 @@ struct TileArgs {
   const int* block_table; int bt_stride; const int* items; int n_items, n_heads, n_kv, page_size; float scale;
   int window; const float* sinks; const float* dist; OutGate gate; hipStream_t stream;
 };
-template <int PAGES, bool PAIR>
-static void launch_pages(const TileArgs& a) {
-  attn_tile_kernel<PAGES, PAIR><<<a.n_items * a.n_kv, PAIR ? 512 : 256, 0, a.stream>>>(
+template <int PAGES, bool PAIR, class... SPLIT>
+static void launch_pages(const TileArgs& a, SPLIT... split) {
+  int groups = a.n_items * a.n_kv;
+  ((groups += a.n_kv * ((split.max_chunks + (PAIR ? 1 : 0)) / (PAIR ? 2 : 1))), ...);
+  attn_tile_kernel<PAGES, PAIR><<<groups, PAIR ? 512 : 256, 0, a.stream>>>(
       a.q, a.q_stride, a.out, a.out_stride, a.k_pages, a.v_pages, a.block_table, a.bt_stride, a.items, a.n_heads,
-      a.n_kv, a.page_size, page_shift_of(a.page_size), a.scale, a.window, a.sinks, a.dist, a.gate);
+      a.n_kv, a.page_size, page_shift_of(a.page_size), a.scale, a.window, a.sinks, a.dist, a.gate, split...);
 }
 template <bool PAIR>
 static void launch_tile(const TileArgs& a) {
@@ -1282,8 +1350,18 @@ static void launch_tile(const TileArgs& a) {
 // the form with two tiles at a time exists up to head size 128 only (its LDS)
 template <bool EXISTS> struct PairForm {
   static void go(const TileArgs& a) { launch_tile<true>(a); }
+  static void go(const TileArgs& a, const SplitPart& split) { launch_pages<PAGES_TILE, true>(a, split); }
 };
-template <> struct PairForm<false> { static void go(const TileArgs&) {} };
+template <> struct PairForm<false> {
+  static void go(const TileArgs&) {}
+  static void go(const TileArgs&, const SplitPart&) {}
+};
+static bool tile_args_ok(const TileArgs& a, int item_rows) {
+  return DIST_BIAS == (a.dist != nullptr) && gate_ok(a.gate.g, a.gate.stride, a.n_heads) && a.scale > 0.f && a.n_kv > 0 &&
+         a.n_heads % a.n_kv == 0 && a.n_heads / a.n_kv <= item_rows && a.page_size >= 8 && a.page_size % 8 == 0 &&
+         (long long)a.n_items * a.n_kv <= 2147483647LL && a.q_stride % 8 == 0 && a.out_stride % 4 == 0 &&
+         (item_rows == TILE_ROWS || item_rows == TILE_ROWS_SMALL);
+}
 
 // item_rows: the rows an item has at most, fg_attn_tile_rows(0) or fg_attn_tile_rows(1): which form of the kernel runs.
 extern "C" int fg_attn_tile_sink(const void* q, int q_stride, void* out, int out_stride, const void* k_pages,
@@ -1292,16 +1370,33 @@ extern "C" int fg_attn_tile_sink(const void* q, int q_stride, void* out, int out
                                  float scale, int window, const float* sinks, const float* dist, const void* gate,
                                  int gate_stride, int gate_sigmoid, hipStream_t stream) {
   if (n_items <= 0) return FG_OK;
-  if (DIST_BIAS != (dist != nullptr) || !gate_ok(gate, gate_stride, n_heads)) return FG_ERR_ARG;
-  if (hd != HD || !(scale > 0.f) || n_kv <= 0 || n_heads % n_kv || n_heads / n_kv > item_rows || page_size < 8 || page_size % 8 ||
-      (long long)n_items * n_kv > 2147483647LL || q_stride % 8 || out_stride % 4 ||
-      (item_rows != TILE_ROWS && item_rows != TILE_ROWS_SMALL))
-    return FG_ERR_ARG;
   const TileArgs a{(const bf16_t*)q, q_stride, (bf16_t*)out, out_stride, (const bf16_t*)k_pages, (const bf16_t*)v_pages,
                    block_table, bt_stride, items, n_items, n_heads, n_kv, page_size, scale, window, sinks, dist,
                    OutGate{(const bf16_t*)gate, gate_stride, gate_sigmoid}, stream};
+  if (hd != HD || !tile_args_ok(a, item_rows)) return FG_ERR_ARG;
   if (TILE_PAIR_OK && item_rows == TILE_ROWS) PairForm<TILE_PAIR_OK>::go(a);
   else launch_tile<false>(a);
+  return fg_launch_status();
+}
+
+// Items of both kinds in one launch, as fg_attn_split_sink (merged) and fg_attn_tile_sink take them one after the other, for
+// pages of a multiple of 64 tokens.
+extern "C" int fg_attn_both(const void* q, int q_stride, void* out, int out_stride, const void* k_pages, const void* v_pages,
+                            const int* block_table, int bt_stride, const int* plan, int n_small, int max_chunks, int max_rows,
+                            float* part_o, float* part_ml, const int* items, int n_items, int item_rows, int n_heads, int n_kv,
+                            int hd, int page_size, float scale, int window, const float* sinks, const float* dist,
+                            const void* gate, int gate_stride, int gate_sigmoid, int ordered, hipStream_t stream) {
+  const TileArgs a{(const bf16_t*)q, q_stride, (bf16_t*)out, out_stride, (const bf16_t*)k_pages, (const bf16_t*)v_pages,
+                   block_table, bt_stride, items, n_items, n_heads, n_kv, page_size, scale, window, sinks, dist,
+                   OutGate{(const bf16_t*)gate, gate_stride, gate_sigmoid}, stream};
+  if (hd != HD || !tile_args_ok(a, item_rows) || page_size % 64 || n_items <= 0 || n_small <= 0 || n_heads / n_kv > 16 ||
+      max_chunks < 2 * n_small || max_chunks > 65535 || n_kv > 65535 || !plan || !part_o || !part_ml || max_rows < 1 ||
+      max_rows > 16 || ((long long)n_items + max_chunks) * n_kv > 2147483647LL)
+    return FG_ERR_ARG;
+  const SplitPart split{plan + PLAN_HEAD + (ordered ? 8LL * max_chunks : 0), part_o, part_ml, max_chunks, ordered, n_items * n_kv};
+  if (TILE_PAIR_OK && item_rows == TILE_ROWS) PairForm<TILE_PAIR_OK>::go(a, split);
+  else launch_pages<PAGES_TILE, false>(a, split);
+  launch_combine(part_o, part_ml, plan, a.out, out_stride, max_chunks, max_rows, n_heads, n_kv, sinks, a.gate, stream);
   return fg_launch_status();
 }
 

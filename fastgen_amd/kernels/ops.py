@@ -786,7 +786,8 @@ def paged_attention_mfma(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tens
     and ``window`` (made here if not given).  ``max_rows``: no small item has
     more rows (tokens times query heads per kv head) than this.  ``tile_rows``: the
     rows the big items were cut for (:func:`attention_tile_rows`; default: the larger form's).
-    With items of both kinds, and enough of the big ones to fill the GPU, the tile kernel runs on a second stream beside
+    With items of both kinds and pages of a multiple of 64 tokens one launch takes both; with other pages, and enough of the
+    big ones to fill the GPU, the tile kernel runs on a second stream beside
     the split kernel and the current stream waits for it before this returns (not while a graph is captured, not with
     ``FG_ONE_STREAM=1``).  ``exact_weights``: the build of the kernels in which the softmax weights enter
     the product with the values as two bfloat16 terms (16 significant bits).  ``sinks`` and ``distance``: as
@@ -824,8 +825,9 @@ def paged_attention_mfma(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tens
     lib = _mfma_attention(hd, exact_weights, dist)
     G = n_heads // n_kv
     beside = None
-    if (small_items is not None and big_items is not None and small_items.numel() and big_items.numel()
-            and _tiles_beside(big_items.numel() // 4 * n_kv) and not torch.cuda.is_current_stream_capturing()):
+    both = small_items is not None and big_items is not None and small_items.numel() > 0 and big_items.numel() > 0
+    together = both and page_size % 64 == 0
+    if (both and not together and _tiles_beside(big_items.numel() // 4 * n_kv) and not torch.cuda.is_current_stream_capturing()):
         # a step with both kinds of items (prompt portions beside decoded tokens): the two kernels write
         # different rows of `out`, one is bound by the matrix cores and one by memory, so the tile kernel
         # runs on a second stream beside the split kernel
@@ -847,14 +849,15 @@ def paged_attention_mfma(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tens
         _need(plan.dtype == torch.int32 and (ordered or more == 0), "the plan does not fit the items and max_chunks")
         part_o = torch.empty((max_chunks * n_kv * 16, hd), dtype=torch.float32, device=q.device)
         part_ml = torch.empty((max_chunks * n_kv * 16, 2), dtype=torch.float32, device=q.device)
-        st = lib.fg_attn_split_sink(
-            _ptr(q), q.stride(0), _ptr(out), out.stride(0), _ptr(k_pages), _ptr(v_pages), _ptr(block_table),
-            block_table.stride(0), _ptr(plan), n, max_chunks, max_rows, _ptr(part_o), _ptr(part_ml), n_heads, n_kv, hd,
-            page_size, float(scale), int(window or 0), _ptr(sinks), _ptr(distance), *gate_args, int(ordered),
-            int(not leave_parts), _stream(q))
-        _check(st, "attn_split")
-        if leave_parts:
-            return AttentionParts(out, part_o, part_ml, plan[10:], sinks, n_heads, n_kv)
+        if not together:
+            st = lib.fg_attn_split_sink(
+                _ptr(q), q.stride(0), _ptr(out), out.stride(0), _ptr(k_pages), _ptr(v_pages), _ptr(block_table),
+                block_table.stride(0), _ptr(plan), n, max_chunks, max_rows, _ptr(part_o), _ptr(part_ml), n_heads, n_kv, hd,
+                page_size, float(scale), int(window or 0), _ptr(sinks), _ptr(distance), *gate_args, int(ordered),
+                int(not leave_parts), _stream(q))
+            _check(st, "attn_split")
+            if leave_parts:
+                return AttentionParts(out, part_o, part_ml, plan[10:], sinks, n_heads, n_kv)
     if big_items is not None and big_items.numel():
         tile_rows = attention_tile_rows(hd, False, exact_weights, dist) if tile_rows is None else int(tile_rows)
         _need(tile_rows in (attention_tile_rows(hd, False, exact_weights, dist), attention_tile_rows(hd, True, exact_weights, dist)),
@@ -862,6 +865,14 @@ def paged_attention_mfma(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tens
         _need(G <= tile_rows, "too many query heads per kv head for the tile kernel")
         _i32(big_items, "big_items")
         _need(big_items.data_ptr() % 16 == 0, "items must be 16-byte aligned")
+        if together:
+            st = lib.fg_attn_both(
+                _ptr(q), q.stride(0), _ptr(out), out.stride(0), _ptr(k_pages), _ptr(v_pages), _ptr(block_table),
+                block_table.stride(0), _ptr(plan), n, max_chunks, max_rows, _ptr(part_o), _ptr(part_ml), _ptr(big_items),
+                big_items.numel() // 4, tile_rows, n_heads, n_kv, hd, page_size, float(scale), int(window or 0), _ptr(sinks),
+                _ptr(distance), *gate_args, int(ordered), _stream(q))
+            _check(st, "attn_both")
+            return out
         st = lib.fg_attn_tile_sink(
             _ptr(q), q.stride(0), _ptr(out), out.stride(0), _ptr(k_pages), _ptr(v_pages), _ptr(block_table),
             block_table.stride(0), _ptr(big_items), big_items.numel() // 4, tile_rows, n_heads, n_kv, hd, page_size,
@@ -914,7 +925,7 @@ def paged_attention(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v
                 small, big = attention_items(ctx.q_lens, ctx.q_start_host, ctx.n_cached, G, tile_rows)
             both = upload(np.concatenate([small, big]).reshape(-1), torch.int32, q.device)
             plan = (both[: small.size] if small.size else None, both[small.size:] if big.size else None, len(small),
-                    tile_rows, 16 if big.size else min(16, G * int(ctx.q_lens.max())))
+                    tile_rows, max((int(n) * G for n in ctx.q_lens if n * G <= 16), default=16))
         ctx.scratch[items_key] = plan
     small_d, big_d, n_small, tile_rows, max_rows = plan  # rows of the largest small item: one token a sequence in a decode step
     chunks = split_plan = None

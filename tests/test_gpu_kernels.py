@@ -1155,14 +1155,45 @@ def test_paged_attention_mfma_pages_of_whole_tiles(ops, H, KV, hd, P, window, sm
     assert torch.allclose(out.cpu().float(), _plain_rows(case, seqs, window or None), atol=1.5e-2, rtol=2e-2)
 
 
-def test_paged_attention_mfma_two_streams(ops, monkeypatch):
+@pytest.mark.parametrize("H,KV,hd,P", [(32, 8, 128, 64), (6, 3, 80, 128), (2, 1, 256, 64), (5, 5, 16, 192)])
+@pytest.mark.parametrize("n_decode", [1, 3, 40])
+@pytest.mark.parametrize("small_tiles", [False, True])
+@pytest.mark.parametrize("with_gate", [False, True])
+def test_paged_attention_mfma_both_kinds_in_one_launch(ops, H, KV, hd, P, n_decode, small_tiles, with_gate):
+    """Prompt portions and decoded tokens in one launch: the bits of a call for each kind, whatever the number of either
+    (more workgroups of the one, of the other, fewer than eight, an odd number of chunks, chunks in both orders) and
+    with what the outputs go through."""
+    import numpy as np
+
+    seqs = [(37 + 113 * i % 1900, 1) for i in range(n_decode)] + [(0, 70), (200, 121)] + ([(64, 700)] if n_decode == 3 else [])
+    case = _paged_case(torch.bfloat16, seqs, H, KV, hd, P, seed=41)
+    q_lens = [b for _, b in seqs]
+    tile_rows = ops.attention_tile_rows(hd, small_tiles)
+    small, big = ops.attention_items(q_lens, np.concatenate([[0], np.cumsum(q_lens)]), [a for a, _ in seqs], H // KV, tile_rows)
+    n = len(small)
+    assert n and len(big)
+    small, big = (torch.from_numpy(a.reshape(-1)).to(DEV) for a in (small, big))
+    gate = torch.randn(len(case["q"]), H * hd, device=DEV).bfloat16() if with_gate else None
+    sinks = torch.randn(H, device=DEV) if with_gate else None
+    for chunks, window in ((2 * n + 1, 0), (None, 90)):
+        def run(small, big):
+            return ops.paged_attention_mfma(case["q"], torch.full_like(case["q"][:, : H * hd], 7.0), case["kp"], case["vp"], case["table"],
+                                            small, big, H, hd ** -0.5, window, None, chunks, 1, H // KV, tile_rows, sinks=sinks,
+                                            gate=gate)
+        a, b, both = run(small, None), run(None, big), run(small, big)
+        apart = torch.cat([a[:n_decode], b[n_decode:]])  # (either leaves the other's rows alone)
+        assert torch.equal(both, apart) and torch.isfinite(both).all()
+
+
+@pytest.mark.parametrize("P", [32, 64])
+def test_paged_attention_mfma_two_streams(ops, monkeypatch, P):
     """Prompt portions beside decoded tokens: the tile kernel runs on a second stream beside the
-    split kernel.  The result is there when the caller's stream goes on (work queued behind the
+    split kernel where one launch cannot take both (pages of 32 tokens).  The result is there when the caller's stream goes on (work queued behind the
     call, on a stream that is not the default one, sees every row), equals the one-stream result
     bit for bit, and a call while a graph is captured stays on the capturing stream."""
     import numpy as np
 
-    H, KV, hd, P = 32, 8, 128, 64
+    H, KV, hd = 32, 8, 128
     seqs = [(900, 1), (0, 700), (2000, 1), (300, 260), (64, 1)]
     case = _paged_case(torch.bfloat16, seqs, H, KV, hd, P, seed=26)
     q_lens = [b for _, b in seqs]
