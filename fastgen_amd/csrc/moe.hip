@@ -30,7 +30,8 @@
 // A workgroup one token, four or eight.  Logits: the WAVES waves take the experts in turns of EPW (a wave
 // reads the rows of x once for its EPW experts, eight elements a lane and round, and an expert's row of the router once
 // for its tokens; the lanes' partial sums are added by the wave in a fixed order, the same in every form), into LDS.  A
-// turn is a chain of reads from the L2, so many waves of two experts each; several tokens, or the router would be read
+// turn is a chain of reads from the L2, so many waves of two experts each and, for one token, four rounds' reads together (12 tokens in a step, router
+// not in the L2: 9.7 -> 8.7 us; several tokens are bound by their multiplications); several tokens, or the router would be read
 // from the L2 once a token.  From there on a wave a token: the `top` largest (ties:
 // the lower expert) by a wave-wide argmax repeated `top` times, and the softmax over them.  LDS, per token: n_experts +
 // n_extra logits, then `top` chosen values, then n_experts scores, then n_groups ranks.
@@ -105,20 +106,46 @@ __global__ __launch_bounds__(64 * WAVES) void moe_route_kernel(
 #pragma unroll
       for (int i = 0; i < TOK; ++i) s[j][i] = 0.f;
     if (dim % 8 == 0 && ldx % 8 == 0) {
-      for (int k = lane * 8; k < dim; k += FG_WAVE * 8) {
-        float xv[TOK][8];
+      constexpr int U = TOK == 1 ? 4 : 1, EIGHT = FG_WAVE * 8;  // rounds whose loads are in flight together
+      typedef uint4 XRaw[sizeof(T) / 2];
+      auto rounds = [&](int k0, auto in_flight) {
+        constexpr int N = in_flight.value;
+        XRaw xraw[N][TOK];
+        float4 wraw[N][EPW][2];
 #pragma unroll
-        for (int i = 0; i < TOK; ++i) load8<T>(xr[i] + k, xv[i]);
-#pragma unroll
-        for (int j = 0; j < EPW; ++j) {
-          float wv[8];
-          load8<float>(wr + (size_t)min(e0 + j, n_rows - 1) * dim + k, wv);
+        for (int u = 0; u < N; ++u) {
+          const int k = k0 + u * EIGHT;
 #pragma unroll
           for (int i = 0; i < TOK; ++i)
 #pragma unroll
-            for (int u = 0; u < 8; ++u) s[j][i] = fmaf(xv[i][u], wv[u], s[j][i]);
+            for (int h = 0; h < (int)sizeof(T) / 2; ++h) xraw[u][i][h] = ((const uint4*)(xr[i] + k))[h];
+#pragma unroll
+          for (int j = 0; j < EPW; ++j)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) wraw[u][j][h] = ((const float4*)(wr + (size_t)min(e0 + j, n_rows - 1) * dim + k))[h];
         }
-      }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < N; ++u) {
+          float xv[TOK][8];
+#pragma unroll
+          for (int i = 0; i < TOK; ++i) load8<T>((const T*)&xraw[u][i], xv[i]);
+#pragma unroll
+          for (int j = 0; j < EPW; ++j) {
+            float wv[8];
+            load8<float>((const float*)&wraw[u][j], wv);
+#pragma unroll
+            for (int i = 0; i < TOK; ++i)
+#pragma unroll
+              for (int e = 0; e < 8; ++e) s[j][i] = fmaf(xv[i][e], wv[e], s[j][i]);
+          }
+        }
+      };
+      int k0 = 0;
+      for (; k0 + U * EIGHT <= dim; k0 += U * EIGHT) rounds(k0 + lane * 8, std::integral_constant<int, U>());
+      if constexpr (U > 1)
+        for (; k0 + EIGHT <= dim; k0 += EIGHT) rounds(k0 + lane * 8, std::integral_constant<int, 1>());
+      if (k0 + lane * 8 < dim) rounds(k0 + lane * 8, std::integral_constant<int, 1>());
     } else {
       for (int k = lane; k < dim; k += FG_WAVE) {
         float xv[TOK];
@@ -269,7 +296,9 @@ extern "C" int fg_moe_route(const void* x, int ldx, int dtype, const float* wr, 
 // tiles[i] = (expert, first pos, rows, 0) for i < max_tiles, rows = 0 for tiles that do not exist.  Experts from
 // n_tiled on have no tiles.
 // LDS: 3 * n_experts ints (count, first pos, first tile).
-#define SORT_THREADS 1024
+// Up to HELD pairs a thread are read once, all at the same time, and keep their number among their expert's from the count
+// (7,588 pairs of 32 experts: 7.4 -> 6.0 us); more are read and numbered again.
+template <int SORT_THREADS, int HELD>
 __global__ __launch_bounds__(SORT_THREADS) void moe_sort_kernel(
     const int* __restrict__ choice, int n_pairs, int n_experts, int n_tiled, int tile_rows, int max_tiles,
     int* __restrict__ sorted, int* __restrict__ tiles) {
@@ -278,8 +307,22 @@ __global__ __launch_bounds__(SORT_THREADS) void moe_sort_kernel(
   int* first = sm + n_experts;
   int* first_tile = sm + 2 * n_experts;
   for (int e = threadIdx.x; e < n_experts; e += SORT_THREADS) count[e] = 0;
+  const bool held = n_pairs <= HELD * SORT_THREADS;  // uniform
+  int expert[HELD], number[HELD];
+  if (held) {
+#pragma unroll
+    for (int i = 0; i < HELD; ++i) expert[i] = choice[min((int)threadIdx.x + i * SORT_THREADS, n_pairs - 1)];
+#pragma unroll
+    for (int i = 0; i < HELD; ++i) expert[i] = min(max(expert[i], 0), n_experts - 1);
+  }
   __syncthreads();
-  for (int p = threadIdx.x; p < n_pairs; p += SORT_THREADS) atomicAdd(&count[min(max(choice[p], 0), n_experts - 1)], 1);
+  if (held) {
+#pragma unroll
+    for (int i = 0; i < HELD; ++i)
+      if ((int)threadIdx.x + i * SORT_THREADS < n_pairs) number[i] = atomicAdd(&count[expert[i]], 1);
+  } else {
+    for (int p = threadIdx.x; p < n_pairs; p += SORT_THREADS) atomicAdd(&count[min(max(choice[p], 0), n_experts - 1)], 1);
+  }
   __syncthreads();
   if (threadIdx.x < FG_WAVE) {  // exclusive sums of rows and of tiles, 64 experts a round
     const int lane = threadIdx.x;
@@ -313,6 +356,14 @@ __global__ __launch_bounds__(SORT_THREADS) void moe_sort_kernel(
     }
     count[e] = 0;  // now the cursor of the second pass
   }
+  if (held) {
+#pragma unroll
+    for (int i = 0; i < HELD; ++i) {
+      const int p = threadIdx.x + i * SORT_THREADS;
+      if (p < n_pairs) sorted[first[expert[i]] + number[i]] = p;
+    }
+    return;
+  }
   __syncthreads();
   for (int p = threadIdx.x; p < n_pairs; p += SORT_THREADS) {
     const int e = min(max(choice[p], 0), n_experts - 1);
@@ -324,8 +375,11 @@ extern "C" int fg_moe_sort(const int* choice, int n_pairs, int n_experts, int n_
                            int* sorted, int* tiles, hipStream_t stream) {
   if (n_pairs <= 0) return FG_OK;
   if (n_experts <= 0 || n_tiled < 0 || n_tiled > n_experts || tile_rows <= 0 || max_tiles <= 0 || (size_t)3 * n_experts * sizeof(int) > 60000) return FG_ERR_ARG;
-  moe_sort_kernel<<<1, SORT_THREADS, (size_t)3 * n_experts * sizeof(int), stream>>>(choice, n_pairs, n_experts, n_tiled,
-                                                                                    tile_rows, max_tiles, sorted, tiles);
+  const size_t lds = (size_t)3 * n_experts * sizeof(int);
+  if (n_pairs <= 256 && n_experts <= 256)
+    moe_sort_kernel<256, 1><<<1, 256, lds, stream>>>(choice, n_pairs, n_experts, n_tiled, tile_rows, max_tiles, sorted, tiles);
+  else
+    moe_sort_kernel<1024, 8><<<1, 1024, lds, stream>>>(choice, n_pairs, n_experts, n_tiled, tile_rows, max_tiles, sorted, tiles);
   return fg_launch_status();
 }
 

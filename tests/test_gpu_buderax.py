@@ -299,6 +299,23 @@ def test_command_lines(cases, tmp_path):
     assert chat.returncode == 0, chat.stderr[-2000:]
 
 
+@pytest.mark.parametrize("pairs,E", [(1, 3), (255, 32), (256, 256), (256, 257), (257, 32), (1025, 7), (8192, 32), (8193, 32), (9001, 300)])
+def test_sort_at_the_edges_of_its_forms(pairs, E):
+    """Pairs that a thread holds, one more, and more experts than the small form counts: every pair once, among its expert's
+    places, and tiles that cover them."""
+    from fastgen_amd.kernels import ops
+
+    torch.manual_seed(pairs)
+    choice = torch.randint(0, E, (pairs, 1), dtype=torch.int32)
+    choice[choice == E // 2] = 0  # (one without pairs)
+    sorted_, tiles = (t.cpu() for t in ops.moe_sort(choice.cuda(), E, 16))
+    assert torch.equal(sorted_.sort().values, torch.arange(pairs, dtype=torch.int32))
+    assert torch.equal(choice[sorted_.long(), 0], choice[:, 0].sort().values)
+    assert int(tiles[:, 2].sum()) == pairs and int(tiles[:, 2].max()) <= 16
+    for e, first, rows, _ in tiles[tiles[:, 2] > 0].tolist():
+        assert (choice[sorted_[first : first + rows].long(), 0] == e).all()
+
+
 @pytest.mark.parametrize("counts,D,F", [((0, 64, 65, 128, 129, 256, 300, 1, 513), 192, 72 * 8), ((700,), 64, 64), ((3,) * 70 + (260,), 128, 136 * 8),
                                         ((1,) * 9, 320, 64), ((5,) * 3 + (0, 128) * 9 + (64, 1), 64, 136 * 8)])
 @pytest.mark.parametrize("tile_rows", [128, 256])
