@@ -32,6 +32,7 @@
 #include "attention_static.h"
 
 #include <stdio.h>
+#include <type_traits>
 
 #ifndef FG_HD
 #error "compile with -DFG_HD=<head size>"
@@ -1009,14 +1010,29 @@ struct SplitPart {
   float *part_o, *part_ml;
   int max_chunks, ordered, tile_groups /* workgroups with an item of the tiles */;
 };
-__device__ __forceinline__ const SplitPart& the_split(const SplitPart& s) { return s; }
-template <int PAGES, bool TILE_PAIR, class... SPLIT>
+// Where the workgroups of a step's items are about as many as the compute units, of which each holds one, the step takes as long as
+// its longest item: the last rows of a prompt see twice the keys of the average.  The host then cuts the items of many keys into
+// parts (KEYS): a part takes its share of the item's passes and leaves maximum, sum and O, in fp32 and in the order
+// its lanes hold them, to attn_parts_kernel.
+// 512 tokens of 32 heads on 8 behind 8,000 cached ones 174.6 -> 98 us, 100 behind 8,000 164.7 -> 65; prompts of 611 and 1,437 tokens of 16
+// heads on 4 40.4 -> 37 us.
+struct KeyParts {
+  const int* list;  // an item's two ints: its place among the parts (-1: the item is whole), part | parts << 16
+  float *o, *ml;    // [place][kv head][8 blocks of 16 rows] x [NDB][64 lanes][4], x [64 lanes][2]
+};
+template <class A, class... B>
+__device__ __forceinline__ const A& the_one(const A& a, const B&...) { return a; }
+template <class A, class B, class... C, class = std::enable_if_t<!std::is_same_v<A, B>>>
+__device__ __forceinline__ const A& the_one(const B&, const C&... c) { return the_one<A>(c...); }
+
+template <int PAGES, bool TILE_PAIR, class... MORE /* SplitPart, KeyParts */>
 __global__ __launch_bounds__(TILE_PAIR ? 512 : 256, TILE_PAIR ? 1 : 2) void attn_tile_kernel(
     const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, int out_stride,
     const bf16_t* __restrict__ k_pages, const bf16_t* __restrict__ v_pages,
     const int* __restrict__ block_table, int bt_stride, const int* __restrict__ items, int n_heads, int n_kv,
     int page_size, int page_shift, float scale, int window, const float* __restrict__ sinks,
-    const float* __restrict__ dist, const OutGate gate, const SPLIT... split) {
+    const float* __restrict__ dist, const OutGate gate, const MORE... more) {
+  constexpr bool SPLIT = (std::is_same_v<MORE, SplitPart> || ...), KEYS = (std::is_same_v<MORE, KeyParts> || ...);
   constexpr bool PERM = PAGES >= PAGES_CHUNK, WHOLE = PAGES == PAGES_TILE;
   constexpr int TILE_RB = TILE_PAIR ? 2 : 1;  // row blocks a wave holds
   constexpr int TILE_THREADS = TILE_PAIR ? 512 : 256;
@@ -1028,8 +1044,8 @@ __global__ __launch_bounds__(TILE_PAIR ? 512 : 256, TILE_PAIR ? 1 : 2) void attn
   __shared__ __attribute__((aligned(16))) bf16_t k_lds[NSLOT][TILE * HD];
   __shared__ __attribute__((aligned(16))) bf16_t v_lds[NSLOT][TILE * HD];
   int block = blockIdx.x;
-  if constexpr (sizeof...(SPLIT)) {
-    const SplitPart& sp = the_split(split...);
+  if constexpr (SPLIT) {
+    const SplitPart& sp = the_one<SplitPart>(more...);
     const int split_groups = gridDim.x - sp.tile_groups, both = min(sp.tile_groups, split_groups) / 8;  // eights of each kind that alternate
     int at;  // among the workgroups of its kind
     bool is_split;
@@ -1215,8 +1231,17 @@ __global__ __launch_bounds__(TILE_PAIR ? 512 : 256, TILE_PAIR ? 1 : 2) void attn
     else
       attend_tile<false, RB, false>(k0, me, qop, scale * LOG2E, m, l, o, load_k, load_v);
   };
-  const int k_first = (first_min / TILE) * TILE;
   constexpr int STEP = NPT * TILE;  // keys per pass of the loop
+  int k_first = (first_min / TILE) * TILE, k_last = pos_last, place = -1;
+  if constexpr (KEYS) {
+    const int2 part = *(const int2*)(the_one<KeyParts>(more...).list + 2 * (size_t)item);
+    place = part.x;
+    if (place >= 0) {  // uniform
+      const int n = part.y >> 16, i = part.y & 0xffff, passes = (pos_last - k_first) / STEP + 1;
+      k_last = min(pos_last, k_first + passes * (i + 1) / n * STEP - 1);
+      k_first += passes * i / n * STEP;
+    }
+  }
   if (NSLOT == 2 * NPT) {
     // Pass i is read from its slots while pass i+1 arrives in the other slots: one barrier a pass.
     // A tile that is one whole page inside the key range goes from memory straight into LDS (a
@@ -1226,7 +1251,7 @@ __global__ __launch_bounds__(TILE_PAIR ? 512 : 256, TILE_PAIR ? 1 : 2) void attn
     // page: the page of key k0, looked up a pass earlier so that nobody waits for the table here
     auto page_ahead = [&](int k0) { return pager.page_of(min(k0, pos_last)); };
     auto bring = [&](int k0, int slot, int page) {
-      if (k0 > pos_last) return;  // uniform
+      if (k0 > k_last) return;  // uniform
       if (WHOLE && k0 >= first_min && k0 + TILE - 1 <= pos_last) {
         const int kin = pager.in_page(k0);
         const bf16_t* base_k = k_pages + ((size_t)page * n_kv + kvh) * head_elems + (size_t)kin * HD;
@@ -1257,7 +1282,7 @@ __global__ __launch_bounds__(TILE_PAIR ? 512 : 256, TILE_PAIR ? 1 : 2) void attn
     bring(k_first, 0, page_ahead(k_first));
     bring(k_first + TILE, 1, page_ahead(k_first + TILE));
     int s0 = 0;
-    for (int k0 = k_first; k0 <= pos_last; k0 += STEP, s0 ^= NPT) {
+    for (int k0 = k_first; k0 <= k_last; k0 += STEP, s0 ^= NPT) {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's share of pass k0 has landed in LDS
       __syncthreads();  // pass k0 is complete in its slots; nobody reads the other slots any more
       bring(k0 + STEP, s0 ^ NPT, page_a);
@@ -1313,6 +1338,19 @@ __global__ __launch_bounds__(TILE_PAIR ? 512 : 256, TILE_PAIR ? 1 : 2) void attn
     }
     if (par == 1) return;
   }
+  if constexpr (KEYS) {
+    if (place >= 0) {  // uniform
+      const KeyParts& to = the_one<KeyParts>(more...);
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) {
+        const size_t at = ((size_t)place * n_kv + kvh) * 8 + rg * RB + rb;
+#pragma unroll
+        for (int db = 0; db < NDB; ++db) *(f32x4*)(to.o + ((at * NDB + db) * FG_WAVE + lane) * 4) = o[rb][db];
+        *(float2*)(to.ml + (at * FG_WAVE + lane) * 2) = make_float2(m[rb], l[rb]);
+      }
+      return;
+    }
+  }
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {
     float lsum = l[rb];
@@ -1328,18 +1366,64 @@ __global__ __launch_bounds__(TILE_PAIR ? 512 : 256, TILE_PAIR ? 1 : 2) void attn
   }
 }
 
+// What the parts of an item's keys left, added up: a wave a block of 16 rows, two workgroups of four an item and kv head.  merges: an item's
+// first flat token, tokens, first place and number of parts.
+__global__ __launch_bounds__(256) void attn_parts_kernel(const KeyParts from, const int* __restrict__ merges, bf16_t* __restrict__ out,
+                                                         int out_stride, int n_heads, int n_kv, const float* __restrict__ sinks,
+                                                         const OutGate gate) {
+  const int lane = threadIdx.x % FG_WAVE, block = blockIdx.x % 2 * 4 + threadIdx.x / FG_WAVE;  // of the item's eight of 16 rows
+  const int kvh = blockIdx.x / 2 % n_kv, G = n_heads / n_kv;
+  const int4 rec = *(const int4*)(merges + 4 * (size_t)(blockIdx.x / 2 / n_kv));
+  if (block * 16 >= rec.y * G) return;
+  f32x4 o[NDB];
+#pragma unroll
+  for (int db = 0; db < NDB; ++db) o[db] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, l = 0.f;
+  for (int i0 = 0; i0 < rec.w; i0 += 2) {  // (two parts' reads in flight; an odd last one is read twice and counts once)
+    f32x4 po[2][NDB];
+    float2 ml[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const size_t at = ((size_t)(rec.z + min(i0 + i, rec.w - 1)) * n_kv + kvh) * 8 + block;
+      ml[i] = *(const float2*)(from.ml + (at * FG_WAVE + lane) * 2);
+#pragma unroll
+      for (int db = 0; db < NDB; ++db) po[i][db] = *(const f32x4*)(from.o + ((at * NDB + db) * FG_WAVE + lane) * 4);
+    }
+    if (i0 + 1 == rec.w) ml[1].x = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const float M = fmaxf(m, ml[i].x);
+      const float fs = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - M);
+      const float fo = ml[i].x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml[i].x - M);
+      l = fs * l + fo * ml[i].y;
+      m = M;
+#pragma unroll
+      for (int db = 0; db < NDB; ++db) o[db] = fs * o[db] + fo * po[i][db];
+    }
+  }
+  l += __shfl_xor(l, 16, FG_WAVE);
+  l += __shfl_xor(l, 32, FG_WAVE);
+  const int row = block * 16 + lane % 16;
+  if (row >= rec.y * G) return;
+  const int t = rec.x + row / G, h = kvh * G + row % G, c = h * HD + 4 * (lane / 16);
+  if (sinks) l += __builtin_amdgcn_exp2f(sinks[h] * LOG2E - m);
+  if (gate.g) store_row(out, out_stride, o, 1.f / l, t, c, gate);  // uniform
+  else store_row(out, out_stride, o, 1.f / l, t, c);
+}
+
 struct TileArgs {
   const bf16_t* q; int q_stride; bf16_t* out; int out_stride; const bf16_t* k_pages; const bf16_t* v_pages;
   const int* block_table; int bt_stride; const int* items; int n_items, n_heads, n_kv, page_size; float scale;
   int window; const float* sinks; const float* dist; OutGate gate; hipStream_t stream;
 };
-template <int PAGES, bool PAIR, class... SPLIT>
-static void launch_pages(const TileArgs& a, SPLIT... split) {
-  int groups = a.n_items * a.n_kv;
-  ((groups += a.n_kv * ((split.max_chunks + (PAIR ? 1 : 0)) / (PAIR ? 2 : 1))), ...);
+template <bool PAIR> static int more_groups(const TileArgs& a, const SplitPart& s) { return a.n_kv * ((s.max_chunks + (PAIR ? 1 : 0)) / (PAIR ? 2 : 1)); }
+template <bool PAIR> static int more_groups(const TileArgs&, const KeyParts&) { return 0; }
+template <int PAGES, bool PAIR, class... MORE>
+static void launch_pages(const TileArgs& a, MORE... more) {
+  const int groups = (more_groups<PAIR>(a, more) + ... + (a.n_items * a.n_kv));
   attn_tile_kernel<PAGES, PAIR><<<groups, PAIR ? 512 : 256, 0, a.stream>>>(
       a.q, a.q_stride, a.out, a.out_stride, a.k_pages, a.v_pages, a.block_table, a.bt_stride, a.items, a.n_heads,
-      a.n_kv, a.page_size, page_shift_of(a.page_size), a.scale, a.window, a.sinks, a.dist, a.gate, split...);
+      a.n_kv, a.page_size, page_shift_of(a.page_size), a.scale, a.window, a.sinks, a.dist, a.gate, more...);
 }
 template <bool PAIR>
 static void launch_tile(const TileArgs& a) {
@@ -1350,11 +1434,11 @@ static void launch_tile(const TileArgs& a) {
 // the form with two tiles at a time exists up to head size 128 only (its LDS)
 template <bool EXISTS> struct PairForm {
   static void go(const TileArgs& a) { launch_tile<true>(a); }
-  static void go(const TileArgs& a, const SplitPart& split) { launch_pages<PAGES_TILE, true>(a, split); }
+  template <class... MORE> static void more(const TileArgs& a, MORE... m) { launch_pages<PAGES_TILE, true>(a, m...); }
 };
 template <> struct PairForm<false> {
   static void go(const TileArgs&) {}
-  static void go(const TileArgs&, const SplitPart&) {}
+  template <class... MORE> static void more(const TileArgs&, MORE...) {}
 };
 static bool tile_args_ok(const TileArgs& a, int item_rows) {
   return DIST_BIAS == (a.dist != nullptr) && gate_ok(a.gate.g, a.gate.stride, a.n_heads) && a.scale > 0.f && a.n_kv > 0 &&
@@ -1362,19 +1446,33 @@ static bool tile_args_ok(const TileArgs& a, int item_rows) {
          (long long)a.n_items * a.n_kv <= 2147483647LL && a.q_stride % 8 == 0 && a.out_stride % 4 == 0 &&
          (item_rows == TILE_ROWS || item_rows == TILE_ROWS_SMALL);
 }
+static bool key_parts_ok(const TileArgs& a, int item_rows, const KeyParts& keys, const int* merges, int n_merges) {
+  return TILE_PAIR_OK && item_rows == TILE_ROWS && a.page_size % 64 == 0 && keys.list && keys.o && keys.ml && merges &&
+         (long long)n_merges * a.n_kv <= 1073741823LL;
+}
+static void launch_merges(const TileArgs& a, const KeyParts& keys, const int* merges, int n_merges) {
+  attn_parts_kernel<<<2 * n_merges * a.n_kv, 256, 0, a.stream>>>(keys, merges, a.out, a.out_stride, a.n_heads, a.n_kv, a.sinks, a.gate);
+}
 
 // item_rows: the rows an item has at most, fg_attn_tile_rows(0) or fg_attn_tile_rows(1): which form of the kernel runs.
+// key_list, merges, n_merges, key_o, key_ml: the items are parts of keys (see KeyParts and attn_parts_kernel); n_merges 0: they are whole.
 extern "C" int fg_attn_tile_sink(const void* q, int q_stride, void* out, int out_stride, const void* k_pages,
                                  const void* v_pages, const int* block_table, int bt_stride, const int* items,
                                  int n_items, int item_rows, int n_heads, int n_kv, int hd, int page_size,
                                  float scale, int window, const float* sinks, const float* dist, const void* gate,
-                                 int gate_stride, int gate_sigmoid, hipStream_t stream) {
+                                 int gate_stride, int gate_sigmoid, const int* key_list, const int* merges, int n_merges,
+                                 float* key_o, float* key_ml, hipStream_t stream) {
   if (n_items <= 0) return FG_OK;
   const TileArgs a{(const bf16_t*)q, q_stride, (bf16_t*)out, out_stride, (const bf16_t*)k_pages, (const bf16_t*)v_pages,
                    block_table, bt_stride, items, n_items, n_heads, n_kv, page_size, scale, window, sinks, dist,
                    OutGate{(const bf16_t*)gate, gate_stride, gate_sigmoid}, stream};
   if (hd != HD || !tile_args_ok(a, item_rows)) return FG_ERR_ARG;
-  if (TILE_PAIR_OK && item_rows == TILE_ROWS) PairForm<TILE_PAIR_OK>::go(a);
+  const KeyParts keys{key_list, key_o, key_ml};
+  if (n_merges > 0) {
+    if (!key_parts_ok(a, item_rows, keys, merges, n_merges)) return FG_ERR_ARG;
+    PairForm<TILE_PAIR_OK>::more(a, keys);
+    launch_merges(a, keys, merges, n_merges);
+  } else if (TILE_PAIR_OK && item_rows == TILE_ROWS) PairForm<TILE_PAIR_OK>::go(a);
   else launch_tile<false>(a);
   return fg_launch_status();
 }
@@ -1385,7 +1483,8 @@ extern "C" int fg_attn_both(const void* q, int q_stride, void* out, int out_stri
                             const int* block_table, int bt_stride, const int* plan, int n_small, int max_chunks, int max_rows,
                             float* part_o, float* part_ml, const int* items, int n_items, int item_rows, int n_heads, int n_kv,
                             int hd, int page_size, float scale, int window, const float* sinks, const float* dist,
-                            const void* gate, int gate_stride, int gate_sigmoid, int ordered, hipStream_t stream) {
+                            const void* gate, int gate_stride, int gate_sigmoid, int ordered, const int* key_list, const int* merges,
+                            int n_merges, float* key_o, float* key_ml, hipStream_t stream) {
   const TileArgs a{(const bf16_t*)q, q_stride, (bf16_t*)out, out_stride, (const bf16_t*)k_pages, (const bf16_t*)v_pages,
                    block_table, bt_stride, items, n_items, n_heads, n_kv, page_size, scale, window, sinks, dist,
                    OutGate{(const bf16_t*)gate, gate_stride, gate_sigmoid}, stream};
@@ -1394,7 +1493,12 @@ extern "C" int fg_attn_both(const void* q, int q_stride, void* out, int out_stri
       max_rows > 16 || ((long long)n_items + max_chunks) * n_kv > 2147483647LL)
     return FG_ERR_ARG;
   const SplitPart split{plan + PLAN_HEAD + (ordered ? 8LL * max_chunks : 0), part_o, part_ml, max_chunks, ordered, n_items * n_kv};
-  if (TILE_PAIR_OK && item_rows == TILE_ROWS) PairForm<TILE_PAIR_OK>::go(a, split);
+  const KeyParts keys{key_list, key_o, key_ml};
+  if (n_merges > 0) {
+    if (!key_parts_ok(a, item_rows, keys, merges, n_merges)) return FG_ERR_ARG;
+    PairForm<TILE_PAIR_OK>::more(a, split, keys);
+    launch_merges(a, keys, merges, n_merges);
+  } else if (TILE_PAIR_OK && item_rows == TILE_ROWS) PairForm<TILE_PAIR_OK>::more(a, split);
   else launch_pages<PAGES_TILE, false>(a, split);
   launch_combine(part_o, part_ml, plan, a.out, out_stride, max_chunks, max_rows, n_heads, n_kv, sinks, a.gate, stream);
   return fg_launch_status();
@@ -1405,7 +1509,7 @@ extern "C" int fg_attn_tile(const void* q, int q_stride, void* out, int out_stri
                             int n_items, int item_rows, int n_heads, int n_kv, int hd, int page_size, float scale,
                             int window, hipStream_t stream) {
   return fg_attn_tile_sink(q, q_stride, out, out_stride, k_pages, v_pages, block_table, bt_stride, items, n_items,
-                           item_rows, n_heads, n_kv, hd, page_size, scale, window, nullptr, nullptr, nullptr, 0, 0, stream);
+                           item_rows, n_heads, n_kv, hd, page_size, scale, window, nullptr, nullptr, nullptr, 0, 0, nullptr, nullptr, 0, nullptr, nullptr, stream);
 }
 
 // query rows (tokens x heads of a kv head's group) of one item of fg_attn_tile: of the larger form, or

@@ -660,6 +660,90 @@ def attention_items(q_lens, q_start, n_cached, group_size: int, tile_rows: int =
     return as_arr(small), as_arr(big)
 
 
+@dataclass
+class KeyParts:
+    """Items of the tile kernel whose keys are cut: ``items`` (device int32 ``[n, 4]``, an item once a part), ``parts`` (``[n, 2]``:
+    the part's place among ``n_places``, -1 of a whole item, and its number | parts << 16) and ``merges`` (``[m, 4]``: first
+    flat token, tokens, first place, parts)."""
+
+    items: torch.Tensor
+    parts: torch.Tensor
+    merges: torch.Tensor
+    n_places: int
+
+
+KEY_PART_MAX_BYTES = 64 << 20  # of the parts' results
+
+
+KEY_PART_START, KEY_PART_MERGE, KEY_PART_GAIN = 3.5, 2.4, 0.93  # the first two in passes of a workgroup (128 keys, 2.5 us)
+SMALL_TILES_MAX_PASSES = 10
+
+
+def item_passes(big: np.ndarray, window: int) -> np.ndarray:
+    """Passes of 128 keys that the larger form of the tile kernel takes for each item."""
+    last = big[:, 3].astype(np.int64) + big[:, 2] - 1
+    first = np.maximum(big[:, 3] - window + 1, 0) if window > 0 else np.zeros_like(last)
+    return (last - first // 64 * 64) // 128 + 1
+
+
+def _passes_until_done(times: np.ndarray, places: int) -> float:
+    """When the last of ``times``, the longest first, ends on so many places."""
+    t = -np.sort(-times)
+    over = min(len(t), 2 * places) - places
+    done = float(t[0])
+    if over > 0:  # the second round's longest behind the first round's shortest
+        done = max(done, float((t[places : places + over] + t[places - over : places][::-1]).max()), float(t.sum()) / places)
+    return done
+
+
+def cut_key_ranges(big: np.ndarray, n_kv: int, head_dim: int, window: int, cus: int, most: Optional[int] = None):
+    """How the keys of a step's items (:func:`attention_items`, of the larger form) are cut into parts: ``(items, parts, merges, n_places)`` as
+    :class:`KeyParts` holds them, the longest parts first, or None where no cut is worth it.  ``most``: cut to at most that many passes.
+
+    A compute unit holds one workgroup, so that a step of up to two workgroups a unit ends with its longest item.  A workgroup takes
+    its passes (2.5 us each) and about 3.5 more until it begins and ends, the merge behind 2.4: counted so, what was measured comes out within 5
+    %.  Cut where that gains 7 % (each step pays 0.1 ms of the host's time for it).  Whole and in parts of at most 3/4, 1/2 and 1/4 of the
+    longest item's passes, us: 2,000 tokens of 16 heads on 4 (252 workgroups; not cut) 48.8 / 46.5 / 49.7 / 55.8; 611 and 1,437 40.4 / 36.5 /
+    37.5 / 43.6; 1,500 39.3 / 36.8 / 34.7 / 39.0; 1,500 of 24 heads on 8 (288; not cut) 41.2 / 45.7 / 47.2 / 52.8; 2,048 of 32 on 8 (512; not
+    cut) 60.9 / 73.3 / 76.2 / -; 512 behind 8,000 cached 174.6 / 98.1 / 99.9 / 105.7; 100 behind 8,000 164.7 / 94.7 / 94.4 / 57.1."""
+    if not len(big) or window < 0 or head_dim > 128 or (most is None and len(big) * n_kv > 2 * cus):
+        return None
+    passes = item_passes(big, window)
+    n = None
+    if most is None:
+        # parts of one and a half times the passes that each unit has if all are spread evenly
+        longest, places, total = int(passes.max()), max(1, cus // n_kv), int(passes.sum())
+        most = -(-3 * total // (2 * places))
+        whole = longest + KEY_PART_START if len(big) <= places else _passes_until_done(passes + KEY_PART_START, places)
+        if longest < 8 or most + KEY_PART_START + KEY_PART_MERGE >= KEY_PART_GAIN * whole:
+            return None
+        n = -(-passes // most)
+        if _passes_until_done(np.repeat(passes / n + KEY_PART_START, n), places) + KEY_PART_MERGE >= KEY_PART_GAIN * whole:
+            return None
+    n = -(-passes // max(1, most)) if n is None else n
+    if (n <= 1).all():
+        return None
+    places = np.where(n > 1, n, 0)
+    n_places = int(places.sum())
+    if n_places * n_kv * 128 * (head_dim + 8) * 4 > KEY_PART_MAX_BYTES or n.max() > 0x7fff:
+        return None
+    first_place = np.cumsum(places) - places
+    cut = np.nonzero(n > 1)[0]
+    merges = np.stack([big[cut, 1], big[cut, 2], first_place[cut], n[cut]], 1).astype(np.int32)
+    of = np.repeat(np.arange(len(big)), n)
+    number = np.arange(len(of)) - np.repeat(np.cumsum(n) - n, n)
+    share = passes[of] * (number + 1) // n[of] - passes[of] * number // n[of]
+    parts = np.stack([np.where(n[of] > 1, first_place[of] + number, -1), number | n[of] << 16], 1).astype(np.int32)
+    order = np.argsort(-share, kind="stable")
+    return np.ascontiguousarray(big[of][order]), np.ascontiguousarray(parts[order]), merges, n_places
+
+
+def upload_key_parts(cut, device) -> KeyParts:
+    items, parts, merges, n_places = cut
+    flat = upload(np.concatenate([items.reshape(-1), merges.reshape(-1), parts.reshape(-1)]), torch.int32, device)
+    return KeyParts(flat[: items.size], flat[items.size + merges.size:], flat[items.size : items.size + merges.size], n_places)
+
+
 def attention_chunks_for(n_items: int, n_kv: int) -> int:
     """Length of the split kernel's chunk list for ``n_items`` items: enough chunks for a few
     workgroups per compute unit, and at least two an item so that a long sequence among short
@@ -778,7 +862,8 @@ def paged_attention_mfma(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tens
                          min_tiles: int = 4, max_rows: int = 16, tile_rows: Optional[int] = None,
                          exact_weights: bool = False, sinks: Optional[torch.Tensor] = None,
                          distance: Optional[torch.Tensor] = None, gate: Optional[torch.Tensor] = None,
-                         gate_sigmoid: bool = True, leave_parts: bool = False) -> "torch.Tensor | AttentionParts":
+                         gate_sigmoid: bool = True, leave_parts: bool = False,
+                         key_parts: Optional[KeyParts] = None) -> "torch.Tensor | AttentionParts":
     """bf16 attention on the matrix cores.  ``small_items`` / ``big_items`` are
     device int32 ``[n, 4]`` lists from :func:`attention_items` (16-byte aligned);
     every query token of the step must be covered by exactly one item.
@@ -794,14 +879,15 @@ def paged_attention_mfma(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tens
     :func:`paged_attention_general` (a build of the kernels with exact weights takes the distance bias).  ``gate`` and
     ``gate_sigmoid``: what :func:`gate_mul` does with them behind the attention, done where the output is stored (the
     same bits), for bfloat16 rows that can be read in fours; else by that kernel.  ``leave_parts``: one token without a
-    gate comes as :class:`AttentionParts` where :func:`attention_parts_fit` the cache's pages."""
+    gate comes as :class:`AttentionParts` where :func:`attention_parts_fit` the cache's pages.  ``key_parts``: the big items, of the
+    larger form and pages of a multiple of 64 tokens, with their keys cut (:func:`cut_key_ranges`)."""
     leave_parts = (leave_parts and gate is None and (big_items is None or not big_items.numel()) and attention_parts_fit(
         q.shape[0], n_heads, k_pages.shape[3], k_pages.shape[1], block_table.shape[1] * k_pages.shape[2]))
     _gpu(q, out, k_pages, v_pages, block_table, small_items, big_items, plan, sinks, distance, gate)
     if gate is not None and (gate.dtype != torch.bfloat16 or gate.data_ptr() % 8 or gate.stride(0) % 4):
         return gate_mul(paged_attention_mfma(q, out, k_pages, v_pages, block_table, small_items, big_items, n_heads, scale,
                                              window, plan, max_chunks, min_tiles, max_rows, tile_rows, exact_weights, sinks,
-                                             distance), gate, gate_sigmoid)
+                                             distance, key_parts=key_parts), gate, gate_sigmoid)
     _need(gate is None or (gate.dim() == 2 and gate.shape[0] == q.shape[0] and gate.shape[1] >= out.shape[1]
                            and gate.stride(1) == 1), "gate must be [T, >= H*hd] with unit column stride")
     gate_args = (_ptr(gate), gate.stride(0) if gate is not None else 0, int(gate_sigmoid))
@@ -865,18 +951,34 @@ def paged_attention_mfma(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tens
         _need(G <= tile_rows, "too many query heads per kv head for the tile kernel")
         _i32(big_items, "big_items")
         _need(big_items.data_ptr() % 16 == 0, "items must be 16-byte aligned")
+        key_args = (0, 0, 0, 0, 0)
+        n_items = big_items.numel() // 4
+        if key_parts is not None:
+            _gpu(q, key_parts.items, key_parts.parts, key_parts.merges)
+            n_items, n_merges = key_parts.items.numel() // 4, key_parts.merges.numel() // 4
+            _need(page_size % 64 == 0 and hd <= 128 and tile_rows == attention_tile_rows(hd, False, exact_weights, dist),
+                  "items with their keys cut are of the larger form, and pages of a multiple of 64 tokens")
+            _need(key_parts.parts.numel() == 2 * n_items and n_merges > 0 and all(
+                t.dtype == torch.int32 and t.is_contiguous() for t in (key_parts.items, key_parts.parts, key_parts.merges))
+                and key_parts.items.data_ptr() % 16 == 0 and key_parts.merges.data_ptr() % 16 == 0
+                and key_parts.parts.data_ptr() % 8 == 0, "key_parts: int32 lists of one length, 16-byte aligned")
+            big_items = key_parts.items
+            rows = key_parts.n_places * n_kv * 128
+            key_o = torch.empty((rows, hd), dtype=torch.float32, device=q.device)
+            key_ml = torch.empty((rows, 8), dtype=torch.float32, device=q.device)
+            key_args = (_ptr(key_parts.parts), _ptr(key_parts.merges), n_merges, _ptr(key_o), _ptr(key_ml))
         if together:
             st = lib.fg_attn_both(
                 _ptr(q), q.stride(0), _ptr(out), out.stride(0), _ptr(k_pages), _ptr(v_pages), _ptr(block_table),
                 block_table.stride(0), _ptr(plan), n, max_chunks, max_rows, _ptr(part_o), _ptr(part_ml), _ptr(big_items),
-                big_items.numel() // 4, tile_rows, n_heads, n_kv, hd, page_size, float(scale), int(window or 0), _ptr(sinks),
-                _ptr(distance), *gate_args, int(ordered), _stream(q))
+                n_items, tile_rows, n_heads, n_kv, hd, page_size, float(scale), int(window or 0), _ptr(sinks),
+                _ptr(distance), *gate_args, int(ordered), *key_args, _stream(q))
             _check(st, "attn_both")
             return out
         st = lib.fg_attn_tile_sink(
             _ptr(q), q.stride(0), _ptr(out), out.stride(0), _ptr(k_pages), _ptr(v_pages), _ptr(block_table),
-            block_table.stride(0), _ptr(big_items), big_items.numel() // 4, tile_rows, n_heads, n_kv, hd, page_size,
-            float(scale), int(window or 0), _ptr(sinks), _ptr(distance), *gate_args,
+            block_table.stride(0), _ptr(big_items), n_items, tile_rows, n_heads, n_kv, hd, page_size,
+            float(scale), int(window or 0), _ptr(sinks), _ptr(distance), *gate_args, *key_args,
             beside.cuda_stream if beside else _stream(q))
         _check(st, "attn_tile")
         if beside is not None:
@@ -907,27 +1009,36 @@ def paged_attention(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v
                                 ctx.positions, n_heads, scale, window, sinks, distance)
         return out if gate is None else gate_mul(out, gate, gate_sigmoid)
     dist = distance is not None
-    items_key = ("attention_items", G, hd, n_kv)  # (how a step is cut into items depends on all three)
+    window = int(window or 0)
+    span = window if window < 0 or 0 < window < int((ctx.n_cached + ctx.q_lens).max()) else 0  # (0: every row sees all keys before it)
+    items_key = ("attention_items", G, hd, n_kv, span)  # (how a step is cut into items depends on all four)
     plan = ctx.scratch.get(items_key)
     if plan is None:
         if ctx.seq_records is not None and int(ctx.q_lens.max()) * G <= 16:
             # every sequence is one item of the split kernel: its records are in the step's buffer
             # already (and are refreshed with it when the step is a replayed graph)
-            plan = (ctx.seq_records, None, ctx.n_seqs, None, min(16, G * int(ctx.q_lens.max())))
+            plan = (ctx.seq_records, None, ctx.n_seqs, None, min(16, G * int(ctx.q_lens.max())), None)
         else:
             tile_rows = attention_tile_rows(hd, False, exact_weights, dist)
             small, big = attention_items(ctx.q_lens, ctx.q_start_host, ctx.n_cached, G, tile_rows)
-            if 0 < len(big) * n_kv <= compute_units() // 2 and attention_tile_rows(hd, True, exact_weights, dist) < tile_rows:
-                # so few items that half the compute units would stand idle: items of half the rows, whose
-                # lighter workgroups share a unit (prompt portions of up to 512 tokens: 11.6 / 17.6 us
-                # against 14.1 / 19.5 at 256 / 512 tokens; equal at 1,024, slower beyond)
-                tile_rows = attention_tile_rows(hd, True, exact_weights, dist)
-                small, big = attention_items(ctx.q_lens, ctx.q_start_host, ctx.n_cached, G, tile_rows)
+            groups, key_parts = len(big) * n_kv, None
+            if groups and attention_tile_rows(hd, True, exact_weights, dist) < tile_rows:
+                few_passes = int(item_passes(big, span).max()) <= SMALL_TILES_MAX_PASSES
+                cut = None if few_passes or k_pages.shape[2] % 64 else cut_key_ranges(big, n_kv, hd, span, compute_units())
+                if cut is not None:
+                    key_parts = upload_key_parts(cut, q.device)
+                elif groups <= (33 * compute_units() // 32 if few_passes else compute_units() // 2):
+                    # items of half the rows, whose lighter workgroups share a unit: where half the compute units would stand idle, and
+                    # of short key ranges up to a workgroup a unit (us with items of 128 and of 64 rows: 512 / 1,024 tokens of 32
+                    # heads on 8 17.5 / 27.8 and 14.8 / 26.8, three of 680 of 16 on 4 (264 workgroups) 23.0 and 20.8, 380 and 874 of 24 on 8 27.1 and
+                    # 25.8; 2,000 of 16 on 4, 16 passes, 48.8 and 49.9; 2,048 of 32 on 8 60.9 and 71.0)
+                    tile_rows = attention_tile_rows(hd, True, exact_weights, dist)
+                    small, big = attention_items(ctx.q_lens, ctx.q_start_host, ctx.n_cached, G, tile_rows)
             both = upload(np.concatenate([small, big]).reshape(-1), torch.int32, q.device)
             plan = (both[: small.size] if small.size else None, both[small.size:] if big.size else None, len(small),
-                    tile_rows, max((int(n) * G for n in ctx.q_lens if n * G <= 16), default=16))
+                    tile_rows, max((int(n) * G for n in ctx.q_lens if n * G <= 16), default=16), key_parts)
         ctx.scratch[items_key] = plan
-    small_d, big_d, n_small, tile_rows, max_rows = plan  # rows of the largest small item: one token a sequence in a decode step
+    small_d, big_d, n_small, tile_rows, max_rows, key_parts = plan  # rows of the largest small item: one token a sequence in a decode step
     chunks = split_plan = None
     if n_small:
         # how the items' key ranges are cut depends on the window: layers with the same one share the cut
@@ -940,7 +1051,7 @@ def paged_attention(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v
     return paged_attention_mfma(q, out, k_pages, v_pages, group.block_table, small_d, big_d, n_heads, scale,
                                 window, split_plan, chunks, max_rows=max_rows, tile_rows=tile_rows,
                                 exact_weights=exact_weights, sinks=sinks, distance=distance, gate=gate,
-                                gate_sigmoid=gate_sigmoid, leave_parts=leave_parts)
+                                gate_sigmoid=gate_sigmoid, leave_parts=leave_parts, key_parts=key_parts)
 
 
 # ----------------------------------------------------------------------- gemm

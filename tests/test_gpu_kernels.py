@@ -1185,6 +1185,40 @@ def test_paged_attention_mfma_both_kinds_in_one_launch(ops, H, KV, hd, P, n_deco
         assert torch.equal(both, apart) and torch.isfinite(both).all()
 
 
+@pytest.mark.parametrize("H,KV,hd,P,seqs,window", [(16, 4, 128, 64, [(0, 700)], 0), (6, 2, 64, 128, [(5, 1300), (70, 33)], 0),
+                                                    (5, 5, 16, 192, [(1000, 129), (0, 40)], 900), (8, 1, 80, 64, [(2000, 21), (64, 64)], 0)])
+@pytest.mark.parametrize("most", [1, 2, 5])
+@pytest.mark.parametrize("n_decode", [0, 3])
+@pytest.mark.parametrize("with_gate", [False, True])
+def test_paged_attention_mfma_keys_in_parts(ops, H, KV, hd, P, seqs, window, most, n_decode, with_gate):
+    """Items whose keys are cut into parts of one pass of 128 keys and of more, alone and beside decoded tokens, with whole items
+    among them, windows that a part lies in front of, and what the outputs go through: what whole items give, but for the order of fp32 sums
+    (one rounding of the output to bfloat16 may go the other way, 2^-8 of it) and the weights' roundings to bfloat16 under another
+    maximum (2^-9 each of the outputs' size, about 1)."""
+    import numpy as np
+
+    seqs = [(37 + 400 * i, 1) for i in range(n_decode)] + seqs
+    case = _paged_case(torch.bfloat16, seqs, H, KV, hd, P, seed=43)
+    q_lens = [b for _, b in seqs]
+    small, big = ops.attention_items(q_lens, np.concatenate([[0], np.cumsum(q_lens)]), [a for a, _ in seqs], H // KV,
+                                     ops.attention_tile_rows(hd))
+    cut = ops.cut_key_ranges(big, KV, hd, window, 256, most)
+    assert cut is not None and len(cut[0]) > len(big) and len(small) >= n_decode
+    small, big = (torch.from_numpy(a.reshape(-1)).to(DEV) if a.size else None for a in (small, big))
+    gate = torch.randn(len(case["q"]), H * hd, device=DEV).bfloat16() if with_gate else None
+    sinks = torch.randn(H, device=DEV) if with_gate else None
+
+    def run(key_parts):
+        return ops.paged_attention_mfma(case["q"], torch.full_like(case["q"][:, : H * hd], float("nan")), case["kp"], case["vp"], case["table"],
+                                        small, big, H, hd ** -0.5, window, None, None, 4, 16, None, sinks=sinks, gate=gate,
+                                        key_parts=key_parts)
+    whole, parts = run(None), run(ops.upload_key_parts(cut, DEV))
+    assert torch.isfinite(parts).all()
+    assert torch.allclose(parts.float(), whole.float(), atol=8e-3, rtol=2 ** -7)
+    if not with_gate:
+        assert torch.allclose(parts.cpu().float(), _plain_rows(case, seqs, window or None), atol=1.5e-2, rtol=2e-2)
+
+
 @pytest.mark.parametrize("P", [32, 64])
 def test_paged_attention_mfma_two_streams(ops, monkeypatch, P):
     """Prompt portions beside decoded tokens: the tile kernel runs on a second stream beside the

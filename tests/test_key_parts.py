@@ -1,0 +1,54 @@
+"""How the tile kernel's items are cut along their keys (host side, no GPU)."""
+
+import random
+
+import numpy as np
+import pytest
+
+from fastgen_amd.kernels import ops
+
+
+@pytest.mark.parametrize("most", [None, 1, 3, 7])
+def test_parts_cover_the_items(most):
+    """Every item once, whole or in all of its parts; places and merges without gaps; results within their limit."""
+    rng = random.Random(str(most))
+    cuts = 0
+    for _ in range(300):
+        lens = [rng.randint(17, 3000) for _ in range(rng.randint(1, 4))]
+        past = [rng.choice([0, 0, rng.randint(1, 20000)]) for _ in lens]
+        n_kv, window = rng.choice([1, 2, 4, 8]), rng.choice([0, 0, 100, 4096])
+        _, big = ops.attention_items(lens, np.concatenate([[0], np.cumsum(lens)]), past, rng.choice([1, 2, 3, 4, 8]), 128)
+        cut = ops.cut_key_ranges(big, n_kv, 128, window, 256, most)
+        if cut is None:
+            continue
+        cuts += 1
+        items, parts, merges, n_places = cut
+        assert n_places * n_kv * 128 * 136 * 4 <= ops.KEY_PART_MAX_BYTES
+        seen = {}
+        for it, (place, code) in zip(items.tolist(), parts.tolist()):
+            seen.setdefault(tuple(it), []).append((place, code & 0xFFFF, code >> 16))
+        assert set(seen) == {tuple(b) for b in big.tolist()}
+        of = {(t, n): (place, k) for t, n, place, k in merges.tolist()}
+        used = []
+        for it, has in seen.items():
+            if has[0][0] < 0:
+                assert len(has) == 1
+                continue
+            place, k = of.pop((it[1], it[2]))
+            assert k > 1 and sorted(has) == [(place + i, i, k) for i in range(k)]
+            used += [p for p, _, _ in has]
+        assert not of and sorted(used) == list(range(n_places))
+    assert cuts > 20
+
+
+def test_what_is_cut():
+    """Long key ranges on few workgroups are cut; short ones, evenly loaded steps, block windows and wide heads are not."""
+    def cut(lens, heads, n_kv, past=0, hd=128, window=0):
+        _, big = ops.attention_items(lens, np.concatenate([[0], np.cumsum(lens)]), [past] * len(lens), heads // n_kv, 128)
+        return ops.cut_key_ranges(big, n_kv, hd, window, 256)
+
+    assert cut([100], 32, 8, past=8000) and cut([512], 32, 8, past=8000) and cut([611, 1437], 16, 4)
+    assert cut([2048], 32, 8) is None and cut([2000], 16, 4) is None and cut([100], 32, 8) is None
+    assert cut([512], 32, 8, past=8000, hd=192) is None and cut([512], 32, 8, past=8000, window=-4096) is None
+    assert cut([512], 32, 8, past=8000, window=300) is None
+    assert ops.cut_key_ranges(np.zeros((0, 4), np.int32), 8, 128, 0, 256) is None
