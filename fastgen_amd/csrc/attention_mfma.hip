@@ -1005,6 +1005,9 @@ enum { PAGES_ANY = 0, PAGES_CHUNK = 1, PAGES_TILE = 2 };  // multiples of 8, 32,
 // Llama 3B's layer, prompts of 380 and 874 tokens beside 24 requests of 100 to 1,500: two launches on two streams took 58 us from
 // the cache's write to the next product (34 the tiles, 22 the split under them, 10 the combine kernel, and 17 of waits between the
 // streams), one launch 38 and the combine kernel, whose grid counts a decoded token's rows and not 16, 5.
+// The chunks' sums lie where the tiles do: with LDS of their own a unit held one workgroup from head size 224 on, not two.
+// 2,000 tokens of 16 heads on 4 beside 32, us: two launches 107 / 124 / 125 at 224 / 240 / 256, one with LDS of its own 207 /
+// 205 / 217, one now 106 / 121 / 124 (the registers are then half as many, and a chunk of these sizes spills 36 to 168 bytes a lane).
 struct SplitPart {
   const int* list;  // the plan's first or second list
   float *part_o, *part_ml;
@@ -1041,8 +1044,9 @@ __global__ __launch_bounds__(TILE_PAIR ? 512 : 256, TILE_PAIR ? 1 : 2) void attn
   // tiles in LDS: with pairs, one pair is read while the next is written (128 KB at head size 128, of
   // the CU's 160 KB: the workgroup has the CU to itself anyway; measured 4 % faster than two slots)
   constexpr int NSLOT = TILE_PAIR ? 4 : 1;
-  __shared__ __attribute__((aligned(16))) bf16_t k_lds[NSLOT][TILE * HD];
-  __shared__ __attribute__((aligned(16))) bf16_t v_lds[NSLOT][TILE * HD];
+  __shared__ __attribute__((aligned(16))) bf16_t kv_lds[2][NSLOT][TILE * HD];
+  auto& k_lds = kv_lds[0];
+  auto& v_lds = kv_lds[1];
   int block = blockIdx.x;
   if constexpr (SPLIT) {
     const SplitPart& sp = the_one<SplitPart>(more...);
@@ -1059,13 +1063,12 @@ __global__ __launch_bounds__(TILE_PAIR ? 512 : 256, TILE_PAIR ? 1 : 2) void attn
     }
     if (is_split) {  // uniform
       constexpr int HALVES = NT / 256, HALF = 2 * (sizeof(SplitO) + sizeof(SplitMl));  // groups of four waves, bytes of each
-      constexpr bool FITS = HALVES * HALF <= (int)sizeof(k_lds);  // (where tiles come in pairs)
-      __shared__ __attribute__((aligned(16))) char own_lds[FITS ? 16 : HALVES * HALF];
+      static_assert(HALVES * HALF <= sizeof(kv_lds), "the chunks' sums lie where tiles do");
       const int half = threadIdx.x / 256, first = at / n_kv * HALVES, mine = min(first + half, sp.max_chunks - 1);
       if (sp.list[(size_t)first * 8 + 6] == 0) return;  // uniform: not in use, and so none behind it
       int4 rec_a = *(const int4*)(sp.list + (size_t)mine * 8), rec_b = *(const int4*)(sp.list + (size_t)mine * 8 + 4);
       if (first + half > mine) rec_a = rec_b = int4{0, 0, 0, 0};
-      char* const at_lds = (FITS ? (char*)&k_lds[0][0] : own_lds) + half * HALF;
+      char* const at_lds = (char*)&kv_lds[0][0][0] + half * HALF;
       split_chunk<PERM>(rec_a, rec_b, sp.ordered ? rec_b.w : mine, at % n_kv, threadIdx.x / FG_WAVE % 4, (SplitO*)at_lds,
                         (SplitMl*)(at_lds + 2 * sizeof(SplitO)), q, q_stride, k_pages, v_pages, block_table, bt_stride,
                         sp.part_o, sp.part_ml, n_heads, n_kv, page_size, page_shift, scale, window, sinks, dist,
