@@ -676,7 +676,7 @@ KEY_PART_MAX_BYTES = 64 << 20  # of the parts' results
 
 
 KEY_PART_START, KEY_PART_MERGE, KEY_PART_GAIN = 3.5, 2.4, 0.93  # the first two in passes of a workgroup (128 keys, 2.5 us)
-SMALL_TILES_MAX_PASSES = 10
+KEY_PART_MIN_PASSES = 11  # of the longest item
 
 
 def item_passes(big: np.ndarray, window: int) -> np.ndarray:
@@ -715,7 +715,7 @@ def cut_key_ranges(big: np.ndarray, n_kv: int, head_dim: int, window: int, cus: 
         longest, places, total = int(passes.max()), max(1, cus // n_kv), int(passes.sum())
         most = -(-3 * total // (2 * places))
         whole = longest + KEY_PART_START if len(big) <= places else _passes_until_done(passes + KEY_PART_START, places)
-        if longest < 8 or most + KEY_PART_START + KEY_PART_MERGE >= KEY_PART_GAIN * whole:
+        if longest < KEY_PART_MIN_PASSES or most + KEY_PART_START + KEY_PART_MERGE >= KEY_PART_GAIN * whole:
             return None
         n = -(-passes // most)
         if _passes_until_done(np.repeat(passes / n + KEY_PART_START, n), places) + KEY_PART_MERGE >= KEY_PART_GAIN * whole:
@@ -1021,17 +1021,17 @@ def paged_attention(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v
         else:
             tile_rows = attention_tile_rows(hd, False, exact_weights, dist)
             small, big = attention_items(ctx.q_lens, ctx.q_start_host, ctx.n_cached, G, tile_rows)
-            groups, key_parts = len(big) * n_kv, None
-            if groups and attention_tile_rows(hd, True, exact_weights, dist) < tile_rows:
-                few_passes = int(item_passes(big, span).max()) <= SMALL_TILES_MAX_PASSES
-                cut = None if few_passes or k_pages.shape[2] % 64 else cut_key_ranges(big, n_kv, hd, span, compute_units())
+            key_parts = None
+            if len(big) and attention_tile_rows(hd, True, exact_weights, dist) < tile_rows:
+                cut = None if k_pages.shape[2] % 64 else cut_key_ranges(big, n_kv, hd, span, compute_units())
                 if cut is not None:
                     key_parts = upload_key_parts(cut, q.device)
-                elif groups <= (33 * compute_units() // 32 if few_passes else compute_units() // 2):
-                    # items of half the rows, whose lighter workgroups share a unit: where half the compute units would stand idle, and
-                    # of short key ranges up to a workgroup a unit (us with items of 128 and of 64 rows: 512 / 1,024 tokens of 32
-                    # heads on 8 17.5 / 27.8 and 14.8 / 26.8, three of 680 of 16 on 4 (264 workgroups) 23.0 and 20.8, 380 and 874 of 24 on 8 27.1 and
-                    # 25.8; 2,000 of 16 on 4, 16 passes, 48.8 and 49.9; 2,048 of 32 on 8 60.9 and 71.0)
+                elif len(big) * n_kv <= compute_units() // 2:
+                    # so few items that half the compute units would stand idle: items of half the rows, whose lighter workgroups
+                    # share a unit (512 tokens of 32 heads on 8, us with items of 128 and of 64 rows: 17.5 and 14.8).  They are the
+                    # quicker ones for short key ranges beyond that too (768 tokens 24.2 and 21.8, 1,024 28.3 and 26.7), but an item of
+                    # 128 rows has two maxima a row and so more weights that are 1 before they are rounded: its error against 64 bits
+                    # is the smaller one by 0.5 to 2.4 % in each of 24 cases, and a prompt keeps it
                     tile_rows = attention_tile_rows(hd, True, exact_weights, dist)
                     small, big = attention_items(ctx.q_lens, ctx.q_start_host, ctx.n_cached, G, tile_rows)
             both = upload(np.concatenate([small, big]).reshape(-1), torch.int32, q.device)

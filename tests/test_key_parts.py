@@ -52,3 +52,27 @@ def test_what_is_cut():
     assert cut([512], 32, 8, past=8000, hd=192) is None and cut([512], 32, 8, past=8000, window=-4096) is None
     assert cut([512], 32, 8, past=8000, window=300) is None
     assert ops.cut_key_ranges(np.zeros((0, 4), np.int32), 8, 128, 0, 256) is None
+
+
+@pytest.mark.parametrize("lens,heads,n_kv,rows", [([300], 32, 8, 64), ([512], 32, 8, 64), ([513], 32, 8, 128), ([380, 874], 24, 8, 128), ([1024], 32, 8, 128),
+                                                   ([680] * 3, 16, 4, 128), ([256] * 8, 16, 4, 128), ([2048], 32, 8, 128)])
+def test_prompts_keep_the_more_precise_items(monkeypatch, lens, heads, n_kv, rows):
+    """Items of 64 rows are for steps that leave half of 256 units idle; from there on the form of 128 rows, whose error against 64
+    bits is the smaller one, takes a prompt's rows."""
+    from types import SimpleNamespace
+
+    import torch
+
+    seen = []
+    monkeypatch.setattr(ops, "compute_units", lambda: 256)
+    monkeypatch.setattr(ops, "attention_tile_rows", lambda hd, small=False, exact=False, dist=False: 64 if small else 128)
+    monkeypatch.setattr(ops, "upload", lambda values, dtype, device: torch.as_tensor(values))
+    monkeypatch.setattr(ops, "paged_attention_mfma", lambda *a, tile_rows, key_parts, **k: seen.append((a[6], tile_rows, key_parts)))
+    starts = np.concatenate([[0], np.cumsum(lens)])
+    ctx = SimpleNamespace(q_lens=np.array(lens), n_cached=np.zeros(len(lens), int), q_start_host=starts, seq_records=None, scratch={})
+    q = torch.empty(1, heads * 128, dtype=torch.bfloat16)
+    pages = torch.empty(1, n_kv, 64, 128, dtype=torch.bfloat16)
+    ops.paged_attention(q, q, pages, pages, SimpleNamespace(block_table=None), ctx, heads, 1.0)
+    (items, got, parts), = seen
+    assert got == rows and parts is None
+    assert int(items.view(-1, 4)[:, 2].max()) <= rows // (heads // n_kv)
