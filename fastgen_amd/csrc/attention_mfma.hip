@@ -32,7 +32,10 @@
 #include "attention_static.h"
 
 #include <stdio.h>
+#include <algorithm>
+#include <functional>
 #include <type_traits>
+#include <vector>
 
 #ifndef FG_HD
 #error "compile with -DFG_HD=<head size>"
@@ -1412,6 +1415,96 @@ __global__ __launch_bounds__(256) void attn_parts_kernel(const KeyParts from, co
   if (sinks) l += __builtin_amdgcn_exp2f(sinks[h] * LOG2E - m);
   if (gate.g) store_row(out, out_stride, o, 1.f / l, t, c, gate);  // uniform
   else store_row(out, out_stride, o, 1.f / l, t, c);
+}
+
+// How the keys of a step's items (of the larger form, host memory) are cut into parts; what a cut gives is counted from a workgroup's
+// passes: a unit holds one workgroup, which takes its passes (128 keys, 2.5 us) and about 3.5 more until it begins and ends, and the
+// merge behind takes 2.4.  Cut where that gains 7 %, into parts of one and a half times the passes that each unit has if all are
+// spread evenly, from items of 11 passes on (the shortest that was measured to gain has 12).
+// Not in Python: a step on new inputs waits for it (prompts of 611 and 1,437 tokens, 65 items: 18 us with the call, 150 there).
+constexpr int KEY_PART_MIN_PASSES = 11;
+constexpr double KEY_PART_START = 3.5, KEY_PART_MERGE = 2.4, KEY_PART_GAIN = 0.93;
+
+// When the last of `t`, the longest first, ends on so many places (two rounds at most).
+static double passes_until_done(std::vector<double>& t, int places) {
+  std::sort(t.begin(), t.end(), std::greater<double>());
+  const int n = (int)t.size(), over = std::min(n, 2 * places) - places;
+  double done = t[0], total = 0.;
+  if (over <= 0) return done;
+  for (int i = 0; i < over; ++i) done = std::max(done, t[places + i] + t[places - 1 - i]);  // the second round's longest behind the first's shortest
+  for (double x : t) total += x;
+  return std::max(done, total / places);
+}
+
+// items: int32 [n_items][4]; places: workgroups that run at once for a kv head.  most: 0, or cut to at most that many passes whatever it gives.
+// cut: int32 [max_parts + n_items][4] items, the longest parts first, list: [max_parts + n_items][2] and merges: [n_items][4] as
+// the kernels take them, count: how many of them, of merges and of places.  No cut (or more than max_parts places): all 0.
+extern "C" int fg_attn_cut_keys(const int* items, int n_items, int window, int places, int most, int max_parts, int* cut, int* list,
+                                int* merges, int* count) try {
+  count[0] = count[1] = count[2] = 0;
+  if (n_items <= 0 || window < 0 || places < 1 || most < 0) return FG_OK;
+  std::vector<long long> passes(n_items), parts(n_items);
+  long long longest = 0, total = 0;
+  for (int i = 0; i < n_items; ++i) {
+    const int* it = items + 4 * (size_t)i;
+    const long long first = window > 0 ? std::max(0LL, (long long)it[3] - window + 1) : 0;
+    passes[i] = (it[3] + (long long)it[2] - 1 - first / 64 * 64) / 128 + 1;
+    longest = std::max(longest, passes[i]);
+    total += passes[i];
+  }
+  const bool asked = most > 0;
+  double whole = 0.;
+  if (!asked) {
+    most = (int)((3 * total + 2 * places - 1) / (2 * places));
+    if (longest < KEY_PART_MIN_PASSES) return FG_OK;
+    whole = longest + KEY_PART_START;
+    if (n_items > places) {
+      std::vector<double> t(n_items);
+      for (int i = 0; i < n_items; ++i) t[i] = passes[i] + KEY_PART_START;
+      whole = passes_until_done(t, places);
+    }
+    if (most + KEY_PART_START + KEY_PART_MERGE >= KEY_PART_GAIN * whole) return FG_OK;
+  }
+  long long n_places = 0, most_parts = 0, n_all = 0;
+  for (int i = 0; i < n_items; ++i) {
+    parts[i] = (passes[i] + most - 1) / most;
+    most_parts = std::max(most_parts, parts[i]);
+    n_all += parts[i];
+    if (parts[i] > 1) n_places += parts[i];
+  }
+  if (most_parts <= 1 || most_parts > 0x7fff || n_places > max_parts) return FG_OK;
+  if (!asked) {
+    std::vector<double> t;
+    t.reserve(n_all);
+    for (int i = 0; i < n_items; ++i) t.insert(t.end(), parts[i], (double)passes[i] / parts[i] + KEY_PART_START);
+    if (passes_until_done(t, places) + KEY_PART_MERGE >= KEY_PART_GAIN * whole) return FG_OK;
+  }
+  struct Part { long long share; int item, place, code; };
+  std::vector<Part> all;
+  all.reserve(n_all);
+  int place = 0;
+  for (int i = 0; i < n_items; ++i) {
+    const int n = (int)parts[i];
+    if (n > 1) {
+      const int* it = items + 4 * (size_t)i;
+      const int m[4] = {it[1], it[2], place, n};
+      std::copy(m, m + 4, merges + 4 * (size_t)count[1]++);
+    }
+    for (int k = 0; k < n; ++k)
+      all.push_back({passes[i] * (k + 1) / n - passes[i] * k / n, i, n > 1 ? place + k : -1, k | n << 16});
+    if (n > 1) place += n;
+  }
+  std::stable_sort(all.begin(), all.end(), [](const Part& a, const Part& b) { return a.share > b.share; });
+  for (size_t i = 0; i < all.size(); ++i) {
+    std::copy(items + 4 * (size_t)all[i].item, items + 4 * (size_t)all[i].item + 4, cut + 4 * i);
+    list[2 * i] = all[i].place;
+    list[2 * i + 1] = all[i].code;
+  }
+  count[0] = (int)all.size();
+  count[2] = (int)n_places;
+  return FG_OK;
+} catch (...) {  // no memory
+  return FG_ERR_ARG;
 }
 
 struct TileArgs {

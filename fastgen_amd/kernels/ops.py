@@ -675,73 +675,43 @@ class KeyParts:
 KEY_PART_MAX_BYTES = 64 << 20  # of the parts' results
 
 
-KEY_PART_START, KEY_PART_MERGE, KEY_PART_GAIN = 3.5, 2.4, 0.93  # the first two in passes of a workgroup (128 keys, 2.5 us)
-KEY_PART_MIN_PASSES = 11  # of the longest item
-
-
-def item_passes(big: np.ndarray, window: int) -> np.ndarray:
-    """Passes of 128 keys that the larger form of the tile kernel takes for each item."""
-    last = big[:, 3].astype(np.int64) + big[:, 2] - 1
-    first = np.maximum(big[:, 3] - window + 1, 0) if window > 0 else np.zeros_like(last)
-    return (last - first // 64 * 64) // 128 + 1
-
-
-def _passes_until_done(times: np.ndarray, places: int) -> float:
-    """When the last of ``times``, the longest first, ends on so many places."""
-    t = -np.sort(-times)
-    over = min(len(t), 2 * places) - places
-    done = float(t[0])
-    if over > 0:  # the second round's longest behind the first round's shortest
-        done = max(done, float((t[places : places + over] + t[places - over : places][::-1]).max()), float(t.sum()) / places)
-    return done
-
-
-def cut_key_ranges(big: np.ndarray, n_kv: int, head_dim: int, window: int, cus: int, most: Optional[int] = None):
+def cut_key_ranges(big: np.ndarray, n_kv: int, head_dim: int, window: int, cus: int, most: Optional[int] = None, exact: bool = False,
+                   dist: bool = False):
     """How the keys of a step's items (:func:`attention_items`, of the larger form) are cut into parts: ``(items, parts, merges, n_places)`` as
-    :class:`KeyParts` holds them, the longest parts first, or None where no cut is worth it.  ``most``: cut to at most that many passes.
+    :class:`KeyParts` holds them, the longest parts first, or None where no cut is worth it (``fg_attn_cut_keys`` counts that).
+    ``most``: cut to at most that many passes of 128 keys.
 
-    A compute unit holds one workgroup, so that a step of up to two workgroups a unit ends with its longest item.  A workgroup takes
-    its passes (2.5 us each) and about 3.5 more until it begins and ends, the merge behind 2.4: counted so, what was measured comes out within 5
-    %.  Cut where that gains 7 % (each step pays 0.1 ms of the host's time for it).  Whole and in parts of at most 3/4, 1/2 and 1/4 of the
-    longest item's passes, us: 2,000 tokens of 16 heads on 4 (252 workgroups; not cut) 48.8 / 46.5 / 49.7 / 55.8; 611 and 1,437 40.4 / 36.5 /
-    37.5 / 43.6; 1,500 39.3 / 36.8 / 34.7 / 39.0; 1,500 of 24 heads on 8 (288; not cut) 41.2 / 45.7 / 47.2 / 52.8; 2,048 of 32 on 8 (512; not
-    cut) 60.9 / 73.3 / 76.2 / -; 512 behind 8,000 cached 174.6 / 98.1 / 99.9 / 105.7; 100 behind 8,000 164.7 / 94.7 / 94.4 / 57.1."""
-    if not len(big) or window < 0 or head_dim > 128 or (most is None and len(big) * n_kv > 2 * cus):
+    Whole and in parts of at most 3/4, 1/2 and 1/4 of the longest item's passes, us: 2,000 tokens of 16 heads on 4 (252 workgroups;
+    not cut) 48.8 / 46.5 / 49.7 / 55.8; 611 and 1,437 40.4 / 36.5 / 37.5 / 43.6; 1,500 39.3 / 36.8 / 34.7 / 39.0; 1,500 of 24 heads on 8 (288;
+    not cut) 41.2 / 45.7 / 47.2 / 52.8; 2,048 of 32 on 8 (512; not cut) 60.9 / 73.3 / 76.2 / -; 512 behind 8,000 cached 174.6 / 98.1 / 99.9 /
+    105.7; 100 behind 8,000 164.7 / 94.7 / 94.4 / 57.1.  The error against 64 bits of items in parts is up to 7 % the smaller one (31 cuts): a
+    part has maxima of its own."""
+    n = len(big)
+    if not n or window < 0 or head_dim > 128 or (most is None and n * n_kv > 2 * cus):
         return None
-    passes = item_passes(big, window)
-    n = None
-    if most is None:
-        # parts of one and a half times the passes that each unit has if all are spread evenly
-        longest, places, total = int(passes.max()), max(1, cus // n_kv), int(passes.sum())
-        most = -(-3 * total // (2 * places))
-        whole = longest + KEY_PART_START if len(big) <= places else _passes_until_done(passes + KEY_PART_START, places)
-        if longest < KEY_PART_MIN_PASSES or most + KEY_PART_START + KEY_PART_MERGE >= KEY_PART_GAIN * whole:
-            return None
-        n = -(-passes // most)
-        if _passes_until_done(np.repeat(passes / n + KEY_PART_START, n), places) + KEY_PART_MERGE >= KEY_PART_GAIN * whole:
-            return None
-    n = -(-passes // max(1, most)) if n is None else n
-    if (n <= 1).all():
+    big = np.ascontiguousarray(big, dtype=np.int32)
+    places = KEY_PART_MAX_BYTES // (n_kv * 128 * (head_dim + 8) * 4)
+    at_merges, at_parts, at_count = 4 * (places + n), 4 * (places + 2 * n), 6 * (places + 2 * n)
+    out = np.empty(at_count + 3, np.int32)
+    to = out.ctypes.data
+    _check(_mfma_attention(head_dim, exact, dist).fg_attn_cut_keys(
+        big.ctypes.data, n, window, max(1, cus // n_kv), 0 if most is None else max(1, most), places, to, to + 4 * at_parts,
+        to + 4 * at_merges, to + 4 * at_count), "attn_cut_keys")
+    n_items, n_merges, n_places = out[at_count:].tolist()
+    if not n_items:
         return None
-    places = np.where(n > 1, n, 0)
-    n_places = int(places.sum())
-    if n_places * n_kv * 128 * (head_dim + 8) * 4 > KEY_PART_MAX_BYTES or n.max() > 0x7fff:
-        return None
-    first_place = np.cumsum(places) - places
-    cut = np.nonzero(n > 1)[0]
-    merges = np.stack([big[cut, 1], big[cut, 2], first_place[cut], n[cut]], 1).astype(np.int32)
-    of = np.repeat(np.arange(len(big)), n)
-    number = np.arange(len(of)) - np.repeat(np.cumsum(n) - n, n)
-    share = passes[of] * (number + 1) // n[of] - passes[of] * number // n[of]
-    parts = np.stack([np.where(n[of] > 1, first_place[of] + number, -1), number | n[of] << 16], 1).astype(np.int32)
-    order = np.argsort(-share, kind="stable")
-    return np.ascontiguousarray(big[of][order]), np.ascontiguousarray(parts[order]), merges, n_places
+    return (out[: 4 * n_items].reshape(-1, 4), out[at_parts : at_parts + 2 * n_items].reshape(-1, 2),
+            out[at_merges : at_merges + 4 * n_merges].reshape(-1, 4), n_places)
 
 
-def upload_key_parts(cut, device) -> KeyParts:
+def upload_key_parts(cut, device, before: Optional[np.ndarray] = None):
+    """:class:`KeyParts` of a cut on the device; with ``before``, other items, ``(them, KeyParts)``, in one copy."""
     items, parts, merges, n_places = cut
-    flat = upload(np.concatenate([items.reshape(-1), merges.reshape(-1), parts.reshape(-1)]), torch.int32, device)
-    return KeyParts(flat[: items.size], flat[items.size + merges.size:], flat[items.size : items.size + merges.size], n_places)
+    lists = ([] if before is None else [before]) + [items, merges, parts]
+    flat = upload(np.concatenate([a.reshape(-1) for a in lists]), torch.int32, device)
+    at = flat.split([a.size for a in lists])
+    kp = KeyParts(at[-3], at[-1], at[-2], n_places)
+    return kp if before is None else (at[0], kp)
 
 
 def attention_chunks_for(n_items: int, n_kv: int) -> int:
@@ -1021,12 +991,10 @@ def paged_attention(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v
         else:
             tile_rows = attention_tile_rows(hd, False, exact_weights, dist)
             small, big = attention_items(ctx.q_lens, ctx.q_start_host, ctx.n_cached, G, tile_rows)
-            key_parts = None
+            cut = None
             if len(big) and attention_tile_rows(hd, True, exact_weights, dist) < tile_rows:
-                cut = None if k_pages.shape[2] % 64 else cut_key_ranges(big, n_kv, hd, span, compute_units())
-                if cut is not None:
-                    key_parts = upload_key_parts(cut, q.device)
-                elif len(big) * n_kv <= compute_units() // 2:
+                cut = None if k_pages.shape[2] % 64 else cut_key_ranges(big, n_kv, hd, span, compute_units(), None, exact_weights, dist)
+                if cut is None and len(big) * n_kv <= compute_units() // 2:
                     # so few items that half the compute units would stand idle: items of half the rows, whose lighter workgroups
                     # share a unit (512 tokens of 32 heads on 8, us with items of 128 and of 64 rows: 17.5 and 14.8).  They are the
                     # quicker ones for short key ranges beyond that too (768 tokens 24.2 and 21.8, 1,024 28.3 and 26.7), but an item of
@@ -1034,8 +1002,13 @@ def paged_attention(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v
                     # is the smaller one by 0.5 to 2.4 % in each of 24 cases, and a prompt keeps it
                     tile_rows = attention_tile_rows(hd, True, exact_weights, dist)
                     small, big = attention_items(ctx.q_lens, ctx.q_start_host, ctx.n_cached, G, tile_rows)
-            both = upload(np.concatenate([small, big]).reshape(-1), torch.int32, q.device)
-            plan = (both[: small.size] if small.size else None, both[small.size:] if big.size else None, len(small),
+            if cut is not None:
+                small_d, key_parts = upload_key_parts(cut, q.device, small)
+                big_d = key_parts.items
+            else:
+                small_d, big_d = upload(np.concatenate([small, big]).reshape(-1), torch.int32, q.device).split([small.size, big.size])
+                key_parts = None
+            plan = (small_d if small.size else None, big_d if big.size else None, len(small),
                     tile_rows, max((int(n) * G for n in ctx.q_lens if n * G <= 16), default=16), key_parts)
         ctx.scratch[items_key] = plan
     small_d, big_d, n_small, tile_rows, max_rows, key_parts = plan  # rows of the largest small item: one token a sequence in a decode step
