@@ -73,10 +73,11 @@ class Model:
     def __init__(self, layout: ModelLayout, dtype: torch.dtype, device: torch.device | str, args: Any = None,
                  architecture: Optional[str] = None, packed_weights: Optional[bool] = None,
                  memory_budget: Optional[int] = None) -> None:
-        """``packed_weights``: whether the matrices get a second copy, bfloat16 ones in the order in which the products of few rows
-        read them, float32 ones in the parts that the products of many rows multiply (``kernels.linear.StreamedMatrix``); None: if the weights twice
-        leave half of ``memory_budget`` (bytes for the model and its cache; default: the GPU's memory) free
-        (``kernels.linear.packing_fits``)."""
+        """``packed_weights``: whether the bfloat16 matrices get a second copy in the order in which the products of few rows
+        read them (``kernels.linear.StreamedMatrix``); None: if the weights twice leave half of ``memory_budget`` (bytes for the
+        model and its cache; default: the GPU's memory) free (``kernels.linear.packing_fits``).  float32 matrices get one of the
+        parts that the products of many rows multiply by that rule alone, and with False none: True does not ask for it (2.5
+        times the memory of a model that may only just fit)."""
         if dtype not in (torch.float32, torch.bfloat16):
             raise ValueError(f"dtype {dtype} is not supported (float32 or bfloat16)")
         self.layout, self.dtype, self.device = layout, dtype, torch.device(device)
@@ -123,11 +124,11 @@ class Model:
     def load(self, source: TensorSource) -> None:
         specs = self.parts.tensor_specs()
         check_against_specs(source, specs, self.parts.duplicates())
-        pack = self.packed_weights
-        if pack is None:
+        pack, bf16 = self.packed_weights, self.dtype == torch.bfloat16
+        if pack is None or (pack and not bf16):
             # (a float32 matrix and its parts are 10 bytes an element, a bfloat16 one twice 4)
-            matrix_bytes = sum(math.prod(s.shape) for s in specs if s.role == MATRIX) * (2 if self.dtype == torch.bfloat16 else 5)
-            pack = packing_fits(matrix_bytes, self.device, self.memory_budget)
+            matrix_bytes = sum(math.prod(s.shape) for s in specs if s.role == MATRIX) * (2 if bf16 else 5)
+            pack = packing_fits(matrix_bytes, self.device, self.memory_budget, may_be_forced=bf16)
         with packing(pack):
             for part in self.parts.all_parts:
                 tensors = {s.name: source.get(s.name) for s in part.tensor_specs()}

@@ -155,12 +155,12 @@ def packing(on: bool):
         _pack_now = before
 
 
-def packing_fits(matrix_bytes: int, device, budget_bytes: Optional[int] = None) -> bool:
-    """The rule for the second copy when nobody says otherwise (``FG_PACKED_WEIGHTS=0`` / ``1`` does): the
-    weights twice take at most half of the memory that the model and its cache may use (``budget_bytes``;
-    default: all of the GPU's), so that at least half stays for the cache."""
+def packing_fits(matrix_bytes: int, device, budget_bytes: Optional[int] = None, may_be_forced: bool = True) -> bool:
+    """The rule for the second copy when nobody says otherwise (``FG_PACKED_WEIGHTS=0`` / ``1`` does; ``1`` only if it
+    ``may_be_forced``): the weights twice take at most half of the memory that the model and its cache may use
+    (``budget_bytes``; default: all of the GPU's), so that at least half stays for the cache."""
     forced = os.environ.get("FG_PACKED_WEIGHTS", "")
-    if forced in ("0", "1"):
+    if forced == "0" or (forced == "1" and may_be_forced):
         return forced == "1"
     dev = torch.device(device)
     if dev.type != "cuda":

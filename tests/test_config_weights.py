@@ -191,8 +191,8 @@ def test_dtype_policy():
 
 def test_second_copy_of_the_matrices_is_a_matter_of_memory(monkeypatch):
     """``packing_fits``: the switch wins; without it nothing is packed off the GPU.  ``streamed`` packs only
-    while a model says so (``packing``), and only bfloat16 matrices on the GPU: the 32-bit path and a part
-    that hands ``linear`` a plain tensor keep one copy."""
+    while a model says so (``packing``), and only matrices on the GPU (bfloat16 ones; of float32 ones it keeps the parts): a part
+    that hands ``linear`` a plain tensor keeps one copy."""
     from fastgen_amd.kernels import linear
 
     monkeypatch.delenv("FG_PACKED_WEIGHTS", raising=False)
@@ -218,6 +218,35 @@ def test_second_copy_of_the_matrices_is_a_matter_of_memory(monkeypatch):
     cut = m.first_rows(32)
     assert cut.rows.shape == (32, 64) and cut.packed is not None and cut.packed.shape == (32, 64)
     assert m.first_rows(20).packed is None  # no multiple of 16: the rows alone
+
+
+@pytest.mark.parametrize("dtype,asked,switch,fits,wanted", [
+    (torch.float32, None, None, True, True), (torch.float32, None, None, False, False), (torch.float32, True, None, False, False),
+    (torch.float32, True, None, True, True), (torch.float32, False, None, True, False), (torch.float32, None, "1", False, False),
+    (torch.float32, None, "1", True, True), (torch.float32, True, "0", True, False), (torch.float32, None, "0", True, False),
+    (torch.bfloat16, True, None, False, True), (torch.bfloat16, None, "1", False, True), (torch.bfloat16, None, None, True, True),
+    (torch.bfloat16, False, "1", True, False), (torch.bfloat16, None, "0", True, False), (torch.bfloat16, None, None, False, False)])
+def test_a_forced_second_copy_is_one_of_bfloat16_matrices(monkeypatch, dtype, asked, switch, fits, wanted):
+    """Asking for the second copy is asking for the decode products' order: a float32 model, whose parts take half as much again as
+    that would, gets them only where the rule finds the memory, whatever is asked."""
+    from fastgen_amd.engine import model as engine_model
+    from fastgen_amd.kernels import linear
+    from plain_llama import TINY_A
+
+    monkeypatch.delenv("FG_PACKED_WEIGHTS", raising=False)
+    if switch is not None:
+        monkeypatch.setenv("FG_PACKED_WEIGHTS", switch)
+    monkeypatch.setattr(torch.cuda, "get_device_properties", lambda dev: type("P", (), {"total_memory": 1 << (40 if fits else 10)})())
+    said, there = [], linear.packing
+    monkeypatch.setattr(engine_model, "packing", lambda on: said.append(bool(on)) or there(on))
+    made = engine_model.Model.from_config(TINY_A, dtype, "cpu", asked)
+    made.device = torch.device("cuda:0")  # as far as the rule is concerned
+    for part in made.parts.all_parts:
+        monkeypatch.setattr(part, "load", lambda *a: None)
+    monkeypatch.setattr(made.parts.head, "tied_to", "", raising=False)
+    monkeypatch.setattr(engine_model, "check_against_specs", lambda *a: None)
+    made.load(type("S", (), {"get": lambda self, name: None})())
+    assert said == [wanted]
 
 
 def ops_pack(w):

@@ -330,3 +330,28 @@ def test_every_kernel_that_may_be_chosen_gives_the_plain_logits(forced, packed, 
     assert ("gemm_large" in taken) == large and (forced not in ("tiled", "tiled256") or taken == {"gemm_tiled"})
     if forced is None:
         assert linear.choices and set(linear.choices.values()) <= {"narrow", "wide", "tiled", "tiled256", "library"}
+
+
+@pytest.mark.parametrize("switch", [None, "0", "1"])
+def test_float32_matrices_and_their_parts(monkeypatch, switch):
+    """A float32 model keeps its matrices' parts beside them (k a multiple of 128, and tokens of a step that go through them), counts
+    them among its weights, and has none with the switch off; its logits are the same bits."""
+    from fastgen_amd.engine import Model, ModelRunner, StepEntry
+    from fastgen_amd.kernels.linear import StreamedMatrix
+
+    cfg = dict(TINY_B, hidden_size=256, num_attention_heads=4, num_key_value_heads=2, intermediate_size=384)
+    monkeypatch.delenv("FG_PACKED_WEIGHTS", raising=False)
+    logits = []
+    for setting in (switch, "0"):
+        if setting is not None:
+            monkeypatch.setenv("FG_PACKED_WEIGHTS", setting)
+        model = Model.random(cfg, 3, torch.float32, "cuda:0")
+        held = [(p, v) for p in model.parts.all_parts for v in vars(p).values() if isinstance(v, StreamedMatrix)]
+        assert len(held) == 4 * cfg["num_hidden_layers"] + 1
+        for part, m in held:
+            assert m.packed is None and (m.cut is not None) == (setting != "0" and part is not model.parts.head)
+            assert m.nbytes() == m.rows.numel() * (4 if m.cut is None else 10) + (6 * m.shape[1] * (-m.shape[0] % 16) if m.cut else 0)
+        assert model.weight_bytes() >= sum(m.nbytes() for _, m in held)
+        runner = ModelRunner(model, page_size=64, max_tokens=1024, max_requests=2)
+        logits.append(runner.step([StepEntry(0, list(range(1, 201)), [17, 199])]).clone())
+    assert torch.equal(*logits)
