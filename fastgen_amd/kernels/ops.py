@@ -1037,7 +1037,7 @@ GEMM_F32_GROUP = 1024
 GEMM_F32_FEW_ROWS, GEMM_F32_MAX_SUMS, GEMM_F32_MAX_SPLIT_ROWS = 8, 256 << 20, 4096
 
 
-def gemm_f32_plan(M: int, N: int, K: int, cus: int, behind: bool = False) -> Tuple[int, int, bool]:
+def gemm_f32_plan(M: int, N: int, K: int, cus: int) -> Tuple[int, int, bool]:
     """How the 32-bit product is cut: (blocks of 16 rows in a tile, waves of 32 outputs in a tile, whether every group of k
     has a workgroup of its own); (0, 0, False): the kernel of 16 rows and 16 outputs.  Every cut gives the same bits.
 
@@ -1051,19 +1051,22 @@ def gemm_f32_plan(M: int, N: int, K: int, cus: int, behind: bool = False) -> Tup
     instructions, 32 x 32 outputs a workgroup, products that fill the chip took 1.3 to 1.7 times as long, and some below 30
     us that do not 1 to 6 us less.)
 
-    ``behind``: the groups' sums are added up by the kernel that follows the product anyway (a norm, an activation, a rotation).  Up
-    to 16 rows the kernel of 16 rows may then be cut too: a round of 1,024 k of its workgroups takes 3.5 us a workgroup and compute unit,
-    3.8 at least; cut, all of W comes at 5.1 TB/s behind 7.5 us, 2 % more a row beyond four, and the sums cost the kernel behind 1 us and
-    0.35 a group.  Measured at 4 rows, uncut and cut, with the kernel behind: 5,120 x 3,072 (320 workgroups) 31 and 25, 3,072 x 8,192 38.1 and 35.2,
-    3,072 x 3,072 19.8 and 20.6, 4,096 x 14,336 61.0 and 62.8."""
-    return _f32_plan(M, N, K, cus, behind, False)[1]
+    (A product with a kernel behind it that adds the groups' sums up, and one of operands cut beforehand: :func:`_f32_plan`.)"""
+    return _f32_plan(M, N, K, cus, False, False)[1]
 
 
 @functools.lru_cache(maxsize=4096)
 def _f32_plan(M: int, N: int, K: int, cus: int, behind: bool, cut: bool) -> Tuple[float, Tuple[int, int, bool]]:
-    """The microseconds of a cut as :func:`gemm_f32_plan` counts them (of no use up to 8 rows), and the cut.  ``cut``: tiles of operands cut
-    into their parts beforehand, whose steps take 0.83 of the time and whose W is half as many bytes again, and the kernel that
-    cuts x (3 us; 4 bytes of an element read and 6 written)."""
+    """The microseconds of a cut as :func:`gemm_f32_plan` counts them (of no use up to 8 rows), and the cut.
+
+    ``behind``: the groups' sums are added up by the kernel that follows the product anyway (a norm, an activation, a rotation).  Up
+    to 16 rows the kernel of 16 rows may then be cut too: a round of 1,024 k of its workgroups takes 3.5 us a workgroup and compute unit,
+    3.8 at least; cut, all of W comes at 5.1 TB/s behind 7.5 us, 2 % more a row beyond four, and the sums cost the kernel behind 1 us and
+    0.35 a group.  Measured at 4 rows, uncut and cut, with the kernel behind: 5,120 x 3,072 (320 workgroups) 31 and 25, 3,072 x 8,192 38.1 and 35.2,
+    3,072 x 3,072 19.8 and 20.6, 4,096 x 14,336 61.0 and 62.8.
+
+    ``cut``: tiles of operands cut into their parts beforehand, whose steps take 0.83 of the time and whose W is half as many bytes
+    again, and the kernel that cuts x (3 us; 4 bytes of an element read and 6 written)."""
     if M <= GEMM_F32_FEW_ROWS and not behind:
         return 0.0, (0, 0, False)
     groups, blocks, streaming = -(-K // GEMM_F32_GROUP), -(-M // 16), N * K * (6 if cut else 4) / 5e6
@@ -1071,7 +1074,7 @@ def _f32_plan(M: int, N: int, K: int, cus: int, behind: bool, cut: bool) -> Tupl
     whole = K // GEMM_F32_GROUP + (max(0.4, part) if part else 0)
     wgs = -(-N // 16) * blocks
     best = 2 + max(whole * (4.8 if wgs <= cus else max(9, 1.6 + 4 * wgs / cus)), streaming), (0, 0, False)
-    if behind and M <= 16 and groups > 1:
+    if behind and M <= 16 and groups > 1 and groups * M * N * 4 <= GEMM_F32_MAX_SUMS:
         uncut = 4 + whole * max(3.8, 3.5 * -(-wgs // cus))
         by_groups = (7.5 + N * K * 4 / 5.1e6) * (1 + 0.02 * max(0, M - 4)) + 1 + 0.35 * groups
         best = min(best if M > GEMM_F32_FEW_ROWS else (uncut, (0, 0, False)), (by_groups, (0, 0, True)))
@@ -1101,7 +1104,8 @@ def _f32_plan(M: int, N: int, K: int, cus: int, behind: bool, cut: bool) -> Tupl
 
 
 def gemm_f32_scratch(M: int, N: int, K: int) -> int:
-    """Bytes of the groups' sums that :func:`gemm_nt` takes at most for up to ``M`` rows (see :func:`gemm_f32_plan`)."""
+    """Bytes of the groups' sums that a 32-bit product takes at most for up to ``M`` rows, whatever is behind it and whether or not its
+    operands are cut beforehand (see :func:`_f32_plan`)."""
     groups = -(-K // GEMM_F32_GROUP)
     sums = min(groups * min(M, GEMM_F32_MAX_SPLIT_ROWS) * N * 4, GEMM_F32_MAX_SUMS)
     return sums if groups > 1 else 0

@@ -678,3 +678,18 @@ def test_step_memory_estimate_counts_what_parts_take_beside_their_rows():
             taken = max((-(-K // ops.GEMM_F32_GROUP) * m * N * 4 for m in range(1, M + 1)
                          if ops.gemm_f32_plan(m, N, K, cus)[2]), default=0)
             assert taken <= ops.gemm_f32_scratch(M, N, K), (M, N, K)
+
+
+@pytest.mark.parametrize("behind", [False, True])
+@pytest.mark.parametrize("cut", [False, True])
+def test_sums_of_32_bit_products_stay_inside_what_is_counted_for_them(behind, cut):
+    """Whatever adds the sums up and however the operands lie, no plan takes more than the estimate knows of, the widest products of few
+    rows included (164,864 outputs of 53,248 at 8 rows would be 274 MB)."""
+    from fastgen_amd.kernels import ops
+
+    for N, K in ((64, 1025), (3072, 8192), (4096, 14336), (16384, 3072), (28672, 8192), (164864, 53248), (128256, 8192)):
+        taken = 0
+        for M in (*range(1, 65), 100, 400, 2048, 4096, 4097, 8192):
+            if ops._f32_plan(M, N, K, 256, behind, cut)[1][2]:
+                taken = max(taken, -(-K // ops.GEMM_F32_GROUP) * M * N * 4)
+            assert taken <= min(ops.gemm_f32_scratch(M, N, K), ops.GEMM_F32_MAX_SUMS), (M, N, K)
