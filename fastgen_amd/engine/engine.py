@@ -16,7 +16,7 @@ from typing import Any, Dict, Hashable, List, Mapping, Optional, Sequence
 
 import torch
 
-from ..kernels.ops import gemm_f32_scratch, gemm_large_scratch
+from ..kernels.ops import gemm_f32_scratch, gemm_large_scratch, key_parts_scratch
 from ..sampling import Sampler, SamplingParams
 from .context import StepEntry
 from .model import Model
@@ -44,17 +44,20 @@ def step_memory_estimate(model: Model, max_step_tokens: int, max_batch: int) -> 
     widest matrix product of a layer (its output, the activation made from it, the fp32 partial sums
     of the product after it) and the fp32 residual stream; per request a row of fp32 logits, twice
     (a captured step keeps its own); and the most that a part takes beside that (the states of a recurrence's
-    chunks, the sums over k of a 32-bit product or of a prompt's).  (``fastgen/utils/tune.py:46-65`` budgets 1.2 x (4 dim + 4 ffn)
+    chunks, the sums over k of a 32-bit product or of a prompt's, the results of a prompt's keys in parts).  (``fastgen/utils/tune.py:46-65`` budgets 1.2 x (4 dim + 4 ffn)
     bytes a token for the same purpose.)"""
     widest, scratch = model.layout.dim, 0
     for part in model.parts.all_parts[1:-1]:  # the layers' parts; the embedding and the head are not per token
         scratch = max(scratch, part.scratch_bytes(max_step_tokens, max_batch))
+        need = part.paged_need() if hasattr(part, "paged_need") else None
+        if need is not None and model.dtype == torch.bfloat16:
+            scratch = max(scratch, key_parts_scratch(need.head_dim))
         for v in vars(part).values():
             shape = getattr(v, "shape", None)  # a tensor or a kernels.linear.StreamedMatrix
             if shape is not None and len(shape) == 2:
                 widest = max(widest, shape[0])
                 if v.dtype == torch.float32:
-                    cut = 6 * max_step_tokens * shape[1] if getattr(v, "cut", None) is not None else 0  # x in its parts
+                    cut = 6 * (-(-max_step_tokens // 16) * 16) * shape[1] if getattr(v, "cut", None) is not None else 0  # x in its parts
                     scratch = max(scratch, gemm_f32_scratch(max_step_tokens, *shape) + cut)
                 elif getattr(v, "packed", None) is not None:
                     scratch = max(scratch, gemm_large_scratch(max_step_tokens, shape[0]))

@@ -675,6 +675,11 @@ class KeyParts:
 KEY_PART_MAX_BYTES = 64 << 20  # of the parts' results
 
 
+def key_parts_scratch(head_dim: int) -> int:
+    """Bytes that the results of a step's keys in parts take at most (:func:`cut_key_ranges`)."""
+    return KEY_PART_MAX_BYTES if head_dim % 16 == 0 and head_dim <= 128 else 0
+
+
 def cut_key_ranges(big: np.ndarray, n_kv: int, head_dim: int, window: int, cus: int, most: Optional[int] = None, exact: bool = False,
                    dist: bool = False):
     """How the keys of a step's items (:func:`attention_items`, of the larger form) are cut into parts: ``(items, parts, merges, n_places)`` as

@@ -693,3 +693,21 @@ def test_sums_of_32_bit_products_stay_inside_what_is_counted_for_them(behind, cu
             if ops._f32_plan(M, N, K, 256, behind, cut)[1][2]:
                 taken = max(taken, -(-K // ops.GEMM_F32_GROUP) * M * N * 4)
             assert taken <= min(ops.gemm_f32_scratch(M, N, K), ops.GEMM_F32_MAX_SUMS), (M, N, K)
+
+
+def test_step_memory_estimate_counts_keys_in_parts():
+    """A bfloat16 model whose prompts' keys may be cut into parts leaves room for the parts' results; a float32 one (the general
+    kernel) and one of wider heads have none."""
+    import torch
+
+    from fastgen_amd.engine import Model
+    from fastgen_amd.engine.engine import step_memory_estimate
+    from fastgen_amd.kernels import ops
+    from plain_llama import TINY_A
+
+    def beside(cfg, dtype):
+        plain = 100 * 12 * 2 * cfg["intermediate_size"] + 3 * 4 * cfg["vocab_size"] * 4
+        return step_memory_estimate(Model.random(cfg, 0, dtype, "cpu"), 100, 4) - plain
+
+    assert beside(TINY_A, torch.bfloat16) == ops.KEY_PART_MAX_BYTES
+    assert beside(TINY_A, torch.float32) == 0 and ops.key_parts_scratch(160) == 0 and ops.key_parts_scratch(128) == ops.KEY_PART_MAX_BYTES
