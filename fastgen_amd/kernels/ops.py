@@ -1249,7 +1249,10 @@ def gemm_f32_norm(x: torch.Tensor, w: torch.Tensor, h: torch.Tensor, weight: tor
     _gpu(x, w, h, weight)
     _need(gemm_f32_norm_ok(x, w, h, weight), "gemm_f32_norm: h [M, N] and weight [N] float32, N a multiple of 8 up to 8,192")
     (M, K), N = x.shape, w.shape[0]
-    y, split = _f32_product(x, w, cut, "gemm_f32_norm")
+    # wide rows are a few loads in flight too many for a workgroup's registers, so the norm takes their sums of a few rows only (M, us with
+    # the sums added in the norm and by a kernel before it: 5,120 x 13,824 4: 74 and 89, 12: 88 and 82, 64: 124 and 119; 6,144 x 6,144 8: 48 and
+    # 51, 12: 58 and 55, 64: 73 and 70; 8,192 x 8,192 32: 95 and 90; 4,096 x 4,096 64: 36 and 38)
+    y, split = _f32_product(x, w, cut, "gemm_f32_norm", 0, N <= 4096 or M <= GEMM_F32_FEW_ROWS)
     out = torch.empty((M, N), dtype=torch.float32, device=x.device)
     if not split:
         return add_rmsnorm(h, y, weight, eps, out)
