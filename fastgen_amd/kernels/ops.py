@@ -1040,6 +1040,7 @@ GEMM_F32_GROUP = 1024
 # Up to this many rows the 32-bit product's kernel of 16 rows takes any size without scratch memory; the largest sums of
 # groups that other cuts put into memory, in bytes and in rows
 GEMM_F32_FEW_ROWS, GEMM_F32_MAX_SUMS, GEMM_F32_MAX_SPLIT_ROWS = 8, 256 << 20, 4096
+GEMM_F32_CUT_64_ROWS = 20 << 20  # numbers of the largest W whose 49 to 64 rows are multiplied cut beforehand
 
 
 def gemm_f32_plan(M: int, N: int, K: int, cus: int) -> Tuple[int, int, bool]:
@@ -1071,7 +1072,10 @@ def _f32_plan(M: int, N: int, K: int, cus: int, behind: bool, cut: bool) -> Tupl
     3,072 x 3,072 19.8 and 20.6, 4,096 x 14,336 61.0 and 62.8.
 
     ``cut``: tiles of operands cut into their parts beforehand, whose steps take 0.83 of the time and whose W is half as many bytes
-    again, and the kernel that cuts x (3 us; 4 bytes of an element read and 6 written)."""
+    again, and the kernel that cuts x (3 us; 4 bytes of an element read and 6 written).  Four blocks of rows of a large W keep the operands as
+    they are: their tiles hold two blocks and read W twice, or all four and wait for its bytes.  64 rows, us as they are and cut:
+    2,048 x 5,632 36.6 and 32.3, 4,096 x 4,096 37.5 and 36.2, 2,048 x 8,192 36.2 and 36.6; 11,264 x 2,048 45.9 and 49.2, 6,144 x 4,096 49.3 and
+    53.4, 3,072 x 8,192 49.0 and 54.7, 5,120 x 13,824 124 and 131; 72 rows of the last four 57.0 / 58.7 / 59.4 / 146 and 47.9 / 51.1 / 53.0 / 142."""
     if M <= GEMM_F32_FEW_ROWS and not behind:
         return 0.0, (0, 0, False)
     groups, blocks, streaming = -(-K // GEMM_F32_GROUP), -(-M // 16), N * K * (6 if cut else 4) / 5e6
@@ -1087,6 +1091,8 @@ def _f32_plan(M: int, N: int, K: int, cus: int, behind: bool, cut: bool) -> Tupl
         return best
     if cut:
         best = float("inf"), best[1]
+        if blocks == 4 and N * K > GEMM_F32_CUT_64_ROWS:
+            return best
     for waves, tallest in ((8, 7), (4, 5)):  # (what the registers hold)
         for b in range(1, tallest + 1):
             row_tiles = -(-blocks // b)
