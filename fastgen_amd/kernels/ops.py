@@ -766,11 +766,12 @@ _second: Dict[int, "torch.cuda.Stream"] = {}
 
 
 def _tiles_beside(n_workgroups: int) -> bool:
-    """Whether the tile kernel goes to the second stream.  Its two waits take the host 40 us a layer, which a step of short prompt
-    portions waits for: 32 requests decoding beside portions of 100 and 500 tokens, one stream and two, us: Buderax's layers
-    1,608 and 2,021, Gisodra's 8 requests 1,728 and 2,206, Llama 3B's 5,722 and 5,939.  From about a workgroup for every compute unit on (portions of 1,000 to
-    2,000 tokens) the two are level, 0.3 % for one stream to 0.8 % for two, and steps of more prompt tokens gain 1 %."""
-    return not _ONE_STREAM and 8 * n_workgroups >= 7 * compute_units()
+    """Whether the tile kernel goes to the second stream (pages that the one launch for both kinds does not take).  Its two waits take
+    the host 40 us a layer, which a step of few prompt tokens waits for.  Steps on pages of 32 tokens, us on one stream and on two, by
+    workgroups of the tile kernel: 136 (Buderax, portions of 100 and 500 beside 32) 1,795 and 2,123, 232 (Llama 3B, 1,200 beside 8) 5,097
+    and 5,205, 273 (Gisodra, 300 and 900 beside 8) 2,022 and 2,440, 490 to 510 2 % less on one to 0.7 % less on two, 764 (Buderax, 6,000
+    beside 32) 6,976 and 7,037, 1,000 (Llama 8B, 4,000 beside 64 of 2,000 to 6,000 tokens) 16,236 and 16,022, 2,000 level."""
+    return not _ONE_STREAM and 2 * n_workgroups >= 7 * compute_units()
 
 
 def _second_stream(device) -> "torch.cuda.Stream":
@@ -846,8 +847,8 @@ def paged_attention_mfma(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tens
     and ``window`` (made here if not given).  ``max_rows``: no small item has
     more rows (tokens times query heads per kv head) than this.  ``tile_rows``: the
     rows the big items were cut for (:func:`attention_tile_rows`; default: the larger form's).
-    With items of both kinds and pages of a multiple of 64 tokens one launch takes both; with other pages, and enough of the
-    big ones to fill the GPU, the tile kernel runs on a second stream beside
+    With items of both kinds and pages of a multiple of 64 tokens one launch takes both; with other pages, and many
+    of the big ones, the tile kernel runs on a second stream beside
     the split kernel and the current stream waits for it before this returns (not while a graph is captured, not with
     ``FG_ONE_STREAM=1``).  ``exact_weights``: the build of the kernels in which the softmax weights enter
     the product with the values as two bfloat16 terms (16 significant bits).  ``sinks`` and ``distance``: as

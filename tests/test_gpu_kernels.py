@@ -1222,7 +1222,8 @@ def test_paged_attention_mfma_keys_in_parts(ops, H, KV, hd, P, seqs, window, mos
 @pytest.mark.parametrize("P", [32, 64])
 def test_paged_attention_mfma_two_streams(ops, monkeypatch, P):
     """Prompt portions beside decoded tokens: the tile kernel runs on a second stream beside the
-    split kernel where one launch cannot take both (pages of 32 tokens).  The result is there when the caller's stream goes on (work queued behind the
+    split kernel where one launch cannot take both (pages of 32 tokens, and as if the step had many more items; pages of 64 stay on
+    the caller's stream).  The result is there when the caller's stream goes on (work queued behind the
     call, on a stream that is not the default one, sees every row), equals the one-stream result
     bit for bit, and a call while a graph is captured stays on the capturing stream."""
     import numpy as np
@@ -1244,6 +1245,9 @@ def test_paged_attention_mfma_two_streams(ops, monkeypatch, P):
     one = run(torch.full_like(case["q"], float("nan")))
     assert torch.allclose(one.cpu().float(), _plain_rows(case, seqs), atol=1.5e-2, rtol=2e-2)
     monkeypatch.setattr(ops, "_ONE_STREAM", False)
+    monkeypatch.setattr(ops, "_tiles_beside", lambda n_workgroups: not ops._ONE_STREAM)
+    beside, second = [], ops._second_stream
+    monkeypatch.setattr(ops, "_second_stream", lambda device: beside.append(device) or second(device))
     mine = torch.cuda.Stream(DEV)
     mine.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(mine):
@@ -1252,6 +1256,7 @@ def test_paged_attention_mfma_two_streams(ops, monkeypatch, P):
             copy = two.clone()  # queued on the caller's stream right behind the call
             mine.synchronize()
             assert torch.equal(copy, one)
+    assert len(beside) == (3 if P == 32 else 0)
     held = torch.empty_like(case["q"])
     g = torch.cuda.CUDAGraph()
     with torch.cuda.graph(g):
@@ -1261,6 +1266,7 @@ def test_paged_attention_mfma_two_streams(ops, monkeypatch, P):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(held, one)
+    assert len(beside) == (3 if P == 32 else 0)
 
 
 @pytest.mark.parametrize("cut", ["coarse", "pairs", "fine"])

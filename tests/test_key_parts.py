@@ -96,3 +96,11 @@ def test_a_cut_takes_the_host_less_than_the_items_do():
         return min(took)
 
     assert shortest(lambda: ops.cut_key_ranges(big, 4, 128, 0, 256)) < shortest(lambda: ops.attention_items(lens, starts, [0, 0], 4, 128))
+
+
+def test_a_second_stream_is_for_many_workgroups(monkeypatch):
+    """The waits between two streams cost what the kernels gain beside each other up to about three workgroups a unit."""
+    monkeypatch.setattr(ops, "compute_units", lambda: 256)
+    assert [ops._tiles_beside(n) for n in (1, 273, 512, 764, 1000, 2000)] == [False] * 4 + [True] * 2
+    monkeypatch.setattr(ops, "_ONE_STREAM", True)
+    assert not ops._tiles_beside(2000)
