@@ -1504,6 +1504,61 @@ def test_gemm_f32_with_what_is_behind_has_the_bits_of_both(ops, M, N, K):
         assert same(q[:, :H * hd], rows[:, :H * hd]) and same(pages[0], pages[2]) and same(pages[1], pages[3])
 
 
+@pytest.mark.parametrize("M,N,K", [(33, 1536, 4096), (300, 1040, 2048), (400, 5120, 3072), (112, 16384, 3072), (400, 3072, 1024)])
+def test_gemm_f32_of_cut_operands_with_what_is_behind_has_the_bits_of_both(ops, monkeypatch, M, N, K):
+    """What a prompt of a float32 model takes: operands cut beforehand, the groups' sums left to the activation, the norm or the
+    rotation behind (and a single group's product stored), against the product of the operands as they are and those kernels one
+    after the other: bit for bit, an output that comes out as no number computed again there too.  Whole groups and not, rows that
+    fill no block, and which entries were called."""
+    called = []
+
+    class Recorder:
+        def __init__(self, lib):
+            self.lib = lib
+
+        def __getattr__(self, name):
+            called.append(name)
+            return getattr(self.lib, name)
+
+    torch.manual_seed(N)
+    x, w = torch.randn(M, K, device=DEV), torch.randn(N, K, device=DEV)
+    x[M // 2, K - 1], w[5, 3] = float("inf"), 3.4e38  # (an infinity's parts' products, and what rounds to one in 16 bits)
+    same = lambda a, b: torch.equal(a[~b.isnan()], b[~b.isnan()]) and torch.equal(a.isnan(), b.isnan())
+    y, cut = ops.gemm_nt(x, w), ops.cut_weight(w)
+    silu, gelu = ops.silu_mul(y), ops.gelu_mul(y)
+    split = K > 1024
+    load = ops._lib.load
+    monkeypatch.setattr(ops._lib, "load", lambda name: Recorder(load(name)))
+
+    def by(*entries):
+        names = [n for n in called if n.startswith("fg_gemm_f32")]
+        called.clear()
+        assert names == ["fg_gemm_f32_cut", "fg_gemm_f32_parts", *(entries if split else ())], names
+
+    for epilogue, want in (("silu", silu), ("gelu_tanh", gelu)):
+        assert same(ops.gemm_f32_gated(x, w, epilogue, cut), want)
+        by("fg_gemm_f32_sum_act")
+    if N <= 8192:
+        h, weight = torch.randn(M, N, device=DEV), torch.randn(N, device=DEV)
+        h1, h2 = h.clone(), h.clone()
+        want = ops.add_rmsnorm(h2, y, weight, 1e-5, torch.empty_like(h))
+        assert same(ops.gemm_f32_norm(x, w, h1, weight, 1e-5, cut), want) and same(h1, h2)
+        by(*(["fg_gemm_f32_sum_norm"] if N <= 4096 else []))
+    hd, n_kv, P, rot = 16, 4, 16, 8
+    for from_key in (False, True):
+        H = N // hd - (1 if from_key else 2) * n_kv
+        pos = torch.arange(M, dtype=torch.int32, device=DEV) * 3
+        table = ops.rope_table(pos, torch.rand(rot // 2, device=DEV))
+        slots = torch.randperm(M + 20)[:M].to(torch.int32).to(DEV)
+        slots[M // 3] = -1
+        pages = [torch.full((M // P + 2, n_kv, *s), 7.0, device=DEV) for s in ((P, hd), (hd, P)) * 2]
+        q = ops.gemm_f32_qkv(x, w, table, pos, slots, *pages[:2], H, n_kv, hd, rot, from_key, cut)
+        by("fg_gemm_f32_sum_rope")
+        rows = y.clone()
+        ops.rope_kv_write(rows, pos, None, slots, *pages[2:], H, n_kv, hd, rot, table=table, v_col=H * hd if from_key else None)
+        assert same(q[:, :H * hd], rows[:, :H * hd]) and same(pages[0], pages[2]) and same(pages[1], pages[3])
+
+
 @pytest.mark.parametrize("M,N,K", [(17, 48, 128), (100, 1000, 1152), (112, 272, 2048), (113, 3072, 1024), (250, 515, 3072), (400, 2048, 256)])
 def test_gemm_f32_of_operands_cut_beforehand_has_the_same_bits(ops, M, N, K):
     """Every tile, with and without a workgroup a group of k, rows and outputs that fill none, against the operands as they are; infinities
