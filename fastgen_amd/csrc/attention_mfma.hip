@@ -1026,12 +1026,32 @@ struct KeyParts {
   const int* list;  // an item's two ints: its place among the parts (-1: the item is whole), part | parts << 16
   float *o, *ml;    // [place][kv head][8 blocks of 16 rows] x [NDB][64 lanes][4], x [64 lanes][2]
 };
+// Items of the smaller form whose even and odd tiles are added up apart and joined at the end, as the two waves of a row group of the
+// larger form do it (TWO): its bits.  Where each workgroup of the larger form had a unit to itself, the smaller ones, out of step with one
+// another, are the quicker way through few keys; one maximum a row instead of two leaves fewer weights that are 1 before
+// they are rounded, and an error against 64 bits that was 0.5 to 2.4 % the larger one in each of 24 cases.
+struct TwoSums {};
+// A row's (maximum, sum, O) and those of its odd tiles, in one (which product of two is rounded is said, not left to the compiler).
+template <class OTHER>
+__device__ __forceinline__ void join_sums(float& m, float& l, f32x4 (&o)[NDB], float mo, float lo, OTHER other) {
+  const float M = fmaxf(m, mo);
+  const float fs = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - M);
+  const float fo = mo == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mo - M);
+  l = fmaf(fs, l, fo * lo);
+  m = M;
+#pragma unroll
+  for (int db = 0; db < NDB; ++db) {
+    const f32x4 x = other(db);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[db][e] = fmaf(fo, x[e], fs * o[db][e]);
+  }
+}
 template <class A, class... B>
 __device__ __forceinline__ const A& the_one(const A& a, const B&...) { return a; }
 template <class A, class B, class... C, class = std::enable_if_t<!std::is_same_v<A, B>>>
 __device__ __forceinline__ const A& the_one(const B&, const C&... c) { return the_one<A>(c...); }
 
-template <int PAGES, bool TILE_PAIR, class... MORE /* SplitPart, KeyParts */>
+template <int PAGES, bool TILE_PAIR, class... MORE /* SplitPart, KeyParts, TwoSums */>
 __global__ __launch_bounds__(TILE_PAIR ? 512 : 256, TILE_PAIR ? 1 : 2) void attn_tile_kernel(
     const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, int out_stride,
     const bf16_t* __restrict__ k_pages, const bf16_t* __restrict__ v_pages,
@@ -1039,6 +1059,7 @@ __global__ __launch_bounds__(TILE_PAIR ? 512 : 256, TILE_PAIR ? 1 : 2) void attn
     int page_size, int page_shift, float scale, int window, const float* __restrict__ sinks,
     const float* __restrict__ dist, const OutGate gate, const MORE... more) {
   constexpr bool SPLIT = (std::is_same_v<MORE, SplitPart> || ...), KEYS = (std::is_same_v<MORE, KeyParts> || ...);
+  constexpr bool TWO = (std::is_same_v<MORE, TwoSums> || ...);
   constexpr bool PERM = PAGES >= PAGES_CHUNK, WHOLE = PAGES == PAGES_TILE;
   constexpr int TILE_RB = TILE_PAIR ? 2 : 1;  // row blocks a wave holds
   constexpr int TILE_THREADS = TILE_PAIR ? 512 : 256;
@@ -1127,15 +1148,25 @@ __global__ __launch_bounds__(TILE_PAIR ? 512 : 256, TILE_PAIR ? 1 : 2) void attn
     w_all_lo = max(w_all_lo, __shfl_xor(w_all_lo, msk, FG_WAVE));
   }
 
-  float m[RB], l[RB];
-  f32x4 o[RB][NDB];
+  struct Sums {
+    float m[RB], l[RB];
+    f32x4 o[RB][NDB];
+    __device__ __forceinline__ void clear() {
 #pragma unroll
-  for (int rb = 0; rb < RB; ++rb) {
-    m[rb] = -INFINITY;
-    l[rb] = 0.f;
+      for (int rb = 0; rb < RB; ++rb) {
+        m[rb] = -INFINITY;
+        l[rb] = 0.f;
 #pragma unroll
-    for (int db = 0; db < NDB; ++db) o[rb][db] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
+        for (int db = 0; db < NDB; ++db) o[rb][db] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+    }
+  };
+  Sums sums, odd;  // (odd: only with TWO)
+  sums.clear();
+  if (TWO) odd.clear();
+  auto& m = sums.m;
+  auto& l = sums.l;
+  auto& o = sums.o;
 
   const size_t head_elems = (size_t)page_size * HD;
   constexpr int KCH = HD / 8;                  // 16-byte chunks in a key
@@ -1221,7 +1252,7 @@ __global__ __launch_bounds__(TILE_PAIR ? 512 : 256, TILE_PAIR ? 1 : 2) void attn
     for (int j = 0; j < VN; ++j)
       if (threadIdx.x + NT * j < VTOT) *(bf16x8*)(v_lds[b] + (size_t)(threadIdx.x + NT * j) * 8) = vr[j];
   };
-  auto compute = [&](int k0, int b) {
+  auto compute = [&](int k0, int b, Sums& to) {
     if (k0 > w_hi || k0 + TILE <= w_lo) return;  // nothing in this tile for this wave's rows
     const bf16_t* k_s = k_lds[b];
     const bf16_t* v_s = v_lds[b];
@@ -1233,9 +1264,9 @@ __global__ __launch_bounds__(TILE_PAIR ? 512 : 256, TILE_PAIR ? 1 : 2) void attn
       return *(const bf16x8*)(v_s + ((db * 8 + 4 * ks + g) * 16 + r16) * 8);
     };
     if (k0 >= w_all_lo && k0 + TILE - 1 <= w_all_hi)  // uniform over the wave
-      attend_tile<false, RB, true>(k0, me, qop, scale * LOG2E, m, l, o, load_k, load_v);
+      attend_tile<false, RB, true>(k0, me, qop, scale * LOG2E, to.m, to.l, to.o, load_k, load_v);
     else
-      attend_tile<false, RB, false>(k0, me, qop, scale * LOG2E, m, l, o, load_k, load_v);
+      attend_tile<false, RB, false>(k0, me, qop, scale * LOG2E, to.m, to.l, to.o, load_k, load_v);
   };
   constexpr int STEP = NPT * TILE;  // keys per pass of the loop
   int k_first = (first_min / TILE) * TILE, k_last = pos_last, place = -1;
@@ -1296,7 +1327,7 @@ __global__ __launch_bounds__(TILE_PAIR ? 512 : 256, TILE_PAIR ? 1 : 2) void attn
       page_a = page_ahead(k0 + 2 * STEP);
       page_b = page_ahead(k0 + 2 * STEP + TILE);
       const int mine = k0 + par * TILE;
-      if (mine <= pos_last) compute(mine, s0 + par);
+      if (mine <= pos_last) compute(mine, s0 + par, sums);
     }
   } else {
     // one tile at a time: the next tile's chunks fly into registers during this tile's MFMAs
@@ -1304,13 +1335,24 @@ __global__ __launch_bounds__(TILE_PAIR ? 512 : 256, TILE_PAIR ? 1 : 2) void attn
     auto page_ahead = [&](int k0) { return WHOLE ? pager.page_of(min(k0, pos_last)) : 0; };
     int page = page_ahead(k_first + STEP);
     fetch(k_first, page_ahead(k_first), kreg, vreg);
-    for (int k0 = k_first; k0 <= pos_last; k0 += STEP) {
+    auto pass = [&](int k0, Sums& to) {
       __syncthreads();  // the previous tile is no longer read
       stash(0, kreg, vreg);
       __syncthreads();
       if (k0 + STEP <= pos_last) fetch(k0 + STEP, page, kreg, vreg);
       page = page_ahead(k0 + 2 * STEP);
-      compute(k0, 0);
+      compute(k0, 0, to);
+    };
+    for (int k0 = k_first; k0 <= pos_last; k0 += STEP) {
+      pass(k0, sums);
+      if constexpr (TWO) {
+        if ((k0 += STEP) <= pos_last) pass(k0, odd);  // uniform
+      }
+    }
+    if constexpr (TWO) {
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb)
+        join_sums(m[rb], l[rb], o[rb], odd.m[rb], odd.l[rb], [&](int db) { return odd.o[rb][db]; });
     }
   }
   if (TILE_PAIR) {
@@ -1330,16 +1372,8 @@ __global__ __launch_bounds__(TILE_PAIR ? 512 : 256, TILE_PAIR ? 1 : 2) void attn
       __syncthreads();
       if (par == 0) {
         const float mo = ml_x[(rg * FG_WAVE + lane) * 2], lo = ml_x[(rg * FG_WAVE + lane) * 2 + 1];
-        const float M = fmaxf(m[rb], mo);
-        const float fs = m[rb] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m[rb] - M);
-        const float fo = mo == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mo - M);
-        l[rb] = fs * l[rb] + fo * lo;
-        m[rb] = M;
-#pragma unroll
-        for (int db = 0; db < NDB; ++db) {
-          const f32x4 other = *(const f32x4*)(o_x + ((size_t)(rg * NDB + db) * FG_WAVE + lane) * 4);
-          o[rb][db] = fs * o[rb][db] + fo * other;
-        }
+        join_sums(m[rb], l[rb], o[rb], mo, lo,
+                  [&](int db) { return *(const f32x4*)(o_x + ((size_t)(rg * NDB + db) * FG_WAVE + lane) * 4); });
       }
     }
     if (par == 1) return;
@@ -1514,6 +1548,7 @@ struct TileArgs {
 };
 template <bool PAIR> static int more_groups(const TileArgs& a, const SplitPart& s) { return a.n_kv * ((s.max_chunks + (PAIR ? 1 : 0)) / (PAIR ? 2 : 1)); }
 template <bool PAIR> static int more_groups(const TileArgs&, const KeyParts&) { return 0; }
+template <bool PAIR> static int more_groups(const TileArgs&, const TwoSums&) { return 0; }
 template <int PAGES, bool PAIR, class... MORE>
 static void launch_pages(const TileArgs& a, MORE... more) {
   const int groups = (more_groups<PAIR>(a, more) + ... + (a.n_items * a.n_kv));
@@ -1531,10 +1566,12 @@ static void launch_tile(const TileArgs& a) {
 template <bool EXISTS> struct PairForm {
   static void go(const TileArgs& a) { launch_tile<true>(a); }
   template <class... MORE> static void more(const TileArgs& a, MORE... m) { launch_pages<PAGES_TILE, true>(a, m...); }
+  template <class... MORE> static void two(const TileArgs& a, MORE... m) { launch_pages<PAGES_TILE, false>(a, m..., TwoSums{}); }
 };
 template <> struct PairForm<false> {
   static void go(const TileArgs&) {}
   template <class... MORE> static void more(const TileArgs&, MORE...) {}
+  template <class... MORE> static void two(const TileArgs&, MORE...) {}
 };
 static bool tile_args_ok(const TileArgs& a, int item_rows) {
   return DIST_BIAS == (a.dist != nullptr) && gate_ok(a.gate.g, a.gate.stride, a.n_heads) && a.scale > 0.f && a.n_kv > 0 &&
@@ -1546,15 +1583,19 @@ static bool key_parts_ok(const TileArgs& a, int item_rows, const KeyParts& keys,
   return TILE_PAIR_OK && item_rows == TILE_ROWS && a.page_size % 64 == 0 && keys.list && keys.o && keys.ml && merges &&
          (long long)n_merges * a.n_kv <= 1073741823LL;
 }
+static bool two_sums_ok(const TileArgs& a, int item_rows, int n_merges) {
+  return TILE_PAIR_OK && item_rows == TILE_ROWS_SMALL && a.page_size % 64 == 0 && n_merges <= 0;
+}
 static void launch_merges(const TileArgs& a, const KeyParts& keys, const int* merges, int n_merges) {
   attn_parts_kernel<<<2 * n_merges * a.n_kv, 256, 0, a.stream>>>(keys, merges, a.out, a.out_stride, a.n_heads, a.n_kv, a.sinks, a.gate);
 }
 
 // item_rows: the rows an item has at most, fg_attn_tile_rows(0) or fg_attn_tile_rows(1): which form of the kernel runs.
+// two_sums: items of the smaller form, added up as the larger one does it (head sizes up to 128, pages of a multiple of 64 tokens).
 // key_list, merges, n_merges, key_o, key_ml: the items are parts of keys (see KeyParts and attn_parts_kernel); n_merges 0: they are whole.
 extern "C" int fg_attn_tile_sink(const void* q, int q_stride, void* out, int out_stride, const void* k_pages,
                                  const void* v_pages, const int* block_table, int bt_stride, const int* items,
-                                 int n_items, int item_rows, int n_heads, int n_kv, int hd, int page_size,
+                                 int n_items, int item_rows, int two_sums, int n_heads, int n_kv, int hd, int page_size,
                                  float scale, int window, const float* sinks, const float* dist, const void* gate,
                                  int gate_stride, int gate_sigmoid, const int* key_list, const int* merges, int n_merges,
                                  float* key_o, float* key_ml, hipStream_t stream) {
@@ -1562,9 +1603,11 @@ extern "C" int fg_attn_tile_sink(const void* q, int q_stride, void* out, int out
   const TileArgs a{(const bf16_t*)q, q_stride, (bf16_t*)out, out_stride, (const bf16_t*)k_pages, (const bf16_t*)v_pages,
                    block_table, bt_stride, items, n_items, n_heads, n_kv, page_size, scale, window, sinks, dist,
                    OutGate{(const bf16_t*)gate, gate_stride, gate_sigmoid}, stream};
-  if (hd != HD || !tile_args_ok(a, item_rows)) return FG_ERR_ARG;
+  if (hd != HD || !tile_args_ok(a, item_rows) || (two_sums && !two_sums_ok(a, item_rows, n_merges))) return FG_ERR_ARG;
   const KeyParts keys{key_list, key_o, key_ml};
-  if (n_merges > 0) {
+  if (two_sums) {
+    PairForm<TILE_PAIR_OK>::two(a);
+  } else if (n_merges > 0) {
     if (!key_parts_ok(a, item_rows, keys, merges, n_merges)) return FG_ERR_ARG;
     PairForm<TILE_PAIR_OK>::more(a, keys);
     launch_merges(a, keys, merges, n_merges);
@@ -1577,7 +1620,7 @@ extern "C" int fg_attn_tile_sink(const void* q, int q_stride, void* out, int out
 // pages of a multiple of 64 tokens.
 extern "C" int fg_attn_both(const void* q, int q_stride, void* out, int out_stride, const void* k_pages, const void* v_pages,
                             const int* block_table, int bt_stride, const int* plan, int n_small, int max_chunks, int max_rows,
-                            float* part_o, float* part_ml, const int* items, int n_items, int item_rows, int n_heads, int n_kv,
+                            float* part_o, float* part_ml, const int* items, int n_items, int item_rows, int two_sums, int n_heads, int n_kv,
                             int hd, int page_size, float scale, int window, const float* sinks, const float* dist,
                             const void* gate, int gate_stride, int gate_sigmoid, int ordered, const int* key_list, const int* merges,
                             int n_merges, float* key_o, float* key_ml, hipStream_t stream) {
@@ -1586,11 +1629,13 @@ extern "C" int fg_attn_both(const void* q, int q_stride, void* out, int out_stri
                    OutGate{(const bf16_t*)gate, gate_stride, gate_sigmoid}, stream};
   if (hd != HD || !tile_args_ok(a, item_rows) || page_size % 64 || n_items <= 0 || n_small <= 0 || n_heads / n_kv > 16 ||
       max_chunks < 2 * n_small || max_chunks > 65535 || n_kv > 65535 || !plan || !part_o || !part_ml || max_rows < 1 ||
-      max_rows > 16 || ((long long)n_items + max_chunks) * n_kv > 2147483647LL)
+      max_rows > 16 || ((long long)n_items + max_chunks) * n_kv > 2147483647LL || (two_sums && !two_sums_ok(a, item_rows, n_merges)))
     return FG_ERR_ARG;
   const SplitPart split{plan + PLAN_HEAD + (ordered ? 8LL * max_chunks : 0), part_o, part_ml, max_chunks, ordered, n_items * n_kv};
   const KeyParts keys{key_list, key_o, key_ml};
-  if (n_merges > 0) {
+  if (two_sums) {
+    PairForm<TILE_PAIR_OK>::two(a, split);
+  } else if (n_merges > 0) {
     if (!key_parts_ok(a, item_rows, keys, merges, n_merges)) return FG_ERR_ARG;
     PairForm<TILE_PAIR_OK>::more(a, split, keys);
     launch_merges(a, keys, merges, n_merges);
@@ -1605,7 +1650,7 @@ extern "C" int fg_attn_tile(const void* q, int q_stride, void* out, int out_stri
                             int n_items, int item_rows, int n_heads, int n_kv, int hd, int page_size, float scale,
                             int window, hipStream_t stream) {
   return fg_attn_tile_sink(q, q_stride, out, out_stride, k_pages, v_pages, block_table, bt_stride, items, n_items,
-                           item_rows, n_heads, n_kv, hd, page_size, scale, window, nullptr, nullptr, nullptr, 0, 0, nullptr, nullptr, 0, nullptr, nullptr, stream);
+                           item_rows, 0, n_heads, n_kv, hd, page_size, scale, window, nullptr, nullptr, nullptr, 0, 0, nullptr, nullptr, 0, nullptr, nullptr, stream);
 }
 
 // query rows (tokens x heads of a kv head's group) of one item of fg_attn_tile: of the larger form, or

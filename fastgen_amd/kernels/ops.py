@@ -709,6 +709,20 @@ def cut_key_ranges(big: np.ndarray, n_kv: int, head_dim: int, window: int, cus: 
             out[at_merges : at_merges + 4 * n_merges].reshape(-1, 4), n_places)
 
 
+SHORT_ITEMS_MAX_PASSES = 10
+
+
+def _short_items(big: np.ndarray, n_kv: int) -> bool:
+    """Whether a step's items (of the larger form, more than half a workgroup a unit) are few and short enough to go as items of 64 rows
+    with two sums: the same bits in less time up to five workgroups for four units.  Heads of 128, us with items of 128 rows and of 64 by
+    workgroups: 192 (6 passes of 128 keys) 23.5 and 21.7, 240 (10) 33.4 and 31.1, 256 (8; 4; 2) 28.4 and 27.6; 19.1 and 17.2; 14.1 and 11.8, 288 (9)
+    30.9 and 30.3, 320 (10; 5) 33.3 and 33.1; 22.6 and 20.0, 352 (11; 6) 35.7 and 35.8; 25.0 and 23.8, 384 (12; 6) 38.2 and 40.4; 27.3 and 26.3, 448
+    (7) 32.5 and 33.7, 512 (8; 4) 37.5 and 40.9; 28.0 and 27.3.  Beside 24 and 64 decoding requests 248 (7) 40.7 and 35.6, 320 (10) 66.3 and
+    64.2; beside 12 of 4 kv heads 240 (10) 37.5 and 39.6."""
+    most_keys = int(big[0, 3]) + int(big[0, 2])  # (the longest stands first)
+    return most_keys <= 128 * SHORT_ITEMS_MAX_PASSES and 4 * len(big) * n_kv <= 5 * compute_units()
+
+
 def upload_key_parts(cut, device, before: Optional[np.ndarray] = None):
     """:class:`KeyParts` of a cut on the device; with ``before``, other items, ``(them, KeyParts)``, in one copy."""
     items, parts, merges, n_places = cut
@@ -839,7 +853,7 @@ def paged_attention_mfma(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tens
                          exact_weights: bool = False, sinks: Optional[torch.Tensor] = None,
                          distance: Optional[torch.Tensor] = None, gate: Optional[torch.Tensor] = None,
                          gate_sigmoid: bool = True, leave_parts: bool = False,
-                         key_parts: Optional[KeyParts] = None) -> "torch.Tensor | AttentionParts":
+                         key_parts: Optional[KeyParts] = None, two_sums: bool = False) -> "torch.Tensor | AttentionParts":
     """bf16 attention on the matrix cores.  ``small_items`` / ``big_items`` are
     device int32 ``[n, 4]`` lists from :func:`attention_items` (16-byte aligned);
     every query token of the step must be covered by exactly one item.
@@ -856,14 +870,16 @@ def paged_attention_mfma(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tens
     ``gate_sigmoid``: what :func:`gate_mul` does with them behind the attention, done where the output is stored (the
     same bits), for bfloat16 rows that can be read in fours; else by that kernel.  ``leave_parts``: one token without a
     gate comes as :class:`AttentionParts` where :func:`attention_parts_fit` the cache's pages.  ``key_parts``: the big items, of the
-    larger form and pages of a multiple of 64 tokens, with their keys cut (:func:`cut_key_ranges`)."""
+    larger form and pages of a multiple of 64 tokens, with their keys cut (:func:`cut_key_ranges`).  ``two_sums``: big items of the
+    smaller form (head sizes up to 128, pages of a multiple of 64 tokens) are added up as the larger form does it, and have its bits
+    where no window hides keys."""
     leave_parts = (leave_parts and gate is None and (big_items is None or not big_items.numel()) and attention_parts_fit(
         q.shape[0], n_heads, k_pages.shape[3], k_pages.shape[1], block_table.shape[1] * k_pages.shape[2]))
     _gpu(q, out, k_pages, v_pages, block_table, small_items, big_items, plan, sinks, distance, gate)
     if gate is not None and (gate.dtype != torch.bfloat16 or gate.data_ptr() % 8 or gate.stride(0) % 4):
         return gate_mul(paged_attention_mfma(q, out, k_pages, v_pages, block_table, small_items, big_items, n_heads, scale,
                                              window, plan, max_chunks, min_tiles, max_rows, tile_rows, exact_weights, sinks,
-                                             distance, key_parts=key_parts), gate, gate_sigmoid)
+                                             distance, key_parts=key_parts, two_sums=two_sums), gate, gate_sigmoid)
     _need(gate is None or (gate.dim() == 2 and gate.shape[0] == q.shape[0] and gate.shape[1] >= out.shape[1]
                            and gate.stride(1) == 1), "gate must be [T, >= H*hd] with unit column stride")
     gate_args = (_ptr(gate), gate.stride(0) if gate is not None else 0, int(gate_sigmoid))
@@ -927,6 +943,8 @@ def paged_attention_mfma(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tens
         _need(G <= tile_rows, "too many query heads per kv head for the tile kernel")
         _i32(big_items, "big_items")
         _need(big_items.data_ptr() % 16 == 0, "items must be 16-byte aligned")
+        _need(not two_sums or (tile_rows < attention_tile_rows(hd, False, exact_weights, dist) and page_size % 64 == 0 and key_parts is None),
+              "two sums are for whole items of the smaller form, and pages of a multiple of 64 tokens")
         key_args = (0, 0, 0, 0, 0)
         n_items = big_items.numel() // 4
         if key_parts is not None:
@@ -947,13 +965,13 @@ def paged_attention_mfma(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tens
             st = lib.fg_attn_both(
                 _ptr(q), q.stride(0), _ptr(out), out.stride(0), _ptr(k_pages), _ptr(v_pages), _ptr(block_table),
                 block_table.stride(0), _ptr(plan), n, max_chunks, max_rows, _ptr(part_o), _ptr(part_ml), _ptr(big_items),
-                n_items, tile_rows, n_heads, n_kv, hd, page_size, float(scale), int(window or 0), _ptr(sinks),
+                n_items, tile_rows, int(two_sums), n_heads, n_kv, hd, page_size, float(scale), int(window or 0), _ptr(sinks),
                 _ptr(distance), *gate_args, int(ordered), *key_args, _stream(q))
             _check(st, "attn_both")
             return out
         st = lib.fg_attn_tile_sink(
             _ptr(q), q.stride(0), _ptr(out), out.stride(0), _ptr(k_pages), _ptr(v_pages), _ptr(block_table),
-            block_table.stride(0), _ptr(big_items), n_items, tile_rows, n_heads, n_kv, hd, page_size,
+            block_table.stride(0), _ptr(big_items), n_items, tile_rows, int(two_sums), n_heads, n_kv, hd, page_size,
             float(scale), int(window or 0), _ptr(sinks), _ptr(distance), *gate_args, *key_args,
             beside.cuda_stream if beside else _stream(q))
         _check(st, "attn_tile")
@@ -993,21 +1011,21 @@ def paged_attention(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v
         if ctx.seq_records is not None and int(ctx.q_lens.max()) * G <= 16:
             # every sequence is one item of the split kernel: its records are in the step's buffer
             # already (and are refreshed with it when the step is a replayed graph)
-            plan = (ctx.seq_records, None, ctx.n_seqs, None, min(16, G * int(ctx.q_lens.max())), None)
+            plan = (ctx.seq_records, None, ctx.n_seqs, None, min(16, G * int(ctx.q_lens.max())), None, False)
         else:
             tile_rows = attention_tile_rows(hd, False, exact_weights, dist)
             small, big = attention_items(ctx.q_lens, ctx.q_start_host, ctx.n_cached, G, tile_rows)
-            cut = None
+            cut, two_sums = None, False
             if len(big) and attention_tile_rows(hd, True, exact_weights, dist) < tile_rows:
                 cut = None if k_pages.shape[2] % 64 else cut_key_ranges(big, n_kv, hd, span, compute_units(), None, exact_weights, dist)
-                if cut is None and len(big) * n_kv <= compute_units() // 2:
+                if cut is None:
                     # so few items that half the compute units would stand idle: items of half the rows, whose lighter workgroups
-                    # share a unit (512 tokens of 32 heads on 8, us with items of 128 and of 64 rows: 17.5 and 14.8).  They are the
-                    # quicker ones for short key ranges beyond that too (768 tokens 24.2 and 21.8, 1,024 28.3 and 26.7), but an item of
-                    # 128 rows has two maxima a row and so more weights that are 1 before they are rounded: its error against 64 bits
-                    # is the smaller one by 0.5 to 2.4 % in each of 24 cases, and a prompt keeps it
-                    tile_rows = attention_tile_rows(hd, True, exact_weights, dist)
-                    small, big = attention_items(ctx.q_lens, ctx.q_start_host, ctx.n_cached, G, tile_rows)
+                    # share a unit (512 tokens of 32 heads on 8, us with items of 128 and of 64 rows: 17.5 and 14.8)
+                    half = len(big) * n_kv <= compute_units() // 2
+                    two_sums = not half and k_pages.shape[2] % 64 == 0 and span == 0 and _short_items(big, n_kv)
+                    if half or two_sums:
+                        tile_rows = attention_tile_rows(hd, True, exact_weights, dist)
+                        small, big = attention_items(ctx.q_lens, ctx.q_start_host, ctx.n_cached, G, tile_rows)
             if cut is not None:
                 small_d, key_parts = upload_key_parts(cut, q.device, small)
                 big_d = key_parts.items
@@ -1015,9 +1033,9 @@ def paged_attention(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v
                 small_d, big_d = upload(np.concatenate([small, big]).reshape(-1), torch.int32, q.device).split([small.size, big.size])
                 key_parts = None
             plan = (small_d if small.size else None, big_d if big.size else None, len(small),
-                    tile_rows, max((int(n) * G for n in ctx.q_lens if n * G <= 16), default=16), key_parts)
+                    tile_rows, max((int(n) * G for n in ctx.q_lens if n * G <= 16), default=16), key_parts, two_sums)
         ctx.scratch[items_key] = plan
-    small_d, big_d, n_small, tile_rows, max_rows, key_parts = plan  # rows of the largest small item: one token a sequence in a decode step
+    small_d, big_d, n_small, tile_rows, max_rows, key_parts, two_sums = plan  # rows of the largest small item: one token a sequence in a decode step
     chunks = split_plan = None
     if n_small:
         # how the items' key ranges are cut depends on the window: layers with the same one share the cut
@@ -1030,7 +1048,7 @@ def paged_attention(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v
     return paged_attention_mfma(q, out, k_pages, v_pages, group.block_table, small_d, big_d, n_heads, scale,
                                 window, split_plan, chunks, max_rows=max_rows, tile_rows=tile_rows,
                                 exact_weights=exact_weights, sinks=sinks, distance=distance, gate=gate,
-                                gate_sigmoid=gate_sigmoid, leave_parts=leave_parts, key_parts=key_parts)
+                                gate_sigmoid=gate_sigmoid, leave_parts=leave_parts, key_parts=key_parts, two_sums=two_sums)
 
 
 # ----------------------------------------------------------------------- gemm

@@ -259,7 +259,7 @@ def paged_attention_mfma(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tens
                          tile_rows=None, exact_weights: bool = False,
                          sinks: Optional[torch.Tensor] = None,
                          distance: Optional[torch.Tensor] = None, gate: Optional[torch.Tensor] = None,
-                         gate_sigmoid: bool = True, leave_parts: bool = False, key_parts=None) -> torch.Tensor:
+                         gate_sigmoid: bool = True, leave_parts: bool = False, key_parts=None, two_sums: bool = False) -> torch.Tensor:
     """The same attention for tokens listed as items (sequence, first flat token, tokens, position of the
     first token).  How the kernels cut the work (``plan`` and what follows it) does not change the result;
     ``exact_weights`` only says how many digits of the softmax weights the kernel keeps (here: all)."""

@@ -31,8 +31,8 @@ def test_launch_for_both_kinds_keeps_a_units_workgroups(hipcc, tmp_path, head_di
     for name, body in re.findall(r"^(_Z\d+attn_tile_kernel\w+):(.*?^; Occupancy: \d+)", (tmp_path / "listing").read_text(), re.S | re.M):
         pages, pair, both = re.match(r"_Z\d+attn_tile_kernelILi(\d)ELb(\d)EJ(.*?)EE", name).groups()
         lds, waves = re.search(r"\.amdhsa_group_segment_fixed_size (\d+)", body), re.search(r"; Occupancy: (\d+)", body)
-        held[pages, pair, "SplitPart" in both, "KeyParts" in both] = int(lds[1]), int(waves[1])
+        held[pages, pair, "SplitPart" in both, "KeyParts" in both, "TwoSums" in both] = int(lds[1]), int(waves[1])
     forms = [f for f in held if f[2]]
-    assert len(forms) == (3 if head_dim <= 128 else 1)
-    for pages, pair, _, parts in forms:
-        assert held[pages, pair, True, parts] == held[pages, pair, False, parts], (pages, pair, parts)
+    assert len(forms) == (4 if head_dim <= 128 else 1)
+    for pages, pair, _, *more in forms:
+        assert held[(pages, pair, True, *more)] == held[(pages, pair, False, *more)], (pages, pair, more)

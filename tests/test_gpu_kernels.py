@@ -1219,6 +1219,36 @@ def test_paged_attention_mfma_keys_in_parts(ops, H, KV, hd, P, seqs, window, mos
         assert torch.allclose(parts.cpu().float(), _plain_rows(case, seqs, window or None), atol=1.5e-2, rtol=2e-2)
 
 
+@pytest.mark.parametrize("H,KV,hd,P,seqs", [(16, 4, 128, 64, [(0, 64)]), (32, 8, 128, 64, [(0, 700), (65, 130)]), (6, 2, 64, 128, [(5, 1300), (70, 33)]),
+                                             (5, 5, 16, 192, [(1000, 129), (0, 65)]), (8, 1, 80, 64, [(700, 21), (64, 64), (0, 128)])])
+@pytest.mark.parametrize("n_decode", [0, 3])
+@pytest.mark.parametrize("build", ["plain", "gate", "exact", "distance"])
+def test_paged_attention_mfma_two_sums_have_the_larger_forms_bits(ops, H, KV, hd, P, seqs, n_decode, build):
+    """Items of 64 rows whose even and odd tiles are added up apart, alone and beside decoded tokens: the bits of items of 128 rows for one
+    tile, for an odd and an even number of them and where a page holds several, whatever the outputs go through."""
+    import numpy as np
+
+    seqs = [(37 + 400 * i, 1) for i in range(n_decode)] + seqs
+    case = _paged_case(torch.bfloat16, seqs, H, KV, hd, P, seed=47)
+    q_lens = [b for _, b in seqs]
+    gate = torch.randn(len(case["q"]), H * hd, device=DEV).bfloat16() if build == "gate" else None
+    sinks = torch.randn(H, device=DEV) if build == "gate" else None
+    distance = torch.rand(H, 2, device=DEV) if build == "distance" else None
+
+    def run(rows_small, two):
+        rows = ops.attention_tile_rows(hd, rows_small)
+        small, big = ops.attention_items(q_lens, np.concatenate([[0], np.cumsum(q_lens)]), [a for a, _ in seqs], H // KV, rows)
+        assert len(big) and len(small) >= n_decode
+        small, big = (torch.from_numpy(a.reshape(-1)).to(DEV) if a.size else None for a in (small, big))
+        return ops.paged_attention_mfma(case["q"], torch.full_like(case["q"][:, : H * hd], float("nan")), case["kp"], case["vp"], case["table"],
+                                        small, big, H, hd ** -0.5, tile_rows=rows, exact_weights=build in ("exact", "distance"), sinks=sinks,
+                                        distance=distance, gate=gate, two_sums=two)
+    whole = run(False, False)
+    assert torch.isfinite(whole).all() and torch.equal(run(True, True), whole)
+    with pytest.raises(ops.KernelArgumentError):
+        run(False, True)
+
+
 @pytest.mark.parametrize("P", [32, 64])
 def test_paged_attention_mfma_two_streams(ops, monkeypatch, P):
     """Prompt portions beside decoded tokens: the tile kernel runs on a second stream beside the

@@ -54,11 +54,15 @@ def test_what_is_cut():
     assert ops.cut_key_ranges(np.zeros((0, 4), np.int32), 8, 128, 0, 256) is None
 
 
-@pytest.mark.parametrize("lens,heads,n_kv,rows", [([300], 32, 8, 64), ([512], 32, 8, 64), ([513], 32, 8, 128), ([380, 874], 24, 8, 128), ([1024], 32, 8, 128),
-                                                   ([680] * 3, 16, 4, 128), ([256] * 8, 16, 4, 128), ([2048], 32, 8, 128)])
-def test_prompts_keep_the_more_precise_items(monkeypatch, lens, heads, n_kv, rows):
-    """Items of 64 rows are for steps that leave half of 256 units idle; from there on the form of 128 rows, whose error against 64
-    bits is the smaller one, takes a prompt's rows."""
+@pytest.mark.parametrize("lens,heads,n_kv,rows,two,more", [
+    ([300], 32, 8, 64, False, {}), ([512], 32, 8, 64, False, {}), ([513], 32, 8, 64, True, {}), ([380, 874], 24, 8, 64, True, {}),
+    ([1280], 32, 8, 64, True, {}), ([1281], 32, 8, 128, False, {}), ([640] * 4, 16, 4, 64, True, {}), ([641] * 4, 16, 4, 128, False, {}),
+    ([2048], 32, 8, 128, False, {}), ([1024], 32, 8, 128, False, dict(window=300)), ([1024], 32, 8, 64, True, dict(window=4096)),
+    ([1024], 32, 8, 128, False, dict(page=32)), ([512], 32, 8, 64, False, dict(page=32)), ([1024], 32, 8, 128, False, dict(window=-64))])
+def test_which_items_a_prompt_gets(monkeypatch, lens, heads, n_kv, rows, two, more):
+    """Items of 64 rows where half of 256 units would stand idle, and, added up as the larger form does it, up to five workgroups for four
+    units and ten passes; from there on, where a window hides keys and on small pages the form of 128 rows, whose error against
+    64 bits is smaller than that of 64 rows with one sum."""
     from types import SimpleNamespace
 
     import torch
@@ -67,14 +71,14 @@ def test_prompts_keep_the_more_precise_items(monkeypatch, lens, heads, n_kv, row
     monkeypatch.setattr(ops, "compute_units", lambda: 256)
     monkeypatch.setattr(ops, "attention_tile_rows", lambda hd, small=False, exact=False, dist=False: 64 if small else 128)
     monkeypatch.setattr(ops, "upload", lambda values, dtype, device: torch.as_tensor(values))
-    monkeypatch.setattr(ops, "paged_attention_mfma", lambda *a, tile_rows, key_parts, **k: seen.append((a[6], tile_rows, key_parts)))
+    monkeypatch.setattr(ops, "paged_attention_mfma", lambda *a, tile_rows, key_parts, two_sums, **k: seen.append((a[6], tile_rows, key_parts, two_sums)))
     starts = np.concatenate([[0], np.cumsum(lens)])
     ctx = SimpleNamespace(q_lens=np.array(lens), n_cached=np.zeros(len(lens), int), q_start_host=starts, seq_records=None, scratch={})
     q = torch.empty(1, heads * 128, dtype=torch.bfloat16)
-    pages = torch.empty(1, n_kv, 64, 128, dtype=torch.bfloat16)
-    ops.paged_attention(q, q, pages, pages, SimpleNamespace(block_table=None), ctx, heads, 1.0)
-    (items, got, parts), = seen
-    assert got == rows and parts is None
+    pages = torch.empty(1, n_kv, more.get("page", 64), 128, dtype=torch.bfloat16)
+    ops.paged_attention(q, q, pages, pages, SimpleNamespace(block_table=None), ctx, heads, 1.0, more.get("window", 0))
+    (items, got, parts, sums), = seen
+    assert got == rows and parts is None and bool(sums) == two
     assert int(items.view(-1, 4)[:, 2].max()) <= rows // (heads // n_kv)
 
 
