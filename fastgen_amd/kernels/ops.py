@@ -709,18 +709,28 @@ def cut_key_ranges(big: np.ndarray, n_kv: int, head_dim: int, window: int, cus: 
             out[at_merges : at_merges + 4 * n_merges].reshape(-1, 4), n_places)
 
 
-SHORT_ITEMS_MAX_PASSES = 10
+SHORT_ITEMS_MAX_PASSES = 10  # (of 128 keys; longer items are what fg_attn_cut_keys considers)
 
 
-def _short_items(big: np.ndarray, n_kv: int) -> bool:
-    """Whether a step's items (of the larger form, more than half a workgroup a unit) are few and short enough to go as items of 64 rows
-    with two sums: the same bits in less time up to five workgroups for four units.  Heads of 128, us with items of 128 rows and of 64 by
+def _prompt_groups(q_lens, n_cached, group_size: int, tile_rows: int, n_kv: int) -> Tuple[int, int]:
+    """The workgroups that a step's items of so many rows take, and the most keys of one, without listing them (a step on new inputs
+    waits for each list, 50 us for prompts of 611 and 1,437 tokens)."""
+    per_tile, items, most_keys = max(1, tile_rows // group_size), 0, 0
+    for n, c in zip(q_lens.tolist(), n_cached.tolist()):
+        if n * group_size > 16:
+            items += -(-n // per_tile)
+            most_keys = max(most_keys, n + c)
+    return items * n_kv, most_keys
+
+
+def _few_short_items(groups: int) -> bool:
+    """Whether a step's short items (so many workgroups of the larger form, more than half a unit's worth) are few enough to go as items
+    of 64 rows with two sums: the same bits in less time up to five workgroups for four units.  Heads of 128, us with items of 128 rows and of 64 by
     workgroups: 192 (6 passes of 128 keys) 23.5 and 21.7, 240 (10) 33.4 and 31.1, 256 (8; 4; 2) 28.4 and 27.6; 19.1 and 17.2; 14.1 and 11.8, 288 (9)
     30.9 and 30.3, 320 (10; 5) 33.3 and 33.1; 22.6 and 20.0, 352 (11; 6) 35.7 and 35.8; 25.0 and 23.8, 384 (12; 6) 38.2 and 40.4; 27.3 and 26.3, 448
     (7) 32.5 and 33.7, 512 (8; 4) 37.5 and 40.9; 28.0 and 27.3.  Beside 24 and 64 decoding requests 248 (7) 40.7 and 35.6, 320 (10) 66.3 and
     64.2; beside 12 of 4 kv heads 240 (10) 37.5 and 39.6."""
-    most_keys = int(big[0, 3]) + int(big[0, 2])  # (the longest stands first)
-    return most_keys <= 128 * SHORT_ITEMS_MAX_PASSES and 4 * len(big) * n_kv <= 5 * compute_units()
+    return 4 * groups <= 5 * compute_units()
 
 
 def upload_key_parts(cut, device, before: Optional[np.ndarray] = None):
@@ -1013,19 +1023,21 @@ def paged_attention(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v
             # already (and are refreshed with it when the step is a replayed graph)
             plan = (ctx.seq_records, None, ctx.n_seqs, None, min(16, G * int(ctx.q_lens.max())), None, False)
         else:
-            tile_rows = attention_tile_rows(hd, False, exact_weights, dist)
+            tile_rows, small_rows = (attention_tile_rows(hd, small, exact_weights, dist) for small in (False, True))
+            cut, two_sums, whole_pages = None, False, k_pages.shape[2] % 64 == 0
+            groups, most_keys = _prompt_groups(ctx.q_lens, ctx.n_cached, G, tile_rows, n_kv)
+            # so few items that half the compute units would stand idle: items of half the rows, whose lighter workgroups share a
+            # unit (512 tokens of 32 heads on 8, us with items of 128 and of 64 rows: 17.5 and 14.8)
+            half = 0 < groups <= compute_units() // 2 and small_rows < tile_rows
+            if 0 < groups and most_keys <= 128 * SHORT_ITEMS_MAX_PASSES:  # (no cut of the keys, so the items are listed once)
+                two_sums = not half and small_rows < tile_rows and whole_pages and span == 0 and _few_short_items(groups)
+                tile_rows = small_rows if half or two_sums else tile_rows
             small, big = attention_items(ctx.q_lens, ctx.q_start_host, ctx.n_cached, G, tile_rows)
-            cut, two_sums = None, False
-            if len(big) and attention_tile_rows(hd, True, exact_weights, dist) < tile_rows:
-                cut = None if k_pages.shape[2] % 64 else cut_key_ranges(big, n_kv, hd, span, compute_units(), None, exact_weights, dist)
-                if cut is None:
-                    # so few items that half the compute units would stand idle: items of half the rows, whose lighter workgroups
-                    # share a unit (512 tokens of 32 heads on 8, us with items of 128 and of 64 rows: 17.5 and 14.8)
-                    half = len(big) * n_kv <= compute_units() // 2
-                    two_sums = not half and k_pages.shape[2] % 64 == 0 and span == 0 and _short_items(big, n_kv)
-                    if half or two_sums:
-                        tile_rows = attention_tile_rows(hd, True, exact_weights, dist)
-                        small, big = attention_items(ctx.q_lens, ctx.q_start_host, ctx.n_cached, G, tile_rows)
+            if len(big) and most_keys > 128 * SHORT_ITEMS_MAX_PASSES and small_rows < tile_rows:
+                cut = cut_key_ranges(big, n_kv, hd, span, compute_units(), None, exact_weights, dist) if whole_pages else None
+                if cut is None and half:
+                    tile_rows = small_rows
+                    small, big = attention_items(ctx.q_lens, ctx.q_start_host, ctx.n_cached, G, tile_rows)
             if cut is not None:
                 small_d, key_parts = upload_key_parts(cut, q.device, small)
                 big_d = key_parts.items

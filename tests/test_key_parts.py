@@ -71,6 +71,8 @@ def test_which_items_a_prompt_gets(monkeypatch, lens, heads, n_kv, rows, two, mo
     monkeypatch.setattr(ops, "compute_units", lambda: 256)
     monkeypatch.setattr(ops, "attention_tile_rows", lambda hd, small=False, exact=False, dist=False: 64 if small else 128)
     monkeypatch.setattr(ops, "upload", lambda values, dtype, device: torch.as_tensor(values))
+    lists, listed = ops.attention_items, []
+    monkeypatch.setattr(ops, "attention_items", lambda *a: listed.append(a) or lists(*a))
     monkeypatch.setattr(ops, "paged_attention_mfma", lambda *a, tile_rows, key_parts, two_sums, **k: seen.append((a[6], tile_rows, key_parts, two_sums)))
     starts = np.concatenate([[0], np.cumsum(lens)])
     ctx = SimpleNamespace(q_lens=np.array(lens), n_cached=np.zeros(len(lens), int), q_start_host=starts, seq_records=None, scratch={})
@@ -79,6 +81,7 @@ def test_which_items_a_prompt_gets(monkeypatch, lens, heads, n_kv, rows, two, mo
     ops.paged_attention(q, q, pages, pages, SimpleNamespace(block_table=None), ctx, heads, 1.0, more.get("window", 0))
     (items, got, parts, sums), = seen
     assert got == rows and parts is None and bool(sums) == two
+    assert len(listed) == 1  # (a step on new inputs waits for each list)
     assert int(items.view(-1, 4)[:, 2].max()) <= rows // (heads // n_kv)
 
 
