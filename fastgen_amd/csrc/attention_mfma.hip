@@ -1453,11 +1453,16 @@ __global__ __launch_bounds__(256) void attn_parts_kernel(const KeyParts from, co
 
 // How the keys of a step's items (of the larger form, host memory) are cut into parts; what a cut gives is counted from a workgroup's
 // passes: a unit holds one workgroup, which takes its passes (128 keys, 2.5 us) and about 3.5 more until it begins and ends, and the
-// merge behind takes 2.4.  Cut where that gains 7 %, into parts of one and a half times the passes that each unit has if all are
+// merge behind takes 2.4.  Cut where that gains 7 % (in the steps of prompts alone up to 43 %, level at the least), into parts of one and a half times the passes that each unit has if all are
 // spread evenly, from items of 11 passes on (the shortest that was measured to gain has 12).
+// Beside decoded tokens (one launch takes both) their chunks fill the units that a long item leaves, and a cut is worth less: it is made
+// where the count says two thirds of the time at most.  Steps of Buderax, Llama 8B (8 layers) and 3B (14) beside 8 to 32 requests, us whole and
+// cut by what the count says: 0.90 (1,500 tokens) 2,546 / 2,618, 0.82 (1,300) 2,360 / 2,422, 0.71 (500 behind 1,500) 3,673 / 3,771, 0.70
+// (800 behind 1,000) 2,054 / 2,134, 0.68 (512 behind 2,000) 3,458 / 3,478; 0.61 (512 behind 4,000) 4,047 / 3,955, 0.55 (600 behind
+// 3,000) 2,351 / 2,203, 0.25 (100 behind 8,000) 2,972 / 2,301.
 // Not in Python: a step on new inputs waits for it (prompts of 611 and 1,437 tokens, 65 items: 18 us with the call, 150 there).
 constexpr int KEY_PART_MIN_PASSES = 11;
-constexpr double KEY_PART_START = 3.5, KEY_PART_MERGE = 2.4, KEY_PART_GAIN = 0.93;
+constexpr double KEY_PART_START = 3.5, KEY_PART_MERGE = 2.4, KEY_PART_GAIN = 0.93, KEY_PART_GAIN_BESIDE = 0.64;
 
 // When the last of `t`, the longest first, ends on so many places (two rounds at most).
 static double passes_until_done(std::vector<double>& t, int places) {
@@ -1470,10 +1475,10 @@ static double passes_until_done(std::vector<double>& t, int places) {
   return std::max(done, total / places);
 }
 
-// items: int32 [n_items][4]; places: workgroups that run at once for a kv head.  most: 0, or cut to at most that many passes whatever it gives.
+// items: int32 [n_items][4]; places: workgroups that run at once for a kv head.  beside: decoded tokens are in the launch.  most: 0, or cut to at most that many passes whatever it gives.
 // cut: int32 [max_parts + n_items][4] items, the longest parts first, list: [max_parts + n_items][2] and merges: [n_items][4] as
 // the kernels take them, count: how many of them, of merges and of places.  No cut (or more than max_parts places): all 0.
-extern "C" int fg_attn_cut_keys(const int* items, int n_items, int window, int places, int most, int max_parts, int* cut, int* list,
+extern "C" int fg_attn_cut_keys(const int* items, int n_items, int window, int places, int beside, int most, int max_parts, int* cut, int* list,
                                 int* merges, int* count) try {
   count[0] = count[1] = count[2] = 0;
   if (n_items <= 0 || window < 0 || places < 1 || most < 0) return FG_OK;
@@ -1487,6 +1492,7 @@ extern "C" int fg_attn_cut_keys(const int* items, int n_items, int window, int p
     total += passes[i];
   }
   const bool asked = most > 0;
+  const double gain = beside ? KEY_PART_GAIN_BESIDE : KEY_PART_GAIN;
   double whole = 0.;
   if (!asked) {
     most = (int)((3 * total + 2 * places - 1) / (2 * places));
@@ -1511,7 +1517,7 @@ extern "C" int fg_attn_cut_keys(const int* items, int n_items, int window, int p
     std::vector<double> t;
     t.reserve(n_all);
     for (int i = 0; i < n_items; ++i) t.insert(t.end(), parts[i], (double)passes[i] / parts[i] + KEY_PART_START);
-    if (passes_until_done(t, places) + KEY_PART_MERGE >= KEY_PART_GAIN * whole) return FG_OK;
+    if (passes_until_done(t, places) + KEY_PART_MERGE >= gain * whole) return FG_OK;
   }
   struct Part { long long share; int item, place, code; };
   std::vector<Part> all;

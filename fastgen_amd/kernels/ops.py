@@ -681,10 +681,10 @@ def key_parts_scratch(head_dim: int) -> int:
 
 
 def cut_key_ranges(big: np.ndarray, n_kv: int, head_dim: int, window: int, cus: int, most: Optional[int] = None, exact: bool = False,
-                   dist: bool = False):
+                   dist: bool = False, beside: bool = False):
     """How the keys of a step's items (:func:`attention_items`, of the larger form) are cut into parts: ``(items, parts, merges, n_places)`` as
     :class:`KeyParts` holds them, the longest parts first, or None where no cut is worth it (``fg_attn_cut_keys`` counts that).
-    ``most``: cut to at most that many passes of 128 keys.
+    ``most``: cut to at most that many passes of 128 keys.  ``beside``: decoded tokens are in the same launch.
 
     Whole and in parts of at most 3/4, 1/2 and 1/4 of the longest item's passes, us: 2,000 tokens of 16 heads on 4 (252 workgroups;
     not cut) 48.8 / 46.5 / 49.7 / 55.8; 611 and 1,437 40.4 / 36.5 / 37.5 / 43.6; 1,500 39.3 / 36.8 / 34.7 / 39.0; 1,500 of 24 heads on 8 (288;
@@ -700,7 +700,7 @@ def cut_key_ranges(big: np.ndarray, n_kv: int, head_dim: int, window: int, cus: 
     out = np.empty(at_count + 3, np.int32)
     to = out.ctypes.data
     _check(_mfma_attention(head_dim, exact, dist).fg_attn_cut_keys(
-        big.ctypes.data, n, window, max(1, cus // n_kv), 0 if most is None else max(1, most), places, to, to + 4 * at_parts,
+        big.ctypes.data, n, window, max(1, cus // n_kv), int(beside), 0 if most is None else max(1, most), places, to, to + 4 * at_parts,
         to + 4 * at_merges, to + 4 * at_count), "attn_cut_keys")
     n_items, n_merges, n_places = out[at_count:].tolist()
     if not n_items:
@@ -1034,7 +1034,8 @@ def paged_attention(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v
                 tile_rows = small_rows if half or two_sums else tile_rows
             small, big = attention_items(ctx.q_lens, ctx.q_start_host, ctx.n_cached, G, tile_rows)
             if len(big) and most_keys > 128 * SHORT_ITEMS_MAX_PASSES and small_rows < tile_rows:
-                cut = cut_key_ranges(big, n_kv, hd, span, compute_units(), None, exact_weights, dist) if whole_pages else None
+                cut = (cut_key_ranges(big, n_kv, hd, span, compute_units(), None, exact_weights, dist, len(small) > 0)
+                       if whole_pages else None)
                 if cut is None and half:
                     tile_rows = small_rows
                     small, big = attention_items(ctx.q_lens, ctx.q_start_host, ctx.n_cached, G, tile_rows)

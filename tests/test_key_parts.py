@@ -54,6 +54,17 @@ def test_what_is_cut():
     assert ops.cut_key_ranges(np.zeros((0, 4), np.int32), 8, 128, 0, 256) is None
 
 
+def test_a_cut_beside_decoded_tokens_has_to_gain_more():
+    """Decoded tokens' chunks fill the units that a long item leaves: prompts whose cut gains little alone stay whole beside them."""
+    def cut(n, past, heads, n_kv, beside):
+        _, big = ops.attention_items([n], [0, n], [past], heads // n_kv, 128)
+        return ops.cut_key_ranges(big, n_kv, 128, 0, 256, beside=beside) is not None
+
+    for n, past, heads, n_kv, worth_it in ((1500, 0, 16, 4, False), (1300, 0, 16, 4, False), (800, 1000, 16, 4, False), (500, 1500, 24, 8, False),
+                                           (512, 2000, 32, 8, False), (512, 4000, 32, 8, True), (600, 3000, 16, 4, True), (100, 8000, 32, 8, True)):
+        assert cut(n, past, heads, n_kv, False) and cut(n, past, heads, n_kv, True) == worth_it
+
+
 @pytest.mark.parametrize("lens,heads,n_kv,rows,two,more", [
     ([300], 32, 8, 64, False, {}), ([512], 32, 8, 64, False, {}), ([513], 32, 8, 64, True, {}), ([380, 874], 24, 8, 64, True, {}),
     ([1280], 32, 8, 64, True, {}), ([1281], 32, 8, 128, False, {}), ([640] * 4, 16, 4, 64, True, {}), ([641] * 4, 16, 4, 128, False, {}),
