@@ -712,25 +712,28 @@ def cut_key_ranges(big: np.ndarray, n_kv: int, head_dim: int, window: int, cus: 
 SHORT_ITEMS_MAX_PASSES = 10  # (of 128 keys; longer items are what fg_attn_cut_keys considers)
 
 
-def _prompt_groups(q_lens, n_cached, group_size: int, tile_rows: int, n_kv: int) -> Tuple[int, int]:
-    """The workgroups that a step's items of so many rows take, and the most keys of one, without listing them (a step on new inputs
-    waits for each list, 50 us for prompts of 611 and 1,437 tokens)."""
-    per_tile, items, most_keys = max(1, tile_rows // group_size), 0, 0
+def _prompt_groups(q_lens, n_cached, group_size: int, tile_rows: int, n_kv: int) -> Tuple[int, int, bool]:
+    """The workgroups that a step's items of so many rows take, the most keys of one, and whether there are decoded tokens (or very short
+    portions) beside them, without listing the items (a step on new inputs waits for each list, 50 us for prompts of 611 and 1,437 tokens)."""
+    per_tile, items, most_keys, beside = max(1, tile_rows // group_size), 0, 0, False
     for n, c in zip(q_lens.tolist(), n_cached.tolist()):
         if n * group_size > 16:
             items += -(-n // per_tile)
             most_keys = max(most_keys, n + c)
-    return items * n_kv, most_keys
+        else:
+            beside = True
+    return items * n_kv, most_keys, beside
 
 
-def _few_short_items(groups: int) -> bool:
-    """Whether a step's short items (so many workgroups of the larger form, more than half a unit's worth) are few enough to go as items
-    of 64 rows with two sums: the same bits in less time up to five workgroups for four units.  Heads of 128, us with items of 128 rows and of 64 by
-    workgroups: 192 (6 passes of 128 keys) 23.5 and 21.7, 240 (10) 33.4 and 31.1, 256 (8; 4; 2) 28.4 and 27.6; 19.1 and 17.2; 14.1 and 11.8, 288 (9)
-    30.9 and 30.3, 320 (10; 5) 33.3 and 33.1; 22.6 and 20.0, 352 (11; 6) 35.7 and 35.8; 25.0 and 23.8, 384 (12; 6) 38.2 and 40.4; 27.3 and 26.3, 448
-    (7) 32.5 and 33.7, 512 (8; 4) 37.5 and 40.9; 28.0 and 27.3.  Beside 24 and 64 decoding requests 248 (7) 40.7 and 35.6, 320 (10) 66.3 and
-    64.2; beside 12 of 4 kv heads 240 (10) 37.5 and 39.6."""
-    return 4 * groups <= 5 * compute_units()
+def _few_short_items(groups: int, most_keys: int, beside: bool) -> bool:
+    """Whether a step's short items (so many workgroups of the larger form, more than half a unit's worth) go as items of 64 rows with two
+    sums, the same bits: where there are no more than units.  Heads of 128, us with items of 128 rows and of 64 by workgroups (and passes of 128
+    keys): 192 (6) 23.5 and 21.7, 240 (10) 33.4 and 31.1, 256 (8; 4; 2) 28.4 and 27.6; 19.1 and 17.2; 14.1 and 11.8, 288 (9) 30.9 and 30.3, 320 (10)
+    33.3 and 33.1, 352 (11) 35.7 and 35.8, 448 (7) 32.5 and 33.7, 512 (8) 37.5 and 40.9; in steps, 240 (10, Buderax) 2,523 and 2,495, 320 (10, Llama
+    8B) 4,884 and 4,893.  Beside decoded tokens (in one launch) only where the keys are fewer still or there are three workgroups for four
+    units: 152 (10) 2,120 and 2,090, 200 (7) 2,353 and 2,319, 248 (7) 4,895 and 4,850; 240 (10) 2,661 and 2,668, 256 (8) 4,011 and 4,041, 320 (10)
+    5,047 and 5,109."""
+    return groups <= compute_units() and (not beside or most_keys <= 128 * 7 or 4 * groups <= 3 * compute_units())
 
 
 def upload_key_parts(cut, device, before: Optional[np.ndarray] = None):
@@ -1025,16 +1028,17 @@ def paged_attention(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v
         else:
             tile_rows, small_rows = (attention_tile_rows(hd, small, exact_weights, dist) for small in (False, True))
             cut, two_sums, whole_pages = None, False, k_pages.shape[2] % 64 == 0
-            groups, most_keys = _prompt_groups(ctx.q_lens, ctx.n_cached, G, tile_rows, n_kv)
+            groups, most_keys, beside = _prompt_groups(ctx.q_lens, ctx.n_cached, G, tile_rows, n_kv)
             # so few items that half the compute units would stand idle: items of half the rows, whose lighter workgroups share a
             # unit (512 tokens of 32 heads on 8, us with items of 128 and of 64 rows: 17.5 and 14.8)
             half = 0 < groups <= compute_units() // 2 and small_rows < tile_rows
             if 0 < groups and most_keys <= 128 * SHORT_ITEMS_MAX_PASSES:  # (no cut of the keys, so the items are listed once)
-                two_sums = not half and small_rows < tile_rows and whole_pages and span == 0 and _few_short_items(groups)
+                two_sums = (not half and small_rows < tile_rows and whole_pages and span == 0
+                            and _few_short_items(groups, most_keys, beside))
                 tile_rows = small_rows if half or two_sums else tile_rows
             small, big = attention_items(ctx.q_lens, ctx.q_start_host, ctx.n_cached, G, tile_rows)
             if len(big) and most_keys > 128 * SHORT_ITEMS_MAX_PASSES and small_rows < tile_rows:
-                cut = (cut_key_ranges(big, n_kv, hd, span, compute_units(), None, exact_weights, dist, len(small) > 0)
+                cut = (cut_key_ranges(big, n_kv, hd, span, compute_units(), None, exact_weights, dist, beside)
                        if whole_pages else None)
                 if cut is None and half:
                     tile_rows = small_rows

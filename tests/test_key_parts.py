@@ -67,12 +67,14 @@ def test_a_cut_beside_decoded_tokens_has_to_gain_more():
 
 @pytest.mark.parametrize("lens,heads,n_kv,rows,two,more", [
     ([300], 32, 8, 64, False, {}), ([512], 32, 8, 64, False, {}), ([513], 32, 8, 64, True, {}), ([380, 874], 24, 8, 64, True, {}),
-    ([1280], 32, 8, 64, True, {}), ([1281], 32, 8, 128, False, {}), ([640] * 4, 16, 4, 64, True, {}), ([641] * 4, 16, 4, 128, False, {}),
+    ([1280], 16, 4, 64, True, {}), ([1281], 16, 4, 128, None, {}), ([512] * 4, 16, 4, 64, True, {}), ([513] * 4, 16, 4, 128, False, {}),
+    ([1280], 32, 8, 128, False, {}), ([1] * 8 + [896], 32, 8, 64, True, {}), ([1] * 8 + [897], 32, 8, 128, False, {}),
+    ([1] * 8 + [768], 32, 8, 64, True, {}), ([1] * 8 + [1200], 16, 4, 64, True, {}), ([1] * 12 + [693, 1204], 16, 4, 128, False, {}),
     ([2048], 32, 8, 128, False, {}), ([1024], 32, 8, 128, False, dict(window=300)), ([1024], 32, 8, 64, True, dict(window=4096)),
     ([1024], 32, 8, 128, False, dict(page=32)), ([512], 32, 8, 64, False, dict(page=32)), ([1024], 32, 8, 128, False, dict(window=-64))])
 def test_which_items_a_prompt_gets(monkeypatch, lens, heads, n_kv, rows, two, more):
-    """Items of 64 rows where half of 256 units would stand idle, and, added up as the larger form does it, up to five workgroups for four
-    units and ten passes; from there on, where a window hides keys and on small pages the form of 128 rows, whose error against
+    """Items of 64 rows where half of 256 units would stand idle, and, added up as the larger form does it, up to a workgroup a unit and ten
+    passes (beside decoded tokens seven, or three workgroups for four units); from there on, where a window hides keys and on small pages the form of 128 rows, whose error against
     64 bits is smaller than that of 64 rows with one sum."""
     from types import SimpleNamespace
 
@@ -82,6 +84,7 @@ def test_which_items_a_prompt_gets(monkeypatch, lens, heads, n_kv, rows, two, mo
     monkeypatch.setattr(ops, "compute_units", lambda: 256)
     monkeypatch.setattr(ops, "attention_tile_rows", lambda hd, small=False, exact=False, dist=False: 64 if small else 128)
     monkeypatch.setattr(ops, "upload", lambda values, dtype, device: torch.as_tensor(values))
+    monkeypatch.setattr(ops, "attention_plan", lambda *a: None)
     lists, listed = ops.attention_items, []
     monkeypatch.setattr(ops, "attention_items", lambda *a: listed.append(a) or lists(*a))
     monkeypatch.setattr(ops, "paged_attention_mfma", lambda *a, tile_rows, key_parts, two_sums, **k: seen.append((a[6], tile_rows, key_parts, two_sums)))
@@ -91,7 +94,9 @@ def test_which_items_a_prompt_gets(monkeypatch, lens, heads, n_kv, rows, two, mo
     pages = torch.empty(1, n_kv, more.get("page", 64), 128, dtype=torch.bfloat16)
     ops.paged_attention(q, q, pages, pages, SimpleNamespace(block_table=None), ctx, heads, 1.0, more.get("window", 0))
     (items, got, parts, sums), = seen
-    assert got == rows and parts is None and bool(sums) == two
+    assert got == rows and bool(sums) == bool(two) and (parts is not None) == (two is None)
+    if two is None:  # (keys in parts)
+        return
     assert len(listed) == 1  # (a step on new inputs waits for each list)
     assert int(items.view(-1, 4)[:, 2].max()) <= rows // (heads // n_kv)
 
