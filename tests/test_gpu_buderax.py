@@ -299,7 +299,8 @@ def test_command_lines(cases, tmp_path):
     assert chat.returncode == 0, chat.stderr[-2000:]
 
 
-@pytest.mark.parametrize("pairs,E", [(1, 3), (255, 32), (256, 256), (256, 257), (257, 32), (1025, 7), (8192, 32), (8193, 32), (9001, 300)])
+@pytest.mark.parametrize("pairs,E", [(1, 3), (255, 32), (256, 256), (256, 257), (257, 32), (1025, 7), (8192, 32), (8193, 32), (9001, 300),
+                                     (1024, 300), (2048, 5), (2049, 32), (4096, 300), (4097, 32)])
 def test_sort_at_the_edges_of_its_forms(pairs, E):
     """Pairs that a thread holds, one more, and more experts than the small form counts: every pair once, among its expert's
     places, and tiles that cover them."""
