@@ -1007,7 +1007,7 @@ enum { PAGES_ANY = 0, PAGES_CHUNK = 1, PAGES_TILE = 2 };  // multiples of 8, 32,
 // and long chunks first, with the heads on the dies where the kernels alone have them.  The same bits as two launches.
 // Llama 3B's layer, prompts of 380 and 874 tokens beside 24 requests of 100 to 1,500: two launches on two streams took 58 us from
 // the cache's write to the next product (34 the tiles, 22 the split under them, 10 the combine kernel, and 17 of waits between the
-// streams), one launch 38 and the combine kernel, whose grid counts a decoded token's rows and not 16, 5.
+// streams), one launch 38 (34 with items of 64 rows, which such a step has) and the combine kernel, whose grid counts a decoded token's rows and not 16, 5.
 // The chunks' sums lie where the tiles do: with LDS of their own a unit held one workgroup from head size 224 on, not two.
 // 2,000 tokens of 16 heads on 4 beside 32, us: two launches 107 / 124 / 125 at 224 / 240 / 256, one with LDS of its own 207 /
 // 205 / 217, one now 106 / 121 / 124 (the registers are then half as many, and a chunk of these sizes spills 36 to 168 bytes a lane).
